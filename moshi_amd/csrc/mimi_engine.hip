@@ -5,6 +5,7 @@
 #include "mmi_graph.h"
 
 #include <math.h>
+#include <algorithm>
 
 namespace {
 
@@ -32,6 +33,91 @@ struct Buf {            // activation buffer [B][C][ld]; first H columns = causa
     bool needs_elu_at_load() const { return !pe && !elu; }
 };
 
+// Scratch of a group program (below): chunks that are kept while the handle lives and handed out again from the start when a program is
+// rebuilt, so that a rebuild neither allocates nor frees.  What is asked for in the same order lies at the same addresses.
+struct MimiSlab {
+    struct Chunk { char* p; size_t size; };
+    std::vector<Chunk> chunks;
+    size_t cur = 0, at = 0;
+    hipError_t alloc(void** p, size_t nb) {
+        nb = (nb + 255) & ~(size_t)255;
+        while (cur < chunks.size() && at + nb > chunks[cur].size) { ++cur; at = 0; }
+        if (cur == chunks.size()) {
+            Chunk c = {nullptr, nb > ((size_t)32 << 20) ? nb : (size_t)32 << 20};
+            hipError_t e = hipMalloc((void**)&c.p, c.size);
+            if (e != hipSuccess) return e;
+            chunks.push_back(c);
+        }
+        *p = chunks[cur].p + at;
+        at += nb;
+        return hipSuccess;
+    }
+    void rewind() { cur = at = 0; }
+    void release() {
+        for (auto& c : chunks) hipFree(c.p);
+        chunks.clear();
+        rewind();
+    }
+};
+
+// Where a program's buffers come from: the stream's arena (zeroed, part of the stream's snapshot), or a slab, whose contents are all
+// written before they are read.  A slab's offset tables are gathered on the host and uploaded at once.
+struct MimiMem {
+    MmiArena* arena = nullptr;
+    MimiSlab* slab = nullptr;
+    int frames = 1;                            // of the program that is built
+    int* tab_dev = nullptr;
+    std::vector<int>* tab_host = nullptr;
+    template <class T>
+    hipError_t alloc(T** p, size_t n) { return arena ? arena->alloc(p, n) : slab->alloc((void**)p, (n ? n : 1) * sizeof(T)); }
+    template <class T>
+    hipError_t zero(T* p, size_t n, hipStream_t s) { return arena ? hipMemsetAsync(p, 0, n * sizeof(T), s) : hipSuccess; }
+    hipError_t table(const std::vector<int>& v, const int** out) {
+        if (slab) {
+            *out = tab_dev + tab_host->size();
+            tab_host->insert(tab_host->end(), v.begin(), v.end());
+            return hipSuccess;
+        }
+        int* dev = nullptr;
+        hipError_t e = arena->alloc(&dev, v.size());
+        if (e == hipSuccess) e = hipMemcpy(dev, v.data(), v.size() * sizeof(int), hipMemcpyHostToDevice);
+        *out = dev;
+        return e;
+    }
+};
+
+// operands of the quantiser's launches, `rows` latents at once
+struct RvqScratch {
+    float* xq = nullptr;                       // [rows][2*Dq] residuals (first | rest)
+    double* best_d = nullptr;
+    int* best_i = nullptr;
+    int* codes = nullptr;                      // [rows][n_q]
+    float *qin_bp = nullptr, *qin_part = nullptr;
+    int rows = 0;
+};
+struct DequantScratch {
+    int* codes = nullptr;                      // [rows][n_q]
+    float* q2 = nullptr;                       // [rows][2*Dq]
+    float *qout_bp = nullptr, *qout_part = nullptr;
+};
+
+// Several consecutive frames of every stream through the network at once: the same launch list as a frame's with `frames` times the
+// columns, so that a launch is worth its latency.  The streaming state stays where the frame program keeps it: the histories are copied
+// in front of the group's rows before its launches and back behind them, everything else is shared.
+// Measured on one stream, 129 frames encoded and decoded (10.3 s of audio): 140 ms frame by frame (176 dependent launches per frame, most of
+// them at the ~4.7 us a dependent launch costs), 7.9 ms in three groups of 43.
+struct MimiGroup {
+    int frames = 0;                            // 0: not built (for this stream)
+    bool refused = false;                      // building failed (shapes, memory): this stream goes frame by frame
+    int tab_B = 0, tab_frames = 0;             // what the slab's tables were uploaded for
+    MimiSlab slab;
+    std::vector<int> tab;
+    MmiProgram prog;
+    Buf in, out;                               // encoder: samples, latents; decoder: latents, samples
+    int* codes = nullptr;
+    HistTable hist;
+};
+
 }  // namespace
 
 struct mmi_mimi {
@@ -51,16 +137,10 @@ struct mmi_mimi {
     ConvW q_in, q_out;                         // stacked first|rest projections
     float* E_all = nullptr;                    // [n_q][bins][D]  (0 = rvq_first.layers.0, 1.. = rvq_rest.layers.*)
     double* e2_all = nullptr;                  // [n_q][bins]
-    // RVQ scratch (max_batch rows)
-    float* xq = nullptr;                       // [maxB][2*Dq] residuals (first | rest)
-    double* best_d = nullptr;
-    int* best_i = nullptr;
-    int* codes_i32 = nullptr;                  // [maxB][n_q]  encoder side: what the RVQ selected
-    int* dec_codes_i32 = nullptr;              // [maxB][n_q]  decoder side: the codes being decoded (its own buffer: an encode of the
-                                               //              next frame may run on another stream while a decode is in flight, duplex.hip)
-    float* q2 = nullptr;                       // [maxB][2*Dq]
-    float* lat_tmp = nullptr;                  // [maxB][dimension]
-    float *qin_bp = nullptr, *qin_part = nullptr, *qout_bp = nullptr, *qout_part = nullptr;   // projection scratch (max_batch)
+    // RVQ scratch (max_batch rows); the decoder side has its own: an encode of the next frame may run on another stream while a decode
+    // is in flight (duplex.hip)
+    RvqScratch rvq;
+    DequantScratch deq;
     int nchunk = 0;
     // streaming state
     bool streaming = false;
@@ -76,6 +156,9 @@ struct mmi_mimi {
     std::vector<long> partial_sizes;           // elements per batch row
     HistDesc* enc_hist = nullptr;
     HistDesc* dec_hist = nullptr;
+    HistTable enc_tab, dec_tab;                // the same tables on the host
+    MimiGroup enc_grp, dec_grp;
+    bool all_exec = true;                      // no exec mask has been set since the stream began (or all of it was reset)
     int enc_nhist = 0, dec_nhist = 0, enc_hist_rows = 0, dec_hist_rows = 0;
     MmiProgram enc_prog, dec_prog;
     hipStream_t cap_stream = nullptr;
@@ -262,7 +345,7 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
 struct ConvPlan {
     bool ln = false;                  // k_gemm_f32_ln: LayerNorm fused in front of the linear
     bool wide = false;
-    int MTB = 1, W = 1, U = 1;        // wide
+    int MTB = 1, W = 1;               // wide
     int NSUB = 1, waves = 4, ksplit = 1, nz = 1;
     bool pack = false;
 };
@@ -285,12 +368,15 @@ void launch_wide_w(hipStream_t s, const ConvGemmArgs& a, int W, dim3 grid) {
 
 int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
     if (p.wide) {
-        const dim3 grid(mmi_cdiv(a.Ntot, 32), mmi_cdiv(a.Mt, p.MTB));
+        const dim3 grid(mmi_cdiv(a.Ntot, 32), mmi_cdiv(a.Mt, p.MTB), p.ksplit);
+        ConvGemmArgs w = a;
+        if (p.ksplit > 1) w.out_mode = MMI_GOUT_PARTIAL;
         switch (p.MTB) {
-            case 1: launch_wide_w<1, 4>(s, a, p.W, grid); break;
-            case 2: launch_wide_w<2, 4>(s, a, p.W, grid); break;
-            default: launch_wide_w<4, 2>(s, a, p.W, grid); break;
+            case 1: launch_wide_w<1, 4>(s, w, p.W, grid); break;
+            case 2: launch_wide_w<2, 4>(s, w, p.W, grid); break;
+            default: launch_wide_w<4, 2>(s, w, p.W, grid); break;
         }
+        if (p.ksplit > 1) MMI_LAUNCH(k_conv_finish, (int)mmi_cdiv64((int64_t)a.Cout * a.Ntot, 256), 256, 0, s, a, p.ksplit);
         MMI_CHECK_LAUNCH();
         return MMI_OK;
     }
@@ -320,11 +406,99 @@ int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
     return MMI_OK;
 }
 
+// k_conv_wide on N columns: m-tiles per wave and waves that split the reduction
+void wide_rule(const ConvGemmArgs& a, int N, int* mtb_out, int* w_out) {
+    const int nsub = mmi_cdiv(N, 32);
+    // m-tiles per wave (each gathered + ELU'd operand element is reused MTB times) vs. waves in flight:
+    // aim for >= 1024 waves, taking the parallelism from split-K waves (W) before shrinking MTB
+    int MTB = 4;                         // 8 m-tiles per wave needs > 256 registers per lane: one wave per SIMD, slower
+    while (MTB > a.Mt) MTB >>= 1;
+    int W = 1;
+    auto waves = [&](int mtb, int w) { return nsub * mmi_cdiv(a.Mt, mtb) * w; };
+    auto wmax = [&](int mtb) { int w = 1; while (w < 8 && w * 2 * mtb <= 16 && a.Q / (w * 2) >= 4) w <<= 1; return w; };
+    while (MTB > 1 && waves(MTB, wmax(MTB)) < 1024) MTB >>= 1;
+    while (W < wmax(MTB) && waves(MTB, W) < 1024) W <<= 1;
+    // Measured tilings of the codec's own layer shapes (profiles/r02_logs/conv_wide_tiling_sweep_b{8,32,64}.txt: every
+    // (MTB, W) forced on every layer, per-site times from the kernel trace).  The rule above is within a few percent of the
+    // best at 8 sessions but leaves 72 us per frame at 32 sessions and 114 us at 64: what it does not see is the workgroup
+    // count against the 256 CUs (a strided conv of 16 column tiles at MTB = 2 is 128 workgroups - half the chip) and the
+    // 64-value epilogue of an unsplit MTB = 4 wave.  Shapes not listed (other codecs, other batch classes) keep the rule.
+    // Same fp32 results up to summation order (W waves split the reduction), like any other tiling.
+    {
+        struct Tune { int Cin, Cout, K, S, nsub, MTB, W; };
+        static const Tune kTune[] = {
+            // 32 sessions (column tiles of the layer at 32 sessions)
+            {128, 256, 10, 5, 96, 4, 4},    // enc.down1   45.9 -> 34.1 us
+            {256, 512, 12, 6, 16, 1, 8},    // enc.down2   47.4 -> 30.8
+            {128, 64, 3, 1, 480, 1, 4},     // resblock 128 ch (enc.res1 / dec.res2), first conv
+            {64, 128, 1, 1, 480, 1, 4},     //   second conv                      32.9 -> 31.9, 32.7 -> 31.2
+            {256, 128, 3, 1, 96, 1, 4},     // resblock 256 ch (enc.res2 / dec.res1)
+            {128, 256, 1, 1, 96, 1, 4},     //                                    24.6 -> 23.3, 26.0 -> 23.0
+            {512, 256, 3, 1, 16, 1, 8},     // resblock 512 ch (enc.res3 / dec.res0)
+            {256, 512, 1, 1, 16, 1, 8},     //                                    21.4 -> 19.4, 21.9 -> 20.1
+            {512, 3072, 1, 1, 16, 1, 8},    // dec.convtr1 (rows = Cout * K)      41.5 -> 34.2 (with its combine)
+            {256, 1280, 1, 1, 96, 4, 4},    // dec.convtr2                        49.1 -> 47.0
+            {128, 512, 1, 1, 480, 1, 2},    // dec.convtr3                        76.6 -> 55.6
+            {64, 1, 7, 1, 1920, 1, 4},      // dec.final                          18.9 -> 16.6
+            // 64 sessions
+            {128, 256, 10, 5, 192, 2, 8},   // enc.down1   78.2 -> 64.1
+            {256, 512, 12, 6, 32, 2, 8},    // enc.down2   54.8 -> 49.0
+            {256, 128, 3, 1, 192, 1, 4},    // resblock 256 ch                    42.3 -> 34.9, 41.4 -> 34.1
+            {128, 256, 1, 1, 192, 1, 4},
+            {512, 256, 3, 1, 32, 1, 8},     // resblock 512 ch                    34.1 -> 22.5, 36.3 -> 22.5
+            {256, 512, 1, 1, 32, 1, 8},
+            {512, 3072, 1, 1, 32, 1, 8},    // dec.convtr1                        61.1 -> 58.9
+            {256, 1280, 1, 1, 192, 4, 4},   // dec.convtr2                       100.2 -> 82.3
+            {128, 512, 1, 1, 960, 1, 2},    // dec.convtr3                       128.8 -> 99.5
+            {64, 1, 7, 1, 3840, 1, 4},      // dec.final                          31.5 -> 28.1
+        };
+        for (const Tune& t : kTune)
+                if (t.Cin == a.Cin && t.Cout == a.Cout && t.K == a.K && t.S == a.S && 4 * nsub >= 3 * t.nsub && 2 * nsub < 3 * t.nsub) {
+                    MTB = t.MTB; W = t.W;
+                    while (MTB > a.Mt) MTB >>= 1;
+                    break;
+                }
+    }
+    if (const char* e = getenv("MMI_CONV_MTB")) { const int v = atoi(e); if (v == 1 || v == 2 || v == 4) MTB = v; }   // test hooks
+    if (const char* e = getenv("MMI_CONV_W")) { const int v = atoi(e); if (v == 1 || v == 2 || v == 4 || v == 8) W = v; }
+    while (W * MTB > 16) W >>= 1;          // split-K reduction buffer: W * MTB * 4 KiB of LDS, keep it within 64 KiB
+    *mtb_out = MTB; *w_out = W;
+}
+
+// k_gemm_f32 on N <= 128 columns: subtiles per workgroup, waves that split the reduction, workgroups that do
+void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
+    const int nsub = mmi_cdiv(N, 32);
+    p->NSUB = nsub <= 1 ? 1 : (nsub == 2 ? 2 : 4);
+    // small weight matrices (the transformer linears, <= 8 MB): one workgroup per n-subtile, up to 16 waves splitting K
+    const bool spread = nsub >= 2 && (size_t)a.Mt * a.Q * 1024 <= ((size_t)8 << 20);
+    int ks = 1;
+    if (a.out_mode == MMI_GOUT_NATURAL) {
+        // only the large strided convs (>= 2048-deep reductions, tens of MB of weights) are worth a finishing launch
+        while (a.Q >= 256 && ks < 8 && a.Mt * ks * 2 <= 256 && a.Q / (ks * 2) >= 32) ks <<= 1;
+    }
+    if (const char* e = getenv("MMI_CONV_KSPLIT")) {   // test hook
+        const int v = atoi(e);
+        if (a.out_mode == MMI_GOUT_NATURAL && v >= 1 && v <= 8 && a.Q >= v) ks = v;
+    }
+    p->ksplit = ks;
+    const int qblk = a.Q / ks;
+    if (spread) {
+        p->NSUB = 1;
+        p->nz = nsub;
+        p->waves = qblk >= 16 ? 8 : 4;
+    } else {
+        p->waves = (p->NSUB <= 2 && qblk >= 32) ? 8 : 4;
+    }
+}
+
 // Decide the launch sequence of one conv and allocate its scratch (offset table / packed operand / partials) from
-// `arena`.  `a.x_packed`: the producer writes a.bp itself.  `a.out_mode` PACKED: the result feeds a linear directly.
-int plan_conv(MmiArena& arena, ConvGemmArgs& a, ConvPlan* p) {
-    const int N = a.Ntot;
-    if (a.Cin * a.K >= (1 << 17) || N >= (1 << 17) || a.T_out >= (1 << 11) || a.K >= (1 << 11))
+// `mem`.  `a.x_packed`: the producer writes a.bp itself.  `a.out_mode` PACKED: the result feeds a linear directly.
+// A group's conv (mem.frames > 1) forms every sum in the order in which the frame program forms it - its reduction is cut into the same
+// pieces, over the waves and over the workgroups - so that frames give the same bits however many are run at once; only what each
+// workgroup covers follows the group's own number of columns.
+int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
+    const int N = a.Ntot, N1 = N / mem.frames;
+    if (a.Cin * a.K >= (1 << 17) || N >= (1 << 17) || a.K >= (1 << 11))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "conv dimensions outside the range of the kernels' index arithmetic (sessions x samples per frame "
                                              "must stay below 131072: 68 sessions per handle at 1920 samples per frame)");
     if (N > 128) {
@@ -332,61 +506,22 @@ int plan_conv(MmiArena& arena, ConvGemmArgs& a, ConvPlan* p) {
             return mmi_fail(MMI_ERR_UNSUPPORTED, "more than 128 columns (sessions x time steps per frame) on a conv with replicate padding or packed "
                                                  "operands: lower max_batch (the 25 Hz layers of the released codec take 64 sessions)");
         p->wide = true;
-        const int nsub = mmi_cdiv(N, 32);
-        // m-tiles per wave (each gathered + ELU'd operand element is reused MTB times) vs. waves in flight:
-        // aim for >= 1024 waves, taking the parallelism from split-K waves (W) before shrinking MTB
-        int MTB = 4;                         // 8 m-tiles per wave needs > 256 registers per lane: one wave per SIMD, slower
-        while (MTB > a.Mt) MTB >>= 1;
-        int W = 1;
-        auto waves = [&](int mtb, int w) { return nsub * mmi_cdiv(a.Mt, mtb) * w; };
-        auto wmax = [&](int mtb) { int w = 1; while (w < 8 && w * 2 * mtb <= 16 && a.Q / (w * 2) >= 4) w <<= 1; return w; };
-        while (MTB > 1 && waves(MTB, wmax(MTB)) < 1024) MTB >>= 1;
-        while (W < wmax(MTB) && waves(MTB, W) < 1024) W <<= 1;
-        // Measured tilings of the codec's own layer shapes (profiles/r02_logs/conv_wide_tiling_sweep_b{8,32,64}.txt: every
-        // (MTB, W) forced on every layer, per-site times from the kernel trace).  The rule above is within a few percent of the
-        // best at 8 sessions but leaves 72 us per frame at 32 sessions and 114 us at 64: what it does not see is the workgroup
-        // count against the 256 CUs (a strided conv of 16 column tiles at MTB = 2 is 128 workgroups - half the chip) and the
-        // 64-value epilogue of an unsplit MTB = 4 wave.  Shapes not listed (other codecs, other batch classes) keep the rule.
-        // Same fp32 results up to summation order (W waves split the reduction), like any other tiling.
-        {
-            struct Tune { int Cin, Cout, K, S, nsub, MTB, W; };
-            static const Tune kTune[] = {
-                // 32 sessions (column tiles of the layer at 32 sessions)
-                {128, 256, 10, 5, 96, 4, 4},    // enc.down1   45.9 -> 34.1 us
-                {256, 512, 12, 6, 16, 1, 8},    // enc.down2   47.4 -> 30.8
-                {128, 64, 3, 1, 480, 1, 4},     // resblock 128 ch (enc.res1 / dec.res2), first conv
-                {64, 128, 1, 1, 480, 1, 4},     //   second conv                      32.9 -> 31.9, 32.7 -> 31.2
-                {256, 128, 3, 1, 96, 1, 4},     // resblock 256 ch (enc.res2 / dec.res1)
-                {128, 256, 1, 1, 96, 1, 4},     //                                    24.6 -> 23.3, 26.0 -> 23.0
-                {512, 256, 3, 1, 16, 1, 8},     // resblock 512 ch (enc.res3 / dec.res0)
-                {256, 512, 1, 1, 16, 1, 8},     //                                    21.4 -> 19.4, 21.9 -> 20.1
-                {512, 3072, 1, 1, 16, 1, 8},    // dec.convtr1 (rows = Cout * K)      41.5 -> 34.2 (with its combine)
-                {256, 1280, 1, 1, 96, 4, 4},    // dec.convtr2                        49.1 -> 47.0
-                {128, 512, 1, 1, 480, 1, 2},    // dec.convtr3                        76.6 -> 55.6
-                {64, 1, 7, 1, 1920, 1, 4},      // dec.final                          18.9 -> 16.6
-                // 64 sessions
-                {128, 256, 10, 5, 192, 2, 8},   // enc.down1   78.2 -> 64.1
-                {256, 512, 12, 6, 32, 2, 8},    // enc.down2   54.8 -> 49.0
-                {256, 128, 3, 1, 192, 1, 4},    // resblock 256 ch                    42.3 -> 34.9, 41.4 -> 34.1
-                {128, 256, 1, 1, 192, 1, 4},
-                {512, 256, 3, 1, 32, 1, 8},     // resblock 512 ch                    34.1 -> 22.5, 36.3 -> 22.5
-                {256, 512, 1, 1, 32, 1, 8},
-                {512, 3072, 1, 1, 32, 1, 8},    // dec.convtr1                        61.1 -> 58.9
-                {256, 1280, 1, 1, 192, 4, 4},   // dec.convtr2                       100.2 -> 82.3
-                {128, 512, 1, 1, 960, 1, 2},    // dec.convtr3                       128.8 -> 99.5
-                {64, 1, 7, 1, 3840, 1, 4},      // dec.final                          31.5 -> 28.1
-            };
-            for (const Tune& t : kTune)
-                    if (t.Cin == a.Cin && t.Cout == a.Cout && t.K == a.K && t.S == a.S && 4 * nsub >= 3 * t.nsub && 2 * nsub < 3 * t.nsub) {
-                        MTB = t.MTB; W = t.W;
-                        while (MTB > a.Mt) MTB >>= 1;
-                        break;
-                    }
+        a.q_blk = a.Q;
+        wide_rule(a, N1 > 128 ? N1 : N, &p->MTB, &p->W);
+        if (mem.frames > 1) {
+            if (N1 <= 128) {
+                gemm_rule(a, N1, p);
+                p->W = p->waves;
+            }
+            // as many m-tiles per wave as leave 2048 waves
+            p->MTB = 4;
+            while (p->MTB > 1 && (p->MTB > a.Mt || p->W * p->MTB > 16 || (long)mmi_cdiv(N, 32) * mmi_cdiv(a.Mt, p->MTB) * p->W * p->ksplit < 2048)) p->MTB >>= 1;
+            a.q_blk = mmi_cdiv(a.Q, p->ksplit);
+            if (p->ksplit > 1) {
+                a.Npad = mmi_cdiv(N, 32) * 32;
+                MMI_HIP_CHECK(mem.alloc(&a.partial, (size_t)p->ksplit * a.Mt * 32 * a.Npad));
+            }
         }
-        if (const char* e = getenv("MMI_CONV_MTB")) { const int v = atoi(e); if (v == 1 || v == 2 || v == 4) MTB = v; }   // test hooks
-        if (const char* e = getenv("MMI_CONV_W")) { const int v = atoi(e); if (v == 1 || v == 2 || v == 4 || v == 8) W = v; }
-        while (W * MTB > 16) W >>= 1;          // split-K reduction buffer: W * MTB * 4 KiB of LDS, keep it within 64 KiB
-        p->MTB = MTB; p->W = W;
         std::vector<int> tab((size_t)a.Q * 8);
         for (int q = 0; q < a.Q; ++q)
             for (int h = 0; h < 2; ++h)
@@ -394,10 +529,7 @@ int plan_conv(MmiArena& arena, ConvGemmArgs& a, ConvPlan* p) {
                     const int kd = (q * 4 + e) * 2 + h;
                     tab[((size_t)q * 2 + h) * 4 + e] = kd < a.Cin * a.K ? (kd / a.K) * a.x_ld + kd % a.K : 0;
                 }
-        int* dev = nullptr;
-        MMI_HIP_CHECK(arena.alloc(&dev, tab.size()));
-        MMI_HIP_CHECK(hipMemcpy(dev, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
-        a.koff = dev;
+        MMI_HIP_CHECK(mem.table(tab, &a.koff));
         return MMI_OK;
     }
     p->wide = false;
@@ -411,40 +543,30 @@ int plan_conv(MmiArena& arena, ConvGemmArgs& a, ConvPlan* p) {
         a.Npad = 32;
         return MMI_OK;
     }
-    p->NSUB = nsub <= 1 ? 1 : (nsub == 2 ? 2 : 4);
-    a.Npad = p->NSUB * 32;
+    gemm_rule(a, N, p);
+    a.Npad = (nsub <= 1 ? 1 : (nsub == 2 ? 2 : 4)) * 32;
+    if (mem.frames > 1) {
+        ConvPlan f;
+        gemm_rule(a, N1, &f);
+        p->ksplit = f.ksplit;
+        if (f.waves == 8 && p->NSUB == 4) {          // (four subtiles of eight waves are not built)
+            p->NSUB = 2;
+            p->nz = mmi_cdiv(nsub, 2);
+        }
+        p->waves = f.waves;
+    }
     if (!a.x_packed) {
         if (!a.bp) {
             float* bp = nullptr;
-            MMI_HIP_CHECK(arena.alloc(&bp, (size_t)nsub * a.Q * 256));
+            MMI_HIP_CHECK(mem.alloc(&bp, (size_t)nsub * a.Q * 256));
             a.bp = bp;
         }
         p->pack = true;
     }
-    // small weight matrices (the transformer linears, <= 8 MB): one workgroup per n-subtile, up to 16 waves splitting K
-    const bool spread = nsub >= 2 && (size_t)a.Mt * a.Q * 1024 <= ((size_t)8 << 20);
-    int ks = 1;
-    if (a.out_mode == MMI_GOUT_NATURAL) {
-        // only the large strided convs (>= 2048-deep reductions, tens of MB of weights) are worth a finishing launch
-        while (a.Q >= 256 && ks < 8 && a.Mt * ks * 2 <= 256 && a.Q / (ks * 2) >= 32) ks <<= 1;
-    }
-    if (const char* e = getenv("MMI_CONV_KSPLIT")) {   // test hook
-        const int v = atoi(e);
-        if (a.out_mode == MMI_GOUT_NATURAL && v >= 1 && v <= 8 && a.Q >= v) ks = v;
-    }
-    p->ksplit = ks;
-    if (ks > 1 && !a.partial) {
+    if (p->ksplit > 1 && !a.partial) {
         float* part = nullptr;
-        MMI_HIP_CHECK(arena.alloc(&part, (size_t)ks * a.Mt * 32 * a.Npad));
+        MMI_HIP_CHECK(mem.alloc(&part, (size_t)p->ksplit * a.Mt * 32 * a.Npad));
         a.partial = part;
-    }
-    const int qblk = a.Q / ks;
-    if (spread) {
-        p->NSUB = 1;
-        p->nz = nsub;
-        p->waves = qblk >= 16 ? 8 : 4;
-    } else {
-        p->waves = (p->NSUB <= 2 && qblk >= 32) ? 8 : 4;
     }
     return MMI_OK;
 }
@@ -461,7 +583,7 @@ ConvGemmArgs conv_args(const ConvW& w, const Buf& in, int x_off, int T_out, cons
     a.out = out.p; a.out_ld = out.ld; a.out_off = out_off;
     a.out2 = out.pe; a.elu_out = out.elu ? 1 : 0;
     a.B = B; a.Cin = w.Cin; a.Cout = w.Cout; a.K = w.K; a.S = w.S; a.T_out = T_out;
-    a.T_magic = mmi_div_magic(T_out); a.K_magic = mmi_div_magic(w.K);
+    a.T_magic = mmi_div_magic(T_out, mmi_div_shift(T_out)); a.T_shift = mmi_div_shift(T_out); a.K_magic = mmi_div_magic(w.K);
     a.Mt = w.Mt; a.Q = w.Q; a.Ntot = B * T_out;
     a.elu_in = elu_in ? 1 : 0;
     a.act_out = MMI_ACT_NONE;
@@ -474,7 +596,7 @@ ConvGemmArgs conv_args(const ConvW& w, const Buf& in, int x_off, int T_out, cons
 // them).  A 32-column tile of a conv's output is then exactly one cache line per row: consecutive workgroups run on different
 // XCDs (different L2s), and with rows starting at arbitrary 8-byte offsets every line was written in part by two of them.
 // MMI_MIMI_NO_ALIGN=1 keeps the dense layout (A/B).  Nothing else knows: every kernel takes (pointer, row stride, H).
-int alloc_buf(mmi_mimi* m, int B, int C, int H, int T, Buf* b, hipStream_t s) {
+int alloc_buf(MimiMem& mem, int B, int C, int H, int T, Buf* b, hipStream_t s) {
     b->C = C; b->H = H; b->ld = H + T; b->lead = 0;
     if (T >= 32 && !getenv("MMI_MIMI_NO_ALIGN")) {
         b->lead = (32 - H % 32) % 32;
@@ -482,18 +604,18 @@ int alloc_buf(mmi_mimi* m, int B, int C, int H, int T, Buf* b, hipStream_t s) {
     }
     size_t n = (size_t)B * C * b->ld + b->lead;
     float* base = nullptr;
-    MMI_HIP_CHECK(m->st.alloc(&base, n));
-    MMI_HIP_CHECK(hipMemsetAsync(base, 0, n * sizeof(float), s));
+    MMI_HIP_CHECK(mem.alloc(&base, n));
+    MMI_HIP_CHECK(mem.zero(base, n, s));
     b->p = base + b->lead;
     return MMI_OK;
 }
 
 // ELU twin of a buffer (same geometry, zero history: ELU(0) = 0)
-int alloc_twin(mmi_mimi* m, int B, Buf* b, hipStream_t s) {
+int alloc_twin(MimiMem& mem, int B, Buf* b, hipStream_t s) {
     size_t n = (size_t)B * b->C * b->ld + b->lead;
     float* base = nullptr;
-    MMI_HIP_CHECK(m->st.alloc(&base, n));
-    MMI_HIP_CHECK(hipMemsetAsync(base, 0, n * sizeof(float), s));
+    MMI_HIP_CHECK(mem.alloc(&base, n));
+    MMI_HIP_CHECK(mem.zero(base, n, s));
     b->pe = base + b->lead;
     return MMI_OK;
 }
@@ -506,9 +628,9 @@ HistDesc hist_of_src(const Buf& b, int T) {
     return hist_of(c, T);
 }
 
-int add_conv(mmi_mimi* m, MmiProgram& prog, ConvGemmArgs a, MmiArena* arena = nullptr) {
+int add_conv(MimiMem& mem, MmiProgram& prog, ConvGemmArgs a) {
     ConvPlan p;
-    int rc = plan_conv(arena ? *arena : m->st, a, &p);
+    int rc = plan_conv(mem, a, &p);
     if (rc) return rc;
     prog.add([a, p](hipStream_t s) { return launch_conv_plan(s, a, p); });
     return MMI_OK;
@@ -516,22 +638,22 @@ int add_conv(mmi_mimi* m, MmiProgram& prog, ConvGemmArgs a, MmiArena* arena = nu
 
 // SEANet residual block (conv K -> hidden, conv 1x1 -> channels, + input): ONE launch (k_resblock) at audio rate when the block
 // has the shape the kernel is built for and enough columns to fill the chip with 32-column workgroups; else the two convs.
-int add_resblock(mmi_mimi* m, MmiProgram& prog, ConvGemmArgs a1, ConvGemmArgs a2, const ConvW& w2) {
+int add_resblock(MimiMem& mem, MmiProgram& prog, ConvGemmArgs a1, ConvGemmArgs a2, const ConvW& w2) {
     const int nblk = mmi_cdiv(a1.Ntot, 32);
     long min_waves = 256;                        // below that the two-launch path (split-K over waves) fills the chip better
     if (const char* e = getenv("MMI_MIMI_RES_FUSION_MIN")) min_waves = atol(e);      // test hook: the tiny shapes
     // Measured on MI355X (profiles/r02_logs/resblock_*): the 64-channel blocks (one hidden tile, 1920 one-wave workgroups) gain
     // 8-13 us each over two launches; the 128 / 256-channel blocks (480 / 96 workgroups of 2 / 4 waves: one wave per SIMD on part of
     // the chip) lost 2-15 us to the two-launch path's split-K over waves and are not instantiated.
-    const bool fuse = a1.Ntot > 128 && a1.S == 1 && a2.K == 1 && a2.S == 1 && a1.Cout == a2.Cin && a1.Ntot == a2.Ntot &&
+    const bool fuse = a1.Ntot / mem.frames > 128 && a1.S == 1 && a2.K == 1 && a2.S == 1 && a1.Cout == a2.Cin && a1.Ntot == a2.Ntot &&
                       a1.T_out == a2.T_out && a1.Mt == 1 && w2.wpk_h && a2.Q <= 4 * a1.Mt &&
-                      a2.Mt >= a1.Mt && (long)nblk * a1.Mt >= min_waves && !a1.first && !a2.first && !a1.res && !a1.scale && !a2.scale &&
-                      a1.T_out % 32 == 0 && a1.Cin <= 64 * a1.Mt && a1.K <= 33 &&
+                      a2.Mt >= a1.Mt && (long)mmi_cdiv(a1.Ntot / mem.frames, 32) * a1.Mt >= min_waves && !a1.first && !a2.first && !a1.res && !a1.scale && !a2.scale &&
+                      a1.T_out / mem.frames % 32 == 0 && a1.Cin <= 64 * a1.Mt && a1.K <= 33 &&
                       a1.act_out == MMI_ACT_NONE && a2.act_out == MMI_ACT_NONE;
     if (!fuse) {
-        int rc = add_conv(m, prog, a1);
+        int rc = add_conv(mem, prog, a1);
         if (rc) return rc;
-        return add_conv(m, prog, a2);
+        return add_conv(mem, prog, a2);
     }
     a2.wpk = w2.wpk_h;
     a2.elu_in = 0;                               // the hidden tensor never exists un-activated
@@ -549,18 +671,19 @@ int add_resblock(mmi_mimi* m, MmiProgram& prog, ConvGemmArgs a1, ConvGemmArgs a2
     return MMI_OK;
 }
 
-// residual vector quantiser: latent [B][dim] (column `lat_off` of rows of length lat_ld) -> codes_i32 [B][n_q]
-// latent_packed: the producer of the latent also wrote it as the packed operand m->qin_bp (ConvGemmArgs::outp): no pack launch
-int add_quantize_ops(mmi_mimi* m, MmiProgram& prog, const float* latent, int lat_ld, int lat_off, int B, bool latent_packed = false) {
+// residual vector quantiser: latent [B][dim] (column `lat_off` of rows of length lat_ld) -> r.codes [B][n_q]
+// latent_packed: the producer of the latent also wrote it as the packed operand r.qin_bp (ConvGemmArgs::outp): no pack launch
+int add_quantize_ops(mmi_mimi* m, MimiMem& mem, const RvqScratch& r, MmiProgram& prog, const float* latent, int lat_ld, int lat_off, int B,
+                     bool latent_packed = false) {
     const mmi_mimi_cfg& c = m->cfg;
     const int D = c.q_dimension, bins = c.q_bins;
     Buf in; in.p = const_cast<float*>(latent); in.C = c.dimension; in.ld = lat_ld; in.H = lat_off;
-    Buf out; out.p = m->xq; out.C = 2 * D; out.ld = 1; out.H = 0;
+    Buf out; out.p = r.xq; out.C = 2 * D; out.ld = 1; out.H = 0;
     {
         ConvGemmArgs a = conv_args(m->q_in, in, lat_off, 1, out, 0, B, false);
-        a.bp = m->qin_bp; a.partial = m->qin_part;
+        a.bp = r.qin_bp; a.partial = r.qin_part;
         a.x_packed = latent_packed ? 1 : 0;
-        int rc = add_conv(m, prog, a);
+        int rc = add_conv(mem, prog, a);
         if (rc) return rc;
     }
     const int K = m->n_codebooks;
@@ -569,15 +692,15 @@ int add_quantize_ops(mmi_mimi* m, MmiProgram& prog, const float* latent, int lat
     auto level = [&](int k, int slot) {
         const bool sem = k < c.q_n_q_semantic;
         RvqLevel L;
-        L.x = m->xq + (sem ? 0 : D);
+        L.x = r.xq + (sem ? 0 : D);
         L.E = m->E_all + (size_t)k * bins * D;
         L.e2 = m->e2_all + (size_t)k * bins;
-        L.best_d = m->best_d + (size_t)slot * nchunk * m->max_batch;
-        L.best_i = m->best_i + (size_t)slot * nchunk * m->max_batch;
+        L.best_d = r.best_d + (size_t)slot * nchunk * r.rows;
+        L.best_i = r.best_i + (size_t)slot * nchunk * r.rows;
         L.level = k;
         return L;
     };
-    int* codes = m->codes_i32; const int nq = c.q_n_q;
+    int* codes = r.codes; const int nq = c.q_n_q;
     // the semantic quantiser's single level and the first acoustic level share their two launches (independent, see RvqLevel)
     const bool pair = c.q_n_q_semantic == 1 && K >= 2 && !getenv("MMI_RVQ_NO_PAIR");
     for (int k = 0; k < K; ++k) {
@@ -596,31 +719,33 @@ int add_quantize_ops(mmi_mimi* m, MmiProgram& prog, const float* latent, int lat
     return MMI_OK;
 }
 
-// codes_i32 [B][n_q] (first K used) -> latent written to out buffer column out_off
+// d.codes [B * T][n_q] (first K used; row b * T + t) -> latents t of stream b, written to out buffer column out_off + t
 // k_from_device: the streaming decoder's captured program (K of each call comes from m->dec_k_dev); the one-shot programs of
 // decode_latent bake their K in
-int add_dequant_ops(mmi_mimi* m, MmiProgram& prog, int K, const Buf& out, int out_off, int B, bool k_from_device = false) {
+int add_dequant_ops(mmi_mimi* m, MimiMem& mem, const DequantScratch& d, MmiProgram& prog, int K, const Buf& out, int out_off, int B, int T = 1,
+                    bool k_from_device = false) {
     const mmi_mimi_cfg& c = m->cfg;
-    const int D = c.q_dimension, bins = c.q_bins, nq = c.q_n_q, nsem = c.q_n_q_semantic;
-    float* q2 = m->q2; const int* codes = m->dec_codes_i32; const float* E = m->E_all; const int* kdev = k_from_device ? m->dec_k_dev : nullptr;
-    const bool packed = B <= 128 && m->q_out.Q * 8 == 2 * D && !getenv("MMI_MIMI_PACK_LAUNCHES");
-    float* qp = packed ? m->qout_bp : nullptr; const int qQ = m->q_out.Q;
+    const int D = c.q_dimension, bins = c.q_bins, nq = c.q_n_q, nsem = c.q_n_q_semantic, rows = B * T;
+    float* q2 = d.q2; const int* codes = d.codes; const float* E = m->E_all; const int* kdev = k_from_device ? m->dec_k_dev : nullptr;
+    const bool packed = rows <= 128 && m->q_out.Q * 8 == 2 * D && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    if (T > 1 && !packed) return mmi_fail(MMI_ERR_UNSUPPORTED, "dequantising several frames needs the packed operand");
+    float* qp = packed ? d.qout_bp : nullptr; const int qQ = m->q_out.Q;
     prog.add([=](hipStream_t s) {
-        MMI_LAUNCH(k_rvq_gather, mmi_cdiv(B * D, 256), 256, 0, s, codes, nq, K, E, bins, D, nsem, q2, B, kdev, qp, qQ);
+        MMI_LAUNCH(k_rvq_gather, mmi_cdiv(rows * D, 256), 256, 0, s, codes, nq, K, E, bins, D, nsem, q2, rows, kdev, qp, qQ);
         MMI_CHECK_LAUNCH();
         return (int)MMI_OK;
     });
-    Buf in; in.p = m->q2; in.C = 2 * D; in.ld = 1; in.H = 0;
-    ConvGemmArgs a = conv_args(m->q_out, in, 0, 1, out, out_off, B, false);
-    a.bp = m->qout_bp; a.partial = m->qout_part;
+    Buf in; in.p = d.q2; in.C = 2 * D; in.ld = 1; in.H = 0;
+    ConvGemmArgs a = conv_args(m->q_out, in, 0, T, out, out_off, B, false);
+    a.bp = d.qout_bp; a.partial = d.qout_part;
     a.x_packed = packed ? 1 : 0;                 // the gather wrote the operand
-    return add_conv(m, prog, a);
+    return add_conv(mem, prog, a);
 }
 
 // one streaming transformer (ProjectedTransformer with conv_layout, transformer.py:932-983) working in place
-// on x = buf[:, :, off:off+T]
-int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& layers, const Buf& xb, int off, int T,
-                    float* kv, const long* offsets, int B, hipStream_t init_stream) {
+// on x = buf[:, :, off:off+T], T = frames * (steps per frame)
+int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vector<TrLayerW>& layers, const Buf& xb, int off, int T,
+                    float* kv, const long* offsets, int B, int frames, hipStream_t init_stream) {
     const mmi_mimi_cfg& c = m->cfg;
     const int d = c.tr_d_model, H = c.tr_num_heads, Dh = d / H, ff = c.tr_dim_feedforward, cap = c.tr_context;
     const int N = B * T;
@@ -629,24 +754,34 @@ int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& 
     const bool packed = N <= 128;
     Buf y, qkv, att, hb;
     int rc;
-    if ((rc = alloc_buf(m, B, d, 0, T, &y, init_stream))) return rc;
-    if ((rc = alloc_buf(m, B, 3 * d, 0, T, &qkv, init_stream))) return rc;
-    if ((rc = alloc_buf(m, B, d, 0, T, &att, init_stream))) return rc;
-    if ((rc = alloc_buf(m, B, ff, 0, T, &hb, init_stream))) return rc;
+    if ((rc = alloc_buf(mem, B, d, 0, T, &y, init_stream))) return rc;
+    if ((rc = alloc_buf(mem, B, 3 * d, 0, T, &qkv, init_stream))) return rc;
+    if ((rc = alloc_buf(mem, B, d, 0, T, &att, init_stream))) return rc;
+    if ((rc = alloc_buf(mem, B, ff, 0, T, &hb, init_stream))) return rc;
     float *yp = nullptr, *attp = nullptr, *hbp = nullptr;
     const int nsub = mmi_cdiv(N, 32), Qd = mmi_cdiv(d, 8), Qff = mmi_cdiv(ff, 8);
     if (packed) {
-        MMI_HIP_CHECK(m->st.alloc(&yp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(m->st.alloc(&attp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(m->st.alloc(&hbp, (size_t)nsub * Qff * 256));
-        MMI_HIP_CHECK(hipMemsetAsync(yp, 0, (size_t)nsub * Qd * 256 * sizeof(float), init_stream));
-        MMI_HIP_CHECK(hipMemsetAsync(attp, 0, (size_t)nsub * Qd * 256 * sizeof(float), init_stream));
-        MMI_HIP_CHECK(hipMemsetAsync(hbp, 0, (size_t)nsub * Qff * 256 * sizeof(float), init_stream));
+        MMI_HIP_CHECK(mem.alloc(&yp, (size_t)nsub * Qd * 256));
+        MMI_HIP_CHECK(mem.alloc(&attp, (size_t)nsub * Qd * 256));
+        MMI_HIP_CHECK(mem.alloc(&hbp, (size_t)nsub * Qff * 256));
+        MMI_HIP_CHECK(mem.zero(yp, (size_t)nsub * Qd * 256, init_stream));
+        MMI_HIP_CHECK(mem.zero(attp, (size_t)nsub * Qd * 256, init_stream));
+        MMI_HIP_CHECK(mem.zero(hbp, (size_t)nsub * Qff * 256, init_stream));
     }
     const size_t kv_layer = (size_t)B * H * cap * Dh;
-    if (T > 2 || (Dh != 16 && Dh != 32 && Dh != 64))
+    if (T / frames > 2 || (Dh != 16 && Dh != 32 && Dh != 64))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: head dim 16/32/64 and 1 or 2 steps per frame are built");
     const size_t attn_smem = ((size_t)T * Dh + (((size_t)T * cap + 3) & ~(size_t)3) + (size_t)(256 / (Dh / 4)) * T * Dh + 8) * sizeof(float);
+    // one memory round trip when a thread's 16 row slots cover the ring (the Mimi shape: 250 slots of 64 floats)
+    const bool one_pass = cap <= 16 * (256 / (Dh / 4)) && !getenv("MMI_MIMI_ATTN_TWO_PASS");
+    // several frames at once: queries, keys and values row by row (the layers' keys and values until the ring takes them all at the end)
+    const size_t rows_d = (size_t)B * H * T * Dh;
+    float *qr = nullptr, *kvn = nullptr;
+    if (frames > 1) {
+        if (!packed || !one_pass) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: too many columns or a too long context for several frames at once");
+        MMI_HIP_CHECK(mem.alloc(&qr, rows_d));
+        MMI_HIP_CHECK(mem.alloc(&kvn, 2 * rows_d * layers.size()));
+    }
     auto add_norm = [&](const float* w, const float* bb) {
         const float* xp = xb.p; int xld = xb.ld; float* yn = y.p;
         prog.add([=](hipStream_t s) {
@@ -661,8 +796,8 @@ int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& 
     const bool fuse_ln = packed && d % 8 == 0 && Qd <= 64 && layers.size() > 0 && layers[0].n1w_pk;
     float* xrp = nullptr;
     if (fuse_ln) {
-        MMI_HIP_CHECK(m->st.alloc(&xrp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(hipMemsetAsync(xrp, 0, (size_t)nsub * Qd * 256 * sizeof(float), init_stream));
+        MMI_HIP_CHECK(mem.alloc(&xrp, (size_t)nsub * Qd * 256));
+        MMI_HIP_CHECK(mem.zero(xrp, (size_t)nsub * Qd * 256, init_stream));
     }
     bool x_is_packed = false;           // xrp holds the current residual stream
     for (size_t l = 0; l < layers.size(); ++l) {
@@ -675,16 +810,32 @@ int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& 
                 add_norm(L.n1w, L.n1b);
                 if (packed) { ai.x_packed = 1; ai.bp = yp; }
             }
-            if ((rc = add_conv(m, prog, ai))) return rc;
+            if ((rc = add_conv(mem, prog, ai))) return rc;
             MimiAttnArgs aa;
             aa.qkv = qkv.p; aa.kc = kv + (2 * l) * kv_layer; aa.vc = kv + (2 * l + 1) * kv_layer;
             aa.offsets = offsets; aa.out = att.p; aa.B = B; aa.H = H; aa.D = Dh; aa.T = T; aa.cap = cap;
             aa.context = c.tr_context; aa.max_period = c.tr_max_period;
             aa.outp = attp; aa.outQ = Qd;
-            // one memory round trip when a thread's 16 row slots cover the ring (the Mimi shape: 250 slots of 64 floats)
-            const bool one_pass = cap <= 16 * (256 / (Dh / 4)) && !getenv("MMI_MIMI_ATTN_TWO_PASS");
-            prog.add([=](hipStream_t s) {
-#define MMI_ATT(D_, T_) do { if (one_pass) MMI_LAUNCH((k_mimi_attn_1pass<D_, T_>), B * H, 256, 0, s, aa); \
+            if (frames > 1) {
+                MimiGroupRows gr;
+                gr.T = T; gr.qkv_ld = qkv.ld; gr.q = qr; gr.kn = kvn + 2 * l * rows_d; gr.vn = gr.kn + rows_d;
+                const int tpf = T / frames;
+                const dim3 grid_r(B * H, mmi_cdiv(T, 32)), grid_a(B * H, frames);
+                prog.add([=](hipStream_t s) {
+#define MMI_ATT(D_, T_) do { MMI_LAUNCH((k_mimi_group_rope<D_>), grid_r, 256, 0, s, aa, gr); \
+                             MMI_LAUNCH((k_mimi_attn_1pass<D_, T_, true>), grid_a, 256, 0, s, aa, gr); } while (0)
+                    if (Dh == 64 && tpf == 2) MMI_ATT(64, 2);
+                    else if (Dh == 64) MMI_ATT(64, 1);
+                    else if (Dh == 32 && tpf == 2) MMI_ATT(32, 2);
+                    else if (Dh == 32) MMI_ATT(32, 1);
+                    else if (tpf == 2) MMI_ATT(16, 2);
+                    else MMI_ATT(16, 1);
+#undef MMI_ATT
+                    MMI_CHECK_LAUNCH();
+                    return (int)MMI_OK;
+                });
+            } else prog.add([=](hipStream_t s) {
+#define MMI_ATT(D_, T_) do { if (one_pass) MMI_LAUNCH((k_mimi_attn_1pass<D_, T_>), B * H, 256, 0, s, aa, MimiGroupRows()); \
                              else MMI_LAUNCH((k_mimi_attn<D_, T_>), B * H, 256, attn_smem, s, aa); } while (0)
                 if (Dh == 64 && T == 2) MMI_ATT(64, 2);
                 else if (Dh == 64 && T == 1) MMI_ATT(64, 1);
@@ -701,7 +852,7 @@ int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& 
             a.res = xb.p; a.res_ld = xb.ld; a.res_off = off; a.scale = L.ls1;
             if (packed) { a.x_packed = 1; a.bp = attp; }
             if (fuse_ln) { a.outp = xrp; a.outQ = Qd; x_is_packed = true; }      // dual store: [B][C][T] and packed
-            if ((rc = add_conv(m, prog, a))) return rc;
+            if ((rc = add_conv(mem, prog, a))) return rc;
         }
         {   // x = x + ls2 * linear2(gelu(linear1(norm2(x))))
             ConvGemmArgs a1 = conv_args(L.lin1, y, 0, T, hb, 0, B, false);
@@ -713,33 +864,46 @@ int add_transformer(mmi_mimi* m, MmiProgram& prog, const std::vector<TrLayerW>& 
                 add_norm(L.n2w, L.n2b);
                 if (packed) { a1.x_packed = 1; a1.bp = yp; a1.out_mode = MMI_GOUT_PACKED; a1.outp = hbp; a1.outQ = Qff; }
             }
-            if ((rc = add_conv(m, prog, a1))) return rc;
+            if ((rc = add_conv(mem, prog, a1))) return rc;
             ConvGemmArgs a2 = conv_args(L.lin2, hb, 0, T, xb, off, B, false);
             a2.res = xb.p; a2.res_ld = xb.ld; a2.res_off = off; a2.scale = L.ls2;
             if (packed) { a2.x_packed = 1; a2.bp = hbp; }
             if (fuse_ln) { a2.outp = xrp; a2.outQ = Qd; x_is_packed = true; }
-            if ((rc = add_conv(m, prog, a2))) return rc;
+            if ((rc = add_conv(mem, prog, a2))) return rc;
         }
+    }
+    if (frames > 1) {
+        const int L = (int)layers.size();
+        const long n = (long)L * 2 * B * H * (T < cap ? T : cap) * (Dh / 4);
+        prog.add([=](hipStream_t s) {
+            MMI_LAUNCH(k_mimi_group_ring, (int)mmi_cdiv64(n, 256), 256, 0, s, (const float*)kvn, kv, offsets, L, B, H, T, cap, Dh);
+            MMI_CHECK_LAUNCH();
+            return (int)MMI_OK;
+        });
     }
     return MMI_OK;
 }
 
-int upload_hist(mmi_mimi* m, std::vector<HistDesc>& h, int B, HistDesc** dev, int* n, int* rows, HistTable* tab = nullptr) {
+// the table by value (n = -1: too many descriptors for it); returns the rows of all buffers
+int make_hist(std::vector<HistDesc>& h, int B, HistTable* tab) {
     int acc = 0;
-    std::vector<HistDesc> keep;
+    memset(tab, 0, sizeof(*tab));
     for (auto& d : h) {
         if (d.H <= 0) continue;
         d.row_begin = acc;
         acc += B * d.C;
-        keep.push_back(d);
+        if (tab->n >= 0 && tab->n < MMI_HIST_MAX) tab->d[tab->n++] = d;
+        else tab->n = -1;
     }
+    return acc;
+}
+
+int upload_hist(mmi_mimi* m, std::vector<HistDesc>& h, int B, HistDesc** dev, int* n, int* rows, HistTable* tab) {
+    *rows = make_hist(h, B, tab);
+    std::vector<HistDesc> keep;
+    for (auto& d : h)
+        if (d.H > 0) keep.push_back(d);
     *n = (int)keep.size();
-    *rows = acc;
-    if (tab) {                                   // by-value copy for k_commit_all (n = -1: too many descriptors, two-launch path)
-        memset(tab, 0, sizeof(*tab));
-        tab->n = keep.size() <= MMI_HIST_MAX ? (int)keep.size() : -1;
-        for (size_t i = 0; i < keep.size() && i < MMI_HIST_MAX; ++i) tab->d[i] = keep[i];
-    }
     MMI_HIP_CHECK(m->st.alloc(dev, keep.size() ? keep.size() : 1));
     if (!keep.empty())
         MMI_HIP_CHECK(hipMemcpy(*dev, keep.data(), keep.size() * sizeof(HistDesc), hipMemcpyHostToDevice));
@@ -752,26 +916,58 @@ HistDesc hist_of(const Buf& b, int T) {
     return d;
 }
 
-int build_encoder(mmi_mimi* m, int B, hipStream_t s0) {
+// the end of a program: histories shifted, transformer offsets advanced, replicate flags cleared
+int add_commit(mmi_mimi* m, MmiProgram& prog, std::vector<HistDesc>& hist, int B, const MimiGroup* g, HistDesc** dev, int* n, int* n_rows, HistTable* tab,
+               long* counters, int inc, uint8_t* first) {
+    int rc, rows;
+    if (g) {
+        rows = make_hist(hist, B, tab);
+        if (tab->n < 0) return mmi_fail(MMI_ERR_UNSUPPORTED, "too many histories for several frames at once");
+    } else {
+        if ((rc = upload_hist(m, hist, B, dev, n, n_rows, tab))) return rc;
+        rows = *n_rows;
+    }
+    const HistDesc* hd = *dev;
+    const int nh = *n;
+    const HistTable t = *tab;
+    const uint8_t* ex = m->exec;
+    const bool one = t.n >= 0 && (g || !getenv("MMI_MIMI_TWO_COMMITS"));
+    prog.add([=](hipStream_t s) {
+        if (one) {
+            MMI_LAUNCH(k_commit_all, mmi_cdiv(rows + B, 256), 256, 0, s, t, rows, ex, counters, 1, inc, first, B);
+            MMI_CHECK_LAUNCH();
+            return (int)MMI_OK;
+        }
+        if (rows > 0) MMI_LAUNCH(k_commit_history, mmi_cdiv(rows, 256), 256, 0, s, hd, nh, rows, ex);
+        MMI_LAUNCH(k_commit_counters, mmi_cdiv(B, 64), 64, 0, s, counters, 1, inc, first, ex, B);
+        MMI_CHECK_LAUNCH();
+        return (int)MMI_OK;
+    });
+    return MMI_OK;
+}
+
+// g: null for the frame program, whose buffers and state are the stream's; otherwise `frames` frames at once in the group's own buffers
+int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hipStream_t s0) {
     const mmi_mimi_cfg& c = m->cfg;
-    MmiProgram& prog = m->enc_prog;
+    MmiProgram& prog = g ? g->prog : m->enc_prog;
+    Buf &ein = g ? g->in : m->enc_in, &lat = g ? g->out : m->latent;
     std::vector<HistDesc> hist;
     int rc;
-    int T = c.frame_size;
+    int T = c.frame_size * frames;
     size_t ci = 0;
     // input PCM buffer with the first conv's history
-    if ((rc = alloc_buf(m, B, c.channels, c.kernel_size - 1, T, &m->enc_in, s0))) return rc;
-    hist.push_back(hist_of(m->enc_in, T));
-    Buf cur = m->enc_in;
+    if ((rc = alloc_buf(mem, B, c.channels, c.kernel_size - 1, T, &ein, s0))) return rc;
+    hist.push_back(hist_of(ein, T));
+    Buf cur = ein;
     int mult = 1;
     // ELU hoisted into the producers (mimi_kernels.h ConvGemmArgs::elu_out / out2): a resblock input is kept raw (residual) AND
     // ELU'd (its first conv reads that, history included); everything else a conv reads through ELU is stored ELU'd only
     {   // conv0: channels -> n_filters, K = kernel_size; consumer = resblock conv (K = residual_kernel_size)
         Buf nxt;
-        if ((rc = alloc_buf(m, B, c.n_filters, c.residual_kernel_size - 1, T, &nxt, s0))) return rc;
-        if ((rc = alloc_twin(m, B, &nxt, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, c.n_filters, c.residual_kernel_size - 1, T, &nxt, s0))) return rc;
+        if ((rc = alloc_twin(mem, B, &nxt, s0))) return rc;
         prog.site("enc.conv0");
-        if ((rc = add_conv(m, prog, conv_args(m->enc_convs[ci++], cur, 0, T, nxt, nxt.H, B, false)))) return rc;
+        if ((rc = add_conv(mem, prog, conv_args(m->enc_convs[ci++], cur, 0, T, nxt, nxt.H, B, false)))) return rc;
         hist.push_back(hist_of_src(nxt, T));
         cur = nxt;
     }
@@ -780,26 +976,26 @@ int build_encoder(mmi_mimi* m, int B, hipStream_t s0) {
         const int ch = mult * c.n_filters;
         // resblock: cur -> (ELU, conv K3 -> hidden) -> (ELU, conv K1 -> ch) + cur ; consumer = strided conv (K=2r, S=r)
         Buf hid, nxt;
-        if ((rc = alloc_buf(m, B, ch / c.compress, 0, T, &hid, s0))) return rc;
-        if ((rc = alloc_buf(m, B, ch, ratio, T, &nxt, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, ch / c.compress, 0, T, &hid, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, ch, ratio, T, &nxt, s0))) return rc;
         hid.elu = nxt.elu = true;               // read only by the block's second conv / the strided conv, both behind an ELU
         prog.site("enc.res" + std::to_string(i));
         const ConvGemmArgs a1 = conv_args(m->enc_convs[ci++], cur, 0, T, hid, 0, B, true);
         const ConvW& w2 = m->enc_convs[ci++];
         ConvGemmArgs a = conv_args(w2, hid, 0, T, nxt, nxt.H, B, true);
         a.res = cur.p; a.res_ld = cur.ld; a.res_off = cur.H;
-        if ((rc = add_resblock(m, prog, a1, a, w2))) return rc;
+        if ((rc = add_resblock(mem, prog, a1, a, w2))) return rc;
         hist.push_back(hist_of(nxt, T));
         cur = nxt;
         // strided conv: ch -> 2ch ; consumer = next resblock conv (K3) or the final conv (last_kernel_size)
         const int Tn = T / ratio;
         const int Hn = (i + 1 < c.n_ratios) ? c.residual_kernel_size - 1 : c.last_kernel_size - 1;
         Buf nx2;
-        if ((rc = alloc_buf(m, B, 2 * ch, Hn, Tn, &nx2, s0))) return rc;
-        if (i + 1 < c.n_ratios) { if ((rc = alloc_twin(m, B, &nx2, s0))) return rc; }   // the next resblock's input
+        if ((rc = alloc_buf(mem, B, 2 * ch, Hn, Tn, &nx2, s0))) return rc;
+        if (i + 1 < c.n_ratios) { if ((rc = alloc_twin(mem, B, &nx2, s0))) return rc; }   // the next resblock's input
         else nx2.elu = true;                                                                     // read by the final conv only
         prog.site("enc.down" + std::to_string(i));
-        if ((rc = add_conv(m, prog, conv_args(m->enc_convs[ci++], cur, 0, Tn, nx2, nx2.H, B, true)))) return rc;
+        if ((rc = add_conv(mem, prog, conv_args(m->enc_convs[ci++], cur, 0, Tn, nx2, nx2.H, B, true)))) return rc;
         hist.push_back(hist_of_src(nx2, Tn));
         cur = nx2;
         T = Tn;
@@ -808,84 +1004,99 @@ int build_encoder(mmi_mimi* m, int B, hipStream_t s0) {
     // final conv -> dimension, written into the downsample conv's input buffer (history = stride)
     const int stride = c.resample_stride;
     Buf dsin;
-    if ((rc = alloc_buf(m, B, c.dimension, 2 * stride - stride, T, &dsin, s0))) return rc;
+    if ((rc = alloc_buf(mem, B, c.dimension, 2 * stride - stride, T, &dsin, s0))) return rc;
     prog.site("enc.final");
-    if ((rc = add_conv(m, prog, conv_args(m->enc_convs[ci++], cur, 0, T, dsin, dsin.H, B, true)))) return rc;
+    if ((rc = add_conv(mem, prog, conv_args(m->enc_convs[ci++], cur, 0, T, dsin, dsin.H, B, true)))) return rc;
     hist.push_back(hist_of(dsin, T));
     // encoder transformer, in place on dsin[:, :, H:H+T]
     {
         const int Dh = c.tr_d_model / c.tr_num_heads;
         size_t kvn = (size_t)2 * c.tr_num_layers * B * c.tr_num_heads * c.tr_context * Dh;
-        MMI_HIP_CHECK(m->st.alloc(&m->enc_kv, kvn));
-        MMI_HIP_CHECK(hipMemsetAsync(m->enc_kv, 0, kvn * sizeof(float), s0));
+        if (!g) {
+            MMI_HIP_CHECK(m->st.alloc(&m->enc_kv, kvn));
+            MMI_HIP_CHECK(hipMemsetAsync(m->enc_kv, 0, kvn * sizeof(float), s0));
+        }
         prog.site("enc.tr");
-        if ((rc = add_transformer(m, prog, m->enc_tr, dsin, dsin.H, T, m->enc_kv, m->counters, B, s0))) return rc;
+        if ((rc = add_transformer(m, mem, prog, m->enc_tr, dsin, dsin.H, T, m->enc_kv, m->counters, B, frames, s0))) return rc;
     }
     const int T_tr = T;
     // downsample (ConvDownsample1d learnt, replicate padding on the first frame)
-    if (T % stride != 0 || T / stride != 1)
+    if (T % stride != 0 || T / stride != frames)
         return mmi_fail(MMI_ERR_UNSUPPORTED, "frame_size must map to exactly one latent column");
-    if ((rc = alloc_buf(m, B, c.dimension, 0, 1, &m->latent, s0))) return rc;
-    const bool latent_packed = B <= 128 && m->q_in.Q * 8 == c.dimension && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    if ((rc = alloc_buf(mem, B, c.dimension, 0, frames, &lat, s0))) return rc;
+    const bool latent_packed = B * frames <= 128 && m->q_in.Q * 8 == c.dimension && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    if (g && !latent_packed) return mmi_fail(MMI_ERR_UNSUPPORTED, "quantising several frames needs the packed operand");
+    RvqScratch rs = m->rvq;
+    if (g) {
+        const size_t n = (size_t)B * frames;
+        rs.rows = (int)n;
+        MMI_HIP_CHECK(mem.alloc(&rs.xq, n * 2 * c.q_dimension));
+        MMI_HIP_CHECK(mem.alloc(&rs.best_d, 2 * m->nchunk * n));
+        MMI_HIP_CHECK(mem.alloc(&rs.best_i, 2 * m->nchunk * n));
+        MMI_HIP_CHECK(mem.alloc(&rs.codes, n * c.q_n_q));
+        MMI_HIP_CHECK(mem.alloc(&rs.qin_bp, (size_t)mmi_cdiv((int)n, 32) * m->q_in.Q * 256));
+        MMI_HIP_CHECK(mem.alloc(&rs.qin_part, (size_t)8 * m->q_in.Mt * 32 * 128));
+        g->codes = rs.codes;
+    }
     {
-        ConvGemmArgs a = conv_args(m->downsample, dsin, 0, 1, m->latent, 0, B, false);
+        ConvGemmArgs a = conv_args(m->downsample, dsin, 0, frames, lat, 0, B, false);
         a.first = m->first; a.exec = m->exec;
-        if (latent_packed) { a.outp = m->qin_bp; a.outQ = m->q_in.Q; }   // the latent, also as the RVQ input projection's operand
+        if (latent_packed) { a.outp = rs.qin_bp; a.outQ = m->q_in.Q; }   // the latent, also as the RVQ input projection's operand
         prog.site("enc.downsample");
-        if ((rc = add_conv(m, prog, a))) return rc;
+        if ((rc = add_conv(mem, prog, a))) return rc;
     }
     prog.site("enc.rvq");
-    if ((rc = add_quantize_ops(m, prog, m->latent.p, 1, 0, B, latent_packed))) return rc;
+    if ((rc = add_quantize_ops(m, mem, rs, prog, lat.p, 1, 0, B * frames, latent_packed))) return rc;
     prog.site("enc.commit");
     // commit
-    HistTable tab;
-    if ((rc = upload_hist(m, hist, B, &m->enc_hist, &m->enc_nhist, &m->enc_hist_rows, &tab))) return rc;
-    {
-        HistDesc* hd = m->enc_hist; int nh = m->enc_nhist, rows = m->enc_hist_rows;
-        const uint8_t* ex = m->exec; uint8_t* fi = m->first; long* cnt = m->counters;
-        const bool one = tab.n >= 0 && !getenv("MMI_MIMI_TWO_COMMITS");
-        prog.add([=](hipStream_t s) {
-            if (one) {
-                MMI_LAUNCH(k_commit_all, mmi_cdiv(rows + B, 256), 256, 0, s, tab, rows, ex, cnt, 1, T_tr, fi, B);
-                MMI_CHECK_LAUNCH();
-                return (int)MMI_OK;
-            }
-            if (rows > 0) MMI_LAUNCH(k_commit_history, mmi_cdiv(rows, 256), 256, 0, s, (const HistDesc*)hd, nh, rows, ex);
-            MMI_LAUNCH(k_commit_counters, mmi_cdiv(B, 64), 64, 0, s, cnt, 1, T_tr, fi, ex, B);
-            MMI_CHECK_LAUNCH();
-            return (int)MMI_OK;
-        });
-    }
-    return MMI_OK;
+    return add_commit(m, prog, hist, B, g, &m->enc_hist, &m->enc_nhist, &m->enc_hist_rows, g ? &g->hist : &m->enc_tab, m->counters, T_tr, m->first);
 }
 
-int build_decoder(mmi_mimi* m, int B, hipStream_t s0) {
+int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hipStream_t s0) {
     const mmi_mimi_cfg& c = m->cfg;
-    MmiProgram& prog = m->dec_prog;
+    MmiProgram& prog = g ? g->prog : m->dec_prog;
+    Buf &lat = g ? g->in : m->dec_codes_lat, &pcm = g ? g->out : m->dec_out;
     std::vector<HistDesc> hist;
     int rc;
     const int stride = c.resample_stride;
-    // dequantised latent [B][dim][1]
-    if ((rc = alloc_buf(m, B, c.dimension, 0, 1, &m->dec_codes_lat, s0))) return rc;
+    size_t np = 0;                                        // the transposed convs' partial sums: the frame program's, in order
+    auto partial = [&](long pn, float** out) -> hipError_t {
+        if (!g) {
+            hipError_t e = m->st.alloc(out, (size_t)B * pn);
+            if (e == hipSuccess) e = hipMemsetAsync(*out, 0, (size_t)B * pn * sizeof(float), s0);
+            if (e != hipSuccess) return e;
+            m->partials.push_back(*out); m->partial_sizes.push_back(pn);
+        }
+        *out = m->partials[np++];
+        return hipSuccess;
+    };
+    // dequantised latents [B][dim][frames]
+    if ((rc = alloc_buf(mem, B, c.dimension, 0, frames, &lat, s0))) return rc;
     prog.site("dec.dequant");
-    if ((rc = add_dequant_ops(m, prog, m->n_codebooks, m->dec_codes_lat, 0, B, /*k_from_device=*/true))) return rc;
+    DequantScratch ds = m->deq;
+    if (g) {
+        const size_t n = (size_t)B * frames;
+        MMI_HIP_CHECK(mem.alloc(&ds.codes, n * c.q_n_q));
+        MMI_HIP_CHECK(mem.alloc(&ds.q2, n * 2 * c.q_dimension));
+        MMI_HIP_CHECK(mem.alloc(&ds.qout_bp, (size_t)mmi_cdiv((int)n, 32) * m->q_out.Q * 256));
+        MMI_HIP_CHECK(mem.alloc(&ds.qout_part, (size_t)8 * m->q_out.Mt * 32 * 128));
+        g->codes = ds.codes;
+    }
+    if ((rc = add_dequant_ops(m, mem, ds, prog, m->n_codebooks, lat, 0, B, frames, /*k_from_device=*/true))) return rc;
     prog.site("dec.upsample");
     // upsample (depthwise transposed conv) into the decoder transformer buffer = input of decoder conv0
-    int T = stride;
+    int T = stride * frames;
     Buf din;
-    if ((rc = alloc_buf(m, B, c.dimension, c.kernel_size - 1, T, &din, s0))) return rc;
+    if ((rc = alloc_buf(mem, B, c.dimension, c.kernel_size - 1, T, &din, s0))) return rc;
     hist.push_back(hist_of(din, T));
     {
         float* part = nullptr;
-        long pn = (long)c.dimension * stride;
-        MMI_HIP_CHECK(m->st.alloc(&part, (size_t)B * pn));
-        MMI_HIP_CHECK(hipMemsetAsync(part, 0, (size_t)B * pn * sizeof(float), s0));
-        m->partials.push_back(part); m->partial_sizes.push_back(pn);
-        const float* x = m->dec_codes_lat.p; const float* w = m->upsample_w; const uint8_t* ex = m->exec;
-        float* out = din.p; int old = din.ld, ooff = din.H; int C = c.dimension;
+        MMI_HIP_CHECK(partial((long)c.dimension * stride, &part));
+        const float* x = lat.p; const float* w = m->upsample_w; const uint8_t* ex = m->exec;
+        float* out = din.p; int old = din.ld, ooff = din.H; int C = c.dimension; const int xld = lat.ld;
         prog.add([=](hipStream_t s) {
-            MMI_LAUNCH(k_upsample_dw, mmi_cdiv(B * C * stride, 256), 256, 0, s, x, 1, 0, w, part, ex, out, old, ooff, B, C,
-                       2 * stride, stride, 1);
+            MMI_LAUNCH(k_upsample_dw, mmi_cdiv(B * C * stride * frames, 256), 256, 0, s, x, xld, 0, w, part, ex, out, old, ooff, B, C,
+                       2 * stride, stride, frames);
             MMI_CHECK_LAUNCH();
             return (int)MMI_OK;
         });
@@ -893,10 +1104,12 @@ int build_decoder(mmi_mimi* m, int B, hipStream_t s0) {
     {
         const int Dh = c.tr_d_model / c.tr_num_heads;
         size_t kvn = (size_t)2 * c.tr_num_layers * B * c.tr_num_heads * c.tr_context * Dh;
-        MMI_HIP_CHECK(m->st.alloc(&m->dec_kv, kvn));
-        MMI_HIP_CHECK(hipMemsetAsync(m->dec_kv, 0, kvn * sizeof(float), s0));
+        if (!g) {
+            MMI_HIP_CHECK(m->st.alloc(&m->dec_kv, kvn));
+            MMI_HIP_CHECK(hipMemsetAsync(m->dec_kv, 0, kvn * sizeof(float), s0));
+        }
         prog.site("dec.tr");
-        if ((rc = add_transformer(m, prog, m->dec_tr, din, din.H, T, m->dec_kv, m->counters + B, B, s0))) return rc;
+        if ((rc = add_transformer(m, mem, prog, m->dec_tr, din, din.H, T, m->dec_kv, m->counters + B, B, frames, s0))) return rc;
     }
     const int T_tr = T;
     size_t ci = 0;
@@ -904,47 +1117,44 @@ int build_decoder(mmi_mimi* m, int B, hipStream_t s0) {
     Buf cur;
     float* conv0_bp = nullptr;                            // dec.conv0's output in the packed operand order of dec.convtr0's GEMM
     {   // conv0: dimension -> mult*n_filters (no activation before it); consumer = conv-transpose GEMM (no history)
-        if ((rc = alloc_buf(m, B, mult * c.n_filters, 0, T, &cur, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, mult * c.n_filters, 0, T, &cur, s0))) return rc;
         cur.elu = true;
         prog.site("dec.conv0");
         ConvGemmArgs a0 = conv_args(m->dec_convs[ci++], din, 0, T, cur, 0, B, false);
         // its (ELU'd) output is read by the first transposed-conv GEMM only: stored as that GEMM's packed operand as well
         const ConvW& wtr0 = m->dec_convs[ci];
         if (B * T <= 128 && wtr0.Q * 8 == mult * c.n_filters && !getenv("MMI_MIMI_PACK_LAUNCHES")) {
-            MMI_HIP_CHECK(m->st.alloc(&conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256));
-            MMI_HIP_CHECK(hipMemsetAsync(conv0_bp, 0, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256 * sizeof(float), s0));
+            MMI_HIP_CHECK(mem.alloc(&conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256));
+            MMI_HIP_CHECK(mem.zero(conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256, s0));
             a0.outp = conv0_bp; a0.outQ = wtr0.Q;
         }
-        if ((rc = add_conv(m, prog, a0))) return rc;
+        if ((rc = add_conv(mem, prog, a0))) return rc;
     }
     for (int i = 0; i < c.n_ratios; ++i) {
         const int ratio = c.ratios[i];
         const int cin = mult * c.n_filters, cout = cin / 2, K = 2 * ratio;
         // ELU + ConvTranspose1d: GEMM over channels, then overlap-add with the streaming partial
         Buf tmp, up;
-        if ((rc = alloc_buf(m, B, cout * K, 0, T, &tmp, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, cout * K, 0, T, &tmp, s0))) return rc;
         const int Tn = T * ratio;
-        if ((rc = alloc_buf(m, B, cout, c.residual_kernel_size - 1, Tn, &up, s0))) return rc;
-        if ((rc = alloc_twin(m, B, &up, s0))) return rc;           // resblock input: raw for the residual, ELU'd for its conv
+        if ((rc = alloc_buf(mem, B, cout, c.residual_kernel_size - 1, Tn, &up, s0))) return rc;
+        if ((rc = alloc_twin(mem, B, &up, s0))) return rc;           // resblock input: raw for the residual, ELU'd for its conv
         const ConvW& wtr = m->dec_convs[ci++];
         prog.site("dec.convtr" + std::to_string(i));
         {
             ConvGemmArgs a = conv_args(wtr, cur, 0, T, tmp, 0, B, true);
             a.bias = nullptr;  // bias is added once, in the combine step
             if (i == 0 && conv0_bp) { a.bp = conv0_bp; a.x_packed = 1; }
-            if ((rc = add_conv(m, prog, a))) return rc;
+            if ((rc = add_conv(mem, prog, a))) return rc;
         }
         {
             float* part = nullptr;
-            long pn = (long)cout * (K - ratio);
-            MMI_HIP_CHECK(m->st.alloc(&part, (size_t)B * pn));
-            MMI_HIP_CHECK(hipMemsetAsync(part, 0, (size_t)B * pn * sizeof(float), s0));
-            m->partials.push_back(part); m->partial_sizes.push_back(pn);
+            MMI_HIP_CHECK(partial((long)cout * (K - ratio), &part));
             const float* tp = tmp.p; const float* bias = wtr.bias; const uint8_t* ex = m->exec;
             float* out = up.p; float* out2 = up.pe; int old = up.ld, ooff = up.H; int Tin = T; const int tld = tmp.ld;
             prog.add([=](hipStream_t s) {
                 MMI_LAUNCH(k_convtr_combine, (int)mmi_cdiv64((int64_t)B * cout * Tin * ratio, 256), 256, 0, s, tp, bias, part,
-                           ex, out, old, ooff, B, cout, K, ratio, Tin, out2, tld);
+                           ex, out, old, ooff, B, cout, K, ratio, Tin, out2, tld, Tin / frames);
                 MMI_CHECK_LAUNCH();
                 return (int)MMI_OK;
             });
@@ -954,43 +1164,84 @@ int build_decoder(mmi_mimi* m, int B, hipStream_t s0) {
         // resblock; consumer = next conv-transpose GEMM (no history) or the final conv (last_kernel_size)
         Buf hid, nxt;
         const int Hn = (i + 1 < c.n_ratios) ? 0 : c.last_kernel_size - 1;
-        if ((rc = alloc_buf(m, B, cout / c.compress, 0, T, &hid, s0))) return rc;
-        if ((rc = alloc_buf(m, B, cout, Hn, T, &nxt, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, cout / c.compress, 0, T, &hid, s0))) return rc;
+        if ((rc = alloc_buf(mem, B, cout, Hn, T, &nxt, s0))) return rc;
         hid.elu = nxt.elu = true;               // read only behind an ELU: by the block's second conv / the next layer
         prog.site("dec.res" + std::to_string(i));
         const ConvGemmArgs a1 = conv_args(m->dec_convs[ci++], up, 0, T, hid, 0, B, true);
         const ConvW& w2 = m->dec_convs[ci++];
         ConvGemmArgs a = conv_args(w2, hid, 0, T, nxt, nxt.H, B, true);
         a.res = up.p; a.res_ld = up.ld; a.res_off = up.H;
-        if ((rc = add_resblock(m, prog, a1, a, w2))) return rc;
+        if ((rc = add_resblock(mem, prog, a1, a, w2))) return rc;
         if (Hn > 0) hist.push_back(hist_of(nxt, T));
         cur = nxt;
         mult /= 2;
     }
-    if (T != c.frame_size) return mmi_fail(MMI_ERR_UNSUPPORTED, "decoder does not reproduce frame_size samples");
-    if ((rc = alloc_buf(m, B, c.channels, 0, T, &m->dec_out, s0))) return rc;
+    if (T != c.frame_size * frames) return mmi_fail(MMI_ERR_UNSUPPORTED, "decoder does not reproduce frame_size samples");
+    if ((rc = alloc_buf(mem, B, c.channels, 0, T, &pcm, s0))) return rc;
     prog.site("dec.final");
-    if ((rc = add_conv(m, prog, conv_args(m->dec_convs[ci++], cur, 0, T, m->dec_out, 0, B, true)))) return rc;
+    if ((rc = add_conv(mem, prog, conv_args(m->dec_convs[ci++], cur, 0, T, pcm, 0, B, true)))) return rc;
     prog.site("dec.commit");
-    HistTable tab;
-    if ((rc = upload_hist(m, hist, B, &m->dec_hist, &m->dec_nhist, &m->dec_hist_rows, &tab))) return rc;
-    {
-        HistDesc* hd = m->dec_hist; int nh = m->dec_nhist, rows = m->dec_hist_rows;
-        const uint8_t* ex = m->exec; long* cnt = m->counters + B;
-        const bool one = tab.n >= 0 && !getenv("MMI_MIMI_TWO_COMMITS");
-        prog.add([=](hipStream_t s) {
-            if (one) {
-                MMI_LAUNCH(k_commit_all, mmi_cdiv(rows + B, 256), 256, 0, s, tab, rows, ex, cnt, 1, T_tr, (uint8_t*)nullptr, B);
-                MMI_CHECK_LAUNCH();
-                return (int)MMI_OK;
-            }
-            if (rows > 0) MMI_LAUNCH(k_commit_history, mmi_cdiv(rows, 256), 256, 0, s, (const HistDesc*)hd, nh, rows, ex);
-            MMI_LAUNCH(k_commit_counters, mmi_cdiv(B, 64), 64, 0, s, cnt, 1, T_tr, (uint8_t*)nullptr, ex, B);
-            MMI_CHECK_LAUNCH();
-            return (int)MMI_OK;
-        });
+    return add_commit(m, prog, hist, B, g, &m->dec_hist, &m->dec_nhist, &m->dec_hist_rows, g ? &g->hist : &m->dec_tab, m->counters + B, T_tr, nullptr);
+}
+
+// ---- groups of frames ---------------------------------------------------------------------------
+// Frames of the next group when `left` frames are to be run (1: frame by frame).  A group takes as many columns as the 25 Hz layers'
+// weight-streaming GEMMs hold (128, as for 64 streams), and what is left is cut into equal groups.  Not while the caller's stream is being
+// captured (a group's launch list is not kept for ever), and not under an exec mask (its rows would have to stand still frame by frame).
+int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left, hipStream_t s) {
+    const mmi_mimi_cfg& c = m->cfg;
+    int most = left;
+    if (const char* e = getenv("MMI_MIMI_GROUP")) most = atoi(e);         // test hook: the largest group
+    if (left < 2 || most < 2 || g.refused || !m->all_exec || tab.n < 0 || getenv("MMI_MIMI_PACK_LAUNCHES")) return 1;
+    const int tpf = c.resample_stride, B = m->batch;
+    most = std::min(most, std::min(128 / (B * tpf), ((1 << 17) - 1) / (B * c.frame_size)));
+    if (most < 2) return 1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 1;
+    return left / mmi_cdiv(left, most);
+}
+
+// the program of `frames` frames, ready to run on s; MMI_ERR_UNSUPPORTED / MMI_ERR_HIP: go frame by frame
+int ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
+    MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
+    if (g.frames == frames) return MMI_OK;
+    g.frames = 0;
+    g.prog.clear();
+    g.slab.rewind();
+    g.tab.clear();
+    size_t cap = 0;
+    for (const ConvW& w : enc ? m->enc_convs : m->dec_convs) cap += (size_t)w.Q * 8;
+    MimiMem mem;
+    mem.slab = &g.slab;
+    mem.frames = frames;
+    mem.tab_host = &g.tab;
+    MMI_HIP_CHECK(g.slab.alloc((void**)&mem.tab_dev, cap * sizeof(int)));
+    int rc = enc ? build_encoder(m, m->batch, frames, mem, &g, s) : build_decoder(m, m->batch, frames, mem, &g, s);
+    if (rc) return rc;
+    if (g.tab.size() > cap) return mmi_fail(MMI_ERR_UNSUPPORTED, "offset tables of a group");
+    if (!g.tab.empty() && (g.tab_B != m->batch || g.tab_frames != frames)) {
+        g.tab_frames = 0;
+        MMI_HIP_CHECK(hipMemcpyAsync(mem.tab_dev, g.tab.data(), g.tab.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        g.tab_B = m->batch;
+        g.tab_frames = frames;
     }
+    g.frames = frames;
     return MMI_OK;
+}
+
+// The group's launches, and behind them on the host - while the GPU works on them - the capture of the frame program, so that a stream's
+// first single frame after a call of several does not wait for it.
+int run_group(mmi_mimi* m, bool enc, hipStream_t s) {
+    MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
+    const HistTable& st = enc ? m->enc_tab : m->dec_tab;
+    const int rows = enc ? m->enc_hist_rows : m->dec_hist_rows;
+    MMI_LAUNCH(k_move_history, mmi_cdiv(rows, 256), 256, 0, s, st, g.hist, rows);
+    int rc = g.prog.run_eager(s);
+    if (rc) return rc;
+    MMI_LAUNCH(k_move_history, mmi_cdiv(rows, 256), 256, 0, s, g.hist, st, rows);
+    MMI_CHECK_LAUNCH();
+    return m->use_graph ? (enc ? m->enc_prog : m->dec_prog).capture_full(m->cap_stream) : MMI_OK;
 }
 
 int check_cfg(const mmi_mimi_cfg& c) {
@@ -1102,17 +1353,17 @@ extern "C" int mmi_mimi_create(const mmi_mimi_cfg* cfg, const mmi_tensor_desc* w
     if ((rc = load_rvq(m, W))) return fail(rc);
     // ---- RVQ scratch
     m->nchunk = mmi_cdiv(c.q_bins, MMI_RVQ_CHUNK);
-    if (hipSuccess != m->wts.alloc(&m->xq, (size_t)max_batch * 2 * c.q_dimension) ||
-        hipSuccess != m->wts.alloc(&m->best_d, (size_t)2 * m->nchunk * max_batch) ||
-        hipSuccess != m->wts.alloc(&m->best_i, (size_t)2 * m->nchunk * max_batch) ||
-        hipSuccess != m->wts.alloc(&m->codes_i32, (size_t)max_batch * c.q_n_q) ||
-        hipSuccess != m->wts.alloc(&m->dec_codes_i32, (size_t)max_batch * c.q_n_q) ||
-        hipSuccess != m->wts.alloc(&m->q2, (size_t)max_batch * 2 * c.q_dimension) ||
-        hipSuccess != m->wts.alloc(&m->lat_tmp, (size_t)max_batch * c.dimension) ||
-        hipSuccess != m->wts.alloc(&m->qin_bp, (size_t)mmi_cdiv(max_batch, 32) * m->q_in.Q * 256) ||
-        hipSuccess != m->wts.alloc(&m->qout_bp, (size_t)mmi_cdiv(max_batch, 32) * m->q_out.Q * 256) ||
-        hipSuccess != m->wts.alloc(&m->qin_part, (size_t)8 * m->q_in.Mt * 32 * 128) ||
-        hipSuccess != m->wts.alloc(&m->qout_part, (size_t)8 * m->q_out.Mt * 32 * 128))
+    m->rvq.rows = max_batch;
+    if (hipSuccess != m->wts.alloc(&m->rvq.xq, (size_t)max_batch * 2 * c.q_dimension) ||
+        hipSuccess != m->wts.alloc(&m->rvq.best_d, (size_t)2 * m->nchunk * max_batch) ||
+        hipSuccess != m->wts.alloc(&m->rvq.best_i, (size_t)2 * m->nchunk * max_batch) ||
+        hipSuccess != m->wts.alloc(&m->rvq.codes, (size_t)max_batch * c.q_n_q) ||
+        hipSuccess != m->wts.alloc(&m->deq.codes, (size_t)max_batch * c.q_n_q) ||
+        hipSuccess != m->wts.alloc(&m->deq.q2, (size_t)max_batch * 2 * c.q_dimension) ||
+        hipSuccess != m->wts.alloc(&m->rvq.qin_bp, (size_t)mmi_cdiv(max_batch, 32) * m->q_in.Q * 256) ||
+        hipSuccess != m->wts.alloc(&m->deq.qout_bp, (size_t)mmi_cdiv(max_batch, 32) * m->q_out.Q * 256) ||
+        hipSuccess != m->wts.alloc(&m->rvq.qin_part, (size_t)8 * m->q_in.Mt * 32 * 128) ||
+        hipSuccess != m->wts.alloc(&m->deq.qout_part, (size_t)8 * m->q_out.Mt * 32 * 128))
         return fail(mmi_fail(MMI_ERR_HIP, "out of device memory (RVQ scratch)"));
     if (hipDeviceSynchronize() != hipSuccess) return fail(mmi_fail(MMI_ERR_HIP, "weight packing failed"));
     if (m->use_graph && hipStreamCreate(&m->cap_stream) != hipSuccess)
@@ -1125,6 +1376,8 @@ extern "C" void mmi_mimi_destroy(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return;
     mmi_mimi_streaming_stop(m);
+    m->enc_grp.slab.release();
+    m->dec_grp.slab.release();
     m->wts.release();
     if (m->cap_stream) hipStreamDestroy(m->cap_stream);
     delete m;
@@ -1148,7 +1401,8 @@ extern "C" int64_t mmi_mimi_launch_list(const mmi_mimi* m, int32_t which, char* 
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m || !m->streaming) return 0;
     const MmiProgram& p = which == 0 ? m->enc_prog : m->dec_prog;
-    if (!p.logged()) return 0;
+    const MmiProgram& g = which == 0 ? m->enc_grp.prog : m->dec_grp.prog;
+    if (!p.logged()) return g.logged() ? mmi_copy_launch_log(g.launch_log(), buf, cap) : 0;      // (frames have only been run in groups so far)
     return mmi_copy_launch_log(p.launch_log(), buf, cap);
 }
 
@@ -1178,8 +1432,11 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
         hipMemsetAsync(m->counters, 0, (size_t)2 * batch * sizeof(long), s) != hipSuccess ||
         hipMemcpyAsync(m->dec_k_dev, &m->dec_k_host, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess)
         return fail(mmi_fail(MMI_ERR_HIP, "initialising the streaming state failed"));
-    if ((rc = build_encoder(m, batch, s))) return fail(rc);
-    if ((rc = build_decoder(m, batch, s))) return fail(rc);
+    MimiMem mem;
+    mem.arena = &m->st;
+    if ((rc = build_encoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
+    if ((rc = build_decoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
+    m->all_exec = true;
     if (hipStreamSynchronize(s) != hipSuccess) return fail(mmi_fail(MMI_ERR_HIP, "hipStreamSynchronize failed"));
     m->streaming = true;
     return MMI_OK;
@@ -1192,6 +1449,11 @@ extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
     hipDeviceSynchronize();
     m->enc_prog.clear();
     m->dec_prog.clear();
+    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {      // their launches name the state that goes now; the slabs stay
+        g->prog.clear();
+        g->frames = 0;
+        g->refused = false;
+    }
     m->st.release();
     m->partials.clear();
     m->partial_sizes.clear();
@@ -1219,6 +1481,7 @@ extern "C" int mmi_mimi_state_load(mmi_mimi* m, const void* src, int64_t bytes, 
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
     if (bytes != (int64_t)m->st.bytes) return mmi_fail(MMI_ERR_SHAPE, "snapshot taken from a different stream (batch)");
     MMI_HIP_CHECK(m->st.load(src, (hipStream_t)stream));
+    m->all_exec = false;      // the snapshot carries its own mask
     m->dec_k_cur = -1;        // the snapshot carries its own device-side K: the next decode re-uploads the caller's
     return MMI_OK;
 }
@@ -1227,6 +1490,7 @@ extern "C" int mmi_mimi_set_exec_mask(mmi_mimi* m, const uint8_t* mask, mmi_stre
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m || !mask) return mmi_fail(MMI_ERR_INVALID, "null argument");
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
+    m->all_exec = false;
     MMI_LAUNCH(k_set_mask, mmi_cdiv(m->batch, 64), 64, 0, (hipStream_t)stream, m->exec, mask, m->batch);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
@@ -1238,6 +1502,7 @@ extern "C" int mmi_mimi_reset(mmi_mimi* m, const uint8_t* mask, mmi_stream strea
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
     hipStream_t s = (hipStream_t)stream;
     const int B = m->batch;
+    if (!mask) m->all_exec = true;
     if (m->enc_hist_rows > 0)
         MMI_LAUNCH(k_reset_history, mmi_cdiv(m->enc_hist_rows, 256), 256, 0, s, (const HistDesc*)m->enc_hist, m->enc_nhist, m->enc_hist_rows, mask);
     if (m->dec_hist_rows > 0)
@@ -1256,16 +1521,20 @@ static int encode_impl(mmi_mimi* m, const float* pcm, int64_t* codes, float* lat
     if (!pcm) return mmi_fail(MMI_ERR_INVALID, "null pcm");
     const mmi_mimi_cfg& c = m->cfg;
     const int F = c.frame_size, K = m->n_codebooks;
-    for (int f = 0; f < n_frames; ++f) {
-        // stage the frame behind the first conv's history
-        MMI_LAUNCH(k_copy2d_f32, (int)mmi_cdiv64((int64_t)batch * c.channels * F, 256), 256, 0, s, pcm + (long)f * F,
-                   (long)n_frames * F, m->enc_in.p + m->enc_in.H, (long)m->enc_in.ld, batch * c.channels, F);
-        if ((rc = m->enc_prog.run(s, m->use_graph, m->cap_stream))) return rc;
+    for (int f = 0, G; f < n_frames; f += G) {
+        G = group_frames(m, m->enc_grp, m->enc_tab, n_frames - f, s);
+        if (G > 1 && ready_group(m, true, G, s)) { m->enc_grp.refused = true; G = 1; }
+        const Buf &in = G > 1 ? m->enc_grp.in : m->enc_in, &lat = G > 1 ? m->enc_grp.out : m->latent;
+        // stage the samples behind the first conv's history
+        MMI_LAUNCH(k_copy2d_f32, (int)mmi_cdiv64((int64_t)batch * c.channels * G * F, 256), 256, 0, s, pcm + (long)f * F,
+                   (long)n_frames * F, in.p + in.H, (long)in.ld, batch * c.channels, G * F);
+        if ((rc = G > 1 ? run_group(m, true, s) : m->enc_prog.run(s, m->use_graph, m->cap_stream))) return rc;
         if (codes)
-            MMI_LAUNCH(k_codes_out, mmi_cdiv(batch * K, 256), 256, 0, s, (const int*)m->codes_i32, c.q_n_q, (long*)codes, batch, K, n_frames, f);
+            MMI_LAUNCH(k_codes_out, mmi_cdiv(batch * G * K, 256), 256, 0, s, (const int*)(G > 1 ? m->enc_grp.codes : m->rvq.codes), c.q_n_q, (long*)codes,
+                       batch, K, n_frames, f, G);
         if (latent)
-            MMI_LAUNCH(k_copy2d_f32, mmi_cdiv(batch * c.dimension, 256), 256, 0, s, (const float*)m->latent.p, 1L, latent + f,
-                       (long)n_frames, batch * c.dimension, 1);
+            MMI_LAUNCH(k_copy2d_f32, mmi_cdiv(batch * c.dimension * G, 256), 256, 0, s, (const float*)lat.p, (long)lat.ld, latent + f,
+                       (long)n_frames, batch * c.dimension, G);
         MMI_CHECK_LAUNCH();
     }
     return MMI_OK;
@@ -1294,12 +1563,14 @@ extern "C" int mmi_mimi_quantize(mmi_mimi* m, const float* latent, int64_t* code
     const mmi_mimi_cfg& c = m->cfg;
     for (int f = 0; f < n_frames; ++f) {
         MmiProgram prog;
-        int rc = add_quantize_ops(m, prog, latent, n_frames, f, batch);
+        MimiMem mem;
+        mem.arena = &m->st;
+        int rc = add_quantize_ops(m, mem, m->rvq, prog, latent, n_frames, f, batch);
         if (rc) return rc;
         rc = prog.run_eager(s);
         if (rc) return rc;
-        MMI_LAUNCH(k_codes_out, mmi_cdiv(batch * m->n_codebooks, 256), 256, 0, s, (const int*)m->codes_i32, c.q_n_q, (long*)codes, batch,
-                   m->n_codebooks, n_frames, f);
+        MMI_LAUNCH(k_codes_out, mmi_cdiv(batch * m->n_codebooks, 256), 256, 0, s, (const int*)m->rvq.codes, c.q_n_q, (long*)codes, batch,
+                   m->n_codebooks, n_frames, f, 1);
         MMI_CHECK_LAUNCH();
     }
     return MMI_OK;
@@ -1315,10 +1586,12 @@ extern "C" int mmi_mimi_decode_latent(mmi_mimi* m, const int64_t* codes, float* 
     const mmi_mimi_cfg& c = m->cfg;
     Buf out; out.p = latent; out.C = c.dimension; out.ld = n_frames; out.H = 0;
     for (int f = 0; f < n_frames; ++f) {
-        MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)n_codebooks * n_frames, m->dec_codes_i32,
-                   c.q_n_q, batch, n_codebooks, n_frames, f);
+        MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)n_codebooks * n_frames, m->deq.codes,
+                   c.q_n_q, batch, n_codebooks, n_frames, f, 1);
         MmiProgram prog;
-        int rc = add_dequant_ops(m, prog, n_codebooks, out, f, batch);
+        MimiMem mem;
+        mem.arena = &m->st;
+        int rc = add_dequant_ops(m, mem, m->deq, prog, n_codebooks, out, f, batch);
         if (rc) return rc;
         rc = prog.run_eager(s);
         if (rc) return rc;
@@ -1349,13 +1622,16 @@ extern "C" int mmi_mimi_decode_step_strided(mmi_mimi* m, const int64_t* codes, i
         MMI_HIP_CHECK(hipStreamSynchronize(s));         // the host word is reused; K changes at most once per model in practice
         m->dec_k_cur = n_codebooks;
     }
-    for (int f = 0; f < n_frames; ++f) {
-        MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)batch_stride, m->dec_codes_i32, c.q_n_q,
-                   batch, n_codebooks, n_frames, f);
+    for (int f = 0, G; f < n_frames; f += G) {
+        G = group_frames(m, m->dec_grp, m->dec_tab, n_frames - f, s);
+        if (G > 1 && ready_group(m, false, G, s)) { m->dec_grp.refused = true; G = 1; }
+        MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * G * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)batch_stride, G > 1 ? m->dec_grp.codes : m->deq.codes,
+                   c.q_n_q, batch, n_codebooks, n_frames, f, G);
         MMI_CHECK_LAUNCH();
-        if ((rc = m->dec_prog.run(s, m->use_graph, m->cap_stream))) return rc;
-        MMI_LAUNCH(k_copy2d_f32, (int)mmi_cdiv64((int64_t)batch * c.channels * F, 256), 256, 0, s, (const float*)m->dec_out.p, (long)m->dec_out.ld,
-                   pcm + (long)f * F, (long)n_frames * F, batch * c.channels, F);
+        if ((rc = G > 1 ? run_group(m, false, s) : m->dec_prog.run(s, m->use_graph, m->cap_stream))) return rc;
+        const Buf& out = G > 1 ? m->dec_grp.out : m->dec_out;
+        MMI_LAUNCH(k_copy2d_f32, (int)mmi_cdiv64((int64_t)batch * c.channels * G * F, 256), 256, 0, s, (const float*)out.p, (long)out.ld,
+                   pcm + (long)f * F, (long)n_frames * F, batch * c.channels, G * F);
         MMI_CHECK_LAUNCH();
     }
     return MMI_OK;

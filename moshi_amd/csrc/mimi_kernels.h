@@ -89,11 +89,13 @@ __global__ void k_codebook_prepare(const float* __restrict__ esum, const float* 
 //                k_pack_b_f32 (im2col + ELU + replicate padding) or by the producing kernel.
 enum { MMI_ACT_NONE = 0, MMI_ACT_GELU = 1, MMI_ACT_ELU = 2 };
 
-// n / d for 0 <= n < 2^17 and 1 <= d < 2^11 (column and tap indices) as one multiply-high: an integer division costs
-// ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^32 / d), 0 means d == 1.
-MMI_HD unsigned mmi_div_magic(int d) { return d <= 1 ? 0u : (unsigned)((0x100000000ull + (unsigned)d - 1) / (unsigned)d); }
-MMI_HD int mmi_fast_div(int n, unsigned magic) {
-    return magic == 0u ? n : (int)(((unsigned long long)(unsigned)n * magic) >> 32);
+// n / d for 0 <= n < 2^17 and 1 <= d < 2^17 (column and tap indices) as one multiply-high and a shift: an integer division costs
+// ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^(32 + shift) / d), 0 means d == 1; exact while
+// n d < 2^(32 + shift), hence the 8 more bits (which still fit the magic number) from d = 2^11 on.
+MMI_HD unsigned mmi_div_shift(int d) { return d < (1 << 11) ? 0u : 8u; }
+MMI_HD unsigned mmi_div_magic(int d, unsigned shift = 0u) { return d <= 1 ? 0u : (unsigned)(((0x100000000ull << shift) + (unsigned)d - 1) / (unsigned)d); }
+MMI_HD int mmi_fast_div(int n, unsigned magic, unsigned shift = 0u) {
+    return magic == 0u ? n : (int)((unsigned)(((unsigned long long)(unsigned)n * magic) >> 32) >> shift);
 }
 enum { MMI_GOUT_NATURAL = 0, MMI_GOUT_PACKED = 1, MMI_GOUT_PARTIAL = 2 };
 
@@ -113,7 +115,7 @@ struct ConvGemmArgs {
     const uint8_t* first; // replicate-pad flags [B] or null (conv.py:253-259)
     const uint8_t* exec;  // exec mask [B] (only read with `first`)
     int B, Cin, Cout, K, S, T_out;
-    unsigned T_magic, K_magic;   // mmi_div_magic(T_out), mmi_div_magic(K)
+    unsigned T_magic, T_shift, K_magic;   // mmi_div_magic(T_out, T_shift), mmi_div_magic(K)
     int Mt, Q;            // M tiles of 32, packed k-quads (Kdim_pad / 8)
     int Ntot;             // B * T_out
     int elu_in;           // apply ELU(alpha=1) to every loaded input (seanet.py:63,205,222)
@@ -132,6 +134,7 @@ struct ConvGemmArgs {
     const float* ln_b;
     float ln_eps;
     // --- filled in by the engine's planner
+    int q_blk;            // k_conv_wide: quads per workgroup of a split reduction (Q: not split)
     const int* koff;      // k_conv_wide: [Q][2][4] input offset of kd = (q*4+e)*2 + h; 0 past Cin*K (the weights there are 0)
     const float* bp;      // k_gemm_f32: packed activations [ceil(N/32)][Q][64][4]
     int x_packed;         // the producer already wrote `bp` (no k_pack_b_f32 launch)
@@ -233,10 +236,12 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
     const int mt0 = (int)blockIdx.y * MTB;
     const bool nvalid = n < a.Ntot;
     const int nn = nvalid ? n : 0;
-    const int b = mmi_fast_div(nn, a.T_magic), t = nn - b * a.T_out;
+    const int b = mmi_fast_div(nn, a.T_magic, a.T_shift), t = nn - b * a.T_out;
     const float* xb = a.x + (long)b * a.x_bstride + a.x_off + t * a.S;
-    const int qper = (a.Q + W - 1) / W;
-    const int q0 = min(a.Q, wave * qper), q1 = min(a.Q, q0 + qper);
+    // gridDim.z > 1: the reduction is also split over workgroups (k_conv_finish adds their sums), cut as k_gemm_f32 cuts it
+    const int qb0 = min(a.Q, (int)blockIdx.z * a.q_blk), qb1 = min(a.Q, qb0 + a.q_blk);
+    const int qper = (qb1 - qb0 + W - 1) / W;
+    const int q0 = min(qb1, qb0 + wave * qper), q1 = min(qb1, q0 + qper);
 
     f32x16 acc[MTB];
 #pragma unroll
@@ -315,12 +320,14 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
                 co[i] = (mt0 + m) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (le >> 5);
                 ok[i] = nn2 < a.Ntot && co[i] < a.Cout;
                 const int n3 = ok[i] ? nn2 : 0;
-                bb[i] = mmi_fast_div(n3, a.T_magic);
+                bb[i] = mmi_fast_div(n3, a.T_magic, a.T_shift);
                 tt[i] = n3 - bb[i] * a.T_out;
                 float s = 0.f;
                 for (int w = 0; w < W; ++w) s += red[w * NE + e];
                 v[i] = s;
+                if (a.out_mode == MMI_GOUT_PARTIAL && (mt0 + m) < a.Mt) a.partial[((long)blockIdx.z * a.Mt * 32 + co[i]) * a.Npad + nn2] = s;
             }
+            if (a.out_mode == MMI_GOUT_PARTIAL) continue;
             mmi_conv_store_n<NV>(a, co, bb, tt, ok, v);
         }
         return;
@@ -393,7 +400,7 @@ __global__ __launch_bounds__(MT1 * 64) void k_resblock(ResBlockArgs ra) {
     const int jl = lane & 31, kh = lane >> 5;
     // the tile's 32 columns belong to ONE session (T_out % 32 == 0, checked by the engine): b, t0 are uniform
     const int n0 = (int)blockIdx.x * 32;
-    const int b = mmi_fast_div(n0, a.T_magic), t0 = n0 - b * a.T_out;
+    const int b = mmi_fast_div(n0, a.T_magic, a.T_shift), t0 = n0 - b * a.T_out;
     const int LD = 32 + a.K - 1;                 // input columns the tile's windows cover (stride 1)
     MMI_DYN_SHARED(float, smem);                 // Xs[Cin][LD] | offs[Q][2][4] | mailbox[MT1][4][64][4]
     float* Xs = smem;
@@ -568,7 +575,7 @@ __global__ void k_pack_b_f32(ConvGemmArgs a, float* __restrict__ bp) {
     {   // columns past Ntot / reduction indices past Cin*K read a clamped (valid) element: they meet zero weights or are
         // discarded, and unconditional loads are not serialised by the compiler
         const int nc = n < a.Ntot ? n : 0;
-        const int b = mmi_fast_div(nc, a.T_magic), t = nc - b * a.T_out;
+        const int b = mmi_fast_div(nc, a.T_magic, a.T_shift), t = nc - b * a.T_out;
         const float* xb = a.x + (long)b * a.x_bstride + a.x_off + t * a.S;
         const bool rep = a.first != nullptr && a.first[b] != 0 && a.exec[b] != 0;
         const int hist = a.H - a.x_off;  // columns (relative to x_off) that belong to the history
@@ -637,7 +644,7 @@ __device__ __forceinline__ void mmi_gemm_f32_finish(const ConvGemmArgs& a, f32x1
     for (int i = 0; i < NV; ++i) {
         ok[i] = nn[i] < a.Ntot && co[i] < a.Cout;
         const int n3 = ok[i] ? nn[i] : 0;
-        bb[i] = mmi_fast_div(n3, a.T_magic);
+        bb[i] = mmi_fast_div(n3, a.T_magic, a.T_shift);
         tt[i] = n3 - bb[i] * a.T_out;
     }
     mmi_conv_store_n<NV>(a, co, bb, tt, ok, v);
@@ -799,7 +806,7 @@ __global__ void k_conv_finish(ConvGemmArgs a, int ksplit) {
     float x = 0.f;
 #pragma unroll
     for (int s = 0; s < 8; ++s) x += s < ksplit ? pv[s] : 0.f;
-    const int bq = mmi_fast_div(n, a.T_magic);
+    const int bq = mmi_fast_div(n, a.T_magic, a.T_shift);
     int co1[1] = {co}, b1[1] = {bq}, t1[1] = {n - bq * a.T_out};
     bool ok1[1] = {true};
     float v1[1] = {x};
@@ -814,7 +821,7 @@ __global__ void k_conv_finish(ConvGemmArgs a, int ksplit) {
 __global__ void k_convtr_combine(const float* __restrict__ tmp, const float* __restrict__ bias,
                                  float* __restrict__ partial, const uint8_t* __restrict__ exec, float* __restrict__ out,
                                  int out_ld, int out_off, int B, int Cout, int K, int S, int T_in, float* __restrict__ out2,
-                                 int tmp_ld) {
+                                 int tmp_ld, int T_frame) {
     long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int Tout = T_in * S;
     if (idx >= (long)B * Cout * Tout) return;
@@ -825,8 +832,11 @@ __global__ void k_convtr_combine(const float* __restrict__ tmp, const float* __r
     int t = p / S, r = p - t * S;
     const float* trow = tmp + row * (long)K * tmp_ld;  // [K][T_in], row stride tmp_ld
     float v = trow[(long)r * tmp_ld + t];
-    if (t > 0) v += trow[(long)(r + S) * tmp_ld + (t - 1)];
+    const bool inside = t > 0 && (T_frame == T_in || t % T_frame != 0);   // what a frame takes over from the one before it is added last, as when it is kept as `partial`
+    const float before = t > 0 ? trow[(long)(r + S) * tmp_ld + (t - 1)] : 0.f;
+    if (inside) v += before;
     if (bias) v += bias[co];
+    if (!inside && t > 0) v += before;
     if (t == 0) {
         // y[..., :PT] += partial; then the thread that consumed partial[b][co][r] also refreshes it
         long pi = row * (long)(K - S) + r;
@@ -910,6 +920,19 @@ __global__ void k_commit_all(HistTable tab, int total_rows, const uint8_t* __res
     if (!exec[b]) return;
     float* r = h.p + (long)row * h.ld;
     for (int p = 0; p < h.H; ++p) r[p] = r[p + h.T];  // ascending: source p+T is always ahead of the write
+}
+
+// the histories of one set of buffers -> the same ones of another
+__global__ void k_move_history(HistTable from, HistTable to, int total_rows) {
+    const int gid = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (gid >= total_rows) return;
+    int d = 0;
+#pragma unroll
+    for (int i = 1; i < MMI_HIST_MAX; ++i)
+        if (i < from.n && from.d[i].row_begin <= gid) d = i;
+    const HistDesc f = from.d[d], t = to.d[d];
+    const long row = gid - f.row_begin;
+    for (int p = 0; p < f.H; ++p) t.p[row * t.ld + p] = f.p[row * f.ld + p];
 }
 
 // offsets[i][b] += inc where exec; first[b] = 0 where exec
@@ -1024,6 +1047,14 @@ struct MimiAttnArgs {
     int outQ;
     int B, H, D, T, cap, context;
     float max_period;
+};
+
+// Several frames at once: T = all of the call's positions.  A frame's positions enter the ring together, so a query sees the positions of
+// (last - cap, own], `last` being its frame's last one.  Those of this call are read from its own rows and reach the ring after all layers
+// (k_mimi_group_ring): the ring cannot hold what the call's oldest and its newest query see at the same time.
+struct MimiGroupRows {
+    int T, qkv_ld;
+    float *q, *kn, *vn;        // [B][H][T][D]
 };
 
 // 256 threads; D/4 lanes share a ring row (one 16-byte load each), so a wave instruction reads 64/(D/4) consecutive
@@ -1168,8 +1199,9 @@ __global__ __launch_bounds__(256) void k_mimi_attn(MimiAttnArgs a) {
 // registers.  Each wave normalises against its own maximum; the four waves are merged through LDS with the usual
 // exp(m_wave - m) rescale.  The slots written by this call are taken from LDS instead of the ring (the ring loads were
 // issued before the write).  Static LDS: qs | kn | vn [T][D], red[4][T][D], mw/sw [4][T].
-template <int D, int T>
-__global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
+// GROUP: one workgroup per (b, head) and frame (blockIdx.y) of a MimiGroupRows call; the same sums in the same order as frame by frame.
+template <int D, int T, bool GROUP = false>
+__global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGroupRows g) {
     constexpr int LPR = D / 4;             // lanes per ring row
     constexpr int RPB = 256 / LPR;         // rows per block pass
     constexpr int IT = 16;                 // passes: cap <= IT * RPB
@@ -1182,7 +1214,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
     MMI_SHARED __attribute__((aligned(16))) float red[4 * T * D];
     MMI_SHARED float mw[4 * T];
     MMI_SHARED float sw[4 * T];
-    const long off = a.offsets[b];
+    const long off0 = a.offsets[b], off = off0 + (GROUP ? (long)blockIdx.y * T : 0);
     const int HD = a.H * D;
     const float* qrow = a.qkv + (long)b * 3 * HD * T;
     float* kcb = a.kc + ((long)b * a.H + h) * cap * D;
@@ -1196,12 +1228,23 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
     f32x4 kk[IT], vv[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        const long r = (long)min(i * RPB + rsub, L - 1) * D + seg * 4;
-        kk[i] = *reinterpret_cast<const f32x4*>(kcb + r);
-        vv[i] = *reinterpret_cast<const f32x4*>(vcb + r);
+        const int slot = min(i * RPB + rsub, L - 1);
+        const long r = (long)slot * D + seg * 4;
+        if constexpr (GROUP) {
+            const long pos = slot <= end_index ? last + slot - end_index : last + slot - end_index - cap, n = pos - off0;
+            const long w = (((long)blockIdx.x * g.T) + (n > 0 ? n : 0)) * D + seg * 4;
+            kk[i] = *reinterpret_cast<const f32x4*>(n >= 0 ? g.kn + w : kcb + r);
+            vv[i] = *reinterpret_cast<const f32x4*>(n >= 0 ? g.vn + w : vcb + r);
+        } else {
+            kk[i] = *reinterpret_cast<const f32x4*>(kcb + r);
+            vv[i] = *reinterpret_cast<const f32x4*>(vcb + r);
+        }
     }
 
     // rope(q), rope(k) -> LDS and ring, v -> LDS and ring (written unconditionally, transformer.py:243-250)
+    if constexpr (GROUP) {
+        for (int i = tid; i < T * D; i += 256) qs[i] = g.q[((long)blockIdx.x * g.T + (long)blockIdx.y * T) * D + i];
+    } else {
     for (int i = tid; i < T * (D / 2); i += 256) {
         const int t = i / (D / 2), j = i % (D / 2);
         const float freq = expf((float)j * (-logf(a.max_period) * 2.0f / (float)D));
@@ -1216,13 +1259,15 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
         const int t = i / D, d = i % D;
         vn[i] = qrow[(long)(2 * HD + h * D + d) * T + t];
     }
-    __syncthreads();
-    for (int i = tid; i < T * D; i += 256) {
-        const int t = i / D, d = i % D;
-        const long slot = (off + t) % cap;
-        kcb[slot * D + d] = kn[i];
-        vcb[slot * D + d] = vn[i];
     }
+    __syncthreads();
+    if constexpr (!GROUP)
+        for (int i = tid; i < T * D; i += 256) {
+            const int t = i / D, d = i % D;
+            const long slot = (off + t) % cap;
+            kcb[slot * D + d] = kn[i];
+            vcb[slot * D + d] = vn[i];
+        }
 
     const float scale = 1.0f / sqrtf((float)D);
     f32x4 qv[T];
@@ -1241,7 +1286,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
         const int slot = i * RPB + rsub;
 #pragma unroll
         for (int t = 0; t < T; ++t)
-            if (slot == newslot[t]) {      // a later token of this call overwrites an earlier one when T > cap never happens (T <= 2 <= cap)
+            if (!GROUP && slot == newslot[t]) {      // a later token of this call overwrites an earlier one when T > cap never happens (T <= 2 <= cap)
                 kk[i] = *reinterpret_cast<const f32x4*>(kn + t * D + seg * 4);
                 vv[i] = *reinterpret_cast<const f32x4*>(vn + t * D + seg * 4);
             }
@@ -1299,9 +1344,51 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a) {
             den += f * sw[w * T + t];
         }
         const float o = num / den;
-        if (a.outp) a.outp[mmi_bp_index(h * D + d, b * T + t, a.outQ)] = o;
+        if constexpr (GROUP) a.outp[mmi_bp_index(h * D + d, b * g.T + (int)blockIdx.y * T + t, a.outQ)] = o;
+        else if (a.outp) a.outp[mmi_bp_index(h * D + d, b * T + t, a.outQ)] = o;
         else a.out[((long)b * HD + h * D + d) * T + t] = o;
     }
+}
+
+// Rows of a call that brings several frames of a stream at once (MimiGroupRows): qkv [B][3 H D][ld] -> rotated queries, rotated keys and
+// values row by row [b][h][T][D], through LDS so that both sides move whole lines.
+template <int D>
+__global__ __launch_bounds__(256) void k_mimi_group_rope(MimiAttnArgs a, MimiGroupRows g) {
+    const int b = (int)blockIdx.x / a.H, h = (int)blockIdx.x % a.H, t0 = (int)blockIdx.y * 32, tid = (int)threadIdx.x;
+    const int HD = a.H * D;
+    MMI_SHARED float tile[3 * D * 33];                     // [q | k | v][d][t]
+    for (int i = tid; i < 3 * D * 32; i += 256) {
+        const int t = i & 31, d = (i >> 5) % D, w = (i >> 5) / D;
+        tile[(w * D + d) * 33 + t] = a.qkv[((long)b * 3 * HD + w * HD + h * D + d) * g.qkv_ld + min(t0 + t, g.T - 1)];
+    }
+    __syncthreads();
+    const long off = a.offsets[b], row0 = (long)blockIdx.x * g.T + t0;
+    for (int i = tid; i < 32 * (D / 2); i += 256) {
+        const int j = i % (D / 2), t = i / (D / 2);
+        if (t0 + t >= g.T) continue;
+        const float freq = expf((float)j * (-logf(a.max_period) * 2.0f / (float)D));
+        const float ang = freq * (float)(off + t0 + t);
+        const float c = cosf(ang), s = sinf(ang);
+        float q0, q1, k0, k1;
+        mmi_rope_rotate(tile[(2 * j) * 33 + t], tile[(2 * j + 1) * 33 + t], c, s, q0, q1);
+        mmi_rope_rotate(tile[(D + 2 * j) * 33 + t], tile[(D + 2 * j + 1) * 33 + t], c, s, k0, k1);
+        const long at = (row0 + t) * D + 2 * j;
+        g.q[at] = q0; g.q[at + 1] = q1;
+        g.kn[at] = k0; g.kn[at + 1] = k1;
+        g.vn[at] = tile[(2 * D + 2 * j) * 33 + t]; g.vn[at + 1] = tile[(2 * D + 2 * j + 1) * 33 + t];
+    }
+}
+
+// kvn [layer][k | v][B][H][T][D] -> kv [layer][k | v][B][H][cap][D], four values per thread
+__global__ void k_mimi_group_ring(const float* __restrict__ kvn, float* __restrict__ kv, const long* __restrict__ offsets, int L, int B, int H, int T,
+                                  int cap, int D) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = T < cap ? T : cap, D4 = D / 4;
+    if (idx >= (long)L * 2 * B * H * n * D4) return;
+    const int d = (int)(idx % D4), t = T - n + (int)(idx / D4 % n);
+    const long row = idx / D4 / n;                         // (layer, k | v, b, h)
+    const int b = (int)(row / H % B);
+    reinterpret_cast<f32x4*>(kv)[(row * cap + (offsets[b] + t) % cap) * D4 + d] = reinterpret_cast<const f32x4*>(kvn)[(row * T + t) * D4 + d];
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1441,20 +1528,20 @@ __global__ void k_rvq_gather(const int* __restrict__ codes, int codes_rstride, i
     }
 }
 
-// int64 <-> int32 code tensors at the ABI boundary: [B][K][F] i64 <-> per-frame [B][K] i32
+// int64 <-> int32 code tensors at the ABI boundary: [B][K][F] i64 <-> [B * G][K] i32 of the G frames from f on
 __global__ void k_codes_out(const int* __restrict__ src, int src_rstride, long* __restrict__ dst, int B, int K, int F,
-                            int f) {
+                            int f, int G) {
     int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (idx >= B * K) return;
-    int b = idx / K, k = idx % K;
-    dst[((long)b * K + k) * F + f] = (long)src[(long)b * src_rstride + k];
+    if (idx >= B * G * K) return;
+    int r = idx / K, k = idx % K, b = r / G;
+    dst[((long)b * K + k) * F + f + r - b * G] = (long)src[(long)r * src_rstride + k];
 }
 // src: i64 [B][K][F] with `src_bstride` elements between batch rows (K * F when dense; larger for a column slice of a wider
 // tensor such as LMGen's [B][1 + dep_q][1] step output read from its second column on)
 __global__ void k_codes_in(const long* __restrict__ src, long src_bstride, int* __restrict__ dst, int dst_rstride, int B, int K,
-                           int F, int f) {
+                           int F, int f, int G) {
     int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (idx >= B * K) return;
-    int b = idx / K, k = idx % K;
-    dst[(long)b * dst_rstride + k] = (int)src[(long)b * src_bstride + (long)k * F + f];
+    if (idx >= B * G * K) return;
+    int r = idx / K, k = idx % K, b = r / G;
+    dst[(long)r * dst_rstride + k] = (int)src[(long)b * src_bstride + (long)k * F + f + r - b * G];
 }

@@ -1,0 +1,59 @@
+"""Calls of several frames run them through the codec together (mimi_engine.hip, MimiGroup): every output bit and the streaming state must be
+those of the same frames one by one - across the attention ring's wrap, between groups of different sizes, around single frames, after a
+reset, under an exec mask (frame by frame then) and after a snapshot."""
+import pytest
+import torch
+
+from moshi_amd import MimiModel, tiny_mimi_config
+from moshi_amd.config import MimiConfig
+from moshi_amd.weights import random_mimi_state_dict
+
+
+def check_calls_equal_frames(make, device, cfg, B, sizes, K=4):
+    sd = random_mimi_state_dict(cfg, seed=5, device=device)
+    gen = torch.Generator().manual_seed(B)
+    n, fs = sum(sizes), cfg.frame_size
+    x = (0.3 * torch.randn(B, 1, n * fs, generator=gen)).to(device)
+    q = torch.randint(0, cfg.q_bins, (B, K, n), generator=gen).to(device)
+    a, b = make(sd, cfg, K, B), make(sd, cfg, K, B)
+
+    def same(at, size, what):
+        part = x[..., at * fs:(at + size) * fs].contiguous()
+        codes = torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(at, at + size)], -1)
+        assert torch.equal(a.encode(part), codes), f"{what}: codes of frames {at}..{at + size}"
+        pcm = torch.cat([b.decode(q[..., f:f + 1].contiguous()) for f in range(at, at + size)], -1)
+        assert torch.equal(a.decode(q[..., at:at + size].contiguous()), pcm), f"{what}: samples of frames {at}..{at + size}"
+    with a.streaming(B), b.streaming(B):
+        at = 0
+        for size in sizes:
+            same(at, size, "stream")
+            at += size
+        for m in (a, b):
+            m.reset_streaming()
+        same(0, sizes[0], "after a reset")
+        if B > 1:
+            mask = torch.arange(B) % 2 == 0
+            for m in (a, b):
+                m.set_exec_mask(mask.to(device))
+            codes = a.encode(x[..., :2 * fs].contiguous())
+            want = torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(2)], -1)
+            assert torch.equal(codes[mask], want[mask]), "under a mask"
+            for m in (a, b):
+                m.set_exec_mask(torch.ones(B, dtype=torch.bool, device=device))
+                m.reset_streaming()
+        b.set_streaming_state(a.get_streaming_state())
+        same(0, sizes[-1], "after a snapshot")
+    whole = a.encode(x)                                        # a fresh, temporary stream
+    with b.streaming(B):
+        assert torch.equal(whole, torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(n)], -1)), "temporary stream"
+
+
+@pytest.mark.parametrize("B,sizes", [(1, (2, 1, 7, 3)), (3, (5, 1, 4))])
+def test_tiny_calls_equal_frames(sim_lib, B, sizes):
+    check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", tiny_mimi_config(), B, sizes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,sizes", [(1, (1, 2, 65, 64, 3)), (3, (21, 1, 22)), (32, (2, 1, 3)), (33, (2,))])
+def test_full_size_calls_equal_frames(B, sizes):
+    check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cuda", max_batch=mb, num_codebooks=K), "cuda", MimiConfig(), B, sizes, K=8)
