@@ -204,6 +204,30 @@ __device__ __forceinline__ int mmi_uniform(int v) { return __builtin_amdgcn_read
 // true in every lane when any lane's flag is set
 __device__ __forceinline__ bool mmi_any(bool v) { return __any(v) != 0; }
 
+// 16 bytes per lane from global memory into LDS without a register in between: lane l's land at lds[at + l] (lds, at: the same in every
+// lane).  Nothing waits for them but mmi_wait_loads (the compiler does not know of them), which counts this wave's loads in the order of
+// their issue, and behind it a barrier for the other waves' ones.  First form: base (uniform) + offset per lane in bytes.
+// (m0 is named as overwritten so that no value of the compiler's own stays in it; it notes that the register is a reserved one)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ unsigned mmi_lds_addr(const void* p) { return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)p; }
+__device__ __forceinline__ void mmi_load_lds(const void* base, unsigned off, u32x4* lds, int at) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(mmi_lds_addr(lds) + 16u * (unsigned)at), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void mmi_load_lds(const u32x4* from, u32x4* lds, int at) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(mmi_lds_addr(lds) + 16u * (unsigned)at), "v"(from) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// until at most N of this wave's loads are in flight
+template <int N>
+__device__ __forceinline__ void mmi_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// the workgroup's waves meet; unlike __syncthreads it does not wait for loads in flight (LDS reads and writes of this wave are done)
+__device__ __forceinline__ void mmi_meet() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // streamed-once weights: non-temporal so they do not evict the activations / KV the other kernels reuse
 __device__ __forceinline__ u32x4 mmi_load_nt(const u32x4* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ f32x4 mmi_load_nt(const f32x4* p) { return __builtin_nontemporal_load(p); }

@@ -141,7 +141,6 @@ struct mmi_tlm {
     uint16_t* samp_rows = nullptr; int samp_ld = 0;
     int* samp_map = nullptr; unsigned long long* samp_rng = nullptr; int* samp_zero = nullptr;
     uint64_t samp_count = 0;
-    long split_elems = 0;          // partial-sum capacity of mix / dn / lat in rows
     // host state
     std::vector<Slot> slots;
     std::vector<int> free_pages;
@@ -159,6 +158,7 @@ struct mmi_tlm {
 namespace {
 
 constexpr int MAX_SPLIT = 8;
+constexpr int TILE_SPLIT = 8, TILE_BLOCKS = 512;      // the tiled kernel: K splits, blocks that a split aims at
 constexpr int ROWS_MAX = 64;       // up to here a step takes the weight-streaming kernel
 constexpr int ATTN_TILE_GROUPS = 128;     // from this many column groups the attention stages keys through LDS
 constexpr int PREFIXES = 6;        // prefix arrays over the sequences per head count: tiles, groups of 4, groups of 8, then those of `split`
@@ -609,7 +609,11 @@ int alloc_buffers(mmi_tlm* m) {
     const mmi_tlm_cfg& c = m->cfg;
     const int T = m->max_T;
     int rc;
-    m->split_elems = std::max((long)T, (long)MAX_SPLIT * ROWS_MAX);
+    // elements of a product that may be split: T (times `top`) rows once, few rows MAX_SPLIT times, and of the tiled kernel's splits what
+    // fewer than 2 TILE_BLOCKS blocks of 128 x 128 hold
+    auto split_room = [&](long top, long ld) {
+        return (size_t)std::max(std::max((long)T, (long)MAX_SPLIT * ROWS_MAX) * top * ld, std::min((long)TILE_SPLIT * T * top * ld, 2L * TILE_BLOCKS * 128 * 128));
+    };
     int gru_w = 0, y_ks = 0, lat_ld = 0, cq_ks = 0, qn_ks = 0, o_ks = 0, hid_ks = 0, gate_ld = 0, nd = 0;
     long q_elems = 0, ao_elems = 0;
     long lin_ld = 0, conv_c = 0, dec_ld = 0, lgate_ld = 0, lo_ld = 0, heads = 0, hd = 0, hv = 0;
@@ -648,7 +652,7 @@ int alloc_buffers(mmi_tlm* m) {
         if (L.c.mlp != MMI_TLM_MLP_NONE) hid_ks = std::max(hid_ks, L.down.KS);
     }
     if ((rc = alloc_f32(m, &m->x, (size_t)T * m->ld)) || (rc = alloc_packed(m, &m->h, std::max(T, m->max_slots), m->h_ks)) ||
-        (rc = alloc_f32(m, &m->mix, (size_t)m->split_elems * m->ld)))
+        (rc = alloc_f32(m, &m->mix, split_room(1, m->ld))))
         return rc;
     if (m->has_gru) {
         const int n_seg = T / TLM_SEG + m->max_slots + 1;
@@ -676,7 +680,7 @@ int alloc_buffers(mmi_tlm* m) {
         MMI_HIP_CHECK(hipMemset(m->prev_tok, 0, 2 * (size_t)m->max_slots * sizeof(int)));
     }
     if (m->has_latent) {
-        if ((rc = alloc_f32(m, &m->lat, (size_t)m->split_elems * lat_ld)) || (rc = alloc_packed(m, &m->cq, T, cq_ks)) || (rc = alloc_packed(m, &m->qn, T, qn_ks)) ||
+        if ((rc = alloc_f32(m, &m->lat, split_room(1, lat_ld))) || (rc = alloc_packed(m, &m->cq, T, cq_ks)) || (rc = alloc_packed(m, &m->qn, T, qn_ks)) ||
             (rc = alloc_packed(m, &m->q, q_elems * 16, 1)) || (rc = alloc_packed(m, &m->ao, ao_elems * 16, 1)) || (rc = alloc_packed(m, &m->o, T, o_ks)) ||
             (rc = alloc_f32(m, &m->gate, (size_t)T * gate_ld)) || (rc = alloc_f32(m, &m->po, (size_t)MAX_PARTIALS * nd * 256)) ||
             (rc = alloc_f32(m, &m->pml, (size_t)MAX_PARTIALS * 32)))
@@ -685,14 +689,14 @@ int alloc_buffers(mmi_tlm* m) {
             if ((rc = alloc_f32(m, &r.out, (size_t)T * r.ld * 2))) return rc;
     }
     if (m->route_host.empty() && hid_ks) {
-        if ((rc = alloc_packed(m, &m->hid, T, hid_ks)) || (rc = alloc_f32(m, &m->dn, (size_t)std::max((long)T, (long)MAX_SPLIT * ROWS_MAX) * m->ld))) return rc;
+        if ((rc = alloc_packed(m, &m->hid, T, hid_ks)) || (rc = alloc_f32(m, &m->dn, split_room(1, m->ld)))) return rc;
     }
     if (!m->route_host.empty()) {
         const size_t nl = m->route_host.size();
         m->list_ld = (long)T * m->max_top;
         m->tile_ld = (long)T * m->max_top / 16 + m->max_experts + 1;
         if ((rc = alloc_packed(m, &m->hid, (long)T * m->max_top, hid_ks)) ||
-            (rc = alloc_f32(m, &m->dn, (size_t)std::max((long)T, (long)MAX_SPLIT * ROWS_MAX) * m->max_top * m->ld)))
+            (rc = alloc_f32(m, &m->dn, split_room(m->max_top, m->ld))))
             return rc;
         MMI_HIP_CHECK(m->scratch.alloc(&m->list, nl * m->list_ld));
         MMI_HIP_CHECK(m->scratch.alloc(&m->tiles, nl * m->tile_ld * 3));
@@ -765,11 +769,14 @@ int alloc_state(mmi_tlm* m) {
 // ------------------------------------------------------------------------------------------------
 // launch list
 // ------------------------------------------------------------------------------------------------
-struct Plan { bool rows; int mt, fm; };      // weight-streaming kernel with mt row tiles, or the tiled kernel with 32 fm rows per block
-Plan plan_rows(int T) {
+// weight-streaming kernel with mt row tiles, or the tiled kernel with 32 fm rows per block
+struct Plan { bool rows; int mt, fm; };
+// 128 rows per block from where they no longer leave the chip idle or, with experts, half-filled blocks behind (an expert's run is cut
+// into blocks): 676 rows x 11264 x 2048 takes 45 us in 128 x 128 blocks and 50 us in 128 x 64 ones, 200 rows x 7680 x 2048 24 and 19
+Plan plan_rows(int T, bool routed) {
     Plan p{T <= ROWS_MAX, 1, 2};
     p.mt = T <= 16 ? 1 : (T <= 32 ? 2 : 4);
-    p.fm = T >= 1024 ? 4 : 2;
+    p.fm = T >= (routed ? 1024 : 640) ? 4 : 2;
     return p;
 }
 int plan_tile(const Plan& p) { return p.rows ? 16 * p.mt : 32 * p.fm; }
@@ -806,48 +813,67 @@ TlmJob routed_job(mmi_tlm* m, const Layer& L, const Mat& w, const void* x, int x
     return j;
 }
 int rows_ntw(const Plan& p);
-// K split so that a product with few n-tiles still covers the chip; the consumer sums the fp32 partials
+// K split so that a product with few n-tiles still covers the chip; the consumer sums the fp32 partials.  `blocks`: what the launch has
+// without a split - n-tiles of the weight-streaming kernel, blocks of the tiled kernel (tile_blocks).  The tiled kernel wants two blocks per
+// CU: 200 rows x 2048 x 2560 takes 18.1, 11.4, 9.2 us with 1, 2, 4 splits, 2048 rows x 2048 x 2560 31.7 and 26.1 with 1 and 2.
 int split_for(const Plan& p, const Mat& w, int blocks) {
-    if (!p.rows) return 1;
     int s = 1;
-    while (s < MAX_SPLIT && blocks * s < 384 * rows_ntw(p) && w.KS / (2 * s) >= 8) s *= 2;
+    if (p.rows) while (s < MAX_SPLIT && blocks * s < 384 * rows_ntw(p) && w.KS / (2 * s) >= 8) s *= 2;
+    else while (s < TILE_SPLIT && blocks * s < TILE_BLOCKS && w.KS / (2 * s) >= 16) s *= 2;
     return s;
 }
+// blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64)
+int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, 2 * p.fm) * (j.list ? j.rblocks : j.groups * mmi_cdiv(j.rows, plan_tile(p))); }
+int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
 
 int rows_ntw(const Plan& p) { return p.mt; }                // n-tiles per workgroup of the weight-streaming kernel
+template <class Tr, int FN, int FM, int ST, int OCC>
+int launch_tile(hipStream_t s, int grid, const TlmJobs& J) {
+    constexpr size_t smem = TlmTile<Tr, FN, FM, 2, 2, ST>::smem();
+    static_assert(smem * OCC <= 160 * 1024, "LDS of a CU");
+    if (smem > 64 * 1024) {
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, 2, 2, ST, OCC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        MMI_HIP_CHECK(attr);
+    }
+    MMI_LAUNCH((k_tlm_gemm_tile<Tr, FN, FM, 2, 2, ST, OCC>), grid, 256, smem, s, J);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
 template <class Tr>
 int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J) {
-    // the tiled kernel takes 256 features at a time where that still covers the chip
-    int fn = p.fm;
-    for (int pass = 0; pass < 2; ++pass) {
-        long total = 0;
-        if (!p.rows && p.fm == 4 && pass == 0) fn = 8;
+    auto cut = [&](int ntw) {                               // n-tiles per block -> blocks of every job, and their number
+        int total = 0;
         for (int i = 0; i < J.n; ++i) {
             TlmJob& j = J.j[i];
             if (!j.list) j.rblocks = mmi_cdiv(j.rows, plan_tile(p));
-            j.blocks = (p.rows ? mmi_cdiv(j.NT, rows_ntw(p)) : mmi_cdiv(j.NT, 2 * fn)) * (j.list ? 1 : j.groups) * j.ksplit * j.rblocks;
+            j.blocks = mmi_cdiv(j.NT, ntw) * (j.list ? 1 : j.groups) * j.ksplit * j.rblocks;
             total += j.blocks;
         }
-        if (fn == 8 && total < 256) {
-            fn = 4;
-            continue;
-        }
-        const int grid = (int)total;
-        if (p.rows) {
-            if (p.mt == 1) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 1, 1, 8, 4>), grid, 512, 0, s, J);
-            else if (p.mt == 2) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 2, 2, 8, 2>), grid, 512, 0, s, J);
-            else MMI_LAUNCH((k_tlm_gemm_rows<Tr, 4, 4, 4, 2>), grid, 256, 0, s, J);
-        } else if (fn == 8) {
-            MMI_LAUNCH((k_tlm_gemm_tile<Tr, 8, 4, 1>), grid, 256, 0, s, J);
-        } else if (p.fm == 4) {
-            MMI_LAUNCH((k_tlm_gemm_tile<Tr, 4, 4, 2>), grid, 256, 0, s, J);
-        } else {
-            MMI_LAUNCH((k_tlm_gemm_tile<Tr, 2, 2, 2>), grid, 256, 0, s, J);
-        }
-        break;
+        return total;
+    };
+    if (p.rows) {
+        const int grid = cut(rows_ntw(p));
+        if (p.mt == 1) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 1, 1, 8, 4>), grid, 512, 0, s, J);
+        else if (p.mt == 2) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 2, 2, 8, 2>), grid, 512, 0, s, J);
+        else MMI_LAUNCH((k_tlm_gemm_rows<Tr, 4, 4, 4, 2>), grid, 256, 0, s, J);
+        MMI_CHECK_LAUNCH();
+        return MMI_OK;
     }
-    MMI_CHECK_LAUNCH();
-    return MMI_OK;
+    // The widest block that still gives nearly every CU two: 256 x 128 in three stages (1773 x 22528 x 4096: 338 us, 0.97 PFLOP/s; in
+    // 128 x 128 blocks 379), then 128 x 128 (2048 x 2048 x 2560: 31.7 us against 47.3), in four stages while two blocks per CU are all there
+    // is, in three where a third one finds work (676 x 11264 x 2048: 47.7 against 58.1).  At fp32 the matrix core bounds every form.
+    if (p.fm == 4) {
+        if constexpr (Tr::V == 8) {
+            const int wide = cut(16);
+            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, wide, J);
+        }
+        const int grid = cut(8);
+        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, grid, J) : launch_tile<Tr, 4, 4, 3, 3>(s, grid, J);
+    }
+    // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
+    const int wide = cut(8);
+    if (Tr::V == 8 && wide >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, wide, J);
+    return launch_tile<Tr, 2, 2, 4, 4>(s, cut(4), J);
 }
 int launch_jobs(mmi_tlm* m, hipStream_t s, const Plan& p, TlmJobs J) {
     return m->f32 ? launch_jobs_t<TlmF32>(s, p, J) : launch_jobs_t<TlmBf16>(s, p, J);
@@ -1029,7 +1055,7 @@ MixerOut build_latent_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, cons
     j.out = m->lat;
     j.out_ld = ld;
     j.out_ps = (long)T * ld;
-    j.ksplit = split_for(p, L.in, L.in.NT);
+    j.ksplit = split_for(p, L.in, p.rows ? L.in.NT : tile_blocks(p, j) + (first.n ? tile_blocks(p, first.j[0]) : 0));
     const int in_p = j.ksplit;
     first.j[first.n++] = j;
     P.site(site + "in");
@@ -1373,7 +1399,7 @@ const char* mixer_site(int mixer) {
 
 void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
     const int T = sh.T;
-    const Plan p = plan_rows(T);
+    const Plan p = plan_rows(T, !m->route_host.empty());
     TlmPrepArgs a;
     memset(&a, 0, sizeof(a));
     a.T = T;
@@ -1438,7 +1464,7 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
             memset(&J, 0, sizeof(J));
             TlmJob& j = J.j[J.n++];
             j = dense_job(m->loop_in, m->cat, 2 * m->h_ks, T);
-            j.ksplit = split_for(p, m->loop_in, j.NT);
+            j.ksplit = split_for(p, m->loop_in, split_blocks(p, j));
             j.epi = TLM_EPI_F32;
             j.out = m->mix;
             j.out_ld = m->ld;
@@ -1489,11 +1515,15 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
         TlmJobs J;
         memset(&J, 0, sizeof(J));
         c = Carry();
+        TlmJob o = dense_job(*mo.w, mo.x, mo.xks, T);
+        const int others = p.rows ? 0 : tile_blocks(p, o);
         if (moe || dense) {
             TlmJob& j = J.j[J.n++];
             c.top = moe ? L.c.top : 1;
             j = moe ? routed_job(m, L, L.down, m->hid, L.down.KS, 1, T, p) : dense_job(L.down, m->hid, L.down.KS, T);
-            j.ksplit = split_for(p, L.down, j.NT * (moe ? j.rblocks : 1));
+            const int mine = split_blocks(p, j);
+            j.ksplit = split_for(p, L.down, mine + others);
+            if (!p.rows) o.ksplit = split_for(p, *mo.w, mine + others);
             j.epi = TLM_EPI_F32;
             j.out = m->dn;
             j.out_ld = m->ld;
@@ -1501,16 +1531,17 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
             c.dn = m->dn;
             c.dn_p = j.ksplit;
             c.ls2 = L.ls2;
+        } else if (!p.rows) {
+            o.ksplit = split_for(p, *mo.w, others);
         }
-        TlmJob& j = J.j[J.n++];
-        j = dense_job(*mo.w, mo.x, mo.xks, T);
-        j.ksplit = split_for(p, *mo.w, j.NT);
-        j.epi = TLM_EPI_F32;
-        j.out = m->mix;
-        j.out_ld = m->ld;
-        j.out_ps = (long)T * m->ld;
+        if (p.rows) o.ksplit = split_for(p, *mo.w, o.NT);
+        o.epi = TLM_EPI_F32;
+        o.out = m->mix;
+        o.out_ld = m->ld;
+        o.out_ps = (long)T * m->ld;
+        J.j[J.n++] = o;
         c.mix = m->mix;
-        c.mix_p = j.ksplit;
+        c.mix_p = o.ksplit;
         c.ls1 = L.ls1;
         P.site(site + "out");
         add_jobs(m, P, p, J, mo.w->bytes() + (dense ? L.down.bytes() : 0));
@@ -1526,7 +1557,7 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
         nm.w = m->final_norm;
         nm.out = m->h;
         add_resid(m, P, sh, c, TLM_EMB_NONE, nullptr, nm, m->meta + sh.m.want, sh.n_want);
-        const Plan hp = plan_rows(sh.n_want);
+        const Plan hp = plan_rows(sh.n_want, false);
         TlmJobs J;
         memset(&J, 0, sizeof(J));
         TlmJob& j = J.j[J.n++];

@@ -545,24 +545,33 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
     });
 }
 
-// Many rows: 2 x 2 waves over a tile of 32 FN features x 32 FM rows, SK k-steps per stage, double-buffered in LDS, with the loads of the
-// two stages after the current one in flight in registers.  Operands arrive as whole fragments (one 16-byte vector per lane), so
-// staging and operand reads are conflict-free without a swizzle.
-template <class Tr, int FN, int FM, int SK>
-__global__ __launch_bounds__(256, 2) void k_tlm_gemm_tile(TlmJobs jobs) {
-    constexpr int NF = 2 * FN + 2 * FM, NI = NF / 4;          // fragments per k-step; per wave
-    MMI_SHARED __attribute__((aligned(16))) u32x4 lds[2 * SK * NF * 64];
+// Many rows: WN x WM waves, each over FN x FM fragments, i.e. 16 FN WN features x 16 FM WM rows per workgroup.  Operands go from global
+// memory straight into a ring of ST stages of one k-step in LDS (whole fragments, so that both sides are conflict-free without a swizzle),
+// ST - 2 stages ahead of the step that reads them into registers, which is one step ahead of the products that use them: a step is one
+// meeting of the waves, its loads and LDS reads lie between the products of the step before.
+template <class Tr, int FN, int FM, int WN, int WM, int ST>
+struct TlmTile {
+    static constexpr int NW = WN * WM, NFN = WN * FN, NFM = WM * FM, NF = NFN + NFM, NIN = NFN / NW, NIM = NFM / NW, NI = NIN + NIM;
+    static_assert(NFN % NW == 0 && NFM % NW == 0 && ST >= 3, "every wave brings whole fragments");
+    static constexpr size_t smem() { return (size_t)ST * NF * 1024; }
+};
+template <class Tr, int FN, int FM, int WN, int WM, int ST, int OCC>
+__global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs jobs) {
+    typedef TlmTile<Tr, FN, FM, WN, WM, ST> P;
+    MMI_DYN_SHARED(u32x4, lds);
     // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous run of tiles so that its L2 sees the shared operand
     const int nb = (int)gridDim.x, xper = nb >> 3, xrem = nb & 7, xcd = (int)blockIdx.x & 7;
     int b = xcd * xper + (xcd < xrem ? xcd : xrem) + ((int)blockIdx.x >> 3), ji = 0;
     while (ji + 1 < jobs.n && b >= jobs.j[ji].blocks) b -= jobs.j[ji++].blocks;
     const TlmJob j = jobs.j[ji];             // (a copy: its fields live in scalar registers)
     const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15;
-    const int ntb = (j.NT + 2 * FN - 1) / (2 * FN);
-    int g, rb, nb0, n, r0;
+    const int ntb = (j.NT + P::NFN - 1) / P::NFN;
+    int g, rb, nb0, n, r0, split = 0;
     if (j.list) {
         nb0 = b % ntb;
-        rb = b / ntb;
+        b /= ntb;
+        split = b % j.ksplit;
+        rb = b / j.ksplit;
         if (rb >= *j.n_tiles) return;
         g = j.tiles[3 * rb];
         r0 = j.tiles[3 * rb + 1];
@@ -571,73 +580,97 @@ __global__ __launch_bounds__(256, 2) void k_tlm_gemm_tile(TlmJobs jobs) {
         rb = b % j.rblocks;
         b /= j.rblocks;
         nb0 = b % ntb;
-        g = b / ntb;
-        r0 = rb * 32 * FM;
-        n = j.rows - r0 < 32 * FM ? j.rows - r0 : 32 * FM;
+        b /= ntb;
+        split = b % j.ksplit;
+        g = b / j.ksplit;
+        r0 = rb * 16 * P::NFM;
+        n = j.rows - r0 < 16 * P::NFM ? j.rows - r0 : 16 * P::NFM;
     }
-    const int nt0 = nb0 * 2 * FN;
-    const u32x4* wbase = j.wp + (long)g * j.wgs;
-    int off[NI];                                              // fragment i of this wave, lane: 16-byte vectors from its operand's base
+    const int nt0 = nb0 * P::NFN, sper = (j.KS + j.ksplit - 1) / j.ksplit, k0 = min(j.KS, split * sper), ns = min(j.KS, k0 + sper) - k0;
+    // fragment i of this wave: weights at a scalar address, activations (gathered rows) at one per lane
+    const u32x4 *wq[P::NIN], *xq[P::NIM];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const int f = wave + 4 * i;
-        if (4 * i < 2 * FN) {
-            const int nt = nt0 + f < j.NT ? nt0 + f : j.NT - 1;
-            off[i] = nt * j.KS * 64 + lane;
-        } else {
-            const int m = (f - 2 * FN) * 16 + bl, ii = m < n ? m : n - 1;
-            const int id = j.list ? j.list[r0 + ii] : r0 + ii;
-            const long in = j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd;
-            off[i] = (int)((in >> 4) * j.xks + (long)g * j.xkg) * 64 + (int)(in & 15) + (lane >> 4) * 16;
-        }
+    for (int i = 0; i < P::NIN; ++i) wq[i] = j.wp + (long)g * j.wgs + ((long)min(nt0 + wave + P::NW * i, j.NT - 1) * j.KS + k0) * 64;
+#pragma unroll
+    for (int i = 0; i < P::NIM; ++i) {                        // (rows past n repeat the last one, and are dropped at the end)
+        const int m = (wave + P::NW * i) * 16 + bl, ii = m < n ? m : n - 1;
+        const int id = j.list ? j.list[r0 + ii] : r0 + ii;
+        const long in = j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd;
+        xq[i] = j.xp + ((in >> 4) * j.xks + (long)g * j.xkg + k0) * 64 + (in & 15) + (lane >> 4) * 16;
     }
-    const int wn = wave & 1, wm = wave >> 1;
+    int to = 0;                                               // the stage's place in the ring, for the next load and the next read
+    int from = 0;
+    auto fetch = [&](int i) __attribute__((always_inline)) {
+        const int at = (to * P::NF + wave + P::NW * i) * 64;
+        if (i < P::NIN) {
+            mmi_load_lds(wq[i < P::NIN ? i : 0], lane * 16, lds, at);
+            wq[i < P::NIN ? i : 0] += 64;
+        } else {
+            mmi_load_lds(xq[i < P::NIN ? 0 : i - P::NIN], lds, at);
+            xq[i < P::NIN ? 0 : i - P::NIN] += 64;
+        }
+    };
+    auto fetch_all = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < P::NI; ++i) fetch(i);
+        to = to + 1 < ST ? to + 1 : 0;
+    };
+    const int wn = wave % WN, wm = wave / WN;
+    u32x4 av[2][FN], bv[2][FM];
     f32x4 acc[FN][FM];
 #pragma unroll
     for (int x = 0; x < FN; ++x)
 #pragma unroll
         for (int y = 0; y < FM; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-    u32x4 st[2][SK][NI];
-#define TLM_FETCH(set, stage)                                                                   \
-    _Pragma("unroll") for (int kk = 0; kk < SK; ++kk) {                                         \
-        const int k_ = (stage) * SK + kk < j.KS ? (stage) * SK + kk : j.KS - 1;                 \
-        _Pragma("unroll") for (int i = 0; i < NI; ++i) st[set][kk][i] = (4 * i < 2 * FN ? wbase : j.xp)[(unsigned)(off[i] + k_ * 64)];  \
-    }
-#define TLM_STAGE(set, buf)                                                                     \
-    _Pragma("unroll") for (int kk = 0; kk < SK; ++kk)                                           \
-        _Pragma("unroll") for (int i = 0; i < NI; ++i) lds[(((buf) * SK + kk) * NF + wave + 4 * i) * 64 + lane] = st[set][kk][i];
-#define TLM_COMPUTE(buf, stage)                                                                 \
-    _Pragma("unroll") for (int kk = 0; kk < SK; ++kk)                                           \
-        if ((stage) * SK + kk < j.KS) {                                                         \
-            const u32x4* base = lds + (((buf) * SK + kk) * NF) * 64 + lane;                     \
-            u32x4 bv[FM];                                                                       \
-            _Pragma("unroll") for (int y = 0; y < FM; ++y) bv[y] = base[(2 * FN + wm * FM + y) * 64]; \
-            _Pragma("unroll") for (int x = 0; x < FN; ++x) {                                    \
-                const u32x4 av = base[(wn * FN + x) * 64];                                      \
-                _Pragma("unroll") for (int y = 0; y < FM; ++y) acc[x][y] = Tr::mfma(av, bv[y], acc[x][y]); \
-            }                                                                                   \
+    auto read = [&](int set, int i) __attribute__((always_inline)) {      // fragment i of FN + FM: rows first, they meet every feature
+        const u32x4* base = lds + from * P::NF * 64 + lane;
+        if (i < FM) bv[set][i < FM ? i : 0] = base[(P::NFN + wm * FM + i) * 64];
+        else av[set][i < FM ? 0 : i - FM] = base[(wn * FN + i - FM) * 64];
+    };
+    auto wait = [&](int behind) __attribute__((always_inline)) {          // until only the last `behind` stages are in flight
+        if (ST > 4 && behind >= 3) { if (ST > 5 && behind >= 4) mmi_wait_loads<(ST > 5 ? 4 : 0) * P::NI>(); else mmi_wait_loads<(ST > 4 ? 3 : 0) * P::NI>(); }
+        else if (ST > 3 && behind == 2) mmi_wait_loads<(ST > 3 ? 2 : 0) * P::NI>();
+        else if (behind == 1) mmi_wait_loads<P::NI>();
+        else mmi_wait_loads<0>();
+    };
+    // products of stage s (register set `cur`); between them the loads of stage s + ST - 1 and the LDS reads of stage s + 1
+    auto step = [&](auto set, int s) __attribute__((always_inline)) {
+        constexpr int cur = decltype(set)::value;
+        const bool more = s + 1 < ns, load = s + ST - 1 < ns;
+        if (more) {
+            wait(min(ns - 1, s + ST - 2) - (s + 1));
+            mmi_meet();
         }
-    // (fetches past the end repeat the last k-step: an unconditional load keeps the wait in front of a stage to the older set)
-    const int ns = (j.KS + SK - 1) / SK;
-    TLM_FETCH(0, 0);
-    TLM_FETCH(1, 1);
-    TLM_STAGE(0, 0);
-    __syncthreads();
-    for (int s = 0; s < ns; s += 2) {                         // stage s in buffer 0 and register set 0, stage s + 1 in 1 and 1
-        TLM_FETCH(0, s + 2);
-        mmi_sched_barrier();
-        TLM_COMPUTE(0, s);
-        TLM_STAGE(1, 1);
-        __syncthreads();
-        TLM_FETCH(1, s + 3);
-        mmi_sched_barrier();
-        TLM_COMPUTE(1, s + 1);
-        TLM_STAGE(0, 0);
-        __syncthreads();
+        if (load) fetch_all();
+#pragma unroll
+        for (int x = 0; x < FN; ++x) {
+            if (more) {
+#pragma unroll
+                for (int i = x * (FN + FM) / FN; i < (x + 1) * (FN + FM) / FN; ++i) read(cur ^ 1, i);
+            }
+            mmi_sched_barrier();
+#pragma unroll
+            for (int y = 0; y < FM; ++y) acc[x][y] = Tr::mfma(av[cur][x], bv[cur][y], acc[x][y]);
+        }
+        from = from + 1 < ST ? from + 1 : 0;
+    };
+    if (ns > 0) {
+        const int first = min(ns, ST - 1);
+        for (int s = 0; s < first; ++s) fetch_all();
+        wait(first - 1);
+        mmi_meet();
+#pragma unroll
+        for (int i = 0; i < FN + FM; ++i) read(0, i);
+        from = 1;
+        int s = 0;
+#pragma unroll 1
+        for (; s + 1 < ns; s += 2) {
+            step(std::integral_constant<int, 0>(), s);
+            step(std::integral_constant<int, 1>(), s + 1);
+        }
+        if (s < ns) step(std::integral_constant<int, 0>(), s);
     }
-#undef TLM_COMPUTE
-#undef TLM_FETCH
-#undef TLM_STAGE
+    __syncthreads();
     tlm_with_epilogue(j.epi, [&](auto epi) __attribute__((always_inline)) {
 #pragma unroll
         for (int y = 0; y < FM; ++y) {
@@ -650,7 +683,7 @@ __global__ __launch_bounds__(256, 2) void k_tlm_gemm_tile(TlmJobs jobs) {
             for (int x = 0; x < FN; ++x) buf[x * 64] = acc[x][y];
             const int nx = min(FN, j.NT - nt0 - wn * FN);
 #pragma unroll 1
-            for (int x = 0; x < nx; ++x) tlm_epilogue<Tr, decltype(epi)::value>(j, g, 0, id, nt0 + wn * FN + x, lane >> 4, buf[x * 64]);
+            for (int x = 0; x < nx; ++x) tlm_epilogue<Tr, decltype(epi)::value>(j, g, split, id, nt0 + wn * FN + x, lane >> 4, buf[x * 64]);
         }
     });
 }

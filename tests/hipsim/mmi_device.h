@@ -347,6 +347,11 @@ inline void mmi_store_relaxed_agent(unsigned* p, unsigned v) { __atomic_store_n(
 inline void mmi_sched_barrier() {}
 inline int mmi_uniform(int v) { return v; }
 inline bool mmi_any(bool v) { unsigned x = v ? 1u : 0u; for (int m = 1; m < 64; m <<= 1) { const unsigned o = mmi_shfl_xor(x, m); x = o > x ? o : x; } return x != 0; }
+inline void mmi_load_lds(const void* base, unsigned off, u32x4* lds, int at) { lds[at + (int)(threadIdx.x & 63)] = *(const u32x4*)((const char*)base + off); }
+inline void mmi_load_lds(const u32x4* from, u32x4* lds, int at) { lds[at + (int)(threadIdx.x & 63)] = *from; }
+template <int N>
+inline void mmi_wait_loads() {}
+inline void mmi_meet() { __syncthreads(); }
 inline u32x4 mmi_load_nt(const u32x4* p) { return *p; }
 inline f32x4 mmi_load_nt(const f32x4* p) { return *p; }
 inline void mmi_store_nt(f32x4* p, f32x4 v) { *p = v; }
