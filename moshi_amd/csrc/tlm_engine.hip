@@ -133,7 +133,7 @@ struct mmi_tlm {
     float *x = nullptr, *mix = nullptr, *dn = nullptr, *zcg = nullptr, *lat = nullptr, *gate = nullptr, *pair = nullptr, *po = nullptr, *pml = nullptr;
     float *lin = nullptr, *qkv = nullptr, *dec = nullptr, *lgate = nullptr, *lo = nullptr, *cw = nullptr, *cq_g = nullptr, *ckt = nullptr, *cu0 = nullptr, *cp = nullptr,
           *cgend = nullptr;
-    void *h2 = nullptr, *cat = nullptr, *lr = nullptr;
+    void *hrow = nullptr, *h2 = nullptr, *cat = nullptr, *lr = nullptr;
     int *brow = nullptr, *prev_tok = nullptr;
     void *h = nullptr, *y = nullptr, *cq = nullptr, *qn = nullptr, *q = nullptr, *ao = nullptr, *o = nullptr, *hid = nullptr;
     int *list = nullptr, *tiles = nullptr, *n_tiles = nullptr, *tok = nullptr, *meta = nullptr, *last_tok = nullptr, *block_table = nullptr;
@@ -695,7 +695,7 @@ int alloc_buffers(mmi_tlm* m) {
         const size_t nl = m->route_host.size();
         m->list_ld = (long)T * m->max_top;
         m->tile_ld = (long)T * m->max_top / 16 + m->max_experts + 1;
-        if ((rc = alloc_packed(m, &m->hid, (long)T * m->max_top, hid_ks)) ||
+        if ((rc = alloc_packed(m, &m->hrow, T, m->h_ks)) || (rc = alloc_packed(m, &m->hid, (long)T * m->max_top, hid_ks)) ||
             (rc = alloc_f32(m, &m->dn, split_room(m->max_top, m->ld))))
             return rc;
         MMI_HIP_CHECK(m->scratch.alloc(&m->list, nl * m->list_ld));
@@ -954,6 +954,7 @@ struct Carry {                    // what the next residual launch has to add
 struct Norms {                    // what it leaves behind: one or two normalised operands, or (raw) the residual itself as an operand
     const float* w = nullptr; void* out = nullptr;
     const float* w2 = nullptr; void* out2 = nullptr;
+    void* rows = nullptr;         // what experts gather, row-major
     void* raw = nullptr;
 };
 
@@ -986,6 +987,8 @@ void add_resid(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Carry& c, int e
     a.w = o.w;
     a.w2 = o.w2;
     a.out2 = o.out2;
+    a.rows_out = o.rows;
+    a.rows_ld = m->h_ks * m->kstep;
     a.raw = o.raw;
     a.raw_ks = 2 * m->h_ks;
     if (emb_mode == TLM_EMB_SET) a.emb_out = m->cat;
@@ -1488,13 +1491,16 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
             nm.w2 = L.norm2;
             nm.out2 = hf = m->h2;
         }
+        if (moe) nm.rows = m->hrow;
         P.site(site + "norm");
         add_resid(m, P, sh, c, emb, tap, nm, nullptr, T);
         TlmJobs first;
         memset(&first, 0, sizeof(first));
         if (moe) {
             TlmJob& j = first.j[first.n++];
-            j = routed_job(m, L, L.up, hf, m->h_ks, L.c.top, T, p);
+            j = routed_job(m, L, L.up, m->hrow, m->h_ks, L.c.top, T, p);
+            j.xrow = 1;
+            j.out_pos = 1;
             j.epi = TLM_EPI_PACK;
             j.act = TLM_ACT_RELU2;
             j.out = m->hid;
@@ -1521,6 +1527,7 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
             TlmJob& j = J.j[J.n++];
             c.top = moe ? L.c.top : 1;
             j = moe ? routed_job(m, L, L.down, m->hid, L.down.KS, 1, T, p) : dense_job(L.down, m->hid, L.down.KS, T);
+            j.in_pos = moe;
             const int mine = split_blocks(p, j);
             j.ksplit = split_for(p, L.down, mine + others);
             if (!p.rows) o.ksplit = split_for(p, *mo.w, mine + others);

@@ -213,6 +213,7 @@ struct TlmResidArgs {
     const float* w; int groups; float eps;
     void* out; int KS;                   // packed; null: no norm
     const float* w2; void* out2;
+    void* rows_out; int rows_ld;         // what the feed-forward reads (the second operand if there is one), row-major, or null
     void* raw; int raw_ks;               // packed x, or null
     void* emb_out; int emb_k0;           // TLM_EMB_SET: packed copy of the embedding from column emb_k0 of rows of raw_ks k-steps, or null
     const int* rows;                     // row list (the residual is then not written back), or null
@@ -295,6 +296,7 @@ __global__ __launch_bounds__(1024) void k_tlm_resid_norm(TlmResidArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = k + q < a.width ? v[q] * inv[(k + q) / gs] : 0.f;
         Tr::store4(out + tlm_index<Tr>(blockIdx.x, k, a.KS), v * w);
+        if (a.rows_out) Tr::store4((typename Tr::elem*)a.rows_out + (long)blockIdx.x * a.rows_ld + k, v * (a.out2 ? *reinterpret_cast<const f32x4*>(a.w2 + k) : w));
         if (a.out2) Tr::store4((typename Tr::elem*)a.out2 + tlm_index<Tr>(blockIdx.x, k, a.KS), v * *reinterpret_cast<const f32x4*>(a.w2 + k));
     }
 }
@@ -321,6 +323,10 @@ struct TlmJob {
     const int* tiles;
     const int* n_tiles;
     int in_div;
+    // routed: rows by their place in the list instead of by pair (activations in / out): the experts' hidden rows lie in the order in which
+    // the down projection reads them, so that nothing is gathered there.  xrow: the activations are row-major (their k-steps xks wide), for
+    // gathered rows: of a fragment-packed matrix a row's k-step is four pieces in four cache lines shared with seven other rows
+    int in_pos, out_pos, xrow;
     int epi, act, act_nt;                // SILU: the first act_nt tiles
     void* out; int out_ld; long out_ps;  // fp32: row stride, stride per K split; packed: k-steps per row tile
     int out_mul, out_gadd, out_k0, out_kg;
@@ -434,6 +440,11 @@ __device__ __forceinline__ void tlm_with_epilogue(int epi, F f) {
     else f(TlmEpi<TLM_EPI_LOGITS>());
 }
 
+// k-step 0 of activation row `in` for a lane
+__device__ __forceinline__ const u32x4* tlm_row(const TlmJob& j, long in, int g, int lane) {
+    return j.xp + (j.xrow ? in * j.xks * 4 + (lane >> 4) : ((in >> 4) * j.xks + (long)g * j.xkg) * 64 + (in & 15) + (lane >> 4) * 16);
+}
+
 // Few rows (<= 16 MT per block): the weights are an HBM stream.  A workgroup owns NTW n-tiles; its waves split K, each with U k-steps
 // of weight fragments in flight per register buffer; partial tiles are summed through LDS in a fixed order.  Every activation fragment
 // (an L2 read) meets NTW weight fragments, so that with many rows the activations do not cost more than the weights.
@@ -461,9 +472,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
     for (int m = 0; m < MT; ++m) {
         const int i = m * 16 + bl < n ? m * 16 + bl : n - 1;
         const int id = j.list ? j.list[r0 + i] : r0 + i;
-        const long in = j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd;
-        xq[m] = j.xp + ((in >> 4) * j.xks + (long)g * j.xkg) * 64 + (in & 15) + (lane >> 4) * 16;
+        const long in = j.in_pos ? r0 + i : (j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd);
+        xq[m] = tlm_row(j, in, g, lane);
     }
+    const int xs = j.xrow ? 4 : 64;
     // K range of this split, then of this wave
     const int sper = (j.KS + j.ksplit - 1) / j.ksplit;
     const int s0 = min(j.KS, split * sper), s1 = min(j.KS, s0 + sper);
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
 #define TLM_LOAD(W_, X_, base)                                                                              \
     _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                         \
         _Pragma("unroll") for (int t = 0; t < NTW; ++t) W_[u][t] = mmi_load_nt(wq[t] + (long)((base) + u) * 64); \
-        _Pragma("unroll") for (int m = 0; m < MT; ++m) X_[u][m] = xq[m][(long)(k0 + (base) + u) * 64];      \
+        _Pragma("unroll") for (int m = 0; m < MT; ++m) X_[u][m] = xq[m][(long)(k0 + (base) + u) * xs];      \
     }
 #define TLM_MMA1(W_, X_, u)                                                                                 \
         _Pragma("unroll") for (int m = 0; m < MT; ++m)                                                      \
@@ -517,7 +529,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
 #pragma unroll
             for (int t = 0; t < NTW; ++t) wA[u][t] = mmi_load_nt(wq[t] + (long)k * 64);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) xA[u][m] = xq[m][(long)(k0 + k) * 64];
+            for (int m = 0; m < MT; ++m) xA[u][m] = xq[m][(long)(k0 + k) * xs];
         }
 #pragma unroll
         for (int u = 0; u < U - 1; ++u)
@@ -540,7 +552,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
             f32x4 v = red[q * 64 + lane];
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) v += red[(w * NTW * MT + q) * 64 + lane];
-            tlm_epilogue<Tr, decltype(epi)::value>(j, g, split, j.list ? j.list[r0 + i] : r0 + i, nt0 + t, lane >> 4, v);
+            tlm_epilogue<Tr, decltype(epi)::value>(j, g, split, j.list && !j.out_pos ? j.list[r0 + i] : r0 + i, nt0 + t, lane >> 4, v);
         }
     });
 }
@@ -549,6 +561,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
 // memory straight into a ring of ST stages of one k-step in LDS (whole fragments, so that both sides are conflict-free without a swizzle),
 // ST - 2 stages ahead of the step that reads them into registers, which is one step ahead of the products that use them: a step is one
 // meeting of the waves, its loads and LDS reads lie between the products of the step before.
+// Bound by the matrix core's power (it runs at 0.95 - 1.2 PFLOP/s where a 16384^3 library product reaches 1.29) and, with few blocks, by
+// the latency of a step (0.3 - 0.56 us).  Against the same tiles staged through registers: 1773 x 38912 x 4096 602 -> 543 us, 1773 x 4096 x
+// (11264 + 4096) 263 -> 203.
 template <class Tr, int FN, int FM, int WN, int WM, int ST>
 struct TlmTile {
     static constexpr int NW = WN * WM, NFN = WN * FN, NFM = WM * FM, NF = NFN + NFM, NIN = NFN / NW, NIM = NFM / NW, NI = NIN + NIM;
@@ -595,9 +610,10 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
     for (int i = 0; i < P::NIM; ++i) {                        // (rows past n repeat the last one, and are dropped at the end)
         const int m = (wave + P::NW * i) * 16 + bl, ii = m < n ? m : n - 1;
         const int id = j.list ? j.list[r0 + ii] : r0 + ii;
-        const long in = j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd;
-        xq[i] = j.xp + ((in >> 4) * j.xks + (long)g * j.xkg + k0) * 64 + (in & 15) + (lane >> 4) * 16;
+        const long in = j.in_pos ? r0 + ii : (j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd);
+        xq[i] = tlm_row(j, in, g, lane) + (long)k0 * (j.xrow ? 4 : 64);
     }
+    const int xs = j.xrow ? 4 : 64;
     int to = 0;                                               // the stage's place in the ring, for the next load and the next read
     int from = 0;
     auto fetch = [&](int i) __attribute__((always_inline)) {
@@ -607,7 +623,7 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
             wq[i < P::NIN ? i : 0] += 64;
         } else {
             mmi_load_lds(xq[i < P::NIN ? 0 : i - P::NIN], lds, at);
-            xq[i < P::NIN ? 0 : i - P::NIN] += 64;
+            xq[i < P::NIN ? 0 : i - P::NIN] += xs;
         }
     };
     auto fetch_all = [&]() __attribute__((always_inline)) {
@@ -676,7 +692,7 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
         for (int y = 0; y < FM; ++y) {
             const int m = (wm * FM + y) * 16 + bl;
             if (m >= n) continue;
-            const int id = j.list ? j.list[r0 + m] : r0 + m;
+            const int id = j.list && !j.out_pos ? j.list[r0 + m] : r0 + m;
             // through LDS (a lane reads what it wrote), so that the epilogue's code is there once per y and not once per tile
             f32x4* buf = reinterpret_cast<f32x4*>(lds) + wave * FN * 64 + lane;
 #pragma unroll

@@ -1,0 +1,43 @@
+"""Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 64, 128 x 64, 128 x 128 in three and four stages, 256 x 128, whole
+and split reductions, gathered and listed expert rows - at row counts just past a tile and sizes that are no multiples of one: a prompt fed at
+once must give the logits that the same prompt gives in portions of at most 64 tokens, which take the weight-streaming kernel."""
+import pytest
+import torch
+
+from moshi_amd.config import (DenseGLUConfig, GroupedAttentionConfig, LatentAttentionConfig, MinGRUConfig, MoEConfig, TokenLayerConfig, TokenLMConfig)
+from moshi_amd.tlm import TokenLM
+from moshi_amd.weights import random_token_lm_state_dict
+
+
+def experts_model(width, ff):
+    att = LatentAttentionConfig(heads=4, dim=64, vdim=64, rot_dim=32, q_rank=200, kv_rank=120, scale=0.1)
+    moe = MoEConfig(experts=5, top=2, ff=ff)
+    return TokenLMConfig("Kesirax", vocab=331, width=width, layers=[TokenLayerConfig(MinGRUConfig(width + 16), moe), TokenLayerConfig(att, moe)])
+
+
+def dense_model(width, ff):
+    att = GroupedAttentionConfig(heads=8, kv_heads=2, dim=64, vdim=64, scale=0.125)
+    return TokenLMConfig("Bibapel", vocab=331, width=width, layers=[TokenLayerConfig(att, DenseGLUConfig(ff=ff, limit=7.0))], norms=2, layer_scales=False, tied_head=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("model,T", [
+    (experts_model(208, 144), 65), (experts_model(528, 400), 130),                    # 64 x 64
+    (dense_model(1040, 4000), 577), (dense_model(1040, 1200), 641),                   # 128 x 64; 128 x 128 in four stages
+    (experts_model(1040, 2064), 1025), (dense_model(1040, 6000), 1157)                # 128 x 128 in three, 256 x 128
+], ids=["65", "130", "577", "641", "1025", "1157"])
+def test_prompt_at_once_equals_portions(model, T, dtype):
+    sd = random_token_lm_state_dict(model, seed=T, device="cuda")
+    lm = TokenLM(sd, model, dtype=dtype, max_slots=2, max_tokens=4096, max_step_tokens=T)
+    prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
+    want = sorted({0, 15, 16, 63, 64, T // 2, T - 2, T - 1})
+    a = lm.open()
+    whole = lm.step([(a, prompt, want)])
+    assert "k_tlm_gemm_tile" in {k for _, k, _ in lm.launch_list()}
+    b = lm.open()
+    parts = torch.cat([lm.step([(b, prompt[i:i + 64], [w - i for w in want if i <= w < i + 64])]) for i in range(0, T, 64)])
+    rel = float((whole - parts).double().norm() / parts.double().norm())
+    # fp32: sums of up to 6000 products in another order, over a handful of layers (eps sqrt(6000) ~ 5e-6); bf16: an activation on the other
+    # side of a rounding boundary here and there (2^-9 each)
+    assert rel < (1e-5 if dtype == torch.float32 else 8e-3), rel
