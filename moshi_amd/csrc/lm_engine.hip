@@ -1671,13 +1671,8 @@ extern "C" int mmi_lm_step(mmi_lm* lm, const int64_t* user_codes, int32_t n_user
     MMI_LAUNCH(k_i32_to_i64, mmi_cdiv(B * (c.dep_q + 1), 256), 256, 0, s, (const int*)lm->out_i32, (long*)out_tokens, B * (c.dep_q + 1));
     if (opt_text_logits)
         MMI_LAUNCH(k_bf16_to_f32, (int)mmi_cdiv64((int64_t)B * c.text_card_out, 256), 256, 0, s, (const uint16_t*)lm->text_logits, opt_text_logits, (long)B * c.text_card_out);
-    if (opt_audio_logits) {
-        // internal layout [dep_q][B][card] -> caller's [B][dep_q][card]
-        for (int k = 0; k < c.dep_q; ++k)
-            for (int b = 0; b < B; ++b)
-                MMI_LAUNCH(k_bf16_to_f32, mmi_cdiv(c.card, 256), 256, 0, s, (const uint16_t*)(lm->dlogits + ((size_t)k * lm->batch + b) * c.card),
-                           opt_audio_logits + ((size_t)b * c.dep_q + k) * c.card, (long)c.card);
-    }
+    if (opt_audio_logits && c.dep_q > 0)
+        MMI_LAUNCH(k_audio_logits, dim3(c.dep_q, B), 256, 0, s, (const uint16_t*)lm->dlogits, lm->batch, opt_audio_logits, c.card);
     MMI_CHECK_LAUNCH();
     if (lm->forced_armed) {   // forcing applies to one step only
         MMI_HIP_CHECK(hipMemsetAsync(lm->use_forced, 0, sizeof(int), s));
