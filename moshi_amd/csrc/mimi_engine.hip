@@ -105,7 +105,7 @@ struct DequantScratch {
 // columns, so that a launch is worth its latency.  The streaming state stays where the frame program keeps it: the histories are copied
 // in front of the group's rows before its launches and back behind them, everything else is shared.
 // Measured on one stream, 129 frames encoded and decoded (10.3 s of audio): 140 ms frame by frame (176 dependent launches per frame, most of
-// them at the ~4.7 us a dependent launch costs), 7.9 ms in three groups of 43.
+// them at the ~4.7 us a dependent launch costs), 7.9 ms in three groups of 43, 5.9 ms in one of 129.
 struct MimiGroup {
     int frames = 0;                            // 0: not built (for this stream)
     bool refused = false;                      // building failed (shapes, memory): this stream goes frame by frame
@@ -346,24 +346,27 @@ struct ConvPlan {
     bool ln = false;                  // k_gemm_f32_ln: LayerNorm fused in front of the linear
     bool wide = false;
     int MTB = 1, W = 1;               // wide
+    bool group = false;
     int NSUB = 1, waves = 4, ksplit = 1, nz = 1;
     bool pack = false;
 };
 
-template <int MTB, int U, bool ELU_IN>
+template <int MTB, int U, bool ELU_IN, bool GROUP>
 void launch_wide_e(hipStream_t s, const ConvGemmArgs& a, int W, dim3 grid) {
     const size_t smem = (size_t)W * MTB * 16 * 64 * sizeof(float);
     switch (W) {
-        case 1: MMI_LAUNCH((k_conv_wide<MTB, 1, U, ELU_IN>), grid, 64, 0, s, a); break;
-        case 2: MMI_LAUNCH((k_conv_wide<MTB, 2, U, ELU_IN>), grid, 128, smem, s, a); break;
-        case 4: MMI_LAUNCH((k_conv_wide<MTB, 4, U, ELU_IN>), grid, 256, smem, s, a); break;
-        default: MMI_LAUNCH((k_conv_wide<MTB, 8, U, ELU_IN>), grid, 512, smem, s, a); break;
+        case 1: MMI_LAUNCH((k_conv_wide<MTB, 1, U, ELU_IN, GROUP>), grid, 64, 0, s, a); break;
+        case 2: MMI_LAUNCH((k_conv_wide<MTB, 2, U, ELU_IN, GROUP>), grid, 128, smem, s, a); break;
+        case 4: MMI_LAUNCH((k_conv_wide<MTB, 4, U, ELU_IN, GROUP>), grid, 256, smem, s, a); break;
+        default: MMI_LAUNCH((k_conv_wide<MTB, 8, U, ELU_IN, GROUP>), grid, 512, smem, s, a); break;
     }
 }
 template <int MTB, int U>
-void launch_wide_w(hipStream_t s, const ConvGemmArgs& a, int W, dim3 grid) {
-    if (a.elu_in) launch_wide_e<MTB, U, true>(s, a, W, grid);      // ELU at the load (inputs nobody pre-activated)
-    else launch_wide_e<MTB, U, false>(s, a, W, grid);
+void launch_wide_w(hipStream_t s, const ConvGemmArgs& a, int W, bool group, dim3 grid) {
+    if (group && a.elu_in) launch_wide_e<MTB, U, true, true>(s, a, W, grid);
+    else if (group) launch_wide_e<MTB, U, false, true>(s, a, W, grid);
+    else if (a.elu_in) launch_wide_e<MTB, U, true, false>(s, a, W, grid);      // ELU at the load (inputs nobody pre-activated)
+    else launch_wide_e<MTB, U, false, false>(s, a, W, grid);
 }
 
 int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
@@ -372,9 +375,9 @@ int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
         ConvGemmArgs w = a;
         if (p.ksplit > 1) w.out_mode = MMI_GOUT_PARTIAL;
         switch (p.MTB) {
-            case 1: launch_wide_w<1, 4>(s, w, p.W, grid); break;
-            case 2: launch_wide_w<2, 4>(s, w, p.W, grid); break;
-            default: launch_wide_w<4, 2>(s, w, p.W, grid); break;
+            case 1: launch_wide_w<1, 4>(s, w, p.W, p.group, grid); break;
+            case 2: launch_wide_w<2, 4>(s, w, p.W, p.group, grid); break;
+            default: launch_wide_w<4, 2>(s, w, p.W, p.group, grid); break;
         }
         if (p.ksplit > 1) MMI_LAUNCH(k_conv_finish, (int)mmi_cdiv64((int64_t)a.Cout * a.Ntot, 256), 256, 0, s, a, p.ksplit);
         MMI_CHECK_LAUNCH();
@@ -498,16 +501,18 @@ void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
 // workgroup covers follows the group's own number of columns.
 int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
     const int N = a.Ntot, N1 = N / mem.frames;
-    if (a.Cin * a.K >= (1 << 17) || N >= (1 << 17) || a.K >= (1 << 11))
+    if (a.Cin * a.K >= (1 << 17) || N1 >= (1 << 17) || N >= (1 << 19) || a.K >= (1 << 11))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "conv dimensions outside the range of the kernels' index arithmetic (sessions x samples per frame "
                                              "must stay below 131072: 68 sessions per handle at 1920 samples per frame)");
-    if (N > 128) {
+    // (a group's layers that the frame program streams the weights of do so for several column groups, up to 512 columns)
+    if (N > (mem.frames > 1 && N1 <= 128 ? 512 : 128)) {
         if (a.first || a.x_packed || a.out_mode != MMI_GOUT_NATURAL)
             return mmi_fail(MMI_ERR_UNSUPPORTED, "more than 128 columns (sessions x time steps per frame) on a conv with replicate padding or packed "
                                                  "operands: lower max_batch (the 25 Hz layers of the released codec take 64 sessions)");
         p->wide = true;
         a.q_blk = a.Q;
         wide_rule(a, N1 > 128 ? N1 : N, &p->MTB, &p->W);
+        p->group = mem.frames > 1;
         if (mem.frames > 1) {
             if (N1 <= 128) {
                 gemm_rule(a, N1, p);
@@ -549,11 +554,10 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         ConvPlan f;
         gemm_rule(a, N1, &f);
         p->ksplit = f.ksplit;
-        if (f.waves == 8 && p->NSUB == 4) {          // (four subtiles of eight waves are not built)
-            p->NSUB = 2;
-            p->nz = mmi_cdiv(nsub, 2);
-        }
         p->waves = f.waves;
+        if (f.waves == 8 && p->NSUB == 4) p->NSUB = 2;          // (four subtiles of eight waves are not built)
+        p->nz = mmi_cdiv(nsub, p->NSUB);
+        a.Npad = p->nz * p->NSUB * 32;
     }
     if (!a.x_packed) {
         if (!a.bp) {
@@ -727,7 +731,7 @@ int add_dequant_ops(mmi_mimi* m, MimiMem& mem, const DequantScratch& d, MmiProgr
     const mmi_mimi_cfg& c = m->cfg;
     const int D = c.q_dimension, bins = c.q_bins, nq = c.q_n_q, nsem = c.q_n_q_semantic, rows = B * T;
     float* q2 = d.q2; const int* codes = d.codes; const float* E = m->E_all; const int* kdev = k_from_device ? m->dec_k_dev : nullptr;
-    const bool packed = rows <= 128 && m->q_out.Q * 8 == 2 * D && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    const bool packed = (rows <= 128 || T > 1) && m->q_out.Q * 8 == 2 * D && !getenv("MMI_MIMI_PACK_LAUNCHES");
     if (T > 1 && !packed) return mmi_fail(MMI_ERR_UNSUPPORTED, "dequantising several frames needs the packed operand");
     float* qp = packed ? d.qout_bp : nullptr; const int qQ = m->q_out.Q;
     prog.add([=](hipStream_t s) {
@@ -751,7 +755,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
     const int N = B * T;
     // At <= 128 columns (every real configuration: T = 2 per session) the linears run on k_gemm_f32 and the producers
     // (LayerNorm, attention, linear1+GELU) write its packed operand directly; otherwise plain [B][C][T] buffers.
-    const bool packed = N <= 128;
+    const bool packed = N <= 128 || frames > 1;
     Buf y, qkv, att, hb;
     int rc;
     if ((rc = alloc_buf(mem, B, d, 0, T, &y, init_stream))) return rc;
@@ -820,7 +824,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
                 MimiGroupRows gr;
                 gr.T = T; gr.qkv_ld = qkv.ld; gr.q = qr; gr.kn = kvn + 2 * l * rows_d; gr.vn = gr.kn + rows_d;
                 const int tpf = T / frames;
-                const dim3 grid_r(B * H, mmi_cdiv(T, 32)), grid_a(B * H, frames);
+                const dim3 grid_r(B * H, mmi_cdiv(T, MIMI_ROPE_T)), grid_a(B * H, frames);
                 prog.add([=](hipStream_t s) {
 #define MMI_ATT(D_, T_) do { MMI_LAUNCH((k_mimi_group_rope<D_>), grid_r, 256, 0, s, aa, gr); \
                              MMI_LAUNCH((k_mimi_attn_1pass<D_, T_, true>), grid_a, 256, 0, s, aa, gr); } while (0)
@@ -1024,7 +1028,7 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     if (T % stride != 0 || T / stride != frames)
         return mmi_fail(MMI_ERR_UNSUPPORTED, "frame_size must map to exactly one latent column");
     if ((rc = alloc_buf(mem, B, c.dimension, 0, frames, &lat, s0))) return rc;
-    const bool latent_packed = B * frames <= 128 && m->q_in.Q * 8 == c.dimension && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    const bool latent_packed = (B <= 128 || g) && m->q_in.Q * 8 == c.dimension && !getenv("MMI_MIMI_PACK_LAUNCHES");
     if (g && !latent_packed) return mmi_fail(MMI_ERR_UNSUPPORTED, "quantising several frames needs the packed operand");
     RvqScratch rs = m->rvq;
     if (g) {
@@ -1035,7 +1039,7 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         MMI_HIP_CHECK(mem.alloc(&rs.best_i, 2 * m->nchunk * n));
         MMI_HIP_CHECK(mem.alloc(&rs.codes, n * c.q_n_q));
         MMI_HIP_CHECK(mem.alloc(&rs.qin_bp, (size_t)mmi_cdiv((int)n, 32) * m->q_in.Q * 256));
-        MMI_HIP_CHECK(mem.alloc(&rs.qin_part, (size_t)8 * m->q_in.Mt * 32 * 128));
+        MMI_HIP_CHECK(mem.alloc(&rs.qin_part, (size_t)8 * m->q_in.Mt * 32 * mmi_cdiv((int)n, 128) * 128));
         g->codes = rs.codes;
     }
     {
@@ -1079,7 +1083,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         MMI_HIP_CHECK(mem.alloc(&ds.codes, n * c.q_n_q));
         MMI_HIP_CHECK(mem.alloc(&ds.q2, n * 2 * c.q_dimension));
         MMI_HIP_CHECK(mem.alloc(&ds.qout_bp, (size_t)mmi_cdiv((int)n, 32) * m->q_out.Q * 256));
-        MMI_HIP_CHECK(mem.alloc(&ds.qout_part, (size_t)8 * m->q_out.Mt * 32 * 128));
+        MMI_HIP_CHECK(mem.alloc(&ds.qout_part, (size_t)8 * m->q_out.Mt * 32 * mmi_cdiv((int)n, 128) * 128));
         g->codes = ds.codes;
     }
     if ((rc = add_dequant_ops(m, mem, ds, prog, m->n_codebooks, lat, 0, B, frames, /*k_from_device=*/true))) return rc;
@@ -1123,7 +1127,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         ConvGemmArgs a0 = conv_args(m->dec_convs[ci++], din, 0, T, cur, 0, B, false);
         // its (ELU'd) output is read by the first transposed-conv GEMM only: stored as that GEMM's packed operand as well
         const ConvW& wtr0 = m->dec_convs[ci];
-        if (B * T <= 128 && wtr0.Q * 8 == mult * c.n_filters && !getenv("MMI_MIMI_PACK_LAUNCHES")) {
+        if ((B * T <= 128 || g) && wtr0.Q * 8 == mult * c.n_filters && !getenv("MMI_MIMI_PACK_LAUNCHES")) {
             MMI_HIP_CHECK(mem.alloc(&conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256));
             MMI_HIP_CHECK(mem.zero(conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256, s0));
             a0.outp = conv0_bp; a0.outQ = wtr0.Q;
@@ -1186,8 +1190,8 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
 }
 
 // ---- groups of frames ---------------------------------------------------------------------------
-// Frames of the next group when `left` frames are to be run (1: frame by frame).  A group takes as many columns as the 25 Hz layers'
-// weight-streaming GEMMs hold (128, as for 64 streams), and what is left is cut into equal groups.  Not while the caller's stream is being
+// Frames of the next group when `left` frames are to be run (1: frame by frame).  A group takes up to 160 frames over all streams - the 25 Hz
+// layers then have 320 columns for weights that they read once, and its buffers about 1 GB - and what is left is cut into equal groups.  Not while the caller's stream is being
 // captured (a group's launch list is not kept for ever), and not under an exec mask (its rows would have to stand still frame by frame).
 int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left, hipStream_t s) {
     const mmi_mimi_cfg& c = m->cfg;
@@ -1195,7 +1199,7 @@ int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, in
     if (const char* e = getenv("MMI_MIMI_GROUP")) most = atoi(e);         // test hook: the largest group
     if (left < 2 || most < 2 || g.refused || !m->all_exec || tab.n < 0 || getenv("MMI_MIMI_PACK_LAUNCHES")) return 1;
     const int tpf = c.resample_stride, B = m->batch;
-    most = std::min(most, std::min(128 / (B * tpf), ((1 << 17) - 1) / (B * c.frame_size)));
+    most = std::min(most, std::min(std::min(160 / B, 512 / (B * tpf)), ((1 << 19) - 1) / (B * c.frame_size)));
     if (most < 2) return 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 1;

@@ -89,7 +89,7 @@ __global__ void k_codebook_prepare(const float* __restrict__ esum, const float* 
 //                k_pack_b_f32 (im2col + ELU + replicate padding) or by the producing kernel.
 enum { MMI_ACT_NONE = 0, MMI_ACT_GELU = 1, MMI_ACT_ELU = 2 };
 
-// n / d for 0 <= n < 2^17 and 1 <= d < 2^17 (column and tap indices) as one multiply-high and a shift: an integer division costs
+// n / d for 0 <= n < 2^20 and 1 <= d < 2^20 (column and tap indices) as one multiply-high and a shift: an integer division costs
 // ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^(32 + shift) / d), 0 means d == 1; exact while
 // n d < 2^(32 + shift), hence the 8 more bits (which still fit the magic number) from d = 2^11 on.
 MMI_HD unsigned mmi_div_shift(int d) { return d < (1 << 11) ? 0u : 8u; }
@@ -228,18 +228,20 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
     }
 }
 
-template <int MTB, int W, int U, bool ELU_IN = true>
+// GROUP: several frames of a stream at once - more columns per stream (T_shift), and the reduction also split over gridDim.z workgroups
+// where the frame program splits it (k_conv_finish adds their sums), cut as k_gemm_f32 cuts it
+template <int MTB, int W, int U, bool ELU_IN, bool GROUP>
 __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
+    const unsigned tsh = GROUP ? a.T_shift : 0u;
     const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
     const int jl = lane & 31, kh = lane >> 5;
     const int n = (int)blockIdx.x * 32 + jl;
     const int mt0 = (int)blockIdx.y * MTB;
     const bool nvalid = n < a.Ntot;
     const int nn = nvalid ? n : 0;
-    const int b = mmi_fast_div(nn, a.T_magic, a.T_shift), t = nn - b * a.T_out;
+    const int b = mmi_fast_div(nn, a.T_magic, tsh), t = nn - b * a.T_out;
     const float* xb = a.x + (long)b * a.x_bstride + a.x_off + t * a.S;
-    // gridDim.z > 1: the reduction is also split over workgroups (k_conv_finish adds their sums), cut as k_gemm_f32 cuts it
-    const int qb0 = min(a.Q, (int)blockIdx.z * a.q_blk), qb1 = min(a.Q, qb0 + a.q_blk);
+    const int qb0 = GROUP ? min(a.Q, (int)blockIdx.z * a.q_blk) : 0, qb1 = GROUP ? min(a.Q, qb0 + a.q_blk) : a.Q;
     const int qper = (qb1 - qb0 + W - 1) / W;
     const int q0 = min(qb1, qb0 + wave * qper), q1 = min(qb1, q0 + qper);
 
@@ -320,14 +322,14 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
                 co[i] = (mt0 + m) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (le >> 5);
                 ok[i] = nn2 < a.Ntot && co[i] < a.Cout;
                 const int n3 = ok[i] ? nn2 : 0;
-                bb[i] = mmi_fast_div(n3, a.T_magic, a.T_shift);
+                bb[i] = mmi_fast_div(n3, a.T_magic, tsh);
                 tt[i] = n3 - bb[i] * a.T_out;
                 float s = 0.f;
                 for (int w = 0; w < W; ++w) s += red[w * NE + e];
                 v[i] = s;
-                if (a.out_mode == MMI_GOUT_PARTIAL && (mt0 + m) < a.Mt) a.partial[((long)blockIdx.z * a.Mt * 32 + co[i]) * a.Npad + nn2] = s;
+                if (GROUP && a.out_mode == MMI_GOUT_PARTIAL && (mt0 + m) < a.Mt) a.partial[((long)blockIdx.z * a.Mt * 32 + co[i]) * a.Npad + nn2] = s;
             }
-            if (a.out_mode == MMI_GOUT_PARTIAL) continue;
+            if (GROUP && a.out_mode == MMI_GOUT_PARTIAL) continue;
             mmi_conv_store_n<NV>(a, co, bb, tt, ok, v);
         }
         return;
@@ -832,11 +834,16 @@ __global__ void k_convtr_combine(const float* __restrict__ tmp, const float* __r
     int t = p / S, r = p - t * S;
     const float* trow = tmp + row * (long)K * tmp_ld;  // [K][T_in], row stride tmp_ld
     float v = trow[(long)r * tmp_ld + t];
-    const bool inside = t > 0 && (T_frame == T_in || t % T_frame != 0);   // what a frame takes over from the one before it is added last, as when it is kept as `partial`
-    const float before = t > 0 ? trow[(long)(r + S) * tmp_ld + (t - 1)] : 0.f;
-    if (inside) v += before;
-    if (bias) v += bias[co];
-    if (!inside && t > 0) v += before;
+    if (T_frame == T_in) {
+        if (t > 0) v += trow[(long)(r + S) * tmp_ld + (t - 1)];
+        if (bias) v += bias[co];
+    } else {                                      // what a frame takes over from the one before it is added last, as when it is kept as `partial`
+        const bool inside = t % T_frame != 0;
+        const float before = t > 0 ? trow[(long)(r + S) * tmp_ld + (t - 1)] : 0.f;
+        if (inside) v += before;
+        if (bias) v += bias[co];
+        if (!inside && t > 0) v += before;
+    }
     if (t == 0) {
         // y[..., :PT] += partial; then the thread that consumed partial[b][co][r] also refreshes it
         long pi = row * (long)(K - S) + r;
@@ -1352,30 +1359,31 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
 
 // Rows of a call that brings several frames of a stream at once (MimiGroupRows): qkv [B][3 H D][ld] -> rotated queries, rotated keys and
 // values row by row [b][h][T][D], through LDS so that both sides move whole lines.
+#define MIMI_ROPE_T 8         // positions per workgroup: one rotation per thread at 64 dimensions
 template <int D>
 __global__ __launch_bounds__(256) void k_mimi_group_rope(MimiAttnArgs a, MimiGroupRows g) {
-    const int b = (int)blockIdx.x / a.H, h = (int)blockIdx.x % a.H, t0 = (int)blockIdx.y * 32, tid = (int)threadIdx.x;
+    const int b = (int)blockIdx.x / a.H, h = (int)blockIdx.x % a.H, t0 = (int)blockIdx.y * MIMI_ROPE_T, tid = (int)threadIdx.x;
     const int HD = a.H * D;
-    MMI_SHARED float tile[3 * D * 33];                     // [q | k | v][d][t]
-    for (int i = tid; i < 3 * D * 32; i += 256) {
-        const int t = i & 31, d = (i >> 5) % D, w = (i >> 5) / D;
-        tile[(w * D + d) * 33 + t] = a.qkv[((long)b * 3 * HD + w * HD + h * D + d) * g.qkv_ld + min(t0 + t, g.T - 1)];
+    MMI_SHARED float tile[3 * D * (MIMI_ROPE_T + 1)];                     // [q | k | v][d][t]
+    for (int i = tid; i < 3 * D * MIMI_ROPE_T; i += 256) {
+        const int t = i % MIMI_ROPE_T, d = i / MIMI_ROPE_T % D, w = i / MIMI_ROPE_T / D;
+        tile[(w * D + d) * (MIMI_ROPE_T + 1) + t] = a.qkv[((long)b * 3 * HD + w * HD + h * D + d) * g.qkv_ld + min(t0 + t, g.T - 1)];
     }
     __syncthreads();
     const long off = a.offsets[b], row0 = (long)blockIdx.x * g.T + t0;
-    for (int i = tid; i < 32 * (D / 2); i += 256) {
+    for (int i = tid; i < MIMI_ROPE_T * (D / 2); i += 256) {
         const int j = i % (D / 2), t = i / (D / 2);
         if (t0 + t >= g.T) continue;
         const float freq = expf((float)j * (-logf(a.max_period) * 2.0f / (float)D));
         const float ang = freq * (float)(off + t0 + t);
         const float c = cosf(ang), s = sinf(ang);
         float q0, q1, k0, k1;
-        mmi_rope_rotate(tile[(2 * j) * 33 + t], tile[(2 * j + 1) * 33 + t], c, s, q0, q1);
-        mmi_rope_rotate(tile[(D + 2 * j) * 33 + t], tile[(D + 2 * j + 1) * 33 + t], c, s, k0, k1);
+        mmi_rope_rotate(tile[(2 * j) * (MIMI_ROPE_T + 1) + t], tile[(2 * j + 1) * (MIMI_ROPE_T + 1) + t], c, s, q0, q1);
+        mmi_rope_rotate(tile[(D + 2 * j) * (MIMI_ROPE_T + 1) + t], tile[(D + 2 * j + 1) * (MIMI_ROPE_T + 1) + t], c, s, k0, k1);
         const long at = (row0 + t) * D + 2 * j;
         g.q[at] = q0; g.q[at + 1] = q1;
         g.kn[at] = k0; g.kn[at + 1] = k1;
-        g.vn[at] = tile[(2 * D + 2 * j) * 33 + t]; g.vn[at + 1] = tile[(2 * D + 2 * j + 1) * 33 + t];
+        g.vn[at] = tile[(2 * D + 2 * j) * (MIMI_ROPE_T + 1) + t]; g.vn[at + 1] = tile[(2 * D + 2 * j + 1) * (MIMI_ROPE_T + 1) + t];
     }
 }
 
