@@ -61,28 +61,17 @@ struct MimiSlab {
 };
 
 // Where a program's buffers come from: the stream's arena (zeroed, part of the stream's snapshot), or a slab, whose contents are all
-// written before they are read.  A slab's offset tables are gathered on the host and uploaded at once.
+// written before they are read.
 struct MimiMem {
     MmiArena* arena = nullptr;
     MimiSlab* slab = nullptr;
     int frames = 1;                            // of the program that is built
-    int* tab_dev = nullptr;
-    std::vector<int>* tab_host = nullptr;
+    hipStream_t stream = nullptr;
     template <class T>
     hipError_t alloc(T** p, size_t n) { return arena ? arena->alloc(p, n) : slab->alloc((void**)p, (n ? n : 1) * sizeof(T)); }
     template <class T>
-    hipError_t zero(T* p, size_t n, hipStream_t s) { return arena ? hipMemsetAsync(p, 0, n * sizeof(T), s) : hipSuccess; }
-    hipError_t table(const std::vector<int>& v, const int** out) {
-        if (slab) {
-            *out = tab_dev + tab_host->size();
-            tab_host->insert(tab_host->end(), v.begin(), v.end());
-            return hipSuccess;
-        }
-        int* dev = nullptr;
-        hipError_t e = arena->alloc(&dev, v.size());
-        if (e == hipSuccess) e = hipMemcpy(dev, v.data(), v.size() * sizeof(int), hipMemcpyHostToDevice);
-        *out = dev;
-        return e;
+    hipError_t zero(T* p, size_t n, hipStream_t s) {
+        return !arena || (arena->cut(p) && !getenv("MMI_DEBUG_POISON")) ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(T), s);      // (a chunk starts zeroed)
     }
 };
 
@@ -109,9 +98,7 @@ struct DequantScratch {
 struct MimiGroup {
     int frames = 0;                            // 0: not built (for this stream)
     bool refused = false;                      // building failed (shapes, memory): this stream goes frame by frame
-    int tab_B = 0, tab_frames = 0;             // what the slab's tables were uploaded for
     MimiSlab slab;
-    std::vector<int> tab;
     MmiProgram prog;
     Buf in, out;                               // encoder: samples, latents; decoder: latents, samples
     int* codes = nullptr;
@@ -527,14 +514,11 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
                 MMI_HIP_CHECK(mem.alloc(&a.partial, (size_t)p->ksplit * a.Mt * 32 * a.Npad));
             }
         }
-        std::vector<int> tab((size_t)a.Q * 8);
-        for (int q = 0; q < a.Q; ++q)
-            for (int h = 0; h < 2; ++h)
-                for (int e = 0; e < 4; ++e) {
-                    const int kd = (q * 4 + e) * 2 + h;
-                    tab[((size_t)q * 2 + h) * 4 + e] = kd < a.Cin * a.K ? (kd / a.K) * a.x_ld + kd % a.K : 0;
-                }
-        MMI_HIP_CHECK(mem.table(tab, &a.koff));
+        int* tab = nullptr;
+        MMI_HIP_CHECK(mem.alloc(&tab, (size_t)a.Q * 8));
+        MMI_LAUNCH(k_conv_offsets, mmi_cdiv(a.Q * 8, 256), 256, 0, mem.stream, tab, a.Q, a.Cin, a.K, a.x_ld);
+        MMI_CHECK_LAUNCH();
+        a.koff = tab;
         return MMI_OK;
     }
     p->wide = false;
@@ -1018,7 +1002,7 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         size_t kvn = (size_t)2 * c.tr_num_layers * B * c.tr_num_heads * c.tr_context * Dh;
         if (!g) {
             MMI_HIP_CHECK(m->st.alloc(&m->enc_kv, kvn));
-            MMI_HIP_CHECK(hipMemsetAsync(m->enc_kv, 0, kvn * sizeof(float), s0));
+            MMI_HIP_CHECK(mem.zero(m->enc_kv, kvn, s0));
         }
         prog.site("enc.tr");
         if ((rc = add_transformer(m, mem, prog, m->enc_tr, dsin, dsin.H, T, m->enc_kv, m->counters, B, frames, s0))) return rc;
@@ -1067,7 +1051,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     auto partial = [&](long pn, float** out) -> hipError_t {
         if (!g) {
             hipError_t e = m->st.alloc(out, (size_t)B * pn);
-            if (e == hipSuccess) e = hipMemsetAsync(*out, 0, (size_t)B * pn * sizeof(float), s0);
+            if (e == hipSuccess) e = mem.zero(*out, (size_t)B * pn, s0);
             if (e != hipSuccess) return e;
             m->partials.push_back(*out); m->partial_sizes.push_back(pn);
         }
@@ -1110,7 +1094,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         size_t kvn = (size_t)2 * c.tr_num_layers * B * c.tr_num_heads * c.tr_context * Dh;
         if (!g) {
             MMI_HIP_CHECK(m->st.alloc(&m->dec_kv, kvn));
-            MMI_HIP_CHECK(hipMemsetAsync(m->dec_kv, 0, kvn * sizeof(float), s0));
+            MMI_HIP_CHECK(mem.zero(m->dec_kv, kvn, s0));
         }
         prog.site("dec.tr");
         if ((rc = add_transformer(m, mem, prog, m->dec_tr, din, din.H, T, m->dec_kv, m->counters + B, B, frames, s0))) return rc;
@@ -1213,23 +1197,12 @@ int ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
     g.frames = 0;
     g.prog.clear();
     g.slab.rewind();
-    g.tab.clear();
-    size_t cap = 0;
-    for (const ConvW& w : enc ? m->enc_convs : m->dec_convs) cap += (size_t)w.Q * 8;
     MimiMem mem;
     mem.slab = &g.slab;
     mem.frames = frames;
-    mem.tab_host = &g.tab;
-    MMI_HIP_CHECK(g.slab.alloc((void**)&mem.tab_dev, cap * sizeof(int)));
+    mem.stream = s;
     int rc = enc ? build_encoder(m, m->batch, frames, mem, &g, s) : build_decoder(m, m->batch, frames, mem, &g, s);
     if (rc) return rc;
-    if (g.tab.size() > cap) return mmi_fail(MMI_ERR_UNSUPPORTED, "offset tables of a group");
-    if (!g.tab.empty() && (g.tab_B != m->batch || g.tab_frames != frames)) {
-        g.tab_frames = 0;
-        MMI_HIP_CHECK(hipMemcpyAsync(mem.tab_dev, g.tab.data(), g.tab.size() * sizeof(int), hipMemcpyHostToDevice, s));
-        g.tab_B = m->batch;
-        g.tab_frames = frames;
-    }
     g.frames = frames;
     return MMI_OK;
 }
@@ -1425,6 +1398,7 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
     hipStream_t s = (hipStream_t)stream;
     m->batch = batch;
     int rc = MMI_OK;
+    m->st.chunk = (size_t)32 << 20;
     auto fail = [&](int code) { m->streaming = true; mmi_mimi_streaming_stop(m); return code; };
     if (hipSuccess != m->st.alloc(&m->exec, (size_t)batch) || hipSuccess != m->st.alloc(&m->first, (size_t)batch) ||
         hipSuccess != m->st.alloc(&m->counters, (size_t)2 * batch) || hipSuccess != m->st.alloc(&m->dec_k_dev, (size_t)1))
@@ -1438,6 +1412,7 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
         return fail(mmi_fail(MMI_ERR_HIP, "initialising the streaming state failed"));
     MimiMem mem;
     mem.arena = &m->st;
+    mem.stream = s;
     if ((rc = build_encoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
     if ((rc = build_decoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
     m->all_exec = true;
@@ -1569,6 +1544,7 @@ extern "C" int mmi_mimi_quantize(mmi_mimi* m, const float* latent, int64_t* code
         MmiProgram prog;
         MimiMem mem;
         mem.arena = &m->st;
+        mem.stream = s;
         int rc = add_quantize_ops(m, mem, m->rvq, prog, latent, n_frames, f, batch);
         if (rc) return rc;
         rc = prog.run_eager(s);
@@ -1595,6 +1571,7 @@ extern "C" int mmi_mimi_decode_latent(mmi_mimi* m, const int64_t* codes, float* 
         MmiProgram prog;
         MimiMem mem;
         mem.arena = &m->st;
+        mem.stream = s;
         int rc = add_dequant_ops(m, mem, m->deq, prog, n_codebooks, out, f, batch);
         if (rc) return rc;
         rc = prog.run_eager(s);

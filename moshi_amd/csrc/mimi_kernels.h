@@ -99,6 +99,14 @@ MMI_HD int mmi_fast_div(int n, unsigned magic, unsigned shift = 0u) {
 }
 enum { MMI_GOUT_NATURAL = 0, MMI_GOUT_PACKED = 1, MMI_GOUT_PARTIAL = 2 };
 
+// k_conv_wide's offset table, see ConvGemmArgs::koff
+__global__ void k_conv_offsets(int* __restrict__ tab, int Q, int Cin, int K, int x_ld) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);          // (q, h, e)
+    if (i >= Q * 8) return;
+    const int kd = ((i >> 3) * 4 + (i & 3)) * 2 + ((i >> 2) & 1);
+    tab[i] = kd < Cin * K ? (kd / K) * x_ld + kd % K : 0;
+}
+
 struct ConvGemmArgs {
     const float* x;       // input [B][Cin][x_ld]; position p of a row = history (p < H) then the T new columns
     long x_bstride;       // Cin * x_ld

@@ -76,16 +76,38 @@ struct MmiWeights {
 };
 
 // device allocation bookkeeping: every engine frees what it allocated
+// chunk > 0: allocations up to an eighth of it are cut out of pieces of that size, zeroed when they are made, instead of each being one of
+// the runtime's (a stream of the codec is some 90 of them: start 0.60 -> 0.30 ms, stop 0.18 -> 0.04)
 struct MmiArena {
     std::vector<void*> ptrs;
     std::vector<size_t> sizes;
-    size_t bytes = 0;
+    size_t bytes = 0, chunk = 0, at = 0;
+    std::vector<char*> chunks;
+    hipError_t take(void** q, size_t nb) {
+        if (nb > chunk / 8) return hipMalloc(q, nb);
+        if (chunks.empty() || at + nb > chunk) {
+            char* c = nullptr;
+            hipError_t e = hipMalloc((void**)&c, chunk);
+            if (e != hipSuccess) return e;
+            chunks.push_back(c);
+            at = 0;
+            if ((e = hipMemset(c, 0, chunk)) != hipSuccess || (e = hipStreamSynchronize(nullptr)) != hipSuccess) return e;      // (the caller's stream need not wait for the null stream)
+        }
+        *q = chunks.back() + at;
+        at += (nb + 255) & ~(size_t)255;
+        return hipSuccess;
+    }
+    bool cut(const void* p) const {                // is it part of a chunk?
+        for (const char* c : chunks)
+            if (p >= c && p < c + chunk) return true;
+        return false;
+    }
     template <class T>
     hipError_t alloc(T** p, size_t count) {
         void* q = nullptr;
         size_t nb = count * sizeof(T);
         if (nb == 0) nb = sizeof(T);
-        hipError_t e = hipMalloc(&q, nb);
+        hipError_t e = take(&q, nb);
         if (e != hipSuccess) return e;
         // MMI_DEBUG_POISON=1 (tests / scripts/gpu_check.sh): every allocation of a handle starts as 0xFF bytes (bf16 / fp32 NaNs,
         // int -1) instead of whatever the allocator hands out, so that a read of state the engine never initialised shows up as
@@ -93,7 +115,7 @@ struct MmiArena {
         // (MMI_DEBUG_POISON=0: zero-fill instead - two sessions then start from identical memory, which is what MMI_DEBUG_TRACE's
         // per-op checksums need to be comparable line by line)
         const char* pz = getenv("MMI_DEBUG_POISON");
-        if (pz && (pz[0] == '1' || pz[0] == '0') && (e = hipMemset(q, pz[0] == '1' ? 0xFF : 0x00, nb)) != hipSuccess) { hipFree(q); return e; }
+        if (pz && (pz[0] == '1' || pz[0] == '0') && (e = hipMemset(q, pz[0] == '1' ? 0xFF : 0x00, nb)) != hipSuccess) { if (!cut(q)) hipFree(q); return e; }
         ptrs.push_back(q);
         sizes.push_back(nb);
         bytes += nb;
@@ -101,7 +123,11 @@ struct MmiArena {
         return hipSuccess;
     }
     void release() {
-        for (void* p : ptrs) hipFree(p);
+        for (void* p : ptrs)
+            if (!cut(p)) hipFree(p);
+        for (char* c : chunks) hipFree(c);
+        chunks.clear();
+        at = 0;
         ptrs.clear();
         sizes.clear();
         bytes = 0;
