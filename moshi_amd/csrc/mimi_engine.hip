@@ -521,7 +521,7 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         a.koff = tab;
         return MMI_OK;
     }
-    p->wide = false;
+    p->wide = false;                    // (at most 512 columns: T_shift is 0)
     const int nsub = mmi_cdiv(N, 32);
     if (a.ln_w) {                       // fused LayerNorm + linear: one 32-column subtile per workgroup, the whole K in registers
         if (!a.x_packed || a.Q > 64 || a.Q * 8 != a.Cin || a.K != 1 || a.out_mode == MMI_GOUT_PARTIAL)
@@ -651,8 +651,10 @@ int add_resblock(MimiMem& mem, MmiProgram& prog, ConvGemmArgs a1, ConvGemmArgs a
     // LDS: input window Cin x (32 + K - 1) | offset table | the waves' hand-off mailbox
     const size_t smem = ((size_t)((a1.Cin * (32 + a1.K - 1) + 3) & ~3) + (size_t)a1.Q * 8 + (mt1 > 1 ? (size_t)mt1 * 1024 : 0)) * sizeof(float);
     if (smem > 65536) return mmi_fail(MMI_ERR_UNSUPPORTED, "k_resblock: input window does not fit in LDS");
-    prog.add([ra, nblk, smem](hipStream_t s) {
-        MMI_LAUNCH((k_resblock<1, 4>), nblk, 64, smem, s, ra);
+    const bool group = mem.frames > 1;
+    prog.add([ra, nblk, smem, group](hipStream_t s) {
+        if (group) MMI_LAUNCH((k_resblock<1, 4, true>), nblk, 64, smem, s, ra);
+        else MMI_LAUNCH((k_resblock<1, 4, false>), nblk, 64, smem, s, ra);
         MMI_CHECK_LAUNCH();
         return (int)MMI_OK;
     });

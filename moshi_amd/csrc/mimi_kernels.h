@@ -123,7 +123,7 @@ struct ConvGemmArgs {
     const uint8_t* first; // replicate-pad flags [B] or null (conv.py:253-259)
     const uint8_t* exec;  // exec mask [B] (only read with `first`)
     int B, Cin, Cout, K, S, T_out;
-    unsigned T_magic, T_shift, K_magic;   // mmi_div_magic(T_out, T_shift), mmi_div_magic(K)
+    unsigned T_magic, K_magic;   // mmi_div_magic(T_out), mmi_div_magic(K)
     int Mt, Q;            // M tiles of 32, packed k-quads (Kdim_pad / 8)
     int Ntot;             // B * T_out
     int elu_in;           // apply ELU(alpha=1) to every loaded input (seanet.py:63,205,222)
@@ -142,7 +142,6 @@ struct ConvGemmArgs {
     const float* ln_b;
     float ln_eps;
     // --- filled in by the engine's planner
-    int q_blk;            // k_conv_wide: quads per workgroup of a split reduction (Q: not split)
     const int* koff;      // k_conv_wide: [Q][2][4] input offset of kd = (q*4+e)*2 + h; 0 past Cin*K (the weights there are 0)
     const float* bp;      // k_gemm_f32: packed activations [ceil(N/32)][Q][64][4]
     int x_packed;         // the producer already wrote `bp` (no k_pack_b_f32 launch)
@@ -151,6 +150,9 @@ struct ConvGemmArgs {
     int outQ;
     float* partial;       // GOUT_PARTIAL: [gridDim.y][Mt*32][Npad] raw sums, finished by k_conv_finish
     int Npad;
+    // groups of frames: T_magic = mmi_div_magic(T_out, T_shift), 0 where T_out < 2^11; quads per workgroup of a split reduction (Q: not split)
+    unsigned T_shift;
+    int q_blk;
 };
 
 __device__ __forceinline__ float mmi_elu(float v) { return v > 0.f ? v : expm1f(v); }
@@ -401,7 +403,7 @@ __global__ void k_pack_a_f32_hperm(const float* __restrict__ W, float* __restric
     P[idx] = v;
 }
 
-template <int MT1, int U>
+template <int MT1, int U, bool GROUP>
 __global__ __launch_bounds__(MT1 * 64) void k_resblock(ResBlockArgs ra) {
     const ConvGemmArgs& a = ra.a1;
     const ConvGemmArgs& c = ra.a2;
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(MT1 * 64) void k_resblock(ResBlockArgs ra) {
     const int jl = lane & 31, kh = lane >> 5;
     // the tile's 32 columns belong to ONE session (T_out % 32 == 0, checked by the engine): b, t0 are uniform
     const int n0 = (int)blockIdx.x * 32;
-    const int b = mmi_fast_div(n0, a.T_magic, a.T_shift), t0 = n0 - b * a.T_out;
+    const int b = mmi_fast_div(n0, a.T_magic, GROUP ? a.T_shift : 0u), t0 = n0 - b * a.T_out;
     const int LD = 32 + a.K - 1;                 // input columns the tile's windows cover (stride 1)
     MMI_DYN_SHARED(float, smem);                 // Xs[Cin][LD] | offs[Q][2][4] | mailbox[MT1][4][64][4]
     float* Xs = smem;
@@ -585,7 +587,7 @@ __global__ void k_pack_b_f32(ConvGemmArgs a, float* __restrict__ bp) {
     {   // columns past Ntot / reduction indices past Cin*K read a clamped (valid) element: they meet zero weights or are
         // discarded, and unconditional loads are not serialised by the compiler
         const int nc = n < a.Ntot ? n : 0;
-        const int b = mmi_fast_div(nc, a.T_magic, a.T_shift), t = nc - b * a.T_out;
+        const int b = mmi_fast_div(nc, a.T_magic), t = nc - b * a.T_out;
         const float* xb = a.x + (long)b * a.x_bstride + a.x_off + t * a.S;
         const bool rep = a.first != nullptr && a.first[b] != 0 && a.exec[b] != 0;
         const int hist = a.H - a.x_off;  // columns (relative to x_off) that belong to the history
@@ -654,7 +656,7 @@ __device__ __forceinline__ void mmi_gemm_f32_finish(const ConvGemmArgs& a, f32x1
     for (int i = 0; i < NV; ++i) {
         ok[i] = nn[i] < a.Ntot && co[i] < a.Cout;
         const int n3 = ok[i] ? nn[i] : 0;
-        bb[i] = mmi_fast_div(n3, a.T_magic, a.T_shift);
+        bb[i] = mmi_fast_div(n3, a.T_magic);
         tt[i] = n3 - bb[i] * a.T_out;
     }
     mmi_conv_store_n<NV>(a, co, bb, tt, ok, v);
