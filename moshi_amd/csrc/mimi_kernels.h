@@ -1143,8 +1143,10 @@ __global__ __launch_bounds__(256) void k_mimi_attn(MimiAttnArgs a) {
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 float dv = (qv[t][0] * kk[i][0] + qv[t][1] * kk[i][1]) + (qv[t][2] * kk[i][2] + qv[t][3] * kk[i][3]);
+                if constexpr (LPR == 16) dv = mmi_row_sum(dv);
+                else
 #pragma unroll
-                for (int m = LPR / 2; m >= 1; m >>= 1) dv += mmi_shfl_xor(dv, m);
+                    for (int m = LPR / 2; m >= 1; m >>= 1) dv += mmi_shfl_xor(dv, m);
                 if (seg == 0 && slot < L) {
                     const long dq = (off + t) - pos;
                     const bool ok = pos >= 0 && dq >= 0 && dq < a.context;
@@ -1217,6 +1219,8 @@ __global__ __launch_bounds__(256) void k_mimi_attn(MimiAttnArgs a) {
 // exp(m_wave - m) rescale.  The slots written by this call are taken from LDS instead of the ring (the ring loads were
 // issued before the write).  Static LDS: qs | kn | vn [T][D], red[4][T][D], mw/sw [4][T].
 // GROUP: one workgroup per (b, head) and frame (blockIdx.y) of a MimiGroupRows call; the same sums in the same order as frame by frame.
+// (Requesting the whole ring before the offset that says how much of it is valid measured slower, 9.0 -> 10.1 us at 50 of 250 rows.)
+// One stream: 10.7 -> 9.0 us with the row sums as rotations inside a row of lanes and one 32-bit remainder; bound by its chain of round trips.
 template <int D, int T, bool GROUP = false>
 __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGroupRows g) {
     constexpr int LPR = D / 4;             // lanes per ring row
@@ -1236,13 +1240,19 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
     const float* qrow = a.qkv + (long)b * 3 * HD * T;
     float* kcb = a.kc + ((long)b * a.H + h) * cap * D;
     float* vcb = a.vc + ((long)b * a.H + h) * cap * D;
+    const int seg = tid % LPR, rsub = tid / LPR;
+    f32x4 kk[IT], vv[IT];
     const long last = off + T - 1;
-    const int end_index = (int)(last % cap);
+    // slot of the first new token (a 64-bit remainder is some 200 dependent instructions)
+    const int slot0 = off < (1L << 31) ? (int)((unsigned)off % (unsigned)cap) : (int)(off % cap);
+    auto new_slot = [&](int t) __attribute__((always_inline)) {
+        const int x = slot0 + t;
+        return x < cap ? x : (T <= cap || x < 2 * cap ? x - cap : x % cap);
+    };
+    const int end_index = new_slot(T - 1);
     const long end_new = off + T;
     const int L = (int)(end_new < (long)cap ? end_new : (long)cap);
-    const int seg = tid % LPR, rsub = tid / LPR;
 
-    f32x4 kk[IT], vv[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int slot = min(i * RPB + rsub, L - 1);
@@ -1281,7 +1291,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
     if constexpr (!GROUP)
         for (int i = tid; i < T * D; i += 256) {
             const int t = i / D, d = i % D;
-            const long slot = (off + t) % cap;
+            const long slot = new_slot(t);
             kcb[slot * D + d] = kn[i];
             vcb[slot * D + d] = vn[i];
         }
@@ -1292,7 +1302,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         qv[t] = *reinterpret_cast<const f32x4*>(qs + t * D + seg * 4);
-        newslot[t] = (int)((off + t) % cap);
+        newslot[t] = new_slot(t);
     }
     float sc[T][IT];
     float mx[T];
@@ -1312,8 +1322,10 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             float dv = (qv[t][0] * kk[i][0] + qv[t][1] * kk[i][1]) + (qv[t][2] * kk[i][2] + qv[t][3] * kk[i][3]);
+            if constexpr (LPR == 16) dv = mmi_row_sum(dv);
+            else
 #pragma unroll
-            for (int m = LPR / 2; m >= 1; m >>= 1) dv += mmi_shfl_xor(dv, m);
+                for (int m = LPR / 2; m >= 1; m >>= 1) dv += mmi_shfl_xor(dv, m);
             const long dq = (off + t) - pos;
             const bool ok = slot < L && pos >= 0 && dq >= 0 && dq < a.context;
             sc[t][i] = ok ? dv * scale : -INFINITY;

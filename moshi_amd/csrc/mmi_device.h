@@ -66,6 +66,15 @@ __device__ __forceinline__ float mmi_group_sum(float x) {
     if constexpr (W >= 16) x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true));
     return x;
 }
+// The same sum over rows of 16 lanes in the order of an exchange over distances 8, 4, 2, 1 (rotations by those distances inside the row: a lane
+// and its partner hold what the exchange would give them), bit for bit what the shuffles give without their trips through LDS
+__device__ __forceinline__ float mmi_row_sum(float x) {
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, true));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xf, 0xf, true));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xf, 0xf, true));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xf, 0xf, true));
+    return x;
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {

@@ -323,6 +323,10 @@ inline unsigned atomicMax(unsigned* p, unsigned v) {
     return old;
 }
 
+inline float mmi_row_sum(float x) {
+    for (int m = 8; m >= 1; m >>= 1) x += mmi_shfl_xor(x, m);
+    return x;
+}
 // sum over groups of W consecutive lanes, every lane receiving the total (the gfx950 build: DPP row operations)
 template <int W>
 inline float mmi_group_sum(float x) {
