@@ -827,15 +827,17 @@ int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, 2 * p.fm
 int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
 
 int rows_ntw(const Plan& p) { return p.mt; }                // n-tiles per workgroup of the weight-streaming kernel
-template <class Tr, int FN, int FM, int ST, int OCC>
-int launch_tile(hipStream_t s, int grid, const TlmJobs& J) {
-    constexpr size_t smem = TlmTile<Tr, FN, FM, 2, 2, ST>::smem();
+template <class Tr, int FN, int FM, int ST, int OCC, int WN = 2, int WM = 2>
+int launch_tile(hipStream_t s, const TlmJobs& J) {
+    constexpr size_t smem = TlmTile<Tr, FN, FM, WN, WM, ST>::smem();
+    int grid = 0;                                          // every XCD's share of every job, rounded up
+    for (int i = 0; i < J.n; ++i) grid += 8 * mmi_cdiv(J.j[i].blocks, 8);
     static_assert(smem * OCC <= 160 * 1024, "LDS of a CU");
     if (smem > 64 * 1024) {
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, 2, 2, ST, OCC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         MMI_HIP_CHECK(attr);
     }
-    MMI_LAUNCH((k_tlm_gemm_tile<Tr, FN, FM, 2, 2, ST, OCC>), grid, 256, smem, s, J);
+    MMI_LAUNCH((k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC>), grid, 256, smem, s, J);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
@@ -865,15 +867,21 @@ int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J) {
     if (p.fm == 4) {
         if constexpr (Tr::V == 8) {
             const int wide = cut(16);
-            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, wide, J);
+            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, J);
         }
         const int grid = cut(8);
-        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, grid, J) : launch_tile<Tr, 4, 4, 3, 3>(s, grid, J);
+        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J) : launch_tile<Tr, 4, 4, 3, 3>(s, J);
     }
     // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
-    const int wide = cut(8);
-    if (Tr::V == 8 && wide >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, wide, J);
-    return launch_tile<Tr, 2, 2, 4, 4>(s, cut(4), J);
+    // at fp32 the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
+    if constexpr (Tr::V == 8) {
+        if (cut(8) >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, J);
+        cut(4);
+        return launch_tile<Tr, 2, 2, 4, 4>(s, J);
+    } else {
+        cut(4);
+        return launch_tile<Tr, 1, 4, 4, 4, 4, 1>(s, J);
+    }
 }
 int launch_jobs(mmi_tlm* m, hipStream_t s, const Plan& p, TlmJobs J) {
     return m->f32 ? launch_jobs_t<TlmF32>(s, p, J) : launch_jobs_t<TlmBf16>(s, p, J);

@@ -574,30 +574,33 @@ template <class Tr, int FN, int FM, int WN, int WM, int ST, int OCC>
 __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs jobs) {
     typedef TlmTile<Tr, FN, FM, WN, WM, ST> P;
     MMI_DYN_SHARED(u32x4, lds);
-    // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous run of tiles so that its L2 sees the shared operand
-    const int nb = (int)gridDim.x, xper = nb >> 3, xrem = nb & 7, xcd = (int)blockIdx.x & 7;
-    int b = xcd * xper + (xcd < xrem ? xcd : xrem) + ((int)blockIdx.x >> 3), ji = 0;
-    while (ji + 1 < jobs.n && b >= jobs.j[ji].blocks) b -= jobs.j[ji++].blocks;
+    // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous run of EVERY job's tiles - its L2 sees the shared operand, and no
+    // XCD has the long tiles, or the experts' unused row blocks, to itself
+    const int xcd = (int)blockIdx.x & 7;
+    int b = (int)blockIdx.x >> 3, ji = 0;
+    for (;; ++ji) {
+        if (ji == jobs.n) return;
+        const int lo = (int)((long)jobs.j[ji].blocks * xcd >> 3), mine = (int)((long)jobs.j[ji].blocks * (xcd + 1) >> 3) - lo;
+        if (b < mine) {
+            b += lo;
+            break;
+        }
+        b -= mine;
+    }
     const TlmJob j = jobs.j[ji];             // (a copy: its fields live in scalar registers)
     const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15;
-    const int ntb = (j.NT + P::NFN - 1) / P::NFN;
-    int g, rb, nb0, n, r0, split = 0;
+    const int ntb = (j.NT + P::NFN - 1) / P::NFN, rb = b % j.rblocks;
+    b /= j.rblocks;
+    const int nb0 = b % ntb;
+    b /= ntb;
+    const int split = b % j.ksplit;
+    int g = b / j.ksplit, n, r0;
     if (j.list) {
-        nb0 = b % ntb;
-        b /= ntb;
-        split = b % j.ksplit;
-        rb = b / j.ksplit;
         if (rb >= *j.n_tiles) return;
         g = j.tiles[3 * rb];
         r0 = j.tiles[3 * rb + 1];
         n = j.tiles[3 * rb + 2];
     } else {
-        rb = b % j.rblocks;
-        b /= j.rblocks;
-        nb0 = b % ntb;
-        b /= ntb;
-        split = b % j.ksplit;
-        g = b / j.ksplit;
         r0 = rb * 16 * P::NFM;
         n = j.rows - r0 < 16 * P::NFM ? j.rows - r0 : 16 * P::NFM;
     }
@@ -632,6 +635,7 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
         to = to + 1 < ST ? to + 1 : 0;
     };
     const int wn = wave % WN, wm = wave / WN;
+    const int ny = (n - wm * FM * 16 + 15) / 16;              // row fragments that hold rows (fp32: 512 cycles each and k-step, worth the branch)
     u32x4 av[2][FN], bv[2][FM];
     f32x4 acc[FN][FM];
 #pragma unroll
@@ -666,7 +670,8 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
             }
             mmi_sched_barrier();
 #pragma unroll
-            for (int y = 0; y < FM; ++y) acc[x][y] = Tr::mfma(av[cur][x], bv[cur][y], acc[x][y]);
+            for (int y = 0; y < FM; ++y)
+                if (Tr::V == 8 || y < ny) acc[x][y] = Tr::mfma(av[cur][x], bv[cur][y], acc[x][y]);
         }
         from = from + 1 < ST ? from + 1 : 0;
     };
