@@ -75,6 +75,17 @@ __device__ __forceinline__ float mmi_row_sum(float x) {
     x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xf, 0xf, true));
     return x;
 }
+// maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48, every one of them gets it: two exchanges of rows between registers
+// (v_permlane16_swap, v_permlane32_swap: a few cycles; the same steps through the LDS crossbar wait some 120 cycles each)
+__device__ __forceinline__ float mmi_rows_max(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned a0 = a[0], a1 = a[1];                           // (a bit cast of a vector's element itself takes element 0)
+    const unsigned w = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1)));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    const unsigned b0 = b[0], b1 = b[1];
+    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {

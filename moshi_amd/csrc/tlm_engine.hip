@@ -901,7 +901,7 @@ int attn_dispatch(int nd, int rk, F f) {
 #undef TLM_ND
     return mmi_fail(MMI_ERR_UNSUPPORTED, "latent too wide");
 }
-int attn_group_tiles(int nd, bool f32) { return nd <= (f32 ? 8 : 16) ? 8 : 4; }      // column tiles a workgroup of k_tlm_attn_tile takes (TlmAttnTile::QT)
+int attn_group_tiles(int nd) { return nd <= 8 ? 8 : 4; }      // column tiles a workgroup of k_tlm_attn_tile takes (TlmAttnTile::QT)
 
 template <class Tr>
 int launch_attn_t(hipStream_t s, const TlmAttnArgs& a, bool tiled) {
@@ -1156,8 +1156,10 @@ MixerOut build_latent_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, cons
     t.out_ks = L.lat_ks;
     t.mask = TlmMask{L.c.window, 0, L.c.scale * 1.44269504088896340736f};
     t.n_entries = sh.n_entries;
-    const bool wide = attn_group_tiles(L.nd, f32) == 8;
-    const bool tiled = sh.groups[L.geo][wide] >= ATTN_TILE_GROUPS && !(f32 && L.nd > 16);     // fp32 with a wide latent: the operands do not fit the registers
+    const bool wide = attn_group_tiles(L.nd) == 8;
+    // (bf16 with 9 to 16 latent blocks: groups of half the columns, two workgroups per CU.  16 heads, 256 latent columns: 600 tokens, 150
+    // groups, 29.7 us against 26.3 with the keys split; 900 tokens, 225 groups, 40.5 against 40.7)
+    const bool tiled = sh.groups[L.geo][wide] >= (!f32 && L.nd > 8 && L.nd <= 16 ? 2 : 1) * ATTN_TILE_GROUPS && !(f32 && L.nd > 16);     // fp32 with a wide latent: the operands do not fit the registers
     const int kind = tiled ? (wide ? 2 : 1) : 0;       // which of the three prefix arrays
     t.n_tiles = tiled ? sh.groups[L.geo][kind - 1] : sh.tiles[L.geo];
     t.nsplit = tiled ? 1 : std::max(1, std::min(sh.nsplit, (L.nd > 16 ? 256 : MAX_PARTIALS) / std::max(1, t.n_tiles)));     // (a wide latent: one workgroup per CU)

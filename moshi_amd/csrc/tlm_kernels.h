@@ -874,37 +874,78 @@ template <int LK>
 __device__ __forceinline__ int tlm_kstep_of(const TlmAttnArgs& a, int s) {
     return s < LK ? min(s, a.out_ks - 1) : min(a.out_ks + s - LK, a.q_ks - 1);
 }
-// scores of 32 keys -> softmax weights as operand fragments, the running maximum and sum moved on; returns the factor of older sums
-// (the lane's keys are k0 .. k0 + 3 and k0 + 16 .. k0 + 19, its column's position is k0 + d0)
-template <class Tr>
-__device__ __forceinline__ float tlm_softmax_block(const TlmMask& a, f32x4 s0, f32x4 s1, int k0, int d0, float& m, float& l, u32x4 (&pf)[32 / (4 * Tr::V)]) {
+// Scores of 32 keys and QT column tiles -> softmax weights as operand fragments, the running maxima, sums and outputs moved on (the lane's
+// keys are k0 .. k0 + 3 and k0 + 16 .. k0 + 19, its column of tile t is at position k0 + d0[t]).
+// In the prompts' kernels the vector unit and its latencies stood in the matrix cores' way (845 vector instructions per block of 32 keys
+// and 32 columns against 72 products; now some 200), so what is not needed is left out: the mask is looked at only where some key of some
+// column lies outside it, the exponential is the hardware's, the maxima cross lanes in registers, and sums are rescaled only once a maximum
+// has grown by more than 2^TLM_SOFT_SLACK.  Until then weights exceed one by as much, which costs no digits: they are rounded relative to
+// themselves (bf16) or not at all (fp32).
+constexpr float TLM_SOFT_SLACK = 8.f;
+template <class Tr, int ND, int QT>
+__device__ __forceinline__ void tlm_softmax_block(const TlmMask& a, f32x4 (&s)[QT][2], int k0, const int (&d0)[QT], float (&m)[QT], float (&l)[QT],
+                                                  u32x4 (&pf)[QT][32 / (4 * Tr::V)], f32x4 (&acc)[QT][ND]) {
     constexpr int NB = 32 / (4 * Tr::V);
-    float mx = m;
+    bool edge = false, moved = false;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int e0 = d0 - r, e1 = d0 - r - 16;
-        s0[r] = e0 >= 0 && (a.window <= 0 || e0 < a.window || k0 + r < a.keep) ? s0[r] * a.scale : -INFINITY;
-        s1[r] = e1 >= 0 && (a.window <= 0 || e1 < a.window || k0 + r + 16 < a.keep) ? s1[r] * a.scale : -INFINITY;
-        mx = fmaxf(mx, fmaxf(s0[r], s1[r]));
+    for (int t = 0; t < QT; ++t) {
+        edge = edge || d0[t] < 19 || (a.window > 0 && d0[t] >= a.window);
+        s[t][0] *= a.scale;
+        s[t][1] *= a.scale;
     }
-    mx = fmaxf(mx, mmi_shfl_xor(mx, 16));
-    mx = fmaxf(mx, mmi_shfl_xor(mx, 32));
-    const float al = exp2f(m - mx);
-    m = mx;
-    l *= al;
+    if (mmi_any(edge)) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        s0[r] = exp2f(s0[r] - mx);
-        s1[r] = exp2f(s1[r] - mx);
-        l += s0[r] + s1[r];
+        for (int t = 0; t < QT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e0 = d0[t] - r, e1 = d0[t] - r - 16;
+                s[t][0][r] = e0 >= 0 && (a.window <= 0 || e0 < a.window || k0 + r < a.keep) ? s[t][0][r] : -INFINITY;
+                s[t][1][r] = e1 >= 0 && (a.window <= 0 || e1 < a.window || k0 + r + 16 < a.keep) ? s[t][1][r] : -INFINITY;
+            }
     }
-    if constexpr (NB == 1) {
-        pf[0] = u32x4{mmi_pack_bf16x2(s0[0], s0[1]), mmi_pack_bf16x2(s0[2], s0[3]), mmi_pack_bf16x2(s1[0], s1[1]), mmi_pack_bf16x2(s1[2], s1[3])};
-    } else {
-        pf[0] = __builtin_bit_cast(u32x4, s0);
-        pf[NB - 1] = __builtin_bit_cast(u32x4, s1);
+    float mx[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        float x = m[t];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x = fmaxf(x, fmaxf(s[t][0][r], s[t][1][r]));
+        mx[t] = mmi_rows_max(x);
+        moved = moved || mx[t] - m[t] > TLM_SOFT_SLACK;
     }
-    return al;
+    if (mmi_any(moved)) {
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const float al = mmi_fast_exp2f(m[t] - mx[t]);
+            m[t] = mx[t];
+            l[t] *= al;
+#pragma unroll
+            for (int d = 0; d < ND; ++d) acc[t][d] *= al;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        f32x4 p0, p1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            p0[r] = mmi_fast_exp2f(s[t][0][r] - m[t]);
+            p1[r] = mmi_fast_exp2f(s[t][1][r] - m[t]);
+            l[t] += p0[r] + p1[r];
+        }
+        if constexpr (NB == 1) {
+            pf[t][0] = u32x4{mmi_pack_bf16x2(p0[0], p0[1]), mmi_pack_bf16x2(p0[2], p0[3]), mmi_pack_bf16x2(p1[0], p1[1]), mmi_pack_bf16x2(p1[2], p1[3])};
+        } else {
+            pf[t][0] = __builtin_bit_cast(u32x4, p0);
+            pf[t][NB - 1] = __builtin_bit_cast(u32x4, p1);
+        }
+    }
+}
+
+template <class Tr, int ND>
+__device__ __forceinline__ void tlm_softmax_block(const TlmMask& a, f32x4 s0, f32x4 s1, int k0, int d0, float& m, float& l, u32x4 (&pf)[32 / (4 * Tr::V)], f32x4 (&acc)[ND]) {
+    f32x4 s[1][2] = {{s0, s1}};
+    const int d[1] = {d0};
+    tlm_softmax_block<Tr, ND, 1>(a, s, k0, d, reinterpret_cast<float (&)[1]>(m), reinterpret_cast<float (&)[1]>(l), reinterpret_cast<u32x4 (&)[1][32 / (4 * Tr::V)]>(pf),
+                                 reinterpret_cast<f32x4 (&)[1][ND]>(acc));
 }
 
 // One block of 32 keys as a stream of fragments out of LDS - keys 0-15 and 16-31 of every k-step, then the turned values - consumed in
@@ -944,28 +985,12 @@ struct TlmAttnStream {
             if (f < 2 * NK) {
 #pragma unroll
                 for (int t = 0; t < QT; ++t) s[t][f & 1] = Tr::mfma(fr[buf][i], q(t, f >> 1), f < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[t][f & 1]);
-                if (f == 2 * NK - 1) soften(a, k0, d0);
+                if (f == 2 * NK - 1) tlm_softmax_block<Tr, ND, QT>(a, s, k0, d0, m, l, pf, acc);
             } else {
                 const int d = (f - 2 * NK) / NB;
 #pragma unroll
                 for (int t = 0; t < QT; ++t) acc[t][d] = Tr::mfma(fr[buf][i], pf[t][(f - 2 * NK) % NB], acc[t][d]);
             }
-        }
-    }
-    // scores -> softmax weights; the sums so far are rescaled when some column's maximum has moved
-    __device__ __forceinline__ void soften(const TlmMask& a, int k0, const int (&d0)[QT]) {
-        float al[QT];
-        bool moved = false;
-#pragma unroll
-        for (int t = 0; t < QT; ++t) {
-            al[t] = tlm_softmax_block<Tr>(a, s[t][0], s[t][1], k0, d0[t], m[t], l[t], pf[t]);
-            moved = moved || al[t] != 1.f;
-        }
-        if (mmi_any(moved)) {
-#pragma unroll
-            for (int t = 0; t < QT; ++t)
-#pragma unroll
-                for (int d = 0; d < ND; ++d) acc[t][d] *= al[t];
         }
     }
 };
@@ -1041,11 +1066,7 @@ __global__ __launch_bounds__(256, Tr::V == 8 && ND <= 16 ? 2 : 1) void k_tlm_att
         for (int k = LK; k < NK; ++k) load(k);
         mmi_sched_barrier();
         u32x4 pf[NB];
-        const float al = tlm_softmax_block<Tr>(a.mask, s0, s1, kb * 32 + 4 * kq, pc - (kb * 32 + 4 * kq), m, l, pf);
-        if (mmi_any(al != 1.f)) {
-#pragma unroll
-            for (int d = 0; d < ND; ++d) acc[d] *= al;
-        }
+        tlm_softmax_block<Tr, ND>(a.mask, s0, s1, kb * 32 + 4 * kq, pc - (kb * 32 + 4 * kq), m, l, pf, acc);
 #pragma unroll
         for (int k0 = 0; k0 < LK; k0 += GK) {
 #pragma unroll
@@ -1101,15 +1122,18 @@ __global__ __launch_bounds__(256, Tr::V == 8 && ND <= 16 ? 2 : 1) void k_tlm_att
 
 // Many columns (prompts): four waves x QT column tiles of one sequence walk the same keys; a block's fragments are staged through LDS
 // once for all of them (NBUF buffers, the next block in flight in registers while this one is used).
+// QT: as many tiles as leave room for a second workgroup on the CU (256 registers per wave), whose products fill the waits of this one's
+// softmax; with 512 registers the compiler also moved the sums between the two register files in every block.  2048 tokens, 16 heads, 256
+// latent columns, window 1024: two tiles and one workgroup per CU 89 us (and 114 before the softmax was trimmed), one tile and two 70.
 template <class Tr, int ND, int RK>
 struct TlmAttnTile {
-    static constexpr int QT = ND <= (Tr::V == 8 ? 16 : 8) ? 2 : 1;
+    static constexpr int QT = ND <= 8 ? 2 : 1;
     static constexpr int NF = 2 * TlmQuery<Tr, ND, RK>::NK + ND * TlmQuery<Tr, ND, RK>::NB;      // fragments per 32 keys
     static constexpr int NBUF = 2 * NF <= 152 ? 2 : 1;
     static constexpr size_t smem() { return (size_t)NBUF * NF * 1024; }
 };
 template <class Tr, int ND, int RK>
-__global__ __launch_bounds__(256) void k_tlm_attn_tile(TlmAttnArgs a) {
+__global__ __launch_bounds__(256, Tr::V == 8 && ND <= 16 ? 2 : 1) void k_tlm_attn_tile(TlmAttnArgs a) {
     typedef TlmQuery<Tr, ND, RK> Q;
     typedef TlmAttnTile<Tr, ND, RK> P;
     constexpr int NB = Q::NB, NK = Q::NK, QT = P::QT, NF = P::NF, NBUF = P::NBUF, NI = (NK + 3) / 4, FH = TlmFlip<Tr>::H;

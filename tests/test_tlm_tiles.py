@@ -1,9 +1,12 @@
 """Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 64, 128 x 64, 128 x 128 in three and four stages, 256 x 128, whole
 and split reductions, gathered and listed expert rows - at row counts just past a tile and sizes that are no multiples of one: a prompt fed at
 once must give the logits that the same prompt gives in portions of at most 64 tokens, which take the weight-streaming kernel."""
+from dataclasses import replace
+
 import pytest
 import torch
 
+from tests import tlm_cases as tc
 from moshi_amd.config import (DenseGLUConfig, GroupedAttentionConfig, LatentAttentionConfig, MinGRUConfig, MoEConfig, TokenLayerConfig, TokenLMConfig)
 from moshi_amd.tlm import TokenLM
 from moshi_amd.weights import random_token_lm_state_dict
@@ -41,3 +44,23 @@ def test_prompt_at_once_equals_portions(model, T, dtype):
     # fp32: sums of up to 6000 products in another order, over a handful of layers (eps sqrt(6000) ~ 5e-6); bf16: an activation on the other
     # side of a rounding boundary here and there (2^-9 each)
     assert rel < (1e-5 if dtype == torch.float32 else 8e-3), rel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("times", [8, -1, 0])
+@pytest.mark.parametrize("name", ["latent_36", "latent_128", "latent_200", "gqa_24", "gqa_128"])
+def test_attention_of_steep_turned_and_flat_scores(name, times):
+    """Prompts' attention where maxima move by more than the slack from block to block (steep), where it is the other end of the scores that
+    counts (a negative scale) and where nothing moves (scale 0); the window's and the sequence's ends fall inside blocks of 32 keys."""
+    cfg = {**tc.WIDE_PROMPTS, **tc.WIDE_PROMPTS_2}[name]
+    mixer = cfg.layers[0].mixer
+    cfg = replace(cfg, layers=[replace(cfg.layers[0], mixer=replace(mixer, scale=mixer.scale * times))])
+    lm, orc = tc.make(cfg, "cuda", None, max_tokens=1024)
+    toks = tc.tokens_of(cfg, 731, seed=7)
+    slot = lm.open()
+    pick = [0, 1, 31, 32, 33, 63, 64, 89, 90, 91, 300, 301, 702, 703, 704, 719]
+    got = lm.step([(slot, toks[:720], pick)])
+    want = orc.logits(toks)
+    # a score is off by some eps |score| and its weight by as much relatively: the steep ones by 8 times what the plain ones are
+    assert tc.rel(got.cpu().numpy(), want[pick]) < tc.TOL[torch.float32] * max(1, times)
+    assert tc.rel(tc.run_cut(lm, toks[720:], [1], slot), want[720:]) < tc.TOL[torch.float32] * max(1, times)
