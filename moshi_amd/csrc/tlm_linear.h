@@ -657,11 +657,12 @@ template <class Tr>
 __global__ __launch_bounds__(256) void k_tlm_gated_norm(TlmLinArgs a, int per_head, const TlmSeg* chunk) {
     MMI_DYN_SHARED(float, inv);                            // [heads], then [4]
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, V = a.vdim_p, ld = a.heads * V;
-    long row = (int)blockIdx.x;
+    const int b = tlm_row_block((int)blockIdx.x, (int)gridDim.x);
+    long row = b;
     if (chunk) {
-        const TlmSeg ck = chunk[blockIdx.x >> 6];
-        if ((int)(blockIdx.x & 63) >= ck.n) return;
-        row = ck.row0 + (int)(blockIdx.x & 63);
+        const TlmSeg ck = chunk[b >> 6];
+        if ((b & 63) >= ck.n) return;
+        row = ck.row0 + (b & 63);
     }
     const float* o = a.o + row * ld;
     if (per_head) {
