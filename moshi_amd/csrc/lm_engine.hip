@@ -641,9 +641,12 @@ int launch_norm_fused(hipStream_t s, int T, int mt, int wq, int NT, const GemmAr
         else if (T == 32) MMI_LAUNCH((k_gemm_xp_norm<32, 2, 8, 4, 1>), NT, 512, 0, s, a);
         else MMI_LAUNCH((k_gemm_xp_norm<16, 1, 8, 4, 1>), NT, 512, 0, s, a);
     } else if (wq == 3) {
-        if (T == 32 && mt == 1) MMI_LAUNCH((k_gemm_q8<32, 1, 8, 4, true>), NT, 512, 0, s, a);
-        else if (T == 32 && q8_tiles_over_grid()) MMI_LAUNCH((k_gemm_q8<32, 1, 8, 4, true>), dim3(NT, mt), 512, 0, s, a);
-        else if (T == 32) MMI_LAUNCH((k_gemm_q8<32, 2, 8, 4, true>), NT, 512, 0, s, a);
+        const bool serial = T == 32 && mt > 1 && !q8_tiles_over_grid();
+        const int half = mmi_cdiv(NT, 2);                // more workgroups than CUs (one each): two tiles per workgroup
+        if (serial) MMI_LAUNCH((k_gemm_q8<32, 2, 8, 4, true>), NT, 512, 0, s, a);
+        else if (NT * mt > 256 && T == 32) MMI_LAUNCH((k_gemm_q8<32, 1, 8, 4, true, 2>), dim3(half, mt), 512, 0, s, a);
+        else if (NT * mt > 256) MMI_LAUNCH((k_gemm_q8<16, 1, 8, 4, true, 2>), half, 512, 0, s, a);
+        else if (T == 32) MMI_LAUNCH((k_gemm_q8<32, 1, 8, 4, true>), dim3(NT, mt), 512, 0, s, a);
         else MMI_LAUNCH((k_gemm_q8<16, 1, 8, 4, true>), NT, 512, 0, s, a);
     } else if (wq == 2) {
         if (T == 32 && mt == 1) MMI_LAUNCH((k_gemm_xp_norm<32, 1, 8, 4, 2>), NT, 512, 0, s, a);

@@ -852,7 +852,11 @@ __device__ __forceinline__ void mmi_gemm_batch_tile_view(GemmArgs& a, int y, int
     a.B = min(TN, a.B - r0);
 }
 
-template <int TN, int MT, int WAVES, int KMAX, bool NORM>
+// NTW n-tiles per workgroup (a.osplit <= 1): every workgroup norms and quantises the rows again, some 1000 vector instructions per wave
+// against 8 products, and at 132 registers it has its CU to itself.  Where the tiles go round the chip a second time two of them share that
+// work (1024 -> 2 x 2816 gated, 352 workgroups -> 176: 64 sessions 14.1 -> 11.5 us, 9 sessions 13.8 -> 11.3; two workgroups per CU at 128
+// registers instead: 13.0).
+template <int TN, int MT, int WAVES, int KMAX, bool NORM, int NTW = 1>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     GemmArgs a = a_in;
     if constexpr (MT == 1) { if (gridDim.y > 1) mmi_gemm_batch_tile_view<TN>(a, (int)blockIdx.y, a.KSTEPS * 2); }
@@ -867,7 +871,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     // octet sharing as in k_gemm_xp (a.osplit > 1): N = 1024 linears have 32 n-tiles for 256 CUs; a workgroup = (tile, part) owns
     // TN / 8 / osplit of the tile's 8-row groups, the lanes of the other groups repeat an owned lane's weight address
     const int os = a.osplit > 1 ? a.osplit : 1;
-    const int nt0 = (int)blockIdx.x / os, part = (int)blockIdx.x - nt0 * os;
+    const int nt0 = (int)blockIdx.x / os * NTW, part = NTW > 1 ? 0 : (int)blockIdx.x - nt0 * os;
     const int g_lo = part * ((TN / 8) / os), g_hi = os > 1 ? g_lo + (TN / 8) / os : TN / 8;
     const int ro = (lane >> 3) & (TN / 8 - 1);
     const int wlane = (ro >= g_lo && ro < g_hi) ? lane : ((lane & ~((TN / 8 - 1) << 3)) | (g_lo << 3));
@@ -875,24 +879,32 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     const int ks0 = min(a.KSTEPS, wave * kper);
     const int nks = min(a.KSTEPS, ks0 + kper) - ks0;
     const int kq = TN == 32 ? (lane >> 5) : (lane >> 4);
-    const u32x4 pre = mmi_gemm_prefetch_addend<TN, MT, 1>(a, nt0);
+    u32x4 pre[NTW];
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) pre[t] = mmi_gemm_prefetch_addend<TN, MT, 1>(a, nt0 + t);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     const int ksl = min(ks0, a.KSTEPS - 1);
-    u32x4 wv[KMAX];
+    u32x4 wv[NTW][KMAX];
 #pragma unroll
-    for (int u = 0; u < KMAX; ++u) {
-        const int uu = min(u, nks > 0 ? nks - 1 : 0);
-        wv[u] = mmi_load_nt(a.wp + ((long)min(nt0, a.NT - 1) * a.KSTEPS + ksl + uu) * 64 + wlane);
-    }
+    for (int t = 0; t < NTW; ++t)
 #pragma unroll
-    for (int u = 0; u < KMAX; ++u) if (u >= nks) wv[u] = zero;
+        for (int u = 0; u < KMAX; ++u) {
+            const int uu = min(u, nks > 0 ? nks - 1 : 0);
+            wv[t][u] = mmi_load_nt(a.wp + ((long)min(nt0 + t, a.NT - 1) * a.KSTEPS + ksl + uu) * 64 + wlane);
+        }
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int u = 0; u < KMAX; ++u) if (u >= nks) wv[t][u] = zero;
     MMI_SHARED float sxl[MT * TN];                       // the rows' absmax, for the epilogue
     MMI_SHARED float redl[2][WAVES][MG][TN];             // [0] sums of squares, [1] absmax, per wave and tile of the group
-    iacc_t acc[MT];
+    iacc_t acc[NTW][MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int t = 0; t < NTW; ++t)
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[m][r] = 0;
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[t][m][r] = 0;
     const int dmax = (a.D - 8) > 0 ? (a.D - 8) : 0;
     u32x4 al[NORM ? XMAX : 1];
     if constexpr (NORM) {
@@ -978,18 +990,25 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
             for (int u = 0; u < KMAX; ++u) {
                 const u32x2 qlo = mmi_quant_i8x8(xv[g][2 * u], scale), qhi = mmi_quant_i8x8(xv[g][2 * u + 1], scale);
                 const u32x4 xq = {qlo[0], qlo[1], qhi[0], qhi[1]};
-                if constexpr (TN == 32) acc[m0 + g] = mmi_mfma_i8_32x32x32(wv[u], xq, acc[m0 + g]);
-                else acc[m0 + g] = mmi_mfma_i8_16x16x64(wv[u], xq, acc[m0 + g]);
+#pragma unroll
+                for (int t = 0; t < NTW; ++t) {
+                    if constexpr (TN == 32) acc[t][m0 + g] = mmi_mfma_i8_32x32x32(wv[t][u], xq, acc[t][m0 + g]);
+                    else acc[t][m0 + g] = mmi_mfma_i8_16x16x64(wv[t][u], xq, acc[t][m0 + g]);
+                }
             }
         }
         __syncthreads();                                 // redl is rewritten by the next group; sxl is read by the epilogue
     }
-    float accv[1][MT][R];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int t = 0; t < NTW; ++t) {
+        if (t) __syncthreads();                              // the epilogue's scratch
+        float accv[1][MT][R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) accv[0][m][r] = __builtin_bit_cast(facc_t, acc[m])[r];     // int32 bit patterns (see the epilogue)
-    mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi, sxl);
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) accv[0][m][r] = __builtin_bit_cast(facc_t, acc[t][m])[r];     // int32 bit patterns (see the epilogue)
+        mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0 + t, pre[t], nullptr, g_lo, g_hi, sxl);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -495,6 +495,14 @@ def test_cross_attention_more_positions_than_slots(sim_lib):
     lm_cases.cross_vs_oracle("cpu", sim_lib, replace(tiny_lm_config(), cross_attention=True), B=18, S=2, Tc=41, seed=8)
 
 
+@pytest.mark.parametrize("B", [3, 40])
+def test_int8_norm_fused_two_tiles_per_workgroup(sim_lib, B):
+    """A gated linear of more than 256 tiles, their number odd and (32-row tile) the last one not full: k_gemm_q8 takes two n-tiles per
+    workgroup, the last workgroup one."""
+    from dataclasses import replace
+    lm_cases.int8_linears_bit_exact("cpu", sim_lib, replace(tiny_lm_config(), depformer_dim_feedforward=3084), B, seed=571)
+
+
 def test_int8_depformer_batch_tiles_walked_by_one_workgroup(sim_lib, monkeypatch):
     """MMI_Q8_TILES=serial: k_gemm_q8<32, 2, ..> (both batch tiles through one workgroup's registers, the round-4 form kept for
     same-box A/Bs) stays bit-identical to the oracle; the default at 33..64 sessions is one batch tile per workgroup (grid.y)."""

@@ -35,6 +35,13 @@ def test_int8_linear_bit_exact_per_linear_at_the_7b_shapes(gpu_lib, B):
     assert B <= 16 or any("[splitk]" in n for n, _ in report)        # the 16-row tile (<= 16 sessions) does not split these GEMMs over K
 
 
+@pytest.mark.parametrize("B", [3, 40])
+def test_int8_norm_fused_two_tiles_per_workgroup(gpu_lib, B):
+    """More than 256 tiles, an odd number, the last one not full (32-row tile): k_gemm_q8's form of two n-tiles per workgroup."""
+    from dataclasses import replace
+    lm_cases.int8_linears_bit_exact(DEV, None, replace(tiny_lm_config(), depformer_dim_feedforward=3084), B, seed=571)
+
+
 def test_int8_linear_bit_exact_on_the_lds_resident_gemm_at_the_7b_shapes(gpu_lib, monkeypatch):
     """k_gemm_xlds<.., WQ = 3> (MMI_GEMM_LDS=1: int8 operand chunks resident in LDS) on the wide temporal GEMMs, two batch tiles."""
     monkeypatch.setenv("MMI_GEMM_LDS", "1")
