@@ -488,9 +488,10 @@ void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
 // workgroup covers follows the group's own number of columns.
 int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
     const int N = a.Ntot, N1 = N / mem.frames;
-    if (a.Cin * a.K >= (1 << 17) || N1 >= (1 << 17) || N >= (1 << 19) || a.K >= (1 << 11))
+    // (T_shift is the group kernels' alone: a frame's columns divide by fewer than 2^11)
+    if (a.Cin * a.K >= (1 << 17) || N1 >= (1 << 17) || N >= (1 << 19) || a.T_out / mem.frames >= (1 << 11) || a.K >= (1 << 11))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "conv dimensions outside the range of the kernels' index arithmetic (sessions x samples per frame "
-                                             "must stay below 131072: 68 sessions per handle at 1920 samples per frame)");
+                                             "must stay below 131072: 68 sessions per handle at 1920 samples per frame; a frame below 2048 samples)");
     // (a group's layers that the frame program streams the weights of do so for several column groups, up to 512 columns)
     if (N > (mem.frames > 1 && N1 <= 128 ? 512 : 128)) {
         if (a.first || a.x_packed || a.out_mode != MMI_GOUT_NATURAL)

@@ -1,6 +1,8 @@
 """Calls of several frames run them through the codec together (mimi_engine.hip, MimiGroup): every output bit and the streaming state must be
 those of the same frames one by one - across the attention ring's wrap, between groups of different sizes, around single frames, after a
 reset, under an exec mask (frame by frame then) and after a snapshot."""
+from dataclasses import replace
+
 import pytest
 import torch
 
@@ -51,6 +53,23 @@ def check_calls_equal_frames(make, device, cfg, B, sizes, K=4):
 @pytest.mark.parametrize("B,sizes", [(1, (2, 1, 7, 3)), (3, (5, 1, 4))])
 def test_tiny_calls_equal_frames(sim_lib, B, sizes):
     check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", tiny_mimi_config(), B, sizes)
+
+
+def test_frames_of_2048_samples_are_refused(sim_lib):
+    """The frame program divides column numbers by the samples of a frame with 11 bits; a stream of longer frames is refused when it
+    starts, however few they are.  One hop less is taken."""
+    cfg = replace(tiny_mimi_config(), n_filters=1, dimension=16, tr_d_model=16, tr_num_heads=1, compress=1)
+    for ratios, ok in (([8, 8, 4, 4], False), ([8, 4, 31, 1], True)):
+        c = replace(cfg, ratios=ratios)
+        c = replace(c, sample_rate=c.hop_length * 25)
+        assert c.frame_size == (1984 if ok else 2048)
+        m = MimiModel(random_mimi_state_dict(c, seed=1, device="cpu"), c, device="cpu", max_batch=1, num_codebooks=2, lib=sim_lib)
+        if ok:
+            with m.streaming(1):
+                assert m.is_streaming
+            continue
+        with pytest.raises(NotImplementedError, match="index arithmetic"):
+            m.streaming_forever(1)
 
 
 @pytest.mark.gpu
