@@ -60,18 +60,30 @@ struct MimiSlab {
     }
 };
 
-// Where a program's buffers come from: the stream's arena (zeroed, part of the stream's snapshot), or a slab, whose contents are all
-// written before they are read.
+// Where a program's buffers come from: the stream's arena (zeroed, part of the stream's snapshot), or a slab, which holds what it held.
+// A group's histories, activations, partial sums and tables are written before they are read; the rows that fill a packed operand's last
+// quad up are not (clear_operand): they meet zero weights, but 0 x NaN is NaN.
 struct MimiMem {
     MmiArena* arena = nullptr;
     MimiSlab* slab = nullptr;
     int frames = 1;                            // of the program that is built
     hipStream_t stream = nullptr;
     template <class T>
-    hipError_t alloc(T** p, size_t n) { return arena ? arena->alloc(p, n) : slab->alloc((void**)p, (n ? n : 1) * sizeof(T)); }
+    hipError_t alloc(T** p, size_t n) {
+        if (arena) return arena->alloc(p, n);
+        hipError_t e = slab->alloc((void**)p, (n ? n : 1) * sizeof(T));
+        const char* pz = getenv("MMI_DEBUG_POISON");                          // as in MmiArena::alloc, behind what still runs in the slab
+        if (e == hipSuccess && pz && (pz[0] == '1' || pz[0] == '0')) e = hipMemsetAsync(*p, pz[0] == '1' ? 0xFF : 0x00, (n ? n : 1) * sizeof(T), stream);
+        return e;
+    }
     template <class T>
     hipError_t zero(T* p, size_t n, hipStream_t s) {
         return !arena || (arena->cut(p) && !getenv("MMI_DEBUG_POISON")) ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(T), s);      // (a chunk starts zeroed)
+    }
+    // a packed operand of nsub x Q quads whose producer stores K rows
+    hipError_t clear_operand(float* p, int nsub, int Q, int K) {
+        const size_t n = (size_t)nsub * Q * 256;
+        return arena ? zero(p, n, stream) : (Q * 8 == K ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(float), stream));
     }
 };
 
@@ -755,9 +767,9 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
         MMI_HIP_CHECK(mem.alloc(&yp, (size_t)nsub * Qd * 256));
         MMI_HIP_CHECK(mem.alloc(&attp, (size_t)nsub * Qd * 256));
         MMI_HIP_CHECK(mem.alloc(&hbp, (size_t)nsub * Qff * 256));
-        MMI_HIP_CHECK(mem.zero(yp, (size_t)nsub * Qd * 256, init_stream));
-        MMI_HIP_CHECK(mem.zero(attp, (size_t)nsub * Qd * 256, init_stream));
-        MMI_HIP_CHECK(mem.zero(hbp, (size_t)nsub * Qff * 256, init_stream));
+        MMI_HIP_CHECK(mem.clear_operand(yp, nsub, Qd, d));
+        MMI_HIP_CHECK(mem.clear_operand(attp, nsub, Qd, d));
+        MMI_HIP_CHECK(mem.clear_operand(hbp, nsub, Qff, ff));
     }
     const size_t kv_layer = (size_t)B * H * cap * Dh;
     if (T / frames > 2 || (Dh != 16 && Dh != 32 && Dh != 64))
@@ -788,7 +800,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
     float* xrp = nullptr;
     if (fuse_ln) {
         MMI_HIP_CHECK(mem.alloc(&xrp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(mem.zero(xrp, (size_t)nsub * Qd * 256, init_stream));
+        MMI_HIP_CHECK(mem.clear_operand(xrp, nsub, Qd, d));
     }
     bool x_is_packed = false;           // xrp holds the current residual stream
     for (size_t l = 0; l < layers.size(); ++l) {
@@ -1116,7 +1128,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         const ConvW& wtr0 = m->dec_convs[ci];
         if ((B * T <= 128 || g) && wtr0.Q * 8 == mult * c.n_filters && !getenv("MMI_MIMI_PACK_LAUNCHES")) {
             MMI_HIP_CHECK(mem.alloc(&conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256));
-            MMI_HIP_CHECK(mem.zero(conv0_bp, (size_t)mmi_cdiv(B * T, 32) * wtr0.Q * 256, s0));
+            MMI_HIP_CHECK(mem.clear_operand(conv0_bp, mmi_cdiv(B * T, 32), wtr0.Q, mult * c.n_filters));
             a0.outp = conv0_bp; a0.outQ = wtr0.Q;
         }
         if ((rc = add_conv(mem, prog, a0))) return rc;

@@ -371,7 +371,7 @@ struct hipsimGraphExec { int dummy; };
 hipError_t hipMalloc(void** p, size_t n) {
     void* q = nullptr;
     if (posix_memalign(&q, 256, n ? ((n + 255) / 256) * 256 : 256) != 0) return hipErrorOutOfMemory;
-    memset(q, 0xCD, n);  // poison: catches reads of uninitialised device memory
+    memset(q, 0xFF, n);  // poison (NaN as fp32 / bf16 / fp64, -1 as an integer): catches reads of uninitialised device memory
     *p = q;
     return hipSuccess;
 }

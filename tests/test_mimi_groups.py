@@ -55,6 +55,15 @@ def test_tiny_calls_equal_frames(sim_lib, B, sizes):
     check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", tiny_mimi_config(), B, sizes)
 
 
+@pytest.mark.parametrize("ff", [60, 63, 65])
+def test_calls_equal_frames_where_operands_are_padded(sim_lib, monkeypatch, ff):
+    """A feed-forward width that is no multiple of 8: the packed operand between its two products has rows that nobody stores, which must
+    not hold what the memory held before (the simulator allocates NaN; a used slab is made to with MMI_DEBUG_POISON)."""
+    monkeypatch.setenv("MMI_DEBUG_POISON", "1")
+    cfg = replace(tiny_mimi_config(), tr_dim_feedforward=ff)
+    check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", cfg, 2, (3, 1, 4))
+
+
 def test_frames_of_2048_samples_are_refused(sim_lib):
     """The frame program divides column numbers by the samples of a frame with 11 bits; a stream of longer frames is refused when it
     starts, however few they are.  One hop less is taken."""
