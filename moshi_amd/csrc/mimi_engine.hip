@@ -33,30 +33,30 @@ struct Buf {            // activation buffer [B][C][ld]; first H columns = causa
     bool needs_elu_at_load() const { return !pe && !elu; }
 };
 
-// Scratch of a group program (below): chunks that are kept while the handle lives and handed out again from the start when a program is
-// rebuilt, so that a rebuild neither allocates nor frees.  What is asked for in the same order lies at the same addresses.
+// Scratch of a group program (below): one reservation of what the largest program so far needs.  A program is built on what there is; where
+// that is too little, the build goes on without launches (`over`) to learn what it needs, and is repeated on a larger reservation.
 struct MimiSlab {
-    struct Chunk { char* p; size_t size; };
-    std::vector<Chunk> chunks;
-    size_t cur = 0, at = 0;
-    hipError_t alloc(void** p, size_t nb) {
-        nb = (nb + 255) & ~(size_t)255;
-        while (cur < chunks.size() && at + nb > chunks[cur].size) { ++cur; at = 0; }
-        if (cur == chunks.size()) {
-            Chunk c = {nullptr, nb > ((size_t)32 << 20) ? nb : (size_t)32 << 20};
-            hipError_t e = hipMalloc((void**)&c.p, c.size);
-            if (e != hipSuccess) return e;
-            chunks.push_back(c);
-        }
-        *p = chunks[cur].p + at;
-        at += nb;
-        return hipSuccess;
+    char* base = nullptr;
+    size_t size = 0, need = 0;
+    bool over = false;
+    void* alloc(size_t nb) {
+        char* p = base + need;
+        need += (nb + 255) & ~(size_t)255;
+        over = over || need > size;
+        return over ? (char*)this : p;         // (not null, which means "none" to the plans; no launch is given it)
     }
-    void rewind() { cur = at = 0; }
+    void rewind() { need = 0; over = false; }
     void release() {
-        for (auto& c : chunks) hipFree(c.p);
-        chunks.clear();
+        hipFree(base);
+        base = nullptr;
+        size = 0;
         rewind();
+    }
+    hipError_t reserve(size_t nb) {            // never beside the old one: nothing of it may be in flight
+        release();
+        hipError_t e = hipMalloc((void**)&base, nb);
+        if (e == hipSuccess) size = nb;
+        return e;
     }
 };
 
@@ -71,11 +71,11 @@ struct MimiMem {
     template <class T>
     hipError_t alloc(T** p, size_t n) {
         if (arena) return arena->alloc(p, n);
-        hipError_t e = slab->alloc((void**)p, (n ? n : 1) * sizeof(T));
+        *p = (T*)slab->alloc((n ? n : 1) * sizeof(T));
         const char* pz = getenv("MMI_DEBUG_POISON");                          // as in MmiArena::alloc, behind what still runs in the slab
-        if (e == hipSuccess && pz && (pz[0] == '1' || pz[0] == '0')) e = hipMemsetAsync(*p, pz[0] == '1' ? 0xFF : 0x00, (n ? n : 1) * sizeof(T), stream);
-        return e;
+        return pz && (pz[0] == '1' || pz[0] == '0') && there() ? hipMemsetAsync(*p, pz[0] == '1' ? 0xFF : 0x00, (n ? n : 1) * sizeof(T), stream) : hipSuccess;
     }
+    bool there() const { return arena || !slab->over; }                       // false: a build that only counts
     template <class T>
     hipError_t zero(T* p, size_t n, hipStream_t s) {
         return !arena || (arena->cut(p) && !getenv("MMI_DEBUG_POISON")) ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(T), s);      // (a chunk starts zeroed)
@@ -83,7 +83,7 @@ struct MimiMem {
     // a packed operand of nsub x Q quads whose producer stores K rows
     hipError_t clear_operand(float* p, int nsub, int Q, int K) {
         const size_t n = (size_t)nsub * Q * 256;
-        return arena ? zero(p, n, stream) : (Q * 8 == K ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(float), stream));
+        return arena ? zero(p, n, stream) : (Q * 8 == K || !there() ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(float), stream));
     }
 };
 
@@ -529,7 +529,7 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         }
         int* tab = nullptr;
         MMI_HIP_CHECK(mem.alloc(&tab, (size_t)a.Q * 8));
-        MMI_LAUNCH(k_conv_offsets, mmi_cdiv(a.Q * 8, 256), 256, 0, mem.stream, tab, a.Q, a.Cin, a.K, a.x_ld);
+        if (mem.there()) MMI_LAUNCH(k_conv_offsets, mmi_cdiv(a.Q * 8, 256), 256, 0, mem.stream, tab, a.Q, a.Cin, a.K, a.x_ld);
         MMI_CHECK_LAUNCH();
         a.koff = tab;
         return MMI_OK;
@@ -1190,8 +1190,9 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
 
 // ---- groups of frames ---------------------------------------------------------------------------
 // Frames of the next group when `left` frames are to be run (1: frame by frame).  A group takes up to 160 frames over all streams - the 25 Hz
-// layers then have 320 columns for weights that they read once, and its buffers about 1 GB - and what is left is cut into equal groups.  Not while the caller's stream is being
-// captured (a group's launch list is not kept for ever), and not under an exec mask (its rows would have to stand still frame by frame).
+// layers then have 320 columns for weights that they read once, and its buffers 0.6 GB (encoder) or 0.8 GB (decoder) - and what is left is cut into
+// equal groups.  Not while the caller's stream is being captured (a group's launch list is not kept for ever), and not under an exec mask (its
+// rows would have to stand still frame by frame).
 int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left, hipStream_t s) {
     const mmi_mimi_cfg& c = m->cfg;
     int most = left;
@@ -1202,24 +1203,41 @@ int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, in
     if (most < 2) return 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 1;
-    return left / mmi_cdiv(left, most);
+    return mmi_cdiv(left, mmi_cdiv(left, most));           // (the larger ones first: a call's slab grows once)
 }
 
 // the program of `frames` frames, ready to run on s; MMI_ERR_UNSUPPORTED / MMI_ERR_HIP: go frame by frame
 int ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
     MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
     if (g.frames == frames) return MMI_OK;
-    g.frames = 0;
-    g.prog.clear();
-    g.slab.rewind();
     MimiMem mem;
     mem.slab = &g.slab;
     mem.frames = frames;
     mem.stream = s;
-    int rc = enc ? build_encoder(m, m->batch, frames, mem, &g, s) : build_decoder(m, m->batch, frames, mem, &g, s);
+    auto build = [&]() {
+        g.frames = 0;
+        g.prog.clear();
+        g.slab.rewind();
+        return enc ? build_encoder(m, m->batch, frames, mem, &g, s) : build_decoder(m, m->batch, frames, mem, &g, s);
+    };
+    int rc = build();
+    if (!rc && g.slab.over) {
+        MMI_HIP_CHECK(hipStreamSynchronize(s));           // the programs that ran in the old reservation
+        MMI_HIP_CHECK(g.slab.reserve(g.slab.need));
+        rc = build();
+        if (!rc && g.slab.over) rc = mmi_fail(MMI_ERR_HIP, "a group's program needs more than it asked for");
+    }
     if (rc) return rc;
     g.frames = frames;
     return MMI_OK;
+}
+
+// A stream that runs single frames gives back what groups of an earlier one have left here.  (Not at the end of every stream: a file encoded or
+// decoded without a stream of its own is one, and hipFree of 100 MB or more takes some 0.3 ms.)
+void give_back_group(MimiGroup& g, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (g.frames || !g.slab.size || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+    g.slab.release();
 }
 
 // The group's launches, and behind them on the host - while the GPU works on them - the capture of the frame program, so that a stream's
@@ -1443,7 +1461,7 @@ extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
     hipDeviceSynchronize();
     m->enc_prog.clear();
     m->dec_prog.clear();
-    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {      // their launches name the state that goes now; the slabs stay
+    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {      // their launches name the state that goes now; the slabs stay (give_back_group)
         g->prog.clear();
         g->frames = 0;
         g->refused = false;
@@ -1518,6 +1536,7 @@ static int encode_impl(mmi_mimi* m, const float* pcm, int64_t* codes, float* lat
     for (int f = 0, G; f < n_frames; f += G) {
         G = group_frames(m, m->enc_grp, m->enc_tab, n_frames - f, s);
         if (G > 1 && ready_group(m, true, G, s)) { m->enc_grp.refused = true; G = 1; }
+        if (G == 1) give_back_group(m->enc_grp, s);
         const Buf &in = G > 1 ? m->enc_grp.in : m->enc_in, &lat = G > 1 ? m->enc_grp.out : m->latent;
         // stage the samples behind the first conv's history
         MMI_LAUNCH(k_copy2d_f32, (int)mmi_cdiv64((int64_t)batch * c.channels * G * F, 256), 256, 0, s, pcm + (long)f * F,
@@ -1621,6 +1640,7 @@ extern "C" int mmi_mimi_decode_step_strided(mmi_mimi* m, const int64_t* codes, i
     for (int f = 0, G; f < n_frames; f += G) {
         G = group_frames(m, m->dec_grp, m->dec_tab, n_frames - f, s);
         if (G > 1 && ready_group(m, false, G, s)) { m->dec_grp.refused = true; G = 1; }
+        if (G == 1) give_back_group(m->dec_grp, s);
         MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * G * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)batch_stride, G > 1 ? m->dec_grp.codes : m->deq.codes,
                    c.q_n_q, batch, n_codebooks, n_frames, f, G);
         MMI_CHECK_LAUNCH();

@@ -8,6 +8,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 namespace hipsim {
@@ -368,16 +369,36 @@ struct hipsimEvent { std::chrono::steady_clock::time_point t; };
 struct hipsimGraph { int dummy; };
 struct hipsimGraphExec { int dummy; };
 
+static std::mutex g_mem_mu;
+static std::unordered_map<void*, size_t> g_mem;      // what is allocated
+static size_t g_mem_bytes = 0, g_mem_peak = 0;
 hipError_t hipMalloc(void** p, size_t n) {
     void* q = nullptr;
     if (posix_memalign(&q, 256, n ? ((n + 255) / 256) * 256 : 256) != 0) return hipErrorOutOfMemory;
+    {
+        std::lock_guard<std::mutex> g(g_mem_mu);
+        g_mem[q] = n;
+        g_mem_bytes += n;
+        g_mem_peak = std::max(g_mem_peak, g_mem_bytes);
+    }
     memset(q, 0xFF, n);  // poison (NaN as fp32 / bf16 / fp64, -1 as an integer): catches reads of uninitialised device memory
     *p = q;
     return hipSuccess;
 }
-hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipFree(void* p) {
+    {
+        std::lock_guard<std::mutex> g(g_mem_mu);
+        auto it = g_mem.find(p);
+        if (it != g_mem.end()) {
+            g_mem_bytes -= it->second;
+            g_mem.erase(it);
+        }
+    }
+    free(p);
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { memmove(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memmove(d, s, n); return hipSuccess; }
 hipError_t hipMemset(void* d, int v, size_t n) { memset(d, v, n); return hipSuccess; }
@@ -408,3 +429,11 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 // C entry points for the tests (ctypes): 0 forward, 1 reverse, 2 random (seed)
 extern "C" void hipsim_set_schedule(int mode, unsigned long long seed) { hipsim::set_schedule(mode, seed); }
 extern "C" int hipsim_get_schedule(void) { return hipsim::schedule(); }
+// bytes allocated now, and the most there were since the peak was last asked for
+extern "C" unsigned long long hipsim_live_bytes(void) { std::lock_guard<std::mutex> g(g_mem_mu); return g_mem_bytes; }
+extern "C" unsigned long long hipsim_peak_bytes(void) {
+    std::lock_guard<std::mutex> g(g_mem_mu);
+    const size_t peak = g_mem_peak;
+    g_mem_peak = g_mem_bytes;
+    return peak;
+}

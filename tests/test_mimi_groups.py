@@ -1,6 +1,8 @@
 """Calls of several frames run them through the codec together (mimi_engine.hip, MimiGroup): every output bit and the streaming state must be
 those of the same frames one by one - across the attention ring's wrap, between groups of different sizes, around single frames, after a
 reset, under an exec mask (frame by frame then) and after a snapshot."""
+import ctypes
+import gc
 from dataclasses import replace
 
 import pytest
@@ -62,6 +64,49 @@ def test_calls_equal_frames_where_operands_are_padded(sim_lib, monkeypatch, ff):
     monkeypatch.setenv("MMI_DEBUG_POISON", "1")
     cfg = replace(tiny_mimi_config(), tr_dim_feedforward=ff)
     check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", cfg, 2, (3, 1, 4))
+
+
+def sim_bytes(lib):
+    lib.cdll.hipsim_live_bytes.restype = lib.cdll.hipsim_peak_bytes.restype = ctypes.c_ulonglong
+    return int(lib.cdll.hipsim_live_bytes())
+
+
+def test_memory_of_groups_is_the_largest_one_s(sim_lib):
+    """What groups hold is what the largest of them needs, whatever sizes came before it, and never two of them at a time; it is given
+    back by a stream that runs single frames, and with the handle.  (256 channels: buffers of more than 32 MB)"""
+    cfg = replace(tiny_mimi_config(), channels=256, n_filters=2, ratios=[8, 8, 4, 3], sample_rate=768 * 25, tr_num_layers=1)
+    sd = random_mimi_state_dict(cfg, seed=1, device="cpu")
+
+    def held(sizes, decode):
+        gc.collect()
+        empty = sim_bytes(sim_lib)
+        m = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=2, lib=sim_lib)
+        before = sim_bytes(sim_lib)
+        sim_lib.cdll.hipsim_peak_bytes()
+
+        def call(n):
+            if decode:
+                m.decode(torch.zeros(1, 2, n, dtype=torch.int64))
+            else:
+                m.encode(torch.zeros(1, cfg.channels, n * cfg.frame_size))
+        with m.streaming(1):
+            for n in sizes:
+                call(n)
+            most = sim_lib.cdll.hipsim_peak_bytes() - before
+            streaming = sim_bytes(sim_lib) - before
+        kept = sim_bytes(sim_lib) - before
+        with m.streaming(1):
+            call(1)
+        given_back = sim_bytes(sim_lib) == before
+        del m
+        gc.collect()
+        assert sim_bytes(sim_lib) == empty
+        return streaming, kept, most, given_back
+
+    for decode in (False, True):
+        alone, alone_kept, alone_most, back = held([28], decode)
+        assert back and alone_kept <= alone == alone_most
+        assert held([24, 26, 28, 3, 25, 2], decode) == (alone, alone_kept, alone_most, True)
 
 
 def test_frames_of_2048_samples_are_refused(sim_lib):
