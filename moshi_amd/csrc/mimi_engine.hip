@@ -1202,14 +1202,16 @@ int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, in
     most = std::min(most, std::min(std::min(160 / B, 512 / (B * tpf)), ((1 << 19) - 1) / (B * c.frame_size)));
     if (most < 2) return 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 1;
-    return mmi_cdiv(left, mmi_cdiv(left, most));           // (the larger ones first: a call's slab grows once)
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    else if (cap == hipStreamCaptureStatusNone) return mmi_cdiv(left, mmi_cdiv(left, most));       // (the larger ones first: a call's slab grows once)
+    return 1;
 }
 
-// the program of `frames` frames, ready to run on s; MMI_ERR_UNSUPPORTED / MMI_ERR_HIP: go frame by frame
-int ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
+// The program of `frames` frames, ready to run on s.  False: this stream goes frame by frame from now on (a shape the plans do not take, no
+// memory), with nothing left of the attempt - no buffers, and no error for the next launch check to find.
+bool ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
     MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
-    if (g.frames == frames) return MMI_OK;
+    if (g.frames == frames) return true;
     MimiMem mem;
     mem.slab = &g.slab;
     mem.frames = frames;
@@ -1220,16 +1222,20 @@ int ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
         g.slab.rewind();
         return enc ? build_encoder(m, m->batch, frames, mem, &g, s) : build_decoder(m, m->batch, frames, mem, &g, s);
     };
-    int rc = build();
-    if (!rc && g.slab.over) {
-        MMI_HIP_CHECK(hipStreamSynchronize(s));           // the programs that ran in the old reservation
-        MMI_HIP_CHECK(g.slab.reserve(g.slab.need));
-        rc = build();
-        if (!rc && g.slab.over) rc = mmi_fail(MMI_ERR_HIP, "a group's program needs more than it asked for");
+    bool ok = build() == MMI_OK;
+    if (ok && g.slab.over) {                              // (what runs on s runs in the old reservation)
+        ok = hipStreamSynchronize(s) == hipSuccess && g.slab.reserve(g.slab.need) == hipSuccess && build() == MMI_OK && !g.slab.over;
     }
-    if (rc) return rc;
-    g.frames = frames;
-    return MMI_OK;
+    if (ok) {
+        g.frames = frames;
+        return true;
+    }
+    hipStreamSynchronize(s);
+    (void)hipGetLastError();
+    g.prog.clear();
+    g.slab.release();
+    g.refused = true;
+    return false;
 }
 
 // A stream that runs single frames gives back what groups of an earlier one have left here.  (Not at the end of every stream: a file encoded or
@@ -1535,7 +1541,7 @@ static int encode_impl(mmi_mimi* m, const float* pcm, int64_t* codes, float* lat
     const int F = c.frame_size, K = m->n_codebooks;
     for (int f = 0, G; f < n_frames; f += G) {
         G = group_frames(m, m->enc_grp, m->enc_tab, n_frames - f, s);
-        if (G > 1 && ready_group(m, true, G, s)) { m->enc_grp.refused = true; G = 1; }
+        if (G > 1 && !ready_group(m, true, G, s)) G = 1;
         if (G == 1) give_back_group(m->enc_grp, s);
         const Buf &in = G > 1 ? m->enc_grp.in : m->enc_in, &lat = G > 1 ? m->enc_grp.out : m->latent;
         // stage the samples behind the first conv's history
@@ -1639,7 +1645,7 @@ extern "C" int mmi_mimi_decode_step_strided(mmi_mimi* m, const int64_t* codes, i
     }
     for (int f = 0, G; f < n_frames; f += G) {
         G = group_frames(m, m->dec_grp, m->dec_tab, n_frames - f, s);
-        if (G > 1 && ready_group(m, false, G, s)) { m->dec_grp.refused = true; G = 1; }
+        if (G > 1 && !ready_group(m, false, G, s)) G = 1;
         if (G == 1) give_back_group(m->dec_grp, s);
         MMI_LAUNCH(k_codes_in, mmi_cdiv(batch * G * n_codebooks, 256), 256, 0, s, (const long*)codes, (long)batch_stride, G > 1 ? m->dec_grp.codes : m->deq.codes,
                    c.q_n_q, batch, n_codebooks, n_frames, f, G);

@@ -371,12 +371,15 @@ struct hipsimGraphExec { int dummy; };
 
 static std::mutex g_mem_mu;
 static std::unordered_map<void*, size_t> g_mem;      // what is allocated
-static size_t g_mem_bytes = 0, g_mem_peak = 0;
+static size_t g_mem_bytes = 0, g_mem_peak = 0, g_mem_total = ~(size_t)0;
+// a call's failure stays the thread's last error until hipGetLastError takes it
+static thread_local hipError_t t_last = hipSuccess;
+static hipError_t failed(hipError_t e) { t_last = e; return e; }
 hipError_t hipMalloc(void** p, size_t n) {
     void* q = nullptr;
-    if (posix_memalign(&q, 256, n ? ((n + 255) / 256) * 256 : 256) != 0) return hipErrorOutOfMemory;
     {
         std::lock_guard<std::mutex> g(g_mem_mu);
+        if (g_mem_bytes + n > g_mem_total || posix_memalign(&q, 256, n ? ((n + 255) / 256) * 256 : 256) != 0) return failed(hipErrorOutOfMemory);
         g_mem[q] = n;
         g_mem_bytes += n;
         g_mem_peak = std::max(g_mem_peak, g_mem_bytes);
@@ -407,7 +410,11 @@ hipError_t hipStreamCreate(hipStream_t* s) { *s = new hipsimStream(); return hip
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = t_last;
+    t_last = hipSuccess;
+    return e;
+}
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "hipSuccess" : "hipsim error"; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new hipsimEvent(); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
@@ -417,10 +424,10 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
     *ms = std::chrono::duration<float, std::milli>(b->t - a->t).count();
     return hipSuccess;
 }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorStreamCaptureUnsupported; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorStreamCaptureUnsupported; }
-hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t) { return hipErrorNotSupported; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return failed(hipErrorStreamCaptureUnsupported); }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return failed(hipErrorStreamCaptureUnsupported); }
+hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t) { return failed(hipErrorNotSupported); }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return failed(hipErrorNotSupported); }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -437,3 +444,5 @@ extern "C" unsigned long long hipsim_peak_bytes(void) {
     g_mem_peak = g_mem_bytes;
     return peak;
 }
+// memory of the device from now on (0: unlimited)
+extern "C" void hipsim_set_memory(unsigned long long bytes) { std::lock_guard<std::mutex> g(g_mem_mu); g_mem_total = bytes ? (size_t)bytes : ~(size_t)0; }

@@ -109,6 +109,37 @@ def test_memory_of_groups_is_the_largest_one_s(sim_lib):
         assert held([24, 26, 28, 3, 25, 2], decode) == (alone, alone_kept, alone_most, True)
 
 
+def test_calls_go_frame_by_frame_where_memory_is_short(sim_lib):
+    """No memory for a group's buffers, from the start or when a call is longer than the ones before: the call gives what its frames give
+    one by one, the next ones too, and nothing of the attempt stays allocated."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    gen = torch.Generator().manual_seed(3)
+    n, fs, set_memory = 20, cfg.frame_size, sim_lib.cdll.hipsim_set_memory
+    set_memory.argtypes = [ctypes.c_ulonglong]
+    x = 0.3 * torch.randn(2, 1, n * fs, generator=gen)
+    q = torch.randint(0, cfg.q_bins, (2, 4, n), generator=gen)
+    a, b = (MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib) for _ in range(2))
+    for first in (0, 2):                                       # frames of a call that finds memory
+        with a.streaming(2), b.streaming(2):
+            codes = [b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(n)]
+            pcm = [b.decode(q[..., f:f + 1].contiguous()) for f in range(n)]
+            empty = sim_bytes(sim_lib)
+            try:
+                at = 0
+                for size in (first, 5, 1, 3, n - 9 - first):
+                    part = slice(at, at + size)
+                    for call, want, arg in ((a.encode, codes, x[..., at * fs:(at + size) * fs]), (a.decode, pcm, q[..., part])):
+                        if at or not first:
+                            set_memory(sim_bytes(sim_lib))
+                        if size:
+                            assert torch.equal(call(arg.contiguous()), torch.cat(want[part], -1)), (first, at)
+                    assert (sim_bytes(sim_lib) > empty) == (first > at)
+                    at += size
+            finally:
+                set_memory(0)
+
+
 def test_frames_of_2048_samples_are_refused(sim_lib):
     """The frame program divides column numbers by the samples of a frame with 11 bits; a stream of longer frames is refused when it
     starts, however few they are.  One hop less is taken."""
