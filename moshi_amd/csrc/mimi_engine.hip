@@ -1247,7 +1247,7 @@ void give_back_group(MimiGroup& g, hipStream_t s) {
 }
 
 // The group's launches, and behind them on the host - while the GPU works on them - the capture of the frame program, so that a stream's
-// first single frame after a call of several does not wait for it.
+// first single frame after a call of several does not wait for it.  (A capture that fails fails there: the group has run.)
 int run_group(mmi_mimi* m, bool enc, hipStream_t s) {
     MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
     const HistTable& st = enc ? m->enc_tab : m->dec_tab;
@@ -1257,7 +1257,8 @@ int run_group(mmi_mimi* m, bool enc, hipStream_t s) {
     if (rc) return rc;
     MMI_LAUNCH(k_move_history, mmi_cdiv(rows, 256), 256, 0, s, g.hist, st, rows);
     MMI_CHECK_LAUNCH();
-    return m->use_graph ? (enc ? m->enc_prog : m->dec_prog).capture_full(m->cap_stream) : MMI_OK;
+    if (m->use_graph && (enc ? m->enc_prog : m->dec_prog).capture_full(m->cap_stream)) (void)hipGetLastError();
+    return MMI_OK;
 }
 
 int check_cfg(const mmi_mimi_cfg& c) {

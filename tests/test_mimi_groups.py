@@ -140,6 +140,22 @@ def test_calls_go_frame_by_frame_where_memory_is_short(sim_lib):
                 set_memory(0)
 
 
+def test_a_group_does_not_need_the_frame_program_s_capture(sim_lib, monkeypatch):
+    """The capture behind a group's launches is for a later call: the simulator cannot capture, which a call of several frames does not
+    notice (its state has moved on by then), and a single frame does."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    x = 0.3 * torch.randn(1, 1, 7 * cfg.frame_size, generator=torch.Generator().manual_seed(4))
+    want = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib).encode(x)
+    monkeypatch.delenv("MMI_NO_GRAPH")
+    m = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+    with m.streaming(1):
+        got = [m.encode(x[..., f * cfg.frame_size:(f + n) * cfg.frame_size].contiguous()) for f, n in ((0, 3), (3, 4))]
+        assert torch.equal(torch.cat(got, -1), want)
+        with pytest.raises(RuntimeError, match="hipStreamBeginCapture"):
+            m.encode(x[..., :cfg.frame_size].contiguous())
+
+
 def test_frames_of_2048_samples_are_refused(sim_lib):
     """The frame program divides column numbers by the samples of a frame with 11 bits; a stream of longer frames is refused when it
     starts, however few they are.  One hop less is taken."""
