@@ -1430,12 +1430,7 @@ extern "C" int mmi_mimi_get_cfg(const mmi_mimi* m, mmi_mimi_cfg* out) {
     return MMI_OK;
 }
 
-extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
-    MmiDeviceGuard dev_guard_(m ? m->device : -1);
-    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
-    if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
-    if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
-    hipStream_t s = (hipStream_t)stream;
+static int start_stream(mmi_mimi* m, int batch, hipStream_t s) {
     m->batch = batch;
     int rc = MMI_OK;
     m->st.chunk = (size_t)32 << 20;
@@ -1459,6 +1454,22 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
     if (hipStreamSynchronize(s) != hipSuccess) return fail(mmi_fail(MMI_ERR_HIP, "hipStreamSynchronize failed"));
     m->streaming = true;
     return MMI_OK;
+}
+
+extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
+    MmiDeviceGuard dev_guard_(m ? m->device : -1);
+    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
+    if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
+    if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
+    int rc = start_stream(m, batch, (hipStream_t)stream);
+    if (rc == MMI_ERR_HIP) (void)hipGetLastError();
+    if (rc == MMI_ERR_HIP && (m->enc_grp.slab.size || m->dec_grp.slab.size)) {      // without what an earlier stream's groups have left
+        m->enc_grp.slab.release();
+        m->dec_grp.slab.release();
+        rc = start_stream(m, batch, (hipStream_t)stream);
+        if (rc == MMI_ERR_HIP) (void)hipGetLastError();
+    }
+    return rc;
 }
 
 extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {

@@ -140,6 +140,33 @@ def test_calls_go_frame_by_frame_where_memory_is_short(sim_lib):
                 set_memory(0)
 
 
+def test_a_stream_starts_where_groups_hold_the_memory(sim_lib):
+    """What groups of an earlier stream have left is given back where the next stream would not start beside it."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    set_memory = sim_lib.cdll.hipsim_set_memory
+    set_memory.argtypes = [ctypes.c_ulonglong]
+    m = MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+    before = sim_bytes(sim_lib)
+    x = torch.zeros(2, 1, 8 * cfg.frame_size)
+    with m.streaming(2):
+        stream = sim_bytes(sim_lib) - before
+    want = m.encode(x)
+    assert sim_bytes(sim_lib) > before
+    try:
+        set_memory(before + stream)
+        with m.streaming(2):
+            assert sim_bytes(sim_lib) == before + stream
+            assert torch.equal(m.encode(x), want)
+        set_memory(before + stream - 1)
+        with pytest.raises(RuntimeError):
+            m.streaming_forever(2)
+        assert sim_bytes(sim_lib) == before
+    finally:
+        set_memory(0)
+    assert torch.equal(m.encode(x), want)
+
+
 def test_a_group_does_not_need_the_frame_program_s_capture(sim_lib, monkeypatch):
     """The capture behind a group's launches is for a later call: the simulator cannot capture, which a call of several frames does not
     notice (its state has moved on by then), and a single frame does."""
