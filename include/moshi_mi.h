@@ -342,7 +342,8 @@ int mmi_lm_debug_linear(mmi_lm* lm, const char* weight_name, const char* alpha_n
  * launch in launch order (sites: "L.in_proj", "L.ffn_in", "dep.out_proj", "text_linear", ...).  scripts/rocpd_sites.py joins
  * it with a rocprofv3 kernel trace by position inside the step, which is how per-site durations of kernels that share one
  * name are recomputed under profiles/.  Returns the bytes needed including the final NUL (call with buf = NULL to size);
- * 0 before the first step.  mmi_mimi_launch_list: which = 0 encoder step, 1 decoder step. */
+ * 0 before the first step.  mmi_mimi_launch_list: which = 0 encoder step, 1 decoder step; 2, 3 the encoder's and the decoder's group of
+ * frames as this stream last ran it (0 bytes if it ran none). */
 int64_t mmi_lm_launch_list(const mmi_lm* lm, char* buf, int64_t cap);
 int64_t mmi_mimi_launch_list(const mmi_mimi* m, int32_t which, char* buf, int64_t cap);
 

@@ -157,7 +157,8 @@ struct mmi_mimi {
     HistDesc* dec_hist = nullptr;
     HistTable enc_tab, dec_tab;                // the same tables on the host
     MimiGroup enc_grp, dec_grp;
-    bool all_exec = true;                      // no exec mask has been set since the stream began (or all of it was reset)
+    int all_exec = 1;                          // does every stream run?  1: yes, 0: no, -1: what `exec` says (mask_changes, all_run)
+    bool mask_in_graph = false;                // a call that changes the mask has been captured: a replay may change it at any time
     int enc_nhist = 0, dec_nhist = 0, enc_hist_rows = 0, dec_hist_rows = 0;
     MmiProgram enc_prog, dec_prog;
     hipStream_t cap_stream = nullptr;
@@ -1188,22 +1189,45 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     return add_commit(m, prog, hist, B, g, &m->dec_hist, &m->dec_nhist, &m->dec_hist_rows, g ? &g->hist : &m->dec_tab, m->counters + B, T_tr, nullptr);
 }
 
+// A call on s changes the exec mask: all_exec becomes `known`, unless the call is only being recorded.
+void mask_changes(mmi_mimi* m, int known, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+    }
+    m->mask_in_graph = m->mask_in_graph || cap != hipStreamCaptureStatusNone;
+    m->all_exec = cap != hipStreamCaptureStatusNone ? -1 : known;
+}
+// After a mask or a snapshot a call of several frames reads the mask back, waiting for the work on s; once, unless it can change unseen.
+bool all_run(mmi_mimi* m, hipStream_t s) {
+    if (m->all_exec < 0 || m->mask_in_graph) {
+        std::vector<uint8_t> ex(m->batch);
+        if (hipMemcpyAsync(ex.data(), m->exec, ex.size(), hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        m->all_exec = std::find(ex.begin(), ex.end(), 0) == ex.end();
+    }
+    return m->all_exec == 1;
+}
+
 // ---- groups of frames ---------------------------------------------------------------------------
 // Frames of the next group when `left` frames are to be run (1: frame by frame).  A group takes up to 160 frames over all streams - the 25 Hz
 // layers then have 320 columns for weights that they read once, and its buffers 0.6 GB (encoder) or 0.8 GB (decoder) - and what is left is cut into
-// equal groups.  Not while the caller's stream is being captured (a group's launch list is not kept for ever), and not under an exec mask (its
-// rows would have to stand still frame by frame).
-int group_frames(const mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left, hipStream_t s) {
+// equal groups.  Not while the caller's stream is being captured (a group's launch list is not kept for ever), and not under an exec mask
+// that leaves streams out (their rows would have to stand still frame by frame).
+int group_frames(mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left, hipStream_t s) {
     const mmi_mimi_cfg& c = m->cfg;
     int most = left;
     if (const char* e = getenv("MMI_MIMI_GROUP")) most = atoi(e);         // test hook: the largest group
-    if (left < 2 || most < 2 || g.refused || !m->all_exec || tab.n < 0 || getenv("MMI_MIMI_PACK_LAUNCHES")) return 1;
+    if (left < 2 || most < 2 || g.refused || tab.n < 0 || getenv("MMI_MIMI_PACK_LAUNCHES")) return 1;
     const int tpf = c.resample_stride, B = m->batch;
     most = std::min(most, std::min(std::min(160 / B, 512 / (B * tpf)), ((1 << 19) - 1) / (B * c.frame_size)));
     if (most < 2) return 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
-    else if (cap == hipStreamCaptureStatusNone) return mmi_cdiv(left, mmi_cdiv(left, most));       // (the larger ones first: a call's slab grows once)
+    else if (cap == hipStreamCaptureStatusNone && all_run(m, s)) return mmi_cdiv(left, mmi_cdiv(left, most));       // (the larger ones first: a call's slab grows once)
     return 1;
 }
 
@@ -1417,9 +1441,10 @@ int64_t mmi_copy_launch_log(const std::vector<std::string>& log, char* buf, int6
 extern "C" int64_t mmi_mimi_launch_list(const mmi_mimi* m, int32_t which, char* buf, int64_t cap) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m || !m->streaming) return 0;
-    const MmiProgram& p = which == 0 ? m->enc_prog : m->dec_prog;
-    const MmiProgram& g = which == 0 ? m->enc_grp.prog : m->dec_grp.prog;
-    if (!p.logged()) return g.logged() ? mmi_copy_launch_log(g.launch_log(), buf, cap) : 0;      // (frames have only been run in groups so far)
+    const bool enc = which == 0 || which == 2;
+    const MmiProgram& p = enc ? m->enc_prog : m->dec_prog;
+    const MmiProgram& g = enc ? m->enc_grp.prog : m->dec_grp.prog;
+    if (which >= 2 || !p.logged()) return g.logged() ? mmi_copy_launch_log(g.launch_log(), buf, cap) : 0;      // (frames have only been run in groups so far)
     return mmi_copy_launch_log(p.launch_log(), buf, cap);
 }
 
@@ -1450,7 +1475,8 @@ static int start_stream(mmi_mimi* m, int batch, hipStream_t s) {
     mem.stream = s;
     if ((rc = build_encoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
     if ((rc = build_decoder(m, batch, 1, mem, nullptr, s))) return fail(rc);
-    m->all_exec = true;
+    m->all_exec = 1;
+    m->mask_in_graph = false;
     if (hipStreamSynchronize(s) != hipSuccess) return fail(mmi_fail(MMI_ERR_HIP, "hipStreamSynchronize failed"));
     m->streaming = true;
     return MMI_OK;
@@ -1511,7 +1537,7 @@ extern "C" int mmi_mimi_state_load(mmi_mimi* m, const void* src, int64_t bytes, 
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
     if (bytes != (int64_t)m->st.bytes) return mmi_fail(MMI_ERR_SHAPE, "snapshot taken from a different stream (batch)");
     MMI_HIP_CHECK(m->st.load(src, (hipStream_t)stream));
-    m->all_exec = false;      // the snapshot carries its own mask
+    mask_changes(m, -1, (hipStream_t)stream);      // the snapshot carries its own mask
     m->dec_k_cur = -1;        // the snapshot carries its own device-side K: the next decode re-uploads the caller's
     return MMI_OK;
 }
@@ -1520,7 +1546,7 @@ extern "C" int mmi_mimi_set_exec_mask(mmi_mimi* m, const uint8_t* mask, mmi_stre
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m || !mask) return mmi_fail(MMI_ERR_INVALID, "null argument");
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
-    m->all_exec = false;
+    mask_changes(m, -1, (hipStream_t)stream);
     MMI_LAUNCH(k_set_mask, mmi_cdiv(m->batch, 64), 64, 0, (hipStream_t)stream, m->exec, mask, m->batch);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
@@ -1532,7 +1558,7 @@ extern "C" int mmi_mimi_reset(mmi_mimi* m, const uint8_t* mask, mmi_stream strea
     if (!m->streaming) return mmi_fail(MMI_ERR_STATE, "not streaming");
     hipStream_t s = (hipStream_t)stream;
     const int B = m->batch;
-    if (!mask) m->all_exec = true;
+    mask_changes(m, !mask || m->all_exec == 1 ? 1 : -1, s);
     if (m->enc_hist_rows > 0)
         MMI_LAUNCH(k_reset_history, mmi_cdiv(m->enc_hist_rows, 256), 256, 0, s, (const HistDesc*)m->enc_hist, m->enc_nhist, m->enc_hist_rows, mask);
     if (m->dec_hist_rows > 0)

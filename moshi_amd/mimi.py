@@ -108,8 +108,9 @@ class MimiModel:
         return m, m.data_ptr()
 
     def launch_list(self, which: str = "encode"):
-        """[(site, kernel)] per kernel launch of one encoder / decoder step (recorded during the first step)."""
-        w = {"encode": 0, "decode": 1}[which]
+        """[(site, kernel)] per kernel launch of one encoder / decoder step (recorded during the first step), or of the last group of
+        frames that this stream ran together (empty if it ran none)."""
+        w = {"encode": 0, "decode": 1, "encode_group": 2, "decode_group": 3}[which]
         return _capi.launch_list(lambda buf, cap: self._lib.mmi_mimi_launch_list(self._handle, w, buf, cap))
 
     # ---- properties (compression.py:232-265) -----------------------------------------------------

@@ -1,6 +1,6 @@
 """Calls of several frames run them through the codec together (mimi_engine.hip, MimiGroup): every output bit and the streaming state must be
 those of the same frames one by one - across the attention ring's wrap, between groups of different sizes, around single frames, after a
-reset, under an exec mask (frame by frame then) and after a snapshot."""
+reset, under an exec mask (frame by frame if it leaves a stream out), after and from a snapshot - and that they were run together."""
 import ctypes
 import gc
 from dataclasses import replace
@@ -21,32 +21,54 @@ def check_calls_equal_frames(make, device, cfg, B, sizes, K=4):
     q = torch.randint(0, cfg.q_bins, (B, K, n), generator=gen).to(device)
     a, b = make(sd, cfg, K, B), make(sd, cfg, K, B)
 
-    def same(at, size, what):
+    def same(at, size, what, a=a, rows=slice(None)):
         part = x[..., at * fs:(at + size) * fs].contiguous()
         codes = torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(at, at + size)], -1)
-        assert torch.equal(a.encode(part), codes), f"{what}: codes of frames {at}..{at + size}"
+        assert torch.equal(a.encode(part)[rows], codes[rows]), f"{what}: codes of frames {at}..{at + size}"
         pcm = torch.cat([b.decode(q[..., f:f + 1].contiguous()) for f in range(at, at + size)], -1)
-        assert torch.equal(a.decode(q[..., at:at + size].contiguous()), pcm), f"{what}: samples of frames {at}..{at + size}"
+        assert torch.equal(a.decode(q[..., at:at + size].contiguous())[rows], pcm[rows]), f"{what}: samples of frames {at}..{at + size}"
+
+    def together(m):                                           # has this stream run a group in each direction (True), or none at all (False)?
+        kernels = [{k for _, k in m.launch_list(which)} for which in ("encode_group", "decode_group")]
+        assert bool(kernels[0]) == bool(kernels[1]) and all("k_mimi_group_rope" in k for k in kernels if k)
+        return bool(kernels[0])
     with a.streaming(B), b.streaming(B):
         at = 0
         for size in sizes:
             same(at, size, "stream")
             at += size
+            assert together(a) == any(n > 1 for n in sizes[:sizes.index(size) + 1])
+        assert not together(b)
         for m in (a, b):
             m.reset_streaming()
         same(0, sizes[0], "after a reset")
-        if B > 1:
-            mask = torch.arange(B) % 2 == 0
+        state = a.get_streaming_state()
+        b.set_streaming_state(state)
+        same(0, sizes[-1], "after a snapshot")
+        b.set_streaming_state(state)
+        c = make(sd, cfg, K, B)
+        with c.streaming(B):
+            c.set_streaming_state(state)
+            same(0, sizes[-1], "from a snapshot", c)
+            assert together(c) == (sizes[-1] > 1)
+    if B > 1:
+        mask = (torch.arange(B) % 2 == 0)
+        with a.streaming(B), b.streaming(B):
             for m in (a, b):
                 m.set_exec_mask(mask.to(device))
-            codes = a.encode(x[..., :2 * fs].contiguous())
-            want = torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(2)], -1)
-            assert torch.equal(codes[mask], want[mask]), "under a mask"
+            same(0, 2, "under a mask", rows=mask)
+            assert not together(a)
+            for m in (a, b):
+                m.reset_streaming(~mask.to(device))            # the others again: they start here
+            same(2, 2, "after a reset of those that stood still")
+            assert together(a)
             for m in (a, b):
                 m.set_exec_mask(torch.ones(B, dtype=torch.bool, device=device))
-                m.reset_streaming()
-        b.set_streaming_state(a.get_streaming_state())
-        same(0, sizes[-1], "after a snapshot")
+            same(1, 3, "under a mask of all streams")
+        with a.streaming(B):
+            a.set_exec_mask(torch.ones(B, dtype=torch.bool, device=device))
+            a.encode(x[..., :2 * fs].contiguous()), a.decode(q[..., :2].contiguous())
+            assert together(a)
     whole = a.encode(x)                                        # a fresh, temporary stream
     with b.streaming(B):
         assert torch.equal(whole, torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(n)], -1)), "temporary stream"
@@ -204,3 +226,33 @@ def test_frames_of_2048_samples_are_refused(sim_lib):
 @pytest.mark.parametrize("B,sizes", [(1, (1, 2, 65, 160, 161, 3)), (3, (21, 1, 53, 54)), (32, (2, 1, 5, 6)), (64, (3, 1))])
 def test_full_size_calls_equal_frames(B, sizes):
     check_calls_equal_frames(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cuda", max_batch=mb, num_codebooks=K), "cuda", MimiConfig(), B, sizes, K=8)
+
+
+@pytest.mark.gpu
+def test_a_mask_set_by_a_graph_is_seen():
+    """A captured set_exec_mask leaves no trace on the host when it is replayed: calls of several frames look at the mask itself."""
+    cfg, B = tiny_mimi_config(), 3
+    sd = random_mimi_state_dict(cfg, seed=5, device="cuda")
+    a, b = (MimiModel(sd, cfg, device="cuda", max_batch=B, num_codebooks=4) for _ in range(2))
+    fs = cfg.frame_size
+    x = (0.3 * torch.randn(B, 1, 12 * fs, generator=torch.Generator().manual_seed(9))).cuda()
+    mask = torch.tensor([True, False, True], device="cuda")
+
+    def same(at, rows):
+        want = torch.cat([b.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(at, at + 3)], -1)
+        assert torch.equal(a.encode(x[..., at * fs:(at + 3) * fs].contiguous())[rows], want[rows]), at
+    with a.streaming(B), b.streaming(B):
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            a.set_exec_mask(mask)                              # (recorded, not run)
+        everyone = torch.ones(B, dtype=torch.bool, device="cuda")
+        same(0, everyone)
+        a.reset_streaming(), b.reset_streaming()
+        same(3, everyone)
+        for at in (6, 9):
+            graph.replay(), b.set_exec_mask(mask)
+            same(at, mask)
+            for m in (a, b):
+                m.set_exec_mask(everyone)
+            same(0, everyone)                                  # the stream that stood still goes on where it stood
