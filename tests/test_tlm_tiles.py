@@ -46,12 +46,40 @@ def test_prompt_at_once_equals_portions(model, T, dtype):
     assert rel < (1e-5 if dtype == torch.float32 else 8e-3), rel
 
 
+@pytest.mark.parametrize("rise", [0.0, 0.3, 3.7, 7.9, 8.1, 40.0])
+def test_the_largest_weight_is_exactly_one(tmp_path, rise):
+    """bf16 attention rounds a weight relative to itself, so it must be formed against the maximum so far: the largest one is then exact,
+    however little the maximum has moved from one block of keys to the next (column c moves by c / 16 of `rise`)."""
+    import ctypes
+    import subprocess
+    import sys
+    from pathlib import Path
+    here = Path(__file__).resolve().parent / "hipsim"
+    sys.path.insert(0, str(here))
+    import build_sim
+    so = tmp_path / "softmax_selftest.so"
+    subprocess.check_call([build_sim._cxx(), "-O1", "-w", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", f"-I{here}", f"-I{build_sim.CSRC}",
+                           str(here / "softmax_selftest.cpp"), str(here / "hipsim.cpp"), "-o", str(so)])
+    lib, blocks = ctypes.CDLL(str(so)), 3
+    scores = torch.rand(blocks, 32, 16, generator=torch.Generator().manual_seed(3)) - 1.0
+    for b in range(1, blocks):
+        scores[b, 5 * b] = b * rise * torch.arange(16) / 16
+    p, m, l = torch.empty_like(scores), torch.empty(blocks, 16), torch.empty(16)
+    lib.softmax_selftest_run(*(ctypes.c_void_p(t.data_ptr()) if torch.is_tensor(t) else t for t in (scores, blocks, p, m, l)))
+    top = scores.amax(1).cummax(0).values
+    assert torch.equal(m, top)
+    want = torch.exp2(scores.double() - top[:, None].double())
+    assert torch.equal(p[scores == top[:, None]], torch.ones(int((scores == top[:, None]).sum())))
+    assert ((p - want).abs() <= want * 2.0 ** -8 + 2.0 ** -126).all()        # one rounding to bf16, 2^-9, and a few of fp32; no subnormal numbers
+    assert torch.allclose(l.double(), (want * torch.exp2(top - top[-1])[:, None].double()).sum((0, 1)), rtol=1e-5)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("times", [8, -1, 0])
 @pytest.mark.parametrize("name", ["latent_36", "latent_128", "latent_200", "gqa_24", "gqa_128"])
 def test_attention_of_steep_turned_and_flat_scores(name, times):
-    """Prompts' attention where maxima move by more than the slack from block to block (steep), where it is the other end of the scores that
-    counts (a negative scale) and where nothing moves (scale 0); the window's and the sequence's ends fall inside blocks of 32 keys."""
+    """Prompts' attention where maxima move far from block to block (steep), where it is the other end of the scores that counts (a
+    negative scale) and where nothing moves (scale 0); the window's and the sequence's ends fall inside blocks of 32 keys."""
     cfg = {**tc.WIDE_PROMPTS, **tc.WIDE_PROMPTS_2}[name]
     mixer = cfg.layers[0].mixer
     cfg = replace(cfg, layers=[replace(cfg.layers[0], mixer=replace(mixer, scale=mixer.scale * times))])
