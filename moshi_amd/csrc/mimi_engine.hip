@@ -909,6 +909,7 @@ int upload_hist(mmi_mimi* m, std::vector<HistDesc>& h, int B, HistDesc** dev, in
         if (d.H > 0) keep.push_back(d);
     *n = (int)keep.size();
     MMI_HIP_CHECK(m->st.alloc(dev, keep.size() ? keep.size() : 1));
+    m->st.own.push_back(*dev);
     if (!keep.empty())
         MMI_HIP_CHECK(hipMemcpy(*dev, keep.data(), keep.size() * sizeof(HistDesc), hipMemcpyHostToDevice));
     return MMI_OK;

@@ -6,6 +6,7 @@
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
+#include <algorithm>
 #include <string>
 #include <vector>
 #include <functional>
@@ -83,6 +84,7 @@ struct MmiArena {
     std::vector<size_t> sizes;
     size_t bytes = 0, chunk = 0, at = 0;
     std::vector<char*> chunks;
+    std::vector<const void*> own;                  // allocations that name places of this arena: saved like the others, but not loaded
     hipError_t take(void** q, size_t nb) {
         if (nb > chunk / 8) return hipMalloc(q, nb);
         if (chunks.empty() || at + nb > chunk) {
@@ -127,6 +129,7 @@ struct MmiArena {
             if (!cut(p)) hipFree(p);
         for (char* c : chunks) hipFree(c);
         chunks.clear();
+        own.clear();
         at = 0;
         ptrs.clear();
         sizes.clear();
@@ -145,7 +148,8 @@ struct MmiArena {
     hipError_t load(const void* src, hipStream_t s) {
         size_t at = 0;
         for (size_t i = 0; i < ptrs.size(); ++i) {
-            hipError_t e = hipMemcpyAsync(ptrs[i], (const char*)src + at, sizes[i], hipMemcpyDeviceToDevice, s);
+            const bool mine = std::find(own.begin(), own.end(), ptrs[i]) != own.end();
+            hipError_t e = mine ? hipSuccess : hipMemcpyAsync(ptrs[i], (const char*)src + at, sizes[i], hipMemcpyDeviceToDevice, s);
             if (e != hipSuccess) return e;
             at += sizes[i];
         }

@@ -189,6 +189,25 @@ def test_a_stream_starts_where_groups_hold_the_memory(sim_lib):
     assert torch.equal(m.encode(x), want)
 
 
+def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
+    """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
+    stream it is called on, and leaves the one that the snapshot came from alone."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    fs = cfg.frame_size
+    x = 0.3 * torch.randn(1, 1, 9 * fs, generator=torch.Generator().manual_seed(6))
+    q = torch.randint(0, cfg.q_bins, (1, 4, 9), generator=torch.Generator().manual_seed(7))
+    a, b = (MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib) for _ in range(2))
+    codes, pcm = b.encode(x), b.decode(q)
+    with a.streaming(1), b.streaming(1):
+        a.encode(x[..., :3 * fs].contiguous()), a.decode(q[..., :3].contiguous())
+        b.set_streaming_state(a.get_streaming_state())
+        b.reset_streaming()
+        assert torch.equal(a.encode(x[..., 3 * fs:].contiguous()), codes[..., 3:])
+        assert torch.equal(a.decode(q[..., 3:].contiguous()), pcm[..., 3 * fs:])
+        assert torch.equal(b.encode(x), codes) and torch.equal(b.decode(q), pcm)
+
+
 def test_a_group_does_not_need_the_frame_program_s_capture(sim_lib, monkeypatch):
     """The capture behind a group's launches is for a later call: the simulator cannot capture, which a call of several frames does not
     notice (its state has moved on by then), and a single frame does."""
