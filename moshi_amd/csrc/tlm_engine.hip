@@ -962,7 +962,7 @@ struct Carry {                    // what the next residual launch has to add
 struct Norms {                    // what it leaves behind: one or two normalised operands, or (raw) the residual itself as an operand
     const float* w = nullptr; void* out = nullptr;
     const float* w2 = nullptr; void* out2 = nullptr;
-    void* rows = nullptr;         // what experts gather, row-major
+    void* rows = nullptr;         // what experts gather, row-major: by w2 if there is one
     void* raw = nullptr;
 };
 
@@ -1496,11 +1496,9 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
         Norms nm;
         nm.w = L.norm;
         nm.out = m->h;
-        void* hf = m->h;                                 // what the feed-forward reads
-        if (L.norm2) {
-            nm.w2 = L.norm2;
-            nm.out2 = hf = m->h2;
-        }
+        void* hf = L.norm2 ? m->h2 : m->h;               // what a dense feed-forward reads; experts gather rows
+        nm.w2 = L.norm2;
+        if (L.norm2 && dense) nm.out2 = hf;
         if (moe) nm.rows = m->hrow;
         P.site(site + "norm");
         add_resid(m, P, sh, c, emb, tap, nm, nullptr, T);

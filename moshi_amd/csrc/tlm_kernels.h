@@ -223,7 +223,7 @@ struct TlmResidArgs {
     const float* w; int groups; float eps;
     void* out; int KS;                   // packed; null: no norm
     const float* w2; void* out2;
-    void* rows_out; int rows_ld;         // what the feed-forward reads (the second operand if there is one), row-major, or null
+    void* rows_out; int rows_ld;         // what experts gather (by w2 if there is one), row-major, or null
     void* raw; int raw_ks;               // packed x, or null
     void* emb_out; int emb_k0;           // TLM_EMB_SET: packed copy of the embedding from column emb_k0 of rows of raw_ks k-steps, or null
     const int* rows;                     // row list (the residual is then not written back), or null
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(1024) void k_tlm_resid_norm(TlmResidArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = k + q < a.width ? v[q] * inv[(k + q) / gs] : 0.f;
         Tr::store4(out + tlm_index<Tr>(o, k, a.KS), v * w);
-        if (a.rows_out) Tr::store4((typename Tr::elem*)a.rows_out + (long)o * a.rows_ld + k, v * (a.out2 ? *reinterpret_cast<const f32x4*>(a.w2 + k) : w));
+        if (a.rows_out) Tr::store4((typename Tr::elem*)a.rows_out + (long)o * a.rows_ld + k, v * (a.w2 ? *reinterpret_cast<const f32x4*>(a.w2 + k) : w));
         if (a.out2) Tr::store4((typename Tr::elem*)a.out2 + tlm_index<Tr>(o, k, a.KS), v * *reinterpret_cast<const f32x4*>(a.w2 + k));
     }
 }
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
 template <class Tr, int FN, int FM, int WN, int WM, int ST>
 struct TlmTile {
     static constexpr int NW = WN * WM, NFN = WN * FN, NFM = WM * FM, NF = NFN + NFM, NIN = NFN / NW, NIM = NFM / NW, NI = NIN + NIM;
-    static_assert(NFN % NW == 0 && NFM % NW == 0 && ST >= 3, "every wave brings whole fragments");
+    static_assert(NFN % NW == 0 && NFM % NW == 0 && (ST == 3 || ST == 4), "every wave brings whole fragments; the waits are for one or two stages");
     static constexpr size_t smem() { return (size_t)ST * NF * 1024; }
 };
 template <class Tr, int FN, int FM, int WN, int WM, int ST, int OCC>
@@ -658,8 +658,7 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
         else av[set][i < FM ? 0 : i - FM] = base[(wn * FN + i - FM) * 64];
     };
     auto wait = [&](int behind) __attribute__((always_inline)) {          // until only the last `behind` stages are in flight
-        if (ST > 4 && behind >= 3) { if (ST > 5 && behind >= 4) mmi_wait_loads<(ST > 5 ? 4 : 0) * P::NI>(); else mmi_wait_loads<(ST > 4 ? 3 : 0) * P::NI>(); }
-        else if (ST > 3 && behind == 2) mmi_wait_loads<(ST > 3 ? 2 : 0) * P::NI>();
+        if (ST > 3 && behind == 2) mmi_wait_loads<(ST > 3 ? 2 : 0) * P::NI>();
         else if (behind == 1) mmi_wait_loads<P::NI>();
         else mmi_wait_loads<0>();
     };

@@ -85,6 +85,7 @@ MECHANISMS.update({
     "lightning_wide": plain_layer(LightningConfig(heads=2, dim=136, vdim=100, decay=[0.9, 0.97])),
     "glu": plain_layer(LIGHT, GLU),
     "glu_odd": plain_layer(replace(LIGHT, heads=1, decay=[0.8]), DenseGLUConfig(ff=37, limit=0.5), width=42),
+    "two_norms_experts": plain_layer(LIGHT, MOE),
     "bigram": plain_layer(LIGHT, None, bigram=BigramConfig(buckets=13, mul_prev=5, mul_cur=3), embed_scale=0.5),
     "positions": plain_layer(LIGHT, None, max_positions=200, embed_scale=2.0),
     "projected_passes": plain_layer(None, layers=[TokenLayerConfig(DELTA, GLU), TokenLayerConfig(GQA, None)], loop_start=0, loop_stop=2, loop_times=3),
