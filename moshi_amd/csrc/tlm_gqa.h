@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) void k_tlm_gqa_combine(TlmGqaArgs a) {
 
 // Many columns (prompts): four waves x QT column tiles of one sequence and kv head walk the same keys; a block's fragments are staged
 // through LDS once for all of them, the next block in flight in registers.  grid: column groups (64 QT columns), kv heads
-// 1773 tokens, 28 heads on 7 of 128, no window: 116 us; 88 with the trimmed softmax; 77 with maxima that cross lanes in registers and a
+// 1773 tokens, 28 heads on 7 of 128, no window: 116 us; 88 with the trimmed softmax; 79 with maxima that cross lanes in registers and a
 // block's address computed once instead of per fragment
 template <class Tr, int D>
 struct TlmGqaTile {
