@@ -1524,6 +1524,7 @@ __global__ __launch_bounds__(256) void k_rvq_select(RvqLevel l0, RvqLevel l1, in
             if (od < bd || (od == bd && oi < bi)) { bd = od; bi = oi; }
         }
         if (threadIdx.x == 0) {
+            if (bi == 0x7fffffff) bi = 0;          // no distance is a number (a NaN or infinite latent): where an argmin over NaNs ends
             widx = bi;
             codes[(long)r * codes_rstride + level] = bi;
         }

@@ -155,3 +155,27 @@ def test_maximum_batch_sizes(sim_lib):
         m = MimiModel(random_mimi_state_dict(mcfg, seed=7), mcfg, device="cpu", max_batch=256, num_codebooks=5, lib=sim_lib)
         with m.streaming(256):
             m.encode(torch.zeros(256, 1, mcfg.frame_size))
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38])
+@pytest.mark.parametrize("together", [False, True])
+def test_a_sample_that_is_no_number_stays_with_its_stream(sim_lib, bad, together):
+    """One NaN or infinite sample leaves a latent that is near to no code: the codes are still codes (0, where an argmin over NaNs ends), and the
+    other stream's are untouched."""
+    cfg = tiny_mimi_config()
+    fs, n = cfg.frame_size, 4
+    m = MimiModel(random_mimi_state_dict(cfg, seed=5), cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+    x = 0.3 * torch.randn(2, 1, n * fs, generator=torch.Generator().manual_seed(2))
+    broken = x.clone()
+    broken[1, 0, fs + 5] = bad
+
+    def encode(x):
+        return m.encode(x) if together else torch.cat([m.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(n)], -1)
+    with m.streaming(2):
+        good = encode(x)
+    with m.streaming(2):
+        codes = encode(broken)
+        assert torch.equal(codes[0], good[0]) and torch.equal(codes[1, :, 0], good[1, :, 0])
+        assert ((codes >= 0) & (codes < cfg.q_bins)).all()
+        if not np.isfinite(bad):
+            assert (codes[1, :, 1:] == 0).all()
