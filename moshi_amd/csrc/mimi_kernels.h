@@ -1252,10 +1252,11 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
     const int end_index = new_slot(T - 1);
     const long end_new = off + T;
     const int L = (int)(end_new < (long)cap ? end_new : (long)cap);
-
+    // rows past the valid ones repeat one that this stream has written since it began: their weight is 0, and 0 x NaN is NaN
+    const int rows = GROUP ? L : (off < (long)cap ? max((int)off, 1) : cap);
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        const int slot = min(i * RPB + rsub, L - 1);
+        const int slot = min(i * RPB + rsub, rows - 1);
         const long r = (long)slot * D + seg * 4;
         if constexpr (GROUP) {
             const long pos = slot <= end_index ? last + slot - end_index : last + slot - end_index - cap, n = pos - off0;
@@ -1267,6 +1268,10 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
             vv[i] = *reinterpret_cast<const f32x4*>(vcb + r);
         }
     }
+
+    if (!GROUP && off == 0)                        // (there is no such row yet)
+#pragma unroll
+        for (int i = 0; i < IT; ++i) vv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // rope(q), rope(k) -> LDS and ring, v -> LDS and ring (written unconditionally, transformer.py:243-250)
     if constexpr (GROUP) {

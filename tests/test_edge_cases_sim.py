@@ -160,8 +160,8 @@ def test_maximum_batch_sizes(sim_lib):
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38])
 @pytest.mark.parametrize("together", [False, True])
 def test_a_sample_that_is_no_number_stays_with_its_stream(sim_lib, bad, together):
-    """One NaN or infinite sample leaves a latent that is near to no code: the codes are still codes (0, where an argmin over NaNs ends), and the
-    other stream's are untouched."""
+    """One NaN or infinite sample leaves a latent that is near to no code: the codes are still codes (0, where an argmin over NaNs ends), the
+    other stream's are untouched, and a reset brings the stream back (what its ring held is not looked at)."""
     cfg = tiny_mimi_config()
     fs, n = cfg.frame_size, 4
     m = MimiModel(random_mimi_state_dict(cfg, seed=5), cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
@@ -179,3 +179,5 @@ def test_a_sample_that_is_no_number_stays_with_its_stream(sim_lib, bad, together
         assert ((codes >= 0) & (codes < cfg.q_bins)).all()
         if not np.isfinite(bad):
             assert (codes[1, :, 1:] == 0).all()
+        m.reset_streaming()
+        assert torch.equal(encode(x), good)
