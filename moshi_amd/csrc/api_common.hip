@@ -5,6 +5,7 @@ static thread_local std::string g_last_error;
 
 void mmi_set_error(const std::string& msg) { g_last_error = msg; }
 int mmi_fail(int code, const std::string& msg) {
+    if (code == MMI_ERR_HIP) (void)hipGetLastError();       // reported here: the next launch check, ours or the caller's, must not find it again
     g_last_error = msg;
     return code;
 }

@@ -1489,12 +1489,10 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
     if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
     if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
     int rc = start_stream(m, batch, (hipStream_t)stream);
-    if (rc == MMI_ERR_HIP) (void)hipGetLastError();
     if (rc == MMI_ERR_HIP && (m->enc_grp.slab.size || m->dec_grp.slab.size)) {      // without what an earlier stream's groups have left
         m->enc_grp.slab.release();
         m->dec_grp.slab.release();
         rc = start_stream(m, batch, (hipStream_t)stream);
-        if (rc == MMI_ERR_HIP) (void)hipGetLastError();
     }
     return rc;
 }

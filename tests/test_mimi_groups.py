@@ -208,6 +208,26 @@ def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
         assert torch.equal(b.encode(x), codes) and torch.equal(b.decode(q), pcm)
 
 
+def test_a_failed_call_is_reported_once(sim_lib):
+    """A failure of the runtime stays its last error until it is taken: it must not fail the next call, of this handle or another's."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    set_memory = sim_lib.cdll.hipsim_set_memory
+    set_memory.argtypes = [ctypes.c_ulonglong]
+    a = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+    x = torch.zeros(1, 1, cfg.frame_size)
+    with a.streaming(1):
+        want = a.encode(x)
+        a.reset_streaming()
+        try:
+            set_memory(sim_bytes(sim_lib) + 4096)
+            with pytest.raises(RuntimeError):
+                MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+        finally:
+            set_memory(0)
+        assert torch.equal(a.encode(x), want)
+
+
 def test_a_group_does_not_need_the_frame_program_s_capture(sim_lib, monkeypatch):
     """The capture behind a group's launches is for a later call: the simulator cannot capture, which a call of several frames does not
     notice (its state has moved on by then), and a single frame does."""
