@@ -46,14 +46,18 @@ struct MimiSlab {
         return over ? (char*)this : p;         // (not null, which means "none" to the plans; no launch is given it)
     }
     void rewind() { need = 0; over = false; }
-    void release() {
-        hipFree(base);
+    bool release() {                           // false: kept, the runtime does not free while another thread captures
+        if (base && hipFree(base) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
         base = nullptr;
         size = 0;
         rewind();
+        return true;
     }
     hipError_t reserve(size_t nb) {            // never beside the old one: nothing of it may be in flight
-        release();
+        if (!release()) return hipErrorOutOfMemory;
         hipError_t e = hipMalloc((void**)&base, nb);
         if (e == hipSuccess) size = nb;
         return e;
@@ -1190,15 +1194,19 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     return add_commit(m, prog, hist, B, g, &m->dec_hist, &m->dec_nhist, &m->dec_hist_rows, g ? &g->hist : &m->dec_tab, m->counters + B, T_tr, nullptr);
 }
 
+// Is s being captured, or (an error: the null stream, while another one is) not to be asked?  Leaves no error behind.
+bool recording(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // A call on s changes the exec mask: all_exec becomes `known`, unless the call is only being recorded.
 void mask_changes(mmi_mimi* m, int known, hipStream_t s) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusActive;
-    }
-    m->mask_in_graph = m->mask_in_graph || cap != hipStreamCaptureStatusNone;
-    m->all_exec = cap != hipStreamCaptureStatusNone ? -1 : known;
+    const bool rec = recording(s);
+    m->mask_in_graph = m->mask_in_graph || rec;
+    m->all_exec = rec ? -1 : known;
 }
 // After a mask or a snapshot a call of several frames reads the mask back, waiting for the work on s; once, unless it can change unseen.
 bool all_run(mmi_mimi* m, hipStream_t s) {
@@ -1226,10 +1234,7 @@ int group_frames(mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left
     const int tpf = c.resample_stride, B = m->batch;
     most = std::min(most, std::min(std::min(160 / B, 512 / (B * tpf)), ((1 << 19) - 1) / (B * c.frame_size)));
     if (most < 2) return 1;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
-    else if (cap == hipStreamCaptureStatusNone && all_run(m, s)) return mmi_cdiv(left, mmi_cdiv(left, most));       // (the larger ones first: a call's slab grows once)
-    return 1;
+    return !recording(s) && all_run(m, s) ? mmi_cdiv(left, mmi_cdiv(left, most)) : 1;       // (the larger ones first: a call's slab grows once)
 }
 
 // The program of `frames` frames, ready to run on s.  False: this stream goes frame by frame from now on (a shape the plans do not take, no
@@ -1266,9 +1271,7 @@ bool ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
 // A stream that runs single frames gives back what groups of an earlier one have left here.  (Not at the end of every stream: a file encoded or
 // decoded without a stream of its own is one, and hipFree of 100 MB or more takes some 0.3 ms.)
 void give_back_group(MimiGroup& g, hipStream_t s) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (g.frames || !g.slab.size || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
-    g.slab.release();
+    if (!g.frames && g.slab.size && !recording(s)) g.slab.release();
 }
 
 // The group's launches, and behind them on the host - while the GPU works on them - the capture of the frame program, so that a stream's

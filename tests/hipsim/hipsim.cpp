@@ -375,7 +375,9 @@ static size_t g_mem_bytes = 0, g_mem_peak = 0, g_mem_total = ~(size_t)0;
 // a call's failure stays the thread's last error until hipGetLastError takes it
 static thread_local hipError_t t_last = hipSuccess;
 static hipError_t failed(hipError_t e) { t_last = e; return e; }
+static std::atomic<int> g_elsewhere{0};              // another thread captures (hipsim_set_capture_elsewhere)
 hipError_t hipMalloc(void** p, size_t n) {
+    if (g_elsewhere) return failed(hipErrorStreamCaptureUnsupported);
     void* q = nullptr;
     {
         std::lock_guard<std::mutex> g(g_mem_mu);
@@ -389,6 +391,7 @@ hipError_t hipMalloc(void** p, size_t n) {
     return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+    if (g_elsewhere) return failed(hipErrorStreamCaptureUnsupported);
     {
         std::lock_guard<std::mutex> g(g_mem_mu);
         auto it = g_mem.find(p);
@@ -424,6 +427,11 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
     *ms = std::chrono::duration<float, std::milli>(b->t - a->t).count();
     return hipSuccess;
 }
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
+    if (g_elsewhere == 2 && !s) return failed(hipErrorStreamCaptureImplicit);
+    *st = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return failed(hipErrorStreamCaptureUnsupported); }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return failed(hipErrorStreamCaptureUnsupported); }
 hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t) { return failed(hipErrorNotSupported); }
@@ -446,3 +454,5 @@ extern "C" unsigned long long hipsim_peak_bytes(void) {
 }
 // memory of the device from now on (0: unlimited)
 extern "C" void hipsim_set_memory(unsigned long long bytes) { std::lock_guard<std::mutex> g(g_mem_mu); g_mem_total = bytes ? (size_t)bytes : ~(size_t)0; }
+// from now on another thread captures in the global mode, 1: a stream that does not block the null stream, 2: one that does, 0: it has ended
+extern "C" void hipsim_set_capture_elsewhere(int on) { g_elsewhere = on; }

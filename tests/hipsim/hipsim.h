@@ -47,7 +47,7 @@ int schedule();
 // ---- minimal HIP host API surface used by the engines -------------------------------------
 typedef int hipError_t;
 enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorNotSupported = 801,
-       hipErrorStreamCaptureUnsupported = 900 };
+       hipErrorStreamCaptureUnsupported = 900, hipErrorStreamCaptureImplicit = 906 };
 typedef struct hipsimStream* hipStream_t;
 typedef struct hipsimEvent* hipEvent_t;
 typedef struct hipsimGraph* hipGraph_t;
@@ -87,7 +87,7 @@ hipError_t hipEventSynchronize(hipEvent_t e);
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b);
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode m);
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g);
-inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) { *st = hipStreamCaptureStatusNone; return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st);
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t);
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s);
 hipError_t hipGraphDestroy(hipGraph_t g);

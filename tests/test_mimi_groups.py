@@ -162,6 +162,35 @@ def test_calls_go_frame_by_frame_where_memory_is_short(sim_lib):
                 set_memory(0)
 
 
+@pytest.mark.parametrize("blocking", [False, True])
+def test_calls_while_another_thread_captures(sim_lib, blocking):
+    """While another thread captures, the runtime neither allocates nor frees, and a capture that blocks the null stream does not let it be
+    asked: single frames go on beside an earlier stream's group memory, calls of several go frame by frame, and the memory is given back
+    by the first single frame after it."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    fs, n, capture_elsewhere = cfg.frame_size, 6, sim_lib.cdll.hipsim_set_capture_elsewhere
+    x = 0.3 * torch.randn(1, 1, n * fs, generator=torch.Generator().manual_seed(4))
+    q = torch.randint(0, cfg.q_bins, (1, 4, n), generator=torch.Generator().manual_seed(7))
+    m, other = (MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib) for _ in range(2))
+    codes, pcm = other.encode(x), other.decode(q)
+    before = sim_bytes(sim_lib)
+    with m.streaming(1):
+        stream = sim_bytes(sim_lib) - before
+    m.encode(x[..., :2 * fs].contiguous()), m.decode(q[..., :2].contiguous())
+    assert sim_bytes(sim_lib) > before
+    with m.streaming(1):
+        try:
+            capture_elsewhere(1 + blocking)
+            for f, k in ((0, 1), (1, 1), (2, 3)):
+                assert torch.equal(m.encode(x[..., f * fs:(f + k) * fs].contiguous()), codes[..., f:f + k])
+                assert torch.equal(m.decode(q[..., f:f + k].contiguous()), pcm[..., f * fs:(f + k) * fs])
+        finally:
+            capture_elsewhere(0)
+        assert torch.equal(m.encode(x[..., 5 * fs:].contiguous()), codes[..., 5:]) and torch.equal(m.decode(q[..., 5:].contiguous()), pcm[..., 5 * fs:])
+        assert sim_bytes(sim_lib) == before + stream
+
+
 def test_a_stream_starts_where_groups_hold_the_memory(sim_lib):
     """What groups of an earlier stream have left is given back where the next stream would not start beside it."""
     cfg = tiny_mimi_config()
