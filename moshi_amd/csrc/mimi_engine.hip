@@ -16,10 +16,14 @@ struct ConvW {          // one conv / linear as an implicit GEMM: rows = Cout, r
     int Cin = 0, Cout = 0, K = 1, S = 1, Mt = 0, Q = 0;
 };
 
+struct LinW {           // a transformer's linear, rows = M (k_pack_lin)
+    float* w = nullptr;
+    int M = 0, K = 0, J = 0;
+};
 struct TrLayerW {
-    ConvW in_proj, out_proj, lin1, lin2;
-    float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr, *ls1 = nullptr, *ls2 = nullptr;
-    float *n1w_pk = nullptr, *n1b_pk = nullptr, *n2w_pk = nullptr, *n2b_pk = nullptr;   // operand order, for k_gemm_f32_ln
+    LinW in_proj, out_proj, lin1, lin2;
+    float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr;       // operand order (k_pack_ln)
+    float *ls1 = nullptr, *ls2 = nullptr;
 };
 
 struct Buf {            // activation buffer [B][C][ld]; first H columns = causal history of its consumer
@@ -84,10 +88,10 @@ struct MimiMem {
     hipError_t zero(T* p, size_t n, hipStream_t s) {
         return !arena || (arena->cut(p) && !getenv("MMI_DEBUG_POISON")) ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(T), s);      // (a chunk starts zeroed)
     }
-    // a packed operand of nsub x Q quads whose producer stores K rows
-    hipError_t clear_operand(float* p, int nsub, int Q, int K) {
-        const size_t n = (size_t)nsub * Q * 256;
-        return arena ? zero(p, n, stream) : (Q * 8 == K || !there() ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(float), stream));
+    // a packed operand of `tiles` x Q fragments of `deep` reduction indices whose producer stores K rows
+    hipError_t clear_operand(float* p, int tiles, int Q, int K, int deep = 8) {
+        const size_t n = (size_t)tiles * Q * 256;
+        return arena ? zero(p, n, stream) : (Q * deep == K || !there() ? hipSuccess : hipMemsetAsync(p, 0, n * sizeof(float), stream));
     }
 };
 
@@ -246,13 +250,18 @@ int load_convtr(mmi_mimi* m, const MmiWeights& W, const std::string& prefix, int
 }
 
 // nn.Linear weight [out][in], no bias
-int load_linear(mmi_mimi* m, const MmiWeights& W, const std::string& name, int in, int out, ConvW* cw) {
+int load_linear(mmi_mimi* m, const MmiWeights& W, const std::string& name, int in, int out, LinW* lw) {
     const mmi_tensor_desc* w;
     int rc = need(W, name, 2, &w);
     if (rc) return rc;
     if (w->shape[0] != out || w->shape[1] != in) return mmi_fail(MMI_ERR_SHAPE, "shape mismatch for " + name);
-    cw->Cin = in; cw->Cout = out; cw->K = 1; cw->S = 1;
-    return pack_matrix(m, (const float*)w->data, out, in, in, 1, cw);
+    lw->M = out; lw->K = in; lw->J = mmi_cdiv(in, 16);
+    const int Mt = mmi_cdiv(out, 16);
+    const size_t n = (size_t)Mt * lw->J * 256;
+    MMI_HIP_CHECK(m->wts.alloc(&lw->w, n));
+    MMI_LAUNCH(k_pack_lin, (int)mmi_cdiv64((int64_t)n, 256), 256, 0, (hipStream_t)0, (const float*)w->data, lw->w, out, in, Mt, lw->J);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
 }
 
 int load_vec(mmi_mimi* m, const MmiWeights& W, const std::string& name, int n, float** out) {
@@ -275,20 +284,16 @@ int load_transformer(mmi_mimi* m, const MmiWeights& W, const std::string& prefix
         if ((rc = load_linear(m, W, p + ".self_attn.out_projs.0.weight", d, d, &L.out_proj))) return rc;
         if ((rc = load_linear(m, W, p + ".linear1.weight", d, ff, &L.lin1))) return rc;
         if ((rc = load_linear(m, W, p + ".linear2.weight", ff, d, &L.lin2))) return rc;
-        if ((rc = load_vec(m, W, p + ".norm1.weight", d, &L.n1w))) return rc;
-        if ((rc = load_vec(m, W, p + ".norm1.bias", d, &L.n1b))) return rc;
-        if ((rc = load_vec(m, W, p + ".norm2.weight", d, &L.n2w))) return rc;
-        if ((rc = load_vec(m, W, p + ".norm2.bias", d, &L.n2b))) return rc;
-        if ((rc = load_vec(m, W, p + ".layer_scale_1.scale", d, &L.ls1))) return rc;
-        if ((rc = load_vec(m, W, p + ".layer_scale_2.scale", d, &L.ls2))) return rc;
-        if (d % 8 == 0) {               // the norms' weight / bias in the packed operand's element order (k_gemm_f32_ln)
-            struct { const float* src; float** dst; } pk[] = {{L.n1w, &L.n1w_pk}, {L.n1b, &L.n1b_pk}, {L.n2w, &L.n2w_pk}, {L.n2b, &L.n2b_pk}};
-            for (auto& e : pk) {
-                MMI_HIP_CHECK(m->wts.alloc(e.dst, (size_t)d));
-                MMI_LAUNCH(k_pack_ln, mmi_cdiv(d, 256), 256, 0, (hipStream_t)0, e.src, *e.dst, d);
-            }
+        struct { const char* name; float** dst; } norms[] = {{".norm1.weight", &L.n1w}, {".norm1.bias", &L.n1b}, {".norm2.weight", &L.n2w}, {".norm2.bias", &L.n2b}};
+        for (auto& e : norms) {
+            float* v = nullptr;
+            if ((rc = load_vec(m, W, p + e.name, d, &v))) return rc;
+            MMI_HIP_CHECK(m->wts.alloc(e.dst, (size_t)mmi_cdiv(d, 16) * 16));
+            MMI_LAUNCH(k_pack_ln, mmi_cdiv(d, 256), 256, 0, (hipStream_t)0, (const float*)v, *e.dst, d & ~15);      // (widths that are no multiple: add_lin)
             MMI_CHECK_LAUNCH();
         }
+        if ((rc = load_vec(m, W, p + ".layer_scale_1.scale", d, &L.ls1))) return rc;
+        if ((rc = load_vec(m, W, p + ".layer_scale_2.scale", d, &L.ls2))) return rc;
     }
     return MMI_OK;
 }
@@ -347,7 +352,6 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
 //   N = B*T_out > 128 columns : k_conv_wide
 //   N <= 128                  : [k_pack_b_f32] -> k_gemm_f32 [-> k_conv_finish when K is split over workgroups]
 struct ConvPlan {
-    bool ln = false;                  // k_gemm_f32_ln: LayerNorm fused in front of the linear
     bool wide = false;
     int MTB = 1, W = 1;               // wide
     bool group = false;
@@ -384,11 +388,6 @@ int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
             default: launch_wide_w<4, 2>(s, w, p.W, p.group, grid); break;
         }
         if (p.ksplit > 1) MMI_LAUNCH(k_conv_finish, (int)mmi_cdiv64((int64_t)a.Cout * a.Ntot, 256), 256, 0, s, a, p.ksplit);
-        MMI_CHECK_LAUNCH();
-        return MMI_OK;
-    }
-    if (p.ln) {
-        MMI_LAUNCH((k_gemm_f32_ln<8, 8>), dim3(a.Mt, 1, p.nz), 512, 0, s, a);
         MMI_CHECK_LAUNCH();
         return MMI_OK;
     }
@@ -499,7 +498,7 @@ void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
 }
 
 // Decide the launch sequence of one conv and allocate its scratch (offset table / packed operand / partials) from
-// `mem`.  `a.x_packed`: the producer writes a.bp itself.  `a.out_mode` PACKED: the result feeds a linear directly.
+// `mem`.  `a.x_packed`: the producer writes a.bp itself.
 // A group's conv (mem.frames > 1) forms every sum in the order in which the frame program forms it - its reduction is cut into the same
 // pieces, over the waves and over the workgroups - so that frames give the same bits however many are run at once; only what each
 // workgroup covers follows the group's own number of columns.
@@ -541,15 +540,6 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
     }
     p->wide = false;                    // (at most 512 columns: T_shift is 0)
     const int nsub = mmi_cdiv(N, 32);
-    if (a.ln_w) {                       // fused LayerNorm + linear: one 32-column subtile per workgroup, the whole K in registers
-        if (!a.x_packed || a.Q > 64 || a.Q * 8 != a.Cin || a.K != 1 || a.out_mode == MMI_GOUT_PARTIAL)
-            return mmi_fail(MMI_ERR_UNSUPPORTED, "fused LayerNorm linear: unsupported shape");
-        p->ln = true;
-        p->NSUB = 1;
-        p->nz = nsub;
-        a.Npad = 32;
-        return MMI_OK;
-    }
     gemm_rule(a, N, p);
     a.Npad = (nsub <= 1 ? 1 : (nsub == 2 ? 2 : 4)) * 32;
     if (mem.frames > 1) {
@@ -592,7 +582,6 @@ ConvGemmArgs conv_args(const ConvW& w, const Buf& in, int x_off, int T_out, cons
     a.T_magic = mmi_div_magic(T_out, mmi_div_shift(T_out)); a.T_shift = mmi_div_shift(T_out); a.K_magic = mmi_div_magic(w.K);
     a.Mt = w.Mt; a.Q = w.Q; a.Ntot = B * T_out;
     a.elu_in = elu_in ? 1 : 0;
-    a.act_out = MMI_ACT_NONE;
     a.out_mode = MMI_GOUT_NATURAL;
     return a;
 }
@@ -653,9 +642,8 @@ int add_resblock(MimiMem& mem, MmiProgram& prog, ConvGemmArgs a1, ConvGemmArgs a
     // the chip) lost 2-15 us to the two-launch path's split-K over waves and are not instantiated.
     const bool fuse = a1.Ntot / mem.frames > 128 && a1.S == 1 && a2.K == 1 && a2.S == 1 && a1.Cout == a2.Cin && a1.Ntot == a2.Ntot &&
                       a1.T_out == a2.T_out && a1.Mt == 1 && w2.wpk_h && a2.Q <= 4 * a1.Mt &&
-                      a2.Mt >= a1.Mt && (long)mmi_cdiv(a1.Ntot / mem.frames, 32) * a1.Mt >= min_waves && !a1.first && !a2.first && !a1.res && !a1.scale && !a2.scale &&
-                      a1.T_out / mem.frames % 32 == 0 && a1.Cin <= 64 * a1.Mt && a1.K <= 33 &&
-                      a1.act_out == MMI_ACT_NONE && a2.act_out == MMI_ACT_NONE;
+                      a2.Mt >= a1.Mt && (long)mmi_cdiv(a1.Ntot / mem.frames, 32) * a1.Mt >= min_waves && !a1.first && !a2.first && !a1.res &&
+                      a1.T_out / mem.frames % 32 == 0 && a1.Cin <= 64 * a1.Mt && a1.K <= 33;
     if (!fuse) {
         int rc = add_conv(mem, prog, a1);
         if (rc) return rc;
@@ -750,32 +738,54 @@ int add_dequant_ops(mmi_mimi* m, MimiMem& mem, const DequantScratch& d, MmiProgr
     return add_conv(mem, prog, a);
 }
 
-// one streaming transformer (ProjectedTransformer with conv_layout, transformer.py:932-983) working in place
-// on x = buf[:, :, off:off+T], T = frames * (steps per frame)
-int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vector<TrLayerW>& layers, const Buf& xb, int off, int T,
+// the residual stream of a transformer as its linears' operand (mmi_lin_index); who produces the stream's input stores it there
+struct TrStream { float* p = nullptr; int J = 0; };
+int alloc_tr_stream(mmi_mimi* m, MimiMem& mem, int N, TrStream* x) {
+    const int d = m->cfg.tr_d_model;
+    x->J = mmi_cdiv(d, 16);
+    MMI_HIP_CHECK(mem.alloc(&x->p, (size_t)mmi_cdiv(N, 16) * x->J * 256));
+    MMI_HIP_CHECK(mem.clear_operand(x->p, mmi_cdiv(N, 16), x->J, d, 16));
+    return MMI_OK;
+}
+
+template <int FN>
+void launch_lin(hipStream_t s, const MimiLinArgs& a) {
+    const dim3 grid(mmi_cdiv(a.M, 16), mmi_cdiv(a.N, 16 * FN));
+    if (!a.ln_w) MMI_LAUNCH((k_mimi_lin<1, FN, (FN == 1 ? 8 : 4), false>), grid, 512, 0, s, a);
+    else if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<1, FN, 4, true>), grid, 512, 0, s, a);
+    else MMI_LAUNCH((k_mimi_lin<1, FN, 8, true>), grid, 512, 0, s, a);
+}
+
+int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
+    if (a.ln_w && (a.J > 64 || a.J * 16 != K)) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi transformer: a width of at most 1024, a multiple of 16");
+    // 16 columns per workgroup while the chip holds all workgroups at once (two per CU): 32 streams 1387 -> 1327 us a frame
+    // with 16 for 32.  Beyond that 32, which read the weights half as often (32 x 32 tiles measured no different).
+    const bool narrow = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16) <= 512;
+    prog.add([=](hipStream_t s) {
+        if (narrow) launch_lin<1>(s, a);
+        else launch_lin<2>(s, a);
+        MMI_CHECK_LAUNCH();
+        return (int)MMI_OK;
+    });
+    return MMI_OK;
+}
+
+// one streaming transformer (ProjectedTransformer with conv_layout, transformer.py:932-983) on the residual stream x, whose result goes to
+// buf[:, :, off:off+T] as well, T = frames * (steps per frame)
+int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vector<TrLayerW>& layers, const TrStream& x, const Buf& xb, int off, int T,
                     float* kv, const long* offsets, int B, int frames, hipStream_t init_stream) {
     const mmi_mimi_cfg& c = m->cfg;
     const int d = c.tr_d_model, H = c.tr_num_heads, Dh = d / H, ff = c.tr_dim_feedforward, cap = c.tr_context;
     const int N = B * T;
-    // At <= 128 columns (every real configuration: T = 2 per session) the linears run on k_gemm_f32 and the producers
-    // (LayerNorm, attention, linear1+GELU) write its packed operand directly; otherwise plain [B][C][T] buffers.
-    const bool packed = N <= 128 || frames > 1;
-    Buf y, qkv, att, hb;
+    Buf qkv;
     int rc;
-    if ((rc = alloc_buf(mem, B, d, 0, T, &y, init_stream))) return rc;
     if ((rc = alloc_buf(mem, B, 3 * d, 0, T, &qkv, init_stream))) return rc;
-    if ((rc = alloc_buf(mem, B, d, 0, T, &att, init_stream))) return rc;
-    if ((rc = alloc_buf(mem, B, ff, 0, T, &hb, init_stream))) return rc;
-    float *yp = nullptr, *attp = nullptr, *hbp = nullptr;
-    const int nsub = mmi_cdiv(N, 32), Qd = mmi_cdiv(d, 8), Qff = mmi_cdiv(ff, 8);
-    if (packed) {
-        MMI_HIP_CHECK(mem.alloc(&yp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(mem.alloc(&attp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(mem.alloc(&hbp, (size_t)nsub * Qff * 256));
-        MMI_HIP_CHECK(mem.clear_operand(yp, nsub, Qd, d));
-        MMI_HIP_CHECK(mem.clear_operand(attp, nsub, Qd, d));
-        MMI_HIP_CHECK(mem.clear_operand(hbp, nsub, Qff, ff));
-    }
+    float *attp = nullptr, *hbp = nullptr;
+    const int nt = mmi_cdiv(N, 16), Jd = x.J, Jff = mmi_cdiv(ff, 16);
+    MMI_HIP_CHECK(mem.alloc(&attp, (size_t)nt * Jd * 256));
+    MMI_HIP_CHECK(mem.alloc(&hbp, (size_t)nt * Jff * 256));
+    MMI_HIP_CHECK(mem.clear_operand(attp, nt, Jd, d, 16));
+    MMI_HIP_CHECK(mem.clear_operand(hbp, nt, Jff, ff, 16));
     const size_t kv_layer = (size_t)B * H * cap * Dh;
     if (T / frames > 2 || (Dh != 16 && Dh != 32 && Dh != 64))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: head dim 16/32/64 and 1 or 2 steps per frame are built");
@@ -786,44 +796,30 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
     const size_t rows_d = (size_t)B * H * T * Dh;
     float *qr = nullptr, *kvn = nullptr;
     if (frames > 1) {
-        if (!packed || !one_pass) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: too many columns or a too long context for several frames at once");
+        if (!one_pass) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: a too long context for several frames at once");
         MMI_HIP_CHECK(mem.alloc(&qr, rows_d));
         MMI_HIP_CHECK(mem.alloc(&kvn, 2 * rows_d * layers.size()));
     }
-    auto add_norm = [&](const float* w, const float* bb) {
-        const float* xp = xb.p; int xld = xb.ld; float* yn = y.p;
-        prog.add([=](hipStream_t s) {
-            MMI_LAUNCH(k_layernorm_ct, B * T, 64, 0, s, xp, xld, off, w, bb, yn, T, 0, d, T, 1e-5f, yp, Qd);
-            MMI_CHECK_LAUNCH();
-            return (int)MMI_OK;
-        });
+    auto lin = [&](const LinW& w, const float* in, int mode) {
+        MimiLinArgs a;
+        memset(&a, 0, sizeof(a));
+        a.w = w.w; a.x = in; a.M = w.M; a.N = N; a.J = w.J; a.mode = mode;
+        a.T = T; a.T_shift = mmi_div_shift(T); a.T_magic = mmi_div_magic(T, a.T_shift);
+        a.ln_eps = 1e-5f;
+        return a;
     };
-    // LayerNorm fused into the linear that consumes it (k_gemm_f32_ln): the producers of the residual stream inside the
-    // transformer (out_proj, linear2) also store it in packed operand order (xrp); only the very first norm, whose input
-    // comes from the conv stack, stays a launch of its own.  32 -> 2 norm launches per frame for the two transformers.
-    const bool fuse_ln = packed && d % 8 == 0 && Qd <= 64 && layers.size() > 0 && layers[0].n1w_pk;
-    float* xrp = nullptr;
-    if (fuse_ln) {
-        MMI_HIP_CHECK(mem.alloc(&xrp, (size_t)nsub * Qd * 256));
-        MMI_HIP_CHECK(mem.clear_operand(xrp, nsub, Qd, d));
-    }
-    bool x_is_packed = false;           // xrp holds the current residual stream
     for (size_t l = 0; l < layers.size(); ++l) {
         const TrLayerW& L = layers[l];
         {   // x = x + ls1 * out_proj(attn(norm1(x)))
-            ConvGemmArgs ai = conv_args(L.in_proj, y, 0, T, qkv, 0, B, false);
-            if (fuse_ln && x_is_packed) {
-                ai.x_packed = 1; ai.bp = xrp; ai.ln_w = L.n1w_pk; ai.ln_b = L.n1b_pk; ai.ln_eps = 1e-5f;
-            } else {
-                add_norm(L.n1w, L.n1b);
-                if (packed) { ai.x_packed = 1; ai.bp = yp; }
-            }
-            if ((rc = add_conv(mem, prog, ai))) return rc;
+            MimiLinArgs ai = lin(L.in_proj, x.p, MIMI_LIN_ROWS);
+            ai.ln_w = L.n1w; ai.ln_b = L.n1b;
+            ai.out = qkv.p; ai.out_ld = qkv.ld;
+            if ((rc = add_lin(prog, ai, L.in_proj.K))) return rc;
             MimiAttnArgs aa;
             aa.qkv = qkv.p; aa.kc = kv + (2 * l) * kv_layer; aa.vc = kv + (2 * l + 1) * kv_layer;
-            aa.offsets = offsets; aa.out = att.p; aa.B = B; aa.H = H; aa.D = Dh; aa.T = T; aa.cap = cap;
+            aa.offsets = offsets; aa.B = B; aa.H = H; aa.D = Dh; aa.T = T; aa.cap = cap;
             aa.context = c.tr_context; aa.max_period = c.tr_max_period;
-            aa.outp = attp; aa.outQ = Qd;
+            aa.outp = attp; aa.outJ = Jd;
             if (frames > 1) {
                 MimiGroupRows gr;
                 gr.T = T; gr.qkv_ld = qkv.ld; gr.q = qr; gr.kn = kvn + 2 * l * rows_d; gr.vn = gr.kn + rows_d;
@@ -856,28 +852,19 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
                 MMI_CHECK_LAUNCH();
                 return (int)MMI_OK;
             });
-            ConvGemmArgs a = conv_args(L.out_proj, att, 0, T, xb, off, B, false);
-            a.res = xb.p; a.res_ld = xb.ld; a.res_off = off; a.scale = L.ls1;
-            if (packed) { a.x_packed = 1; a.bp = attp; }
-            if (fuse_ln) { a.outp = xrp; a.outQ = Qd; x_is_packed = true; }      // dual store: [B][C][T] and packed
-            if ((rc = add_conv(mem, prog, a))) return rc;
+            MimiLinArgs a = lin(L.out_proj, attp, MIMI_LIN_RESID);
+            a.outp = x.p; a.outJ = x.J; a.scale = L.ls1;
+            if ((rc = add_lin(prog, a, L.out_proj.K))) return rc;
         }
         {   // x = x + ls2 * linear2(gelu(linear1(norm2(x))))
-            ConvGemmArgs a1 = conv_args(L.lin1, y, 0, T, hb, 0, B, false);
-            a1.act_out = MMI_ACT_GELU;
-            if (fuse_ln && x_is_packed) {
-                a1.x_packed = 1; a1.bp = xrp; a1.ln_w = L.n2w_pk; a1.ln_b = L.n2b_pk; a1.ln_eps = 1e-5f;
-                a1.out_mode = MMI_GOUT_PACKED; a1.outp = hbp; a1.outQ = Qff;
-            } else {
-                add_norm(L.n2w, L.n2b);
-                if (packed) { a1.x_packed = 1; a1.bp = yp; a1.out_mode = MMI_GOUT_PACKED; a1.outp = hbp; a1.outQ = Qff; }
-            }
-            if ((rc = add_conv(mem, prog, a1))) return rc;
-            ConvGemmArgs a2 = conv_args(L.lin2, hb, 0, T, xb, off, B, false);
-            a2.res = xb.p; a2.res_ld = xb.ld; a2.res_off = off; a2.scale = L.ls2;
-            if (packed) { a2.x_packed = 1; a2.bp = hbp; }
-            if (fuse_ln) { a2.outp = xrp; a2.outQ = Qd; x_is_packed = true; }
-            if ((rc = add_conv(mem, prog, a2))) return rc;
+            MimiLinArgs a1 = lin(L.lin1, x.p, MIMI_LIN_GELU);
+            a1.ln_w = L.n2w; a1.ln_b = L.n2b;
+            a1.outp = hbp; a1.outJ = Jff;
+            if ((rc = add_lin(prog, a1, L.lin1.K))) return rc;
+            MimiLinArgs a2 = lin(L.lin2, hbp, MIMI_LIN_RESID);
+            a2.outp = x.p; a2.outJ = x.J; a2.scale = L.ls2;
+            if (l + 1 == layers.size()) { a2.out = xb.p; a2.out_ld = xb.ld; a2.out_off = off; }      // what the convs behind read
+            if ((rc = add_lin(prog, a2, L.lin2.K))) return rc;
         }
     }
     if (frames > 1) {
@@ -1014,10 +1001,16 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     const int stride = c.resample_stride;
     Buf dsin;
     if ((rc = alloc_buf(mem, B, c.dimension, 2 * stride - stride, T, &dsin, s0))) return rc;
+    TrStream xs;
+    if ((rc = alloc_tr_stream(m, mem, B * T, &xs))) return rc;
     prog.site("enc.final");
-    if ((rc = add_conv(mem, prog, conv_args(m->enc_convs[ci++], cur, 0, T, dsin, dsin.H, B, true)))) return rc;
+    {
+        ConvGemmArgs a = conv_args(m->enc_convs[ci++], cur, 0, T, dsin, dsin.H, B, true);
+        a.outp = xs.p; a.outJ = xs.J;
+        if ((rc = add_conv(mem, prog, a))) return rc;
+    }
     hist.push_back(hist_of(dsin, T));
-    // encoder transformer, in place on dsin[:, :, H:H+T]
+    // encoder transformer, its result in dsin[:, :, H:H+T]
     {
         const int Dh = c.tr_d_model / c.tr_num_heads;
         size_t kvn = (size_t)2 * c.tr_num_layers * B * c.tr_num_heads * c.tr_context * Dh;
@@ -1026,7 +1019,7 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
             MMI_HIP_CHECK(mem.zero(m->enc_kv, kvn, s0));
         }
         prog.site("enc.tr");
-        if ((rc = add_transformer(m, mem, prog, m->enc_tr, dsin, dsin.H, T, m->enc_kv, m->counters, B, frames, s0))) return rc;
+        if ((rc = add_transformer(m, mem, prog, m->enc_tr, xs, dsin, dsin.H, T, m->enc_kv, m->counters, B, frames, s0))) return rc;
     }
     const int T_tr = T;
     // downsample (ConvDownsample1d learnt, replicate padding on the first frame)
@@ -1098,6 +1091,8 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     Buf din;
     if ((rc = alloc_buf(mem, B, c.dimension, c.kernel_size - 1, T, &din, s0))) return rc;
     hist.push_back(hist_of(din, T));
+    TrStream xs;
+    if ((rc = alloc_tr_stream(m, mem, B * T, &xs))) return rc;
     {
         float* part = nullptr;
         MMI_HIP_CHECK(partial((long)c.dimension * stride, &part));
@@ -1105,7 +1100,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
         float* out = din.p; int old = din.ld, ooff = din.H; int C = c.dimension; const int xld = lat.ld;
         prog.add([=](hipStream_t s) {
             MMI_LAUNCH(k_upsample_dw, mmi_cdiv(B * C * stride * frames, 256), 256, 0, s, x, xld, 0, w, part, ex, out, old, ooff, B, C,
-                       2 * stride, stride, frames);
+                       2 * stride, stride, frames, xs.p, xs.J);
             MMI_CHECK_LAUNCH();
             return (int)MMI_OK;
         });
@@ -1118,7 +1113,7 @@ int build_decoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
             MMI_HIP_CHECK(mem.zero(m->dec_kv, kvn, s0));
         }
         prog.site("dec.tr");
-        if ((rc = add_transformer(m, mem, prog, m->dec_tr, din, din.H, T, m->dec_kv, m->counters + B, B, frames, s0))) return rc;
+        if ((rc = add_transformer(m, mem, prog, m->dec_tr, xs, din, din.H, T, m->dec_kv, m->counters + B, B, frames, s0))) return rc;
     }
     const int T_tr = T;
     size_t ci = 0;

@@ -87,8 +87,6 @@ __global__ void k_codebook_prepare(const float* __restrict__ esum, const float* 
 //                projections; weights dominate).  Same shape as the LM's weight-streaming GEMM: one m-tile per
 //                workgroup, K split over waves (+ workgroups), activations pre-packed into B-fragment order by
 //                k_pack_b_f32 (im2col + ELU + replicate padding) or by the producing kernel.
-enum { MMI_ACT_NONE = 0, MMI_ACT_GELU = 1, MMI_ACT_ELU = 2 };
-
 // n / d for 0 <= n < 2^20 and 1 <= d < 2^20 (column and tap indices) as one multiply-high and a shift: an integer division costs
 // ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^(32 + shift) / d), 0 means d == 1; exact while
 // n d < 2^(32 + shift), hence the 8 more bits (which still fit the magic number) from d = 2^11 on.
@@ -97,7 +95,7 @@ MMI_HD unsigned mmi_div_magic(int d, unsigned shift = 0u) { return d <= 1 ? 0u :
 MMI_HD int mmi_fast_div(int n, unsigned magic, unsigned shift = 0u) {
     return magic == 0u ? n : (int)((unsigned)(((unsigned long long)(unsigned)n * magic) >> 32) >> shift);
 }
-enum { MMI_GOUT_NATURAL = 0, MMI_GOUT_PACKED = 1, MMI_GOUT_PARTIAL = 2 };
+enum { MMI_GOUT_NATURAL = 0, MMI_GOUT_PARTIAL = 1 };
 
 // k_conv_wide's offset table, see ConvGemmArgs::koff
 __global__ void k_conv_offsets(int* __restrict__ tab, int Q, int Cin, int K, int x_ld) {
@@ -119,7 +117,6 @@ struct ConvGemmArgs {
     int out_ld, out_off;
     const float* res;     // residual [B][Cout][res_ld] read at res_off + t, or null
     int res_ld, res_off;
-    const float* scale;   // LayerScale [Cout] or null: out = res + scale * (acc + bias)
     const uint8_t* first; // replicate-pad flags [B] or null (conv.py:253-259)
     const uint8_t* exec;  // exec mask [B] (only read with `first`)
     int B, Cin, Cout, K, S, T_out;
@@ -127,7 +124,6 @@ struct ConvGemmArgs {
     int Mt, Q;            // M tiles of 32, packed k-quads (Kdim_pad / 8)
     int Ntot;             // B * T_out
     int elu_in;           // apply ELU(alpha=1) to every loaded input (seanet.py:63,205,222)
-    int act_out;          // MMI_ACT_*
     // ELU hoisted out of the consumers: every SEANet conv but the first reads ELU(x) (seanet.py:63,205,222), and an audio-rate
     // conv reads each input K * (Cout / 32) times, so the PRODUCER applies it once per element: elu_out = 1 stores ELU(result)
     // instead of the result (buffers whose only readers are such convs), out2 != null additionally stores ELU(result) there
@@ -135,19 +131,13 @@ struct ConvGemmArgs {
     // as applying it at the consumer's load - bit-identical.
     int elu_out;
     float* out2;
-    // k_gemm_f32_ln: nn.LayerNorm over the Cin channels of every column fused in front of the linear (the Mimi transformer's
-    // norm1 -> in_proj and norm2 -> linear1): `bp` then holds the RAW residual stream in packed order, ln_w / ln_b the norm's
-    // weight and bias in the operand's element order (k_pack_ln), ln_eps its epsilon
-    const float* ln_w;
-    const float* ln_b;
-    float ln_eps;
     // --- filled in by the engine's planner
     const int* koff;      // k_conv_wide: [Q][2][4] input offset of kd = (q*4+e)*2 + h; 0 past Cin*K (the weights there are 0)
     const float* bp;      // k_gemm_f32: packed activations [ceil(N/32)][Q][64][4]
     int x_packed;         // the producer already wrote `bp` (no k_pack_b_f32 launch)
     int out_mode;         // MMI_GOUT_*
-    float* outp;          // GOUT_PACKED: packed B operand of the consuming linear, [ceil(N/32)][outQ][64][4]
-    int outQ;
+    float* outp;          // packed B operand of the consumer, also stored: [ceil(N/32)][outQ][64][4], or with outJ the transformers'
+    int outQ, outJ;       //   fragments of 16 columns (mmi_lin_index)
     float* partial;       // GOUT_PARTIAL: [gridDim.y][Mt*32][Npad] raw sums, finished by k_conv_finish
     int Npad;
     // groups of frames: T_magic = mmi_div_magic(T_out, T_shift), 0 where T_out < 2^11; quads per workgroup of a split reduction (Q: not split)
@@ -163,27 +153,29 @@ __device__ __forceinline__ long mmi_bp_index(int kd, int n, int Q) {
     return ((((long)(n >> 5) * Q + (kd >> 3)) * 64) + (kd & 1) * 32 + (n & 31)) * 4 + ((kd & 7) >> 1);
 }
 
-// bias / activation / LayerScale / residual, then the store to [B][Cout][out_ld] - shared by the epilogues.
+// element (k, n) of a transformer linear's operand, fragments of 16 columns x 16 reduction indices (J of them): lane (k & 3, n) of
+// fragment k / 16 holds k = 4 e + its own quarter at element e, so that four v_mfma_f32_16x16x4_f32 walk them in rising order
+MMI_HD long mmi_lin_index(int k, int n, int J) {
+    return ((((long)(n >> 4) * J + (k >> 4)) * 64) + (k & 3) * 16 + (n & 15)) * 4 + ((k >> 2) & 3);
+}
+
+// bias / residual, then the store to [B][Cout][out_ld] - shared by the epilogues.
 // NV results of one thread are finished together: all bias / scale / residual loads are issued first (under branches
 // that are uniform for the launch), so that the epilogue costs one memory round trip instead of NV of them.
 template <int NV>
 __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
                                                  const bool (&ok)[NV], float (&v)[NV]) {
-    float bia[NV], scl[NV], rsv[NV];
+    float bia[NV], rsv[NV];
     long row[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int cc = ok[i] ? co[i] : 0;
         row[i] = (long)(ok[i] ? b[i] : 0) * a.Cout + cc;
-        bia[i] = 0.f; scl[i] = 1.f; rsv[i] = 0.f;
+        bia[i] = 0.f; rsv[i] = 0.f;
     }
     if (a.bias) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) bia[i] = a.bias[ok[i] ? co[i] : 0];
-    }
-    if (a.scale) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) scl[i] = a.scale[ok[i] ? co[i] : 0];
     }
     if (a.res) {
 #pragma unroll
@@ -194,17 +186,6 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
     if (a.bias) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) v[i] += bia[i];
-    }
-    if (a.act_out == MMI_ACT_GELU) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] = mmi_gelu_erf(v[i]);
-    } else if (a.act_out == MMI_ACT_ELU) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] = mmi_elu(v[i]);
-    }
-    if (a.scale) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] *= scl[i];
     }
     if (a.res) {
 #pragma unroll
@@ -228,13 +209,13 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
         for (int i = 0; i < NV; ++i)
             if (ok[i]) a.out[at[i]] = v[i];
     }
-    // also stored as the packed operand of the consuming linear (what `out` holds: the ELU'd value where that is what is stored):
-    // the residual stream of the Mimi transformers for the next fused norm + linear, the decoder's first conv for the first
-    // transposed-conv GEMM, the latent for the RVQ input projection - no k_pack_b_f32 launch in between
+    // also stored as the packed operand of the consumer (what `out` holds: the ELU'd value where that is what is stored): the encoder's
+    // last conv for its transformer, the decoder's first conv for the first transposed-conv GEMM, the latent for the RVQ input projection -
+    // no launch that packs in between
     if (a.outp && a.out_mode == MMI_GOUT_NATURAL) {
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-            if (ok[i]) a.outp[mmi_bp_index(co[i], b[i] * a.T_out + t[i], a.outQ)] = v[i];
+            if (ok[i]) a.outp[a.outJ ? mmi_lin_index(co[i], b[i] * a.T_out + t[i], a.outJ) : mmi_bp_index(co[i], b[i] * a.T_out + t[i], a.outQ)] = v[i];
     }
 }
 
@@ -606,7 +587,7 @@ __global__ void k_pack_b_f32(ConvGemmArgs a, float* __restrict__ bp) {
     reinterpret_cast<f32x4*>(bp)[idx] = o;
 }
 
-// split-K reduction over the workgroup's waves (fixed order) + the epilogue of k_gemm_f32 / k_gemm_f32_ln
+// split-K reduction over the workgroup's waves (fixed order) + the epilogue of k_gemm_f32
 template <int NSUB, int WAVES>
 __device__ __forceinline__ void mmi_gemm_f32_finish(const ConvGemmArgs& a, f32x16 (&acc)[NSUB], int mt, int s0, int wave, int lane) {
     constexpr int NE = NSUB * 16 * 64;
@@ -633,21 +614,6 @@ __device__ __forceinline__ void mmi_gemm_f32_finish(const ConvGemmArgs& a, f32x1
     if (a.out_mode == MMI_GOUT_PARTIAL) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) a.partial[((long)blockIdx.y * a.Mt * 32 + co[i]) * a.Npad + nn[i]] = v[i];   // padded rows / columns included
-        return;
-    }
-    if (a.out_mode == MMI_GOUT_PACKED) {
-        float bia[NV];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) bia[i] = a.bias ? a.bias[co[i] < a.Cout ? co[i] : 0] : 0.f;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            if (nn[i] >= a.Ntot || co[i] >= a.Cout) continue;
-            float x = v[i];
-            if (a.bias) x += bia[i];
-            if (a.act_out == MMI_ACT_GELU) x = mmi_gelu_erf(x);
-            else if (a.act_out == MMI_ACT_ELU) x = mmi_elu(x);
-            a.outp[mmi_bp_index(co[i], nn[i], a.outQ)] = x;
-        }
         return;
     }
     int bb[NV], tt[NV];
@@ -730,81 +696,221 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_f32(ConvGemmArgs a) {
     mmi_gemm_f32_finish<NSUB, WAVES>(a, acc, mt, s0, wave, lane);
 }
 
-// LayerNorm fused in front of a Mimi transformer linear (norm1 -> in_proj, norm2 -> linear1; transformer.py:125-126,
-// 752-776): grid (Mt, 1, n-subtiles), one 32-column subtile per workgroup; the 8 waves split the Cin / 8 <= 8 * KQ k-quads and
-// hold their whole slice - raw residual-stream fragments, weight fragments, the norm's weight / bias - in registers (everything
-// in flight at once: these GEMMs are latency bound).  Column statistics: per-wave partial sums of the lane's column, the two
-// lane halves folded by one shuffle, the 8 waves through LDS; mean first, then sum (x - mean)^2 (two-pass, like
-// k_layernorm_ct), y = (x - mean) * rsqrt(var + eps) * w + b, then the MFMAs.  Needs Q * 8 == Cin (no padded channels).
-template <int WAVES, int KQ>
-__global__ __launch_bounds__(WAVES * 64) void k_gemm_f32_ln(ConvGemmArgs a) {
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-    const int mt = blockIdx.x, s0 = blockIdx.z;
-    const int qper = (a.Q + WAVES - 1) / WAVES;            // <= KQ (checked by the planner)
-    const int q0 = min(a.Q, wave * qper);
-    const int nq = min(a.Q, q0 + qper) - q0;
-    const int kh = lane >> 5;
-    const int ql = min(q0, a.Q - 1);
-    f32x4 wv[KQ], xv[KQ], gv[KQ], bv[KQ];
-    const f32x4* wp = reinterpret_cast<const f32x4*>(a.wpk) + ((long)mt * a.Q + ql) * 64 + lane;
-    const f32x4* bp = reinterpret_cast<const f32x4*>(a.bp) + ((long)s0 * a.Q + ql) * 64 + lane;
-    const f32x4* gp = reinterpret_cast<const f32x4*>(a.ln_w) + (long)ql * 2 + kh;
-    const f32x4* hp = reinterpret_cast<const f32x4*>(a.ln_b) + (long)ql * 2 + kh;
-#pragma unroll
-    for (int u = 0; u < KQ; ++u) {                         // unconditional loads from clamped (valid) quads, masked afterwards
-        const int uu = min(u, nq > 0 ? nq - 1 : 0);
-        xv[u] = bp[(long)uu * 64];
-        wv[u] = mmi_load_nt(wp + (long)uu * 64);
-        gv[u] = gp[(long)uu * 2];
-        bv[u] = hp[(long)uu * 2];
-    }
-    MMI_SHARED float stat[2][WAVES][32];
-    float s1 = 0.f;
-#pragma unroll
-    for (int u = 0; u < KQ; ++u)
-        if (u < nq) s1 += (xv[u][0] + xv[u][1]) + (xv[u][2] + xv[u][3]);
-    s1 += mmi_shfl_xor(s1, 32);
-    if (lane < 32) stat[0][wave][lane] = s1;
-    __syncthreads();
-    float tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) tot += stat[0][w][lane & 31];
-    const float mean = tot / (float)a.Cin;
-    float s2 = 0.f;
-#pragma unroll
-    for (int u = 0; u < KQ; ++u)
-        if (u < nq) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { const float dlt = xv[u][e] - mean; s2 += dlt * dlt; }
-        }
-    s2 += mmi_shfl_xor(s2, 32);
-    if (lane < 32) stat[1][wave][lane] = s2;
-    __syncthreads();
-    float var = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) var += stat[1][w][lane & 31];
-    const float rstd = mmi_rsqrtf(var / (float)a.Cin + a.ln_eps);
-    f32x16 acc[1];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[0][r] = 0.f;
-#pragma unroll
-    for (int u = 0; u < KQ; ++u)
-        if (u < nq) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float y = (xv[u][e] - mean) * rstd * gv[u][e] + bv[u][e];
-                acc[0] = mmi_mfma_f32_32x32x2(wv[u][e], y, acc[0]);
-            }
-        }
-    mmi_gemm_f32_finish<1, WAVES>(a, acc, mt, s0, wave, lane);
+// ------------------------------------------------------------------------------------------------
+// linears of the Mimi transformers
+// ------------------------------------------------------------------------------------------------
+// W[m][k] (m < M, k < K) -> P[ceil(M/16)][J][lane][e], element (row, k) where mmi_lin_index has (k, column); zero padded
+__global__ void k_pack_lin(const float* __restrict__ W, float* __restrict__ P, int M, int K, int Mt, int J) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (long)Mt * J * 256) return;
+    const int e = (int)(idx & 3), lane = (int)((idx >> 2) & 63);
+    const long f = idx >> 8;
+    const int j = (int)(f % J), m = (int)(f / J) * 16 + (lane & 15), k = 16 * j + 4 * e + (lane >> 4);
+    P[idx] = m < M && k < K ? W[(long)m * K + k] : 0.f;
 }
-
-// LayerNorm weight / bias [C] -> the element order of the packed operand: out[(q * 2 + kh) * 4 + e] = v[(q * 4 + e) * 2 + kh]
+// LayerNorm weight / bias [C] in the operand's element order: out[(j * 4 + quarter) * 4 + e] = v[16 j + 4 e + quarter]; C % 16 == 0
 __global__ void k_pack_ln(const float* __restrict__ v, float* __restrict__ out, int C) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= C) return;
-    const int e = i & 3, kh = (i >> 2) & 1, q = i >> 3;
-    out[i] = v[(q * 4 + e) * 2 + kh];
+    if (i < C) out[i] = v[16 * (i >> 4) + 4 * (i & 3) + ((i >> 2) & 3)];
+}
+
+enum { MIMI_LIN_ROWS = 0, MIMI_LIN_GELU = 1, MIMI_LIN_RESID = 2 };
+struct MimiLinArgs {
+    const float* w;              // [Mt][J] fragments (k_pack_lin)
+    const float* x;              // [ceil(N/16)][J] fragments (mmi_lin_index)
+    int M, N, J;                 // rows, columns n = b * T + t, 16-deep pieces of the reduction
+    const float *ln_w, *ln_b;    // LayerNorm over the 16 J values of a column in front (k_pack_ln)
+    float ln_eps;
+    int mode;                    // ROWS: out = W x;  GELU: outp = gelu(W x);  RESID: outp += scale * W x (the residual stream), and out too where it is set
+    float* outp;
+    int outJ;
+    const float* scale;
+    float* out;                  // [B][M][out_ld] from column out_off on
+    int out_ld, out_off, T;
+    unsigned T_magic, T_shift;
+};
+
+// out[m][n] = sum_k W[m][k] x[k][n] on v_mfma_f32_16x16x4_f32 (an exact fma chain), LayerNorm of the columns in front where LN.
+// grid (ceil(Mt/FM), ceil(N/(16 FN))); a workgroup owns 16 FM rows x 16 FN columns; its 8 waves cut the reduction into 8 pieces, their sums are
+// added in rising order.  What a workgroup covers changes no bit (a piece and its order are the reduction's alone), so one stream, many
+// streams and groups of frames agree.
+// Measured, 1 stream (N = 2): norm + linear 8.2 -> 5.1 us, K = 2048 9.3 (with its second launch) -> 6.9; 32 streams (N = 64) 8.4 -> 7.3, 9.6 -> 7.5;
+// a file's 258 columns: norm + linear 18.6 -> 18.7, K = 2048 19.2 -> 16.
+// Bound by latency: one column tile has M / 16 workgroups of 16 KB - 64 KB of weights and a few hundred cycles of matrix work each.  Hence
+// 16-wide tiles (a live stream has two columns: a 32-wide tile keeps the matrix core busy four times as long, 1.7 us at K = 512, on half the
+// CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (KJ fragments per wave), and
+// no reduction split over workgroups (K = 2048 needed a second launch to add the sums).
+template <int FM, int FN, int U, bool LN>
+__global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int m0 = (int)blockIdx.x * FM, n0 = (int)blockIdx.y * FN;
+    const int Mt = (a.M + 15) >> 4, Nt = (a.N + 15) >> 4;
+    const int per = (a.J + 7) >> 3;                          // LN: <= U (the planner checks)
+    const int j0 = min(a.J, wave * per), nj = min(a.J, j0 + per) - j0;
+    const int jl = min(j0, a.J - 1), last = nj > 0 ? nj - 1 : 0;
+    const f32x4* wp[FM];
+    const f32x4* xp[FN];
+#pragma unroll
+    for (int m = 0; m < FM; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.w) + ((long)min(m0 + m, Mt - 1) * a.J + jl) * 64 + lane;
+#pragma unroll
+    for (int n = 0; n < FN; ++n)                             // (a column past the last one reads the last one: nobody need have stored it)
+        xp[n] = reinterpret_cast<const f32x4*>(a.x) + ((long)min(n0 + n, Nt - 1) * a.J + jl) * 64 + (lane & 48) + min(lane & 15, max(a.N - (n0 + n) * 16, 1) - 1);
+
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int m = 0; m < FM; ++m)
+#pragma unroll
+        for (int n = 0; n < FN; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // results of this thread: element idx & 255 of tile idx >> 8, idx = tid + 512 i.  In operand order (GELU, RESID) that is the tile's place in
+    // outp; in the accumulators' order (ROWS) 16 columns of a row lie side by side.
+    constexpr int NV = (FM * FN + 1) / 2;
+    int rm[NV], rn[NV];
+    float scl[NV], res[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int idx = tid + 512 * i, f = idx >> 8, q = idx & 255;
+        const int row = a.mode == MIMI_LIN_ROWS ? 4 * ((q >> 4) & 3) + (q >> 6) : 4 * (q & 3) + (q >> 6);
+        rm[i] = (m0 + f / FN) * 16 + row;
+        rn[i] = (n0 + f % FN) * 16 + (a.mode == MIMI_LIN_ROWS ? q & 15 : (q >> 2) & 15);
+        if (idx >= FM * FN * 256 || rm[i] >= a.M) rn[i] = a.N;          // nothing to store
+        scl[i] = 0.f; res[i] = 0.f;
+    }
+    if (a.mode == MIMI_LIN_RESID) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const bool ok = rn[i] < a.N;
+            scl[i] = a.scale[ok ? rm[i] : 0];
+            res[i] = a.outp[ok ? mmi_lin_index(rm[i], rn[i], a.outJ) : 0];
+        }
+    }
+
+    if constexpr (LN) {
+        MMI_SHARED float stat[2][8][FN * 16];
+        const f32x4* gp = reinterpret_cast<const f32x4*>(a.ln_w) + (long)jl * 4 + (lane >> 4);
+        const f32x4* hp = reinterpret_cast<const f32x4*>(a.ln_b) + (long)jl * 4 + (lane >> 4);
+        f32x4 wv[U][FM], xv[U][FN], gv[U], bv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {                        // unconditional loads from clamped (valid) places, masked afterwards
+            const int uu = min(u, last);
+#pragma unroll
+            for (int n = 0; n < FN; ++n) xv[u][n] = xp[n][uu * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int uu = min(u, last);
+#pragma unroll
+            for (int m = 0; m < FM; ++m) wv[u][m] = mmi_load_nt(wp[m] + uu * 64);
+            gv[u] = gp[uu * 4];
+            bv[u] = hp[uu * 4];
+        }
+        auto column_sum = [&](int which, float (&s)[FN]) __attribute__((always_inline)) {      // over the lanes that hold a column, then over the waves
+#pragma unroll
+            for (int n = 0; n < FN; ++n) {
+                s[n] += mmi_shfl_xor(s[n], 16);
+                s[n] += mmi_shfl_xor(s[n], 32);
+                if (lane < 16) stat[which][wave][n * 16 + lane] = s[n];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int n = 0; n < FN; ++n) {
+                float t = 0.f;
+#pragma unroll
+                for (int w = 0; w < 8; ++w) t += stat[which][w][n * 16 + (lane & 15)];
+                s[n] = t;
+            }
+        };
+        float mean[FN], rstd[FN];
+#pragma unroll
+        for (int n = 0; n < FN; ++n) mean[n] = rstd[n] = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < nj)
+#pragma unroll
+                for (int n = 0; n < FN; ++n) mean[n] += (xv[u][n][0] + xv[u][n][1]) + (xv[u][n][2] + xv[u][n][3]);
+        column_sum(0, mean);
+#pragma unroll
+        for (int n = 0; n < FN; ++n) mean[n] /= (float)(a.J * 16);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < nj)
+#pragma unroll
+                for (int n = 0; n < FN; ++n)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float d = xv[u][n][e] - mean[n];
+                        rstd[n] += d * d;
+                    }
+        column_sum(1, rstd);
+#pragma unroll
+        for (int n = 0; n < FN; ++n) rstd[n] = mmi_rsqrtf(rstd[n] / (float)(a.J * 16) + a.ln_eps);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < nj)
+#pragma unroll
+                for (int n = 0; n < FN; ++n)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float y = (xv[u][n][e] - mean[n]) * rstd[n] * gv[u][e] + bv[u][e];
+#pragma unroll
+                        for (int m = 0; m < FM; ++m) acc[m][n] = mmi_mfma_f32_16x16x4(wv[u][m][e], y, acc[m][n]);
+                    }
+    } else {
+        f32x4 wA[U][FM], xA[U][FN], wB[U][FM], xB[U][FN];
+        auto load = [&](f32x4 (&w)[U][FM], f32x4 (&x)[U][FN], int at) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int uu = min(at + u, last);
+#pragma unroll
+                for (int m = 0; m < FM; ++m) w[u][m] = mmi_load_nt(wp[m] + (long)uu * 64);
+#pragma unroll
+                for (int n = 0; n < FN; ++n) x[u][n] = xp[n][(long)uu * 64];
+            }
+        };
+        auto mma = [&](const f32x4 (&w)[U][FM], const f32x4 (&x)[U][FN], int at) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (at + u < nj)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int m = 0; m < FM; ++m)
+#pragma unroll
+                            for (int n = 0; n < FN; ++n) acc[m][n] = mmi_mfma_f32_16x16x4(w[u][m][e], x[u][n][e], acc[m][n]);
+        };
+        load(wA, xA, 0);
+        for (int at = 0; at < nj; at += 2 * U) {
+            load(wB, xB, at + U);
+            mma(wA, xA, at);
+            if (at + 2 * U < nj) load(wA, xA, at + 2 * U);
+            mma(wB, xB, at + U);
+        }
+    }
+
+    MMI_SHARED float red[8 * FM * FN * 256];
+#pragma unroll
+    for (int m = 0; m < FM; ++m)
+#pragma unroll
+        for (int n = 0; n < FN; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[((wave * FM + m) * FN + n) * 256 + r * 64 + lane] = acc[m][n][r];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int idx = tid + 512 * i, q = idx & 255;
+        if (rn[i] >= a.N) continue;
+        const int at = (idx & ~255) + (a.mode == MIMI_LIN_ROWS ? q : (q >> 6) * 64 + (q & 3) * 16 + ((q >> 2) & 15));
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) v += red[w * FM * FN * 256 + at];
+        if (a.mode == MIMI_LIN_GELU) v = mmi_gelu_erf(v);
+        if (a.mode == MIMI_LIN_RESID) v = res[i] + scl[i] * v;
+        if (a.mode != MIMI_LIN_ROWS) a.outp[mmi_lin_index(rm[i], rn[i], a.outJ)] = v;
+        if (a.out) {
+            const int b = mmi_fast_div(rn[i], a.T_magic, a.T_shift), t = rn[i] - b * a.T;
+            a.out[((long)b * a.M + rm[i]) * a.out_ld + a.out_off + t] = v;
+        }
+    }
 }
 
 // sum of the split-K partials + epilogue -> [B][Cout][out_ld]
@@ -867,7 +973,7 @@ __global__ void k_convtr_combine(const float* __restrict__ tmp, const float* __r
 // depthwise (groups == C) transposed conv, K == 2*S, no bias: ConvTrUpsample1d (resample.py:68-119)
 __global__ void k_upsample_dw(const float* __restrict__ x, int x_ld, int x_off, const float* __restrict__ w,
                               float* __restrict__ partial, const uint8_t* __restrict__ exec, float* __restrict__ out,
-                              int out_ld, int out_off, int B, int C, int K, int S, int T_in) {
+                              int out_ld, int out_off, int B, int C, int K, int S, int T_in, float* __restrict__ outp, int outJ) {
     long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int Tout = T_in * S;
     if (idx >= (long)B * C * Tout) return;
@@ -885,6 +991,7 @@ __global__ void k_upsample_dw(const float* __restrict__ x, int x_ld, int x_off, 
         if (exec[b]) partial[pi] = w[c * K + r + S] * xr[T_in - 1];
     }
     out[row * (long)out_ld + out_off + p] = v;
+    outp[mmi_lin_index(c, b * Tout + p, outJ)] = v;        // the transformer's residual stream
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1004,64 +1111,17 @@ __global__ void k_set_mask(uint8_t* __restrict__ dst, const uint8_t* __restrict_
 // ------------------------------------------------------------------------------------------------
 // Mimi transformer pieces ([B][C][T] layout)
 // ------------------------------------------------------------------------------------------------
-// nn.LayerNorm(C, eps) over the channel axis of x[b][:, off + t]  (transformer.py:125-126)
-__global__ __launch_bounds__(64) void k_layernorm_ct(const float* __restrict__ x, int x_ld, int x_off,
-                                                     const float* __restrict__ w, const float* __restrict__ bvec,
-                                                     float* __restrict__ y, int y_ld, int y_off, int C, int T,
-                                                     float eps, float* __restrict__ yp, int yQ) {
-    const int b = blockIdx.x / T, t = blockIdx.x % T;
-    const int lane = threadIdx.x;
-    const float* xc = x + (long)b * C * x_ld + x_off + t;
-    constexpr int NR = 16;                 // channels per lane held in registers (C <= 1024), one round of loads
-    float xv[NR], wv[NR], bv[NR];          // weight and bias ride along with the input: one memory round trip in all
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const int c = lane + i * 64;
-        const int cc = c < C ? c : 0;
-        xv[i] = xc[(long)cc * x_ld];
-        wv[i] = w[cc];
-        bv[i] = bvec[cc];
-    }
-#pragma unroll
-    for (int i = 0; i < NR; ++i) s += (lane + i * 64) < C ? xv[i] : 0.f;
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) s += mmi_shfl_xor(s, m);
-    const float mean = s / (float)C;
-    float v = 0.f;
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const float d = xv[i] - mean;
-        v += (lane + i * 64) < C ? d * d : 0.f;
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += mmi_shfl_xor(v, m);
-    const float rstd = mmi_rsqrtf(v / (float)C + eps);
-    float* yc = y + (long)b * C * y_ld + y_off + t;
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const int c = lane + i * 64;
-        if (c < C) {
-            const float o = (xv[i] - mean) * rstd * wv[i] + bv[i];
-            if (yp) yp[mmi_bp_index(c, blockIdx.x, yQ)] = o;   // packed B operand of the consuming linear (column n = b*T + t)
-            else yc[(long)c * y_ld] = o;
-        }
-    }
-}
-
 // RoPE (rope.py:11-82, interleaved) on q,k + ring-KV write (transformer.py:236-253) + masked attention over the
 // valid part of the ring (transformer.py:574-585).  One block per (b, head); T queries (T <= 8).
 //   qkv  [B][3*H*D][T]  rows: q = h*D + d, k = H*D + h*D + d, v = 2*H*D + h*D + d   (transformer.py:557-559)
 //   kc/vc [B][H][cap][D];  offsets[b] = tokens seen so far (== RingKVCache.end_offset == MHA offset)
-//   out  [B][H*D][T]
 struct MimiAttnArgs {
     const float* qkv;
     float* kc;
     float* vc;
     const long* offsets;
-    float* out;
-    float* outp;   // when set: packed B operand of out_proj (feature h*D+d, column b*T+t) instead of `out`
-    int outQ;
+    float* outp;   // operand of out_proj (mmi_lin_index: feature h*D+d, column b*T+t)
+    int outJ;
     int B, H, D, T, cap, context;
     float max_period;
 };
@@ -1207,8 +1267,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn(MimiAttnArgs a) {
         float s = 0.f;
 #pragma unroll 8
         for (int r = 0; r < RPB; ++r) s += red[(r * T + t) * D + d];
-        if (a.outp) a.outp[mmi_bp_index(h * D + d, b * T + t, a.outQ)] = s;
-        else a.out[((long)b * HD + h * D + d) * T + t] = s;
+        a.outp[mmi_lin_index(h * D + d, b * T + t, a.outJ)] = s;
     }
 }
 
@@ -1378,9 +1437,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_1pass(MimiAttnArgs a, MimiGro
             den += f * sw[w * T + t];
         }
         const float o = num / den;
-        if constexpr (GROUP) a.outp[mmi_bp_index(h * D + d, b * g.T + (int)blockIdx.y * T + t, a.outQ)] = o;
-        else if (a.outp) a.outp[mmi_bp_index(h * D + d, b * T + t, a.outQ)] = o;
-        else a.out[((long)b * HD + h * D + d) * T + t] = o;
+        a.outp[mmi_lin_index(h * D + d, GROUP ? b * g.T + (int)blockIdx.y * T + t : b * T + t, a.outJ)] = o;
     }
 }
 

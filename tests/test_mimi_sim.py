@@ -141,3 +141,12 @@ def test_c2_recipe_on_the_tiny_codec(factory):
     same case the GPU suite runs at full size for 200 frames (tests/test_a_mimi_gpu.py)."""
     res = mimi_cases.check_c2_recipe(factory, "cpu", tiny_mimi_config(), B=4, F=14, K=5)
     assert res["wrapped"]
+
+
+@pytest.mark.parametrize("heads,Dh,ff,B", [(2, 16, 40, 1), (2, 64, 72, 9), (9, 64, 48, 2), (5, 16, 528, 17)])
+def test_transformer_linears(factory, heads, Dh, ff, B):
+    """k_mimi_lin where its tiles are cut: rows, columns (2, 18, 34) and reductions (40, 72, 528) that are no multiple of 16, pieces of the
+    reduction that some waves have none of, a norm over more than 512 channels."""
+    from dataclasses import replace
+    cfg = replace(tiny_mimi_config(), dimension=heads * Dh, tr_d_model=heads * Dh, tr_num_heads=heads, tr_dim_feedforward=ff)
+    mimi_cases.oracle_vs_engine(lambda sd, cfg, K: factory(sd, cfg, K, max_batch=B), "cpu", cfg, seed=70 + heads, B=B, F=2, K=2)
