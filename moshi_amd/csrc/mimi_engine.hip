@@ -791,7 +791,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
         return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: head dim 16/32/64 and 1 or 2 steps per frame are built");
     const size_t attn_smem = ((size_t)T * Dh + (((size_t)T * cap + 3) & ~(size_t)3) + (size_t)(256 / (Dh / 4)) * T * Dh + 8) * sizeof(float);
     // one memory round trip when a thread's 16 row slots cover the ring (the Mimi shape: 250 slots of 64 floats)
-    const bool one_pass = cap <= 16 * (256 / (Dh / 4)) && !getenv("MMI_MIMI_ATTN_TWO_PASS");
+    const bool one_pass = cap <= 8 * (512 / (Dh / 4)) && !getenv("MMI_MIMI_ATTN_TWO_PASS");
     // several frames at once: queries, keys and values row by row (the layers' keys and values until the ring takes them all at the end)
     const size_t rows_d = (size_t)B * H * T * Dh;
     float *qr = nullptr, *kvn = nullptr;
@@ -827,7 +827,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
                 const dim3 grid_r(B * H, mmi_cdiv(T, MIMI_ROPE_T)), grid_a(B * H, frames);
                 prog.add([=](hipStream_t s) {
 #define MMI_ATT(D_, T_) do { MMI_LAUNCH((k_mimi_group_rope<D_>), grid_r, 256, 0, s, aa, gr); \
-                             MMI_LAUNCH((k_mimi_attn_1pass<D_, T_, true>), grid_a, 256, 0, s, aa, gr); } while (0)
+                             MMI_LAUNCH((k_mimi_attn_1pass<D_, T_, true>), grid_a, 512, 0, s, aa, gr); } while (0)
                     if (Dh == 64 && tpf == 2) MMI_ATT(64, 2);
                     else if (Dh == 64) MMI_ATT(64, 1);
                     else if (Dh == 32 && tpf == 2) MMI_ATT(32, 2);
@@ -839,7 +839,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
                     return (int)MMI_OK;
                 });
             } else prog.add([=](hipStream_t s) {
-#define MMI_ATT(D_, T_) do { if (one_pass) MMI_LAUNCH((k_mimi_attn_1pass<D_, T_>), B * H, 256, 0, s, aa, MimiGroupRows()); \
+#define MMI_ATT(D_, T_) do { if (one_pass) MMI_LAUNCH((k_mimi_attn_1pass<D_, T_>), B * H, 512, 0, s, aa, MimiGroupRows()); \
                              else MMI_LAUNCH((k_mimi_attn<D_, T_>), B * H, 256, attn_smem, s, aa); } while (0)
                 if (Dh == 64 && T == 2) MMI_ATT(64, 2);
                 else if (Dh == 64 && T == 1) MMI_ATT(64, 1);

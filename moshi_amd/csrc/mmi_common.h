@@ -10,6 +10,8 @@
 #include <string>
 #include <vector>
 #include <functional>
+#include <type_traits>
+#include <utility>
 
 #define MMI_HD __host__ __device__ __forceinline__
 MMI_HD uint16_t mmi_f32_to_bf16_bits(float f);
@@ -29,6 +31,12 @@ MMI_HD uint16_t mmi_f32_to_bf16(float f) { return mmi_cvt_bf16(f); }
 MMI_HD uint32_t mmi_pack_bf16x2(float lo, float hi) { return mmi_cvt_pk_bf16(lo, hi); }
 // round an fp32 value to the nearest bf16 and return it widened again ("bf16 rounding point")
 MMI_HD float mmi_round_bf16(float f) { return mmi_bf16_to_f32(mmi_f32_to_bf16(f)); }
+
+// f(std::integral_constant<int, 0>()), ..., f(std::integral_constant<int, N - 1>()): a loop whose index is a constant in every pass
+template <class F, int... I>
+__device__ __forceinline__ void mmi_static_for(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
+template <int N, class F>
+__device__ __forceinline__ void mmi_static_for(F&& f) { mmi_static_for(f, std::make_integer_sequence<int, N>()); }
 
 static inline int mmi_cdiv(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t mmi_cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -86,6 +86,32 @@ __device__ __forceinline__ float mmi_rows_max(float x) {
     const unsigned b0 = b[0], b1 = b[1];
     return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
 }
+// the sum over the same four lanes
+__device__ __forceinline__ float mmi_rows_sum(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned a0 = a[0], a1 = a[1];
+    const unsigned w = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, a0) + __builtin_bit_cast(float, a1));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    const unsigned b0 = b[0], b1 = b[1];
+    return __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+}
+// maximum over the whole wave, every lane gets it
+__device__ __forceinline__ float mmi_wave_max_f32(float x) {
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true)));
+    return mmi_rows_max(x);
+}
+// x of lane K of every group of W lanes (W = 4, 8, 16), to the whole group
+template <int W, int K>
+__device__ __forceinline__ float mmi_group_bcast(float x) {
+    static_assert((W == 4 || W == 8 || W == 16) && K < W, "group of 4, 8 or 16 lanes");
+    if constexpr (W == 16) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + K, 0xf, 0xf, true));
+    else if constexpr (W == 4) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x55 * K, 0xf, 0xf, true));
+    else return __shfl(x, (int)(threadIdx.x & 56u) + K, 64);
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {

@@ -331,6 +331,16 @@ inline float mmi_rows_max(float x) {
     x = fmaxf(x, mmi_shfl_xor(x, 16));
     return fmaxf(x, mmi_shfl_xor(x, 32));
 }
+inline float mmi_rows_sum(float x) {
+    x += mmi_shfl_xor(x, 16);
+    return x + mmi_shfl_xor(x, 32);
+}
+inline float mmi_wave_max_f32(float x) {
+    for (int m = 1; m < 64; m <<= 1) x = fmaxf(x, mmi_shfl_xor(x, m));
+    return x;
+}
+template <int W, int K>
+inline float mmi_group_bcast(float x) { return mmi_shfl(x, (hipsim::lane_id() & ~(W - 1)) + K); }
 // sum over groups of W consecutive lanes, every lane receiving the total (the gfx950 build: DPP row operations)
 template <int W>
 inline float mmi_group_sum(float x) {
