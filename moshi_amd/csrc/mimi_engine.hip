@@ -97,8 +97,8 @@ struct MimiMem {
 
 // operands of the quantiser's launches, `rows` latents at once
 struct RvqScratch {
-    float* xq = nullptr;                       // [rows][2*Dq] residuals (first | rest)
-    double* best_d = nullptr;
+    float* xq = nullptr;                       // 2 x [rows][2*Dq] residuals (first | rest)
+    double* best_d = nullptr;                  // 4 x [rows][nchunk] (two of each half)
     int* best_i = nullptr;
     int* codes = nullptr;                      // [rows][n_q]
     float *qin_bp = nullptr, *qin_part = nullptr;
@@ -684,34 +684,53 @@ int add_quantize_ops(mmi_mimi* m, MimiMem& mem, const RvqScratch& r, MmiProgram&
     }
     const int K = m->n_codebooks;
     const int nchunk = m->nchunk;
-    const size_t smem = ((size_t)MMI_RVQ_CHUNK * (D + 4) + (size_t)8 * D) * sizeof(float);
-    auto level = [&](int k, int slot) {
-        const bool sem = k < c.q_n_q_semantic;
+    const size_t smem = (size_t)8 * D * sizeof(double);
+    int depth[2] = {0, 0};                                // levels of the acoustic / semantic half so far
+    // the next level of its half: two buffers of residuals and two of chunk winners, one read and one written by a launch
+    auto level = [&](int k, bool sem) {
+        const int n = depth[sem]++;
+        const auto buf = [&](int i) { return r.xq + (size_t)(i & 1) * r.rows * 2 * D + (sem ? 0 : D); };
+        const auto slot = [&](int i) { return (size_t)((sem ? 2 : 0) + (i & 1)) * nchunk * r.rows; };
         RvqLevel L;
-        L.x = r.xq + (sem ? 0 : D);
+        memset(&L, 0, sizeof(L));
+        L.x = buf(n > 0 ? n - 1 : 0); L.x_next = buf(n);
+        L.best_d = r.best_d + slot(n); L.best_i = r.best_i + slot(n);
         L.E = m->E_all + (size_t)k * bins * D;
         L.e2 = m->e2_all + (size_t)k * bins;
-        L.best_d = r.best_d + (size_t)slot * nchunk * r.rows;
-        L.best_i = r.best_i + (size_t)slot * nchunk * r.rows;
-        L.level = k;
+        if (n > 0) {
+            L.prev_E = L.E - (size_t)bins * D;
+            L.prev_d = r.best_d + slot(n - 1); L.prev_i = r.best_i + slot(n - 1);
+            L.prev_level = k - 1;
+        }
         return L;
     };
     int* codes = r.codes; const int nq = c.q_n_q;
-    // the semantic quantiser's single level and the first acoustic level share their two launches (independent, see RvqLevel)
+    // rows per workgroup: as few as leave the chip two workgroups per CU (32 rows: 9.0 us with 8, 8.0 with 4); more of them share a code's load
+    int group = 1;
+    while (group < 8 && (long)nchunk * mmi_cdiv(B, group) > 512) group *= 2;
+    // the semantic quantiser's single level and the first acoustic level share a launch (independent, see RvqLevel)
     const bool pair = c.q_n_q_semantic == 1 && K >= 2 && !getenv("MMI_RVQ_NO_PAIR");
     for (int k = 0; k < K; ++k) {
-        const RvqLevel a0 = level(k, 0);
+        const RvqLevel a0 = level(k, k < c.q_n_q_semantic);
         const bool two = pair && k == 0;
-        const RvqLevel a1 = two ? level(1, 1) : a0;
+        const RvqLevel a1 = two ? level(++k, false) : a0;
         const int nz = two ? 2 : 1;
         prog.add([=](hipStream_t s) {
-            MMI_LAUNCH(k_rvq_dist, dim3(nchunk, mmi_cdiv(B, 8), nz), 256, smem, s, a0, a1, 2 * D, B, D, bins);
-            MMI_LAUNCH(k_rvq_select, dim3(B, nz), 256, 0, s, a0, a1, nchunk, 2 * D, codes, nq, B, D);
+            MMI_LAUNCH(k_rvq_level, dim3(nchunk, mmi_cdiv(B, group), nz), 256, smem, s, a0, a1, 2 * D, B, group, D, bins, nchunk, codes, nq);
             MMI_CHECK_LAUNCH();
             return (int)MMI_OK;
         });
-        if (two) ++k;
     }
+    RvqLevel end[2];
+    int ends = 0;
+    for (int sem = 0; sem < 2; ++sem)
+        if (depth[sem] > 0) end[ends++] = level(sem ? std::min(K, c.q_n_q_semantic) : K, sem);       // (its prev_* is the half's last level)
+    const RvqLevel e0 = end[0], e1 = end[ends > 1 ? 1 : 0];
+    prog.add([=](hipStream_t s) {
+        MMI_LAUNCH(k_rvq_last, dim3(mmi_cdiv(B, 4), ends), 256, 0, s, e0, e1, B, nchunk, codes, nq);
+        MMI_CHECK_LAUNCH();
+        return (int)MMI_OK;
+    });
     return MMI_OK;
 }
 
@@ -1032,9 +1051,9 @@ int build_encoder(mmi_mimi* m, int B, int frames, MimiMem& mem, MimiGroup* g, hi
     if (g) {
         const size_t n = (size_t)B * frames;
         rs.rows = (int)n;
-        MMI_HIP_CHECK(mem.alloc(&rs.xq, n * 2 * c.q_dimension));
-        MMI_HIP_CHECK(mem.alloc(&rs.best_d, 2 * m->nchunk * n));
-        MMI_HIP_CHECK(mem.alloc(&rs.best_i, 2 * m->nchunk * n));
+        MMI_HIP_CHECK(mem.alloc(&rs.xq, 2 * n * 2 * c.q_dimension));
+        MMI_HIP_CHECK(mem.alloc(&rs.best_d, 4 * m->nchunk * n));
+        MMI_HIP_CHECK(mem.alloc(&rs.best_i, 4 * m->nchunk * n));
         MMI_HIP_CHECK(mem.alloc(&rs.codes, n * c.q_n_q));
         MMI_HIP_CHECK(mem.alloc(&rs.qin_bp, (size_t)mmi_cdiv((int)n, 32) * m->q_in.Q * 256));
         MMI_HIP_CHECK(mem.alloc(&rs.qin_part, (size_t)8 * m->q_in.Mt * 32 * mmi_cdiv((int)n, 128) * 128));
@@ -1394,9 +1413,9 @@ extern "C" int mmi_mimi_create(const mmi_mimi_cfg* cfg, const mmi_tensor_desc* w
     // ---- RVQ scratch
     m->nchunk = mmi_cdiv(c.q_bins, MMI_RVQ_CHUNK);
     m->rvq.rows = max_batch;
-    if (hipSuccess != m->wts.alloc(&m->rvq.xq, (size_t)max_batch * 2 * c.q_dimension) ||
-        hipSuccess != m->wts.alloc(&m->rvq.best_d, (size_t)2 * m->nchunk * max_batch) ||
-        hipSuccess != m->wts.alloc(&m->rvq.best_i, (size_t)2 * m->nchunk * max_batch) ||
+    if (hipSuccess != m->wts.alloc(&m->rvq.xq, (size_t)2 * max_batch * 2 * c.q_dimension) ||
+        hipSuccess != m->wts.alloc(&m->rvq.best_d, (size_t)4 * m->nchunk * max_batch) ||
+        hipSuccess != m->wts.alloc(&m->rvq.best_i, (size_t)4 * m->nchunk * max_batch) ||
         hipSuccess != m->wts.alloc(&m->rvq.codes, (size_t)max_batch * c.q_n_q) ||
         hipSuccess != m->wts.alloc(&m->deq.codes, (size_t)max_batch * c.q_n_q) ||
         hipSuccess != m->wts.alloc(&m->deq.q2, (size_t)max_batch * 2 * c.q_dimension) ||

@@ -1508,110 +1508,136 @@ __global__ void k_mimi_group_ring(const float* __restrict__ kvn, float* __restri
 // nearest centroid of the fp32 inputs, lowest index on ties - the answer the reference's fp32 cdist
 // agrees with except at ~1e-7-relative near-ties.
 #define MMI_RVQ_CHUNK 32
-// grid (chunks of 32 codes, groups of 8 rows); 256 threads: thread (c, g) owns code c0+c and row rg0+g.  The chunk of the
-// codebook and the 8 rows are staged in LDS with 16-byte accesses (row stride D+4 floats keeps ds_read_b128 conflict
-// free); the dot product runs in four independent fp64 chains.  D % 4 == 0.
-// one level's operands; a launch carries two of them (grid.z / grid.y picks): the semantic quantiser's only level and the acoustic
-// quantiser's first level work on different halves of the projected latent and do not depend on each other
-// (vq.py:269-287 SplitResidualVectorQuantizer.encode), so they share their launches
+// One level of one half of the split quantiser.  A launch carries two of them (grid.z picks): the semantic quantiser's only level and the
+// acoustic quantiser's first level work on different halves of the projected latent and do not depend on each other
+// (vq.py:269-287 SplitResidualVectorQuantizer.encode).
 struct RvqLevel {
-    float* x;              // residual rows [Bn][x_rstride], updated in place by k_rvq_select
+    const float* x;        // residual rows [Bn][x_rstride] in front of the previous level
+    float* x_next;         // ... and behind it, for the next level (another buffer)
     const float* E;        // codebook [bins][D]
     const double* e2;      // ||e||^2
-    double* best_d;        // [nchunk][Bn]
+    double* best_d;        // [Bn][nchunk] nearest code of each chunk
     int* best_i;
-    int level;             // column of `codes` this level writes
+    const float* prev_E;   // the previous level, null in front of a half's first one
+    const double* prev_d;
+    const int* prev_i;
+    int prev_level;        // column of `codes`
 };
 
-__global__ __launch_bounds__(256) void k_rvq_dist(RvqLevel l0, RvqLevel l1, int x_rstride, int Bn, int D, int bins) {
-    const RvqLevel& L = blockIdx.z == 0 ? l0 : l1;
-    const float* __restrict__ x = L.x;
-    const float* __restrict__ E = L.E;
-    const double* __restrict__ e2 = L.e2;
-    double* __restrict__ best_d = L.best_d;
-    int* __restrict__ best_i = L.best_i;
-    MMI_DYN_SHARED(float, sm);
-    const int ldE = D + 4;
-    float* Es = sm;                          // [CHUNK][D+4]
-    float* xs = sm + MMI_RVQ_CHUNK * ldE;    // [8][D]
-    const int chunk = blockIdx.x;
-    const int c0 = chunk * MMI_RVQ_CHUNK;
-    const int tid = threadIdx.x;
-    const int rg0 = (int)blockIdx.y * 8;     // this block's 8 rows (grid.y = ceil(Bn / 8))
-    const int D4 = D >> 2;
-    {   // 8 threads per code / row, each copying every 8th float4 of it
-        const int r = tid >> 3, j0 = tid & 7;
-        const int code = min(c0 + r, bins - 1);
-        for (int j = j0; j < D4; j += 8)
-            *reinterpret_cast<f32x4*>(Es + r * ldE + 4 * j) = *reinterpret_cast<const f32x4*>(E + (long)code * D + 4 * j);
-        if (r < 8) {
-            const int row = min(rg0 + r, Bn - 1);
-            for (int j = j0; j < D4; j += 8)
-                *reinterpret_cast<f32x4*>(xs + r * D + 4 * j) = *reinterpret_cast<const f32x4*>(x + (long)row * x_rstride + 4 * j);
-        }
-    }
-    __syncthreads();
-    const int c = tid & 31, g = tid >> 5;  // 8 rows, 32 codes
-    const bool cvalid = (c0 + c) < bins;
-    const double en = cvalid ? e2[c0 + c] : 0.0;
-    const int r = rg0 + g;
-    const bool rvalid = r < Bn;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    for (int j = 0; j < D4; ++j) {
-        const f32x4 ev = *reinterpret_cast<const f32x4*>(Es + c * ldE + 4 * j);
-        const f32x4 xv = *reinterpret_cast<const f32x4*>(xs + g * D + 4 * j);
-        a0 += (double)ev[0] * (double)xv[0];
-        a1 += (double)ev[1] * (double)xv[1];
-        a2 += (double)ev[2] * (double)xv[2];
-        a3 += (double)ev[3] * (double)xv[3];
-    }
-    const double acc = (a0 + a1) + (a2 + a3);
-    double dist = (cvalid && rvalid) ? en - 2.0 * acc : INFINITY;
-    int idx = c0 + c;
-    // argmin over the 32 codes held by this half-wave (xor masks < 32 stay inside it)
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) {
-        double od = mmi_shfl_xor(dist, m);
-        int oi = mmi_shfl_xor(idx, m);
-        if (od < dist || (od == dist && oi < idx)) { dist = od; idx = oi; }
-    }
-    if (c == 0 && rvalid) { best_d[(long)chunk * Bn + r] = dist; best_i[(long)chunk * Bn + r] = idx; }
+// the winning code of a row: a strided scan of the chunk winners by one wave (lowest index on ties)
+__device__ __forceinline__ int mmi_rvq_winner(const double* __restrict__ best_d, const int* __restrict__ best_i, int nchunk, int lane) {
+    double bd = INFINITY;
+    int bi = 0x7fffffff;
+    for (int ch = lane; ch < nchunk; ch += 64) mmi_pair_min(bd, bi, best_d[ch], best_i[ch]);
+    mmi_wave_pair_min(bd, bi);
+    return bi == 0x7fffffff ? 0 : bi;              // no distance is a number (a NaN or infinite latent): where an argmin over NaNs ends
 }
 
-// pick the winning chunk per row, emit the code, subtract the centroid from the residual
-__global__ __launch_bounds__(256) void k_rvq_select(RvqLevel l0, RvqLevel l1, int nchunk, int x_rstride, int* __restrict__ codes,
-                                                    int codes_rstride, int Bn, int D) {
-    const RvqLevel& L = blockIdx.y == 0 ? l0 : l1;
-    const double* __restrict__ best_d = L.best_d;
-    const int* __restrict__ best_i = L.best_i;
-    float* __restrict__ x = L.x;
-    const float* __restrict__ E = L.E;
-    const int level = L.level;
-    const int r = blockIdx.x;
-    MMI_SHARED int widx;
-    if (threadIdx.x < 64) {   // first wave: strided scan of the chunk winners, then a wave argmin (lowest index on ties)
-        double bd = INFINITY;
-        int bi = 0x7fffffff;
-        for (int ch = threadIdx.x; ch < nchunk; ch += 64) {
-            double d = best_d[(long)ch * Bn + r];
-            int i = best_i[(long)ch * Bn + r];
-            if (d < bd || (d == bd && i < bi)) { bd = d; bi = i; }
-        }
+// grid (chunks of 32 codes, groups of `group` <= 8 rows, levels); 256 threads, D % 4 == 0.  Every workgroup picks the previous level's winners of its rows
+// and takes their centroids off (the first chunk's workgroup stores codes and residuals), then thread (code c, part p) forms the products of its
+// part of a code - the quads p, p + 8, ... - with all of its rows.
+// Bound by its chain of dependent loads (winners, centroid).  The selection was a launch of its own behind every level (one stream: 9.5 + 4.4 us a
+// level, now 5.0); thread (code, row) with the whole dot product left 7 of 8 threads idle at one row and read every code from LDS once per row
+// (32 rows: 11.9 + 4.5 us, now 8.0; 129 rows: 22.6 + 4.7, now 16.4, with the rows' LDS reads in front).
+template <int NR>
+__device__ __forceinline__ void mmi_rvq_products(double (&acc)[8], const f32x4 (&ev)[8], const double* xs, int D, int q0, int p) {
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            double od = mmi_shfl_xor(bd, m);
-            int oi = mmi_shfl_xor(bi, m);
-            if (od < bd || (od == bd && oi < bi)) { bd = od; bi = oi; }
+    for (int i = 0; i < 8; ++i) {
+        const int q = q0 + p + 8 * i;
+        if (4 * q >= D) break;
+        const double e0 = ev[i][0], e1 = ev[i][1], e2 = ev[i][2], e3 = ev[i][3];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const double* x = xs + r * D + 4 * q;
+            acc[r] = fma(e3, x[3], fma(e2, x[2], fma(e1, x[1], fma(e0, x[0], acc[r]))));
         }
-        if (threadIdx.x == 0) {
-            if (bi == 0x7fffffff) bi = 0;          // no distance is a number (a NaN or infinite latent): where an argmin over NaNs ends
-            widx = bi;
-            codes[(long)r * codes_rstride + level] = bi;
+    }
+}
+__global__ __launch_bounds__(256) void k_rvq_level(RvqLevel l0, RvqLevel l1, int x_rstride, int Bn, int group, int D, int bins, int nchunk,
+                                                   int* __restrict__ codes, int codes_rstride) {
+    const RvqLevel& L = blockIdx.z == 0 ? l0 : l1;
+    MMI_DYN_SHARED(double, xs);              // [8][D]
+    MMI_SHARED int win[8];
+    MMI_SHARED double wd[4 * 8];
+    MMI_SHARED int wi[4 * 8];
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int chunk = blockIdx.x, c0 = chunk * MMI_RVQ_CHUNK, rg0 = (int)blockIdx.y * group, nr = min(group, Bn - rg0);
+    const int D4 = D >> 2, c = tid >> 3, p = tid & 7;
+    const int code = min(c0 + c, bins - 1);
+    const f32x4* Ec = reinterpret_cast<const f32x4*>(L.E + (long)code * D);
+    f32x4 ev[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ev[i] = Ec[min(p + 8 * i, D4 - 1)];
+    const double en = L.e2[code];
+    const int xr = tid >> 5, j0 = tid & 31;
+    const f32x4* xp = reinterpret_cast<const f32x4*>(L.x + (long)(rg0 + min(xr, nr - 1)) * x_rstride);
+    const f32x4 xa = xp[min(j0, D4 - 1)], xb = xp[min(j0 + 32, D4 - 1)];
+    if (L.prev_E) {
+        for (int r = wave; r < nr; r += 4) {
+            const int best = mmi_rvq_winner(L.prev_d + (long)(rg0 + r) * nchunk, L.prev_i + (long)(rg0 + r) * nchunk, nchunk, lane);
+            if (lane == 0) {
+                win[r] = best;
+                if (chunk == 0) codes[(long)(rg0 + r) * codes_rstride + L.prev_level] = best;
+            }
+        }
+        __syncthreads();
+    }
+    if (xr < nr) {
+        const f32x4* pe = L.prev_E ? reinterpret_cast<const f32x4*>(L.prev_E + (long)win[xr] * D) : nullptr;
+        f32x4* xn = reinterpret_cast<f32x4*>(L.x_next + (long)(rg0 + xr) * x_rstride);
+        for (int j = j0; j < D4; j += 32) {
+            f32x4 v = j == j0 ? xa : (j == j0 + 32 ? xb : xp[j]);
+            if (pe) {
+                const f32x4 e = pe[j];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] -= e[k];
+                if (chunk == 0) xn[j] = v;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xs[xr * D + 4 * j + k] = (double)v[k];
         }
     }
     __syncthreads();
-    const int idx = widx;
-    for (int d = threadIdx.x; d < D; d += blockDim.x) x[(long)r * x_rstride + d] -= E[(long)idx * D + d];
+    double acc[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[r] = 0.0;
+    for (int q0 = 0;;) {                     // 256 dimensions at a time
+        if (nr == 1) mmi_rvq_products<1>(acc, ev, xs, D, q0, p);
+        else if (nr == 2) mmi_rvq_products<2>(acc, ev, xs, D, q0, p);
+        else if (nr <= 4) mmi_rvq_products<4>(acc, ev, xs, D, q0, p);
+        else mmi_rvq_products<8>(acc, ev, xs, D, q0, p);
+        if ((q0 += 64) >= D4) break;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ev[i] = Ec[min(q0 + p + 8 * i, D4 - 1)];
+    }
+    double dot = 0.0;                        // lane (c, p): row p
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const double t = mmi_group8_sum_f64(acc[r]);
+        dot = r == p ? t : dot;
+    }
+    double dist = en - 2.0 * dot;
+    int idx = c0 + c;
+    if (idx >= bins || p >= nr || dist != dist) { dist = INFINITY; idx = 0x7fffffff; }
+    mmi_group8_pair_min(dist, idx);
+    if (lane < 8) { wd[wave * 8 + lane] = dist; wi[wave * 8 + lane] = idx; }
+    __syncthreads();
+    if (tid < nr) {
+        dist = wd[tid]; idx = wi[tid];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) mmi_pair_min(dist, idx, wd[w * 8 + tid], wi[w * 8 + tid]);
+        L.best_d[(long)(rg0 + tid) * nchunk + chunk] = dist;
+        L.best_i[(long)(rg0 + tid) * nchunk + chunk] = idx;
+    }
+}
+
+// the codes of the halves' last levels: prev_* of l0 (and l1), one wave per row
+__global__ __launch_bounds__(256) void k_rvq_last(RvqLevel l0, RvqLevel l1, int Bn, int nchunk, int* __restrict__ codes, int codes_rstride) {
+    const RvqLevel& L = blockIdx.y == 0 ? l0 : l1;
+    const int r = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    if (r >= Bn) return;
+    const int best = mmi_rvq_winner(L.prev_d + (long)r * nchunk, L.prev_i + (long)r * nchunk, nchunk, lane);
+    if (lane == 0) codes[(long)r * codes_rstride + L.prev_level] = best;
 }
 
 // decode: q[b][0:D] = E_0[c_0]; q[b][D:2D] = ((0 + E_1[c_1]) + E_2[c_2]) + ...   (core_vq.py:521-528)

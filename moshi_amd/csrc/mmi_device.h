@@ -112,6 +112,56 @@ __device__ __forceinline__ float mmi_group_bcast(float x) {
     else if constexpr (W == 4) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x55 * K, 0xf, 0xf, true));
     else return __shfl(x, (int)(threadIdx.x & 56u) + K, 64);
 }
+// a double of another lane of the row of 16 (a DPP control)
+template <int CTRL>
+__device__ __forceinline__ double mmi_dpp_f64(double x) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// sum over groups of 8 consecutive lanes, every lane of the group gets it
+__device__ __forceinline__ double mmi_group8_sum_f64(double x) {
+    x += mmi_dpp_f64<0xB1>(x);
+    x += mmi_dpp_f64<0x4E>(x);
+    return x + mmi_dpp_f64<0x141>(x);
+}
+// the smaller of two (value, index) pairs, the lower index where the values are equal
+__device__ __forceinline__ void mmi_pair_min(double& d, int& i, double od, int oi) {
+    const bool take = od < d || (od == d && oi < i);
+    d = take ? od : d;
+    i = take ? oi : i;
+}
+template <int CTRL>
+__device__ __forceinline__ void mmi_pair_min_dpp(double& d, int& i) {
+    const double od = mmi_dpp_f64<CTRL>(d);
+    mmi_pair_min(d, i, od, __builtin_amdgcn_update_dpp(0, i, CTRL, 0xf, 0xf, true));
+}
+// smallest pair over the four lanes l, l ^ 16, l ^ 32, l ^ 48, every one of them gets it (mmi_rows_max)
+__device__ __forceinline__ void mmi_pair_min_rows(double& d, int& i) {
+    auto step = [&](auto swap) __attribute__((always_inline)) {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, d);
+        const auto l = swap((unsigned)u), h = swap((unsigned)(u >> 32)), j = swap((unsigned)i);
+        const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1], j0 = j[0], j1 = j[1];
+        d = __builtin_bit_cast(double, ((unsigned long long)h0 << 32) | l0);
+        i = (int)j0;
+        mmi_pair_min(d, i, __builtin_bit_cast(double, ((unsigned long long)h1 << 32) | l1), (int)j1);
+    };
+    step([](unsigned v) __attribute__((always_inline)) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); });
+    step([](unsigned v) __attribute__((always_inline)) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); });
+}
+// ... over the whole wave; ... over the lanes l, l ^ 8, l ^ 16, ..., l ^ 56
+__device__ __forceinline__ void mmi_wave_pair_min(double& d, int& i) {
+    mmi_pair_min_dpp<0xB1>(d, i);
+    mmi_pair_min_dpp<0x4E>(d, i);
+    mmi_pair_min_dpp<0x141>(d, i);
+    mmi_pair_min_dpp<0x140>(d, i);
+    mmi_pair_min_rows(d, i);
+}
+__device__ __forceinline__ void mmi_group8_pair_min(double& d, int& i) {
+    mmi_pair_min_dpp<0x128>(d, i);
+    mmi_pair_min_rows(d, i);
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {

@@ -341,6 +341,24 @@ inline float mmi_wave_max_f32(float x) {
 }
 template <int W, int K>
 inline float mmi_group_bcast(float x) { return mmi_shfl(x, (hipsim::lane_id() & ~(W - 1)) + K); }
+inline double mmi_group8_sum_f64(double x) {
+    for (int m = 1; m < 8; m <<= 1) x += mmi_shfl_xor(x, m);
+    return x;
+}
+inline void mmi_pair_min(double& d, int& i, double od, int oi) {
+    const bool take = od < d || (od == d && oi < i);
+    d = take ? od : d;
+    i = take ? oi : i;
+}
+inline void mmi_lanes_pair_min(double& d, int& i, int from) {
+    for (int m = from; m < 64; m <<= 1) {
+        const double od = mmi_shfl_xor(d, m);
+        const int oi = mmi_shfl_xor(i, m);
+        mmi_pair_min(d, i, od, oi);
+    }
+}
+inline void mmi_wave_pair_min(double& d, int& i) { mmi_lanes_pair_min(d, i, 1); }
+inline void mmi_group8_pair_min(double& d, int& i) { mmi_lanes_pair_min(d, i, 8); }
 // sum over groups of W consecutive lanes, every lane receiving the total (the gfx950 build: DPP row operations)
 template <int W>
 inline float mmi_group_sum(float x) {

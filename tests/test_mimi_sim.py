@@ -150,3 +150,12 @@ def test_transformer_linears(factory, heads, Dh, ff, B):
     from dataclasses import replace
     cfg = replace(tiny_mimi_config(), dimension=heads * Dh, tr_d_model=heads * Dh, tr_num_heads=heads, tr_dim_feedforward=ff)
     mimi_cases.oracle_vs_engine(lambda sd, cfg, K: factory(sd, cfg, K, max_batch=B), "cpu", cfg, seed=70 + heads, B=B, F=2, K=2)
+
+
+@pytest.mark.parametrize("dim,bins,sem,B", [(264, 70, 1, 3), (20, 2048, 1, 9), (4, 33, 2, 2)])
+def test_quantiser_levels(factory, dim, bins, sem, B):
+    """k_rvq_level where its work is cut: more than 256 dimensions and no multiple of 32, a last chunk that is not full, several rows per
+    workgroup with a last one that has fewer, two semantic levels in front of the acoustic ones."""
+    from dataclasses import replace
+    cfg = replace(tiny_mimi_config(), q_dimension=dim, q_bins=bins, q_n_q_semantic=sem)
+    mimi_cases.oracle_vs_engine(lambda sd, c, K: factory(sd, c, K, max_batch=B), "cpu", cfg, seed=60 + B, B=B, F=2, K=5)
