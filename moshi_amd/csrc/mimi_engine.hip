@@ -350,9 +350,10 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
 // ---- launch helpers ---------------------------------------------------------------------------
 // A conv / linear becomes one of two launch sequences, chosen when the frame program is built (mimi_kernels.h):
 //   N = B*T_out > 128 columns : k_conv_wide
-//   N <= 128                  : [k_pack_b_f32] -> k_gemm_f32 [-> k_conv_finish when K is split over workgroups]
+//   N <= 128                  : k_conv_few [-> k_conv_finish], or [k_pack_b_f32] -> k_gemm_f32 [-> k_conv_finish when K is split over workgroups]
 struct ConvPlan {
     bool wide = false;
+    bool few = false;                 // k_conv_few
     int MTB = 1, W = 1;               // wide
     bool group = false;
     int NSUB = 1, waves = 4, ksplit = 1, nz = 1;
@@ -397,8 +398,13 @@ int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
     }
     ConvGemmArgs g = a;
     if (p.ksplit > 1) g.out_mode = MMI_GOUT_PARTIAL;
-    const dim3 grid(a.Mt, p.ksplit, p.nz);
-    if (p.NSUB == 1) {
+    const dim3 grid(a.Mt, p.ksplit, p.nz), grid_few(mmi_cdiv(a.Cout, 16), mmi_cdiv(a.Ntot, 16), p.ksplit);
+    if (p.few) {
+        g.q_blk = mmi_cdiv(a.Q, p.ksplit);
+        if (a.x_packed) MMI_LAUNCH((k_conv_few<true, false>), grid_few, p.waves * 64, 0, s, g);
+        else if (a.first) MMI_LAUNCH((k_conv_few<false, true>), grid_few, p.waves * 64, 0, s, g);
+        else MMI_LAUNCH((k_conv_few<false, false>), grid_few, p.waves * 64, 0, s, g);
+    } else if (p.NSUB == 1) {
         if (p.waves == 8) MMI_LAUNCH((k_gemm_f32<1, 8, 2>), grid, 512, 0, s, g);
         else MMI_LAUNCH((k_gemm_f32<1, 4, 2>), grid, 256, 0, s, g);
     } else if (p.NSUB == 2) {
@@ -551,7 +557,12 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         p->nz = mmi_cdiv(nsub, p->NSUB);
         a.Npad = p->nz * p->NSUB * 32;
     }
-    if (!a.x_packed) {
+    // 16 x 16 tiles while the chip holds them all at once (two workgroups per CU) and a load of 16 columns reaches few streams' rows (a frame of 4
+    // streams 778 -> 763 us against the launch that packs in front, of 8 streams 845 -> 847).  With a packed operand there is no such launch to
+    // save: only where 32 x 32 tiles leave CUs idle (512 -> 512 on 2 columns 6.1 -> 4.8 us; 1024 -> 8192 on 2 columns 9.4 -> 11.8)
+    const long tiles = (long)mmi_cdiv(a.Cout, 16) * mmi_cdiv(N, 16);
+    p->few = mem.frames == 1 && !a.elu_in && (a.x_packed ? tiles <= 256 : tiles <= 512 && a.B <= 4) && !getenv("MMI_MIMI_PACK_LAUNCHES");
+    if (!a.x_packed && !p->few) {
         if (!a.bp) {
             float* bp = nullptr;
             MMI_HIP_CHECK(mem.alloc(&bp, (size_t)nsub * a.Q * 256));

@@ -163,10 +163,8 @@ MMI_HD long mmi_lin_index(int k, int n, int J) {
 // NV results of one thread are finished together: all bias / scale / residual loads are issued first (under branches
 // that are uniform for the launch), so that the epilogue costs one memory round trip instead of NV of them.
 template <int NV>
-__device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
-                                                 const bool (&ok)[NV], float (&v)[NV]) {
-    float bia[NV], rsv[NV];
-    long row[NV];
+__device__ __forceinline__ void mmi_conv_ask_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
+                                               const bool (&ok)[NV], long (&row)[NV], float (&bia)[NV], float (&rsv)[NV]) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int cc = ok[i] ? co[i] : 0;
@@ -181,6 +179,10 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
 #pragma unroll
         for (int i = 0; i < NV; ++i) rsv[i] = a.res[row[i] * a.res_ld + a.res_off + (ok[i] ? t[i] : 0)];
     }
+}
+template <int NV>
+__device__ __forceinline__ void mmi_conv_put_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
+                                               const bool (&ok)[NV], const long (&row)[NV], const float (&bia)[NV], const float (&rsv)[NV], float (&v)[NV]) {
     // launch-uniform flags are tested once per group of NV values, not per value: these kernels are instruction bound, and a
     // per-value maze of scalar branches (with the erf and expm1 bodies in line) was a third of a residual block's time
     if (a.bias) {
@@ -217,6 +219,15 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
         for (int i = 0; i < NV; ++i)
             if (ok[i]) a.outp[a.outJ ? mmi_lin_index(co[i], b[i] * a.T_out + t[i], a.outJ) : mmi_bp_index(co[i], b[i] * a.T_out + t[i], a.outQ)] = v[i];
     }
+}
+
+template <int NV>
+__device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
+                                                 const bool (&ok)[NV], float (&v)[NV]) {
+    float bia[NV], rsv[NV];
+    long row[NV];
+    mmi_conv_ask_n<NV>(a, co, b, t, ok, row, bia, rsv);
+    mmi_conv_put_n<NV>(a, co, b, t, ok, row, bia, rsv, v);
 }
 
 // GROUP: several frames of a stream at once - more columns per stream (T_shift), and the reduction also split over gridDim.z workgroups
@@ -694,6 +705,116 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_f32(ConvGemmArgs a) {
 #undef MMI_F_MMA
 
     mmi_gemm_f32_finish<NSUB, WAVES>(a, acc, mt, s0, wave, lane);
+}
+
+// A conv of few columns on v_mfma_f32_16x16x4_f32: grid (ceil(Cout/16), ceil(Ntot/16), ks), one 16 x 16 tile per workgroup.  The reduction is cut as
+// k_gemm_f32 cuts it - into gridDim.z pieces of a.q_blk quads, each of them over the workgroup's waves - and added up in the same order, so the
+// results are the same bits (k_conv_finish adds the gridDim.z sums).  Operands come from the conv's input as it lies (PACKED: from `bp`).
+// Weights and `bp` hold quads of 8 reduction indices for 32 rows: the lanes of the upper half take the next quad, an exchange of register halves
+// (mmi_swap32) turns two quads into the four operands of the 16 x 16 form, in rising order.
+// Bound by latency, like k_mimi_lin: the launch that packed the input (4.5 us) is gone, 32 x 32 tiles left 8 - 32 CUs at work.  One stream:
+// 256 -> 128, K 3 on 96 columns 4.4 + 6.8 -> 5.6 us; 512 -> 256, K 3 on 16 columns 4.5 + 10.7 -> 7.6; 512 -> 1024, K 16 on 2 columns
+// 4.6 + 11.3 -> 13.1.  All pieces of a split reduction in one workgroup, without the launch that adds them, measured slower (1024 -> 512, K 3 on
+// 2 columns: 12.0 against 4.9 + 4.8 - one CU streams 20 - 50 KB of weights per us).
+template <bool PACKED, bool FIRST>
+__global__ __launch_bounds__(512) void k_conv_few(ConvGemmArgs a) {
+    constexpr int U = 5;                                     // pairs of quads per group; two groups are in flight
+    MMI_SHARED float red[8 * 256];
+    const int tid = (int)threadIdx.x, wave = mmi_uniform(tid >> 6), lane = tid & 63, nw = (int)blockDim.x >> 6;
+    const int r16 = lane & 15, quarter = lane >> 4, kh = quarter & 1, hi = quarter >> 1;
+    const int m0 = (int)blockIdx.x * 16, n0 = (int)blockIdx.y * 16;
+
+    // what this thread stores: element tid of the tile in the accumulators' order
+    int co[1] = {m0 + 4 * ((tid >> 4) & 3) + ((tid >> 6) & 3)}, bb[1], tt[1];
+    const int no = n0 + (tid & 15);
+    bool ok[1] = {tid < 256 && no < a.Ntot && co[0] < a.Cout};
+    bb[0] = mmi_fast_div(ok[0] ? no : 0, a.T_magic);
+    tt[0] = (ok[0] ? no : 0) - bb[0] * a.T_out;
+    long row[1];
+    float bia[1], rsv[1];
+    mmi_conv_ask_n<1>(a, co, bb, tt, ok, row, bia, rsv);
+
+    const int qb0 = min(a.Q, (int)blockIdx.z * a.q_blk), qb1 = min(a.Q, qb0 + a.q_blk), qper = (qb1 - qb0 + nw - 1) / nw;
+    const int qa = min(qb1, qb0 + wave * qper), qz = min(qb1, qa + qper), last = max(qz - 1, 0);
+    const f32x4* wp = reinterpret_cast<const f32x4*>(a.wpk) + (long)(m0 >> 5) * a.Q * 64 + kh * 32 + (m0 & 16) + r16;
+    const f32x4* bp = nullptr;
+    // the input's places of the four values of a pair of quads (bytes from a.x on), and their taps: 16 indices further is a few additions
+    unsigned off[4], top = 0, step = 0, carry = 0;
+    int tap[4], tap_step = 0, tap_min = 0;
+    if constexpr (PACKED) {
+        const int ntn = (a.Ntot + 31) / 32;
+        bp = reinterpret_cast<const f32x4*>(a.bp) + (long)min(n0 >> 5, ntn - 1) * a.Q * 64 + kh * 32 + (n0 & 16) + r16;
+    } else {
+        const int nc = n0 + r16 < a.Ntot ? n0 + r16 : 0;     // (columns past the last one are computed and dropped)
+        const int b = mmi_fast_div(nc, a.T_magic), t = nc - b * a.T_out;
+        const unsigned base = 4u * (unsigned)(b * (int)a.x_bstride + a.x_off + t * a.S);
+        if (FIRST && a.first[b] != 0 && a.exec[b] != 0) tap_min = a.H - a.x_off - t * a.S;      // replicate x[..., :1]
+        const int c16 = mmi_fast_div(16, a.K_magic);
+        tap_step = 16 - c16 * a.K;
+        step = 4u * (unsigned)(c16 * a.x_ld + tap_step);
+        carry = 4u * (unsigned)(a.x_ld - a.K);
+        top = base + 4u * (unsigned)((a.Cin - 1) * a.x_ld + a.K - 1);        // (reduction indices past the last one meet zero weights or no product)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int kd = (qa + (e >> 1)) * 8 + 4 * (e & 1) + quarter, ci = mmi_fast_div(kd, a.K_magic);
+            tap[e] = kd - ci * a.K;
+            off[e] = base + 4u * (unsigned)(ci * a.x_ld + tap[e]);
+        }
+    }
+    auto load = [&](f32x4 (&w)[U], f32x4 (&x)[U], int q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            w[u] = mmi_load_nt(wp + (long)min(q + 2 * u + hi, last) * 64);
+            if constexpr (PACKED) x[u] = bp[(long)min(q + 2 * u + hi, last) * 64];
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    unsigned o = off[e];
+                    if (FIRST) o += 4u * (unsigned)max(tap_min - tap[e], 0);
+                    x[u][e] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.x) + min(o, top));
+                    tap[e] += tap_step;
+                    off[e] += step;
+                    const bool over = tap[e] >= a.K;
+                    tap[e] -= over ? a.K : 0;
+                    off[e] += over ? carry : 0u;
+                }
+        }
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto quads = [](f32x4& v) __attribute__((always_inline)) {     // element e of quads (q, q + 1) -> steps 0, 1 of q, steps 0, 1 of q + 1
+        float e0 = v[0], e1 = v[1], e2 = v[2], e3 = v[3];
+        mmi_swap32(e0, e1);
+        mmi_swap32(e2, e3);
+        v = f32x4{e0, e2, e1, e3};
+    };
+    auto mma = [&](f32x4 (&w)[U], f32x4 (&x)[U], int q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            quads(w[u]);
+            if constexpr (PACKED) quads(x[u]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (q + 2 * u + (e >> 1) < qz) acc = mmi_mfma_f32_16x16x4(w[u][e], x[u][e], acc);
+        }
+    };
+    if (qa < qz) {
+        f32x4 wA[U], xA[U], wB[U], xB[U];
+        load(wA, xA, qa);
+        for (int q = qa; q < qz; q += 4 * U) {
+            if (q + 2 * U < qz) load(wB, xB, q + 2 * U);
+            mma(wA, xA, q);
+            if (q + 4 * U < qz) load(wA, xA, q + 4 * U);
+            if (q + 2 * U < qz) mma(wB, xB, q + 2 * U);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave * 256 + r * 64 + lane] = acc[r];
+    __syncthreads();
+    if (tid >= 256) return;
+    float v[1] = {0.f};
+    for (int w = 0; w < nw; ++w) v[0] += red[w * 256 + tid];
+    if (a.out_mode == MMI_GOUT_PARTIAL) a.partial[((long)blockIdx.z * a.Mt * 32 + co[0]) * a.Npad + no] = v[0];       // padded rows / columns included
+    else mmi_conv_put_n<1>(a, co, bb, tt, ok, row, bia, rsv, v);
 }
 
 // ------------------------------------------------------------------------------------------------

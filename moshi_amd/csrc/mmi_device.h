@@ -162,6 +162,13 @@ __device__ __forceinline__ void mmi_group8_pair_min(double& d, int& i) {
     mmi_pair_min_dpp<0x128>(d, i);
     mmi_pair_min_rows(d, i);
 }
+// the upper 32 lanes of a change places with the lower 32 of b
+__device__ __forceinline__ void mmi_swap32(float& a, float& b) {
+    const auto v = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned v0 = v[0], v1 = v[1];
+    a = __builtin_bit_cast(float, v0);
+    b = __builtin_bit_cast(float, v1);
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {

@@ -341,6 +341,11 @@ inline float mmi_wave_max_f32(float x) {
 }
 template <int W, int K>
 inline float mmi_group_bcast(float x) { return mmi_shfl(x, (hipsim::lane_id() & ~(W - 1)) + K); }
+inline void mmi_swap32(float& a, float& b) {
+    const float oa = mmi_shfl_xor(a, 32), ob = mmi_shfl_xor(b, 32);
+    if (hipsim::lane_id() < 32) b = oa;
+    else a = ob;
+}
 inline double mmi_group8_sum_f64(double x) {
     for (int m = 1; m < 8; m <<= 1) x += mmi_shfl_xor(x, m);
     return x;

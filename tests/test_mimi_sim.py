@@ -159,3 +159,20 @@ def test_quantiser_levels(factory, dim, bins, sem, B):
     from dataclasses import replace
     cfg = replace(tiny_mimi_config(), q_dimension=dim, q_bins=bins, q_n_q_semantic=sem)
     mimi_cases.oracle_vs_engine(lambda sd, c, K: factory(sd, c, K, max_batch=B), "cpu", cfg, seed=60 + B, B=B, F=2, K=5)
+
+
+@pytest.mark.parametrize("ks,B,filters", [(1, 1, 4), (3, 4, 4), (8, 2, 12)])
+def test_convs_of_few_columns(factory, monkeypatch, ks, B, filters):
+    """k_conv_few: reductions that are split over 1, 3 and 8 workgroups (pieces of an odd number of quads, pieces that are empty), channel counts
+    that are no multiple of 16, the replicated first frame, one to four streams; and frames against groups of frames, bit for bit."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_CONV_KSPLIT", str(ks))
+    cfg = replace(tiny_mimi_config(), n_filters=filters)
+    mimi_cases.oracle_vs_engine(factory, "cpu", cfg, seed=80 + ks, B=B, F=3, K=3)
+    m = factory(random_mimi_state_dict(cfg, seed=5), cfg, 3)
+    x = 0.3 * torch.randn(B, 1, cfg.frame_size * 3, generator=torch.Generator().manual_seed(1))
+    with m.streaming(B):
+        whole = m.decode(m.encode(x))
+    with m.streaming(B):
+        codes = torch.cat([m.encode(x[..., f * cfg.frame_size:(f + 1) * cfg.frame_size]) for f in range(3)], -1)
+        assert torch.equal(whole, torch.cat([m.decode(codes[..., f:f + 1]) for f in range(3)], -1))
