@@ -772,11 +772,13 @@ int alloc_state(mmi_tlm* m) {
 // weight-streaming kernel with mt row tiles, or the tiled kernel with 32 fm rows per block
 struct Plan { bool rows; int mt, fm; };
 // 128 rows per block from where they no longer leave the chip idle or, with experts, half-filled blocks behind (an expert's run is cut
-// into blocks): 676 rows x 11264 x 2048 takes 45 us in 128 x 128 blocks and 50 us in 128 x 64 ones, 200 rows x 7680 x 2048 24 and 19
-Plan plan_rows(int T, bool routed) {
+// into blocks): 676 rows x 11264 x 2048 takes 45 us in 128 x 128 blocks and 50 us in 128 x 64 ones, 200 rows x 7680 x 2048 24 and 19.
+// 32 rows at fp32, where a row costs eight times the matrix time: blocks of 64 rows run up to three on one CU beside idle ones, and an expert's few
+// rows fill half of one (Kesirax 1024, 320 rows: 1191 -> 1031 us; Bibapel 2048, 200 rows: 2785 -> 2399; Kesirax 1024, 900 rows: 2206 -> 1828)
+Plan plan_rows(int T, bool routed, bool f32) {
     Plan p{T <= ROWS_MAX, 1, 2};
     p.mt = T <= 16 ? 1 : (T <= 32 ? 2 : 4);
-    p.fm = T >= (routed ? 1024 : 640) ? 4 : 2;
+    p.fm = T >= (routed ? 1024 : 640) ? 4 : (f32 ? 1 : 2);
     return p;
 }
 int plan_tile(const Plan& p) { return p.rows ? 16 * p.mt : 32 * p.fm; }
@@ -823,21 +825,21 @@ int split_for(const Plan& p, const Mat& w, int blocks) {
     return s;
 }
 // blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64)
-int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, 2 * p.fm) * (j.list ? j.rblocks : j.groups * mmi_cdiv(j.rows, plan_tile(p))); }
+int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, p.fm == 4 ? 8 : 4) * (j.list ? j.rblocks : j.groups * mmi_cdiv(j.rows, plan_tile(p))); }
 int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
 
 int rows_ntw(const Plan& p) { return p.mt; }                // n-tiles per workgroup of the weight-streaming kernel
-template <class Tr, int FN, int FM, int ST, int OCC, int WN = 2, int WM = 2>
+template <class Tr, int FN, int FM, int ST, int OCC, int WN = 2, int WM = 2, int KK = 1>
 int launch_tile(hipStream_t s, const TlmJobs& J) {
-    constexpr size_t smem = TlmTile<Tr, FN, FM, WN, WM, ST>::smem();
+    constexpr size_t smem = TlmTile<Tr, FN, FM, WN, WM, ST, KK>::smem();
     int grid = 0;                                          // every XCD's share of every job, rounded up
     for (int i = 0; i < J.n; ++i) grid += 8 * mmi_cdiv(J.j[i].blocks, 8);
     static_assert(smem * OCC <= 160 * 1024, "LDS of a CU");
     if (smem > 64 * 1024) {
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC, KK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         MMI_HIP_CHECK(attr);
     }
-    MMI_LAUNCH((k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC>), grid, 256, smem, s, J);
+    MMI_LAUNCH((k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC, KK>), grid, 256, smem, s, J);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
@@ -873,14 +875,22 @@ int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J) {
         return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J) : launch_tile<Tr, 4, 4, 3, 3>(s, J);
     }
     // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
-    // at fp32 the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
     if constexpr (Tr::V == 8) {
         if (cut(8) >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, J);
-        cut(4);
+        // 64 x 64 with stages of two k-steps while two blocks per CU are all there is, or the blocks are long (a meeting of the waves per k-step was
+        // what a step of 8 products took: 676 x 2048 x (2048 + 5632), 640 blocks: 40.7 -> 35.9 us; 300 rows of Bibapel 4096 2713 -> 2618 us); one k-step
+        // each, four blocks per CU, where more of them are short or expert blocks of a few rows (100 rows of Kesirax 2048: 833 against 989 us)
+        bool long_dense = true;
+        for (int i = 0; i < J.n; ++i) long_dense = long_dense && !J.j[i].list;
+        int steps = 0;
+        for (int i = 0; i < J.n; ++i) steps = std::max(steps, mmi_cdiv(J.j[i].KS, J.j[i].ksplit));
+        if (cut(4) <= 512 || (long_dense && steps >= 64)) return launch_tile<Tr, 2, 2, 4, 2, 2, 2, 2>(s, J);
         return launch_tile<Tr, 2, 2, 4, 4>(s, J);
     } else {
-        cut(4);
-        return launch_tile<Tr, 1, 4, 4, 4, 4, 1>(s, J);
+        // at fp32 the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
+        // 32 rows and two k-steps per stage (plan_rows); more stages while all blocks fit the chip with them (three per CU, expert blocks without rows aside; Kesirax 1024, 194 rows: 911 and
+        // 865 us; 320 rows, with more blocks: 1030 and 1045)
+        return cut(4) <= 1024 ? launch_tile<Tr, 1, 2, 4, 3, 4, 1, 2>(s, J) : launch_tile<Tr, 1, 2, 3, 4, 4, 1, 2>(s, J);
     }
 }
 int launch_jobs(mmi_tlm* m, hipStream_t s, const Plan& p, TlmJobs J) {
@@ -1412,7 +1422,7 @@ const char* mixer_site(int mixer) {
 
 void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
     const int T = sh.T;
-    const Plan p = plan_rows(T, !m->route_host.empty());
+    const Plan p = plan_rows(T, !m->route_host.empty(), m->f32);
     TlmPrepArgs a;
     memset(&a, 0, sizeof(a));
     a.T = T;
@@ -1572,7 +1582,7 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
         nm.w = m->final_norm;
         nm.out = m->h;
         add_resid(m, P, sh, c, TLM_EMB_NONE, nullptr, nm, m->meta + sh.m.want, sh.n_want);
-        const Plan hp = plan_rows(sh.n_want, false);
+        const Plan hp = plan_rows(sh.n_want, false, m->f32);
         TlmJobs J;
         memset(&J, 0, sizeof(J));
         TlmJob& j = J.j[J.n++];

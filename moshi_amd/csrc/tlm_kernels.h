@@ -570,19 +570,22 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void k_tlm_gemm_row
 // Many rows: WN x WM waves, each over FN x FM fragments, i.e. 16 FN WN features x 16 FM WM rows per workgroup.  Operands go from global
 // memory straight into a ring of ST stages of one k-step in LDS (whole fragments, so that both sides are conflict-free without a swizzle),
 // ST - 2 stages ahead of the step that reads them into registers, which is one step ahead of the products that use them: a step is one
-// meeting of the waves, its loads and LDS reads lie between the products of the step before.
+// meeting of the waves, its loads and LDS reads lie between the products of the step before.  KK = 2: a stage is two k-steps, with one meeting
+// for both, where a wave has 8 products or fewer in a k-step (the blocks of 64 features).
 // Bound by the matrix core's power (it runs at 0.95 - 1.2 PFLOP/s where a 16384^3 library product reaches 1.29) and, with few blocks, by
 // the latency of a step (0.3 - 0.56 us).  Against the same tiles staged through registers: 1773 x 38912 x 4096 602 -> 543 us, 1773 x 4096 x
 // (11264 + 4096) 263 -> 203.
-template <class Tr, int FN, int FM, int WN, int WM, int ST>
+template <class Tr, int FN, int FM, int WN, int WM, int ST, int KK>
 struct TlmTile {
-    static constexpr int NW = WN * WM, NFN = WN * FN, NFM = WM * FM, NF = NFN + NFM, NIN = NFN / NW, NIM = NFM / NW, NI = NIN + NIM;
-    static_assert(NFN % NW == 0 && NFM % NW == 0 && (ST == 3 || ST == 4), "every wave brings whole fragments; the waits are for one or two stages");
-    static constexpr size_t smem() { return (size_t)ST * NF * 1024; }
+    static constexpr int NW = WN * WM, NFN = WN * FN, NFM = WM * FM, NF = NFN + NFM;
+    static constexpr int NIN = KK * NFN / NW, NIM = KK * NFM / NW, NI = NIN + NIM;      // fragments that a wave brings to a stage
+    static_assert(NFN % NW == 0 && (NFM % NW == 0 || (NW % NFM == 0 && KK * NFM % NW == 0)) && (ST == 3 || ST == 4), "every wave brings whole fragments; the waits are for one or two stages");
+    static_assert(KK == 1 || KK == 2, "k-steps per stage: the register sets go round in pairs");
+    static constexpr size_t smem() { return (size_t)ST * KK * NF * 1024; }
 };
-template <class Tr, int FN, int FM, int WN, int WM, int ST, int OCC>
+template <class Tr, int FN, int FM, int WN, int WM, int ST, int OCC, int KK>
 __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs jobs) {
-    typedef TlmTile<Tr, FN, FM, WN, WM, ST> P;
+    typedef TlmTile<Tr, FN, FM, WN, WM, ST, KK> P;
     MMI_DYN_SHARED(u32x4, lds);
     // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous run of EVERY job's tiles - its L2 sees the shared operand, and no
     // XCD has the long tiles, or the experts' unused row blocks, to itself
@@ -615,33 +618,35 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
         n = j.rows - r0 < 16 * P::NFM ? j.rows - r0 : 16 * P::NFM;
     }
     const int nt0 = nb0 * P::NFN, sper = (j.KS + j.ksplit - 1) / j.ksplit, k0 = min(j.KS, split * sper), ns = min(j.KS, k0 + sper) - k0;
-    // fragment i of this wave: weights at a scalar address, activations (gathered rows) at one per lane
+    // fragment i of this wave, of one of the stage's k-steps: weights at a scalar address, activations (gathered rows) at one per lane
     const u32x4 *wq[P::NIN], *xq[P::NIM];
+    constexpr auto kn = [](int i) { return P::NW * i / P::NFN; };
+    auto km = [&](int i) __attribute__((always_inline)) { return P::NFM % P::NW == 0 ? P::NW * i / P::NFM : (wave + P::NW * i) / P::NFM; };
 #pragma unroll
-    for (int i = 0; i < P::NIN; ++i) wq[i] = j.wp + (long)g * j.wgs + ((long)min(nt0 + wave + P::NW * i, j.NT - 1) * j.KS + k0) * 64;
+    for (int i = 0; i < P::NIN; ++i) wq[i] = j.wp + (long)g * j.wgs + ((long)min(nt0 + wave + P::NW * i - kn(i) * P::NFN, j.NT - 1) * j.KS + k0 + kn(i)) * 64;
+    const int xs = j.xrow ? 4 : 64;
 #pragma unroll
     for (int i = 0; i < P::NIM; ++i) {                        // (rows past n repeat the last one, and are dropped at the end)
-        const int m = (wave + P::NW * i) * 16 + bl, ii = m < n ? m : n - 1;
+        const int m = (wave + P::NW * i - km(i) * P::NFM) * 16 + bl, ii = m < n ? m : n - 1;
         const int id = j.list ? j.list[r0 + ii] : r0 + ii;
         const long in = j.in_pos ? r0 + ii : (j.list ? id / j.in_div : (long)id * j.in_mul + (long)g * j.in_gadd);
-        xq[i] = tlm_row(j, in, g, lane) + (long)k0 * (j.xrow ? 4 : 64);
+        xq[i] = tlm_row(j, in, g, lane) + (long)(k0 + km(i)) * xs;
     }
-    const int xs = j.xrow ? 4 : 64;
-    int to = 0;                                               // the stage's place in the ring, for the next load and the next read
-    int from = 0;
-    auto fetch = [&](int i) __attribute__((always_inline)) {
-        const int at = (to * P::NF + wave + P::NW * i) * 64;
-        if (i < P::NIN) {
-            mmi_load_lds(wq[i < P::NIN ? i : 0], lane * 16, lds, at);
-            wq[i < P::NIN ? i : 0] += 64;
-        } else {
-            mmi_load_lds(xq[i < P::NIN ? 0 : i - P::NIN], lds, at);
-            xq[i < P::NIN ? 0 : i - P::NIN] += xs;
-        }
-    };
+    const int stages = KK == 1 ? ns : (ns + 1) / 2;
+    int to = 0, from = 0, left = stages;                      // places in the ring: of the next stage to load, of the next k-step to read; stages to load
     auto fetch_all = [&]() __attribute__((always_inline)) {
+        // (an odd number of k-steps: the last stage gets the last one twice - stages are counted in loads)
+        const int back = KK == 2 && --left == 0 && (ns & 1) ? 1 : 0;
 #pragma unroll
-        for (int i = 0; i < P::NI; ++i) fetch(i);
+        for (int i = 0; i < P::NIN; ++i) {
+            mmi_load_lds(KK == 1 ? wq[i] : wq[i] - back * kn(i) * 64, lane * 16, lds, (to * KK * P::NF + wave + P::NW * i + kn(i) * P::NFM) * 64);
+            wq[i] += KK * 64;
+        }
+#pragma unroll
+        for (int i = 0; i < P::NIM; ++i) {
+            mmi_load_lds(KK == 1 ? xq[i] : xq[i] - back * km(i) * xs, lds, (to * KK * P::NF + wave + P::NW * i + (km(i) + 1) * P::NFN) * 64);
+            xq[i] += KK * xs;
+        }
         to = to + 1 < ST ? to + 1 : 0;
     };
     const int wn = wave % WN, wm = wave / WN;
@@ -662,15 +667,19 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
         else if (behind == 1) mmi_wait_loads<P::NI>();
         else mmi_wait_loads<0>();
     };
-    // products of stage s (register set `cur`); between them the loads of stage s + ST - 1 and the LDS reads of stage s + 1
+    // products of k-step s (register set `cur`); between them the LDS reads of k-step s + 1 and, where that one begins a stage, the loads
+    // of the stage ST - 2 behind it
     auto step = [&](auto set, int s) __attribute__((always_inline)) {
         constexpr int cur = decltype(set)::value;
-        const bool more = s + 1 < ns, load = s + ST - 1 < ns;
-        if (more) {
-            wait(min(ns - 1, s + ST - 2) - (s + 1));
-            mmi_meet();
+        const bool more = s + 1 < ns;
+        if (KK == 1 || cur == KK - 1) {
+            const int c = KK == 1 ? s : s / KK;              // this stage
+            if (more) {
+                wait(ST == 3 ? 0 : min(stages - 1, c + ST - 2) - (c + 1));
+                mmi_meet();
+            }
+            if (c + ST - 1 < stages) fetch_all();
         }
-        if (load) fetch_all();
 #pragma unroll
         for (int x = 0; x < FN; ++x) {
             if (more) {
@@ -682,10 +691,10 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
             for (int y = 0; y < FM; ++y)
                 if (Tr::V == 8 || y < ny) acc[x][y] = Tr::mfma(av[cur][x], bv[cur][y], acc[x][y]);
         }
-        from = from + 1 < ST ? from + 1 : 0;
+        from = from + 1 < ST * KK ? from + 1 : 0;
     };
     if (ns > 0) {
-        const int first = min(ns, ST - 1);
+        const int first = min(stages, ST - 1);
         for (int s = 0; s < first; ++s) fetch_all();
         wait(first - 1);
         mmi_meet();

@@ -1,4 +1,4 @@
-"""Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 64, 128 x 64, 128 x 128 in three and four stages, 256 x 128, whole
+"""Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 32, 64 x 64, 128 x 64, 128 x 128 in three and four stages, 256 x 128, whole
 and split reductions, gathered and listed expert rows - at row counts just past a tile and sizes that are no multiples of one: a prompt fed at
 once must give the logits that the same prompt gives in portions of at most 64 tokens, which take the weight-streaming kernel."""
 from dataclasses import replace
@@ -26,10 +26,11 @@ def dense_model(width, ff):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("model,T", [
-    (experts_model(208, 144), 65), (experts_model(528, 400), 130),                    # 64 x 64
+    (experts_model(208, 144), 65), (experts_model(528, 400), 130),                    # 64 x 64 in stages of two k-steps, the last one half empty; fp32: 64 x 32
+    (dense_model(2080, 3800), 200),                                                   # ... more blocks than the chip holds at once
     (dense_model(1040, 4000), 577), (dense_model(1040, 1200), 641),                   # 128 x 64; 128 x 128 in four stages
     (experts_model(1040, 2064), 1025), (dense_model(1040, 6000), 1157)                # 128 x 128 in three, 256 x 128
-], ids=["65", "130", "577", "641", "1025", "1157"])
+], ids=["65", "130", "200", "577", "641", "1025", "1157"])
 def test_prompt_at_once_equals_portions(model, T, dtype):
     sd = random_token_lm_state_dict(model, seed=T, device="cuda")
     lm = TokenLM(sd, model, dtype=dtype, max_slots=2, max_tokens=4096, max_step_tokens=T)
