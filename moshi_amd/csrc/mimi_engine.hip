@@ -354,6 +354,7 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
 struct ConvPlan {
     bool wide = false;
     bool few = false;                 // k_conv_few
+    bool cols = false;                // k_conv_cols
     int MTB = 1, W = 1;               // wide
     bool group = false;
     int NSUB = 1, waves = 4, ksplit = 1, nz = 1;
@@ -378,7 +379,26 @@ void launch_wide_w(hipStream_t s, const ConvGemmArgs& a, int W, bool group, dim3
     else launch_wide_e<MTB, U, false, false>(s, a, W, grid);
 }
 
+template <int MTB, int U>
+void launch_cols(hipStream_t s, const ConvGemmArgs& a, int pieces, dim3 grid) {
+    if (a.x_packed) MMI_LAUNCH((k_conv_cols<MTB, U, false, true>), grid, 256, 0, s, a, pieces);
+    else if (a.elu_in) MMI_LAUNCH((k_conv_cols<MTB, U, true, false>), grid, 256, 0, s, a, pieces);
+    else MMI_LAUNCH((k_conv_cols<MTB, U, false, false>), grid, 256, 0, s, a, pieces);
+}
+
 int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
+    if (p.cols) {
+        const dim3 grid(mmi_cdiv(a.Ntot, 128), mmi_cdiv(a.Mt, p.MTB), p.ksplit);
+        ConvGemmArgs w = a;
+        if (p.ksplit > 1) w.out_mode = MMI_GOUT_PARTIAL;
+        const bool fours = mmi_cdiv(w.q_blk, p.W) % 4 == 0;          // (a group ends with its piece)
+        if (p.MTB == 4) launch_cols<4, 2>(s, w, p.W, grid);
+        else if (p.MTB == 2) fours ? launch_cols<2, 4>(s, w, p.W, grid) : launch_cols<2, 2>(s, w, p.W, grid);
+        else fours ? launch_cols<1, 4>(s, w, p.W, grid) : launch_cols<1, 2>(s, w, p.W, grid);
+        if (p.ksplit > 1) MMI_LAUNCH(k_conv_finish, (int)mmi_cdiv64((int64_t)a.Cout * a.Ntot, 256), 256, 0, s, a, p.ksplit);
+        MMI_CHECK_LAUNCH();
+        return MMI_OK;
+    }
     if (p.wide) {
         const dim3 grid(mmi_cdiv(a.Ntot, 32), mmi_cdiv(a.Mt, p.MTB), p.ksplit);
         ConvGemmArgs w = a;
@@ -510,7 +530,8 @@ void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
 // workgroup covers follows the group's own number of columns.
 int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
     const int N = a.Ntot, N1 = N / mem.frames;
-    // (T_shift is the group kernels' alone: a frame's columns divide by fewer than 2^11)
+    // (T_shift is the group kernels' alone: a frame's columns divide by fewer than 2^11; inputs are addressed by 32 bits of bytes)
+    if ((unsigned long)a.B * (unsigned long)a.x_bstride >= (1ul << 30)) return mmi_fail(MMI_ERR_UNSUPPORTED, "a conv's input of 4 GiB and more: lower max_batch");
     if (a.Cin * a.K >= (1 << 17) || N1 >= (1 << 17) || N >= (1 << 19) || a.T_out / mem.frames >= (1 << 11) || a.K >= (1 << 11))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "conv dimensions outside the range of the kernels' index arithmetic (sessions x samples per frame "
                                              "must stay below 131072: 68 sessions per handle at 1920 samples per frame; a frame below 2048 samples)");
@@ -537,11 +558,15 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
                 MMI_HIP_CHECK(mem.alloc(&a.partial, (size_t)p->ksplit * a.Mt * 32 * a.Npad));
             }
         }
-        int* tab = nullptr;
-        MMI_HIP_CHECK(mem.alloc(&tab, (size_t)a.Q * 8));
-        if (mem.there()) MMI_LAUNCH(k_conv_offsets, mmi_cdiv(a.Q * 8, 256), 256, 0, mem.stream, tab, a.Q, a.Cin, a.K, a.x_ld);
-        MMI_CHECK_LAUNCH();
-        a.koff = tab;
+        // a group's waves each take a whole reduction where there are tiles enough to give most SIMDs one; several m-tiles share a gathered value
+        // (128 -> 256, K 10 on 12384 columns with 1, 2, 4 of them: 144, 123, 115 us), except for reductions so short that the stores count (K 32 on
+        // 247680: 40 and 52 us).  With fewer tiles the waves of k_conv_wide share a reduction (512 -> 256, K 3 on 2064 columns: 42 against 53 us)
+        const long tiles = (long)mmi_cdiv(N, 32) * p->ksplit;
+        p->cols = mem.frames > 1 && tiles * a.Mt >= 700;
+        if (p->cols) {
+            p->MTB = a.Q < 8 ? 1 : 4;
+            while (p->MTB > 1 && (p->MTB > a.Mt || tiles * mmi_cdiv(a.Mt, p->MTB) < 700)) p->MTB >>= 1;
+        }
         return MMI_OK;
     }
     p->wide = false;                    // (at most 512 columns: T_shift is 0)

@@ -97,14 +97,6 @@ MMI_HD int mmi_fast_div(int n, unsigned magic, unsigned shift = 0u) {
 }
 enum { MMI_GOUT_NATURAL = 0, MMI_GOUT_PARTIAL = 1 };
 
-// k_conv_wide's offset table, see ConvGemmArgs::koff
-__global__ void k_conv_offsets(int* __restrict__ tab, int Q, int Cin, int K, int x_ld) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);          // (q, h, e)
-    if (i >= Q * 8) return;
-    const int kd = ((i >> 3) * 4 + (i & 3)) * 2 + ((i >> 2) & 1);
-    tab[i] = kd < Cin * K ? (kd / K) * x_ld + kd % K : 0;
-}
-
 struct ConvGemmArgs {
     const float* x;       // input [B][Cin][x_ld]; position p of a row = history (p < H) then the T new columns
     long x_bstride;       // Cin * x_ld
@@ -132,7 +124,6 @@ struct ConvGemmArgs {
     int elu_out;
     float* out2;
     // --- filled in by the engine's planner
-    const int* koff;      // k_conv_wide: [Q][2][4] input offset of kd = (q*4+e)*2 + h; 0 past Cin*K (the weights there are 0)
     const float* bp;      // k_gemm_f32: packed activations [ceil(N/32)][Q][64][4]
     int x_packed;         // the producer already wrote `bp` (no k_pack_b_f32 launch)
     int out_mode;         // MMI_GOUT_*
@@ -230,6 +221,43 @@ __device__ __forceinline__ void mmi_conv_store_n(const ConvGemmArgs& a, const in
     mmi_conv_put_n<NV>(a, co, b, t, ok, row, bia, rsv, v);
 }
 
+// The input's places (bytes from a.x on) of the four values of a quad that a lane of the 32 x 32 form takes, kd = 8 q + 2 e + kh for column
+// (b, t): the next quad's are a few additions away, where a table of offsets is one more load in front of the gathers (and a launch per conv
+// that fills it whenever a stream starts).  Reduction indices past the last one read some valid place: they meet zero weights.
+struct ConvWalk {
+    unsigned off[4], top, step, carry;
+    int tap[4], tap_step;
+    __device__ __forceinline__ void begin(const ConvGemmArgs& a, int b, int t, int q, int kh) {
+        const unsigned base = 4u * (unsigned)(b * (int)a.x_bstride + a.x_off + t * a.S);
+        const int c8 = mmi_fast_div(8, a.K_magic);
+        tap_step = 8 - c8 * a.K;
+        step = 4u * (unsigned)(c8 * a.x_ld + tap_step);
+        carry = 4u * (unsigned)(a.x_ld - a.K);
+        top = base + 4u * (unsigned)((a.Cin - 1) * a.x_ld + a.K - 1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int kd = q * 8 + 2 * e + kh, ci = mmi_fast_div(kd, a.K_magic);
+            tap[e] = kd - ci * a.K;
+            off[e] = base + 4u * (unsigned)(ci * a.x_ld + tap[e]);
+        }
+    }
+    __device__ __forceinline__ float at(const ConvGemmArgs& a, int e) const {
+        return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.x) + min(off[e], top));
+    }
+    __device__ __forceinline__ void advance(const ConvGemmArgs& a, bool on = true) {      // (selected, not branched around: the loads stay in one block)
+        const int ts = on ? tap_step : 0;
+        const unsigned st = on ? step : 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            tap[e] += ts;
+            off[e] += st;
+            const bool over = tap[e] >= a.K;
+            tap[e] -= over ? a.K : 0;
+            off[e] += over ? carry : 0u;
+        }
+    }
+};
+
 // GROUP: several frames of a stream at once - more columns per stream (T_shift), and the reduction also split over gridDim.z workgroups
 // where the frame program splits it (k_conv_finish adds their sums), cut as k_gemm_f32 cuts it
 template <int MTB, int W, int U, bool ELU_IN, bool GROUP>
@@ -242,7 +270,6 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
     const bool nvalid = n < a.Ntot;
     const int nn = nvalid ? n : 0;
     const int b = mmi_fast_div(nn, a.T_magic, tsh), t = nn - b * a.T_out;
-    const float* xb = a.x + (long)b * a.x_bstride + a.x_off + t * a.S;
     const int qb0 = GROUP ? min(a.Q, (int)blockIdx.z * a.q_blk) : 0, qb1 = GROUP ? min(a.Q, qb0 + a.q_blk) : a.Q;
     const int qper = (qb1 - qb0 + W - 1) / W;
     const int q0 = min(qb1, qb0 + wave * qper), q1 = min(qb1, q0 + qper);
@@ -255,8 +282,8 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
     const f32x4* wp[MTB];
 #pragma unroll
     for (int m = 0; m < MTB; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.wpk) + (long)min(mt0 + m, a.Mt - 1) * a.Q * 64 + lane;
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    const i32x4* ko = reinterpret_cast<const i32x4*>(a.koff) + kh;
+    ConvWalk in;
+    in.begin(a, b, t, q0, kh);
 
     // groups of U k-quads, double buffered: the gathers / weight fragments of group g+1 are in flight while group g
     // runs on the matrix core.  Loads past the slice are clamped to its last quad and their MFMAs skipped.
@@ -265,10 +292,10 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
 #define MMI_W_LOAD(AV, BV, qb)                                                                      \
     _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                 \
         const int qq = min((qb) + u, q1 - 1);                                                       \
-        const i32x4 o = ko[qq * 2];                                                                 \
-        /* plain unconditional gathers (a conditional load would be serialised behind s_waitcnt vmcnt(0)): reduction   \
-           indices past Cin*K point at offset 0 and meet zero weights; columns past Ntot are computed and discarded */  \
-        _Pragma("unroll") for (int e = 0; e < 4; ++e) BV[u][e] = xb[o[e]];                          \
+        /* plain unconditional gathers (a conditional load would be serialised behind s_waitcnt vmcnt(0)); columns past Ntot  \
+           are computed and discarded */                                                            \
+        _Pragma("unroll") for (int e = 0; e < 4; ++e) BV[u][e] = in.at(a, e);                       \
+        in.advance(a);                                                                              \
         _Pragma("unroll") for (int m = 0; m < MTB; ++m) AV[u][m] = wp[m][(long)qq * 64];           \
     }
 #define MMI_W_MMA(AV, BV, qb)                                                                       \
@@ -352,6 +379,109 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
                 v[i] = acc[m][r];
             }
             mmi_conv_store_n<8>(a, co, bb, tt, ok, v);
+        }
+    }
+}
+
+// k_conv_wide's sums by waves of their own: a wave owns 32 columns x MTB m-tiles and takes the `pieces` of its reduction - what k_conv_wide's waves
+// would split it into - one after the other, each from zero, and adds them up in the same order: the same bits without the exchange through LDS.
+// Four waves of a workgroup own neighbouring column tiles and read the same weights.  grid (ceil(column tiles / 4), ceil(Mt / MTB), ks).
+// PACKED: the operand as its producer packed it (`bp`).  Bound by the matrix core where a wave's reduction is long; what it loses are the gathers
+// (one load per value and wave, met by MTB m-tiles).
+// A file's 129 frames: 64 -> 128, K 8 on 61920 columns 151 -> 98 us (83 TFLOP/s), 128 -> 256, K 10 on 12384 144 -> 117, 512 -> 3072 on 2064 103 -> 87,
+// 256 -> 1280 on 12384 143 -> 99, 128 -> 512 on 61920 144 -> 112; stores bound the convs of few products (32 -> 64 on 247680: 59 -> 43).
+template <int MTB, int U, bool ELU_IN, bool PACKED>
+__global__ __launch_bounds__(256, 2) void k_conv_cols(ConvGemmArgs a, int pieces) {
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63, jl = lane & 31, kh = lane >> 5;
+    const int nt = (int)blockIdx.x * 4 + wave, n = nt * 32 + jl, mt0 = (int)blockIdx.y * MTB;
+    if (nt * 32 >= a.Ntot) return;
+    const bool nvalid = n < a.Ntot;
+    const int nn = nvalid ? n : 0, b = mmi_fast_div(nn, a.T_magic, a.T_shift), t = nn - b * a.T_out;
+    const f32x4* bp = PACKED ? reinterpret_cast<const f32x4*>(a.bp) + (long)nt * a.Q * 64 + lane : nullptr;
+    const int q0 = min(a.Q, (int)blockIdx.z * a.q_blk), q1 = min(a.Q, q0 + a.q_blk), qper = max((q1 - q0 + pieces - 1) / pieces, 1);
+    const f32x4* wp[MTB];
+#pragma unroll
+    for (int m = 0; m < MTB; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.wpk) + (long)min(mt0 + m, a.Mt - 1) * a.Q * 64 + lane;
+    ConvWalk in;
+    if constexpr (!PACKED) in.begin(a, b, t, q0, kh);
+    f32x16 acc[MTB], sum[MTB];
+#pragma unroll
+    for (int m = 0; m < MTB; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[m][r] = sum[m][r] = 0.f;
+    f32x4 avA[U][MTB], avB[U][MTB], bvA[U], bvB[U];
+    struct At { int q, end; };                               // a group of U quads: its first one, the end of its piece (where the group ends too)
+    auto after = [&](const At& at) __attribute__((always_inline)) {
+        At n = {at.q + U, at.end};
+        if (n.q >= at.end) { n.q = at.end; n.end = min(q1, at.end + qper); }
+        return n;
+    };
+    // no load is conditional, so that the wait in front of a product covers the older group only
+    auto load = [&](f32x4 (&av)[U][MTB], f32x4 (&bv)[U], const At& at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int qq = min(at.q + u, q1 - 1);
+            if constexpr (PACKED) bv[u] = bp[(long)qq * 64];
+            else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv[u][e] = in.at(a, e);
+                in.advance(a, at.q + u < at.end);
+            }
+#pragma unroll
+            for (int m = 0; m < MTB; ++m) av[u][m] = wp[m][(long)qq * 64];
+        }
+    };
+    auto mma = [&](f32x4 (&av)[U][MTB], f32x4 (&bv)[U], const At& at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool on = at.q + u < at.end;               // (quads past the piece's end meet zeros: a branch around them would cost a wait for all loads)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = ELU_IN ? mmi_elu(bv[u][e]) : bv[u][e], v = on ? x : 0.f;
+#pragma unroll
+                for (int m = 0; m < MTB; ++m) acc[m] = mmi_mfma_f32_32x32x2(av[u][m][e], v, acc[m]);
+            }
+        }
+        if (pieces > 1 && at.q + U >= at.end)
+#pragma unroll
+            for (int m = 0; m < MTB; ++m)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { sum[m][r] += acc[m][r]; acc[m][r] = 0.f; }
+    };
+    if (q0 < q1) {
+        At cur = {q0, min(q1, q0 + qper)};
+        load(avA, bvA, cur);
+        At next = after(cur);
+        while (next.q < q1) {                                // (one way out, at the end of a pair: a break between its halves costs a wait for all loads)
+            load(avB, bvB, next);
+            mmi_sched_barrier();
+            mma(avA, bvA, cur);
+            cur = after(next);
+            load(avA, bvA, cur);
+            mmi_sched_barrier();
+            mma(avB, bvB, next);
+            next = after(cur);
+        }
+        if (cur.q < q1) mma(avA, bvA, cur);
+    }
+#pragma unroll
+    for (int m = 0; m < MTB; ++m) {
+        if (mt0 + m >= a.Mt) break;
+#pragma unroll
+        for (int r0 = 0; r0 < 16; r0 += 8) {
+            int co[8], bb[8], tt[8];
+            bool ok[8];
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int r = r0 + i;
+                co[i] = (mt0 + m) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh;
+                ok[i] = nvalid && co[i] < a.Cout;
+                bb[i] = b; tt[i] = t;
+                v[i] = pieces > 1 ? sum[m][r] : acc[m][r];
+                if (a.out_mode == MMI_GOUT_PARTIAL) a.partial[((long)blockIdx.z * a.Mt * 32 + co[i]) * a.Npad + n] = v[i];
+            }
+            if (a.out_mode != MMI_GOUT_PARTIAL) mmi_conv_store_n<8>(a, co, bb, tt, ok, v);
         }
     }
 }
