@@ -803,22 +803,34 @@ int alloc_tr_stream(mmi_mimi* m, MimiMem& mem, int N, TrStream* x) {
     return MMI_OK;
 }
 
-template <int FN>
+template <int FN, bool NT>
 void launch_lin(hipStream_t s, const MimiLinArgs& a) {
     const dim3 grid(mmi_cdiv(a.M, 16), mmi_cdiv(a.N, 16 * FN));
-    if (!a.ln_w) MMI_LAUNCH((k_mimi_lin<1, FN, (FN == 1 ? 8 : 4), false>), grid, 512, 0, s, a);
-    else if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<1, FN, 4, true>), grid, 512, 0, s, a);
-    else MMI_LAUNCH((k_mimi_lin<1, FN, 8, true>), grid, 512, 0, s, a);
+    if (!a.ln_w) MMI_LAUNCH((k_mimi_lin<1, FN, (FN == 1 ? 8 : 4), false, NT>), grid, 512, 0, s, a);
+    else if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<1, FN, 4, true, NT>), grid, 512, 0, s, a);
+    else MMI_LAUNCH((k_mimi_lin<1, FN, 8, true, NT>), grid, 512, 0, s, a);
 }
 
 int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
     if (a.ln_w && (a.J > 64 || a.J * 16 != K)) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi transformer: a width of at most 1024, a multiple of 16");
     // 16 columns per workgroup while the chip holds all workgroups at once (two per CU): 32 streams 1387 -> 1327 us a frame
-    // with 16 for 32.  Beyond that 32, which read the weights half as often (32 x 32 tiles measured no different).
+    // with 16 for 32.  Beyond that 32, which read the weights half as often (32 x 32 tiles measured no different); with a norm 128 rows
+    // per workgroup where those fill half the chip.  Weights that one tile of columns reads leave no line behind, others' are read again
+    // (32 streams 1211 -> 1201 us)
     const bool narrow = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16) <= 512;
+    const bool rows = a.ln_w && (long)mmi_cdiv(a.M, 128) * mmi_cdiv(a.N, 16) >= 128;
+    int waves = 8;                                           // more of them where that gives every workgroup a CU of its own (2048 x 258: 19.5 -> 15.6 us)
+    while (waves < 12 && (long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) ++waves;
+    if ((long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) waves = 8;
     prog.add([=](hipStream_t s) {
-        if (narrow) launch_lin<1>(s, a);
-        else launch_lin<2>(s, a);
+        if (rows) {
+            const dim3 grid(mmi_cdiv(a.M, 16 * waves), mmi_cdiv(a.N, 16));
+            const size_t smem = (size_t)a.J * 64 * sizeof(f32x4);
+            if (a.J <= 32) MMI_LAUNCH((k_mimi_lin_rows<4>), grid, 64 * waves, smem, s, a);
+            else MMI_LAUNCH((k_mimi_lin_rows<8>), grid, 64 * waves, smem, s, a);
+        } else if (narrow && a.N <= 16) launch_lin<1, true>(s, a);
+        else if (narrow) launch_lin<1, false>(s, a);
+        else launch_lin<2, false>(s, a);
         MMI_CHECK_LAUNCH();
         return (int)MMI_OK;
     });

@@ -991,8 +991,9 @@ struct MimiLinArgs {
 // 16-wide tiles (a live stream has two columns: a 32-wide tile keeps the matrix core busy four times as long, 1.7 us at K = 512, on half the
 // CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (KJ fragments per wave), and
 // no reduction split over workgroups (K = 2048 needed a second launch to add the sums).
-template <int FM, int FN, int U, bool LN>
+template <int FM, int FN, int U, bool LN, bool NT>
 __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
+    auto weight = [](const f32x4* p) __attribute__((always_inline)) { return NT ? mmi_load_nt(p) : *p; };
     const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int m0 = (int)blockIdx.x * FM, n0 = (int)blockIdx.y * FN;
     const int Mt = (a.M + 15) >> 4, Nt = (a.N + 15) >> 4;
@@ -1051,7 +1052,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
         for (int u = 0; u < U; ++u) {
             const int uu = min(u, last);
 #pragma unroll
-            for (int m = 0; m < FM; ++m) wv[u][m] = mmi_load_nt(wp[m] + uu * 64);
+            for (int m = 0; m < FM; ++m) wv[u][m] = weight(wp[m] + uu * 64);
             gv[u] = gp[uu * 4];
             bv[u] = hp[uu * 4];
         }
@@ -1113,7 +1114,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
             for (int u = 0; u < U; ++u) {
                 const int uu = min(at + u, last);
 #pragma unroll
-                for (int m = 0; m < FM; ++m) w[u][m] = mmi_load_nt(wp[m] + (long)uu * 64);
+                for (int m = 0; m < FM; ++m) w[u][m] = weight(wp[m] + (long)uu * 64);
 #pragma unroll
                 for (int n = 0; n < FN; ++n) x[u][n] = xp[n][(long)uu * 64];
             }
@@ -1161,6 +1162,105 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
             const int b = mmi_fast_div(rn[i], a.T_magic, a.T_shift), t = rn[i] - b * a.T;
             a.out[((long)b * a.M + rm[i]) * a.out_ld + a.out_off + t] = v;
         }
+    }
+}
+
+// norm + linear of many columns: a workgroup of 8 to 12 waves owns 16 rows per wave x 16 columns, grid (row tiles / waves, ceil(N/16)).  Wave w < 8
+// normalises piece w of the reduction, as k_mimi_lin's does, and leaves it in LDS; then a wave takes the eight pieces one after the other, each from zero, added in
+// rising order: k_mimi_lin's bits.  With 16 rows per workgroup every column was normalised by 96 - 128 of them - 570 vector instructions around 32
+// products per wave: a file's 258 columns 512 -> 1536 15.5 -> 11.5 us, 512 -> 2048 20.1 -> 15.6.  J <= 64.
+template <int KJ>
+__global__ __launch_bounds__(768) void k_mimi_lin_rows(MimiLinArgs a) {
+    constexpr int U = 8;
+    MMI_DYN_SHARED(f32x4, y);                                // [J][64]
+    MMI_SHARED float stat[2][8][16];
+    const int tid = (int)threadIdx.x, wave = mmi_uniform(tid >> 6), lane = tid & 63;
+    const int rt = (int)blockIdx.x * ((int)blockDim.x >> 6) + wave, n0 = (int)blockIdx.y * 16, Mt = (a.M + 15) >> 4;
+    const int per = (a.J + 7) >> 3, j0 = min(a.J, wave * per), nj = min(a.J, j0 + per) - j0;      // <= KJ (the planner checks)
+    const int jl = min(j0, a.J - 1), last = nj > 0 ? nj - 1 : 0;
+    const f32x4* xp = reinterpret_cast<const f32x4*>(a.x) + ((long)blockIdx.y * a.J + jl) * 64 + (lane & 48) + min(lane & 15, a.N - n0 - 1);
+    const f32x4* gp = reinterpret_cast<const f32x4*>(a.ln_w) + (long)jl * 4 + (lane >> 4);
+    const f32x4* hp = reinterpret_cast<const f32x4*>(a.ln_b) + (long)jl * 4 + (lane >> 4);
+    const f32x4* wp = reinterpret_cast<const f32x4*>(a.w) + (long)min(rt, Mt - 1) * a.J * 64 + lane;
+    f32x4 xv[KJ], gv[KJ], bv[KJ], wA[U], wB[U];
+    auto load = [&](f32x4 (&w)[U], int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = wp[(long)min(j + u, a.J - 1) * 64];
+    };
+#pragma unroll
+    for (int u = 0; u < KJ; ++u) xv[u] = xp[min(u, last) * 64];
+#pragma unroll
+    for (int u = 0; u < KJ; ++u) { gv[u] = gp[min(u, last) * 4]; bv[u] = hp[min(u, last) * 4]; }
+    load(wA, 0);
+    mmi_sched_barrier();
+    auto column_sum = [&](int which, float s) __attribute__((always_inline)) {
+        s += mmi_shfl_xor(s, 16);
+        s += mmi_shfl_xor(s, 32);
+        if (lane < 16 && wave < 8) stat[which][wave][lane] = s;
+        __syncthreads();
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) t += stat[which][w][lane & 15];
+        return t;
+    };
+    float s = 0.f;
+#pragma unroll
+    for (int u = 0; u < KJ; ++u)
+        if (u < nj) s += (xv[u][0] + xv[u][1]) + (xv[u][2] + xv[u][3]);
+    const float mean = column_sum(0, s) / (float)(a.J * 16);
+    s = 0.f;
+#pragma unroll
+    for (int u = 0; u < KJ; ++u)
+        if (u < nj)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float d = xv[u][e] - mean;
+                s += d * d;
+            }
+    const float rstd = mmi_rsqrtf(column_sum(1, s) / (float)(a.J * 16) + a.ln_eps);
+#pragma unroll
+    for (int u = 0; u < KJ; ++u)
+        if (u < nj) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (xv[u][e] - mean) * rstd * gv[u][e] + bv[u][e];
+            y[(j0 + u) * 64 + lane] = v;
+        }
+    __syncthreads();
+    if (rt >= Mt) return;
+
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sum = acc;
+    int end = per;
+    auto mma = [&](f32x4 (&w)[U], int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j + u == end) { sum += acc; acc = f32x4{0.f, 0.f, 0.f, 0.f}; end += per; }
+            f32x4 v = y[min(j + u, a.J - 1) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = mmi_mfma_f32_16x16x4(w[u][e], j + u < a.J ? v[e] : 0.f, acc);
+        }
+    };
+    int j = 0;
+    while (j + U < a.J) {                                    // pairs of groups, one way out (k_conv_cols)
+        load(wB, j + U);
+        mmi_sched_barrier();
+        mma(wA, j);
+        load(wA, j + 2 * U);
+        mmi_sched_barrier();
+        mma(wB, j + U);
+        j += 2 * U;
+    }
+    if (j < a.J) mma(wA, j);
+    sum += acc;
+    const int n = n0 + (lane & 15);
+    if (n >= a.N) return;
+    const int b = mmi_fast_div(n, a.T_magic, a.T_shift), t = n - b * a.T;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int m = rt * 16 + 4 * (lane >> 4) + r;
+        if (m >= a.M) continue;
+        if (a.mode == MIMI_LIN_GELU) a.outp[mmi_lin_index(m, n, a.outJ)] = mmi_gelu_erf(sum[r]);
+        else a.out[((long)b * a.M + m) * a.out_ld + a.out_off + t] = sum[r];
     }
 }
 

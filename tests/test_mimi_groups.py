@@ -324,3 +324,16 @@ def test_a_mask_set_by_a_graph_is_seen():
             for m in (a, b):
                 m.set_exec_mask(everyone)
             same(0, everyone)                                  # the stream that stood still goes on where it stood
+
+
+@pytest.mark.parametrize("heads,ff", [(9, 2056), (33, 2048)])
+def test_norms_and_linears_of_many_columns(sim_lib, heads, ff):
+    """k_mimi_lin_rows (a feed-forward of some 2048 rows on 114 columns, enough workgroups for it) against k_mimi_lin's frame-by-frame bits: rows
+    that fill no whole workgroup, a norm over 9 and over 33 fragments (pieces that are empty, and longer than four)."""
+    cfg = replace(tiny_mimi_config(), dimension=16 * heads, tr_d_model=16 * heads, tr_num_heads=heads, tr_dim_feedforward=ff, tr_num_layers=1)
+    m = MimiModel(random_mimi_state_dict(cfg, seed=8), cfg, device="cpu", max_batch=1, num_codebooks=2, lib=sim_lib)
+    codes = torch.randint(0, cfg.q_bins, (1, 2, 57), generator=torch.Generator().manual_seed(3))
+    with m.streaming(1):
+        whole = m.decode(codes)
+    with m.streaming(1):
+        assert torch.equal(whole, torch.cat([m.decode(codes[..., f:f + 1]) for f in range(57)], -1))
