@@ -465,6 +465,22 @@ int launch_once(hipStream_t s, int T, int mt, int kmax, dim3 groups, const GemmA
     return MMI_OK;
 }
 
+// while profiling: the event in front of a launch of the dominant linear, and the one that goes behind it (*ev; null: not profiling)
+hipError_t dominant_begin(mmi_lm* lm, hipStream_t s, EvPair** ev) {
+    *ev = nullptr;
+    if (!lm->profiling) return hipSuccess;
+    if (lm->ev_used == lm->ev_pool.size()) {
+        EvPair pr;
+        hipError_t e = hipEventCreate(&pr.a);
+        if (e == hipSuccess) e = hipEventCreate(&pr.b);
+        if (e != hipSuccess) return e;
+        lm->ev_pool.push_back(pr);
+    }
+    *ev = &lm->ev_pool[lm->ev_used++];
+    lm->prof_stream = s;
+    return hipEventRecord((*ev)->a, s);
+}
+
 int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_dominant) {
     a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT;
     a.wscale = g.scale; a.wscb = g.scb; a.gate_rows = g.gate ? g.N : 0;
@@ -475,17 +491,7 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
     a.osplit = plan_osplit(g, p, a.epi, g.T);
     const XldsPlan xl = plan_xlds(lm, g, a, mt);
     EvPair* ev = nullptr;
-    if (lm->profiling && is_dominant) {
-        if (lm->ev_used == lm->ev_pool.size()) {
-            EvPair pr;
-            MMI_HIP_CHECK(hipEventCreate(&pr.a));
-            MMI_HIP_CHECK(hipEventCreate(&pr.b));
-            lm->ev_pool.push_back(pr);
-        }
-        ev = &lm->ev_pool[lm->ev_used++];
-        lm->prof_stream = s;
-        MMI_HIP_CHECK(hipEventRecord(ev->a, s));
-    }
+    if (is_dominant) MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
     int rc;
     mmi_record_bytes((long)g.bytes);
     if (is_dominant) lm->dominant_xlds = xl.on;
@@ -733,6 +739,23 @@ void add_norm_gemm(mmi_lm* lm, const GemmW& g, uint16_t* x, const uint16_t* alph
     }, gbytes);
 }
 
+// Does one launch take norm and linear (k_gemm_norm_one)?  One session, bf16 weights on the 16-row tile, a row of at most 4096 features and whole
+// pieces of 8, no split sums pending; with more sessions a workgroup's rows would cost as much as its weights.
+bool norm_one(const mmi_lm* lm, const GemmW& g, const Pending& pd, int D) {
+    return lm->batch == 1 && lm->T == 16 && g.T == 16 && g.wq == 0 && pd.P == 0 && D % 8 == 0 && D <= 4096 && g.KSTEPS <= 128 && !getenv("MMI_NO_NORM_FUSION");
+}
+int launch_norm_one(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, const uint16_t* x, const uint16_t* alpha, int D, bool is_dominant) {
+    a.xp = reinterpret_cast<const u32x4*>(x); a.alpha = alpha; a.D = D; a.eps = 1e-8f;
+    a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT; a.gate_rows = g.gate ? g.N : 0; a.osplit = 1;
+    mmi_record_bytes((long)g.bytes);
+    EvPair* ev = nullptr;
+    if (is_dominant) MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
+    MMI_LAUNCH(k_gemm_norm_one<4>, g.NT, 512, 0, s, a);
+    MMI_CHECK_LAUNCH();
+    if (ev) MMI_HIP_CHECK(hipEventRecord(ev->b, s));
+    return MMI_OK;
+}
+
 // bf16 packed tensor -> its row-wise int8 copy + the rows' absmax (lm->act8): one workgroup per row
 void add_quant_rows(mmi_lm* lm, const uint16_t* xp, uint8_t* xq, float* sx, int features, int tile = 0) {
     const int B = lm->batch, T = tile ? tile : lm->T, ksteps = packed_ksteps_t(lm, T, features);
@@ -954,7 +977,8 @@ int build_program(mmi_lm* lm) {
     for (int l = 0; l < c.num_layers; ++l) {
         const LayerW& L = lm->layers[l];
         P.site("L.norm1");
-        add_resid_rmsnorm(lm, lm->x, pending, L.n1, lm->xn, d, a8 ? lm->xnq : nullptr, a8 ? lm->sx_xn : nullptr);
+        const bool one1 = !a8 && norm_one(lm, L.in_proj, pending, d);
+        if (!one1) add_resid_rmsnorm(lm, lm->x, pending, L.n1, lm->xn, d, a8 ? lm->xnq : nullptr, a8 ? lm->sx_xn : nullptr);
         if (l == 1) add_hidden_tap(lm, 0);     // x is complete (the previous linear_out's partials folded in) right after this norm
         LmAttnArgs a;
         a.qrot = lm->qrot; a.kc = lm->kc + l * kv_layer; a.vc = lm->vc + l * kv_layer;
@@ -971,7 +995,9 @@ int build_program(mmi_lm* lm) {
             ga.qrot = a.qrot; ga.kc = a.kc; ga.vc = a.vc; ga.offsets = lm->offsets_m; ga.H = H; ga.Dh = Dh; ga.cap = c.context; ga.kv8 = kv8 ? 1 : 0;
             ga.max_period = c.max_period; ga.rope = lm->rope;
             GemmW gw = L.in_proj;
-            P.add([lm, gw, ga](hipStream_t s) { return launch_gemm(lm, s, gw, ga, false); }, (long)gw.bytes);
+            const uint16_t *x = lm->x, *alpha = L.n1;
+            if (one1) P.add([lm, gw, ga, x, alpha, d](hipStream_t s) { return launch_norm_one(lm, s, gw, ga, x, alpha, d, false); }, (long)gw.bytes);
+            else P.add([lm, gw, ga](hipStream_t s) { return launch_gemm(lm, s, gw, ga, false); }, (long)gw.bytes);
         }
         P.site("L.attn");
         P.add([=](hipStream_t s) {
@@ -1022,7 +1048,8 @@ int build_program(mmi_lm* lm) {
             pending = add_gemm_resid(lm, L.x_out, lm->att, lm->x, d);
         }
         P.site("L.norm2");
-        add_resid_rmsnorm(lm, lm->x, pending, L.n2, lm->xn, d, a8 ? lm->xnq : nullptr, a8 ? lm->sx_xn : nullptr);
+        const bool one2 = !a8 && norm_one(lm, L.ffn_in, pending, d);
+        if (!one2) add_resid_rmsnorm(lm, lm->x, pending, L.n2, lm->xn, d, a8 ? lm->xnq : nullptr, a8 ? lm->sx_xn : nullptr);
         P.site("L.ffn_in");
         if (a8) {
             Q8 qi{3, lm->sx_xn};
@@ -1034,6 +1061,15 @@ int build_program(mmi_lm* lm) {
             pending = add_gemm_resid(lm, L.ffn_out, reinterpret_cast<const uint16_t*>(lm->hbq), lm->x, d, &qo);
             continue;
         }
+        if (one2) {
+            GemmArgs ga;
+            memset(&ga, 0, sizeof(ga));
+            ga.out = lm->hb; ga.epi = MMI_EPI_GATE; ga.B = B; ga.tok_rows = lm->gen_batch;
+            ga.out_mode = MMI_OUT_PACKED; ga.out_ld = c.ffn_hidden; ga.out_ksteps = packed_ksteps(lm, c.ffn_hidden);
+            const GemmW gw = L.ffn_in;
+            const uint16_t *x = lm->x, *alpha = L.n2;
+            P.add([lm, gw, ga, x, alpha, d](hipStream_t s) { return launch_norm_one(lm, s, gw, ga, x, alpha, d, /*dominant=*/true); }, (long)gw.bytes);
+        } else
         add_gemm(lm, L.ffn_in, lm->xn, lm->hb, c.ffn_hidden, true, MMI_EPI_GATE, nullptr, nullptr, nullptr, 0, /*dominant=*/true);
         P.site("L.ffn_out");
         pending = add_gemm_resid(lm, L.ffn_out, lm->hb, lm->x, d);

@@ -707,6 +707,82 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
     mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi);
 }
 
+// ONE session: RMSNorm + a weight stream on the 16-row tile (the temporal in_proj and linear_in).  A workgroup's 512 threads normalise the row -
+// k_resid_rmsnorm's pieces, sums and roundings, so its bits - into LDS, with the wave's first two groups of weights on their way; the main loop takes its
+// activations from there, 16 bytes for all 16 columns of the tile (column 0 is the session).  The norm was a launch of 4.6 us in front of each, 64 per
+// step; here it costs a workgroup a trip for 8 KB under another workgroup's stream: in_proj 21.6 + 4.6 -> 24.1 us, linear_in 36.3 + 4.6 -> 37.4.
+template <int U>
+__global__ __launch_bounds__(512, 4) void k_gemm_norm_one(GemmArgs a) {
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63, kq = lane >> 4, nt0 = (int)blockIdx.x;
+    const int kper = (a.KSTEPS + 7) >> 3, ks0 = min(a.KSTEPS, wave * kper), nks = min(a.KSTEPS, ks0 + kper) - ks0;
+    const u32x4* wp = a.wp + ((long)nt0 * a.KSTEPS + min(ks0, a.KSTEPS - 1)) * 64 + lane;
+    MMI_SHARED __attribute__((aligned(16))) u32x4 row[512];          // [k-step][kq]: D <= 4096 (the planner checks)
+    MMI_SHARED float part[8];
+    u32x4 wA[U], wB[U];
+    auto load = [&](u32x4 (&w)[U], int k) __attribute__((always_inline)) {      // unconditional, past the slice its last k-step again
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = mmi_load_nt(wp + (long)max(min(k + u, nks - 1), 0) * 64);
+    };
+    load(wA, 0);
+    load(wB, U);
+    {
+        const int i = tid * 8, at = min(i, a.D - 8);
+        const u32x4 v = a.xp[(at >> 5) * 64 + ((at >> 3) & 3) * 16], al = *reinterpret_cast<const u32x4*>(a.alpha + at);
+        float f[8], ss = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f[2 * q] = mmi_bf16_to_f32((uint16_t)(v[q] & 0xffffu));
+            f[2 * q + 1] = mmi_bf16_to_f32((uint16_t)(v[q] >> 16));
+        }
+        if (i < a.D)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) ss += mmi_shfl_xor(ss, m);
+        if (lane == 0) part[wave] = ss;
+        __syncthreads();
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) tot += part[w];
+        const float rs = mmi_rsqrtf(a.eps + tot / (float)a.D);
+        u32x4 o = {0u, 0u, 0u, 0u};
+        if (i < a.D)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float alo = mmi_bf16_to_f32((uint16_t)(al[q] & 0xffffu)), ahi = mmi_bf16_to_f32((uint16_t)(al[q] >> 16));
+                o[q] = mmi_pack_bf16x2(f[2 * q] * (alo * rs), f[2 * q + 1] * (ahi * rs));
+            }
+        row[tid] = o;
+        __syncthreads();
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto mma = [&](u32x4 (&w)[U], int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool on = k + u < nks;
+            u32x4 x = row[min(ks0 + k + u, a.KSTEPS - 1) * 4 + kq];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = on ? x[q] : 0u;
+            acc = mmi_mfma_bf16_16x16x32(w[u], x, acc);
+        }
+    };
+    int k = 0;
+    while (k + U < nks) {
+        mma(wA, k);
+        load(wA, k + 2 * U);
+        mmi_sched_barrier();
+        mma(wB, k + U);
+        load(wB, k + 3 * U);
+        mmi_sched_barrier();
+        k += 2 * U;
+    }
+    if (k < nks) mma(wA, k);
+    float accv[1][1][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) accv[0][0][r] = acc[r];
+    mmi_gemm_epilogue<16, 1, 1, 8>(a, accv, wave, lane, nt0, u32x4{0u, 0u, 0u, 0u}, nullptr, 0, 2);
+}
+
 // RMSNorm fused into the GEMM that consumes it (the depth transformer: norm1 -> in_proj, norm2 -> linear_in; rows of
 // 1024 features): y = (x.float() * (alpha.float() * rsqrt(eps + mean(x^2)))).to(bf16) (transformer.py:45-58), then
 // out = y @ W^T.  A wave's whole K-slice of activation and weight fragments (<= KMAX k-steps) is loaded in one go -

@@ -533,3 +533,13 @@ def test_debug_trace_of_two_sessions_is_identical(sim_lib, monkeypatch, tmp_path
     assert len(traces) == 2 and traces[0].read_text() == traces[1].read_text() and len(traces[0].read_text().splitlines()) > 100
     dumps = sorted(tmp_path.glob("trace.*.a10"))
     assert len(dumps) == 2 and dumps[0].read_bytes() == dumps[1].read_bytes() and any(dumps[0].read_bytes())
+
+
+@pytest.mark.parametrize("dim,heads", [(96, 3), (128, 4), (1088, 17)])
+def test_norm_and_linear_in_one_launch(sim_lib, dim, heads):
+    """k_gemm_norm_one at one session against the oracle: fewer k-steps than waves, slices that are no multiple of a group of loads, a row that leaves
+    most of a workgroup's threads without a piece."""
+    from dataclasses import replace
+    st = {}
+    lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), dim=dim, num_heads=heads), seed=60 + heads, B=1, S=3, stats=st)
+    assert st["launch_sites"].get("L.norm1", 0) == 0 and st["launch_sites"].get("L.in_proj", 0) == 2
