@@ -803,21 +803,25 @@ int alloc_tr_stream(mmi_mimi* m, MimiMem& mem, int N, TrStream* x) {
     return MMI_OK;
 }
 
-template <int FN, bool NT>
+template <int FM, int FN, int U, bool NT>
 void launch_lin(hipStream_t s, const MimiLinArgs& a) {
-    const dim3 grid(mmi_cdiv(a.M, 16), mmi_cdiv(a.N, 16 * FN));
-    if (!a.ln_w) MMI_LAUNCH((k_mimi_lin<1, FN, (FN == 1 ? 8 : 4), false, NT>), grid, 512, 0, s, a);
-    else if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<1, FN, 4, true, NT>), grid, 512, 0, s, a);
-    else MMI_LAUNCH((k_mimi_lin<1, FN, 8, true, NT>), grid, 512, 0, s, a);
+    MMI_LAUNCH((k_mimi_lin<FM, FN, U, false, NT>), dim3(mmi_cdiv(a.M, 16 * FM), mmi_cdiv(a.N, 16 * FN)), 512, 0, s, a);
+}
+template <int FM, int FN, bool NT>
+void launch_lin_norm(hipStream_t s, const MimiLinArgs& a) {
+    const dim3 grid(mmi_cdiv(a.M, 16 * FM), mmi_cdiv(a.N, 16 * FN));
+    if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<FM, FN, 4, true, NT>), grid, 512, 0, s, a);
+    else MMI_LAUNCH((k_mimi_lin<FM, FN, 8, true, NT>), grid, 512, 0, s, a);
 }
 
 int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
     if (a.ln_w && (a.J > 64 || a.J * 16 != K)) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi transformer: a width of at most 1024, a multiple of 16");
-    // 16 columns per workgroup while the chip holds all workgroups at once (two per CU): 32 streams 1387 -> 1327 us a frame
-    // with 16 for 32.  Beyond that 32, which read the weights half as often (32 x 32 tiles measured no different); with a norm 128 rows
-    // per workgroup where those fill half the chip.  Weights that one tile of columns reads leave no line behind, others' are read again
-    // (32 streams 1211 -> 1201 us)
-    const bool narrow = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16) <= 512;
+    // 16 x 16 tiles while the chip holds all workgroups at once (two per CU); with a norm 32 rows share it from 256 tiles on (32 streams 1203 -> 1186
+    // us a frame; with 192 - 256 tiles, 16 streams, 973 -> 1000).  Beyond that 32 x 32 in groups of two fragments (258 columns, K = 2048: 17.5 -> 13.0
+    // us, 16 x 16 13.9), with a norm 128 rows per workgroup where those fill half the chip.  Groups of 4 fragments, not 8: with K = 512 a wave has
+    // 4 (one stream 717 -> 688 us a frame, 16 streams 973 -> 946).  Weights that one tile of columns reads leave no line behind, others' are read
+    // again (32 streams 1211 -> 1201 us).
+    const long tiles = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16);
     const bool rows = a.ln_w && (long)mmi_cdiv(a.M, 128) * mmi_cdiv(a.N, 16) >= 128;
     int waves = 8;                                           // more of them where that gives every workgroup a CU of its own (2048 x 258: 19.5 -> 15.6 us)
     while (waves < 12 && (long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) ++waves;
@@ -828,9 +832,16 @@ int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
             const size_t smem = (size_t)a.J * 64 * sizeof(f32x4);
             if (a.J <= 32) MMI_LAUNCH((k_mimi_lin_rows<4>), grid, 64 * waves, smem, s, a);
             else MMI_LAUNCH((k_mimi_lin_rows<8>), grid, 64 * waves, smem, s, a);
-        } else if (narrow && a.N <= 16) launch_lin<1, true>(s, a);
-        else if (narrow) launch_lin<1, false>(s, a);
-        else launch_lin<2, false>(s, a);
+        } else if (!a.ln_w) {
+            if (a.N <= 16) launch_lin<1, 1, 4, true>(s, a);
+            else if (tiles <= 512) launch_lin<1, 1, 4, false>(s, a);
+            else launch_lin<2, 2, 2, false>(s, a);
+        } else {
+            if (a.N <= 16 && tiles <= 512) launch_lin_norm<1, 1, true>(s, a);
+            else if (tiles <= 256) launch_lin_norm<1, 1, false>(s, a);
+            else if (tiles <= 512) launch_lin_norm<2, 1, false>(s, a);
+            else launch_lin_norm<1, 2, false>(s, a);
+        }
         MMI_CHECK_LAUNCH();
         return (int)MMI_OK;
     });

@@ -985,8 +985,8 @@ struct MimiLinArgs {
 // grid (ceil(Mt/FM), ceil(N/(16 FN))); a workgroup owns 16 FM rows x 16 FN columns; its 8 waves cut the reduction into 8 pieces, their sums are
 // added in rising order.  What a workgroup covers changes no bit (a piece and its order are the reduction's alone), so one stream, many
 // streams and groups of frames agree.
-// Measured, 1 stream (N = 2): norm + linear 8.2 -> 5.1 us, K = 2048 9.3 (with its second launch) -> 6.9; 32 streams (N = 64) 8.4 -> 7.3, 9.6 -> 7.5;
-// a file's 258 columns: norm + linear 18.6 -> 18.7, K = 2048 19.2 -> 16.
+// Measured, 1 stream (N = 2): norm + linear 8.2 -> 5.0 us, K = 512 5.9 -> 4.7, K = 2048 9.3 (with a second launch that added its sums) -> 6.6; 32 streams
+// (N = 64): norm + linear 8.4 -> 6.3, K = 2048 9.6 -> 6.9; a file's 258 columns: K = 512 7.9 -> 6.2, K = 2048 19.2 -> 13.0 (norm + linear: k_mimi_lin_rows).
 // Bound by latency: one column tile has M / 16 workgroups of 16 KB - 64 KB of weights and a few hundred cycles of matrix work each.  Hence
 // 16-wide tiles (a live stream has two columns: a 32-wide tile keeps the matrix core busy four times as long, 1.7 us at K = 512, on half the
 // CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (KJ fragments per wave), and
@@ -1121,22 +1121,30 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
         };
         auto mma = [&](const f32x4 (&w)[U][FM], const f32x4 (&x)[U][FN], int at) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (at + u < nj)
+            for (int u = 0; u < U; ++u) {
+                const bool on = at + u < nj;                 // (past the slice: zeros, not a branch - see k_conv_cols)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-                        for (int m = 0; m < FM; ++m)
+                    for (int n = 0; n < FN; ++n) {
+                        const float v = on ? x[u][n][e] : 0.f;
 #pragma unroll
-                            for (int n = 0; n < FN; ++n) acc[m][n] = mmi_mfma_f32_16x16x4(w[u][m][e], x[u][n][e], acc[m][n]);
+                        for (int m = 0; m < FM; ++m) acc[m][n] = mmi_mfma_f32_16x16x4(w[u][m][e], v, acc[m][n]);
+                    }
+            }
         };
         load(wA, xA, 0);
-        for (int at = 0; at < nj; at += 2 * U) {
+        int at = 0;
+        while (at + U < nj) {
             load(wB, xB, at + U);
+            mmi_sched_barrier();
             mma(wA, xA, at);
-            if (at + 2 * U < nj) load(wA, xA, at + 2 * U);
+            load(wA, xA, at + 2 * U);
+            mmi_sched_barrier();
             mma(wB, xB, at + U);
+            at += 2 * U;
         }
+        if (at < nj) mma(wA, xA, at);
     }
 
     MMI_SHARED float red[8 * FM * FN * 256];
