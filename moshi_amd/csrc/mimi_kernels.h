@@ -78,15 +78,17 @@ __global__ void k_codebook_prepare(const float* __restrict__ esum, const float* 
 // implicit-GEMM conv / linear
 // ------------------------------------------------------------------------------------------------
 // out[co][n=(b,t)] = sum_{kd=(ci,k)} W[co][kd] * act(in[b][ci][t*S + k]), fp32 MFMA 32x32x2 (exact fma chain).
-// Two kernels cover the codec:
 //   k_conv_wide  (N = B*T_out > 128 columns: SEANet layers at audio rate).  A wave owns 32 columns x MTB m-tiles x a
 //                K-slice; lane (j, h) gathers exactly the B-operand elements its own MFMA lane consumes
 //                (column j, reduction index kd = 2q+h), applies ELU once, and reuses them for the MTB m-tiles.
-//                The reduction index -> input offset map (ci*x_ld + k) is a per-layer table, 16 bytes per k-quad.
-//   k_gemm_f32   (N <= 128: the 12.5/25 Hz layers - transformer linears, last strided convs, resampling, RVQ
-//                projections; weights dominate).  Same shape as the LM's weight-streaming GEMM: one m-tile per
-//                workgroup, K split over waves (+ workgroups), activations pre-packed into B-fragment order by
-//                k_pack_b_f32 (im2col + ELU + replicate padding) or by the producing kernel.
+//                The input offsets (ci*x_ld + k) of the next quad are a few additions away (ConvWalk).
+//   k_conv_cols  the same sums, bit for bit, in groups of frames: a wave takes all slices of a reduction in turn.
+//   k_gemm_f32   (N <= 128: the 12.5/25 Hz layers - last strided convs, resampling, RVQ projections; weights
+//                dominate).  Same shape as the LM's weight-streaming GEMM: one m-tile per workgroup, K split over
+//                waves (+ workgroups), activations pre-packed into B-fragment order by k_pack_b_f32 (im2col + ELU +
+//                replicate padding) or by the producing kernel.
+//   k_conv_few   the same sums, bit for bit, for few streams: 16 x 16 tiles, operands from the input as it lies.
+// The transformers' linears have kernels of their own (k_mimi_lin, k_mimi_lin_rows).
 // n / d for 0 <= n < 2^20 and 1 <= d < 2^20 (column and tap indices) as one multiply-high and a shift: an integer division costs
 // ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^(32 + shift) / d), 0 means d == 1; exact while
 // n d < 2^(32 + shift), hence the 8 more bits (which still fit the magic number) from d = 2^11 on.

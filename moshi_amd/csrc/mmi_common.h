@@ -86,7 +86,7 @@ struct MmiWeights {
 
 // device allocation bookkeeping: every engine frees what it allocated
 // chunk > 0: allocations up to an eighth of it are cut out of pieces of that size, zeroed when they are made, instead of each being one of
-// the runtime's (a stream of the codec is some 90 of them: start 0.60 -> 0.20 ms, with its offset tables written by the GPU; stop 0.18 -> 0.09)
+// the runtime's (a stream of the codec is some 90 of them: start 0.60 -> 0.20 ms, when its convs still had offset tables, written by the GPU; stop 0.18 -> 0.09)
 struct MmiArena {
     std::vector<void*> ptrs;
     std::vector<size_t> sizes;
