@@ -822,7 +822,7 @@ int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
     // 4 (one stream 717 -> 688 us a frame, 16 streams 973 -> 946).  Weights that one tile of columns reads leave no line behind, others' are read
     // again (32 streams 1211 -> 1201 us).
     const long tiles = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16);
-    const bool rows = a.ln_w && (long)mmi_cdiv(a.M, 128) * mmi_cdiv(a.N, 16) >= 128;
+    const bool rows = a.ln_w && a.J <= 60 && (long)mmi_cdiv(a.M, 128) * mmi_cdiv(a.N, 16) >= 128;      // (J KB of LDS and a little more, below 64)
     int waves = 8;                                           // more of them where that gives every workgroup a CU of its own (2048 x 258: 19.5 -> 15.6 us)
     while (waves < 12 && (long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) ++waves;
     if ((long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) waves = 8;

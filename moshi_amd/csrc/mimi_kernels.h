@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
 // norm + linear of many columns: a workgroup of 8 to 12 waves owns 16 rows per wave x 16 columns, grid (row tiles / waves, ceil(N/16)).  Wave w < 8
 // normalises piece w of the reduction, as k_mimi_lin's does, and leaves it in LDS; then a wave takes the eight pieces one after the other, each from zero, added in
 // rising order: k_mimi_lin's bits.  With 16 rows per workgroup every column was normalised by 96 - 128 of them - 570 vector instructions around 32
-// products per wave: a file's 258 columns 512 -> 1536 15.5 -> 11.5 us, 512 -> 2048 20.1 -> 15.6.  J <= 64.
+// products per wave: a file's 258 columns 512 -> 1536 15.5 -> 11.5 us, 512 -> 2048 20.1 -> 15.6.  J <= 60.
 template <int KJ>
 __global__ __launch_bounds__(768) void k_mimi_lin_rows(MimiLinArgs a) {
     constexpr int U = 8;
