@@ -8,6 +8,8 @@
 #include <math.h>
 #include <stdio.h>
 #include <map>
+#include <mutex>
+#include <set>
 
 namespace {
 
@@ -140,7 +142,7 @@ struct mmi_lm {
                                                     // only lower offsets): picks the step program's variant (attn_variant)
     long xlds_launches = 0;         // launches (or graph nodes captured) that took k_gemm_xlds: mmi_lm_stat(lm, 0)
     bool precapture_failed = false; // capturing the second attention program ahead of time failed once: not tried again for this stream
-    bool dominant_xlds = false;     // the profiled (dominant) GEMM ran on k_gemm_xlds
+    const char* dominant_name = ""; // what the profiled (dominant) linear last ran on
     MmiProgram prog;
     // MMI_DEBUG_TRACE=<prefix> (debug: finding which launch of the step is not reproducible): every step runs its launch list
     // eagerly and, after EVERY op, checksums every allocation of the streaming state; lines "step op site allocation bytes
@@ -329,15 +331,19 @@ int launch_gemm_q(hipStream_t s, dim3 groups, int waves, const GemmArgs& a) {
     return MMI_OK;
 }
 
+// int8 x int8 has no conversion to hold in registers: four entries per register buffer instead of two (MMI_Q8_U=2: the
+// weight-only depth, same-box A/B)
+bool q8_four() {
+    static const bool u4 = !(getenv("MMI_Q8_U") && getenv("MMI_Q8_U")[0] == '2');
+    return u4;
+}
+
 template <int TN, int MT, int NTW>
 int launch_gemm_w(hipStream_t s, dim3 groups, int waves, int u, int wq, const GemmArgs& a) {
     if (wq == 1) return launch_gemm_q<TN, MT, NTW, 1>(s, groups, waves, a);
     if (wq == 2) return launch_gemm_q<TN, MT, NTW, 2>(s, groups, waves, a);
     if (wq == 3) {
-        // int8 x int8 has no conversion to hold in registers: four entries per register buffer instead of two (MMI_Q8_U=2: the
-        // weight-only depth, same-box A/B)
-        static const bool u4 = !(getenv("MMI_Q8_U") && getenv("MMI_Q8_U")[0] == '2');
-        if (u4 && waves == 8) {
+        if (q8_four() && waves == 8) {
             if constexpr (MT * NTW <= 2) {
                 MMI_LAUNCH((k_gemm_xp<TN, MT, NTW, 8, 4, 3>), groups, 512, 0, s, a);
                 MMI_CHECK_LAUNCH();
@@ -481,6 +487,23 @@ hipError_t dominant_begin(mmi_lm* lm, hipStream_t s, EvPair** ev) {
     return hipEventRecord((*ev)->a, s);
 }
 
+// its name with the instantiation (launch_xlds, launch_gemm_w) and what it computes; valid for ever, whoever holds it
+const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XldsPlan& xl, int mt, int wq) {
+    const std::string on = wq == 3 ? ", int8 weights x int8 activations" : (wq == 1 ? ", int8 weights" : (wq == 2 ? ", fp8 weights on the fp8 MFMA" : ""));
+    const auto args = [](std::initializer_list<int> v) {
+        std::string t;
+        for (int x : v) t += (t.empty() ? "<" : ", ") + std::to_string(x);
+        return t;
+    };
+    const int u = wq == 0 ? (p.waves == 8 && p.u == 2 && mt == 1 ? 2 : 4) : (wq == 3 && q8_four() && p.waves == 8 ? 4 : 2);
+    std::string k = xl.on ? "k_gemm_xlds" + args({mt, xl.kc, 3}) + (xl.stagger ? ", true, " : ", false, ") + std::to_string(wq)
+                          : "k_gemm_xp" + args({g.T, mt, 1, p.waves, u}) + (wq ? ", " + std::to_string(wq) : "");
+    static std::mutex names_lock;
+    static std::set<std::string> names;
+    std::lock_guard<std::mutex> hold(names_lock);
+    return names.insert(k + "> (temporal FFN linear_in" + on + " + SiLU gate)").first->c_str();
+}
+
 int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_dominant) {
     a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT;
     a.wscale = g.scale; a.wscb = g.scb; a.gate_rows = g.gate ? g.N : 0;
@@ -491,10 +514,10 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
     a.osplit = plan_osplit(g, p, a.epi, g.T);
     const XldsPlan xl = plan_xlds(lm, g, a, mt);
     EvPair* ev = nullptr;
+    if (is_dominant && lm->profiling) lm->dominant_name = dominant_kernel(g, p, xl, mt, a.wq);
     if (is_dominant) MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
     int rc;
     mmi_record_bytes((long)g.bytes);
-    if (is_dominant) lm->dominant_xlds = xl.on;
     if (xl.on) {
         lm->xlds_launches += 1;
         rc = mt == 1 ? launch_xlds<1>(s, xl, a) : launch_xlds<2>(s, xl, a);
@@ -749,7 +772,10 @@ int launch_norm_one(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, const
     a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT; a.gate_rows = g.gate ? g.N : 0; a.osplit = 1;
     mmi_record_bytes((long)g.bytes);
     EvPair* ev = nullptr;
-    if (is_dominant) MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
+    if (is_dominant) {
+        lm->dominant_name = "k_gemm_norm_one<4> (RMSNorm + temporal FFN linear_in + SiLU gate)";
+        MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
+    }
     MMI_LAUNCH(k_gemm_norm_one<4>, g.NT, 512, 0, s, a);
     MMI_CHECK_LAUNCH();
     if (ev) MMI_HIP_CHECK(hipEventRecord(ev->b, s));
@@ -2101,13 +2127,7 @@ extern "C" int mmi_lm_profile_end(mmi_lm* lm, double* mean_ms, int64_t* n_launch
         const int64_t wbytes = lm->q8 >= 1 ? (int64_t)2 * c.ffn_hidden * c.dim + (int64_t)2 * c.ffn_hidden * 4 : (int64_t)2 * c.ffn_hidden * c.dim * 2;
         *bytes_per_launch = wbytes + (int64_t)lm->batch * c.dim * 2 + (int64_t)lm->batch * c.ffn_hidden * 2;
     }
-    if (kernel_name)
-        *kernel_name = lm->act8      ? "k_gemm_xp<32, MT, 1, 8, 2, 3> (temporal FFN linear_in, int8 weights x int8 activations on v_mfma_i32_32x32x32_i8 + SiLU gate)"
-                       : lm->q8 == 1 ? "k_gemm_xp<32, 1, 1, 8, 2, 1> (temporal FFN linear_in, int8 weights + SiLU gate)"
-                       : lm->q8 == 2 ? "k_gemm_xp<32, 1, 1, 8, 2, 2> (temporal FFN linear_in, fp8 weights on the fp8 MFMA + SiLU gate)"
-                       : lm->dominant_xlds ? (lm->batch > 32 ? "k_gemm_xlds<2, 32, 3, true, 0> (temporal FFN linear_in + SiLU gate)"
-                                                             : "k_gemm_xlds<1, 64, 3, true, 0> (temporal FFN linear_in + SiLU gate)")
-                                     : "k_gemm_xp<32, 1, 1, 8, 2> (temporal FFN linear_in + SiLU gate)";
+    if (kernel_name) *kernel_name = lm->dominant_name;
     lm->ev_used = 0;
     return MMI_OK;
 }

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from moshi_amd.config import tiny_lm_config
+from moshi_amd.lm import LMGen, LMModel
 from moshi_amd.weights import random_lm_state_dict
 from tests import lm_cases
 
@@ -543,3 +544,26 @@ def test_norm_and_linear_in_one_launch(sim_lib, dim, heads):
     st = {}
     lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), dim=dim, num_heads=heads), seed=60 + heads, B=1, S=3, stats=st)
     assert st["launch_sites"].get("L.norm1", 0) == 0 and st["launch_sites"].get("L.in_proj", 0) == 2
+
+
+@pytest.mark.parametrize("B,quantize,switch,kernel", [
+    (1, False, None, "k_gemm_norm_one<4>"), (1, False, "MMI_NO_NORM_FUSION", "k_gemm_xp<16, 1, 1, 4, 4>"), (3, False, None, "k_gemm_xp<16, 1, 1, 4, 4>"),
+    (18, False, None, "k_gemm_xp<32, 1, 1, 4, 4>"), (34, False, None, "k_gemm_xp<32, 2, 1, 4, 4>"), (3, True, None, "k_gemm_xp<16, 1, 1, 4, 2, 3>"),
+])
+def test_profile_names_the_kernel_it_timed(sim_lib, monkeypatch, B, quantize, switch, kernel):
+    """mmi_lm_profile_end's name is that of the launches between its events: the one the launch list has at the same site, at its tile."""
+    import ctypes as C
+    if switch:
+        monkeypatch.setenv(switch, "1")
+    cfg = tiny_lm_config()
+    gen = LMGen(LMModel(random_lm_state_dict(cfg, seed=4), cfg, device="cpu", max_batch=B, lib=sim_lib, quantize=quantize), use_sampling=False)
+    h, us, n, nbytes, name = gen.lm_model._handle, C.c_double(), C.c_int64(), C.c_int64(), C.c_char_p()
+    with gen.streaming(B):
+        gen.step(torch.zeros(B, 8, 1, dtype=torch.long))
+        sim_lib.check(sim_lib.mmi_lm_profile_begin(h))
+        for _ in range(2):
+            gen.step(torch.zeros(B, 8, 1, dtype=torch.long))
+        sim_lib.check(sim_lib.mmi_lm_profile_end(h, C.byref(us), C.byref(n), C.byref(nbytes), C.byref(name)))
+        launched = {k for site, k in gen.launch_list() if site == "L.ffn_in"}
+    assert n.value == 2 * cfg.num_layers
+    assert name.value.decode().startswith(kernel + " (") and launched == {kernel.split("<")[0]}
