@@ -379,22 +379,17 @@ void launch_wide_w(hipStream_t s, const ConvGemmArgs& a, int W, bool group, dim3
     else launch_wide_e<MTB, U, false, false>(s, a, W, grid);
 }
 
-template <int MTB, int U>
-void launch_cols(hipStream_t s, const ConvGemmArgs& a, int pieces, dim3 grid) {
-    if (a.x_packed) MMI_LAUNCH((k_conv_cols<MTB, U, false, true>), grid, 256, 0, s, a, pieces);
-    else if (a.elu_in) MMI_LAUNCH((k_conv_cols<MTB, U, true, false>), grid, 256, 0, s, a, pieces);
-    else MMI_LAUNCH((k_conv_cols<MTB, U, false, false>), grid, 256, 0, s, a, pieces);
-}
-
 int launch_conv_plan(hipStream_t s, const ConvGemmArgs& a, const ConvPlan& p) {
     if (p.cols) {
         const dim3 grid(mmi_cdiv(a.Ntot, 128), mmi_cdiv(a.Mt, p.MTB), p.ksplit);
         ConvGemmArgs w = a;
         if (p.ksplit > 1) w.out_mode = MMI_GOUT_PARTIAL;
         const bool fours = mmi_cdiv(w.q_blk, p.W) % 4 == 0;          // (a group ends with its piece)
-        if (p.MTB == 4) launch_cols<4, 2>(s, w, p.W, grid);
-        else if (p.MTB == 2) fours ? launch_cols<2, 4>(s, w, p.W, grid) : launch_cols<2, 2>(s, w, p.W, grid);
-        else fours ? launch_cols<1, 4>(s, w, p.W, grid) : launch_cols<1, 2>(s, w, p.W, grid);
+        if (p.MTB == 4) MMI_LAUNCH((k_conv_cols<4, 2>), grid, 256, 0, s, w, p.W);
+        else if (p.MTB == 2 && fours) MMI_LAUNCH((k_conv_cols<2, 4>), grid, 256, 0, s, w, p.W);
+        else if (p.MTB == 2) MMI_LAUNCH((k_conv_cols<2, 2>), grid, 256, 0, s, w, p.W);
+        else if (fours) MMI_LAUNCH((k_conv_cols<1, 4>), grid, 256, 0, s, w, p.W);
+        else MMI_LAUNCH((k_conv_cols<1, 2>), grid, 256, 0, s, w, p.W);
         if (p.ksplit > 1) MMI_LAUNCH(k_conv_finish, (int)mmi_cdiv64((int64_t)a.Cout * a.Ntot, 256), 256, 0, s, a, p.ksplit);
         MMI_CHECK_LAUNCH();
         return MMI_OK;
@@ -562,7 +557,7 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         // (128 -> 256, K 10 on 12384 columns with 1, 2, 4 of them: 144, 123, 115 us), except for reductions so short that the stores count (K 32 on
         // 247680: 40 and 52 us).  With fewer tiles the waves of k_conv_wide share a reduction (512 -> 256, K 3 on 2064 columns: 42 against 53 us)
         const long tiles = (long)mmi_cdiv(N, 32) * p->ksplit;
-        p->cols = mem.frames > 1 && tiles * a.Mt >= 700;
+        p->cols = mem.frames > 1 && !a.elu_in && tiles * a.Mt >= 700;
         if (p->cols) {
             p->MTB = a.Q < 8 ? 1 : 4;
             while (p->MTB > 1 && (p->MTB > a.Mt || tiles * mmi_cdiv(a.Mt, p->MTB) < 700)) p->MTB >>= 1;

@@ -388,24 +388,23 @@ __global__ __launch_bounds__(W * 64) void k_conv_wide(ConvGemmArgs a) {
 // k_conv_wide's sums by waves of their own: a wave owns 32 columns x MTB m-tiles and takes the `pieces` of its reduction - what k_conv_wide's waves
 // would split it into - one after the other, each from zero, and adds them up in the same order: the same bits without the exchange through LDS.
 // Four waves of a workgroup own neighbouring column tiles and read the same weights.  grid (ceil(column tiles / 4), ceil(Mt / MTB), ks).
-// PACKED: the operand as its producer packed it (`bp`).  Bound by the matrix core where a wave's reduction is long; what it loses are the gathers
+// Bound by the matrix core where a wave's reduction is long; what it loses are the gathers
 // (one load per value and wave, met by MTB m-tiles).
 // A file's 129 frames: 64 -> 128, K 8 on 61920 columns 151 -> 98 us (83 TFLOP/s), 128 -> 256, K 10 on 12384 144 -> 117, 512 -> 3072 on 2064 103 -> 87,
 // 256 -> 1280 on 12384 143 -> 99, 128 -> 512 on 61920 144 -> 112; stores bound the convs of few products (32 -> 64 on 247680: 59 -> 43).
-template <int MTB, int U, bool ELU_IN, bool PACKED>
+template <int MTB, int U>
 __global__ __launch_bounds__(256, 2) void k_conv_cols(ConvGemmArgs a, int pieces) {
     const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63, jl = lane & 31, kh = lane >> 5;
     const int nt = (int)blockIdx.x * 4 + wave, n = nt * 32 + jl, mt0 = (int)blockIdx.y * MTB;
     if (nt * 32 >= a.Ntot) return;
     const bool nvalid = n < a.Ntot;
     const int nn = nvalid ? n : 0, b = mmi_fast_div(nn, a.T_magic, a.T_shift), t = nn - b * a.T_out;
-    const f32x4* bp = PACKED ? reinterpret_cast<const f32x4*>(a.bp) + (long)nt * a.Q * 64 + lane : nullptr;
     const int q0 = min(a.Q, (int)blockIdx.z * a.q_blk), q1 = min(a.Q, q0 + a.q_blk), qper = max((q1 - q0 + pieces - 1) / pieces, 1);
     const f32x4* wp[MTB];
 #pragma unroll
     for (int m = 0; m < MTB; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.wpk) + (long)min(mt0 + m, a.Mt - 1) * a.Q * 64 + lane;
     ConvWalk in;
-    if constexpr (!PACKED) in.begin(a, b, t, q0, kh);
+    in.begin(a, b, t, q0, kh);
     f32x16 acc[MTB], sum[MTB];
 #pragma unroll
     for (int m = 0; m < MTB; ++m)
@@ -423,12 +422,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_cols(ConvGemmArgs a, int pieces
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int qq = min(at.q + u, q1 - 1);
-            if constexpr (PACKED) bv[u] = bp[(long)qq * 64];
-            else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) bv[u][e] = in.at(a, e);
-                in.advance(a, at.q + u < at.end);
-            }
+            for (int e = 0; e < 4; ++e) bv[u][e] = in.at(a, e);
+            in.advance(a, at.q + u < at.end);
 #pragma unroll
             for (int m = 0; m < MTB; ++m) av[u][m] = wp[m][(long)qq * 64];
         }
@@ -439,7 +435,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_cols(ConvGemmArgs a, int pieces
             const bool on = at.q + u < at.end;               // (quads past the piece's end meet zeros: a branch around them would cost a wait for all loads)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float x = ELU_IN ? mmi_elu(bv[u][e]) : bv[u][e], v = on ? x : 0.f;
+                const float v = on ? bv[u][e] : 0.f;
 #pragma unroll
                 for (int m = 0; m < MTB; ++m) acc[m] = mmi_mfma_f32_32x32x2(av[u][m][e], v, acc[m]);
             }
