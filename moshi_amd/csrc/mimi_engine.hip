@@ -557,10 +557,12 @@ int plan_conv(MimiMem& mem, ConvGemmArgs& a, ConvPlan* p) {
         // (128 -> 256, K 10 on 12384 columns with 1, 2, 4 of them: 144, 123, 115 us), except for reductions so short that the stores count (K 32 on
         // 247680: 40 and 52 us).  With fewer tiles the waves of k_conv_wide share a reduction (512 -> 256, K 3 on 2064 columns: 42 against 53 us)
         const long tiles = (long)mmi_cdiv(N, 32) * p->ksplit;
-        p->cols = mem.frames > 1 && !a.elu_in && tiles * a.Mt >= 700;
+        long enough = 700;
+        if (const char* e = getenv("MMI_CONV_COLS")) enough = atol(e);         // test hook: the tiny shapes
+        p->cols = mem.frames > 1 && !a.elu_in && tiles * a.Mt >= enough;
         if (p->cols) {
             p->MTB = a.Q < 8 ? 1 : 4;
-            while (p->MTB > 1 && (p->MTB > a.Mt || tiles * mmi_cdiv(a.Mt, p->MTB) < 700)) p->MTB >>= 1;
+            while (p->MTB > 1 && (p->MTB > a.Mt || tiles * mmi_cdiv(a.Mt, p->MTB) < enough)) p->MTB >>= 1;
         }
         return MMI_OK;
     }

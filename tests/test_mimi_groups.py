@@ -337,3 +337,24 @@ def test_norms_and_linears_of_many_columns(sim_lib, heads, ff):
         whole = m.decode(codes)
     with m.streaming(1):
         assert torch.equal(whole, torch.cat([m.decode(codes[..., f:f + 1]) for f in range(57)], -1))
+
+
+@pytest.mark.parametrize("enough,ks,filters,B,frames", [(1, 1, 10, 1, 23), (1, 8, 10, 1, 29), (1, 1, 14, 1, 23), (1, 3, 22, 1, 23), (60, 3, 12, 2, 13)])
+def test_convs_of_many_columns(sim_lib, monkeypatch, enough, ks, filters, B, frames):
+    """k_conv_cols (one, two and four m-tiles per wave, groups of two and of four quads) against the frame program's bits: column tiles that are cut
+    (552 columns, 696, 1104), workgroups with waves past the last one, channels that are no multiple of 32 and m-tiles that are none of a
+    wave's, reductions in pieces that are empty, shorter than a group and of an odd length, sums split over 3 and 8 workgroups, two streams."""
+    monkeypatch.setenv("MMI_CONV_COLS", str(enough))
+    monkeypatch.setenv("MMI_CONV_KSPLIT", str(ks))
+    monkeypatch.setenv("MMI_DEBUG_POISON", "1")
+    cfg = replace(tiny_mimi_config(), n_filters=filters)
+    sd, fs = random_mimi_state_dict(cfg, seed=6, device="cpu"), cfg.frame_size
+    m = MimiModel(sd, cfg, device="cpu", max_batch=B, num_codebooks=3, lib=sim_lib)
+    x = 0.3 * torch.randn(B, 1, fs * frames, generator=torch.Generator().manual_seed(filters))
+    with m.streaming(B):
+        codes = m.encode(x)
+        pcm = m.decode(codes)
+        assert all("k_conv_cols" in {k for _, k in m.launch_list(which)} for which in ("encode_group", "decode_group"))
+    with m.streaming(B):
+        assert torch.equal(codes, torch.cat([m.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(frames)], -1))
+        assert torch.equal(pcm, torch.cat([m.decode(codes[..., f:f + 1].contiguous()) for f in range(frames)], -1))
