@@ -358,3 +358,18 @@ def test_convs_of_many_columns(sim_lib, monkeypatch, enough, ks, filters, B, fra
     with m.streaming(B):
         assert torch.equal(codes, torch.cat([m.encode(x[..., f * fs:(f + 1) * fs].contiguous()) for f in range(frames)], -1))
         assert torch.equal(pcm, torch.cat([m.decode(codes[..., f:f + 1].contiguous()) for f in range(frames)], -1))
+
+
+@pytest.mark.parametrize("heads,frames,rows", [(60, 57, True), (61, 57, False), (61, 10, False), (64, 65, False)])
+def test_widths_whose_columns_fit_the_group_memory(sim_lib, heads, frames, rows):
+    """k_mimi_lin_rows keeps the normalised columns in 64 KB of LDS, 1 KB for every 16 channels beside 1 KB of its own: widths of up to 960 take it,
+    wider ones k_mimi_lin - two row tiles to a norm (20 columns), two column tiles (114, 130), 32 x 32 tiles (130 columns) - with the frames' bits."""
+    cfg = replace(tiny_mimi_config(), dimension=16 * heads, tr_d_model=16 * heads, tr_num_heads=heads, tr_dim_feedforward=2048, tr_num_layers=1, n_filters=1, compress=1)
+    m = MimiModel(random_mimi_state_dict(cfg, seed=9), cfg, device="cpu", max_batch=1, num_codebooks=2, lib=sim_lib)
+    codes = torch.randint(0, cfg.q_bins, (1, 2, frames), generator=torch.Generator().manual_seed(3))
+    with m.streaming(1):
+        whole = m.decode(codes)
+        kernels = {k for _, k in m.launch_list("decode_group")}
+    assert "k_mimi_lin" in kernels and ("k_mimi_lin_rows" in kernels) == rows
+    with m.streaming(1):
+        assert torch.equal(whole[..., :4 * cfg.frame_size], torch.cat([m.decode(codes[..., f:f + 1]) for f in range(4)], -1))
