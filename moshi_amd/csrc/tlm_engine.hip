@@ -17,6 +17,7 @@
 #include "tlm_linear.h"
 
 #include <math.h>
+#include <stdio.h>
 #include <algorithm>
 #include <array>
 #include <map>
@@ -152,6 +153,7 @@ struct mmi_tlm {
     hipStream_t cap_stream = nullptr;
     std::map<std::tuple<int, int, int>, std::unique_ptr<MmiProgram>> progs;
     std::vector<std::string> last_log;
+    bool say_forms = false;        // test hook (MMI_TLM_FORMS): a line on stderr for every launch of the tiled kernel
     long weight_bytes = 0;
 };
 
@@ -824,16 +826,17 @@ int split_for(const Plan& p, const Mat& w, int blocks) {
     else while (s < TILE_SPLIT && blocks * s < TILE_BLOCKS && w.KS / (2 * s) >= 16) s *= 2;
     return s;
 }
-// blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64)
+// blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64, at fp32 64 x 32)
 int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, p.fm == 4 ? 8 : 4) * (j.list ? j.rblocks : j.groups * mmi_cdiv(j.rows, plan_tile(p))); }
 int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
 
 int rows_ntw(const Plan& p) { return p.mt; }                // n-tiles per workgroup of the weight-streaming kernel
 template <class Tr, int FN, int FM, int ST, int OCC, int WN = 2, int WM = 2, int KK = 1>
-int launch_tile(hipStream_t s, const TlmJobs& J) {
+int launch_tile(hipStream_t s, const TlmJobs& J, bool say) {
     constexpr size_t smem = TlmTile<Tr, FN, FM, WN, WM, ST, KK>::smem();
     int grid = 0;                                          // every XCD's share of every job, rounded up
     for (int i = 0; i < J.n; ++i) grid += 8 * mmi_cdiv(J.j[i].blocks, 8);
+    if (say) fprintf(stderr, "tile %dx%d stages %d of %d, %d workgroups\n", 16 * FN * WN, 16 * FM * WM, ST, KK, grid);
     static_assert(smem * OCC <= 160 * 1024, "LDS of a CU");
     if (smem > 64 * 1024) {
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_tile<Tr, FN, FM, WN, WM, ST, OCC, KK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -844,7 +847,7 @@ int launch_tile(hipStream_t s, const TlmJobs& J) {
     return MMI_OK;
 }
 template <class Tr>
-int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J) {
+int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J, bool say) {
     auto cut = [&](int ntw) {                               // n-tiles per block -> blocks of every job, and their number
         int total = 0;
         for (int i = 0; i < J.n; ++i) {
@@ -869,32 +872,40 @@ int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J) {
     if (p.fm == 4) {
         if constexpr (Tr::V == 8) {
             const int wide = cut(16);
-            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, J);
+            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, J, say);
         }
         const int grid = cut(8);
-        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J) : launch_tile<Tr, 4, 4, 3, 3>(s, J);
+        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J, say) : launch_tile<Tr, 4, 4, 3, 3>(s, J, say);
     }
     // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
     if constexpr (Tr::V == 8) {
-        if (cut(8) >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, J);
-        // 64 x 64 with stages of two k-steps while two blocks per CU are all there is, or the blocks are long (a meeting of the waves per k-step was
-        // what a step of 8 products took: 676 x 2048 x (2048 + 5632), 640 blocks: 40.7 -> 35.9 us; 300 rows of Bibapel 4096 2713 -> 2618 us); one k-step
-        // each, four blocks per CU, where more of them are short or expert blocks of a few rows (100 rows of Kesirax 2048: 833 against 989 us)
-        bool long_dense = true;
-        for (int i = 0; i < J.n; ++i) long_dense = long_dense && !J.j[i].list;
-        int steps = 0;
-        for (int i = 0; i < J.n; ++i) steps = std::max(steps, mmi_cdiv(J.j[i].KS, J.j[i].ksplit));
-        if (cut(4) <= 512 || (long_dense && steps >= 64)) return launch_tile<Tr, 2, 2, 4, 2, 2, 2, 2>(s, J);
-        return launch_tile<Tr, 2, 2, 4, 4>(s, J);
+        if (cut(8) >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, J, say);
+        // 64 x 64 with stages of two k-steps, two blocks per CU, while those are all there is or a second round of them is short ones in the shadow of the
+        // first: 512 blocks of 176 and 64 k-steps 54 -> 39 us, 640 of them 56 -> 45, 768 of 352 and 128 113 -> 106 (896: 118 and 117).  Otherwise one
+        // k-step each, four blocks per CU: 576 blocks of 256 k-steps 84 us against 103, 896 of 64 36 against 38, 640 of 16 12 against 16; expert blocks,
+        // of a few rows or none, likewise (100 rows of Kesirax 2048: 833 against 989 us)
+        const int total = cut(4);
+        bool listed = false;
+        long longest = 0, work = 0, heavy = 0;               // k-steps of a block and of all of them; blocks of more than half the longest
+        auto ksteps = [](const TlmJob& j) { return (long)mmi_cdiv(j.KS, j.ksplit); };
+        for (int i = 0; i < J.n; ++i) longest = std::max(longest, ksteps(J.j[i]));
+        for (int i = 0; i < J.n; ++i) {
+            const TlmJob& j = J.j[i];
+            listed = listed || j.list;
+            work += j.blocks * ksteps(j);
+            if (2 * ksteps(j) > longest) heavy += j.blocks;
+        }
+        if (total <= 512 || (!listed && heavy <= 512 && 16 * work <= 17 * 512 * longest)) return launch_tile<Tr, 2, 2, 4, 2, 2, 2, 2>(s, J, say);
+        return launch_tile<Tr, 2, 2, 4, 4>(s, J, say);
     } else {
         // at fp32 the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
         // 32 rows and two k-steps per stage (plan_rows); more stages while all blocks fit the chip with them (three per CU, expert blocks without rows aside; Kesirax 1024, 194 rows: 911 and
         // 865 us; 320 rows, with more blocks: 1030 and 1045)
-        return cut(4) <= 1024 ? launch_tile<Tr, 1, 2, 4, 3, 4, 1, 2>(s, J) : launch_tile<Tr, 1, 2, 3, 4, 4, 1, 2>(s, J);
+        return cut(4) <= 1024 ? launch_tile<Tr, 1, 2, 4, 3, 4, 1, 2>(s, J, say) : launch_tile<Tr, 1, 2, 3, 4, 4, 1, 2>(s, J, say);
     }
 }
 int launch_jobs(mmi_tlm* m, hipStream_t s, const Plan& p, TlmJobs J) {
-    return m->f32 ? launch_jobs_t<TlmF32>(s, p, J) : launch_jobs_t<TlmBf16>(s, p, J);
+    return m->f32 ? launch_jobs_t<TlmF32>(s, p, J, m->say_forms) : launch_jobs_t<TlmBf16>(s, p, J, m->say_forms);
 }
 
 // the instantiation for a layer's latent blocks and rotated k-steps
@@ -1741,6 +1752,7 @@ int create_impl(mmi_tlm* m, const mmi_tensor_desc* weights, int n_weights) {
     for (int i = m->max_pages - 1; i >= 0; --i) m->free_pages.push_back(i);
     if ((rc = alloc_state(m)) || (rc = alloc_buffers(m))) return rc;
     m->graphs = mmi_graphs_enabled();
+    m->say_forms = getenv("MMI_TLM_FORMS") != nullptr;
     if (m->graphs) MMI_HIP_CHECK(hipStreamCreateWithFlags(&m->cap_stream, hipStreamNonBlocking));
     MMI_HIP_CHECK(hipDeviceSynchronize());
     return MMI_OK;

@@ -1,6 +1,7 @@
-"""Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 32, 64 x 64, 128 x 64, 128 x 128 in three and four stages, 256 x 128, whole
-and split reductions, gathered and listed expert rows - at row counts just past a tile and sizes that are no multiples of one: a prompt fed at
-once must give the logits that the same prompt gives in portions of at most 64 tokens, which take the weight-streaming kernel."""
+"""Every block form of the tiled product kernel (k_tlm_gemm_tile) - 64 x 32 in three and four stages, 64 x 64 in stages of one and of two k-steps,
+128 x 64, 128 x 128 in three and four stages, 256 x 128, whole and split reductions, gathered and listed expert rows - at row counts just past a
+tile and sizes that are no multiples of one: a prompt fed at once must give the logits that the same prompt gives in portions of at most 64
+tokens, which take the weight-streaming kernel.  Each case says which forms its launches must have."""
 from dataclasses import replace
 
 import pytest
@@ -23,22 +24,34 @@ def dense_model(width, ff):
     return TokenLMConfig("Bibapel", vocab=331, width=width, layers=[TokenLayerConfig(att, DenseGLUConfig(ff=ff, limit=7.0))], norms=2, layer_scales=False, tied_head=True)
 
 
+# form: features x rows of a block, stages in its ring, k-steps per stage
+SMALL32, SMALL16 = {"64x32 stages 4 of 2"}, {"64x64 stages 4 of 2"}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("model,T", [
-    (experts_model(208, 144), 65), (experts_model(528, 400), 130),                    # 64 x 64 in stages of two k-steps, the last one half empty; fp32: 64 x 32
-    (dense_model(2080, 3800), 200),                                                   # ... more blocks than the chip holds at once
-    (dense_model(1040, 4000), 577), (dense_model(1040, 1200), 641),                   # 128 x 64; 128 x 128 in four stages
-    (experts_model(1040, 2064), 1025), (dense_model(1040, 6000), 1157)                # 128 x 128 in three, 256 x 128
-], ids=["65", "130", "200", "577", "641", "1025", "1157"])
-def test_prompt_at_once_equals_portions(model, T, dtype):
+@pytest.mark.parametrize("model,T,fp32,bf16", [
+    (experts_model(208, 144), 65, SMALL32, SMALL16), (experts_model(528, 400), 130, SMALL32, SMALL16),        # (a reduction's last stage half empty)
+    (dense_model(2080, 3800), 200, SMALL32, {"64x64 stages 4 of 1", "64x64 stages 4 of 2"}),                  # 524 equal blocks; 264 long beside 132 short
+    (experts_model(2080, 3800), 100, {"64x32 stages 3 of 2", "64x32 stages 4 of 2"}, {"64x64 stages 4 of 1", "64x64 stages 4 of 2"}),
+    (dense_model(2080, 3800), 460, {"64x32 stages 3 of 2", "64x32 stages 4 of 2"}, {"128x64 stages 4 of 1", "64x64 stages 4 of 2"}),   # 264 long beside 264 short
+    (dense_model(1040, 4000), 577, {"64x32 stages 3 of 2", "64x32 stages 4 of 2"}, {"128x64 stages 4 of 1", "64x64 stages 4 of 2"}),
+    (dense_model(1040, 1200), 641, {"128x128 stages 4 of 1"}, {"128x128 stages 4 of 1"}),
+    (experts_model(1040, 2064), 1025, {"128x128 stages 3 of 1", "128x128 stages 4 of 1"}, {"128x128 stages 3 of 1", "128x128 stages 4 of 1"}),
+    (dense_model(1040, 6000), 1157, {"128x128 stages 3 of 1"}, {"256x128 stages 3 of 1", "128x128 stages 4 of 1"}),
+], ids=["65", "130", "200", "100", "460", "577", "641", "1025", "1157"])
+def test_prompt_at_once_equals_portions(model, T, fp32, bf16, dtype, monkeypatch, capfd):
+    monkeypatch.setenv("MMI_TLM_FORMS", "1")
     sd = random_token_lm_state_dict(model, seed=T, device="cuda")
     lm = TokenLM(sd, model, dtype=dtype, max_slots=2, max_tokens=4096, max_step_tokens=T)
     prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
     want = sorted({0, 15, 16, 63, 64, T // 2, T - 2, T - 1})
     a = lm.open()
+    capfd.readouterr()
     whole = lm.step([(a, prompt, want)])
     assert "k_tlm_gemm_tile" in {k for _, k, _ in lm.launch_list()}
+    forms = {line[5:line.index(",")] for line in capfd.readouterr().err.splitlines() if line.startswith("tile ")}
+    assert forms == (fp32 if dtype == torch.float32 else bf16)
     b = lm.open()
     parts = torch.cat([lm.step([(b, prompt[i:i + 64], [w - i for w in want if i <= w < i + 64])]) for i in range(0, T, 64)])
     rel = float((whole - parts).double().norm() / parts.double().norm())
