@@ -2,7 +2,7 @@
 // kernel simulator use (OCP e4m3fn, round-to-nearest-even, clamp to +-448):
 //   1. v_cvt_pk_fp8_f32 on EVERY finite bf16 value (after the kernels' med3 clamp) and on exact ties
 //   2. v_mfma_f32_32x32x16_fp8_fp8 / v_mfma_f32_16x16x32_fp8_fp8 on random fp8 codes incl. subnormals: exact products, fp32 sums
-// Build + run on the GPU box:  hipcc --offload-arch=gfx950 -O2 -I moshi_amd/csrc scripts/fp8_probe.hip -o /tmp/fp8_probe && /tmp/fp8_probe
+// Build + run:  hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O2 -I moshi_amd/csrc scripts/fp8_probe.hip -o /tmp/fp8_probe && /tmp/fp8_probe
 #include "mmi_device.h"
 #include <cstdio>
 #include <cmath>

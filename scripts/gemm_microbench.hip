@@ -3,7 +3,7 @@
 // achieved weight-streaming rate.  Weights cycle through enough distinct buffers (> 1 GiB) that the 256 MiB
 // Infinity Cache cannot serve them.  Measurement tool only - the product picks its plan in lm_engine.hip:plan_gemm.
 //
-//   hipcc --offload-arch=gfx950 -O3 -std=c++17 -ffp-contract=off -Imoshi_amd/csrc scripts/gemm_microbench.hip \
+//   hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 -std=c++17 -ffp-contract=off -Imoshi_amd/csrc scripts/gemm_microbench.hip \
 //         moshi_amd/csrc/api_common.hip -o gpurun_out/gemm_microbench && gpurun_out/gemm_microbench [B]
 #include "lm_kernels.h"
 

@@ -2,7 +2,7 @@
 // dispatch's acquire invalidates it), so code that a wave executes once is fetched line by line from L2.  Kernels of NI
 // independent fp32 FMAs (8 accumulators round-robin: no dependent-issue stall) as straight-line code vs the same dynamic count
 // as a loop over a 64-instruction body, 1 / 2 / 4 waves per SIMD, in a dependent hipGraph chain.  Measurement tool only.
-//   hipcc --offload-arch=gfx950 -O3 scripts/icache_probe.hip -o build/icache_probe
+//   hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 scripts/icache_probe.hip -o build/icache_probe
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

@@ -1,7 +1,7 @@
 // Where does the sampler's time go?  k_sample (lm_kernels.h) on random bf16 logits of the two real vocabulary sizes, 32 sessions,
 // as a dependent chain in one stream: greedy (argmax only), the production path (top-k + counter RNG) and the supplied-noise path
 // (softmax, ordered compaction, rank), with and without the next micro-step's input row.  Measurement tool only.
-//   hipcc --offload-arch=gfx950 -O3 -std=c++17 -ffp-contract=off -Imoshi_amd/csrc scripts/sample_microbench.hip moshi_amd/csrc/api_common.hip -o build/sample_microbench
+//   hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 -std=c++17 -ffp-contract=off -Imoshi_amd/csrc scripts/sample_microbench.hip moshi_amd/csrc/api_common.hip -o build/sample_microbench
 #include <hip/hip_runtime.h>
 __device__ long long g_stamps[16];
 // stage stamps of workgroup 0 / thread 0 (shader clock), read back after the run
