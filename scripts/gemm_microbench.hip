@@ -70,7 +70,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_probe_xcost(const u32x4* __restr
 }
 
 
-// ---- prototype: activations resident in LDS (DESIGN.md 9e) ----------------------------------------------------------------------
+// ---- prototype: activations resident in LDS ----------------------------------------------------------------------
 // One workgroup per CU walks a contiguous range of n-tiles.  K is cut into chunks of KC k-steps whose activation fragments
 // (MT x KC KiB = 64 KiB) are staged in LDS, double-buffered: every activation byte leaves the L2 ONCE per workgroup instead
 // of once per n-tile.  The 8 waves split each chunk's k-steps; per (chunk, tile) segment a wave streams its KPW weight

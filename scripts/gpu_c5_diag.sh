@@ -1,4 +1,4 @@
-# VERDICT r4 item 1, on one box (gpurun -- 'bash scripts/gpu_c5_diag.sh'):
+# Is the int8 model at 64 sessions reproducible, on one box:
 #  (a) the C5 file (per-linear bit equality + the network gates), as pytest runs it;
 #  (b) the 64-session int8 network case in FRESH processes, graph and eager: is the engine's output the same bits every time?
 #  (c) the same case with the oracle's BLAS on 1 thread and on all: does the checker move?

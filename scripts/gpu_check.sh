@@ -1,12 +1,12 @@
-# The round's GPU check on one MI355X box (gpurun -- 'bash scripts/gpu_check.sh'): smoke, every -m gpu test, the default benchmark
-# line as the driver runs it (with its extras and its CPU-baseline leg), and the other named configurations (BASELINE.json
+# The GPU check on one MI355X: smoke, every -m gpu test, the default benchmark
+# line (with its extras and its CPU-baseline leg), and the other named configurations (
 # configs 1, 2, 4) as logged lines.
 cd $GRAFT_REPO_ROOT
 mkdir -p gpurun_out
 O=$GRAFT_REPO_ROOT/gpurun_out
 python scripts/isa_scan_packed_swizzle.py moshi_amd/libmoshi_mi.so | tail -1
 timeout 300 python -c "import __graft_entry__ as g; g.smoke()" > $O/smoke.log 2>&1; echo "smoke rc=$?"
-# exactly as the driver runs it (-x: the first failure stops the run), plus the slowest tests for the suite's time budget (600 s)
+# (-x: the first failure stops the run), plus the slowest tests for the suite's time budget (600 s)
 timeout 1500 python -m pytest tests -x -q -m gpu --durations=12 > $O/pytest_gpu.log 2>&1; echo "pytest rc=$?"; tail -18 $O/pytest_gpu.log | cut -c1-200
 ( time timeout 900 python bench.py --steps 20 --warmup 5 ) > $O/bench_default.log 2>&1; grep '"metric"' $O/bench_default.log | cut -c1-400
 timeout 300 python bench.py --no-cpu-baseline --no-extras --serial > $O/bench_default_serial.log 2>&1

@@ -3,7 +3,7 @@ mkdir -p gpurun_out
 export TMPDIR=/tmp
 O=$GRAFT_REPO_ROOT/gpurun_out
 # HBM traffic of the dominant kernel INSIDE the step (the product library, eager launches so that every dispatch is a packet the
-# counters can be attributed to).  rocprofv3 --pmc crashed inside the profiler when attached to the Python process in rounds 1-2
+# counters can be attributed to).  rocprofv3 --pmc crashed inside the profiler when attached to the Python process
 # (profiles/r01_logs); tried again each round, bounded, and the standalone-launcher figure stays the committed one if it still does.
 for ctr in FETCH_SIZE WRITE_SIZE; do
   cd /tmp && MMI_NO_GRAPH=1 timeout 150 rocprofv3 --pmc $ctr --kernel-trace -d /tmp/prof_pmc_$ctr -o pmc -- python $GRAFT_REPO_ROOT/bench.py --no-cpu-baseline --workload lm --steps 2 --warmup 1 > $O/rocprof_pmc_$ctr.log 2>&1; rc=$?; echo "pmc $ctr rc=$rc"

@@ -1,5 +1,5 @@
 # L2 request counters over the bf16 LM step at 64 and at 32 sessions (eager launches, product library): what the second batch tile costs
-# k_gemm_xlds in L2 requests.  gpurun -- 'bash scripts/gpu_pmc_b64.sh'
+# k_gemm_xlds in L2 requests.
 cd $GRAFT_REPO_ROOT; mkdir -p gpurun_out; export TMPDIR=/tmp; O=$GRAFT_REPO_ROOT/gpurun_out
 TCC="TCC_REQ_sum TCC_MISS_sum TCC_HIT_sum"
 for B in 64 32; do

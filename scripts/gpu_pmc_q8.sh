@@ -1,5 +1,5 @@
 # Counter passes over the LM step at C5's shape (64 sessions, int8 linears) on the product library, eager launches: what binds the
-# int8 GEMMs on k_gemm_xp (default) and on k_gemm_xlds (MMI_GEMM_LDS=1).  gpurun -- 'bash scripts/gpu_pmc_q8.sh'
+# int8 GEMMs on k_gemm_xp (default) and on k_gemm_xlds (MMI_GEMM_LDS=1).
 cd $GRAFT_REPO_ROOT; mkdir -p gpurun_out; export TMPDIR=/tmp; O=$GRAFT_REPO_ROOT/gpurun_out
 SQ="SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_WAIT_INST_ANY SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_ACTIVE_INST_ANY"
 TCC="TCC_REQ_sum TCC_MISS_sum TCC_HIT_sum"

@@ -1,5 +1,5 @@
 # Counter passes over the LM step on the product library, eager launches (every dispatch is a packet the counters can be
-# attributed to).  gpurun -- 'bash scripts/gpu_pmc_step.sh'.  VERDICT r4 items 3 and 7:
+# attributed to).
 #  * 32 sessions, bf16, mid-run ring depth: FETCH_SIZE / WRITE_SIZE / TCC for the dominant GEMM (k_gemm_xlds) AND the decode attention
 #    (k_lm_attn_wave), so that roofline.traffic is a figure of THIS round and the attention's clamped re-reads are counted;
 #  * the same FETCH_SIZE pass with every ring 3000 deep (--kv-depth full);

@@ -1,4 +1,4 @@
-# rocprofv3 evidence for profiles/ (gpurun -- 'bash scripts/gpu_profile.sh'): kernel stats + per-site table of the default
+# rocprofv3 evidence for profiles/: kernel stats + per-site table of the default
 # benchmark command in its SERIAL schedule (the tracer serialises the LM's queue against the codec's, so the pipelined overlap
 # cannot be seen in a kernel trace - the pipeline's own timeline is in the bench line and scripts/duplex_timeline.py), the queue
 # view of the pipelined run.

@@ -1,5 +1,5 @@
-# SQ counter passes over the codec's kernels at 32 streams (round 6): how busy the matrix core is in the fp32 convolutions and how long
-# their waves wait ("12 % of the fp32 MFMA peak").  Three counters per pass.  gpurun -- 'bash scripts/gpu_sq_mimi.sh'
+# SQ counter passes over the codec's kernels at 32 streams: how busy the matrix core is in the fp32 convolutions and how long
+# their waves wait (12 % of the fp32 MFMA peak).  Three counters per pass.
 cd $GRAFT_REPO_ROOT; mkdir -p gpurun_out; export TMPDIR=/tmp; O=$GRAFT_REPO_ROOT/gpurun_out
 HDR="MMI_NO_GRAPH=1 python bench.py --no-cpu-baseline --no-extras --workload mimi --steps 6 --warmup 2 --batch 32"
 i=0

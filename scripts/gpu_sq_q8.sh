@@ -1,5 +1,5 @@
-# SQ counter passes over the int8 x int8 temporal GEMMs at C5's shape, three counters per pass (a pass with
-# seven did not finish in 200 s in this round's first attempt).  gpurun -- 'bash scripts/gpu_sq_q8.sh'
+# SQ counter passes over the int8 x int8 temporal GEMMs at 64 sessions, three counters per pass (a pass with
+# seven did not finish in 200 s at first).
 cd $GRAFT_REPO_ROOT; mkdir -p gpurun_out; export TMPDIR=/tmp; O=$GRAFT_REPO_ROOT/gpurun_out
 HDR="MMI_NO_GRAPH=1 python bench.py --no-cpu-baseline --no-extras --workload lm --steps 2 --warmup 1 --batch 64"
 i=0

@@ -1,6 +1,6 @@
 """Scan the gfx950 code objects of a built library for packed-fp32 VALU instructions (v_pk_mul_f32 / v_pk_add_f32 / v_pk_fma_f32)
 that CROSS-swizzle their halves (`op_sel:[..]`) while writing one of their own source pairs in place - the instruction form that
-stood in k_gemm_xp's RoPE epilogue when its output was not reproducible (DESIGN.md 10a).
+stood in k_gemm_xp's RoPE epilogue when its output was not reproducible.
 
     python scripts/isa_scan_packed_swizzle.py [lib.so]
 

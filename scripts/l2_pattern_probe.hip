@@ -1,13 +1,13 @@
 // What does the L2 deliver to the access pattern of the temporal GEMMs' ACTIVATION operand?  In k_gemm_xlds / k_gemm_xp every
 // workgroup re-reads the whole packed activation matrix (256 KB at 32 sessions, 512 KB at 64) from its XCD's L2, all 256
 // workgroups walking the SAME addresses in the SAME order; under the TCC counters these kernels run at 7.4-9.8 TB/s of L2 requests
-// (HISTORY.md round 4 10e), while MI355X_MICROARCH.md puts the L2 at ~34.5 TB/s.  This probe separates the candidate
+// while the L2 is quoted at ~34.5 TB/s.  This probe separates the candidate
 // explanations with 16-byte-per-lane loads (one 1 KiB line group per wave instruction, as the GEMMs issue them):
 //   same      every workgroup reads the same buffer, chunk order identical in all workgroups (the GEMMs' pattern)
 //   rotated   same buffer, every workgroup starts at its own offset (requests of one instant spread over the L2 channels)
 //   distinct  every workgroup reads its own buffer of the same size (no two workgroups ever want the same line)
 // for footprints of 64 / 256 / 512 KiB per workgroup.  Bounded loops only, no inter-workgroup communication; runs in < 1 s.
-// Measurement tool for DESIGN.md; not part of the product.
+// Measurement tool; not part of the product.
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

@@ -1,6 +1,6 @@
 // How much does one dependent kernel in a hipGraph chain cost on MI355X, as a function of what the kernel does?
 // (empty / load-modify-store of the predecessor's output / + a block barrier / + a second dependent load).
-// Measurement tool for DESIGN.md's launch-count arithmetic; not part of the product.
+// Measurement tool for launch-count arithmetic; not part of the product.
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

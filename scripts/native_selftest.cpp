@@ -1,4 +1,4 @@
-// A Python-free self-test of an installed libmoshi_mi.so on a GPU box: a tiny Mimi and a tiny Moshi LM are built through the C ABI
+// A Python-free self-test of an installed libmoshi_mi.so on a GPU: a tiny Mimi and a tiny Moshi LM are built through the C ABI
 // (include/moshi_mi.h) from weights this program generates itself (an integer hash, the same one
 // tests/golden/make_native_selftest.py uses), run for a few frames, and compared with what the numpy oracle computed for them
 // (tests/golden/native_selftest/expected.bin): RVQ codes and teacher-forced token-ring outputs bit-exact, PCM within 2e-5, logits

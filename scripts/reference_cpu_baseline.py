@@ -1,6 +1,6 @@
 """The REFERENCE's own PyTorch CPU path (kyutai-labs/moshi, imported read-only from /root/reference) timed on THIS host: the
 recipe of scripts/moshi_benchmark.py:76-100 (zeros / noise chunk -> mimi.encode -> lm_gen.step -> mimi.decode per 80 ms
-frame), BASELINE.md section 3.  The reference cannot travel to the GPU box (no copy of its sources is kept in this repository),
+frame).  The reference is not part of a checkout (no copy of its sources is kept in this repository),
 so bench.py's `cpu_baseline` times the numpy port there and quotes this file's output beside it (profiles/r03_logs/
 reference_cpu_baseline.json; labelled with the host it was measured on).
 
@@ -35,7 +35,7 @@ def main():
     import re
     m = re.search(r"model name\s*:\s*(.*)", open("/proc/cpuinfo").read())
     out = {"host": {"cpu": m.group(1).strip() if m else platform.processor(), "cores": threads, "torch": torch.__version__,
-                    "where": "the build container (not the GPU box)"},
+                    "where": "a host without a GPU"},
            "recipe": "scripts/moshi_benchmark.py:76-100 on device='cpu', NO_TORCH_COMPILE=1, random-init weights, 0.1*N(0,1) PCM"}
     torch.manual_seed(1234)
     mimi = loaders.get_mimi(None, None, "cpu", num_codebooks=8)

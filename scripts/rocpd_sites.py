@@ -24,7 +24,7 @@ HBM_PEAK_GBS = 8000.0
 
 
 def site_bytes_7b():
-    """Packed weight bytes one launch of each weight-streaming site reads (Moshi-7B, bf16): SURVEY.md 8(a) shapes."""
+    """Packed weight bytes one launch of each weight-streaming site reads (Moshi-7B, bf16)."""
     d, h, dd, dh, V, card, q = 4096, 11264, 1024, 2816, 32000, 2048, 8
     return {
         "L.in_proj": 2 * 3 * d * d, "L.out_proj": 2 * d * d, "L.ffn_in": 2 * 2 * h * d, "L.ffn_out": 2 * d * h,
