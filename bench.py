@@ -22,7 +22,7 @@ import torch
 ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
-HBM_PEAK_GBS = 8000.0  # MI355X HBM3E spec peak (MI355X_MICROARCH.md)
+HBM_PEAK_GBS = 8000.0  # MI355X HBM3E spec peak
 
 
 def trace(msg):
@@ -39,11 +39,11 @@ def parse():
     ap.add_argument("--workload", default="auto", choices=["auto", "duplex", "mimi", "lm", "served", "launchcheck", "tlm"],
                     help="tlm: token language models (bench_tlm.py, one GPU); served: the duplex step driven through the session batcher with HOST PCM in / PCM + tokens out "
                          "(pinned staging, H2D + D2H and one synchronisation per step included): the PCIe-inclusive rate")
-    ap.add_argument("--batch", type=int, default=32, help="sessions per GPU (BASELINE.json configs[3]: 32)")
+    ap.add_argument("--batch", type=int, default=32, help="sessions per GPU")
     ap.add_argument("--no-cpu-baseline", action="store_true")
-    ap.add_argument("--stagger", type=int, default=8, help="frames between session starts (SURVEY.md 8d C4)")
+    ap.add_argument("--stagger", type=int, default=8, help="frames between session starts")
     ap.add_argument("--quant", default="none", choices=["none", "q8", "fp8"],
-                    help="BASELINE configs[4] weight formats: q8 = row-wise int8 linears x row-wise int8 activations on the int8 MFMA (the reference's "
+                    help="weight formats: q8 = row-wise int8 linears x row-wise int8 activations on the int8 MFMA (the reference's "
                          "bitsandbytes rule; MMI_Q8_ACT=bf16 in the environment: weight-only, widened to bf16 in registers); fp8 = e4m3 linears on the fp8 MFMA")
     ap.add_argument("--kv", default="bf16", choices=["bf16", "fp8"], help="KV ring of the temporal transformer: the reference's bf16, or e4m3 (half the attention stream)")
     ap.add_argument("--launch-lists", default="", help="directory to write the step's launch lists (site per kernel launch) into, for scripts/rocpd_sites.py")
@@ -53,8 +53,8 @@ def parse():
     ap.add_argument("--lm-layers", type=int, default=0, help="debug: override the number of temporal layers (invalidates the result)")
     ap.add_argument("--kv-depth", default="mid", choices=["mid", "start", "full"],
                     help="mid (default): before the warm-up every session is moved (mmi_lm_seek) to the MIDPOINT of the configuration's run "
-                         "(SURVEY.md 8d: C4 = 500 steps, sessions 8 frames apart -> ring depth 250 + 8 b; C3 = 300 steps -> depth 150), so "
-                         "the measured step does not depend on --steps; start: sessions start at depth 8 b (rounds 1-3); "
+                         "(500 steps, sessions 8 frames apart -> ring depth 250 + 8 b; one session: 300 steps -> depth 150), so "
+                         "the measured step does not depend on --steps; start: sessions start at depth 8 b; "
                          "full: every ring full (depth = context, 3000)")
     ap.add_argument("--kv-seek", type=int, default=-1,
                     help="debug / tuning: move every session to this ring depth instead (overrides --kv-depth; not a named configuration)")
@@ -189,7 +189,7 @@ def job_time(dt_local, dist, dev):
 
 
 def job_latency(p50, p95, dist, dev, world):
-    """BASELINE.json's second figure is the JOB's step latency: MAX over ranks, with the per-rank figures alongside."""
+    """The second figure is the JOB's step latency: MAX over ranks, with the per-rank figures alongside."""
     if dist is None:
         return p50, p95, [p50], [p95]
     t = torch.tensor([p50, p95], device=dev, dtype=torch.float64)
@@ -205,7 +205,7 @@ def job_value(world, sessions_per_gpu, steps, dt):
 
 
 def mimi_algorithmic_bytes(cfg, B, frames_so_far):
-    """weights once per step for the whole batch + per-stream KV/ring/IO traffic (fp32 here)."""
+    """Weights once per step for the whole batch + per-stream KV/ring/IO traffic (fp32 here)."""
     from moshi_amd.weights import mimi_state_spec
     used = 0
     for name, shape, _ in mimi_state_spec(cfg):
@@ -403,10 +403,10 @@ def main():
     if lm_gen is not None:
         from bench_lm import stagger
         staggered = stagger(mimi if workload == "duplex" else None, lm_gen, step, B, args.stagger, dev, before_mask=join)
-    # ring depth of session b when the warm-up starts.  "mid": the midpoint of the configuration's run as SURVEY.md 8d states it
+    # ring depth of session b when the warm-up starts.  "mid": the midpoint of the configuration's run
     # (C4: 500 steps, sessions `stagger` frames apart; C3: one session, 300 steps) - the rings' skipped positions hold zeros, the
     # kernels read them all the same (no data-dependent control flow), and the codec's rings are where the stagger left them
-    # (rows >= 16 of 32 are past their 250-slot wrap).  "start": what the stagger alone leaves (rounds 1-3).
+    # (rows >= 16 of 32 are past their 250-slot wrap).  "start": what the stagger alone leaves.
     base_depth = [args.stagger * b if B > 1 else staggered for b in range(B)]
     if lm_gen is not None and args.kv_depth != "start":
         join()
@@ -449,7 +449,7 @@ def main():
         for k, v in lists.items():
             (d / f"launch_list_{k}.tsv").write_text("".join("\t".join(str(x) for x in row) + "\n" for row in v))
 
-    # p50 / p95 latency of a single step (BASELINE.json's second figure): a separate, untimed-for-`value` pass with a
+    # p50 / p95 latency of a single step: a separate, untimed-for-`value` pass with a
     # device event before and after every step and no host synchronisation inside the loop.  Pipelined: every frame completes
     # before the next is submitted, so the figure is PCM-in -> PCM-out of ONE frame with nothing else in flight (what a
     # session waits for), not the steady-state step interval `ms_per_step` reports.
@@ -525,7 +525,7 @@ def main():
             # ring depth of every session in the middle of the profiled steps (they follow the timed region and the latency pass)
             done = args.warmup + args.steps + max(8, min(args.steps, 40)) + max(4, min(args.steps, 20)) // 2
             out["roofline"] = roofline_lm(lm_gen, step, args, sync, kv_rows=[base_depth[b] + done for b in range(B)])
-            # the WHOLE step against the HBM roofline (SURVEY.md 8d): LM weights once + every session's KV at its depth at
+            # the WHOLE step against the HBM roofline: LM weights once + every session's KV at its depth at
             # the middle of the timed region (+ Mimi's weights / rings / KV when the step includes the codec)
             mid = args.warmup + args.steps // 2
             L_rows = [base_depth[b] + mid for b in range(B)]
@@ -538,12 +538,11 @@ def main():
             out["roofline"]["step"] = {"algorithmic_bytes": step_bytes, "parts": parts, "achieved": ach, "unit": "GB/s",
                                        "frac": ach / HBM_PEAK_GBS, "ms_per_step": ms}
         if workload == "duplex" and world == 1 and not args.no_extras and not args.lm_layers and args.quant == "none" and args.kv == "bf16":
-            # the other figures SURVEY 8d asks of this model, measured in the same process after the headline
+            # the other figures of this model, measured in the same process after the headline
             from bench_lm import extra_full_context, extra_c3
             join()
             if args.kv_depth == "mid":
-                # the same pipelined step at the ring depth rounds 1-3 quoted (sessions 8 b deep + warm-up): the figure comparable
-                # with BENCH_r01..r03 (6.19 ms in round 3), beside the mid-run headline
+                # the same pipelined step with shallow rings (sessions 8 b deep + warm-up), beside the mid-run headline
                 lm_gen.seek([args.stagger * b for b in range(B)])
                 for _ in range(3):
                     step()

@@ -16,7 +16,7 @@ HBM_PEAK_GBS = 8000.0
 def replicated_state_dict(draw, spec, dtype, dev):
     """One process per GPU: rank 0 draws the (7.7 B parameter, bf16, seeded) weights on its GPU and replicates them to the
     other ranks with RCCL broadcasts in 1 GiB buckets (moshi_amd/dist.py) - the deployment's only collective, at load, as in
-    SURVEY.md 8e.  Single process, or MMI_BENCH_NO_BCAST=1: every rank draws the same seeded weights itself."""
+    Single process, or MMI_BENCH_NO_BCAST=1: every rank draws the same seeded weights itself."""
     import torch.distributed as dist
     if not (dist.is_available() and dist.is_initialized()) or dist.get_world_size() == 1 or os.environ.get("MMI_BENCH_NO_BCAST"):
         return draw()
@@ -50,7 +50,7 @@ def make_lm(dev, B, args, streaming=True):
 
 
 def stagger(mimi, lm_gen, step_fn, B, frames_apart, dev, before_mask=None):
-    """sessions start staggered (row b has run frames_apart*b frames when timing starts).
+    """Sessions start staggered (row b has run frames_apart*b frames when timing starts).
     before_mask: called before every mask change (the pipelined step joins its streams there)."""
     if frames_apart <= 0 or B == 1:
         return 0
@@ -72,7 +72,7 @@ def stagger(mimi, lm_gen, step_fn, B, frames_apart, dev, before_mask=None):
 
 
 def lm_step_algorithmic_bytes(cfg, L_per_row, quant="none", kv="bf16"):
-    """weights once per step (2 B bf16; 1 B + a 4-byte scale per output row for int8 / fp8) + per-stream KV
+    """Weights once per step (2 B bf16; 1 B + a 4-byte scale per output row for int8 / fp8) + per-stream KV
     read of the valid positions and write of the new one (2 B bf16, 1 B fp8)."""
     d, dd, h, dh = cfg.dim, cfg.depformer_dim, cfg.ffn_hidden, cfg.depformer_ffn_hidden
     per_layer = 3 * d * d + d * d + 2 * h * d + d * h
@@ -125,7 +125,7 @@ def roofline_lm(lm_gen, step_fn, args, sync, kv_rows=None):
             rec.update({"bytes_per_op": wbytes, "GBps": wbytes / us / 1e3, "frac": wbytes / us / 1e3 / HBM_PEAK_GBS})
         sites[site] = rec
     out["sites"] = sites
-    # the largest site by time per step (VERDICT r4 item 7: at the mid-run depth the decode attention outweighs the dominant GEMM)
+    # the largest site by time per step (at the mid-run depth the decode attention outweighs the dominant GEMM)
     timed = {k: dict(v) for k, v in sites.items() if "frac" in v and v.get("ops_per_step", 0) > 0}
     if "L.ffn_in" in timed and mean_ms.value > 0:
         # this site's ops carry a SECOND event pair (the dominant-kernel tap above): rank it by that tap's own figure instead
@@ -136,8 +136,8 @@ def roofline_lm(lm_gen, step_fn, args, sync, kv_rows=None):
         big = max(timed, key=lambda k: timed[k]["us_per_step"])
         out["largest_site"] = {"site": big, "kernel": {"L.attn": "k_lm_attn_wave"}.get(big, "see mmi_lm_launch_list"), **timed[big],
                                "note": "live hipEvents around each op of un-graphed steps (a few us of dispatch per op included)"}
-    # secondary figure (north_star: "achieved MFMA/HBM fraction"): the same launch's matrix-core rate.  The GEMM is
-    # 2 * N * K * B flops with N = 2 * ffn_hidden rows, K = dim, B sessions; dense peaks from MI355X_MICROARCH.md.
+    # secondary figure: the same launch's matrix-core rate.  The GEMM is
+    # 2 * N * K * B flops with N = 2 * ffn_hidden rows, K = dim, B sessions; dense peaks.
     cfg = lm_gen.lm_model.config
     flops = 2.0 * (2 * cfg.ffn_hidden) * cfg.dim * lm_gen._batch
     quant = getattr(args, "quant", "none")
@@ -147,7 +147,7 @@ def roofline_lm(lm_gen, step_fn, args, sync, kv_rows=None):
                    "instruction": "v_mfma_f32_32x32x16_fp8_fp8" if quant == "fp8" else "v_mfma_f32_32x32x16_bf16",
                    "note": "decode GEMM at B sessions: arithmetic intensity ~B flop/byte, far below the ~310 flop/byte ridge"}
     # HBM bytes per launch from the PMC counters: a counter pass cannot run inside the timed benchmark (it serialises every
-    # dispatch), so the figure is the committed measurement of the same kernel, shape and batch - since round 3 collected on
+    # dispatch), so the figure is the committed measurement of the same kernel, shape and batch, collected on
     # THIS library inside the LM step (scripts/gpu_pmc.sh: eager launches under rocprofv3 --pmc), before that on a standalone launcher.
     pmc = Path(__file__).resolve().parent / "profiles" / "pmc_dominant_kernel.json"
     if pmc.exists() and lm_gen._batch == 32:
@@ -182,8 +182,8 @@ def _time_lm_steps(gen, codes, n_warm, n, dev):
 
 
 def extra_full_context(lm_gen, user_codes, B, dev, steps=10):
-    """`full_context` of the default line: LMGen.step ALONE on the benchmark's handle with every session's ring full (SURVEY.md
-    8d: "B=32, L=3000: 14.75 + 50.3 GB -> 8.1 ms" floor) - the sessions are moved to position `context` (mmi_lm_seek), so every
+    """`full_context` of the default line: LMGen.step ALONE on the benchmark's handle with every session's ring full (32 sessions,
+    3000 rows: 14.75 + 50.3 GB, a floor of 8.1 ms) - the sessions are moved to position `context` (mmi_lm_seek), so every
     step reads all 3000 slots of every ring.  Runs after everything else (it leaves the sessions there)."""
     cfg = lm_gen.lm_model.config
     lm_gen.seek([cfg.context] * B)
@@ -196,8 +196,8 @@ def extra_full_context(lm_gen, user_codes, B, dev, steps=10):
 
 
 def extra_c3(dev, args, steps=30):
-    """`c3` of the default line (BASELINE configs[2]: Moshi-7B bf16 LMGen.step, batch 1 - the single real-time session): a
-    second handle built for ONE session (16-row MFMA tile), moved to the midpoint of SURVEY 8d's 300-step run, sampled."""
+    """`c3` of the default line (Moshi-7B bf16 LMGen.step, batch 1 - the single real-time session): a
+    second handle built for ONE session (16-row MFMA tile), moved to the midpoint of a 300-step run, sampled."""
     import copy
     a1 = copy.copy(args)
     gen = make_lm(dev, 1, a1)
@@ -222,7 +222,7 @@ def extra_c3(dev, args, steps=30):
 
 
 def extra_c5(args):
-    """`c5` of the default line (BASELINE configs[4]: q8 weights on the 8-bit matrix core, 64 sessions per GPU): the same duplex
+    """`c5` of the default line (q8 weights on the 8-bit matrix core, 64 sessions per GPU): the same duplex
     step - Mimi encode -> LMGen.step -> Mimi decode, pipelined, mid-run ring depth - with row-wise int8 linears x row-wise int8
     activations (the reference's bitsandbytes arithmetic) and the e4m3 KV ring, measured by a child process running this very
     benchmark with `--batch 64 --quant q8 --kv fp8` (its own handles, its own memory; the parent's stay resident), plus the same
@@ -248,7 +248,7 @@ def extra_c5(args):
 
 
 def extra_c2(args):
-    """`c2` of the default line (BASELINE configs[1]: Mimi streaming encode + RVQ + decode, 8 streams, one GPU): a child process running
+    """`c2` of the default line (Mimi streaming encode + RVQ + decode, 8 streams, one GPU): a child process running
     this very benchmark with `--workload mimi --batch 8` (fp32 codec, the reference's own width - what keeps the codes bit-exact)."""
     import subprocess
     import sys
@@ -277,7 +277,7 @@ def _mem_available_gib():
 def cpu_lm_measured(dev, timed=3):
     """The LM oracle at the model's FULL depth (32 temporal layers, full depformer and text head, fp32 numpy on the host cores,
     B = 1): one warm-up step, then the median of `timed` steps.  The weights are the benchmark's own (same seed), drawn on the
-    GPU and copied to the host (15 GB bf16 -> 30 GB fp32).  Needs a host with >= 64 GB free (SURVEY.md 8d)."""
+    GPU and copied to the host (15 GB bf16 -> 30 GB fp32).  Needs a host with >= 64 GB free."""
     from moshi_amd.config import LMConfig
     from moshi_amd.weights import random_lm_state_dict
     from oracle.lm_oracle import LMOracle
@@ -314,7 +314,7 @@ def _host_info():
 
 
 def _reference_quote():
-    """The reference ITSELF cannot travel to the GPU box (no copy of its sources is kept here): its own CPU path, timed on the
+    """The reference ITSELF is not here (no copy of its sources is kept here): its own CPU path, timed on the
     build container by scripts/reference_cpu_baseline.py (recipe of scripts/moshi_benchmark.py:76-100), is quoted beside the port."""
     rp = Path(__file__).resolve().parent / "profiles" / "r03_logs" / "reference_cpu_baseline.json"
     if not rp.exists():
@@ -330,13 +330,13 @@ def cpu_baseline_duplex(mimi_base, args, layers=(1, 5), timed=5, dev=None):
     """`port` baseline for the full frame on the host cores: the numpy oracles (the reference itself cannot travel to the GPU
     box).  Mimi is timed directly (mimi_base); the LM oracle (fp32, B=1, full depformer and text head) is timed at two reduced
     depths - median of `timed` steps after one warm-up step each, the temporal stack (`forward_text`) also on its own clock -
-    and extrapolated linearly to the model's 32 temporal layers with the per-layer cost of that stack: the layer-scaled proxy BASELINE.md section 3 allows when the full 7B fp32 oracle (30 GB) is too heavy for a
-    default run.  The slope must be positive (a 32-layer model that costs what one layer costs is not a baseline)."""
+    and extrapolated linearly to the model's 32 temporal layers with the per-layer cost of that stack: the proxy for where the full
+    7B fp32 oracle (30 GB) is too heavy for a default run.  The slope must be positive (a 32-layer model that costs what one layer costs is not a baseline)."""
     from moshi_amd.config import LMConfig
     from moshi_amd.weights import random_lm_state_dict
     from oracle.lm_oracle import LMOracle
-    # the full 32-layer oracle, MEASURED, whenever the host can hold it (VERDICT r3 item 8); the layer-scaled proxy below is the
-    # fallback SURVEY.md 8d describes for a host that cannot (or a run with --lm-layers / MMI_BENCH_CPU_PROXY=1)
+    # the full 32-layer oracle, MEASURED, whenever the host can hold it; the layer-scaled proxy below is the
+    # fallback for a host that cannot (or a run with --lm-layers / MMI_BENCH_CPU_PROXY=1)
     if dev is not None and not args.lm_layers and not os.environ.get("MMI_BENCH_CPU_PROXY") and _mem_available_gib() >= 64:
         lm_s, ts, t_build = cpu_lm_measured(dev)
         mimi_s = 1.0 / mimi_base["value"]

@@ -1,4 +1,4 @@
-"""The binding a maintainer of kyutai-labs/moshi would add to call libmoshi_mi.so (INTEGRATION.md section 2), as a module that
+"""The binding a maintainer of kyutai-labs/moshi would add to call libmoshi_mi.so, as a module that
 RUNS: ctypes + torch only, nothing of `moshi_amd` is imported.  It would live in the reference as `moshi/models/_mi355x.py`; the
 two classes take what the reference already has in hand - a model's `state_dict()` and the configuration dictionaries of
 `moshi/moshi/models/loaders.py` (`_seanet_kwargs`, `_quantizer_kwargs`, `_transformer_kwargs` inside a `mimi_config`; `_lm_kwargs`)
@@ -48,7 +48,7 @@ class Sampling(C.Structure):
 
 
 _DT = {torch.float32: 0, torch.bfloat16: 1, torch.int64: 2, torch.float16: 3, torch.int8: 4}
-_ERR = {-2: AssertionError, -3: RuntimeError, -5: KeyError, -1: ValueError}       # the reference's exception types (SURVEY.md 8b)
+_ERR = {-2: AssertionError, -3: RuntimeError, -5: KeyError, -1: ValueError}       # the reference's exception types
 _P = C.c_void_p
 
 

@@ -50,7 +50,7 @@ typedef enum mmi_dtype { MMI_F32 = 0, MMI_BF16 = 1, MMI_I64 = 2, MMI_F16 = 3, MM
 typedef void* mmi_stream; /* hipStream_t */
 
 /* One state-dict entry, named exactly as in the reference checkpoints
- * (SURVEY.md Appendix A; loaders.py:356-358,413-422).  `data` is a device pointer. */
+ * (loaders.py:356-358,413-422).  `data` is a device pointer. */
 typedef struct mmi_tensor_desc {
     const char* name;
     const void* data;
@@ -181,7 +181,7 @@ typedef struct mmi_lm_cfg {
     int32_t extra_heads_num_heads;    /* 0: nn.Linear(dim, extra_heads_dim) heads on the transformer output (lm.py:101-102, 224-226) */
     int32_t extra_heads_dim;          /* 6 */
     int32_t kv_cache_dtype;           /* 0 / MMI_BF16: the reference's bf16 ring (transformer.py:453-455); MMI_F8E4M3: e4m3 ring -
-                                         half the attention stream and half the per-session state (SURVEY.md 8d C5 "fp8 KV") */
+                                         half the attention stream and half the per-session state */
     int32_t cross_attention;          /* 1: every temporal layer has a cross-attention block (`cross_attention.{in,out}_projs.0`,
                                          `norm_cross.{weight,bias}`; transformer.py:727-732, 779-786) fed by mmi_guidance.condition_cross */
 } mmi_lm_cfg;
@@ -200,7 +200,7 @@ typedef struct mmi_lm mmi_lm;
 
 /* loaders.get_moshi_lm (loaders.py:366-446): build LMModel from state-dict tensors - bf16, or with the linears in the
  * reference's quantised storage (utils/quantize.py:13-22): `<linear>.weight` MMI_I8 [out,in] row-wise absmax codes plus
- * `<linear>.weight_scb` MMI_F32 [out] row absmax; or as fp8 (BASELINE configs[4], run on the fp8 MFMA): `<linear>.weight`
+ * `<linear>.weight_scb` MMI_F32 [out] row absmax; or as fp8 (run on the fp8 MFMA): `<linear>.weight`
  * MMI_F8E4M3 [out,in] codes, `<linear>.weight_scale` MMI_F32 [out] (W ~= code * scale) and an optional scalar
  * `<linear>.input_scale` MMI_F32 (static activation scale: x8 = e4m3(x / input_scale), default 1).  Embeddings and norms
  * stay bf16.  The linears must be all bf16, all int8 or all fp8. */
@@ -210,7 +210,7 @@ void mmi_lm_destroy(mmi_lm* lm);
 
 /* LMGen.streaming(batch) enter/exit (lm.py:605-666). */
 int mmi_lm_streaming_start(mmi_lm* lm, int32_t batch, const mmi_sampling* sampling, mmi_stream stream);
-/* LMGen's classifier-free guidance and conditioning arguments (lm.py:566-574, 612-651; SURVEY.md 8f-3).  With
+/* LMGen's classifier-free guidance and conditioning arguments (lm.py:566-574, 612-651).  With
  * cfg_coef != 1 the model runs two rows per session (conditioned, unconditioned) - 2 * batch must fit max_batch - and every
  * sampling site draws from logits_null + (logits - logits_null) * cfg_coef (lm.py:727-733, 828-832).
  *   cfg_is_masked_until  host i64 [batch] or NULL: the unconditioned row reads zero tokens until offset > delay + value (lm.py:713-721)
@@ -426,7 +426,7 @@ int mmi_duplex_get_stamps(mmi_duplex* d, double* ms40, int64_t* last_frame);
 /* ------------------------------------------------------------------------------------------ */
 /* Session batcher: many live dialogue sessions on one GPU                                    */
 /* ------------------------------------------------------------------------------------------ */
-/* SURVEY.md 8f-1.  The reference's Python server runs ONE session under a lock (server.py:45,57,154-169);
+/* The reference's Python server runs ONE session under a lock (server.py:45,57,154-169);
  * its Rust server packs up to `batch_size` live channels into one batched model step with a per-row stream
  * mask and a per-row reset when a channel is (re)opened (rust/moshi-server/src/batched_asr.rs:188-276 model
  * loop, :279-374 pre_process, :376-437 post_process; py_module.rs:443-470 slot allocation).  This is that

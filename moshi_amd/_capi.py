@@ -214,7 +214,7 @@ class Lib:
 
     def check(self, rc: int) -> None:
         """Map a status to the exception type the reference raises in the same situation
-        (SURVEY.md 8b: RuntimeError for streaming misuse, AssertionError for shape/batch mismatch)."""
+        (RuntimeError for streaming misuse, AssertionError for shape/batch mismatch)."""
         if rc == MMI_OK:
             return
         msg = f"{self.last_error()} (mmi status {rc})"
@@ -226,7 +226,7 @@ class Lib:
             raise KeyError(msg)
         if rc == MMI_ERR_BUSY:
             raise BufferError(msg)
-        if rc == MMI_ERR_NO_CHANNEL:                # its own status (ADVICE r4): no matching on the message text
+        if rc == MMI_ERR_NO_CHANNEL:                # its own status: no matching on the message text
             from .errors import UnknownChannel
             raise UnknownChannel(msg)
         if rc == MMI_ERR_UNSUPPORTED:

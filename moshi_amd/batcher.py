@@ -1,4 +1,4 @@
-"""`SessionBatcher` - many live full-duplex sessions on one GPU (SURVEY.md 8f-1), host mirror of `mmi_batcher_*`.
+"""`SessionBatcher` - many live full-duplex sessions on one GPU, host mirror of `mmi_batcher_*`.
 
 The reference's Python server holds one session under a lock (moshi/moshi/server.py:45,57,154-169); its Rust server is the
 model for batching: fixed slots, one channel per slot with a PCM FIFO, a model loop that each iteration takes one 80 ms

@@ -1,5 +1,5 @@
 // Session batcher behind the C ABI (include/moshi_mi.h, "Session batcher"): the model loop that packs many live
-// full-duplex dialogue sessions into the batched frame step of one GPU (SURVEY.md 8f-1).
+// full-duplex dialogue sessions into the batched frame step of one GPU.
 //
 // The reference's Python server holds ONE session under an asyncio lock (moshi/moshi/server.py:45,57,154-169); the
 // reference's Rust server is the model for batching: a fixed number of slots, a channel per slot with a PCM FIFO, and a

@@ -173,7 +173,7 @@ int create_impl(mmi_duplex* d) {
     // back to back, they land on different hardware queues of the pool of GPU_MAX_HW_QUEUES (4).
     MMI_HIP_CHECK(hipMalloc((void**)&d->flags, (size_t)F_COUNT * 16 * sizeof(long)));
     MMI_HIP_CHECK(hipMemset(d->flags, 0, (size_t)F_COUNT * 16 * sizeof(long)));
-    // MMI_DUPLEX_CODEC_CUS=n (experiment, round 6): the codec streams confined to n of the CUs (a CU mask of n bits, which the driver
+    // MMI_DUPLEX_CODEC_CUS=n (experiment): the codec streams confined to n of the CUs (a CU mask of n bits, which the driver
     // deals out over the XCDs), so that the depth transformer's launches - 96..176 workgroups that need a whole CU's wave slots each -
     // find free CUs while the codec of the neighbouring frames runs beside them
     const int codec_cus = getenv("MMI_DUPLEX_CODEC_CUS") ? atoi(getenv("MMI_DUPLEX_CODEC_CUS")) : 0;
@@ -258,7 +258,7 @@ int submit_impl(mmi_duplex* d, const float* pcm_caller, float* pcm_out, int64_t*
     if (t >= 2) MMI_HIP_CHECK(hipEventSynchronize(d->ev_lm[p]));
     // host-kept gate: the frame is enqueued once LMGen.step(t-1) has reached its depth-transformer phase
     if (t >= 1) MMI_HIP_CHECK(hipEventSynchronize(d->ev_phase[p ^ 1]));
-    // the frame's input -> the pipeline's own ring, in the caller's stream order (ADVICE r3: the caller's buffer is free again
+    // the frame's input -> the pipeline's own ring, in the caller's stream order (the caller's buffer is free again
     // when this call returns, as after MimiModel.encode)
     float* pcm_in = d->pcm_in[t % d->in_slots];
     MMI_HIP_CHECK(hipMemcpyAsync(pcm_in, pcm_caller, (size_t)d->B * d->F * sizeof(float), hipMemcpyDeviceToDevice, (hipStream_t)caller));

@@ -49,10 +49,10 @@ struct mmi_lm {
     int max_batch = 0;
     int T = 32;                     // MFMA tile of the temporal transformer and the heads: 16 when max_batch <= 16, else 32 (lm_kernels.h)
     int Td = 32;                    // MFMA tile of the depth transformer (its linears, dx / dxn / datt / dhb): T.  MMI_DEP_TILE=16 (17..32
-                                    // sessions, bf16): two 16-row batch tiles per 16-row weight tile - measured in round 6 inside the step
+                                    // sessions, bf16): two 16-row batch tiles per 16-row weight tile - measured inside the step
                                     // (profiles/r06_logs/ab_dep_tile_once.txt): in_proj -0.14 us, linear_out -0.6, but the gated
                                     // linear_in +3.0 (352 tiles at 128 registers: spills) and out_proj +0.3 -> +0.15 ms per step; the
-                                    // microbenchmark's -0.13 ms (round 5, independent launches) does not survive the dependent chain.
+                                    // microbenchmark's -0.13 ms (independent launches) does not survive the dependent chain.
                                     // Kept as an opt-in: the boundaries are row-major either way (dpre, dqkv, the logits)
     int q8 = -1;                    // -1 undecided, 0 bf16 linears, 1 int8 linears (`weight` int8 + `weight_scb`, utils/quantize.py),
                                     // 2 fp8 linears (`weight` e4m3fn + `weight_scale` [+ `input_scale`]) run on the fp8 MFMA
@@ -105,8 +105,8 @@ struct mmi_lm {
     unsigned* attn_done = nullptr;                  // [B][H] arrival counters of the split decode attention (k_lm_attn_wave), 0 between launches
     float* partial = nullptr;                       // [4][B][max(dim, depformer_dim)] split-K partial sums
     float* rope = nullptr;                          // [B][Dh/2][2] (cos, sin) of the step's new position
-    // int8 activations (BASELINE configs[4], the reference's own arithmetic: QLinear.forward -> bitsandbytes' int8 x int8 matmul,
-    // utils/quantize.py:24-40): on for int8 linears unless MMI_Q8_ACT=bf16 (weight-only, rounds 1-3) or the model has
+    // int8 activations (the reference's own arithmetic: QLinear.forward -> bitsandbytes' int8 x int8 matmul,
+    // utils/quantize.py:24-40): on for int8 linears unless MMI_Q8_ACT=bf16 (weight-only) or the model has
     // cross-attention layers.  xnq / attq / hbq / toutq: the int8 operand Xq[mt][kp][lane][16] next to its bf16 tensor, sx_*: its
     // rows' absmax (bitsandbytes' SCA).  Who quantises: the norm kernel for its own output (one workgroup per row); a
     // k_quant_rows_i8 launch for the temporal attention output and the gated FFN tensor (rows written by many workgroups); the
@@ -373,7 +373,7 @@ int launch_gemm_t(hipStream_t s, const GemmPlan& p, int NT, int mt, const GemmAr
     const dim3 groups(mmi_cdiv(NT, p.ntw) * (a.osplit > 1 ? a.osplit : 1), p.ksplit);
     const int w8 = a.wq;
     if (mt == 1) return launch_gemm_w<TN, 1, 1>(s, groups, p.waves, p.u, w8, a);     // one n-tile per workgroup (two measured slower
-    if (mt == 2) return launch_gemm_w<TN, 2, 1>(s, groups, p.waves, p.u, w8, a);     // in the step, DESIGN 9e: not instantiated)
+    if (mt == 2) return launch_gemm_w<TN, 2, 1>(s, groups, p.waves, p.u, w8, a);     // in the step: not instantiated)
     return mmi_fail(MMI_ERR_UNSUPPORTED, "batch too large for the skinny GEMM");
 }
 
@@ -657,7 +657,7 @@ void add_hidden_tap(mmi_lm* lm, int which) {
 }
 
 // k_gemm_q8 at 33..64 sessions: one batch tile per workgroup (grid.y = tiles; the default) or both tiles walked by one workgroup
-// (MMI_Q8_TILES=serial: the round-4 form, same-box A/B)
+// (MMI_Q8_TILES=serial, same-box A/B)
 static bool q8_tiles_over_grid() {
     const char* e = getenv("MMI_Q8_TILES");
     return !(e && e[0] == 's');
@@ -873,8 +873,8 @@ void add_sample(mmi_lm* lm, uint16_t* logits, int ld, int V, bool text, int site
     });
 }
 
-// MMI_ATTN: "wave" (default since round 4) = k_lm_attn_wave, one online softmax per wave, no barrier in the loop; "split" = the
-// chunked kernel of rounds 1-3 (same-box A/Bs)
+// MMI_ATTN: "wave" (default) = k_lm_attn_wave, one online softmax per wave, no barrier in the loop; "split" = the
+// chunked kernel (same-box A/Bs)
 static bool attn_wave_kernel() {
     const char* e = getenv("MMI_ATTN");
     return !(e && e[0] == 's');
@@ -883,7 +883,7 @@ static bool attn_wave_kernel() {
 // workgroups per (session, head) of the decode attention.  k_lm_attn_wave: ONE from 128 pairs (4 sessions) on - one workgroup per
 // pair walking the whole ring beats ring split + merge launch at every depth there (4 / 8 / 16 sessions, 3000 rows: -0.03 / -0.16 /
 // -0.16 ms per step, profiles/r04_logs/call_v_summary.txt); below that the ring is split (and still walked by one workgroup while
-// it is short: attn_solo_rows).  The chunked kernel of rounds 1-3: 1 once B*H alone fills the chip.
+// it is short: attn_solo_rows).  The chunked kernel: 1 once B*H alone fills the chip.
 int attn_splits(const mmi_lm_cfg& c, int B) {
     if (const char* e = getenv("MMI_ATTN_NS")) {          // test hook: the split + combine path on rings too short to need it
         const int v = atoi(e);
@@ -909,7 +909,7 @@ static int attn_solo_rows(int pairs) {
 //      each (session, head) walks the ring and writes the output.  One launch per layer instead of two: 4.4 us x 32 layers of a
 //      4.7 ms single-session step.  (Should a ring be longer all the same, the kernel merges in its last-arriving workgroup:
 //      correct whatever the host believes, 8 us per layer slower than a launch - measured, profiles/r04_logs/call_j_summary.txt)
-//   1  deeper rings: partials from every workgroup + the k_lm_attn_combine launch, as in rounds 1-3.
+//   1  deeper rings: partials from every workgroup + the k_lm_attn_combine launch.
 // MMI_ATTN_MERGE=kernel (test hook) stays on variant 0 whatever the depth.
 static int attn_variant(const mmi_lm* lm, int NS) {
     if (NS <= 1 || !attn_wave_kernel()) return 0;
@@ -1720,7 +1720,7 @@ extern "C" int mmi_lm_step(mmi_lm* lm, const int64_t* user_codes, int32_t n_user
         // both attention programs exist from the stream's first step on: the switch at depth solo_rows is then a graph launch
         // like any other (without this the deep program was captured + instantiated ~61 s into a live single-session stream)
         // The step above is already committed: a failure to capture the OTHER program (out of memory at instantiate, ...) must not
-        // turn it into a failed call - the program is then captured when first needed, as before round 5.  The capture
+        // turn it into a failed call - the program is then captured when first needed.  The capture
         // re-runs every op closure: its GEMMs are not launches of this stream (mmi_lm_stat 0).
         const bool split = lm->phase_fn != nullptr;
         const long counted = lm->xlds_launches;
@@ -1844,7 +1844,7 @@ extern "C" int mmi_lm_state_load(mmi_lm* lm, const void* src, int64_t bytes, int
     MMI_HIP_CHECK(lm->st.load(src, (hipStream_t)stream));
     lm->offset_cpu = (long)host_word;
     {   // the snapshot's offsets bound the ring depth (which step program the next steps take): read them back - a restore is not
-        // a per-frame call, and without this a shallow restored session paid the merge launch for the rest of the stream (ADVICE r4)
+        // a per-frame call, and without this a shallow restored session paid the merge launch for the rest of the stream
         std::vector<long> off(lm->batch);
         MMI_HIP_CHECK(hipStreamSynchronize((hipStream_t)stream));
         MMI_HIP_CHECK(hipMemcpy(off.data(), lm->offsets_m, (size_t)lm->batch * sizeof(long), hipMemcpyDeviceToHost));

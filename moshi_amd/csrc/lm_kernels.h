@@ -112,7 +112,7 @@ __device__ __forceinline__ void mmi_i8x16_to_bf16(u32x4 q, u32x4& lo, u32x4& hi)
     }
 }
 
-// fp8 linears (BASELINE configs[4]: fp8 MFMA GEMMs): `weight` e4m3fn codes + `weight_scale` fp32 per output row (W ~= code *
+// fp8 linears (fp8 MFMA GEMMs): `weight` e4m3fn codes + `weight_scale` fp32 per output row (W ~= code *
 // scale), packed exactly like the int8 bytes (two k-steps per 16-byte lane entry).  The activations stay bf16 in HBM and are
 // converted to e4m3 in registers on their way into v_mfma_f32_{32x32x16,16x16x32}_fp8_fp8: x8 = e4m3(x / input_scale) with a
 // static per-linear `input_scale` (a calibration constant, default 1), and the fp32 accumulator is scaled by
@@ -164,7 +164,7 @@ __device__ __forceinline__ u32x2 mmi_quant_i8x8(u32x4 v, float scale) {
 __device__ __forceinline__ float mmi_i8_scale(float sca) { return sca > 0.f ? 127.0f / sca : 0.f; }
 // The dequantisation of oracle/lm_oracle.py `linear_int8` - a RESTATEMENT of bitsandbytes' int8_mm_dequant, `out32 * (row_stats *
 // col_stats) * (1 / 127^2)` left to right in fp32, as its "default" backend writes it; not verified against the library, whose CUDA
-// kernel multiplies by a literal constant and returns fp16 (PARITY UNPINNED).  The engine's int8 x int8 linears
+// kernel multiplies by a literal constant and returns fp16 (parity unpinned).  The engine's int8 x int8 linears
 // are bit-identical to THAT RESTATEMENT for the same bf16 input row (tests: *_int8_linear_bit_exact_*)
 __device__ __forceinline__ float mmi_i8_dequant(int out32, float sca, float scb) {
     return ((float)out32 * (sca * scb)) * (1.0f / (127.0f * 127.0f));
@@ -429,7 +429,7 @@ __device__ __forceinline__ void mmi_gemm_epilogue(const GemmArgs& a, float (&acc
                     // `re * c - im * sn` the compiler packs the four pairs into v_pk_mul_f32 / v_pk_add_f32 with op_sel swizzles,
                     // one of them in place, and on gfx950 that sequence inside k_gemm_xp<32, 2, ..> (64 sessions) returned, now and
                     // then, a stale last element for lanes 48-63 - q / k of 16 sessions wrong in one feature, a different one
-                    // from run to run: the "row 17" failure of the driver's round-4 suite (profiles/r05_logs/c5_trace_*.txt)
+                    // from run to run (profiles/r05_logs/c5_trace_*.txt)
                     const float re = v8[2 * j], im = v8[2 * j + 1];
                     mmi_rope_rotate(re, im, c, sn, v8[2 * j], v8[2 * j + 1]);
                 }
@@ -1092,7 +1092,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
 // ------------------------------------------------------------------------------------------------
 // k_gemm_xp re-reads the whole activation matrix from L2 in every workgroup (one per n-tile): at 32 sessions that is as many
 // L2 bytes as the weights themselves, at 64 twice as many, and the L2 (about 10-11 TB/s of 128-byte requests) - not HBM -
-// becomes the bound (DESIGN.md 9e, profiles/r01_pmc_sq_tcc_ffn_in_b32_b64.csv).  Here ONE workgroup per CU walks a contiguous
+// becomes the bound (profiles/r01_pmc_sq_tcc_ffn_in_b32_b64.csv).  Here ONE workgroup per CU walks a contiguous
 // range of up to NTMAX n-tiles.  K is cut into chunks of KC k-steps whose activation fragments (MT x KC KiB) are staged in LDS,
 // double-buffered, so every activation byte leaves the L2 once per workgroup; the 8 waves split a chunk's k-steps, stream their
 // KPW weight fragments per (chunk, tile) segment from HBM one segment ahead of the MFMAs (register double buffer) and read
@@ -1674,7 +1674,7 @@ __global__ __launch_bounds__(256) void k_lm_attn_split(LmAttnArgs a) {
     constexpr int RPW = 64 / LPR;      // rows per wave instruction
     constexpr int CH = MMI_ATTN_CHUNK;
     // (a mirrored session order - every second group of 8 sessions walked backwards, for load balance across CUs under a linear
-    // stagger of ring depths - measured neutral, round 2: not built in)
+    // stagger of ring depths - measured neutral: not built in)
     const int bh = blockIdx.x;
     const int b = bh / a.H;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -1819,10 +1819,10 @@ __global__ __launch_bounds__(256) void k_lm_attn_split(LmAttnArgs a) {
     }
 }
 
-// The same attention with ONE online softmax per lane group and no workgroup barrier inside the loop (round 4).  k_lm_attn_split
+// The same attention with ONE online softmax per lane group and no workgroup barrier inside the loop.  k_lm_attn_split
 // walks a 256-row chunk in four dependent memory round trips (keys x 2, softmax through LDS, values x 2) with three barriers
 // in between, and all of a CU's co-resident workgroups do so in lockstep: at the benchmark's ring depths (150 ... 550 rows per
-// head) the kernel is bound by those round trips, not by HBM (23 us for 78 MB, DESIGN.md).  Here the ring's rows are dealt out in
+// head) the kernel is bound by those round trips, not by HBM (23 us for 78 MB).  Here the ring's rows are dealt out in
 // row groups (one wave instruction = RPW consecutive rows = 1 KiB) round-robin over ALL waves that serve the (session, head)
 // pair - 4 per workgroup x gridDim.y workgroups - and every wave keeps, per row slot (the lanes that share `rsub`), its own
 // running (max, sum, accumulator): a round requests NB key groups AND their NB value groups at once (the values do not depend
@@ -2584,7 +2584,7 @@ __global__ __launch_bounds__(NT) void k_sample(SampleArgs a) {
     const int k = a.k < V ? a.k : V;
     int want = k;
     unsigned Tkey = 0u;
-    // ---- production path (round 6): the k-th largest key WITHOUT the two 256-bin LDS histograms over every entry.  The logits of
+    // ---- production path: the k-th largest key WITHOUT the two 256-bin LDS histograms over every entry.  The logits of
     // a head share a handful of exponents, so the first histogram is 2048 (text head: 32000) LDS atomics on two or three
     // addresses - serialised - and each pass costs six workgroup barriers.  Instead: the block's largest key, then per-thread
     // PRIVATE counts (8 bits each, packed in 64) of the 8 high bytes at and below it, summed over the wave by shuffles and over
@@ -2844,7 +2844,7 @@ __global__ __launch_bounds__(NT) void k_sample(SampleArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// LMGen delay ring (lm.py:668-783, SURVEY.md Appendix B5)
+// LMGen delay ring (lm.py:668-783)
 // ------------------------------------------------------------------------------------------------
 struct TokArgs {
     int* cache;            // [B][NC][CT]

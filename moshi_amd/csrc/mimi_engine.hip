@@ -348,8 +348,8 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
 }
 
 // ---- launch helpers ---------------------------------------------------------------------------
-// A conv / linear becomes one of two launch sequences, chosen when the frame program is built (mimi_kernels.h):
-//   N = B*T_out > 128 columns : k_conv_wide
+// A conv becomes one of these launch sequences, chosen when the program is built (mimi_kernels.h; the transformers' linears: add_lin):
+//   N = B*T_out > 128 columns : k_conv_wide, in groups of frames also k_conv_cols [-> k_conv_finish when K is split over workgroups]
 //   N <= 128                  : k_conv_few [-> k_conv_finish], or [k_pack_b_f32] -> k_gemm_f32 [-> k_conv_finish when K is split over workgroups]
 struct ConvPlan {
     bool wide = false;
@@ -496,7 +496,8 @@ void wide_rule(const ConvGemmArgs& a, int N, int* mtb_out, int* w_out) {
 void gemm_rule(const ConvGemmArgs& a, int N, ConvPlan* p) {
     const int nsub = mmi_cdiv(N, 32);
     p->NSUB = nsub <= 1 ? 1 : (nsub == 2 ? 2 : 4);
-    // small weight matrices (the transformer linears, <= 8 MB): one workgroup per n-subtile, up to 16 waves splitting K
+    // small weight matrices (<= 8 MB - the released codec's last encoder conv, resampling, quantiser projections): one workgroup per n-subtile, 4 or 8
+    // waves splitting K
     const bool spread = nsub >= 2 && (size_t)a.Mt * a.Q * 1024 <= ((size_t)8 << 20);
     int ks = 1;
     if (a.out_mode == MMI_GOUT_NATURAL) {
@@ -865,7 +866,7 @@ int add_transformer(mmi_mimi* m, MimiMem& mem, MmiProgram& prog, const std::vect
     if (T / frames > 2 || (Dh != 16 && Dh != 32 && Dh != 64))
         return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi attention: head dim 16/32/64 and 1 or 2 steps per frame are built");
     const size_t attn_smem = ((size_t)T * Dh + (((size_t)T * cap + 3) & ~(size_t)3) + (size_t)(256 / (Dh / 4)) * T * Dh + 8) * sizeof(float);
-    // one memory round trip when a thread's 16 row slots cover the ring (the Mimi shape: 250 slots of 64 floats)
+    // one memory round trip when a thread's 8 row slots cover the ring (the Mimi shape: 250 slots of 64 floats)
     const bool one_pass = cap <= 8 * (512 / (Dh / 4)) && !getenv("MMI_MIMI_ATTN_TWO_PASS");
     // several frames at once: queries, keys and values row by row (the layers' keys and values until the ring takes them all at the end)
     const size_t rows_d = (size_t)B * H * T * Dh;

@@ -87,7 +87,8 @@ __global__ void k_codebook_prepare(const float* __restrict__ esum, const float* 
 //                dominate).  Same shape as the LM's weight-streaming GEMM: one m-tile per workgroup, K split over
 //                waves (+ workgroups), activations pre-packed into B-fragment order by k_pack_b_f32 (im2col + ELU +
 //                replicate padding) or by the producing kernel.
-//   k_conv_few   the same sums, bit for bit, for few streams: 16 x 16 tiles, operands from the input as it lies.
+//   k_conv_few   the same sums, bit for bit, for few streams (operands from the input as it lies) and for small products of a packed
+//                operand: 16 x 16 tiles.
 // The transformers' linears have kernels of their own (k_mimi_lin, k_mimi_lin_rows).
 // n / d for 0 <= n < 2^20 and 1 <= d < 2^20 (column and tap indices) as one multiply-high and a shift: an integer division costs
 // ~30 instructions, and the small kernels here are instruction bound.  magic = ceil(2^(32 + shift) / d), 0 means d == 1; exact while
@@ -177,7 +178,7 @@ template <int NV>
 __device__ __forceinline__ void mmi_conv_put_n(const ConvGemmArgs& a, const int (&co)[NV], const int (&b)[NV], const int (&t)[NV],
                                                const bool (&ok)[NV], const long (&row)[NV], const float (&bia)[NV], const float (&rsv)[NV], float (&v)[NV]) {
     // launch-uniform flags are tested once per group of NV values, not per value: these kernels are instruction bound, and a
-    // per-value maze of scalar branches (with the erf and expm1 bodies in line) was a third of a residual block's time (DESIGN 9i)
+    // per-value maze of scalar branches (with the erf and expm1 bodies in line) was a third of a residual block's time
     if (a.bias) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) v[i] += bia[i];
@@ -987,7 +988,7 @@ struct MimiLinArgs {
 // (N = 64): norm + linear 8.4 -> 6.3, K = 2048 9.6 -> 6.9; a file's 258 columns: K = 512 7.9 -> 6.2, K = 2048 19.2 -> 13.0 (norm + linear: k_mimi_lin_rows).
 // Bound by latency: one column tile has M / 16 workgroups of 16 KB - 64 KB of weights and a few hundred cycles of matrix work each.  Hence
 // 16-wide tiles (a live stream has two columns: a 32-wide tile keeps the matrix core busy four times as long, 1.7 us at K = 512, on half the
-// CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (KJ fragments per wave), and
+// CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (U fragments per wave), and
 // no reduction split over workgroups (K = 2048 needed a second launch to add the sums).
 template <int FM, int FN, int U, bool LN, bool NT>
 __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
@@ -1863,7 +1864,7 @@ __global__ void k_mimi_group_ring(const float* __restrict__ kvn, float* __restri
 // ------------------------------------------------------------------------------------------------
 // Distances are evaluated in fp64 (||e||^2 - 2 x.e; the ||x||^2 term is constant per row), i.e. the exact
 // nearest centroid of the fp32 inputs, lowest index on ties - the answer the reference's fp32 cdist
-// agrees with except at ~1e-7-relative near-ties (SURVEY.md Appendix D).
+// agrees with except at ~1e-7-relative near-ties.
 #define MMI_RVQ_CHUNK 32
 // One level of one half of the split quantiser.  A launch carries two of them (grid.z picks): the semantic quantiser's only level and the
 // acoustic quantiser's first level work on different halves of the projected latent and do not depend on each other

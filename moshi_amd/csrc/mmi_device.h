@@ -262,7 +262,7 @@ __device__ __forceinline__ f32x4 mmi_mfma_fp8_16x16x32(u32x2 a, u32x2 b, f32x4 c
     return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b), c, 0, 0, 0);
 }
 
-// ---- int8 x int8 on the matrix core (BASELINE configs[4]: the reference's bitsandbytes int8 matmul, utils/quantize.py:24-40) ----
+// ---- int8 x int8 on the matrix core (the reference's bitsandbytes int8 matmul, utils/quantize.py:24-40) ----
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 // D(32x32) += A(32x32) * B(32x32), int8 in / int32 acc (v_mfma_i32_32x32x32_i8): 16 bytes per operand per lane.  Both operands
@@ -287,7 +287,7 @@ __device__ __forceinline__ float mmi_rint(float x) { return __builtin_rintf(x); 
 // "Last arriver finishes" inside one launch (k_lm_attn_wave's ring split): a workgroup publishes its partial result with plain
 // stores, then ONE lane releases at agent scope (L2 write-back), drains, and bumps the arrival counter; the workgroup that sees
 // the final count acquires at agent scope (invalidates its CU's L1) and reads the others' partials with plain loads - the
-// producer / consumer forms MI355X_MICROARCH.md lists as valid across XCDs.  Call from ONE thread, between two __syncthreads().
+// producer / consumer form that is valid across XCDs.  Call from ONE thread, between two __syncthreads().
 __device__ __forceinline__ unsigned mmi_arrive_release(unsigned* counter) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (the compiler may drop the fence's own wait: keep one it cannot see through)

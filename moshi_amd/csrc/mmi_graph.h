@@ -100,7 +100,7 @@ struct MmiProgram {
         return MMI_OK;
     }
 
-    // Variant v made ready AHEAD of the step that first needs it (ADVICE r4: a stream whose rings grow past the short-ring program
+    // Variant v made ready AHEAD of the step that first needs it (a stream whose rings grow past the short-ring program
     // would otherwise capture and instantiate the other program in the middle of a live session - a one-off latency spike in a
     // real-time stream): its graph(s) captured and instantiated now, nothing launched.  split: the two-graph form run_split uses.
     int precapture(int v, hipStream_t capture_stream, bool split, size_t cut) {

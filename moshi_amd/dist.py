@@ -1,4 +1,4 @@
-"""Weight replication at load for the one-process-per-GPU deployment (SURVEY.md 8e): rank `src` holds the state dict
+"""Weight replication at load for the one-process-per-GPU deployment: rank `src` holds the state dict
 (read from disk, or drawn), every other rank receives it through `torch.distributed` - backend "nccl" is RCCL over xGMI on
 MI355X nodes, "gloo" in the CPU tests.  This is the ONLY collective of the engine: the frame step itself shards by
 session and never communicates.
@@ -17,7 +17,7 @@ Spec = Sequence[Tuple[str, Tuple[int, ...], str]]
 # What the replication cost on THIS rank, accumulated over every broadcast_state_dict call of the process: bytes that went through
 # the collective, seconds inside it (device-synchronised around each bucket), buckets.  bench.py prints it per rank, next to the
 # rank's PCI bus id, so that the first real multi-GPU run says by itself whether RCCL saw N ranks and at what rate the weights
-# crossed xGMI (VERDICT r4 item 8).
+# crossed xGMI.
 BROADCAST_STATS = {"bytes": 0, "seconds": 0.0, "buckets": 0, "world": 1}
 
 

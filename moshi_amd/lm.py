@@ -92,12 +92,12 @@ class LMModel:
     """Weights + architecture of the Moshi LM on the engine (reference: lm.py:49-320).
 
     Args:
-        state_dict: bf16 tensors named as in the reference checkpoints.
+        state_dict: bf16 tensors named as in the reference checkpoints (lm.py:135-232).
         config: architecture hyper-parameters (defaults = Moshi-7B, loaders.py:90-119).
         device: a ROCm `cuda` device for the product library.
         max_batch: largest number of concurrent sessions `LMGen.streaming` will be asked for.
         quantize: True converts the linears to row-wise int8 (`weight` + `weight_scb`), like the reference's `quantize=True`;
-            "fp8" converts them to e4m3fn (`weight` + `weight_scale`) for the fp8 MFMA path (BASELINE configs[4]);
+            "fp8" converts them to e4m3fn (`weight` + `weight_scale`) for the fp8 MFMA path;
             a state dict that already carries int8 / fp8 weights is used as is.
     """
 
@@ -220,7 +220,7 @@ class LMModel:
             return c.card
         raise KeyError(weight_name)
 
-    # attributes callers read (SURVEY.md 8b)
+    # attributes callers read
     @property
     def dep_q(self) -> int:
         return self.config.dep_q
@@ -283,7 +283,7 @@ class LMModel:
         return self.config.existing_text_padding_id
 
     # lm.py:176-183 builds a ConditionProvider from the checkpoint's `conditioners`; turning attributes (a speaker wav, a text
-    # description) into tensors is not on the frame step and is out of scope here (DESIGN.md 9).  Callers that branch on
+    # description) into tensors is not on the frame step and is out of scope here.  Callers that branch on
     # `lm.condition_provider is not None` (run_inference.py:38, tts.py:449-460) see None and pass `condition_tensors` to LMGen.
     condition_provider = None
 

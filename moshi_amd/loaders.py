@@ -1,5 +1,5 @@
 """Checkpoint loading for the engine: same function names, arguments and file formats as the reference's
-`moshi.models.loaders` (moshi/moshi/models/loaders.py:145-446; SURVEY.md 8f-2), minus the Hugging Face download
+`moshi.models.loaders` (moshi/moshi/models/loaders.py:145-446), minus the Hugging Face download
 (there is no network path in the engine: `hf://` names must already be local files).
 
     mimi = loaders.get_mimi("tokenizer-e351c8d8-checkpoint125.safetensors", device="cuda", num_codebooks=8)
@@ -42,7 +42,7 @@ def hf_get(filename: str | Path, hf_repo: str | None = None, check_local_file_ex
            revision: str | None = None) -> Path:
     """loaders.py:122-142 without the download: a Path, a `file://` name or a plain name is returned as a local path exactly as
     the reference does; a name that the reference would fetch (`hf://...`, or a bare name with `hf_repo` that is not already a
-    local file) raises - the engine has no network path (section 9 of DESIGN.md)."""
+    local file) raises - the engine has no network path."""
     if isinstance(filename, Path):
         return filename
     if filename.startswith("file://"):

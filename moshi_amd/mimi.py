@@ -50,7 +50,7 @@ class MimiModel:
     """Mimi codec running on the MI355X engine.
 
     Args:
-        state_dict: tensors named as in the reference checkpoints, fp32.
+        state_dict: tensors named as in the reference checkpoints (loaders.py:356-358), fp32.
         config: architecture hyper-parameters.
         device: where the tensors and the engine live (a ROCm `cuda` device for the product library).
         max_batch: largest streaming batch this instance will be asked for.

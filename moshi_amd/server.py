@@ -1,4 +1,4 @@
-"""Websocket front end for many live full-duplex sessions on one GPU (SURVEY.md 8f-1 / 8f-4).
+"""Websocket front end for many live full-duplex sessions on one GPU.
 
 The reference's Python server (moshi/moshi/server.py:73-169) serves ONE session under a lock; its Rust server batches.  This is
 the Python server's wire behaviour - the binary protocol of rust/protocol.md:1-31, handshake first, audio in / audio + text

@@ -1,5 +1,5 @@
 """State-dict layout of the two models (names/shapes exactly as the reference checkpoints carry them,
-SURVEY.md Appendix A; reference: seanet.py:169-236,315-388, transformer.py:407-418, vq.py:76-84,
+reference: seanet.py:169-236,315-388, transformer.py:407-418, vq.py:76-84,
 core_vq.py:158-160, lm.py:135-232) and seeded synthetic weights of that layout.
 
 There is no network and no released checkpoint in this environment, so benchmarks and parity tests use
@@ -316,7 +316,7 @@ E4M3_MAX = 448.0
 
 
 def quantize_lm_state_dict_fp8(sd: Dict[str, torch.Tensor], input_scale: float = 1.0) -> Dict[str, torch.Tensor]:
-    """fp8 linears for the fp8 MFMA path (BASELINE.json configs[4]): per-output-row scaling, `weight` =
+    """fp8 linears for the fp8 MFMA path: per-output-row scaling, `weight` =
     e4m3fn(W / weight_scale) with weight_scale = absmax_row / 448 (fp32, `<key>_scale`), and a static scalar activation
     scale `<linear>.input_scale` (a calibration constant; powers of two cost no precision).  W ~= weight * weight_scale."""
     out: Dict[str, torch.Tensor] = {}

@@ -77,7 +77,7 @@ class QWeight:
       (1 in 36 608 codes in tests/test_oracle_pinned.py::test_int8_rule_agrees_with_a_torch_restatement_of_the_library_ops).  Two deliberate differences, both no-ops in range:
       `x.half()` (bf16 -> fp16 is exact for |x| in [2^-14, 65504]; smaller values quantise to 0 either way) is skipped, and
       the result is rounded to the engine's activation type bf16 where bnb returns fp16.
-    * act8 = False - weight-only dequantisation (activations stay bf16; the engine's `MMI_Q8_ACT=bf16` mode, rounds 1-3)."""
+    * act8 = False - weight-only dequantisation (activations stay bf16; the engine's `MMI_Q8_ACT=bf16` mode)."""
 
     def __init__(self, q: np.ndarray, scb: np.ndarray):
         self.q = q.astype(f32)
@@ -481,7 +481,7 @@ class LMOracle:
             return np.zeros((self.gen_B, 0), np.int64), np.zeros((self.gen_B, 0, c.card), f32)
         return np.stack(tokens, 1), np.stack(logits_all, 1)
 
-    # ---- LMGen._step (lm.py:668-783; SURVEY.md Appendix B5) ---------------------------------------------
+    # ---- LMGen._step (lm.py:668-783) ---------------------------------------------
     def step(self, user_codes: np.ndarray, use_sampling: bool = False, temp: float = 0.8, temp_text: float = 0.7,
              top_k: int = 250, top_k_text: int = 25, noise: Optional[np.ndarray] = None,
              forced: Optional[np.ndarray] = None, support_out_of_sync: bool = False):

@@ -230,7 +230,7 @@ class TransformerLayer:
 
 def cdist_argmin(x: np.ndarray, E: np.ndarray) -> np.ndarray:
     """EuclideanCodebook._quantize (core_vq.py:270-276): torch.cdist takes ATen's `_euclidean_dist` matmul form
-    sqrt(clamp([-2x, |x|^2, 1] . [e, 1, |e|^2]^T, 0)) (SURVEY.md Appendix D); argmin = first minimum."""
+    sqrt(clamp([-2x, |x|^2, 1] . [e, 1, |e|^2]^T, 0)); argmin = first minimum."""
     x = x.astype(f32)
     x_norm = (x * x).sum(-1, keepdims=True, dtype=f32)
     e_norm = (E * E).sum(-1, keepdims=True, dtype=f32)

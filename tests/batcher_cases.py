@@ -1,6 +1,6 @@
 """Cases for the session batcher (moshi_amd/csrc/batcher.hip) shared by the simulator tests (CPU) and the GPU tests.
 
-What is pinned here is the model loop of SURVEY.md 8f-1 (rust/moshi-server/src/batched_asr.rs:188-437; server.py:132-146,
+What is pinned here is the model loop (rust/moshi-server/src/batched_asr.rs:188-437; server.py:132-146,
 163-164): which rows run, which are reset, what reaches which channel.  The arithmetic of the rows themselves is pinned
 against the oracle / the reference golden vectors by the Mimi and LM cases; here the batcher is compared bit for bit with
 the same schedule driven by hand through `MimiModel` / `LMGen` (the reference's own API).

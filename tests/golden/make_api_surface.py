@@ -1,5 +1,5 @@
 """Writes tests/golden/api_surface.json: the PUBLIC Python surface of the reference's MimiModel, LMModel and LMGen (the drop-in
-boundary of SURVEY.md 8b) - every public attribute of the class that torch.nn.Module does not already have, with the parameter
+boundary) - every public attribute of the class that torch.nn.Module does not already have, with the parameter
 names of the callables - obtained by importing the reference in this container:
 
     cd /tmp && PYTHONPATH=/root/reference/moshi NO_TORCH_COMPILE=1 PYTHONDONTWRITEBYTECODE=1 python /root/repo/tests/golden/make_api_surface.py

@@ -75,7 +75,7 @@ def gen_mimi_full(loaders):
     g = torch.Generator().manual_seed(5)
     t = torch.arange(cfg.frame_size * F) / cfg.sample_rate
     x = 0.2 * torch.randn(B, 1, cfg.frame_size * F, generator=g)
-    x[1, 0] += 0.5 * torch.sin(2 * torch.pi * 440.0 * t)           # a sine row, as in SURVEY.md C1/C2
+    x[1, 0] += 0.5 * torch.sin(2 * torch.pi * 440.0 * t)           # a sine row
     lat, codes, pcm = [], [], []
     with torch.no_grad(), ref.streaming(B):
         for f in range(F):
@@ -84,7 +84,7 @@ def gen_mimi_full(loaders):
             c = ref.quantizer.encode(l)
             p = ref.decode(c)
             lat.append(l.numpy()); codes.append(c.numpy()); pcm.append(p.numpy())
-    # non-streaming encode of the same signal must give the same codes
+    # non-streaming encode of the same signal must give the same codes (as the reference's do)
     with torch.no_grad():
         c_batch = ref.encode(x).numpy()
     out = {"x": x.numpy(), "latent": np.stack(lat), "codes": np.stack(codes), "pcm": np.stack(pcm),

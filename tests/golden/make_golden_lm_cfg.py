@@ -1,4 +1,4 @@
-"""Golden vectors for `LMGen.step` with classifier-free guidance, sum-conditioning and extra heads (SURVEY.md 8f-3 / 8f-4),
+"""Golden vectors for `LMGen.step` with classifier-free guidance, sum-conditioning and extra heads,
 produced by RUNNING THE REFERENCE (build container only: `python tests/golden/make_golden_lm_cfg.py`).
 
 lm_cfg.npz - tiny Moshi LM (moshi_amd.config.tiny_lm_config), bf16, seeded weights re-drawn from the stored seed, B=2, greedy,

@@ -1,4 +1,4 @@
-"""Golden vectors for `LMGen.step` on a model with cross-attention layers (second half), produced by RUNNING THE
+"""Golden vectors for `LMGen.step` on a model with cross-attention layers, produced by RUNNING THE
 REFERENCE (build container only: `python tests/golden/make_golden_lm_cross.py`).
 
 lm_cross.npz - tiny Moshi LM with `cross_attention=True` (every temporal layer: self-attention, then

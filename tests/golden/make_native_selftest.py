@@ -1,5 +1,5 @@
 """Writes tests/golden/native_selftest/{manifest.txt,expected.bin}: what scripts/native_selftest.cpp needs to check an installed
-libmoshi_mi.so on a GPU box WITHOUT Python - a tiny Mimi and a tiny Moshi LM whose weights and inputs both sides generate from the
+libmoshi_mi.so on a GPU WITHOUT Python - a tiny Mimi and a tiny Moshi LM whose weights and inputs both sides generate from the
 same integer hash (so no weight file travels), and the outputs the numpy ORACLE (oracle/, test infrastructure) computes for them.
 
     python tests/golden/make_native_selftest.py

@@ -18,7 +18,7 @@ GOLDEN = Path(__file__).resolve().parent / "golden"
 # Yardstick: the distance between two CORRECT implementations of this bf16 model on the same inputs - the reference's PyTorch
 # CPU path (the golden vectors) and the numpy oracle - is max 3.12 % / mean 0.90 % of max|logit| in the worst of 162 (row,
 # site) pairs (median 1.2 % / 0.4 %): pure bf16 rounding-order noise through 2 + 8 x 2 transformer layers (the reviewer of
-# round 4 measured the reference moving 1.2 % against ITSELF between two hosts).  The gate is that distance x 1.6 (max) and
+# the reference was measured moving 1.2 % against ITSELF between two hosts).  The gate is that distance x 1.6 (max) and
 # x 1.33 (mean): above the yardstick, because an engine is a third correct implementation and cannot be asked to sit closer to
 # the reference than the checker does, and below twice the yardstick - tests/test_oracle_pinned.py
 # (test_bf16_logit_gate_is_under_twice_the_distance_between_two_correct_implementations) re-measures the yardstick and holds
@@ -52,7 +52,7 @@ _SD_CACHE: "dict" = {}
 def cached_lm_state_dict(cfg, seed: int, keep: int = 2):
     """`random_lm_state_dict(cfg, seed)` (the CPU draw the golden generators and every earlier measurement used), kept for the
     next test that asks for the same (architecture, seed): drawing ~1 B parameters on the host is 10 s of each full-width test,
-    and the GPU suite has a time budget (VERDICT r4 weak 3).  The tensors are shared: callers must not modify them."""
+    and the GPU suite has a time budget.  The tensors are shared: callers must not modify them."""
     key = (repr(cfg), int(seed))
     if key not in _SD_CACHE:
         while len(_SD_CACHE) >= keep:
@@ -166,7 +166,7 @@ def check_golden_wide(device, lib):
 # implementations - is worst max 6.10 % / mean 1.15 % of max|logit| (parity_golden_full_oracle); gate = yardstick x 1.5 = 9.2 %
 # -> FULL_WIDEN = 9.2 / 5 (mean: 1.2 % x 1.85 = 2.2 %, x 1.9 the yardstick's mean); tests/test_oracle_pinned.py re-measures the
 # yardstick and holds the gate inside [1 x, 2 x) of it.  The engine on MI355X against the same file: worst max 4.85 % / mean
-# 1.09 % (text head 2.30 % / 0.44 %; profiles/r05_logs/parity_golden_full_cuda.json; round 3: 5.77 % / 1.13 %) - inside the yardstick.
+# 1.09 % (text head 2.30 % / 0.44 %; profiles/r05_logs/parity_golden_full_cuda.json) - inside the yardstick.
 FULL_WIDEN = 1.85
 
 
@@ -216,7 +216,7 @@ def check_golden_full(device, lib, max_batch=None, name=None):
 
 
 def check_free_running(device, lib, g, cfg, widen, name, max_batch=None, on_cuda_weights=False, sd=None):
-    """NOT teacher-forced (VERDICT r3 2c): the engine runs greedy on its own tokens through a golden run of the reference - what
+    """NOT teacher-forced: the engine runs greedy on its own tokens through a golden run of the reference - what
     it samples at step s is what it reads at step s + 1.  Per row, the first (step, site) where its token differs from the
     reference's is reported, and it must be a near-tie of the REFERENCE's logits at that site (all inputs up to there were
     identical, so those logits are comparable); from there on the row is on another trajectory and is not compared (until a
@@ -342,7 +342,7 @@ def oracle_vs_engine(device, lib, cfg, seed, B, S, use_masks=True, quantize=Fals
     if quantize is True and int8_activations:      # int8 x int8 linears: per-linear bit equality + a statistical network gate (below)
         return int8_network_vs_oracle(device, lib, cfg, seed, B, S, use_masks=use_masks, stats=stats)
     sd = cached_lm_state_dict(cfg, seed)
-    if quantize == "fp8":   # e4m3fn linears on the fp8 MFMA (BASELINE configs[4]); engine and oracle get the same fp8 tensors
+    if quantize == "fp8":   # e4m3fn linears on the fp8 MFMA; engine and oracle get the same fp8 tensors
         from moshi_amd.weights import quantize_lm_state_dict_fp8
         sd = quantize_lm_state_dict_fp8(sd, input_scale=input_scale)
     elif quantize:  # row-wise int8 linears (the reference's `quantize=True` storage); engine and oracle get the same int8 tensors
@@ -488,7 +488,7 @@ def full_depth_vs_oracle(device, lib, B=32, S=3, num_layers=32, seed=4242, name=
     cfg = cfg or LMConfig(num_layers=num_layers)
     sd = random_lm_state_dict(cfg, seed=seed, device=device)
     gen = make_engine(cfg, sd, device, lib, B, use_sampling=False, support_out_of_sync=True)
-    gen.lm_model.enable_hidden_taps()              # the residual stream after temporal layers 0 and num_layers - 1 (VERDICT r3 2d)
+    gen.lm_model.enable_hidden_taps()              # the residual stream after temporal layers 0 and num_layers - 1
     hid, hid_yard = HiddenLog(), HiddenLog()
     lazy = lazy_temporal_linears(sd)
     orc = LMOracle(lazy, replace(cfg, context=64))
@@ -641,7 +641,7 @@ def smoke_lm(dev):
     print("smoke: LMGen.step ring outputs identical to the oracle, logits within tolerance")
 
 
-# ---- classifier-free guidance, sum-conditioning, extra heads (SURVEY.md 8f-3 / 8f-4; tests/golden/lm_cfg.npz) -------------------
+# ---- classifier-free guidance, sum-conditioning, extra heads (tests/golden/lm_cfg.npz) -------------------
 CFG_SCENARIOS = {
     "a": dict(cfg_coef=2.0, masked_until=True),
     "b": dict(cfg_coef=1.5, cfg_is_no_text=True),
@@ -735,7 +735,7 @@ def check_cfg_engine(device, lib, name):
             state["gen"]._stop_streaming()
 
 
-# ---- cross-attention conditioning (second half; tests/golden/lm_cross.npz) -----------------------------------------
+# ---- cross-attention conditioning (tests/golden/lm_cross.npz) -----------------------------------------
 CROSS_SCENARIOS = {
     "e": dict(cfg_coef=1.0, cross=["cross_e"], sum="sum_e"),
     "f": dict(cfg_coef=2.0, cross=["cross_f1", "cross_f2"], pos_emb=0.5),
@@ -1083,7 +1083,7 @@ def check_topk_device_rng(device, lib, cfg=None, top_k=20, top_k_text=10, steps=
     assert near[0] <= 2, f"{near[0]} sampled tokens sat on a near-tie of the two best scores"
 
 
-# ---- C5, per linear, bit for bit ("the int8 GEMM is integer work") ------------------------------------------------
+# ---- int8 x int8, per linear, bit for bit (the int8 GEMM is integer work) ------------------------------------------------
 # `QLinear.forward` (utils/quantize.py:24-40) of ONE module on the same bf16 rows, engine (`mmi_lm_debug_linear`: the kernels the
 # step uses) against the oracle's restatement of bitsandbytes' rule: the int8 codes, the row absmax and the bf16 output must be
 # IDENTICAL - row-wise quantisation, an exact int32 dot product and one fp32 expression `out32 * (SCA * SCB) * (1 / 127^2)` leave
@@ -1180,14 +1180,14 @@ def int8_linears_bit_exact(device, lib, cfg, B, seed, report=None, weights_seed=
     return checked
 
 
-# ---- C5 at network level: a statistical gate with a yardstick ------------------------------------------------------
+# ---- int8 x int8 at network level: a statistical gate with a yardstick ------------------------------------------------------
 # With every int8 linear bit-identical to the oracle for the same input rows (int8_linears_bit_exact), engine and oracle can
 # only part ways at the pieces that are NOT integer work - RMSNorm's mean of squares and rsqrt, the softmax of the attentions,
 # SiLU, RoPE - where summation order / the device's exp move a bf16 result by one rounding flip now and then.  Re-quantising
 # every activation row to 8 bits is a discontinuous map: most flips vanish (the int8 codes do not change: the (row, site) pair
 # is bit-identical to the oracle), a few are carried to the logits, and a flip of a row's absmax entry moves the whole row.  The
 # error per (row, site) is therefore heavy-tailed, and a threshold on its MAXIMUM over a few thousand pairs is a coin that
-# eventually lands wrong - it did, at the driver, in round 4.  The gate: (1) token-ring outputs exact under teacher forcing;
+# eventually lands wrong - it did.  The gate: (1) token-ring outputs exact under teacher forcing;
 # (2) the share of pairs inside the plain bf16 tolerance, the median and the 90th percentile of the error are no worse than
 # those of ANOTHER correct implementation of the same network (the oracle with its norm / softmax / SiLU statistics in fp64,
 # `LMOracle(stat64=True)`), with a margin; (3) no pair is grossly wrong (a broken kernel gives errors of order max|logit|).
@@ -1279,7 +1279,7 @@ def int8_network_vs_oracle(device, lib, cfg, seed, B, S, use_masks=True, name=No
     return res
 
 
-# ---- C5 against the PINNED reference ("C5 parity = against the bf16 oracle with a stated quantisation tolerance") ------
+# ---- int8 x int8 against the PINNED reference: the bf16 oracle with a stated quantisation tolerance ------
 # The int8 rule itself cannot be pinned (bitsandbytes is not in /root/reference and cannot run here), but the distance of the int8
 # ENGINE to the reference's own bf16 logits can be measured: the goldens lm_wide.npz (7B layer shapes, 1 temporal layer) and
 # lm_full.npz (the benchmark model, 32 layers) are outputs of the reference itself.  The int8 network is a different function than
@@ -1352,7 +1352,7 @@ def int8_engine_vs_bf16_reference(device, lib, which="wide", max_batch=None, nam
 
 # ---- the step is a function of its inputs: two streams of one handle fed the same frames produce the same bits ----------------------
 def reproducible_between_streams(device, lib, cfg, B, quantize=False, steps=3, repeats=4, seed=77, before_repeat=None, guided_cross=None):
-    """Round 5's root cause (the driver's round-4 failure) was a launch whose output changed from run to run; what caught it was
+    """What once failed here was a launch whose output changed from run to run; what caught it was
     comparing runs, not comparing with the checker.  Greedy, masks and a partial reset, hidden taps on: every repeat must equal the
     first in tokens, text / audio logits and the residual stream after the first and the last temporal layer, bit for bit."""
     sd = cached_lm_state_dict(cfg, seed)

@@ -81,7 +81,7 @@ def check_full_against_golden(model_factory, device, frames=None):
             assert np.array_equal(c, g["codes"][f]), f"RVQ indices differ on the reference latent at frame {f}"
             p = m.decode(torch.from_numpy(g["codes"][f]).to(device)).cpu().numpy()
             assert close(p, g["pcm"][f], PCM_ATOL, PCM_RTOL), f"pcm differs at frame {f}"
-    # end to end, the product call itself: encode(pcm) codes against the reference's codes, directly (VERDICT r3 2b).  The
+    # end to end, the product call itself: encode(pcm) codes against the reference's codes, directly.  The
     # engine's latent differs from the reference's in the last bits (summation order), so an index may legitimately flip at a
     # near-tie of the reference's own distances: the match rate is printed and every mismatch audited on the golden latent.
     mism = []
@@ -155,10 +155,10 @@ def oracle_vs_engine(model_factory, device, cfg, seed, B, F, K, use_masks=True):
 
 
 def check_c2_recipe(model_factory, device, cfg, B=8, F=200, K=8, seed=0, p_exec=0.5, max_flips=2, oracle_rows=None):
-    """SURVEY.md 8d's C2 recipe against the oracle: B streams of 0.1 * N(0, 1) PCM plus a sine row, F frames, a random exec
+    """A long recipe against the oracle: B streams of 0.1 * N(0, 1) PCM plus a sine row, F frames, a random exec
     mask per frame and ONE mid-run `reset_streaming(mask)`.  Row 0 always executes and row 1 executes nine frames in ten, so
     that at the full size (context 250, two positions per frame) their KV rings WRAP inside the run (frame 126 for row 0):
-    the state the benchmark runs in and, before round 4, no full-size parity test reached (transformer.py:236-288).  Codes
+    the state the benchmark runs in and no other full-size parity test reaches (transformer.py:236-288).  Codes
     equal on executed rows (near-tie flips audited, at most `max_flips` vectors), PCM of the oracle's codes within 2e-5.
     oracle_rows: the engine runs all B streams, the (slow, numpy) checker only these rows of the batch - streams are independent
     (`test_batch_rows_are_independent_and_graph_equals_eager`), and the GPU suite has a time budget; default: every row."""

@@ -37,13 +37,13 @@ def test_full_size_matches_oracle(factory):
 
 
 def test_full_size_c2_recipe_crosses_the_ring_wrap(factory):
-    """SURVEY.md 8d C2: 8 streams, 200 frames, random exec masks, one mid-run reset - the 250-slot rings of the codec's
-    transformers wrap at frame 126 (the state bench.py runs in, never parity-tested at full size before)."""
+    """8 streams, 200 frames, random exec masks, one mid-run reset - the 250-slot rings of the codec's
+    transformers wrap at frame 126 (the state bench.py runs in)."""
     import json
     from pathlib import Path
     # the engine runs the 8 streams; the numpy checker follows three of them (the always-executing row whose rings wrap at frame
     # 126, the nine-in-ten row (wraps ~140), the sine row, which is also reset mid-run) for 160 frames: ~85 s instead of 210 in a
-    # suite with a time budget (four rows: 114 s on MI355X in round 5)
+    # suite with a time budget (four rows: 114 s on MI355X)
     res = mimi_cases.check_c2_recipe(factory, DEV, MimiConfig(), B=8, F=160, oracle_rows=[0, 1, 7])
     assert res["wrapped"]
     out = Path(__file__).resolve().parent.parent / "gpurun_out"
@@ -54,7 +54,7 @@ def test_full_size_c2_recipe_crosses_the_ring_wrap(factory):
 def test_rvq_indices_bit_exact_on_many_vectors(factory):
     """131 072 index decisions (4096 latents x 32 levels) against the oracle's fp32 cdist restatement.
     The engine evaluates distances in fp64, i.e. it returns the exact nearest centroid; the fp32 reference formula
-    can only disagree with that at a near-tie below its own resolution (SURVEY.md Appendix D: relative gaps down to
+    can only disagree with that at a near-tie below its own resolution (relative gaps down to
     3e-6 occur about once in 1e5 decisions).  Any disagreement is therefore audited in fp64: it must be such a
     near-tie AND the engine must hold the exact argmin."""
     from oracle.mimi_oracle import MimiOracle
@@ -68,7 +68,7 @@ def test_rvq_indices_bit_exact_on_many_vectors(factory):
     co = orc.quantize(lat)
     assert ce.shape == co.shape == (64, 32, 64)
     bad = np.argwhere((ce != co).any(1))
-    # the observed count goes on record (VERDICT round 1): printed, and written next to the other parity summaries
+    # the observed count goes on record: printed, and written next to the other parity summaries
     n_dec = int((ce != co).sum())
     print(f"[parity] rvq_indices: {len(bad)} of 4096 vectors ({n_dec} of {ce.size} index decisions) differ from the fp32 cdist restatement")
     import json
@@ -122,7 +122,7 @@ def test_batch_rows_are_independent_and_graph_equals_eager(factory, monkeypatch)
 def test_codec_is_bit_reproducible_between_streams(factory, B):
     """The full-size codec at the C2 batch (8 streams) and the benchmark batch (32): three frames encoded and decoded, then four
     more streams on the SAME handle fed the same PCM - codes and PCM bit for bit equal to the first stream's (a launch that is not
-    a function of its inputs - round 4's LM failure - is the one bug class a tolerance against the checker cannot see)."""
+    a function of its inputs is the one bug class a tolerance against the checker cannot see)."""
     cfg = MimiConfig()
     sd = random_mimi_state_dict(cfg, seed=1234)
     g = torch.Generator().manual_seed(19 + B)
@@ -144,7 +144,7 @@ def test_codec_is_bit_reproducible_between_streams(factory, B):
 
 
 def test_round_trip_sine_c1(factory):
-    """BASELINE.json configs[0] restated: 1 s 440 Hz sine, streaming == non-streaming codes, PCM shape."""
+    """1 s 440 Hz sine, streaming == non-streaming codes, PCM shape."""
     cfg = MimiConfig()
     m = factory(random_mimi_state_dict(cfg, seed=1234), cfg, 8, max_batch=1)
     t = torch.arange(24000) / 24000.0

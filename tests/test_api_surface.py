@@ -1,4 +1,4 @@
-"""The drop-in boundary (SURVEY.md 8b): moshi_amd's MimiModel / LMModel / LMGen against the PUBLIC surface of the reference's
+"""The drop-in boundary: moshi_amd's MimiModel / LMModel / LMGen against the PUBLIC surface of the reference's
 classes of the same names, as listed by importing the reference (tests/golden/api_surface.json, written by
 tests/golden/make_api_surface.py).  Every public name of the reference class must exist here with the same kind (method /
 property) and the reference's parameter names in the reference's order (extra trailing optional parameters are allowed); what is
@@ -23,7 +23,7 @@ WAIVED = {
     ("LMModel", "__init__"): "built from a state dict + LMConfig; loaders.get_moshi_lm keeps the reference's factory signature",
     ("LMModel", "forward_text"): "internal to LMGen._step in the reference (lm.py:719); fused into mmi_lm_step",
     ("LMModel", "forward_depformer"): "internal to LMGen.depformer_step (lm.py:835); fused into mmi_lm_step",
-    ("LMModel", "forward_depformer_training"): "training-mode forward: out of scope (DESIGN.md 9)",
+    ("LMModel", "forward_depformer_training"): "training-mode forward: out of scope",
     ("LMModel", "streaming"): _HANDLE + "no caller of the reference streams an LMModel directly",
     ("LMModel", "streaming_forever"): _HANDLE + "see streaming",
     ("LMModel", "reset_streaming"): _HANDLE + "see streaming",
@@ -36,7 +36,7 @@ WAIVED = {
 
 
 LOADERS_WAIVED = {
-    "get_conditioner": "condition PROVIDERS (attributes -> tensors) are not on the frame step (DESIGN.md 9); their output enters as LMGen(condition_tensors=...)",
+    "get_conditioner": "condition PROVIDERS (attributes -> tensors) are not on the frame step; their output enters as LMGen(condition_tensors=...)",
     "get_conditioner_provider": "builds a ConditionProvider out of get_conditioner results: see get_conditioner",
     "get_lora_moshi": "wraps nn.Linear modules in LoRA modules; the engine has no modules - get_moshi_lm(lora_weights=...) merges the adapter at load (loaders.py:486-516 with fuse_lora=True)",
 }
@@ -70,7 +70,7 @@ def test_waivers_name_things_the_reference_has():
 def test_properties_and_caller_read_attributes_on_live_instances(sim_lib):
     """Every reference property reads on an instance, with the reference's values where they are constants of the format
     (lm.py:246-277: initial 2048-style ids = card / text_card, zero -1, ungenerated -2; compression.py:160-190), plus the instance
-    attributes the reference's callers read (SURVEY.md 8b: lm_model.{dep_q, delays, device, card, text_card, num_codebooks})."""
+    attributes the reference's callers read (lm_model.{dep_q, delays, device, card, text_card, num_codebooks})."""
     mcfg, lcfg = tiny_mimi_config(), tiny_lm_config()
     mimi = MimiModel(random_mimi_state_dict(mcfg, seed=1), mcfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
     lm = LMModel(random_lm_state_dict(lcfg, seed=1), lcfg, device="cpu", max_batch=2, lib=sim_lib)

@@ -79,7 +79,7 @@ def test_long_ring_split_over_workgroups_matches_oracle(gpu_lib, monkeypatch, kv
 
 @pytest.mark.parametrize("name", ["a", "b", "c", "d"])
 def test_guidance_conditioning_and_extra_heads_match_reference_golden(gpu_lib, name):
-    """SURVEY.md 8f-3 / 8f-4 on the GPU: classifier-free guidance (masked-until / no-text / condition tensors), a `sum`
+    """On the GPU: classifier-free guidance (masked-until / no-text / condition tensors), a `sum`
     condition and extra heads against the reference's own LMGen runs (tests/golden/lm_cfg.npz)."""
     lm_cases.check_cfg_engine(DEV, None, name)
 
@@ -169,7 +169,7 @@ def test_c5_int8_engine_against_the_reference_at_full_depth(gpu_lib):
 @pytest.mark.parametrize("B", [40, 64])
 def test_two_batch_tiles_at_full_width_match_oracle(gpu_lib, B):
     """33..64 sessions at the 7B layer shapes on the DEFAULT GEMM path (k_gemm_xp with two batch tiles per weight fragment:
-    what BASELINE configs[4] runs at 64 sessions)."""
+    what 64 sessions run on)."""
     cfg = LMConfig(num_layers=2, context=64)
     lm_cases.oracle_vs_engine(DEV, None, cfg, seed=300 + B, B=B, S=2, use_masks=True)
 
@@ -259,7 +259,7 @@ def test_cross_attention_at_full_width_matches_oracle(gpu_lib, B, Tc):
 
 
 def test_attention_program_switch_is_a_graph_launch_not_a_capture(gpu_lib, monkeypatch):
-    """with the ring split over workgroups (< 4 sessions) a stream moves from the short-ring step program to the
+    """With the ring split over workgroups (< 4 sessions) a stream moves from the short-ring step program to the
     deep-ring one after ~768 steps.  Both programs are captured and instantiated at the stream's FIRST step (mmi_lm_stat 1 == 0b11),
     so the step at the switch costs what its neighbours cost (host wall time with a synchronisation per step: no spike), and a
     snapshot restored at a shallow depth goes back to the short-ring program (mmi_lm_stat 2 = the restored offsets' maximum)."""

@@ -1,4 +1,4 @@
-"""Session batcher (SURVEY.md 8f-1) on the CPU kernel simulator: slot allocation, per-row reset, stream masks, routing."""
+"""Session batcher on the CPU kernel simulator: slot allocation, per-row reset, stream masks, routing."""
 import numpy as np
 import pytest
 
@@ -87,7 +87,7 @@ def test_io_threads_push_and_pop_while_the_loop_steps(sim_lib):
 
 
 def test_a_vanished_channel_has_its_own_status(sim_lib):
-    """ADVICE r4: push / pop / close on a channel id that names no open channel return MMI_ERR_NO_CHANNEL, which the binding maps
+    """push / pop / close on a channel id that names no open channel return MMI_ERR_NO_CHANNEL, which the binding maps
     to `UnknownChannel` (a ValueError) - no matching on the message text; a REAL argument error stays a plain ValueError."""
     from moshi_amd.batcher import SessionBatcher
     from moshi_amd.errors import UnknownChannel

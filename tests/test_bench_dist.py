@@ -91,11 +91,11 @@ def test_bench_spawns_its_own_ranks():
     assert out["p50_ms_per_step"] == 6.0 and out["p95_ms_per_step"] == 7.0
     assert out["p50_ms_per_rank"] == [5.0, 6.0] and out["p95_ms_per_rank"] == [6.0, 7.0]
     # per-rank step time beside the job's (rank 0: 0.5 s, rank 1: 0.75 s over 10 steps), and each rank's host thread pinned to
-    # its own block of cores (VERDICT r3 item 7b/c)
+    # its own block of cores
     assert out["ms_per_step_per_rank"] == [50.0, 75.0] and out["ms_per_step"] == 75.0
     cores = out["host_first_core_per_rank"]
     assert len(cores) == 2 and (cores[0] != cores[1] or len(os.sched_getaffinity(0)) < 2)
-    # every rank reports the device it drives and what the weight broadcast at load moved (VERDICT r4 item 8): a first real
+    # every rank reports the device it drives and what the weight broadcast at load moved: a first real
     # N-GPU run shows by itself that the collective saw N ranks, and at what rate
     info = out["ranks"]
     assert [r["rank"] for r in info] == [0, 1] and all(r["bcast_world"] == 2 and r["bcast_gb"] > 0 and r["bcast_buckets"] >= 1 for r in info)

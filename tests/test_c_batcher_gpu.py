@@ -1,4 +1,4 @@
-"""Session batcher (SURVEY.md 8f-1) on a real MI355X: the same schedule cases as on the simulator, through hipGraph replay,
+"""Session batcher on a real MI355X: the same schedule cases as on the simulator, through hipGraph replay,
 pinned staging and the batcher's own stream, plus a full-size Mimi + Moshi-width LM run."""
 import numpy as np
 import pytest

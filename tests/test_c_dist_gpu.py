@@ -1,8 +1,8 @@
 """The engine's one collective on a real device: `broadcast_state_dict` (moshi_amd/dist.py) packs rank 0's weights into flat
-buckets, broadcasts them over RCCL and unpacks views on the receivers.  A 1-GPU box has no second rank, so the test forces the
+buckets, broadcasts them over RCCL and unpacks views on the receivers.  One GPU has no second rank, so the test forces the
 device path at world size 1 (MMI_FORCE_BCAST): the RCCL communicator is created, every bucket goes through `ncclBroadcast`
 (rank 0 -> itself), and in "recv" mode the result is what a receiving rank keeps - the views into the buckets - which must be
-bit-equal to the source.  Peak device memory of the source path: weights + 2 buckets (VERDICT r3 item 7a)."""
+bit-equal to the source.  Peak device memory of the source path: weights + 2 buckets."""
 import datetime
 import socket
 

@@ -1,4 +1,4 @@
-"""Checkpoint loading on the real device (SURVEY.md 8f-2): a released-style directory (config.json + safetensors with the
+"""Checkpoint loading on the real device: a released-style directory (config.json + safetensors with the
 reference's keys) -> CheckpointInfo -> MimiModel / LMModel on cuda:0 through the product library, and the quantised exports
 through the same door.  The models built straight from the state dict are pinned on the oracle / the reference's golden vectors
 by test_b_lm_gpu.py and test_a_mimi_gpu.py; here the loaders must hand the engine exactly the same weights."""

@@ -187,7 +187,7 @@ for name, (res, args) in sorted(_capi.SIGNATURES.items()):
 
 
 def test_every_entry_point_survives_null_arguments(sim_lib, tmp_path):
-    """"Return 0 / a negative status, never throw across the ABI" (SURVEY.md 8b): every entry point called with a NULL handle,
+    """"Return 0 / a negative status, never throw across the ABI": every entry point called with a NULL handle,
     NULL pointers and zero sizes returns - a status < 0 from everything that acts on a handle, 0 from the pure queries
     (`*_batch`, `*_state_bytes`, `*_launch_list`, ...) - and the process is still alive afterwards.  Host code only, so the
     simulator build of the library (the same sources) answers for the product; run in a child process so that a crash is a

@@ -70,7 +70,7 @@ def test_device_clock_stamps_follow_the_pipeline_order(sim_lib):
 
 
 def test_step_rejects_a_batch_that_is_not_the_streaming_batch(sim_lib):
-    """ADVICE round 3: `DuplexStream.step` with fewer rows than the streaming batch must fail like `lm_gen.step` does
+    """`DuplexStream.step` with fewer rows than the streaming batch must fail like `lm_gen.step` does
     (AssertionError, lm.py:679-682) instead of encoding rows it was never given; the C entry refuses it on its own too."""
     import ctypes as C
     import torch
@@ -96,7 +96,7 @@ def test_step_rejects_a_batch_that_is_not_the_streaming_batch(sim_lib):
 
 
 def test_the_callers_input_buffer_may_be_refilled_in_place(sim_lib):
-    """the frame's input is copied into the pipeline's ring in stream order, so a caller that reuses ONE
+    """The frame's input is copied into the pipeline's ring in stream order, so a caller that reuses ONE
     preallocated input tensor (safe with `mimi.encode`) gets the same bits as one that hands over a fresh tensor per frame."""
     import numpy as np
     import torch
@@ -132,7 +132,7 @@ def test_the_callers_input_buffer_may_be_refilled_in_place(sim_lib):
 
 
 def test_a_hooked_lmgen_is_refused(sim_lib):
-    """ADVICE round 3: LMGen's hooks work on the caller's stream while the pipeline steps the LM on its own - refused
+    """LMGen's hooks work on the caller's stream while the pipeline steps the LM on its own - refused
     (NotImplementedError) rather than racing; without hooks the same objects run."""
     import torch
     from moshi_amd.duplex import DuplexStream
@@ -184,7 +184,7 @@ def _replica(rank, out):
 
 
 def test_eight_replicas_in_eight_processes_stay_bit_identical_under_contention(sim_lib):
-    """the pipeline's gate is a host wait, so N ranks on one node are N host threads competing for cores.
+    """The pipeline's gate is a host wait, so N ranks on one node are N host threads competing for cores.
     Eight processes, each with its own simulator-backed DuplexStream over the same seeded session group, oversubscribing this
     machine's cores: every replica must produce the very same tokens and PCM as the serial loop run alone."""
     import hashlib

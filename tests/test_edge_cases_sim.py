@@ -1,4 +1,4 @@
-"""Edge cases of the streaming control surface (SURVEY.md a18: `set_exec_mask`, `reset_streaming(mask | None)`, `streaming(B)`)
+"""Edge cases of the streaming control surface (`set_exec_mask`, `reset_streaming(mask | None)`, `streaming(B)`)
 against the numpy oracle, on the simulator: a step in which NO row executes, a reset before the first step, a reset of every row
 (`None`) in mid-run, a reset of a row that does not execute in that step, the same handle streaming a second time with another
 batch size, several frames through one codec call under a mask.  The seeded cases of tests/{mimi,lm}_cases.py always keep row 0
@@ -140,7 +140,7 @@ def test_lm_control_surface_edges_match_the_oracle(sim_lib):
 
 
 def test_maximum_batch_sizes(sim_lib):
-    """The largest batch a handle takes (64 sessions per GPU: BASELINE configs[4]) against the oracle, and what lies beyond it is
+    """The largest batch a handle takes (64 sessions per GPU) against the oracle, and what lies beyond it is
     refused loudly at construction / at the first plan, with a message that names the limit - never computed wrongly."""
     cfg = tiny_lm_config()
     lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=164, B=64, S=2)

@@ -1,4 +1,4 @@
-"""INTEGRATION.md section 2 promises a binding "a maintainer of the reference would add".  examples/reference_side_binding.py IS
+"""The integration guide promises a binding "a maintainer of the reference would add".  examples/reference_side_binding.py IS
 that binding (ctypes + torch, nothing of moshi_amd imported); here it runs - on the simulator build of the library - from the
 reference's own configuration dictionaries and state-dict keys, and must give, bit for bit, what moshi_amd's classes give."""
 import importlib.util

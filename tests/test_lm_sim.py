@@ -95,7 +95,7 @@ def test_gemm_with_the_whole_slice_requested_at_once(sim_lib, monkeypatch, B, ti
 def test_attention_ring_split_over_several_workgroups(sim_lib, monkeypatch, kernel):
     """Fewer (session, head) pairs than CUs (one real-time session: 32 pairs): the ring is shared out over several workgroups
     per pair and their partial (max, sum, output) merged by k_lm_attn_combine - forced here on the tiny model, for the
-    barrier-free kernel of round 4 ("wave") and the chunked one it replaces ("split").  The wave kernel's other paths
+    barrier-free kernel ("wave") and the chunked one it replaces ("split").  The wave kernel's other paths
     (lm_engine.hip attn_variant): "wave-solo" = rings of up to MMI_ATTN_SOLO rows, workgroup 0 alone and no merge at all;
     "wave-switch" = the engine changes from that step program to the one with the merge launch when its host-side bound on the
     ring depth passes the threshold (here after 4 of the 9 steps); "wave-kernel" = the merge done by the last workgroup to
@@ -168,7 +168,7 @@ def test_depformer_attention_launch_at_micro_step_0_is_optional(sim_lib, monkeyp
 
 @pytest.mark.parametrize("B,grid,mode", [(18, 8, "1"), (34, 8, "1"), (20, 64, "1"), (18, 8, "2"), (34, 8, "2"), (18, 5, "2"), (18, 7, "1")])
 def test_gemm_with_activations_resident_in_lds(sim_lib, monkeypatch, B, grid, mode):
-    """k_gemm_xlds (one workgroup walking several n-tiles with the activation chunks staged in LDS, DESIGN.md 9e) on the tiny
+    """k_gemm_xlds (one workgroup walking several n-tiles with the activation chunks staged in LDS) on the tiny
     shapes: gated FFN input, in_proj with RoPE / ring write and the row-major heads, one and two batch tiles, 1..3 tiles per
     workgroup (grid 8: 22 gated tiles -> 2-3 whole tiles per workgroup, 12 in_proj tiles -> 6 row octets = 1.5 tiles each, the
     shared tile written half by each owner; grids 5 / 7: uneven octet shares, ranges that would span 4 tiles fall back to
@@ -203,7 +203,7 @@ def test_depformer_in_per_step_launches(sim_lib, monkeypatch):
 
 @pytest.mark.parametrize("B", [2, 18, 34])
 def test_int8_linears_on_the_int8_matrix_core_match_the_bitsandbytes_restatement(sim_lib, B):
-    """`quantize=True` (BASELINE configs[4]): the reference's QLinear.forward is bitsandbytes' int8 x int8 matmul
+    """`quantize=True`: the reference's QLinear.forward is bitsandbytes' int8 x int8 matmul
     (utils/quantize.py:24-40) - activations quantised row-wise (absmax / 127, round half even), int32 accumulation on
     v_mfma_i32_*_i8, dequantised by SCA * SCB / 127^2.  Against the oracle's restatement of that published rule (bnb itself is
     absent: unpinned against the library), same tolerance as the bf16 path; 2 sessions = the 16-row tile (16x16x64), 18 / 34
@@ -215,7 +215,7 @@ def test_int8_linears_on_the_int8_matrix_core_match_the_bitsandbytes_restatement
 
 @pytest.mark.parametrize("B", [2, 18])
 def test_int8_weight_only_mode_matches_its_oracle(sim_lib, monkeypatch, B):
-    """MMI_Q8_ACT=bf16: the weight-only form of rounds 1-3 (int8 weights widened to bf16 in registers, bf16 activations),
+    """MMI_Q8_ACT=bf16: the weight-only form (int8 weights widened to bf16 in registers, bf16 activations),
     against the oracle in the same mode."""
     monkeypatch.setenv("MMI_Q8_ACT", "bf16")
     lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=80 + B, B=B, S=3, quantize=True, int8_activations=False)
@@ -238,7 +238,7 @@ def test_int8_activations_on_the_lds_resident_gemm(sim_lib, monkeypatch):
 
 @pytest.mark.parametrize("B", [3, 18, 40])
 def test_int8_linear_bit_exact_per_linear_against_the_oracle(sim_lib, B):
-    """VERDICT r4 item 1: `QLinear.forward` of ONE module (utils/quantize.py:24-40) through the step's kernels
+    """`QLinear.forward` of ONE module (utils/quantize.py:24-40) through the step's kernels
     (`mmi_lm_debug_linear`) - int8 codes, row absmax and bf16 output IDENTICAL to the oracle's restatement, for every linear
     family of the model (k_quant_rows_i8 + k_gemm_xp, the norm launch's int8 copy, k_gemm_q8 with and without the norm), at the
     16-row tile, one and two batch tiles of the 32-row tile."""
@@ -279,7 +279,7 @@ def test_bitsandbytes_rule_restated_known_answers():
 
 @pytest.mark.parametrize("B,input_scale", [(2, 1.0), (18, 0.25), (34, 1.0)])
 def test_fp8_weights_on_the_fp8_mfma_match_the_fp8_oracle(sim_lib, B, input_scale):
-    """`quantize="fp8"` (BASELINE configs[4]): e4m3fn linears with per-row scales, activations converted to e4m3 in registers,
+    """`quantize="fp8"`: e4m3fn linears with per-row scales, activations converted to e4m3 in registers,
     v_mfma_*_fp8_fp8.  Same tolerance as the bf16 path against an oracle that holds the same fp8 tensors and quantises the
     activations at the same points."""
     lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=90 + B, B=B, S=3, quantize="fp8", input_scale=input_scale)
@@ -287,7 +287,7 @@ def test_fp8_weights_on_the_fp8_mfma_match_the_fp8_oracle(sim_lib, B, input_scal
 
 @pytest.mark.parametrize("B,S,quantize", [(2, 15, False), (18, 3, False), (3, 4, "fp8")])
 def test_fp8_kv_ring_matches_the_oracle(sim_lib, B, S, quantize):
-    """`kv_cache_dtype="fp8"` (SURVEY.md 8d C5 "fp8 KV"): keys (after RoPE) and values enter the ring as e4m3 bytes, the decode
+    """`kv_cache_dtype="fp8"`: keys (after RoPE) and values enter the ring as e4m3 bytes, the decode
     attention widens them exactly; S > context: the ring wraps.  Oracle: the same e4m3 rounding at the ring write."""
     from dataclasses import replace
     lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), kv_cache_dtype="fp8"), seed=120 + B, B=B, S=S, quantize=quantize)
@@ -400,7 +400,7 @@ def test_none_during_delay_and_errors(sim_lib):
 
 @pytest.mark.parametrize("name", ["a", "b", "c", "d"])
 def test_guidance_conditioning_and_extra_heads_match_reference_golden(sim_lib, name):
-    """classifier-free guidance (a: masked-until, b: no-text, c: condition tensors), a `sum`
+    """Classifier-free guidance (a: masked-until, b: no-text, c: condition tensors), a `sum`
     condition and extra heads (d), against the reference's own LMGen runs (tests/golden/lm_cfg.npz)."""
     lm_cases.check_cfg_engine("cpu", sim_lib, name)
 
@@ -505,7 +505,7 @@ def test_int8_norm_fused_two_tiles_per_workgroup(sim_lib, B):
 
 
 def test_int8_depformer_batch_tiles_walked_by_one_workgroup(sim_lib, monkeypatch):
-    """MMI_Q8_TILES=serial: k_gemm_q8<32, 2, ..> (both batch tiles through one workgroup's registers, the round-4 form kept for
+    """MMI_Q8_TILES=serial: k_gemm_q8<32, 2, ..> (both batch tiles through one workgroup's registers, kept for
     same-box A/Bs) stays bit-identical to the oracle; the default at 33..64 sessions is one batch tile per workgroup (grid.y)."""
     monkeypatch.setenv("MMI_Q8_TILES", "serial")
     lm_cases.int8_linears_bit_exact("cpu", sim_lib, tiny_lm_config(), 40, seed=561)
@@ -513,7 +513,7 @@ def test_int8_depformer_batch_tiles_walked_by_one_workgroup(sim_lib, monkeypatch
 
 
 def test_debug_trace_of_two_sessions_is_identical(sim_lib, monkeypatch, tmp_path):
-    """MMI_DEBUG_TRACE (the tool that found round 5's unreproducible launch): every op followed by a checksum of every
+    """MMI_DEBUG_TRACE (the tool that found an unreproducible launch): every op followed by a checksum of every
     allocation of the streaming state.  Two sessions of one handle that start from identical memory (MMI_DEBUG_POISON=0) and are
     fed the same frames write the same file - on the simulator by construction; on MI355X it is the property under test."""
     monkeypatch.setenv("MMI_DEBUG_TRACE", str(tmp_path / "trace"))

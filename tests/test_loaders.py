@@ -1,4 +1,4 @@
-"""Checkpoint loading (SURVEY.md 8f-2): safetensors files with the reference's keys and config dictionaries -> engine models,
+"""Checkpoint loading: safetensors files with the reference's keys and config dictionaries -> engine models,
 quantised export.  Runs on the CPU kernel simulator."""
 import json
 from dataclasses import replace

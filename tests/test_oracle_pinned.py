@@ -50,7 +50,7 @@ def test_mimi_oracle_full_size_matches_reference():
         assert close(lat, g["latent"][f], 2e-5, 2e-5)
         assert np.array_equal(orc.quantize(g["latent"][f]), g["codes"][f])
         assert close(orc.decode(g["codes"][f]), g["pcm"][f], 2e-5, 2e-5)
-    # streaming codes == non-streaming codes in the reference (BASELINE.md section 2)
+    # streaming codes == non-streaming codes in the reference
     assert np.array_equal(np.concatenate(list(g["codes"]), -1), g["codes_nonstreaming"])
 
 
@@ -91,7 +91,7 @@ def test_lm_oracle_matches_reference_golden():
 
 
 def test_bf16_logit_gate_is_under_twice_the_distance_between_two_correct_implementations():
-    """the LM gates must rest on a yardstick, not on a multiple of what the engine happened to measure.  The
+    """The LM gates must rest on a yardstick, not on a multiple of what the engine happened to measure.  The
     yardstick of the bf16 gate (tests/lm_cases.py LOGIT_MAX_REL / LOGIT_MEAN_REL) is the distance between two CORRECT
     implementations of the same bf16 model on the same inputs - the reference's PyTorch CPU path (the golden file) and the numpy
     oracle, which differ only in summation order and in where intermediate roundings fall - measured here per (row, sampling site)

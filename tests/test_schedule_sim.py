@@ -5,8 +5,8 @@ The simulator's default schedule - wave 0 first, lane 0 first - is only ONE of t
 a kernel with a missing `__syncthreads()` (wave 1 reading what wave 0 has just written to LDS) passes under it by luck and fails on
 the GPU now and then.  `hipsim_set_schedule` (tests/hipsim/hipsim.cpp) walks waves and lanes BACKWARDS, or in a fresh random
 permutation at every scheduling pass; the engine's outputs - tokens, codes, logits, hidden states, PCM - must come out bit for bit
-as under the default schedule.  (Round 5's nondeterministic launch was found by comparing runs with each other, not with the
-checker: DESIGN.md 10a.  That one was an instruction-level hazard no simulator sees; this test covers the class a simulator CAN see.)
+as under the default schedule.  (A nondeterministic launch was once found by comparing runs with each other, not with the
+checker.  That one was an instruction-level hazard no simulator sees; this test covers the class a simulator CAN see.)
 
 The whole simulator suite was also run once under `HIPSIM_SCHED=reverse` and `HIPSIM_SCHED=random:7`
 (profiles/r05_logs/sim_suite_schedule_{reverse,random7}.log)."""
@@ -72,7 +72,7 @@ def test_perturbed_schedules_expose_a_missing_barrier(sim_lib, tmp_path):
     (18, False, {"MMI_GEMM_LDS": "2", "MMI_GEMM_KSPLIT": "2"}),        # 32-row tile, LDS-resident GEMM with split-K (the benchmark's form)
     (34, True, {}),                                                    # two batch tiles, int8 x int8: k_gemm_xp<32, 2> + k_gemm_q8 per tile
     (5, "fp8", {"MMI_ATTN_NS": "3"}),                                  # fp8 MFMA; the ring split over workgroups + merge
-    (18, False, {"MMI_GEMM_ONCE": "a", "MMI_GEMM_LDS": "0"}),          # round 6: k_gemm_xp_once on every GEMM whose slices fit
+    (18, False, {"MMI_GEMM_ONCE": "a", "MMI_GEMM_LDS": "0"}),          # k_gemm_xp_once on every GEMM whose slices fit
     (9, "guided-cross", {}),                                           # guidance twins + cross-attention block + k_cfg_mix
 ])
 def test_lm_step_is_independent_of_the_wave_schedule(sim_lib, monkeypatch, B, quantize, env):
@@ -146,7 +146,7 @@ def test_duplex_pipeline_is_independent_of_the_wave_schedule(sim_lib):
 
 
 def test_full_size_codec_at_the_c2_batch_is_independent_of_the_wave_schedule(sim_lib):
-    """The released codec's shapes, 8 streams (BASELINE configs[1]): every kernel at its production tiling (the wide-batch convs, the
+    """The released codec's shapes, 8 streams: every kernel at its production tiling (the wide-batch convs, the
     split-K GEMMs of the 12.5 / 25 Hz layers, both transformers, the RVQ).  ~1 minute.  (The LM's benchmark kernels at the 7B widths
     take minutes per run: tests/tools/sim_full_width_schedules.py, profiles/r05_logs/sim_full_width_schedules.log.)"""
     from moshi_amd import MimiConfig

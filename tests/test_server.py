@@ -1,4 +1,4 @@
-"""The websocket shell around the session batcher (moshi_amd/server.py; SURVEY.md 8f-1 / 8f-4): wire format of
+"""The websocket shell around the session batcher (moshi_amd/server.py): wire format of
 rust/protocol.md, the PCM codec seam, and concurrent fake clients against the engine on the CPU kernel simulator."""
 import asyncio
 
@@ -141,7 +141,7 @@ def test_concurrent_clients_each_get_their_own_stream(sim_lib):
 def test_a_vanished_channel_does_not_stop_the_model_loop():
     """A handler may close (disconnect) or re-open (RESTART) a channel between the loop's `closed` check and its pop - the
     batcher then reports an unknown channel.  That must end nothing but this session's drain: the loop keeps stepping and
-    the other sessions keep receiving (server.py model loop)."""
+    the other sessions keep receiving."""
     import threading
     import time
 
@@ -185,7 +185,7 @@ def test_a_vanished_channel_does_not_stop_the_model_loop():
 
 def test_any_other_invalid_argument_is_not_swallowed_by_the_model_loop():
     """Only the unknown-channel status ends a session's drain quietly; every other MMI_ERR_INVALID (a ValueError) is a real
-    failure of the model loop and is recorded as one (ADVICE round 3)."""
+    failure of the model loop and is recorded as one."""
     import time
 
     class FakeBatcher:

@@ -1,4 +1,4 @@
-"""BASELINE configs[4] on a real MI355X, part 2: e4m3 linears on the fp8 MFMA and the fp8 KV ring (engine options; the reference
+"""Eight-bit linears on a real MI355X, part 2: e4m3 linears on the fp8 MFMA and the fp8 KV ring (engine options; the reference
 has no fp8 path, so the gates are the format's own conditioning - tests/lm_cases.py "fp8 on hardware").  Collected after every
 core-path file and after the int8 file: `pytest -x` reaches it last but for the experimental GEMM plans."""
 import numpy as np
@@ -42,7 +42,7 @@ def test_fp8_hardware_primitives_match_their_definition(gpu_lib, tmp_path):
 
 @pytest.mark.parametrize("B,input_scale", [(2, 1.0), (18, 0.25), (40, 1.0)])
 def test_fp8_engine_is_within_the_conditioning_of_the_fp8_network(gpu_lib, B, input_scale):
-    """BASELINE configs[4]'s fp8 MFMA GEMMs (`quantize="fp8"`) on the tiny model, all three batch tilings: ring outputs exact;
+    """fp8 MFMA GEMMs (`quantize="fp8"`) on the tiny model, all three batch tilings: ring outputs exact;
     logits as close to the exact-accumulation fp8 oracle as that oracle stays to itself under the hardware's measured
     accumulate error, and as accurate against the bf16 model as the fp8 oracle (tests/lm_cases.py, "fp8 on hardware")."""
     print(lm_cases.fp8_engine_within_format_conditioning(DEV, None, tiny_lm_config(), seed=90 + B, B=B, S=3, input_scale=input_scale))
@@ -54,7 +54,7 @@ def test_fp8_full_width_within_the_conditioning_of_the_fp8_network(gpu_lib):
 
 
 def test_c5_shape_fp8_linears_at_64_sessions_within_the_conditioning_of_the_fp8_network(gpu_lib):
-    """BASELINE configs[4]'s own shape: 64 sessions, 7B layer widths (2 temporal layers), e4m3 linears on the fp8 MFMA."""
+    """64 sessions, 7B layer widths (2 temporal layers), e4m3 linears on the fp8 MFMA."""
     print(lm_cases.fp8_engine_within_format_conditioning(DEV, None, LMConfig(num_layers=2, context=64), seed=464, B=64, S=2))
 
 

@@ -22,7 +22,7 @@ def test_non_default_gemm_paths_at_full_width_match_oracle(gpu_lib, monkeypatch,
 
 def test_gemm_xp_with_rope_epilogue_is_bit_reproducible_at_two_batch_tiles(gpu_lib, monkeypatch):
     """MMI_GEMM_LDS=0 at 64 sessions, bf16: the temporal in_proj on k_gemm_xp<32, 2, ..> with the RoPE + ring-write epilogue - the
-    launch whose q / k output changed from run to run before round 5 (packed-math rotation, lm_kernels.h) - repeated streams equal
+    launch whose q / k output once changed from run to run (packed-math rotation, lm_kernels.h) - repeated streams equal
     the first bit for bit."""
     monkeypatch.setenv("MMI_GEMM_LDS", "0")
     lm_cases.reproducible_between_streams(DEV, None, LMConfig(num_layers=2, context=64), B=64, quantize=False, seed=15)

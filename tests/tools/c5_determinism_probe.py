@@ -1,4 +1,4 @@
-"""C5 at 64 sessions on a real MI355X: is it the ENGINE or the CHECKER that moves between runs?  
+"""C5 at 64 sessions on a real MI355X: is it the ENGINE or the CHECKER that moves between runs?
 
     python tests/tools/c5_determinism_probe.py <tag> [--quant none]
 
