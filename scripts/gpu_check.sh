@@ -1,6 +1,6 @@
 # The GPU check on one MI355X: smoke, every -m gpu test, the default benchmark
-# line (with its extras and its CPU-baseline leg), and the other named configurations (
-# configs 1, 2, 4) as logged lines.
+# line (with its extras and its CPU-baseline leg), and the other configurations as
+# logged lines.
 cd $GRAFT_REPO_ROOT
 mkdir -p gpurun_out
 O=$GRAFT_REPO_ROOT/gpurun_out
