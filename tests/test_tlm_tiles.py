@@ -24,6 +24,25 @@ def dense_model(width, ff):
     return TokenLMConfig("Bibapel", vocab=331, width=width, layers=[TokenLayerConfig(att, DenseGLUConfig(ff=ff, limit=7.0))], norms=2, layer_scales=False, tied_head=True)
 
 
+def check_prompt_at_once(device, lib, model, T, dtype, want_forms, monkeypatch, capfd):
+    monkeypatch.setenv("MMI_TLM_FORMS", "1")
+    sd = random_token_lm_state_dict(model, seed=T, device=device)
+    lm = TokenLM(sd, model, dtype=dtype, max_slots=2, max_tokens=4096, max_step_tokens=T, **({} if lib is None else {"device": device, "lib": lib}))
+    prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
+    want = sorted({0, 15, 16, 63, 64, T // 2, T - 2, T - 1})
+    a = lm.open()
+    capfd.readouterr()
+    whole = lm.step([(a, prompt, want)])
+    assert "k_tlm_gemm_tile" in {k for _, k, _ in lm.launch_list()}
+    assert {line[5:line.index(",")] for line in capfd.readouterr().err.splitlines() if line.startswith("tile ")} == want_forms
+    b = lm.open()
+    parts = torch.cat([lm.step([(b, prompt[i:i + 64], [w - i for w in want if i <= w < i + 64])]) for i in range(0, T, 64)])
+    rel = float((whole - parts).double().norm() / parts.double().norm())
+    # fp32: sums of up to 6000 products in another order, over a handful of layers (eps sqrt(6000) ~ 5e-6); bf16: an activation on the other
+    # side of a rounding boundary here and there (2^-9 each)
+    assert rel < (1e-5 if dtype == torch.float32 else 8e-3), rel
+
+
 # form: features x rows of a block, stages in its ring, k-steps per stage
 SMALL32, SMALL16 = {"64x32 stages 4 of 2"}, {"64x64 stages 4 of 2"}
 
@@ -41,23 +60,25 @@ SMALL32, SMALL16 = {"64x32 stages 4 of 2"}, {"64x64 stages 4 of 2"}
     (dense_model(1040, 6000), 1157, {"128x128 stages 3 of 1"}, {"256x128 stages 3 of 1", "128x128 stages 4 of 1"}),
 ], ids=["65", "130", "200", "100", "460", "577", "641", "1025", "1157"])
 def test_prompt_at_once_equals_portions(model, T, fp32, bf16, dtype, monkeypatch, capfd):
-    monkeypatch.setenv("MMI_TLM_FORMS", "1")
-    sd = random_token_lm_state_dict(model, seed=T, device="cuda")
-    lm = TokenLM(sd, model, dtype=dtype, max_slots=2, max_tokens=4096, max_step_tokens=T)
-    prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
-    want = sorted({0, 15, 16, 63, 64, T // 2, T - 2, T - 1})
-    a = lm.open()
-    capfd.readouterr()
-    whole = lm.step([(a, prompt, want)])
-    assert "k_tlm_gemm_tile" in {k for _, k, _ in lm.launch_list()}
-    forms = {line[5:line.index(",")] for line in capfd.readouterr().err.splitlines() if line.startswith("tile ")}
-    assert forms == (fp32 if dtype == torch.float32 else bf16)
-    b = lm.open()
-    parts = torch.cat([lm.step([(b, prompt[i:i + 64], [w - i for w in want if i <= w < i + 64])]) for i in range(0, T, 64)])
-    rel = float((whole - parts).double().norm() / parts.double().norm())
-    # fp32: sums of up to 6000 products in another order, over a handful of layers (eps sqrt(6000) ~ 5e-6); bf16: an activation on the other
-    # side of a rounding boundary here and there (2^-9 each)
-    assert rel < (1e-5 if dtype == torch.float32 else 8e-3), rel
+    check_prompt_at_once("cuda", None, model, T, dtype, fp32 if dtype == torch.float32 else bf16, monkeypatch, capfd)
+
+
+@pytest.mark.parametrize("model,T,forms", [
+    (dense_model(64, 8200), 70, {"64x64 stages 4 of 1", "64x64 stages 4 of 2"}),               # 538 equal blocks of two k-steps; then a few
+    (dense_model(2080, 8000), 66, {"64x64 stages 4 of 1", "64x64 stages 4 of 2"}),             # 524 equal blocks of 65 k-steps; then 66 long ones beside 66 short
+    (experts_model(80, 4200), 96, {"64x64 stages 4 of 1", "64x64 stages 4 of 2"}),             # listed blocks: more than 512, and fewer
+], ids=["dense", "long", "experts"])
+def test_prompt_at_once_on_the_simulator(model, T, forms, monkeypatch, capfd):
+    """64 x 64 blocks in stages of one and of two k-steps, the forms that no tiny model's launches are large enough for."""
+    import os
+    import sys
+    from pathlib import Path
+    from moshi_amd import _capi
+    monkeypatch.setenv("MMI_NO_GRAPH", "1")
+    sys.path.insert(0, str(Path(__file__).resolve().parent / "hipsim"))
+    import build_sim
+    lib = _capi.load_tlm(os.environ.get("MMI_TLM_SIM_LIB") or build_sim.build_tlm())
+    check_prompt_at_once("cpu", lib, model, T, torch.bfloat16, forms, monkeypatch, capfd)
 
 
 @pytest.mark.parametrize("rise", [0.0, 0.3, 3.7, 7.9, 8.1, 40.0])
