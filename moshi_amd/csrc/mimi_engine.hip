@@ -44,10 +44,10 @@ struct MimiSlab {
     size_t size = 0, need = 0;
     bool over = false;
     void* alloc(size_t nb) {
-        char* p = base + need;
+        const size_t at = need;
         need += (nb + 255) & ~(size_t)255;
         over = over || need > size;
-        return over ? (char*)this : p;         // (not null, which means "none" to the plans; no launch is given it)
+        return over ? (char*)this : base + at;         // (not null, which means "none" to the plans; no launch is given it)
     }
     void rewind() { need = 0; over = false; }
     bool release() {                           // false: kept, the runtime does not free while another thread captures
