@@ -342,6 +342,7 @@ __device__ __forceinline__ float mmi_rsqrtf(float x) { return 1.0f / sqrtf(x); }
 // base-2 exponential and logarithm in hardware (v_exp_f32, v_log_f32: ~1 ulp, denormals flushed)
 __device__ __forceinline__ float mmi_fast_exp2f(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float mmi_fast_log2f(float x) { return __builtin_amdgcn_logf(x); }
+__device__ __forceinline__ float mmi_fast_rcpf(float x) { return __builtin_amdgcn_rcpf(x); }      // ~1 ulp
 __device__ __forceinline__ float mmi_fast_logf(float x) { return __logf(x); }
 __device__ __forceinline__ unsigned mmi_atomic_add(unsigned* p, unsigned v) { return atomicAdd(p, v); }
 
