@@ -153,7 +153,8 @@ struct mmi_tlm {
     hipStream_t cap_stream = nullptr;
     std::map<std::tuple<int, int, int>, std::unique_ptr<MmiProgram>> progs;
     std::vector<std::string> last_log;
-    bool say_forms = false;        // test hook (MMI_TLM_FORMS): a line on stderr for every launch of the tiled kernel
+    bool say_forms = false;        // test hook (MMI_TLM_FORMS): a line on stderr for every launch of the tiled kernels
+    int force_wide = 0;            // test hook (MMI_TLM_WIDE): every product that k_tlm_gemm_wide can take goes there, in blocks of so many rows
     long weight_bytes = 0;
 };
 
@@ -784,6 +785,7 @@ Plan plan_rows(int T, bool routed, bool f32) {
     return p;
 }
 int plan_tile(const Plan& p) { return p.rows ? 16 * p.mt : 32 * p.fm; }
+constexpr int WIDE_ROWS = 256, WIDE_KS = 48;              // k_tlm_gemm_wide: rows of a block, k-steps that it is worth it for
 
 TlmJob base_job(const Mat& w, const void* x, int xks) {
     TlmJob j;
@@ -820,10 +822,10 @@ int rows_ntw(const Plan& p);
 // K split so that a product with few n-tiles still covers the chip; the consumer sums the fp32 partials.  `blocks`: what the launch has
 // without a split - n-tiles of the weight-streaming kernel, blocks of the tiled kernel (tile_blocks).  The tiled kernel wants two blocks per
 // CU: 200 rows x 2048 x 2560 takes 18.1, 11.4, 9.2 us with 1, 2, 4 splits, 2048 rows x 2048 x 2560 31.7 and 26.1 with 1 and 2.
-int split_for(const Plan& p, const Mat& w, int blocks) {
+int split_for(const Plan& p, int KS, int blocks) {
     int s = 1;
-    if (p.rows) while (s < MAX_SPLIT && blocks * s < 384 * rows_ntw(p) && w.KS / (2 * s) >= 8) s *= 2;
-    else while (s < TILE_SPLIT && blocks * s < TILE_BLOCKS && w.KS / (2 * s) >= 16) s *= 2;
+    if (p.rows) while (s < MAX_SPLIT && blocks * s < 384 * rows_ntw(p) && KS / (2 * s) >= 8) s *= 2;
+    else while (s < TILE_SPLIT && blocks * s < TILE_BLOCKS && KS / (2 * s) >= 16) s *= 2;
     return s;
 }
 // blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64, at fp32 64 x 32)
@@ -831,6 +833,7 @@ int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, p.fm == 
 int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
 
 int rows_ntw(const Plan& p) { return p.mt; }                // n-tiles per workgroup of the weight-streaming kernel
+
 template <class Tr, int FN, int FM, int ST, int OCC, int WN = 2, int WM = 2, int KK = 1>
 int launch_tile(hipStream_t s, const TlmJobs& J, bool say) {
     constexpr size_t smem = TlmTile<Tr, FN, FM, WN, WM, ST, KK>::smem();
@@ -846,62 +849,202 @@ int launch_tile(hipStream_t s, const TlmJobs& J, bool say) {
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
+// n-tiles per block -> blocks of every job, and their number
+int cut_blocks(const Plan& p, TlmJobs& J, int ntw) {
+    int total = 0;
+    for (int i = 0; i < J.n; ++i) {
+        TlmJob& j = J.j[i];
+        if (!j.list) j.rblocks = J.height ? mmi_cdiv(j.rows, J.height) : mmi_cdiv(j.rows, plan_tile(p));
+        j.blocks = mmi_cdiv(j.NT, ntw) * (j.list ? 1 : j.groups) * j.ksplit * j.rblocks;
+        total += j.blocks;
+    }
+    return total;
+}
+enum Form { FORM_256x128, FORM_128x128, FORM_128x128_3, FORM_128x64, FORM_64x64_2, FORM_64x64 };
+// the tiled kernel's form for a launch at bf16; its blocks are cut
+Form bf16_form(const Plan& p, TlmJobs& J) {
+    // The widest block that still gives nearly every CU two: 256 x 128 in three stages (1773 x 22528 x 4096: 338 us, 0.97 PFLOP/s; in
+    // 128 x 128 blocks 379), then 128 x 128 (2048 x 2048 x 2560: 31.7 us against 47.3), in four stages while two blocks per CU are all there
+    // is, in three where a third one finds work (676 x 11264 x 2048: 47.7 against 58.1).
+    if (p.fm == 4) {
+        if (cut_blocks(p, J, 16) >= 400) return FORM_256x128;
+        return cut_blocks(p, J, 8) <= 512 ? FORM_128x128 : FORM_128x128_3;
+    }
+    // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
+    if (cut_blocks(p, J, 8) >= 512) return FORM_128x64;
+    // 64 x 64 with stages of two k-steps, two blocks per CU, while those are all there is or a second round of them is short ones in the shadow of the
+    // first: 512 blocks of 176 and 64 k-steps 54 -> 39 us, 640 of them 56 -> 45, 768 of 352 and 128 113 -> 106 (896: 118 and 117).  Otherwise one
+    // k-step each, four blocks per CU: 576 blocks of 256 k-steps 84 us against 103, 896 of 64 36 against 38, 640 of 16 12 against 16; expert blocks,
+    // of a few rows or none, likewise (100 rows of Kesirax 2048: 833 against 989 us)
+    const int total = cut_blocks(p, J, 4);
+    bool listed = false;
+    long longest = 0, work = 0, heavy = 0;                   // k-steps of a block and of all of them; blocks of more than half the longest
+    auto ksteps = [](const TlmJob& j) { return (long)mmi_cdiv(j.KS, j.ksplit); };
+    for (int i = 0; i < J.n; ++i) longest = std::max(longest, ksteps(J.j[i]));
+    for (int i = 0; i < J.n; ++i) {
+        const TlmJob& j = J.j[i];
+        listed = listed || j.list;
+        work += j.blocks * ksteps(j);
+        if (2 * ksteps(j) > longest) heavy += j.blocks;
+    }
+    return total <= 512 || (!listed && heavy <= 512 && 16 * work <= 17 * 512 * longest) ? FORM_64x64_2 : FORM_64x64;
+}
+
+// ---- which launches take k_tlm_gemm_wide, in blocks of which height, with which splits ----
+// What launches take, in us, by their blocks and k-steps: fitted to 120 launches of the two kernels (65 - 2048 rows, widths 2048 and 4096, weights from
+// HBM), which it meets within 5 and 7 % (rms).  The narrower forms: so many blocks to a CU, a k-step of 1 .. that many of them, the rest of a block.
+struct FormTime { int ntw, places; float fixed, step[4]; };
+const FormTime form_times[] = {{16, 2, 12.f, {0.66f, 0.88f}},        {8, 2, 8.f, {0.34f, 0.54f}}, {8, 3, 8.f, {0.50f, 0.66f, 0.82f}},
+                               {8, 3, 6.f, {0.40f, 0.45f, 0.55f}}, {4, 2, 6.f, {0.165f, 0.25f}}, {4, 4, 6.f, {0.25f, 0.28f, 0.37f, 0.50f}}};
+float narrow_time(Form form, const TlmJobs& J) {
+    const FormTime& f = form_times[form];
+    int longest = 0;
+    float work = 0.f;
+    for (int i = 0; i < J.n; ++i) {
+        longest = std::max(longest, mmi_cdiv(J.j[i].KS, J.j[i].ksplit));
+        work += (float)J.j[i].blocks * mmi_cdiv(J.j[i].KS, J.j[i].ksplit);
+    }
+    const float rounds = work / longest / (256 * f.places), full = longest * f.step[f.places - 1] + f.fixed;
+    const int whole = (int)rounds;
+    const float on_cu = (rounds - whole) * f.places;         // of the last round
+    if (on_cu < 0.02f) return whole * full;
+    const int i = std::min(f.places - 1, std::max(0, (int)on_cu - 1));
+    float step = f.step[i];
+    if (i + 1 < f.places && on_cu > 1.f) step += (f.step[i + 1] - step) * (on_cu - 1 - i);
+    const float last = longest * step + f.fixed;
+    // (behind whole rounds the CUs are out of step: the last one is half hidden)
+    return whole * full + (whole ? 0.6f * last + 0.4f * on_cu / f.places * full : last);
+}
+// blocks of up to three lengths on one place per CU, the longest first, each where one falls free: when the last one ends
+float deal(const float* length, const int* blocks, int n) {
+    float at[32] = {0.f};                                    // groups of places by when they fall free
+    int count[32] = {256}, k = 1, order[3] = {0, 1, 2};
+    std::sort(order, order + n, [&](int a, int b) { return length[a] > length[b]; });
+    float end = 0.f;
+    for (int o = 0; o < n; ++o) {
+        const int i = order[o];
+        for (int left = blocks[i]; left > 0;) {
+            int a = 0;
+            for (int x = 1; x < k; ++x)
+                if (at[x] < at[a]) a = x;
+            const int c = std::min(left, count[a]);
+            left -= c;
+            end = std::max(end, at[a] + length[i]);
+            if (c == count[a] || k == 32) {
+                at[a] += length[i];
+            } else {
+                count[a] -= c;
+                at[k] = at[a] + length[i];
+                count[k++] = c;
+            }
+        }
+    }
+    return end;
+}
+float wide_block(int rows, int ks, int epi) {
+    static const float step[8] = {0.33f, 0.36f, 0.41f, 0.48f, 0.57f, 0.64f, 0.70f, 0.78f};
+    return 8.5f + rows * (epi == TLM_EPI_F32 || epi == TLM_EPI_PACK ? 0.03f : 0.045f) + ks * step[(rows - 1) / 32];
+}
+// Splits of the jobs in `may_split` (fp32 partials, summed by who reads them) and, at bf16, whether the launch takes k_tlm_gemm_wide and in blocks of
+// which height: where it is 3 % faster than the form that bf16_form takes, in whole and with the partials' traffic.  Reductions of fewer than
+// WIDE_KS k-steps keep to blocks of which several share a CU, and so do experts' runs: a block of them has its weights to itself, they bound it
+// (Kesirax 2048, 2048 tokens, expert blocks of up to 160, 192, 256 rows: 2523, 2539, 2579 us against 2475).
+void plan_jobs(const mmi_tlm* m, const Plan& p, TlmJobs& J, unsigned may_split) {
+    int blocks = 0;
+    bool wide = !m->f32 && !p.rows;
+    for (int i = 0; i < J.n; ++i) {
+        blocks += split_blocks(p, J.j[i]);
+        wide = wide && J.j[i].groups == 1 && !J.j[i].list && (J.j[i].KS >= WIDE_KS || m->force_wide);
+    }
+    for (int i = 0; i < J.n; ++i)
+        if (may_split >> i & 1) J.j[i].ksplit = split_for(p, J.j[i].KS, p.rows ? split_blocks(p, J.j[i]) : blocks);
+    if (!wide) return;
+    if (m->force_wide) {
+        J.height = m->force_wide;
+        return;
+    }
+    auto partials = [&](const int* split) {                  // us that the splits' partials take to be written and read
+        float us = 0.f;
+        for (int i = 0; i < J.n; ++i)
+            if (split[i] > 1) us += (split[i] - 1) * (float)J.j[i].out_ps * 8.f / 4e6f;
+        return us;
+    };
+    int split[3] = {1, 1, 1}, T = 0;
+    for (int i = 0; i < J.n; ++i) {
+        split[i] = J.j[i].ksplit;
+        T = std::max(T, J.j[i].rows);
+    }
+    const Form form = bf16_form(p, J);
+    float best = 0.97f * (narrow_time(form, J) + partials(split));
+    int last = 0;
+    for (int rb = mmi_cdiv(T, WIDE_ROWS), tries = 0; tries < 6; ++rb, ++tries) {
+        const int height = (mmi_cdiv(T, rb) + 31) / 32 * 32;
+        if (height == last) continue;
+        last = height;
+        for (int most = 1 << 20; most >= 16; most = most > 256 ? 256 : most / 2) {      // k-steps of a block
+            bool fits = true, cuts = most > 256;
+            float length[3];
+            int count[3];
+            for (int i = 0; i < J.n; ++i) {
+                const TlmJob& j = J.j[i];
+                split[i] = 1;
+                if (may_split >> i & 1)
+                    while (split[i] < TILE_SPLIT && mmi_cdiv(j.KS, split[i]) > most) split[i] *= 2;
+                cuts = cuts || split[i] > 1;
+                fits = fits && (split[i] == 1 || split[i] * j.out_ps <= 2L * TILE_BLOCKS * 128 * 128);
+                length[i] = wide_block(height, mmi_cdiv(j.KS, split[i]), j.epi);
+                count[i] = mmi_cdiv(j.NT, TlmWide::NFN) * mmi_cdiv(T, height) * split[i];
+            }
+            if (!fits || !cuts) continue;
+            const float us = deal(length, count, J.n) + partials(split);
+            if (us >= best) continue;
+            best = us;
+            J.height = height;
+            for (int i = 0; i < J.n; ++i) J.j[i].ksplit = split[i];
+        }
+    }
+}
+int launch_wide(hipStream_t s, const Plan& p, TlmJobs& J, bool say) {
+    // the jobs of the longest blocks first
+    std::sort(J.j, J.j + J.n, [](const TlmJob& a, const TlmJob& b) { return mmi_cdiv(a.KS, a.ksplit) > mmi_cdiv(b.KS, b.ksplit); });
+    cut_blocks(p, J, TlmWide::NFN);
+    int grid = 0;                                          // every XCD's share of every job, rounded up
+    for (int i = 0; i < J.n; ++i) grid += 8 * mmi_cdiv(J.j[i].blocks, 8);
+    if (say) fprintf(stderr, "wide 256x%d, %d workgroups\n", J.height, grid);
+    static_assert(TlmWide::smem() <= 160 * 1024, "LDS of a CU");
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gemm_wide<TlmBf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)TlmWide::smem());
+    MMI_HIP_CHECK(attr);
+    MMI_LAUNCH((k_tlm_gemm_wide<TlmBf16>), grid, 512, TlmWide::smem(), s, J);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
 template <class Tr>
 int launch_jobs_t(hipStream_t s, const Plan& p, TlmJobs& J, bool say) {
-    auto cut = [&](int ntw) {                               // n-tiles per block -> blocks of every job, and their number
-        int total = 0;
-        for (int i = 0; i < J.n; ++i) {
-            TlmJob& j = J.j[i];
-            if (!j.list) j.rblocks = mmi_cdiv(j.rows, plan_tile(p));
-            j.blocks = mmi_cdiv(j.NT, ntw) * (j.list ? 1 : j.groups) * j.ksplit * j.rblocks;
-            total += j.blocks;
-        }
-        return total;
-    };
     if (p.rows) {
-        const int grid = cut(rows_ntw(p));
+        const int grid = cut_blocks(p, J, rows_ntw(p));
         if (p.mt == 1) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 1, 1, 8, 4>), grid, 512, 0, s, J);
         else if (p.mt == 2) MMI_LAUNCH((k_tlm_gemm_rows<Tr, 2, 2, 8, 2>), grid, 512, 0, s, J);
         else MMI_LAUNCH((k_tlm_gemm_rows<Tr, 4, 4, 4, 2>), grid, 256, 0, s, J);
         MMI_CHECK_LAUNCH();
         return MMI_OK;
     }
-    // The widest block that still gives nearly every CU two: 256 x 128 in three stages (1773 x 22528 x 4096: 338 us, 0.97 PFLOP/s; in
-    // 128 x 128 blocks 379), then 128 x 128 (2048 x 2048 x 2560: 31.7 us against 47.3), in four stages while two blocks per CU are all there
-    // is, in three where a third one finds work (676 x 11264 x 2048: 47.7 against 58.1).  At fp32 the matrix core bounds every form.
-    if (p.fm == 4) {
-        if constexpr (Tr::V == 8) {
-            const int wide = cut(16);
-            if (wide >= 400) return launch_tile<Tr, 8, 4, 3, 2>(s, J, say);
-        }
-        const int grid = cut(8);
-        return grid <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J, say) : launch_tile<Tr, 4, 4, 3, 3>(s, J, say);
-    }
-    // 128 x 64 where that leaves two blocks per CU (676 x 11264 x 2048: 49 us, 64 x 64: 57; 200 x 7680 x 2048: 20.0 and 18.9)
     if constexpr (Tr::V == 8) {
-        if (cut(8) >= 512) return launch_tile<Tr, 4, 2, 4, 3>(s, J, say);
-        // 64 x 64 with stages of two k-steps, two blocks per CU, while those are all there is or a second round of them is short ones in the shadow of the
-        // first: 512 blocks of 176 and 64 k-steps 54 -> 39 us, 640 of them 56 -> 45, 768 of 352 and 128 113 -> 106 (896: 118 and 117).  Otherwise one
-        // k-step each, four blocks per CU: 576 blocks of 256 k-steps 84 us against 103, 896 of 64 36 against 38, 640 of 16 12 against 16; expert blocks,
-        // of a few rows or none, likewise (100 rows of Kesirax 2048: 833 against 989 us)
-        const int total = cut(4);
-        bool listed = false;
-        long longest = 0, work = 0, heavy = 0;               // k-steps of a block and of all of them; blocks of more than half the longest
-        auto ksteps = [](const TlmJob& j) { return (long)mmi_cdiv(j.KS, j.ksplit); };
-        for (int i = 0; i < J.n; ++i) longest = std::max(longest, ksteps(J.j[i]));
-        for (int i = 0; i < J.n; ++i) {
-            const TlmJob& j = J.j[i];
-            listed = listed || j.list;
-            work += j.blocks * ksteps(j);
-            if (2 * ksteps(j) > longest) heavy += j.blocks;
+        if (J.height) return launch_wide(s, p, J, say);
+        switch (bf16_form(p, J)) {
+            case FORM_256x128: return launch_tile<Tr, 8, 4, 3, 2>(s, J, say);
+            case FORM_128x128: return launch_tile<Tr, 4, 4, 4, 2>(s, J, say);
+            case FORM_128x128_3: return launch_tile<Tr, 4, 4, 3, 3>(s, J, say);
+            case FORM_128x64: return launch_tile<Tr, 4, 2, 4, 3>(s, J, say);
+            case FORM_64x64_2: return launch_tile<Tr, 2, 2, 4, 2, 2, 2, 2>(s, J, say);
+            default: return launch_tile<Tr, 2, 2, 4, 4>(s, J, say);
         }
-        if (total <= 512 || (!listed && heavy <= 512 && 16 * work <= 17 * 512 * longest)) return launch_tile<Tr, 2, 2, 4, 2, 2, 2, 2>(s, J, say);
-        return launch_tile<Tr, 2, 2, 4, 4>(s, J, say);
     } else {
-        // at fp32 the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
+        // the matrix core bounds every form: 128 x 128 from plan_rows' rows on, in four stages while two blocks per CU are all there is
+        if (p.fm == 4) return cut_blocks(p, J, 8) <= 512 ? launch_tile<Tr, 4, 4, 4, 2>(s, J, say) : launch_tile<Tr, 4, 4, 3, 3>(s, J, say);
+        // the waves share the features, so that all of them gain by the row fragments an expert's last block leaves out
         // 32 rows and two k-steps per stage (plan_rows); more stages while all blocks fit the chip with them (three per CU, expert blocks without rows aside; Kesirax 1024, 194 rows: 911 and
         // 865 us; 320 rows, with more blocks: 1030 and 1045)
-        return cut(4) <= 1024 ? launch_tile<Tr, 1, 2, 4, 3, 4, 1, 2>(s, J, say) : launch_tile<Tr, 1, 2, 3, 4, 4, 1, 2>(s, J, say);
+        return cut_blocks(p, J, 4) <= 1024 ? launch_tile<Tr, 1, 2, 4, 3, 4, 1, 2>(s, J, say) : launch_tile<Tr, 1, 2, 3, 4, 4, 1, 2>(s, J, say);
     }
 }
 int launch_jobs(mmi_tlm* m, hipStream_t s, const Plan& p, TlmJobs J) {
@@ -1054,6 +1197,7 @@ MixerOut build_mingru(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
     j.bias = L.bias;
     first.j[first.n++] = j;
     P.site(site + "in");
+    plan_jobs(m, p, first, 0);
     add_jobs(m, P, p, first, L.zcg.bytes());
     TlmScanArgs a;
     memset(&a, 0, sizeof(a));
@@ -1087,9 +1231,9 @@ MixerOut build_latent_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, cons
     j.out = m->lat;
     j.out_ld = ld;
     j.out_ps = (long)T * ld;
-    j.ksplit = split_for(p, L.in, p.rows ? L.in.NT : tile_blocks(p, j) + (first.n ? tile_blocks(p, first.j[0]) : 0));
-    const int in_p = j.ksplit;
     first.j[first.n++] = j;
+    plan_jobs(m, p, first, 1u << (first.n - 1));
+    const int in_p = first.j[first.n - 1].ksplit;
     P.site(site + "in");
     add_jobs(m, P, p, first, L.in.bytes());
 
@@ -1221,6 +1365,7 @@ MixerOut build_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer
     j.qkv = TlmQkv{r.kc, r.vc, m->meta + sh.m.crow, H * L.dim_p / 16, G * L.dim_p / 16, L.dim_p / 16, L.nd, H, G};
     first.j[first.n++] = j;
     P.site(site + "in");
+    plan_jobs(m, p, first, 0);
     add_jobs(m, P, p, first, L.in.bytes());
 
     TlmGqaArgs t;
@@ -1316,6 +1461,7 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         first.j[first.n++] = j;
     }
     P.site(site + "in");
+    plan_jobs(m, p, first, 0);
     add_jobs(m, P, p, first, L.in.bytes() + L.lr.bytes());
 
     TlmLinArgs a;
@@ -1498,11 +1644,11 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
             memset(&J, 0, sizeof(J));
             TlmJob& j = J.j[J.n++];
             j = dense_job(m->loop_in, m->cat, 2 * m->h_ks, T);
-            j.ksplit = split_for(p, m->loop_in, split_blocks(p, j));
             j.epi = TLM_EPI_F32;
             j.out = m->mix;
             j.out_ld = m->ld;
             j.out_ps = (long)T * m->ld;
+            plan_jobs(m, p, J, 1);
             c = Carry();
             c.mix = m->mix;
             c.mix_p = j.ksplit;
@@ -1550,32 +1696,26 @@ void build_program(mmi_tlm* m, MmiProgram& P, const Shape& sh) {
         TlmJobs J;
         memset(&J, 0, sizeof(J));
         c = Carry();
-        TlmJob o = dense_job(*mo.w, mo.x, mo.xks, T);
-        const int others = p.rows ? 0 : tile_blocks(p, o);
         if (moe || dense) {
             TlmJob& j = J.j[J.n++];
             c.top = moe ? L.c.top : 1;
             j = moe ? routed_job(m, L, L.down, m->hid, L.down.KS, 1, T, p) : dense_job(L.down, m->hid, L.down.KS, T);
             j.in_pos = moe;
-            const int mine = split_blocks(p, j);
-            j.ksplit = split_for(p, L.down, mine + others);
-            if (!p.rows) o.ksplit = split_for(p, *mo.w, mine + others);
             j.epi = TLM_EPI_F32;
             j.out = m->dn;
             j.out_ld = m->ld;
             j.out_ps = (long)T * c.top * m->ld;
             c.dn = m->dn;
-            c.dn_p = j.ksplit;
             c.ls2 = L.ls2;
-        } else if (!p.rows) {
-            o.ksplit = split_for(p, *mo.w, others);
         }
-        if (p.rows) o.ksplit = split_for(p, *mo.w, o.NT);
+        TlmJob& o = J.j[J.n++];
+        o = dense_job(*mo.w, mo.x, mo.xks, T);
         o.epi = TLM_EPI_F32;
         o.out = m->mix;
         o.out_ld = m->ld;
         o.out_ps = (long)T * m->ld;
-        J.j[J.n++] = o;
+        plan_jobs(m, p, J, (1u << J.n) - 1);
+        if (c.dn) c.dn_p = J.j[0].ksplit;
         c.mix = m->mix;
         c.mix_p = o.ksplit;
         c.ls1 = L.ls1;
@@ -1753,6 +1893,7 @@ int create_impl(mmi_tlm* m, const mmi_tensor_desc* weights, int n_weights) {
     if ((rc = alloc_state(m)) || (rc = alloc_buffers(m))) return rc;
     m->graphs = mmi_graphs_enabled();
     m->say_forms = getenv("MMI_TLM_FORMS") != nullptr;
+    if (const char* h = getenv("MMI_TLM_WIDE")) m->force_wide = std::min(256, std::max(32, atoi(h) / 32 * 32));
     if (m->graphs) MMI_HIP_CHECK(hipStreamCreateWithFlags(&m->cap_stream, hipStreamNonBlocking));
     MMI_HIP_CHECK(hipDeviceSynchronize());
     return MMI_OK;

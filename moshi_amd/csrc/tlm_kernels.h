@@ -361,6 +361,7 @@ struct TlmJob {
 struct TlmJobs {
     TlmJob j[3];
     int n;
+    int height;                          // k_tlm_gemm_wide: rows per block, a multiple of 32
 };
 
 // cached values of grouped attention: the transposed operand of the value product, [page][kv head][keys / KSTEP][16-wide value blocks]
@@ -733,6 +734,169 @@ __global__ __launch_bounds__(WN * WM * 64, OCC) void k_tlm_gemm_tile(TlmJobs job
             const int nx = min(FN, j.NT - nt0 - wn * FN);
 #pragma unroll 1
             for (int x = 0; x < nx; ++x) tlm_epilogue<Tr, decltype(epi)::value>(j, g, split, id, nt0 + wn * FN + x, lane >> 4, buf[x * 64]);
+        }
+    });
+}
+
+// Dense products of many rows at bf16: 256 features x up to 256 rows per workgroup of 8 waves, 4 along the features and 2 along the rows, one
+// workgroup per CU.  A wave has 64 features x 16 FM rows, FM = 1 .. 8 by the rows the block has: rows are cut evenly into blocks of a height
+// that suits the chip (plan_jobs).  Operands as in k_tlm_gemm_tile; here a stage's place in the ring is loaded again as soon as its last
+// k-step is in registers.  KK = 2 (two k-steps per meeting) where a wave has 12 products or fewer in a k-step.
+// What bounds it: a CU has some 26 KB of loads on their way, whatever is asked for, so that a k-step takes the time in which its operands
+// pass (64 rows: 0.36 us, most of them behind weights that come from HBM) unless its products take longer (256 rows: 0.78 us, 1.3 PFLOP/s).
+// 256 x 256 loads 8 KB per MFLOP, 256 x 128 11, 128 x 64 24; against those, one workgroup per CU leaves its first loads and its last stores
+// bare (8 us, and 8 - 19 us for 256 rows).  Width 2048, 639 rows, 14336 - 19456 features: 63.5 - 79.3 us in 128 x 64 blocks, 56.6 - 68.6 here;
+// width 4096, 420 rows, 4096 x 11264 and 4096 x 4096 together: 95.5 and 83.8; 1773 rows: 282 and 238.
+struct TlmWide {
+    static constexpr int FN = 4, NFN = 16;                   // feature fragments of a wave, of the block
+    static constexpr int kk(int fm) { return fm <= 3 ? 2 : 1; }
+    static constexpr int stages(int fm) { return fm <= 3 ? 3 : 4; }
+    static constexpr size_t smem() { return (size_t)3 * 2 * (NFN + 2 * 3) * 1024; }      // the largest ring: FM = 3 (8: 4 x 32 KB)
+};
+template <class Tr>
+__global__ __launch_bounds__(512, 2) void k_tlm_gemm_wide(TlmJobs jobs) {
+    constexpr int FN = TlmWide::FN, NFN = TlmWide::NFN, FMAX = 8;
+    MMI_DYN_SHARED(u32x4, lds);
+    const int xcd = (int)blockIdx.x & 7;                      // (every XCD a run of every job's blocks: k_tlm_gemm_tile)
+    int b = (int)blockIdx.x >> 3, ji = 0;
+    for (;; ++ji) {
+        if (ji == jobs.n) return;
+        const int lo = (int)((long)jobs.j[ji].blocks * xcd >> 3), mine = (int)((long)jobs.j[ji].blocks * (xcd + 1) >> 3) - lo;
+        if (b < mine) {
+            b += lo;
+            break;
+        }
+        b -= mine;
+    }
+    const TlmJob j = jobs.j[ji];             // (a copy: its fields live in scalar registers)
+    const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15;
+    const int ntb = (j.NT + NFN - 1) / NFN, rb = b % j.rblocks;
+    b /= j.rblocks;
+    const int nt0 = b % ntb * NFN;
+    const int split = b / ntb, r0 = rb * jobs.height, n = min(j.rows - r0, jobs.height);
+    const int fm = (n + 31) / 32;                             // row fragments of a wave
+    const int sper = (j.KS + j.ksplit - 1) / j.ksplit, k0 = min(j.KS, split * sper), ns = min(j.KS, k0 + sper) - k0;
+    const int wn = wave & 3, wm = wave >> 2;
+    f32x4 acc[FN][FMAX];
+#pragma unroll
+    for (int x = 0; x < FN; ++x)
+#pragma unroll
+        for (int y = 0; y < FMAX; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](auto fmc) __attribute__((always_inline)) {
+        constexpr int FM = decltype(fmc)::value, KK = TlmWide::kk(FM), ST = TlmWide::stages(FM), NF = NFN + 2 * FM;
+        static_assert((size_t)ST * KK * NF * 1024 <= TlmWide::smem(), "the ring");
+        // fragments that this wave brings to a stage: NW of the weights, NX of the KK x 2 FM of the activations, the last one in the first REST waves
+        constexpr int NW = 2 * KK, AF = KK * 2 * FM, NX = (AF + 7) / 8, REST = AF % 8;
+        const bool all = REST == 0 || wave < REST;
+        auto act = [&](int i) __attribute__((always_inline)) { return min(wave + 8 * i, AF - 1); };
+        const u32x4 *wq[NW], *xq[NX];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) wq[i] = j.wp + ((long)min(nt0 + wave + 8 * (i / KK), j.NT - 1) * j.KS + k0 + i % KK) * 64;
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {                        // (rows past n repeat the last one, and are dropped at the end)
+            xq[i] = tlm_row(j, r0 + min(act(i) % (2 * FM) * 16 + bl, n - 1), 0, lane) + (long)(k0 + act(i) / (2 * FM)) * 64;
+        }
+        const int stages = (ns + KK - 1) / KK;
+        int to = 0, from = 0, left = stages;                  // places in the ring: of the next stage to load, of the next k-step to read; stages to load
+        auto fetch = [&]() __attribute__((always_inline)) {
+            // (an odd number of k-steps: the last stage gets the last one twice - stages are counted in loads)
+            const int back = KK == 2 && --left == 0 && (ns & 1) ? 1 : 0;
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                mmi_load_lds(i % KK ? wq[i] - back * 64 : wq[i], lane * 16, lds, ((to * KK + i % KK) * NF + wave + 8 * (i / KK)) * 64);
+                wq[i] += KK * 64;
+            }
+#pragma unroll
+            for (int i = 0; i < NX; ++i)
+                if (i + 1 < NX || all) {
+                    const int k = act(i) / (2 * FM);
+                    mmi_load_lds(k ? xq[i] - back * 64 : xq[i], lds, ((to * KK + k) * NF + NFN + act(i) - k * 2 * FM) * 64);
+                    xq[i] += KK * 64;
+                }
+            to = to + 1 < ST ? to + 1 : 0;
+        };
+        auto wait = [&](int behind) __attribute__((always_inline)) {      // until only the last `behind` stages are in flight
+            if (all) {
+                if (ST > 3 && behind == 3) mmi_wait_loads<(ST > 3 ? 3 : 0) * (NW + NX)>();
+                else if (behind == 2) mmi_wait_loads<2 * (NW + NX)>();
+                else if (behind == 1) mmi_wait_loads<NW + NX>();
+                else mmi_wait_loads<0>();
+            } else {
+                if (ST > 3 && behind == 3) mmi_wait_loads<(ST > 3 ? 3 : 0) * (NW + NX - 1)>();
+                else if (behind == 2) mmi_wait_loads<2 * (NW + NX - 1)>();
+                else if (behind == 1) mmi_wait_loads<NW + NX - 1>();
+                else mmi_wait_loads<0>();
+            }
+        };
+        u32x4 av[2][FN], bv[2][FM];
+        auto read = [&](int set, int i) __attribute__((always_inline)) {      // fragment i of FN + FM: rows first, they meet every feature
+            const u32x4* base = lds + from * NF * 64 + lane;
+            if (i < FM) bv[set][i < FM ? i : 0] = base[(NFN + wm * FM + i) * 64];
+            else av[set][i < FM ? 0 : i - FM] = base[(wn * FN + i - FM) * 64];
+        };
+        // products of k-step s (register set `cur`); between them the LDS reads of k-step s + 1.  Where that one begins a stage, every wave has
+        // the stage in hand in its registers: its place is loaded again
+        auto step = [&](auto set, int s) __attribute__((always_inline)) {
+            constexpr int cur = decltype(set)::value;
+            const bool more = s + 1 < ns;
+            if ((KK == 1 || cur == 1) && more) {
+                const int c = s / KK;                         // this stage
+                wait(min(stages - 1, c + ST - 1) - (c + 1));
+                mmi_meet();
+                if (c + ST < stages) fetch();
+            }
+#pragma unroll
+            for (int x = 0; x < FN; ++x) {
+                if (more) {
+#pragma unroll
+                    for (int i = x * (FN + FM) / FN; i < (x + 1) * (FN + FM) / FN; ++i) read(cur ^ 1, i);
+                }
+                mmi_sched_barrier();
+#pragma unroll
+                for (int y = 0; y < FM; ++y) acc[x][y] = Tr::mfma(av[cur][x], bv[cur][y], acc[x][y]);
+            }
+            from = from + 1 < ST * KK ? from + 1 : 0;
+        };
+        const int first = min(stages, ST);
+        for (int s = 0; s < first; ++s) fetch();
+        wait(first - 1);
+        mmi_meet();
+#pragma unroll
+        for (int i = 0; i < FN + FM; ++i) read(0, i);
+        from = 1;
+        int s = 0;
+#pragma unroll 1
+        for (; s + 1 < ns; s += 2) {
+            step(std::integral_constant<int, 0>(), s);
+            step(std::integral_constant<int, 1>(), s + 1);
+        }
+        if (s < ns) step(std::integral_constant<int, 0>(), s);
+    };
+    if (ns > 0) {
+        if (fm == 8) products(std::integral_constant<int, 8>());
+        else if (fm == 7) products(std::integral_constant<int, 7>());
+        else if (fm == 6) products(std::integral_constant<int, 6>());
+        else if (fm == 5) products(std::integral_constant<int, 5>());
+        else if (fm == 4) products(std::integral_constant<int, 4>());
+        else if (fm == 3) products(std::integral_constant<int, 3>());
+        else if (fm == 2) products(std::integral_constant<int, 2>());
+        else products(std::integral_constant<int, 1>());
+    }
+    __syncthreads();
+    tlm_with_epilogue(j.epi, [&](auto epi) __attribute__((always_inline)) {
+        const int nx = min(FN, j.NT - nt0 - wn * FN);
+        f32x4* buf = reinterpret_cast<f32x4*>(lds) + wave * FN * 64 + lane;
+#pragma unroll 1
+        for (int y = 0; y < fm; ++y) {                        // through LDS (a lane reads what it wrote): the epilogue's code is there once
+#pragma unroll
+            for (int c = 0; c < FMAX; ++c)
+                if (c == y)
+#pragma unroll
+                    for (int x = 0; x < FN; ++x) buf[x * 64] = acc[x][c];
+            const int m = (wm * fm + y) * 16 + bl;
+            if (m >= n) continue;
+#pragma unroll 1
+            for (int x = 0; x < nx; ++x) tlm_epilogue<Tr, decltype(epi)::value>(j, 0, split, r0 + m, nt0 + wn * FN + x, lane >> 4, buf[x * 64]);
         }
     });
 }

@@ -81,6 +81,64 @@ def test_prompt_at_once_on_the_simulator(model, T, forms, monkeypatch, capfd):
     check_prompt_at_once("cpu", lib, model, T, torch.bfloat16, forms, monkeypatch, capfd)
 
 
+def check_wide_heights(device, lib, model, T, heights, monkeypatch, capfd):
+    """k_tlm_gemm_wide forms every sum as k_tlm_gemm_tile does: with the same splits a prompt's logits have the same bits, however high its blocks are."""
+    monkeypatch.setenv("MMI_TLM_FORMS", "1")
+    sd = random_token_lm_state_dict(model, seed=T, device=device)
+    prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
+    want = sorted({0, 15, 16, 31, 32, 63, 64, T // 2, T - 2, T - 1})
+    base = None
+    for height in [None, *heights]:
+        monkeypatch.setenv("MMI_TLM_WIDE", str(height)) if height else monkeypatch.delenv("MMI_TLM_WIDE", raising=False)
+        lm = TokenLM(sd, model, dtype=torch.bfloat16, max_slots=1, max_tokens=4096, max_step_tokens=T, **({} if lib is None else {"device": device, "lib": lib}))
+        capfd.readouterr()
+        got = lm.step([(lm.open(), prompt, want)])
+        forms = {line.split(",")[0] for line in capfd.readouterr().err.splitlines() if line.startswith("wide ")}
+        assert forms == ({f"wide 256x{height}"} if height else set())
+        base = got if base is None else base
+        assert torch.equal(got, base), height
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model,T,heights", [
+    (dense_model(1040, 1200), 641, [32, 64, 96, 128, 160, 192, 224, 256]),      # 33 k-steps (one more than whole pairs), 65 and 163 n-tiles, a last block of one row
+    (dense_model(1024, 2048), 97, [32, 96, 256]),                               # 32 and 64 k-steps, three rows in the last fragment, blocks higher than the rows
+    (dense_model(48, 80), 300, [96, 160, 256]),                                 # two k-steps: fewer than the ring has places
+], ids=["odd", "even", "short"])
+def test_wide_blocks_have_the_bits_of_the_narrow_ones(model, T, heights, monkeypatch, capfd):
+    check_wide_heights("cuda", None, model, T, heights, monkeypatch, capfd)
+
+
+@pytest.mark.parametrize("model,T,heights", [(dense_model(144, 200), 270, [32, 64, 96, 128, 160, 192, 224, 256]), (dense_model(48, 80), 97, [64, 128, 256])], ids=["odd", "short"])
+def test_wide_blocks_on_the_simulator(model, T, heights, monkeypatch, capfd):
+    import os
+    import sys
+    from pathlib import Path
+    from moshi_amd import _capi
+    monkeypatch.setenv("MMI_NO_GRAPH", "1")
+    sys.path.insert(0, str(Path(__file__).resolve().parent / "hipsim"))
+    import build_sim
+    lib = _capi.load_tlm(os.environ.get("MMI_TLM_SIM_LIB") or build_sim.build_tlm())
+    check_wide_heights("cpu", lib, model, T, heights, monkeypatch, capfd)
+
+
+@pytest.mark.gpu
+def test_large_prompts_take_wide_blocks(monkeypatch, capfd):
+    """Chosen by the sizes alone, with splits of its own: the logits of a prompt fed at once are those of the same prompt in portions of 64."""
+    monkeypatch.setenv("MMI_TLM_FORMS", "1")
+    model, T = dense_model(4160, 12000), 300
+    sd = random_token_lm_state_dict(model, seed=T, device="cuda")
+    lm = TokenLM(sd, model, dtype=torch.bfloat16, max_slots=2, max_tokens=4096, max_step_tokens=T)
+    prompt = torch.randint(0, model.vocab, (T,), generator=torch.Generator().manual_seed(T)).tolist()
+    want = [0, 63, 64, 159, 160, T - 1]
+    capfd.readouterr()
+    whole = lm.step([(lm.open(), prompt, want)])
+    assert "wide 256x160" in {line.split(",")[0] for line in capfd.readouterr().err.splitlines()}
+    b = lm.open()
+    parts = torch.cat([lm.step([(b, prompt[i:i + 64], [w - i for w in want if i <= w < i + 64])]) for i in range(0, T, 64)])
+    assert float((whole - parts).double().norm() / parts.double().norm()) < 8e-3      # (as in check_prompt_at_once)
+
+
 @pytest.mark.parametrize("rise", [0.0, 0.3, 3.7, 7.9, 8.1, 40.0])
 def test_the_largest_weight_is_exactly_one(tmp_path, rise):
     """bf16 attention rounds a weight relative to itself, so it must be formed against the maximum so far: the largest one is then exact,
