@@ -111,6 +111,10 @@ int mmi_mimi_num_codebooks(const mmi_mimi* m);
  * zero the streaming state of `batch` rows; exec mask all ones. */
 int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream);
 int mmi_mimi_streaming_stop(mmi_mimi* m);
+/* The same around one call on whole files (compression.py:354-359, 412-416): a fresh stream of `batch` rows, which ends with the work on the
+ * device done.  What it has allocated and built may stay for the next one (at most 128 MB, until mmi_mimi_streaming_start or destroy). */
+int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream);
+int mmi_mimi_file_stop(mmi_mimi* m);
 /* Rows of the current stream (StreamingModule._streaming_state.batch_size); 0 when not streaming. */
 int mmi_mimi_streaming_batch(const mmi_mimi* m);
 

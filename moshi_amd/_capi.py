@@ -122,6 +122,8 @@ SIGNATURES = {
     "mmi_mimi_decode_latent": (C.c_int, [_P, _P, _P, C.c_int32, C.c_int32, C.c_int32, _P]),
     "mmi_mimi_decode_step": (C.c_int, [_P, _P, _P, C.c_int32, C.c_int32, C.c_int32, _P]),
     "mmi_mimi_decode_step_strided": (C.c_int, [_P, _P, C.c_int64, _P, C.c_int32, C.c_int32, C.c_int32, _P]),
+    "mmi_mimi_file_start": (C.c_int, [_P, C.c_int32, _P]),
+    "mmi_mimi_file_stop": (C.c_int, [_P]),
     "mmi_mimi_streaming_batch": (C.c_int, [_P]),
     "mmi_lm_streaming_batch": (C.c_int, [_P]),
     "mmi_duplex_create": (C.c_int, [_P, _P, C.POINTER(_P)]),

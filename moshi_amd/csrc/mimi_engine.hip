@@ -117,6 +117,7 @@ struct DequantScratch {
 // them at the ~4.7 us a dependent launch costs; 136 launches and 90 ms now), 3.7 ms in one group of 129, both with the stream's start and stop.
 struct MimiGroup {
     int frames = 0;                            // 0: not built (for this stream)
+    bool earlier = false;                      // built for an earlier file, and not used by this one yet
     bool refused = false;                      // building failed (shapes, memory): this stream goes frame by frame
     MimiSlab slab;
     MmiProgram prog;
@@ -171,6 +172,8 @@ struct mmi_mimi {
     MmiProgram enc_prog, dec_prog;
     hipStream_t cap_stream = nullptr;
     bool use_graph = true;
+    bool parked = false;                       // not streaming; the state and the programs of the last file's stream are still here ...
+    int parked_k = 0;                          // ... built for so many codebooks
 };
 
 namespace {
@@ -1312,6 +1315,7 @@ int group_frames(mmi_mimi* m, const MimiGroup& g, const HistTable& tab, int left
 // memory), with nothing left of the attempt - no buffers, and no error for the next launch check to find.
 bool ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
     MimiGroup& g = enc ? m->enc_grp : m->dec_grp;
+    g.earlier = false;
     if (g.frames == frames) return true;
     MimiMem mem;
     mem.slab = &g.slab;
@@ -1342,7 +1346,10 @@ bool ready_group(mmi_mimi* m, bool enc, int frames, hipStream_t s) {
 // A stream that runs single frames gives back what groups of an earlier one have left here.  (Not at the end of every stream: a file encoded or
 // decoded without a stream of its own is one, and hipFree of 100 MB or more takes some 0.3 ms.)
 void give_back_group(MimiGroup& g, hipStream_t s) {
-    if (!g.frames && g.slab.size && !recording(s)) g.slab.release();
+    if ((g.frames && !g.earlier) || !g.slab.size || recording(s)) return;
+    g.prog.clear();
+    g.frames = 0;
+    g.slab.release();
 }
 
 // The group's launches, and behind them on the host - while the GPU works on them - the capture of the frame program, so that a stream's
@@ -1488,9 +1495,18 @@ extern "C" int mmi_mimi_create(const mmi_mimi_cfg* cfg, const mmi_tensor_desc* w
     return MMI_OK;
 }
 
+// lets go what the last file's stream has left
+static void drop_parked(mmi_mimi* m) {
+    if (!m->parked) return;
+    m->parked = false;
+    m->streaming = true;
+    mmi_mimi_streaming_stop(m);
+}
+
 extern "C" void mmi_mimi_destroy(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return;
+    drop_parked(m);
     mmi_mimi_streaming_stop(m);
     m->enc_grp.slab.release();
     m->dec_grp.slab.release();
@@ -1562,6 +1578,7 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
     if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
     if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
+    drop_parked(m);
     int rc = start_stream(m, batch, (hipStream_t)stream);
     if (rc == MMI_ERR_HIP && (m->enc_grp.slab.size || m->dec_grp.slab.size)) {      // without what an earlier stream's groups have left
         m->enc_grp.slab.release();
@@ -1588,6 +1605,43 @@ extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
     m->partial_sizes.clear();
     m->streaming = false;
     m->batch = 0;
+    return MMI_OK;
+}
+
+// A file is a stream that nobody else sees.  Starting and stopping one took 350 us - 32 MB allocated, zeroed and freed, two launch lists built,
+// captured and dropped - where 8 frames take the GPU some 250; so what it has built stays for the next file of as many streams, which resets the
+// state instead.  At most MIMI_PARK bytes stay (the full-size codec: three streams), until a stream of the caller's own starts, a file of
+// another number of streams or codebooks, or the handle goes.
+constexpr size_t MIMI_PARK = (size_t)128 << 20;
+
+extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
+    MmiDeviceGuard dev_guard_(m ? m->device : -1);
+    if (!m || !m->parked || m->batch != batch || m->parked_k != m->n_codebooks || recording((hipStream_t)stream)) return mmi_mimi_streaming_start(m, batch, stream);
+    m->parked = false;
+    m->streaming = true;
+    m->all_exec = 1;
+    m->mask_in_graph = false;
+    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {
+        g->refused = false;
+        g->earlier = true;
+    }
+    const int rc = mmi_mimi_reset(m, nullptr, stream);
+    if (rc) mmi_mimi_streaming_stop(m);
+    return rc;
+}
+
+extern "C" int mmi_mimi_file_stop(mmi_mimi* m) {
+    MmiDeviceGuard dev_guard_(m ? m->device : -1);
+    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
+    if (!m->streaming) return MMI_OK;
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess || m->st.held() > MIMI_PARK || getenv("MMI_DEBUG_POISON")) {
+        mmi_mimi_streaming_stop(m);
+        return e == hipSuccess ? (int)MMI_OK : mmi_fail(MMI_ERR_HIP, std::string("hipDeviceSynchronize: ") + hipGetErrorString(e));
+    }
+    m->streaming = false;
+    m->parked = true;
+    m->parked_k = m->n_codebooks;
     return MMI_OK;
 }
 
@@ -1632,6 +1686,27 @@ extern "C" int mmi_mimi_reset(mmi_mimi* m, const uint8_t* mask, mmi_stream strea
     hipStream_t s = (hipStream_t)stream;
     const int B = m->batch;
     mask_changes(m, !mask || m->all_exec == 1 ? 1 : -1, s);
+    if (m->enc_tab.n >= 0 && m->dec_tab.n >= 0 && m->partials.size() <= MMI_PARTIALS_MAX) {
+        ResetTable t;
+        memset(&t, 0, sizeof(t));
+        t.hist[0] = m->enc_tab;
+        t.hist[1] = m->dec_tab;
+        t.rows[0] = m->enc_hist_rows;
+        t.rows[1] = m->dec_hist_rows;
+        t.B = B;
+        t.counters = m->counters;
+        t.first = m->first;
+        t.exec = m->exec;
+        long n = 0;
+        for (size_t i = 0; i < m->partials.size(); ++i) {
+            t.part[t.n_part] = m->partials[i];
+            t.part_row[t.n_part] = m->partial_sizes[i];
+            t.part_end[t.n_part++] = n += (long)B * m->partial_sizes[i];
+        }
+        MMI_LAUNCH(k_reset_all, (int)mmi_cdiv64(t.rows[0] + t.rows[1] + n + B, 256), 256, 0, s, t, mask);
+        MMI_CHECK_LAUNCH();
+        return MMI_OK;
+    }
     if (m->enc_hist_rows > 0)
         MMI_LAUNCH(k_reset_history, mmi_cdiv(m->enc_hist_rows, 256), 256, 0, s, (const HistDesc*)m->enc_hist, m->enc_nhist, m->enc_hist_rows, mask);
     if (m->dec_hist_rows > 0)

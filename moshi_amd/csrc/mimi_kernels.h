@@ -1441,6 +1441,48 @@ __global__ void k_reset_history(const HistDesc* __restrict__ descs, int ndesc, i
     for (int p = 0; p < h.H; ++p) r[p] = 0.f;
 }
 
+// A reset in one launch: the histories of both directions, the overlap-adds' partial rows, then a stream's offsets and flags, where mask
+// (null: everywhere)
+#define MMI_PARTIALS_MAX 12
+struct ResetTable {
+    HistTable hist[2];
+    int rows[2];
+    float* part[MMI_PARTIALS_MAX];
+    long part_end[MMI_PARTIALS_MAX], part_row[MMI_PARTIALS_MAX];      // running ends in elements, elements per stream
+    int n_part, B;
+    long* counters; uint8_t *first, *exec;
+};
+__global__ void k_reset_all(ResetTable t, const uint8_t* __restrict__ mask) {
+    long at = (long)blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        if (at >= 0 && at < t.rows[side]) {
+            int d = 0;
+#pragma unroll
+            for (int i = 1; i < MMI_HIST_MAX; ++i)
+                if (i < t.hist[side].n && t.hist[side].d[i].row_begin <= at) d = i;
+            const HistDesc h = t.hist[side].d[d];
+            const int row = (int)at - h.row_begin;
+            if (mask && !mask[row / h.C]) return;
+            for (int p = 0; p < h.H; ++p) h.p[(long)row * h.ld + p] = 0.f;
+            return;
+        }
+        at -= t.rows[side];
+    }
+    long begin = 0;
+    for (int i = 0; i < t.n_part; ++i) {
+        if (at >= begin && at < t.part_end[i]) {
+            if (!mask || mask[(at - begin) / t.part_row[i]]) t.part[i][at - begin] = 0.f;
+            return;
+        }
+        begin = t.part_end[i];
+    }
+    const int b = (int)(at - begin);
+    if (b < 0 || b >= t.B || (mask && !mask[b])) return;
+    t.counters[b] = t.counters[t.B + b] = 0;
+    t.first[b] = t.exec[b] = 1;
+}
+
 // generic masked fill of per-row state: buf[b][0..n) = 0 where mask
 __global__ void k_reset_rows_f32(float* __restrict__ buf, long n_per_row, int B, const uint8_t* __restrict__ mask) {
     long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -107,6 +107,12 @@ struct MmiArena {
         at += (nb + 255) & ~(size_t)255;
         return hipSuccess;
     }
+    size_t held() const {                          // bytes of device memory
+        size_t n = chunks.size() * chunk;
+        for (size_t i = 0; i < ptrs.size(); ++i)
+            if (!cut(ptrs[i])) n += sizes[i];
+        return n;
+    }
     bool cut(const void* p) const {                // is it part of a chunk?
         for (const char* c : chunks)
             if (p >= c && p < c + chunk) return true;

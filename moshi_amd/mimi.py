@@ -164,6 +164,17 @@ class MimiModel:
         self._batch = None
 
     @contextmanager
+    def _file(self, batch_size: int):
+        """The stream of a call on whole files (a fresh one; done with the device's work when the call returns)."""
+        self._lib.check(self._lib.mmi_mimi_file_start(self._handle, int(batch_size), self._stream()))
+        self._batch = int(batch_size)
+        try:
+            yield
+        finally:
+            self._lib.check(self._lib.mmi_mimi_file_stop(self._handle))
+            self._batch = None
+
+    @contextmanager
     def streaming(self, batch_size: int):
         self.streaming_forever(batch_size)
         try:
@@ -218,27 +229,25 @@ class MimiModel:
 
     def _encode_impl(self, x: torch.Tensor, want_latent: bool) -> torch.Tensor:
         x = self._check_audio(x)
-        temporary = not self.is_streaming
-        if temporary:
+        if not self.is_streaming:
             # non-streaming call == streaming from a fresh state over the right-padded signal (compression.py:354-359)
-            fs = self.frame_size
-            pad = (-x.shape[-1]) % fs
+            pad = (-x.shape[-1]) % self.frame_size
             if pad:
                 x = torch.nn.functional.pad(x, (0, pad))
-            self.streaming_forever(x.shape[0])
-        try:
-            B = x.shape[0]
-            n = self._frames_streaming(x)
-            if want_latent:
-                out = torch.empty(B, self.dimension, n, device=self.device, dtype=torch.float32)
-                rc = self._lib.mmi_mimi_encode_latent_step(self._handle, x.data_ptr(), out.data_ptr(), B, n, self._stream())
-            else:
-                out = torch.empty(B, self.num_codebooks, n, device=self.device, dtype=torch.int64)
-                rc = self._lib.mmi_mimi_encode_step(self._handle, x.data_ptr(), out.data_ptr(), B, n, self._stream())
-            self._lib.check(rc)
-        finally:
-            if temporary:
-                self._stop_streaming()
+            with self._file(x.shape[0]):
+                return self._encode_frames(x, want_latent)
+        return self._encode_frames(x, want_latent)
+
+    def _encode_frames(self, x: torch.Tensor, want_latent: bool) -> torch.Tensor:
+        B = x.shape[0]
+        n = self._frames_streaming(x)
+        if want_latent:
+            out = torch.empty(B, self.dimension, n, device=self.device, dtype=torch.float32)
+            rc = self._lib.mmi_mimi_encode_latent_step(self._handle, x.data_ptr(), out.data_ptr(), B, n, self._stream())
+        else:
+            out = torch.empty(B, self.num_codebooks, n, device=self.device, dtype=torch.int64)
+            rc = self._lib.mmi_mimi_encode_step(self._handle, x.data_ptr(), out.data_ptr(), B, n, self._stream())
+        self._lib.check(rc)
         return out
 
     def encode(self, x: torch.Tensor) -> torch.Tensor:
@@ -276,14 +285,14 @@ class MimiModel:
         strided = codes.stride(2) == 1 and codes.stride(1) == n and codes.stride(0) >= K * n
         if not strided:
             codes = codes.contiguous()
-        temporary = not self.is_streaming
-        if temporary:
-            self.streaming_forever(B)
-        try:
-            out = torch.empty(B, self.channels, n * self.frame_size, device=self.device, dtype=torch.float32)
-            self._lib.check(self._lib.mmi_mimi_decode_step_strided(self._handle, codes.data_ptr(), codes.stride(0), out.data_ptr(),
-                                                                   B, K, n, self._stream()))
-        finally:
-            if temporary:
-                self._stop_streaming()
+        if not self.is_streaming:
+            with self._file(B):
+                return self._decode_frames(codes)
+        return self._decode_frames(codes)
+
+    def _decode_frames(self, codes: torch.Tensor) -> torch.Tensor:
+        B, K, n = codes.shape
+        out = torch.empty(B, self.channels, n * self.frame_size, device=self.device, dtype=torch.float32)
+        self._lib.check(self._lib.mmi_mimi_decode_step_strided(self._handle, codes.data_ptr(), codes.stride(0), out.data_ptr(),
+                                                               B, K, n, self._stream()))
         return out

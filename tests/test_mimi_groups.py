@@ -218,6 +218,70 @@ def test_a_stream_starts_where_groups_hold_the_memory(sim_lib):
     assert torch.equal(m.encode(x), want)
 
 
+def check_files_in_a_row(make, device, cfg, lengths, K=4):
+    """A handle keeps what one file's stream has built for the next one: every file gives the bits that a fresh handle gives - after files of
+    other lengths, of NaNs and infinities, of more rows, after a stream of the caller's own, with other codebooks, in either direction."""
+    sd = random_mimi_state_dict(cfg, seed=11, device=device)
+    gen = torch.Generator().manual_seed(13)
+    m, fs = make(sd, cfg, K, 3), cfg.frame_size
+
+    def file(B, n, k=K, bad=None):
+        x = (0.3 * torch.randn(B, 1, n * fs - 5, generator=gen)).to(device)
+        q = torch.randint(0, cfg.q_bins, (B, k, n), generator=gen).to(device)
+        if bad is not None:
+            x[:, :, ::7] = bad
+        return x, q
+
+    def same(x, q):
+        fresh = make(sd, cfg, m.num_codebooks, 3)
+        for got, want in ((m.encode(x), fresh.encode(x)), (m.decode(q), fresh.decode(q)), (m.encode_to_latent(x, quantize=False), fresh.encode_to_latent(x, quantize=False))):
+            assert torch.equal(got, want) or (torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()))
+    for n in lengths:
+        same(*file(1, n))
+    for bad in (float("nan"), float("inf")):
+        same(*file(1, lengths[0], bad=bad)), same(*file(1, lengths[0]))
+    same(*file(2, 3)), same(*file(2, 3)), same(*file(1, lengths[0]))
+    x, q = file(1, 3)
+    with m.streaming(1):
+        m.encode(x[..., :fs].contiguous()), m.decode(q)
+    same(x, q)
+    m.set_num_codebooks(2)
+    same(x, q[:, :2]), same(x, q[:, :1])
+    with pytest.raises(AssertionError, match="codebooks"):
+        m.decode(torch.zeros(1, cfg.q_n_q + 1, 2, dtype=torch.int64, device=device))
+    same(x, q[:, :2])
+
+
+def test_files_in_a_row(sim_lib):
+    check_files_in_a_row(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", tiny_mimi_config(), (4, 1, 4, 6))
+
+
+@pytest.mark.gpu
+def test_full_size_files_in_a_row():
+    check_files_in_a_row(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cuda", max_batch=mb, num_codebooks=K), "cuda", MimiConfig(), (40, 1, 40, 170, 9), K=8)
+
+
+def test_what_a_file_leaves_goes_with_the_next_stream(sim_lib):
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    gc.collect()
+    empty = sim_bytes(sim_lib)
+    m = MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+    before = sim_bytes(sim_lib)
+    with m.streaming(2):
+        stream = sim_bytes(sim_lib) - before
+    m.encode(torch.zeros(1, 1, cfg.frame_size))
+    assert 0 < sim_bytes(sim_lib) - before <= 128 << 20
+    assert not m.is_streaming
+    with m.streaming(2):
+        assert sim_bytes(sim_lib) == before + stream
+    assert sim_bytes(sim_lib) == before
+    m.encode(torch.zeros(1, 1, cfg.frame_size))
+    del m
+    gc.collect()
+    assert sim_bytes(sim_lib) == empty
+
+
 def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
     """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
     stream it is called on, and leaves the one that the snapshot came from alone."""
