@@ -301,6 +301,11 @@ __device__ __forceinline__ void mmi_store_relaxed_agent(unsigned* p, unsigned v)
 // The instruction scheduler moves nothing across this point: keeps a batch of loads issued ahead of the products that consume the batch
 // before it (left alone it sinks each load to its use when registers are short, and the loads then wait for one another)
 __device__ __forceinline__ void mmi_sched_barrier() { __builtin_amdgcn_sched_barrier(0); }
+// x is computed here and unknown from here on.  Without it the compiler moves arithmetic whose result is only used much later down to that
+// use, across barriers, and keeps all the operands it read from LDS until then; and it computes the addresses of all a kernel's phases, where
+// they follow from one lane index, at the kernel's start, and keeps those
+template <class T>
+__device__ __forceinline__ void mmi_here(T& x) { asm volatile("" : "+v"(x)); }
 // a value that is the same in every lane (a wave index, what was loaded through one), told to the compiler: it stays in scalar registers,
 // and loads addressed by it are scalar loads - they do not queue behind the vector loads in flight
 __device__ __forceinline__ int mmi_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }

@@ -1432,6 +1432,18 @@ int launch_state_step(hipStream_t s, const TlmLinArgs& a, int n) {
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
+template <int NP>
+int launch_chunk_delta_t(hipStream_t s, const TlmLinArgs& a, int n_chunk) {
+    const size_t smem = tlm_chunk_delta_smem();
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta<NP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    MMI_HIP_CHECK(attr);
+    MMI_LAUNCH(k_tlm_chunk_delta<NP>, dim3(n_chunk, a.heads), 512, smem, s, a);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
+int launch_chunk_delta(hipStream_t s, const TlmLinArgs& a, int n_chunk) {
+    return a.dim_p <= 64 ? launch_chunk_delta_t<1>(s, a, n_chunk) : (a.dim_p <= 128 ? launch_chunk_delta_t<2>(s, a, n_chunk) : launch_chunk_delta_t<4>(s, a, n_chunk));
+}
 template <bool DELTA>
 int launch_chunk_scan(hipStream_t s, const TlmLinArgs& a, int n_unit) {
     const int grid = 8 * mmi_cdiv(n_unit * a.heads, 8) * (a.vdim_p / 16), nd = a.dim_p / 16;
@@ -1539,10 +1551,8 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         P.site(site + "chunk");
         P.add([=](hipStream_t s) {
             if (delta) {
-                const size_t smem = tlm_chunk_delta_smem();
-                static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-                MMI_HIP_CHECK(attr);
-                MMI_LAUNCH(k_tlm_chunk_delta, dim3(n_chunk, a.heads), 256, smem, s, a);
+                const int rc = launch_chunk_delta(s, a, n_chunk);
+                if (rc != MMI_OK) return rc;
             } else {
                 MMI_LAUNCH(k_tlm_chunk_lightning, dim3(n_chunk, a.heads), 256, 0, s, a);
             }

@@ -13,8 +13,8 @@
 //   S_end = G_end S_0 + sum_s (G_end/G_s k_s) u_s^T
 //
 // so W = (I + A)^-1 diag(b) (G K) and U0 = (I + A)^-1 diag(b) V turn the system into U = U0 - W S_0.  Decay ratios are never formed by a
-// division or from logarithms: inside 16 tokens they are running products, across them (product to the end of s's 16) x (whole 16s between)
-// x (product from the start of t's 16), so that they lose nothing however strong the decay is, and underflow to the zero they stand for.
+// division or from logarithms: inside 8 tokens they are running products, across them (product to the end of s's 8) x (whole 8s between)
+// x (product from the start of t's 8), so that they lose nothing however strong the decay is, and underflow to the zero they stand for.
 #pragma once
 #include "tlm_kernels.h"
 
@@ -47,19 +47,29 @@ struct TlmLinArgs {
 
 // decay of channel d of a head: exp(-factor softplus(z)), z = projection + summand, as 2^(-factor log2(1 + e^z)).  With u = e^z rounded
 // and w = 1 + u rounded, log2(w) u / (w - 1) is log2(1 + u) to the last bits however small u is.
-__device__ __forceinline__ float tlm_decay(const TlmLinArgs& a, long row, int h, int d) {
+__device__ __forceinline__ float tlm_decay(float z, float factor) {
     constexpr float LOG2E = 1.44269504088896340736f;
-    const int c = h * a.dim_p + d;
-    const float z = a.decay[row * a.heads * a.dim_p + c] + a.decay_c[c];
     const float u = mmi_fast_exp2f(fminf(z, 30.f) * LOG2E), w = 1.0f + u;
     float l = w > 1.0f ? mmi_fast_log2f(w) * u / (w - 1.0f) : u * LOG2E;
     if (z > 20.f) l = z * LOG2E;
-    return mmi_fast_exp2f(-a.decay_c[a.heads * a.dim_p + c] * l);
+    return mmi_fast_exp2f(-factor * l);
+}
+__device__ __forceinline__ float tlm_decay(const TlmLinArgs& a, long row, int h, int d) {
+    const int c = h * a.dim_p + d;
+    return tlm_decay(a.decay[row * a.heads * a.dim_p + c] + a.decay_c[c], a.decay_c[a.heads * a.dim_p + c]);
 }
 __device__ __forceinline__ float tlm_silu(float x) { return x * tlm_sigmoid(x); }
 
 // element (row, k) of an operand with `ks` 16-wide blocks per 16 rows
 MMI_HD long tlm_tile(int row, int k, int ks) { return (((long)(row >> 4) * ks + (k >> 4)) * 64 + ((k & 15) >> 2) * 16 + (row & 15)) * 4 + (k & 3); }
+
+// four floats of a buffer whose start is the same in every lane: its address stays in scalar registers, a lane adds 32 bits
+template <class T = f32x4, class F>
+__device__ __forceinline__ auto& tlm_quad(F* base, int at) {
+    using C = std::conditional_t<std::is_const_v<F>, const char, char>;
+    using E = std::conditional_t<std::is_const_v<F>, const T, T>;
+    return *reinterpret_cast<E*>(reinterpret_cast<C*>(base) + 4u * (unsigned)at);
+}
 
 // channel(s) from c of the convolution at token t of a sequence whose rows start at row0 of the projection; four taps are requested at a
 // time (a tap before the sequence's start reads some valid address and counts as zero).  `now`: where the taps - 1 inputs that the next
@@ -301,200 +311,337 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_chunk_lightning(TlmLinArg
 }
 
 // ------------------------------------------------------------------------------------------------
-// chunks, delta: P, W, U0, the decayed queries and transposed keys.  grid: chunks, heads; wave w owns tokens 16 w .. 16 w + 15
+// chunks, delta: P, W, U0, the decayed queries and transposed keys.  grid: chunks, heads; NP: panels of 64 channels, 1, 2 or 4
+// Its bytes bound it where chunks are many (896 of 128 x 128: 250 MB, 65 us = 3.8 TB/s; 113 before), the chain of one workgroup's phases where
+// they are few (192: 23 us; 47 before).  So: eight waves, two on every SIMD and two workgroups on a CU while the registers (126) allow it; the
+// next panel's operands and U0's are asked for a phase ahead; pairs are taken one by one only inside 8 tokens (half the vector work of 16), all
+// others by the matrix core; no right side goes through memory: W's stay in the registers of the wave that solves for them.
 // ------------------------------------------------------------------------------------------------
-inline size_t tlm_chunk_delta_smem() { return (size_t)(3 * TLM_CHUNK * TLM_PST + 4 * 64 + TLM_CHUNK) * sizeof(float); }
-inline __global__ __launch_bounds__(256, 2) void k_tlm_chunk_delta(TlmLinArgs a) {
+constexpr int TLM_SUB = 8;               // tokens whose pairs are taken one by one; decays across them are whole products
+inline size_t tlm_chunk_delta_smem() { return (size_t)(3 * TLM_CHUNK * TLM_PST + (3 * (TLM_CHUNK / TLM_SUB) + 1) * 64) * sizeof(float); }
+template <int NP>
+__global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLinArgs a) {
     MMI_DYN_SHARED(float, sh);
-    float *K = sh, *Q = K + TLM_CHUNK * TLM_PST, *G = Q + TLM_CHUNK * TLM_PST;      // [64][TLM_PST] each
-    float *tot = G + TLM_CHUNK * TLM_PST, *beta = tot + 4 * 64;                     // [4][64], [64]
-    float *A = K, *ti = Q;                                                          // once the panels are done: [64][TLM_PST], [4][16][20]
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), bl = lane & 15, kq = lane >> 4, h = (int)blockIdx.y;
+    float *Q = sh, *K = Q + TLM_CHUNK * TLM_PST, *G = K + TLM_CHUNK * TLM_PST;      // [64][TLM_PST] each
+    float *tot = G + TLM_CHUNK * TLM_PST, *pre = tot + TLM_CHUNK / TLM_SUB * 64, *suf = pre + TLM_CHUNK / TLM_SUB * 64;      // [8][64] each: decay over 8 tokens, over all 8s before, behind
+    float* beta = suf + TLM_CHUNK / TLM_SUB * 64;          // [64]
+    float *A = K, *Pl = Q, *part = G, *ti = G;                                      // once the panels are done: [64][TLM_PST] twice; [4][64][4], then [4][16][20]
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), h = (int)blockIdx.y;
+    int bl = lane & 15, kq = lane >> 4;
     const TlmSeg ck = a.chunk[blockIdx.x];
-    const int D = a.dim_p, V = a.vdim_p, kh = h / (a.heads / a.kv_heads);
+    const int D = a.dim_p, V = a.vdim_p, kh = h / (a.heads / a.kv_heads), nd = D / 16, nv = V / 16;
     const long id = (long)blockIdx.x * a.heads + h;
-    const float* qkv = a.qkv + (long)ck.row0 * a.conv_c;
+    const float *qp = a.qkv + (long)ck.row0 * a.conv_c + a.q0 + kh * D, *kp = qp + (a.k0 - a.q0), *vp = a.qkv + (long)ck.row0 * a.conv_c + a.v0 + h * V;
+    const float *zp = a.decay + ((long)ck.row0 * a.heads + h) * D, *cp = a.decay_c + h * D;
     float *Wg = a.w + id * TLM_CHUNK * D, *Qg = a.qg + id * TLM_CHUNK * D, *Kt = a.kt + id * TLM_CHUNK * D, *Ug = a.u0 + id * TLM_CHUNK * V;
     float* P = a.p + id * (TLM_CHUNK * TLM_CHUNK);
-    if (tid < TLM_CHUNK) beta[tid] = tid < ck.n ? tlm_sigmoid(a.in[(long)(ck.row0 + tid) * a.in_ld + a.b0 + h]) : 0.f;
-    float dA[16], dP[16];                                  // pairs (16 w + bl, 16 w + s) of this lane's quarter of the channels
+    const float bv = a.in[(long)(ck.row0 + min(lane, ck.n - 1)) * a.in_ld + a.b0 + h];
+    // a panel's operands: token lt and the one 32 further on, 4 channels from lc (past the end: a valid address, not used)
+    f32x4 qv[2], kv[2], zv[2], zs, zf;
+    auto load = [&](int c0, int lt, int lc) __attribute__((always_inline)) {
+        const int c = c0 + min(lc, min(64, D - c0) - 4);
+        zs = tlm_quad(cp, c);
+        zf = tlm_quad(cp + a.heads * D, c);
 #pragma unroll
-    for (int s = 0; s < 16; ++s) dA[s] = dP[s] = 0.f;
-    // blocks below the diagonal: wave w takes entries w and w + 4 of (3,0) (3,1) (3,2) (2,0) (2,1) (1,0)
-    const int bi[2] = {wave < 3 ? 3 : 2, wave == 0 ? 2 : 1}, bj[2] = {wave < 3 ? wave : 0, wave == 0 ? 1 : 0};
-    const int nblk = wave < 2 ? 2 : 1;
-    f32x4 oA[2], oP[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) oA[b] = oP[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < D; c0 += 64) {
-        const int cn = min(64, D - c0);                    // a multiple of 16
-        __syncthreads();
-        for (int i = tid; i < TLM_CHUNK * 16; i += 256) {
-            const int t = i >> 4, c = 4 * (i & 15);
-            f32x4 qv = {0.f, 0.f, 0.f, 0.f}, kv = qv, gv = {1.f, 1.f, 1.f, 1.f};
-            if (t < ck.n && c < cn) {
-                qv = *reinterpret_cast<const f32x4*>(qkv + (long)t * a.conv_c + a.q0 + kh * D + c0 + c);
-                kv = *reinterpret_cast<const f32x4*>(qkv + (long)t * a.conv_c + a.k0 + kh * D + c0 + c);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) gv[e] = tlm_decay(a, ck.row0 + t, h, c0 + c + e);
-            }
-            *reinterpret_cast<f32x4*>(Q + t * TLM_PST + c) = qv;
-            *reinterpret_cast<f32x4*>(K + t * TLM_PST + c) = kv;
-            *reinterpret_cast<f32x4*>(G + t * TLM_PST + c) = gv;
+        for (int i = 0; i < 2; ++i) {
+            const int t = min(lt + 32 * i, ck.n - 1);
+            zv[i] = tlm_quad(zp, t * a.heads * D + c);
+            qv[i] = tlm_quad(qp, t * a.conv_c + c);
+            kv[i] = tlm_quad(kp, t * a.conv_c + c);
         }
-        __syncthreads();
-        for (int c = 4 * kq; c < cn; c += 16) {            // the 16 x 16 blocks on the diagonal, pair by pair with a running decay
-            const int t0 = 16 * wave;
-            const f32x4 kt = *reinterpret_cast<const f32x4*>(K + (t0 + bl) * TLM_PST + c), qt = *reinterpret_cast<const f32x4*>(Q + (t0 + bl) * TLM_PST + c);
-            f32x4 d = {1.f, 1.f, 1.f, 1.f};
+    };
+    load(0, tid >> 4, 4 * (tid & 15));
+    if (tid < TLM_CHUNK) beta[tid] = tid < ck.n ? tlm_sigmoid(bv) : 0.f;
+    float dA[TLM_SUB], dP[TLM_SUB];                        // pairs (t, t - i), t = 16 (wave % 4) + bl, of this lane's share of the channels
 #pragma unroll
-            for (int s = 15; s >= 0; --s) {
-                if (s > bl) continue;
-                const f32x4 x = d * *reinterpret_cast<const f32x4*>(K + (t0 + s) * TLM_PST + c);
+    for (int i = 0; i < TLM_SUB; ++i) dA[i] = dP[i] = 0.f;
+    // the 16 x 16 blocks that are products: waves 0 .. 5 those below the diagonal, (3,0) (3,1) (3,2) (2,0) (2,1) (1,0); waves 6, 7 the lower left
+    // quarters of two blocks on the diagonal each (rows 8 .. 15 of a block against its columns 0 .. 7; the other two quarters are dropped)
+    const int bi = wave < 3 ? 3 : (wave < 5 ? 2 : 1), bj = wave < 3 ? wave : (wave < 5 ? wave - 3 : 0);
+    auto row = [&](int l) __attribute__((always_inline)) { return wave < 6 ? 16 * bi + l : 32 * (wave - 6) + 16 * (l >> 3) + (l & 7) + 8; };
+    auto column = [&](int l) __attribute__((always_inline)) { return wave < 6 ? 16 * bj + l : 32 * (wave - 6) + 16 * (l >> 3) + (l & 7); };
+    f32x4 oA = {0.f, 0.f, 0.f, 0.f}, oP = oA;              // transposed: lane (kq, bl) holds columns 4 kq .. 4 kq + 3 of row bl
+    // 16-column strips of [W | U0] that this wave solves for: strip 4 p + wave % 4 of W for every other panel p, then every eighth of U0
+    constexpr int NS = (NP + 1) / 2;
+    f32x4 x[NS + 1][4] = {};
+    const int v0 = (wave + 8 - (4 * NP & 7)) & 7;
+    auto load_u0 = [&](f32x4* u, int v, int bl, int kq) __attribute__((always_inline)) {       // (past the end: the last strip again, not stored)
+        const int at = 16 * min(v, nv - 1) + bl;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u[i][r] = tlm_quad<float>(vp, min(16 * i + 4 * kq + r, ck.n - 1) * a.conv_c + at);
+    };
+    auto panel = [&](int c0, bool mine, f32x4* strip) __attribute__((always_inline)) {
+        const int cn = min(64, D - c0);                    // a multiple of 16
+        int l = lane;
+        mmi_here(l);
+        const int bl = l & 15, kq = l >> 4, lt = 4 * wave + (l >> 4), lc = 4 * (l & 15);
+        if (c0) mmi_meet();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int t = lt + 32 * i;
+            const bool in = t < ck.n && lc < cn;
+            f32x4 g = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float d = tlm_decay(zv[i][e] + zs[e], zf[e]);
+                g[e] = in ? d : 1.f;
+                qv[i][e] = in ? qv[i][e] : 0.f;
+                kv[i][e] = in ? kv[i][e] : 0.f;
+            }
+            *reinterpret_cast<f32x4*>(Q + t * TLM_PST + lc) = qv[i];
+            *reinterpret_cast<f32x4*>(K + t * TLM_PST + lc) = kv[i];
+            *reinterpret_cast<f32x4*>(G + t * TLM_PST + lc) = g;
+        }
+        mmi_meet();
+        if (NP <= 2 ? c0 < 64 * (NP - 1) : c0 < 128 || c0 + 64 < D) load(c0 + 64, lt, lc);
+        else load_u0(x[NS], v0, bl, kq);
+        // pairs inside 8 tokens, with a running decay: token t against t - i.  What t - i before t's 8 gives is dropped at the end: those rows are
+        // others of the chunk, or rows of the panel that lies in front in LDS
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = 16 * (wave & 3) + bl, c = 32 * (wave >> 2) + 16 * j + 4 * kq;
+            const f32x4 kt = *reinterpret_cast<const f32x4*>(K + t * TLM_PST + c), qt = *reinterpret_cast<const f32x4*>(Q + t * TLM_PST + c);
+            f32x4 d = *reinterpret_cast<const f32x4*>(G + t * TLM_PST + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dP[0] = mmi_fma(qt[e], kt[e], dP[0]);
+#pragma unroll
+            for (int i = 1; i < TLM_SUB; ++i) {
+                const f32x4 y = d * *reinterpret_cast<const f32x4*>(K + (t - i) * TLM_PST + c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    dA[s] = mmi_fma(kt[e], x[e], dA[s]);
-                    dP[s] = mmi_fma(qt[e], x[e], dP[s]);
+                    dA[i] = mmi_fma(kt[e], y[e], dA[i]);
+                    dP[i] = mmi_fma(qt[e], y[e], dP[i]);
                 }
-                d *= *reinterpret_cast<const f32x4*>(G + (t0 + s) * TLM_PST + c);
+                if (i + 1 < TLM_SUB) d *= *reinterpret_cast<const f32x4*>(G + (t - i) * TLM_PST + c);
             }
         }
-        __syncthreads();
-        {                                                  // K -> k x (decay from the start of its 16), Q likewise, G -> k x (decay to the end)
-            const int c = lane;
-            float g[16], kk[16];
-            float run = 1.f;
 #pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const int at = (16 * wave + t) * TLM_PST + c;
-                g[t] = G[at];
-                kk[t] = K[at];
-                run *= g[t];
-                K[at] = kk[t] * run;
-                Q[at] *= run;
+        for (int i = 0; i < TLM_SUB; ++i) {
+            mmi_here(dA[i]);
+            mmi_here(dP[i]);
+        }
+        mmi_meet();
+        {                                                  // K -> k x (decay from the start of its 8), Q likewise, G -> k x (decay to the end)
+            const int at = TLM_SUB * wave * TLM_PST + lane;
+            float g[TLM_SUB], kk[TLM_SUB], qq[TLM_SUB], run = 1.f;
+#pragma unroll
+            for (int t = 0; t < TLM_SUB; ++t) {
+                kk[t] = K[at + t * TLM_PST];
+                qq[t] = Q[at + t * TLM_PST];
+                g[t] = G[at + t * TLM_PST];
             }
-            tot[wave * 64 + c] = run;
+#pragma unroll
+            for (int t = 0; t < TLM_SUB; ++t) {
+                run *= g[t];
+                K[at + t * TLM_PST] = kk[t] * run;
+                Q[at + t * TLM_PST] = qq[t] * run;
+            }
+            tot[wave * 64 + lane] = run;
             run = 1.f;
 #pragma unroll
-            for (int t = 15; t >= 0; --t) {
-                G[(16 * wave + t) * TLM_PST + c] = kk[t] * run;
+            for (int t = TLM_SUB - 1; t >= 0; --t) {
+                G[at + t * TLM_PST] = kk[t] * run;
                 run *= g[t];
             }
         }
-        __syncthreads();
+        mmi_meet();
+        {
+            float fp = 1.f, fs = 1.f;                      // this wave's rows of pre and suf
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            if (b >= nblk) continue;
-            for (int c = 4 * kq; c < cn; c += 16) {
-                f32x4 mid = {1.f, 1.f, 1.f, 1.f};
-                for (int m = bj[b] + 1; m < bi[b]; ++m) mid *= *reinterpret_cast<const f32x4*>(tot + m * 64 + c);
-                const u32x4 kv = __builtin_bit_cast(u32x4, *reinterpret_cast<const f32x4*>(G + (16 * bj[b] + bl) * TLM_PST + c) * mid);
-                oA[b] = TlmF32::mfma(*reinterpret_cast<const u32x4*>(K + (16 * bi[b] + bl) * TLM_PST + c), kv, oA[b]);
-                oP[b] = TlmF32::mfma(*reinterpret_cast<const u32x4*>(Q + (16 * bi[b] + bl) * TLM_PST + c), kv, oP[b]);
+            for (int m = 0; m < TLM_CHUNK / TLM_SUB; ++m) {
+                const float v = tot[m * 64 + lane];
+                fp *= m < wave ? v : 1.f;
+                fs *= m > wave ? v : 1.f;
+            }
+            pre[wave * 64 + lane] = fp;
+            suf[wave * 64 + lane] = fs;
+            f32x4 mid[4];                                  // decay of the whole 8s between a row's token and a column's
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mid[j] = f32x4{1.f, 1.f, 1.f, 1.f};
+            if (wave < 6)
+                for (int m = 2 * bj + 2; m < 2 * bi; ++m)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) mid[j] *= *reinterpret_cast<const f32x4*>(tot + m * 64 + 16 * j + 4 * kq);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {                  // (channels past the end: zeros)
+                const int c = 16 * j + 4 * kq;
+                f32x4 kt = *reinterpret_cast<const f32x4*>(K + row(bl) * TLM_PST + c), qt = *reinterpret_cast<const f32x4*>(Q + row(bl) * TLM_PST + c);
+                f32x4 ks = *reinterpret_cast<const f32x4*>(G + column(bl) * TLM_PST + c);
+                if (wave < 6) {
+                    const f32x4 tt = *reinterpret_cast<const f32x4*>(tot + 2 * bi * 64 + c), ts = *reinterpret_cast<const f32x4*>(tot + (2 * bj + 1) * 64 + c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float f = bl & 8 ? tt[e] : 1.f;
+                        kt[e] *= f;
+                        qt[e] *= f;
+                        ks[e] *= bl & 8 ? 1.f : ts[e];
+                    }
+                    ks *= mid[j];
+                }
+                const u32x4 kb = __builtin_bit_cast(u32x4, ks);
+                oA = TlmF32::mfma(kb, __builtin_bit_cast(u32x4, kt), oA);
+                oP = TlmF32::mfma(kb, __builtin_bit_cast(u32x4, qt), oP);
             }
         }
-        for (int i = tid; i < TLM_CHUNK * 16; i += 256) {  // decayed queries, right sides of W
-            const int t = i >> 4, c = 4 * (i & 15);
-            if (c >= cn) continue;
-            f32x4 f = {1.f, 1.f, 1.f, 1.f};
-            for (int m = 0; m < t >> 4; ++m) f *= *reinterpret_cast<const f32x4*>(tot + m * 64 + c);
-            *reinterpret_cast<f32x4*>(Qg + tlm_tile(t, c0 + c, D / 16)) = *reinterpret_cast<const f32x4*>(Q + t * TLM_PST + c) * f;
-            *reinterpret_cast<f32x4*>(Wg + tlm_tile(t, c0 + c, D / 16)) = *reinterpret_cast<const f32x4*>(K + t * TLM_PST + c) * f * beta[t];
+        mmi_meet();
+        if (lc < cn)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {                  // decayed queries
+                const int t = lt + 32 * i;
+                tlm_quad(Qg, (int)tlm_tile(t, c0 + lc, nd)) =
+                    *reinterpret_cast<const f32x4*>(Q + t * TLM_PST + lc) * *reinterpret_cast<const f32x4*>(pre + t / TLM_SUB * 64 + lc);
+            }
+        if (mine && 16 * (wave & 3) < cn) {                // this wave's right sides of W
+            const int c = 16 * (wave & 3) + bl;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float f = pre[(2 * i + (kq >> 1)) * 64 + c];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 16 * i + 4 * kq + r;
+                    strip[i][r] = K[t * TLM_PST + c] * f * beta[t];
+                }
+            }
         }
-        for (int i = wave; i < cn / 4; i += 4) {           // transposed fragments: 16 channels x 16 tokens
-            const int c = 16 * (i >> 2) + bl, t = 16 * (i & 3) + 4 * kq;
-            float f = 1.f;
-            for (int m = (i & 3) + 1; m < 4; ++m) f *= tot[m * 64 + c];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {                      // transposed fragments: 16 channels x 16 tokens
+            const int at = wave + 8 * i, c = 16 * (at >> 2) + bl, t = 16 * (at & 3) + 4 * kq;
+            if (at >= cn / 4) continue;
+            const float f = suf[t / TLM_SUB * 64 + c];
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = G[(t + e) * TLM_PST + c] * f;
-            *reinterpret_cast<f32x4*>(Kt + tlm_tile(c0 + c, t, 4)) = v;
+            tlm_quad(Kt, (int)tlm_tile(c0 + c, t, 4)) = v;
         }
-        if (tid < cn) a.gend[id * D + c0 + tid] = tot[tid] * tot[64 + tid] * tot[128 + tid] * tot[192 + tid];
-    }
-    __syncthreads();
-    // - A: the strictly lower triangle (columns right of it inside the diagonal blocks: zero), P
+        if (tid < cn) a.gend[id * D + c0 + tid] = pre[(TLM_CHUNK / TLM_SUB - 1) * 64 + tid] * tot[(TLM_CHUNK / TLM_SUB - 1) * 64 + tid];
+    };
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        float x = dA[s], y = dP[s];
-        x += mmi_shfl_xor(x, 16);
-        x += mmi_shfl_xor(x, 32);
-        y += mmi_shfl_xor(y, 16);
-        y += mmi_shfl_xor(y, 32);
-        const int t = 16 * wave + bl, at = 16 * wave + s;
-        if (kq == 0) {
-            A[t * TLM_PST + at] = s < bl ? -beta[t] * x : 0.f;
-            P[tlm_tile(t, at, 4)] = s <= bl ? y : 0.f;
+    for (int k = 0; k < NS; ++k)
+#pragma unroll
+        for (int p = 0; p < min(2, NP); ++p)
+            if (128 * k + 64 * p < D) panel(128 * k + 64 * p, wave >> 2 == p, x[k]);
+    mmi_meet();
+    // -A (strictly lower) and P, whole rows in LDS
+    int l = lane;
+    mmi_here(l);
+    bl = l & 15;
+    kq = l >> 4;
+#pragma unroll
+    for (int i = 0; i < TLM_SUB; ++i) {
+        dA[i] = mmi_rows_sum(dA[i]);
+        dP[i] = mmi_rows_sum(dP[i]);
+    }
+    f32x4 mine;                                            // lane (kq, bl): pairs t - 2 kq and t - 2 kq - 1
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        mine[i] = kq < 2 ? (kq ? dA[2 + i] : dA[i]) : (kq == 2 ? dA[4 + i] : dA[6 + i]);
+        mine[2 + i] = kq < 2 ? (kq ? dP[2 + i] : dP[i]) : (kq == 2 ? dP[4 + i] : dP[6 + i]);
+    }
+    if (wave >= 4) *reinterpret_cast<f32x4*>(part + ((wave - 4) * 64 + lane) * 4) = mine;
+    if (wave < 6 || (bl >> 3) == (kq >> 1)) {              // (a quarter's operands took rows of two blocks: the pairs inside one are wanted)
+        const int t = row(bl), s = wave < 6 ? 16 * bj + 4 * kq : 32 * (wave - 6) + 16 * (kq >> 1) + 4 * (kq & 1);
+        *reinterpret_cast<f32x4*>(A + t * TLM_PST + s) = oA * -beta[t];
+        *reinterpret_cast<f32x4*>(Pl + t * TLM_PST + s) = oP;
+    }
+    mmi_meet();
+    if (wave < 4) {
+        mine += *reinterpret_cast<const f32x4*>(part + (wave * 64 + lane) * 4);
+        const int t = 16 * wave + bl;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int s = t - 2 * kq - i;
+            if (2 * kq + i > (t & 7)) continue;
+            if (s < t) A[t * TLM_PST + s] = -beta[t] * mine[i];
+            Pl[t * TLM_PST + s] = mine[2 + i];
         }
     }
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-        if (b < nblk)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * bi[b] + 4 * kq + r, s = 16 * bj[b] + bl;
-                A[t * TLM_PST + s] = -beta[t] * oA[b][r];
-                P[tlm_tile(t, s, 4)] = oP[b][r];
-            }
-    __syncthreads();
-    {                                                      // (I + A_ww)^-1, one column per lane
-        float x[16];
+    mmi_meet();
+    if (wave < 4) {                                        // (I + A_ww)^-1, one column per lane
+        float y[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             float s = t == bl ? 1.f : 0.f;
 #pragma unroll
-            for (int j = 0; j < t; ++j) s = mmi_fma(A[(16 * wave + t) * TLM_PST + 16 * wave + j], x[j], s);
-            x[t] = s;
-            if (kq == 0) ti[(wave * 16 + t) * 20 + bl] = s;
+            for (int j = 0; j < t; j += 4) {
+                const f32x4 r = *reinterpret_cast<const f32x4*>(A + (16 * wave + t) * TLM_PST + 16 * wave + j);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (j + e < t) s = mmi_fma(r[e], y[j + e], s);
+            }
+            y[t] = s;
+        }
+        if (kq == 0)
+#pragma unroll
+            for (int t = 0; t < 16; ++t) ti[(wave * 16 + t) * 20 + bl] = y[t];
+    } else {
+        for (int i = wave - 4; i < 10; i += 4) {           // P's blocks, those right of the diagonal left out
+            const int ti_ = i < 1 ? 0 : (i < 3 ? 1 : (i < 6 ? 2 : 3)), si = i - ti_ * (ti_ + 1) / 2, t = 16 * ti_ + bl, s = 16 * si + 4 * kq;
+            f32x4 v = *reinterpret_cast<const f32x4*>(Pl + t * TLM_PST + s);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = s + e <= t ? v[e] : 0.f;
+            tlm_quad(P, (int)tlm_tile(t, s, 4)) = v;
         }
     }
-    __syncthreads();
-    // forward substitution by blocks of 16; a wave takes four 16-column strips of [W | U0] at a time
-    const int nd = D / 16, ns = nd + V / 16;
-    for (int s0 = wave; s0 < ns; s0 += 16) {
-        f32x4 x[4][4];
+    auto scale_u0 = [&](f32x4* u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int st = min(s0 + 4 * k, ns - 1);        // (past the end: the last strip again, not stored)
-            const float* src = st < nd ? Wg : qkv + a.v0 + h * V + 16 * (st - nd) + bl;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = 16 * i + 4 * kq + r;
-                    x[k][i][r] = src[st < nd ? tlm_tile(t, 16 * st + bl, nd) : (long)min(t, ck.n - 1) * a.conv_c];
-                }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = 16 * i + 4 * kq + r;
-                    x[k][i][r] = t < ck.n ? x[k][i][r] * (st < nd ? 1.f : beta[t]) : 0.f;
-                }
-        }
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * i + 4 * kq + r;
+                u[i][r] = t < ck.n ? u[i][r] * beta[t] : 0.f;
+            }
+    };
+    scale_u0(x[NS]);
+    mmi_meet();
+    // forward substitution by blocks of 16, all strips of this wave side by side
+    mmi_here(l);
+    bl = l & 15;
+    kq = l >> 4;
+    auto solve = [&](f32x4 (*y)[4], auto count) __attribute__((always_inline)) {
+        constexpr int N = decltype(count)::value;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
 #pragma unroll
             for (int j = 0; j < i; ++j) {
                 const u32x4 av = *reinterpret_cast<const u32x4*>(A + (16 * i + bl) * TLM_PST + 16 * j + 4 * kq);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) x[k][i] = TlmF32::mfma(av, __builtin_bit_cast(u32x4, x[k][j]), x[k][i]);
+                for (int k = 0; k < N; ++k) y[k][i] = TlmF32::mfma(av, __builtin_bit_cast(u32x4, y[k][j]), y[k][i]);
             }
             const u32x4 tv = *reinterpret_cast<const u32x4*>(ti + (i * 16 + bl) * 20 + 4 * kq);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) x[k][i] = TlmF32::mfma(tv, __builtin_bit_cast(u32x4, x[k][i]), f32x4{0.f, 0.f, 0.f, 0.f});
+            for (int k = 0; k < N; ++k) y[k][i] = TlmF32::mfma(tv, __builtin_bit_cast(u32x4, y[k][i]), f32x4{0.f, 0.f, 0.f, 0.f});
         }
+    };
+    auto store_u0 = [&](const f32x4* u, int v) __attribute__((always_inline)) {
+        if (v < nv)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (s0 + 4 * k < ns)
+            for (int i = 0; i < 4; ++i) tlm_quad(Ug, ((i * nv + v) * 64 + lane) * 4) = u[i];
+    };
+    solve(x, std::integral_constant<int, NS + 1>{});
+    store_u0(x[NS], v0);
+    for (int v = v0 + 8; v < nv; v += 8) {                 // (more than 128 value columns)
+        load_u0(x[NS], v, bl, kq);
+        scale_u0(x[NS]);
+        solve(x + NS, std::integral_constant<int, 1>{});
+        store_u0(x[NS], v);
+    }
+    // W goes out as the walk's left operand: a strip's blocks turn round in LDS
+    float* T = sh + wave * (TLM_CHUNK * 20);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int st = s0 + 4 * k;
-                    if (st >= nd) *reinterpret_cast<f32x4*>(Ug + (((long)i * (V / 16) + st - nd) * 64 + lane) * 4) = x[k][i];
-                    else
+    for (int k = 0; k < NS; ++k) {
+        mmi_meet();
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) Wg[tlm_tile(16 * i + 4 * kq + r, 16 * st + bl, nd)] = x[k][i][r];
-                }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) T[(16 * i + 4 * kq + r) * 20 + bl] = x[k][i][r];
+        mmi_meet();
+        const int st = 8 * k + wave;
+        if (st < nd)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                tlm_quad(Wg, ((i * nd + st) * 64 + lane) * 4) = *reinterpret_cast<const f32x4*>(T + (16 * i + bl) * 20 + 4 * kq);
     }
 }
 

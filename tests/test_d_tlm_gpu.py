@@ -74,6 +74,11 @@ def test_greedy_generation_through_the_scheduler_bibapel(lib):
     tc.check_generation(DEV, lib, name="bibapel")
 
 
+@pytest.mark.parametrize("dim,vdim,n", tc.CHUNK_EDGES)
+def test_chunk_edges(lib, dim, vdim, n):
+    tc.check_chunk_edges(DEV, lib, dim, vdim, n)
+
+
 @pytest.mark.parametrize("window", [70, 64, 0])
 def test_single_keys(lib, window):
     tc.check_single_keys(DEV, lib, window)

@@ -31,6 +31,11 @@ def test_mechanism_bf16(tlm_lib, name):
     tc.check_mechanism(name, DEV, tlm_lib, tc.BF16)
 
 
+@pytest.mark.parametrize("dim,vdim,n", tc.CHUNK_EDGES)
+def test_chunk_edges(tlm_lib, dim, vdim, n):
+    tc.check_chunk_edges(DEV, tlm_lib, dim, vdim, n)
+
+
 def test_activation_branches(tlm_lib):
     tc.check_activation_branches(DEV, tlm_lib)
 

@@ -496,6 +496,19 @@ def check_decay_extremes(dev, lib):
             assert rel(run_cut(lm, toks, cuts), want) < TOL[F32], (amp, cuts)
 
 
+# (dim, vdim, tokens): around the edges of 64 channel panels, of 128 value columns, of 8 and 64 tokens
+CHUNK_EDGES = [(16, 16, 5), (48, 144, 64), (64, 16, 72), (65, 24, 65), (128, 256, 9), (129, 16, 129), (200, 40, 71), (256, 128, 63)]
+
+
+def check_chunk_edges(dev, lib, dim, vdim, n):
+    """Both matrix mixers in chunks, a second portion on top of the state that the first left.  Tolerance: that of the fp32 mechanisms."""
+    for mixer in (replace(DELTA, heads=2, kv_heads=1, dim=dim, vdim=vdim), replace(LIGHT, heads=3, dim=dim, vdim=vdim)):
+        cfg = plain_layer(mixer)
+        lm, orc = make(cfg, dev, lib)
+        toks = tokens_of(cfg, n + 6)
+        assert rel(run_cut(lm, toks, [n, 6]), orc.logits(toks)) < TOL[F32], mixer
+
+
 def check_glu_limits(dev, lib):
     """Gate above its limit (and far below zero: unlimited), up beyond both of its limits."""
     cfg = MECHANISMS["glu"]
