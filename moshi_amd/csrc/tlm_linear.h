@@ -648,12 +648,15 @@ __global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLin
 // ------------------------------------------------------------------------------------------------
 // chunks: the walk over a sequence's chunks.  One workgroup per (sequence, head, 16 columns of S).  Wave w owns token block w of every chunk
 // and a quarter of the rows of S, in the layout the matrix core leaves them in, which is also the layout it takes them as an operand; S and
-// U go round through LDS.
+// U go round through LDS.  A chunk is 112 matrix instructions of 32 cycles per SIMD and asks a CU for 116 KB: requests in one burst kept the
+// waves from issuing for 2400 of 7500 cycles, so they stand between the products, a phase or more before their use, and what follows an exchange
+// through LDS does not need it (Q S, P U).  One sequence of 1773 tokens, 32 heads of 128 x 128: 98 us before, 77 now (5200 cycles per chunk; with all
+// of it in the L2 no less: what is left is the distance of dependent instructions in one wave per SIMD); 331 tokens 24.6 and 20.0.
 // grid: 8 x ceil(sequences x heads / 8) x vdim_p / 16, the column blocks of one head on one XCD (they read the same W, Qg, Kt, P)
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float tlm_f(unsigned v) { return __builtin_bit_cast(float, v); }
 template <bool DELTA, int NDW>
-__global__ __launch_bounds__(256, 1) void k_tlm_chunk_scan(TlmLinArgs a, int n_units) {
+__global__ __launch_bounds__(256, NDW <= 2 ? 2 : 1) void k_tlm_chunk_scan(TlmLinArgs a, int n_units) {
     constexpr int ND = 4 * NDW;                            // 16-row blocks of S; past the model's: zeros
     MMI_SHARED __attribute__((aligned(16))) f32x4 Sl[ND][64], Ul[4][64];
     const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15, kq = lane >> 4;
@@ -662,129 +665,149 @@ __global__ __launch_bounds__(256, 1) void k_tlm_chunk_scan(TlmLinArgs a, int n_u
     if (uh >= n_units * a.heads) return;
     const TlmUnit un = a.unit[uh / a.heads];
     const int h = uh % a.heads, D = a.dim_p, V = a.vdim_p, nd = D / 16;
-    float* S = a.state + ((long)un.slot * a.heads + h) * D * V + 16 * cb + bl;
-    f32x4 s[NDW];
+    float* S = a.state + ((long)un.slot * a.heads + h) * D * V + 16 * cb;
+    // a chunk's operands in registers: keys, P and decays are asked for while W S is computed, queries again as they are used up, W and U0 of
+    // the next chunk while S is brought up to date
+    u32x4 w[DELTA ? ND : 1], q[ND], k[NDW][4], p[4];
+    f32x4 u0, g[NDW], s[NDW], sl[ND], u[4];
+    // (blocks past the end: a valid address, against rows of S that stay zero)
+    auto load_w = [&](long id, int d) __attribute__((always_inline)) { w[d] = tlm_quad<u32x4>(a.w + id * TLM_CHUNK * D, ((wave * nd + min(d, nd - 1)) * 64 + lane) * 4); };
+    auto load_q = [&](long id, int d) __attribute__((always_inline)) { q[d] = tlm_quad<u32x4>(a.qg + id * TLM_CHUNK * D, ((wave * nd + min(d, nd - 1)) * 64 + lane) * 4); };
+    auto load_k = [&](long id, int i, int t) __attribute__((always_inline)) { k[i][t] = tlm_quad<u32x4>(a.kt + id * TLM_CHUNK * D, ((min(wave * NDW + i, nd - 1) * 4 + t) * 64 + lane) * 4); };
+    auto load_g = [&](long id, int i) __attribute__((always_inline)) { g[i] = tlm_quad(a.gend + id * D, 16 * min(wave * NDW + i, nd - 1) + 4 * kq); };
+    auto load_p = [&](long id, int t) __attribute__((always_inline)) { p[t] = tlm_quad<u32x4>(a.p + id * (TLM_CHUNK * TLM_CHUNK), ((wave * 4 + min(t, wave)) * 64 + lane) * 4); };
+    auto load_u = [&](long id, int c) __attribute__((always_inline)) {
+        if constexpr (DELTA) {
+            u0 = tlm_quad(a.u0 + id * TLM_CHUNK * V, ((wave * ncb + cb) * 64 + lane) * 4);
+        } else {
+            const int n = min(TLM_CHUNK, un.n - c * TLM_CHUNK);
+            const float* v = a.in + (long)(un.row0 + c * TLM_CHUNK) * a.in_ld + a.v0 + h * V + 16 * cb;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u0[r] = tlm_quad<float>(v, min(16 * wave + 4 * kq + r, n - 1) * a.in_ld + bl);
+        }
+    };
+    {
+        const long id = (long)un.chunk0 * a.heads + h;
+        load_u(id, 0);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            if constexpr (DELTA) load_w(id, d);
+            load_q(id, d);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < NDW; ++i) {
         s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int d = wave * NDW + i;
         if (!un.fresh && d < nd)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s[i][r] = S[(long)(16 * d + 4 * kq + r) * V];
+            for (int r = 0; r < 4; ++r) s[i][r] = tlm_quad<float>(S, (16 * d + 4 * kq + r) * V + bl);
         Sl[d][lane] = s[i];
     }
-    __syncthreads();
-    struct Frags {
-        u32x4 w[DELTA ? ND : 1], q[ND], k[NDW][4], p[4];
-        f32x4 u, g[NDW];
-    };
-    auto load = [&](Frags& f, int c) __attribute__((always_inline)) {      // (blocks past the end: a valid address, against rows of S that stay zero)
-        const long id = (long)(un.chunk0 + c) * a.heads + h;
-        const int n = min(TLM_CHUNK, un.n - c * TLM_CHUNK);
+    mmi_meet();
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            const long at = id * TLM_CHUNK * D + (((long)wave * nd + min(d, nd - 1)) * 64 + lane) * 4;
-            if constexpr (DELTA) f.w[d] = *reinterpret_cast<const u32x4*>(a.w + at);
-            f.q[d] = *reinterpret_cast<const u32x4*>(a.qg + at);
-        }
-#pragma unroll
-        for (int i = 0; i < NDW; ++i) {
-            const int d = min(wave * NDW + i, nd - 1);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) f.k[i][t] = *reinterpret_cast<const u32x4*>(a.kt + id * TLM_CHUNK * D + (((long)d * 4 + t) * 64 + lane) * 4);
-            f.g[i] = *reinterpret_cast<const f32x4*>(a.gend + id * D + 16 * d + 4 * kq);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            f.p[t] = *reinterpret_cast<const u32x4*>(a.p + id * (TLM_CHUNK * TLM_CHUNK) + ((wave * 4 + min(t, wave)) * 64 + lane) * 4);
-        if constexpr (DELTA) {
-            f.u = *reinterpret_cast<const f32x4*>(a.u0 + id * TLM_CHUNK * V + (((long)wave * ncb + cb) * 64 + lane) * 4);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int tok = 16 * wave + 4 * kq + r;
-                const float v = a.in[(long)(un.row0 + c * TLM_CHUNK + min(tok, n - 1)) * a.in_ld + a.v0 + h * V + 16 * cb + bl];
-                f.u[r] = tok < n ? v : 0.f;
-            }
-        }
-    };
-    auto chunk = [&](const Frags& f, int c) __attribute__((always_inline)) {
-        const int n = min(TLM_CHUNK, un.n - c * TLM_CHUNK);
-        // four independent sums go round, one step of four each: a matrix instruction never waits for the one before it
+    for (int d = 0; d < ND; ++d) sl[d] = Sl[d][lane];
+    for (int c = 0; c < un.n_chunks; ++c) {
+        const int n = min(TLM_CHUNK, un.n - c * TLM_CHUNK), cn = min(c + 1, un.n_chunks - 1);      // (the last chunk asks for itself again)
+        const long id = (long)(un.chunk0 + c) * a.heads + h, next = (long)(un.chunk0 + cn) * a.heads + h;
+        // two independent sums, steps in turn: a matrix instruction never waits for the one before it
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         f32x4 x0 = zero, x1 = zero, o0 = zero, o1 = zero;
-        if constexpr (!DELTA) Ul[wave][lane] = f.u;
-#pragma unroll
-        for (int d = 0; d < ND; d += 2) {
-            const f32x4 sa = Sl[d][lane], sb = Sl[d + 1][lane];
+        auto outputs = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if constexpr (DELTA) {
-                    x0 = mmi_mfma_f32_16x16x4(tlm_f(f.w[d][e]), sa[e], x0);
-                    x1 = mmi_mfma_f32_16x16x4(tlm_f(f.w[d + 1][e]), sb[e], x1);
-                }
-                o0 = mmi_mfma_f32_16x16x4(tlm_f(f.q[d][e]), sa[e], o0);
-                o1 = mmi_mfma_f32_16x16x4(tlm_f(f.q[d + 1][e]), sb[e], o1);
+                o0 = mmi_mfma_f32_16x16x4(tlm_f(q[d][e]), sl[d][e], o0);
+                o1 = mmi_mfma_f32_16x16x4(tlm_f(q[d + 1][e]), sl[d + 1][e], o1);
             }
+            mmi_sched_barrier();
+            load_q(next, d);
+            load_q(next, d + 1);
+            mmi_sched_barrier();
+        };
+        auto rest = [&](int d) __attribute__((always_inline)) {
+            load_k(id, d / 4, d % 4);
+            if (d % 4 == 0) load_g(id, d / 4);
+            if (d < 4) load_p(id, d);
+        };
+        if constexpr (DELTA) {
+#pragma unroll
+            for (int d = 0; d < ND; d += 2) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x0 = mmi_mfma_f32_16x16x4(tlm_f(w[d][e]), sl[d][e], x0);
+                    x1 = mmi_mfma_f32_16x16x4(tlm_f(w[d + 1][e]), sl[d + 1][e], x1);
+                }
+                mmi_sched_barrier();
+                rest(d);
+                rest(d + 1);
+                mmi_sched_barrier();
+            }
+            Ul[wave][lane] = u0 - (x0 + x1);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u0[r] = 16 * wave + 4 * kq + r < n ? u0[r] : 0.f;
+            Ul[wave][lane] = u0;
+#pragma unroll
+            for (int d = 0; d < ND; ++d) rest(d);
+            mmi_sched_barrier();
         }
-        if constexpr (DELTA) Ul[wave][lane] = f.u - (x0 + x1);
-        __syncthreads();
-        f32x4 u[4], sh[NDW];
+        // the exchange of U stands between the halves of Q S, that of S between those of P U: what a wave waits for is on its way meanwhile
+#pragma unroll
+        for (int d = 0; d < ND / 2; d += 2) outputs(d);
+        mmi_meet();
 #pragma unroll
         for (int t = 0; t < 4; ++t) u[t] = Ul[t][lane];
+        mmi_sched_barrier();
+#pragma unroll
+        for (int d = ND / 2; d < ND; d += 2) outputs(d);
+        f32x4 sh[NDW];
 #pragma unroll
         for (int i = 0; i < NDW; ++i) {
-            s[i] *= f.g[i];
+            s[i] *= g[i];
             sh[i] = zero;
         }
 #pragma unroll
-        for (int t = 0; t < 4; t += 2)
+        for (int t = 0; t < 4; t += 2) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int i = 0; i < NDW; ++i) {
-                    s[i] = mmi_mfma_f32_16x16x4(tlm_f(f.k[i][t][e]), u[t][e], s[i]);
-                    sh[i] = mmi_mfma_f32_16x16x4(tlm_f(f.k[i][t + 1][e]), u[t + 1][e], sh[i]);
+                    s[i] = mmi_mfma_f32_16x16x4(tlm_f(k[i][t][e]), u[t][e], s[i]);
+                    sh[i] = mmi_mfma_f32_16x16x4(tlm_f(k[i][t + 1][e]), u[t + 1][e], sh[i]);
                 }
+            mmi_sched_barrier();
+            if constexpr (DELTA)
+#pragma unroll
+                for (int d = t * NDW; d < (t + 2) * NDW; ++d) load_w(next, d);
+            if (t) load_u(next, cn);
+            mmi_sched_barrier();
+        }
 #pragma unroll
         for (int i = 0; i < NDW; ++i) {
             s[i] += sh[i];
             if (wave * NDW + i >= nd) s[i] = zero;
             Sl[wave * NDW + i][lane] = s[i];
         }
-#pragma unroll
-        for (int t = 0; t < 4; t += 2)                     // (blocks right of the diagonal: zeros instead)
+        auto inside = [&](int t) __attribute__((always_inline)) {      // (blocks right of the diagonal: zeros instead)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                o0 = mmi_mfma_f32_16x16x4(t <= wave ? tlm_f(f.p[t][e]) : 0.f, u[t][e], o0);
-                o1 = mmi_mfma_f32_16x16x4(t + 1 <= wave ? tlm_f(f.p[t + 1][e]) : 0.f, u[t + 1][e], o1);
+                o0 = mmi_mfma_f32_16x16x4(t <= wave ? tlm_f(p[t][e]) : 0.f, u[t][e], o0);
+                o1 = mmi_mfma_f32_16x16x4(t + 1 <= wave ? tlm_f(p[t + 1][e]) : 0.f, u[t + 1][e], o1);
             }
+            mmi_sched_barrier();
+        };
+        inside(0);
+        mmi_meet();
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sl[d] = Sl[d][lane];
+        mmi_sched_barrier();
+        inside(2);
         const f32x4 o = o0 + o1;
+        float* out = a.o + ((long)(un.row0 + c * TLM_CHUNK) * a.heads + h) * V + 16 * cb;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int tok = 16 * wave + 4 * kq + r;
-            if (tok < n) a.o[((long)(un.row0 + c * TLM_CHUNK + tok) * a.heads + h) * V + 16 * cb + bl] = o[r];
-        }
-        __syncthreads();
-    };
-    if constexpr (NDW <= 2) {
-        // the next chunk's operands are on their way while a chunk is computed (the last one asks for itself again)
-        Frags fa, fb;
-        load(fa, 0);
-        for (int c = 0; c < un.n_chunks; c += 2) {
-            load(fb, min(c + 1, un.n_chunks - 1));
-            mmi_sched_barrier();
-            chunk(fa, c);
-            if (c + 1 == un.n_chunks) break;
-            load(fa, min(c + 2, un.n_chunks - 1));
-            mmi_sched_barrier();
-            chunk(fb, c + 1);
-        }
-    } else {
-        Frags f;
-        for (int c = 0; c < un.n_chunks; ++c) {
-            load(f, c);
-            chunk(f, c);
+            if (tok < n) tlm_quad<float>(out, tok * a.heads * V + bl) = o[r];
         }
     }
 #pragma unroll
@@ -792,7 +815,7 @@ __global__ __launch_bounds__(256, 1) void k_tlm_chunk_scan(TlmLinArgs a, int n_u
         const int d = wave * NDW + i;
         if (d < nd)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) S[(long)(16 * d + 4 * kq + r) * V] = s[i][r];
+            for (int r = 0; r < 4; ++r) tlm_quad<float>(S, (16 * d + 4 * kq + r) * V + bl) = s[i][r];
     }
 }
 
