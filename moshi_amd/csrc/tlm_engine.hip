@@ -1543,7 +1543,8 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         if (delta) {
             P.site(site + "conv");
             P.add([=](hipStream_t s) {
-                MMI_LAUNCH(k_tlm_conv, dim3(n_chunk, 2 * a.kv_heads + a.heads), 256, 0, s, a, tlm_step_groups(a.dim_p), tlm_step_groups(a.vdim_p));
+                const int kg = tlm_step_groups(a.dim_p), vg = tlm_step_groups(a.vdim_p), rounds = std::max(1, TLM_CHUNK * std::max(kg, vg) / 1024);
+                MMI_LAUNCH(k_tlm_conv, dim3(n_chunk, 2 * a.kv_heads + a.heads, rounds), 256, 0, s, a, kg, vg);
                 MMI_CHECK_LAUNCH();
                 return (int)MMI_OK;
             });

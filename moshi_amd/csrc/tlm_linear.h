@@ -221,32 +221,61 @@ __global__ __launch_bounds__(MAXB, MAXB == 512 && !DELTA ? 5 : 4) void k_tlm_sta
 }
 
 // ------------------------------------------------------------------------------------------------
-// chunks: convolutions and unit norms (delta).  grid: chunks, 2 kv_heads + heads; a lane takes 4 channels, a power of two of lanes a token
+// chunks: convolutions and unit norms (delta).  grid: chunks, 2 kv_heads + heads, shares of a chunk; a lane takes 4 channels of 4 tokens in a row, which share
+// seven inputs per four taps; a power of two of lanes stand side by side.  Bound by its bytes with many chunks, by two trips to memory with few,
+// so a workgroup goes round once.  1773 tokens, 32 heads of 128 x 128 (174 MB): 42.7 us with a token per lane, 37.6 now; 662 tokens of 16 heads 16.0
+// and 11.8 (going round twice 13.4); 200 tokens of 8 heads 11.5 and 7.1
 // ------------------------------------------------------------------------------------------------
-inline __global__ __launch_bounds__(256) void k_tlm_conv(TlmLinArgs a, int kgroups, int vgroups) {
+inline __global__ __launch_bounds__(256, 4) void k_tlm_conv(TlmLinArgs a, int kgroups, int vgroups) {
     const int y = (int)blockIdx.y;
     const TlmSeg ck = a.chunk[blockIdx.x];
     const int kind = y < a.kv_heads ? 0 : (y < 2 * a.kv_heads ? 1 : 2);
     const int width = kind == 2 ? a.vdim_p : a.dim_p, groups = kind == 2 ? vgroups : kgroups;
     const int c0 = kind == 0 ? a.q0 + y * a.dim_p : (kind == 1 ? a.k0 + (y - a.kv_heads) * a.dim_p : a.v0 + (y - 2 * a.kv_heads) * a.vdim_p);
-    const float* old = a.conv_state + ((long)ck.slot * 2 + ck.par) * (a.taps - 1) * a.conv_c;
-    float* now = a.conv_state + ((long)ck.slot * 2 + (ck.par ^ 1)) * (a.taps - 1) * a.conv_c;
-    const int first = ck.row0 - ck.index * TLM_CHUNK;      // the sequence's first row of this step
-    const int c = 4 * ((int)threadIdx.x & (groups - 1)), step = 256 / groups;
-    for (int t0 = 0; t0 < ck.n; t0 += step) {              // (every lane of a wave goes round as often)
-        const int t = t0 + (int)threadIdx.x / groups;
-        f32x4 x = {0.f, 0.f, 0.f, 0.f};
-        if (t < ck.n && c < width) {
-            x = tlm_conv<f32x4>(a, old, ck.fresh, first, ck.index * TLM_CHUNK + t, c0 + c, ck.last && t + 1 == ck.n ? now : nullptr);
+    const int back = a.taps - 1, s0 = ck.index * TLM_CHUNK;
+    const float* old = a.conv_state + ((long)ck.slot * 2 + ck.par) * back * a.conv_c + c0;
+    float* now = a.conv_state + ((long)ck.slot * 2 + (ck.par ^ 1)) * back * a.conv_c + c0;
+    const float *in = a.in + (long)(ck.row0 - s0) * a.in_ld + c0, *cw = a.conv_w + c0;       // in: the sequence's first row of this step
+    const int c = 4 * ((int)threadIdx.x & (groups - 1)), cc = min(c, width - 4), step = 4 * (256 / groups);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    for (int t0 = (int)blockIdx.z * step; t0 < ck.n; t0 += (int)gridDim.z * step) {      // (every lane of a wave goes round as often)
+        const int t = t0 + 4 * ((int)threadIdx.x / groups);
+        f32x4 x[4] = {zero, zero, zero, zero};
+        for (int j0 = 0; j0 < a.taps; j0 += 4) {           // (inputs past the chunk or the taps: a valid address, not used)
+            f32x4 v[7], w[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = tlm_silu(x[e]);
+            for (int j = 0; j < 4; ++j) w[j] = *reinterpret_cast<const f32x4*>(cw + (long)min(j0 + j, back) * a.conv_c + cc);
+#pragma unroll
+            for (int m = 0; m < 7; ++m) {
+                const int at = s0 + min(t + j0 + m - back, ck.n - 1);
+                v[m] = *reinterpret_cast<const f32x4*>(at >= 0 || ck.fresh ? in + (long)max(at, 0) * a.in_ld + cc : old + (long)(back + at) * a.conv_c + cc);
+                if (at < 0 && ck.fresh) v[m] = zero;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (j0 + j <= back) x[r] += w[j] * v[r + j];
+            if (ck.last && t < ck.n && t + 4 >= ck.n && c < width)      // the inputs that the next step's first tokens need
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (t + r + 1 == ck.n)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (j0 + j >= 1 && j0 + j <= back) *reinterpret_cast<f32x4*>(now + (long)(j0 + j - 1) * a.conv_c + c) = v[r + j];
         }
-        if (kind != 2) {
-            float ss = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
-            for (int m = 1; m < groups; m *= 2) ss += mmi_shfl_xor(ss, m);
-            x *= (kind == 0 ? a.q_scale : 1.0f) / sqrtf(ss + 1e-6f);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool in_place = t + r < ck.n && c < width;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[r][e] = in_place ? x[r][e] * tlm_sigmoid(x[r][e]) : 0.f;
+            if (kind != 2) {
+                float ss = x[r][0] * x[r][0] + x[r][1] * x[r][1] + x[r][2] * x[r][2] + x[r][3] * x[r][3];
+                for (int m = 1; m < groups; m *= 2) ss += mmi_shfl_xor(ss, m);
+                x[r] *= (kind == 0 ? a.q_scale : 1.0f) / sqrtf(ss + 1e-6f);
+            }
+            if (in_place) *reinterpret_cast<f32x4*>(a.qkv + (long)(ck.row0 + t + r) * a.conv_c + c0 + c) = x[r];
         }
-        if (t < ck.n && c < width) *reinterpret_cast<f32x4*>(a.qkv + (long)(ck.row0 + t) * a.conv_c + c0 + c) = x;
     }
 }
 
