@@ -2048,24 +2048,38 @@ __global__ __launch_bounds__(256, KV8 ? 2 : 4) void k_lm_attn_wave(LmAttnArgs a)
     }
 }
 
-// merge the chunk partials: out = sum_c e^{m_c-M} O_c / sum_c e^{m_c-M} l_c  -> bf16 [B][H*Dh]
+// merge the chunk partials: out = sum_c e^{m_c-M} O_c / sum_c e^{m_c-M} l_c  -> bf16 [B][H*Dh].  One trip to memory bounds it: the first
+// MAXC partials are requested together, whatever their weights turn out to be (an empty one, m = -inf, is not added).  12 partials of
+// 32 heads of 128: 4.8 us, 6.0 with a loop that waited for every partial
 __global__ void k_lm_attn_combine(LmAttnArgs a) {
-    const int bh = blockIdx.x;
-    const int Dh = a.Dh;
-    const float* ml = a.ml + (long)bh * a.NS * 2;
-    float M = -INFINITY;
-    for (int c = 0; c < a.NS; ++c) M = fmaxf(M, ml[2 * c]);
-    for (int d = threadIdx.x; d < Dh; d += blockDim.x) {
-        float num = 0.f, den = 0.f;
-        for (int c = 0; c < a.NS; ++c) {
-            float m = ml[2 * c];
-            if (m == -INFINITY) continue;
-            float w = expf(m - M);
-            num += w * a.opart[((long)bh * a.NS + c) * Dh + d];
-            den += w * ml[2 * c + 1];
-        }
-        a.out[mmi_xp_index(a.T, bh / a.H, (bh % a.H) * Dh + d, a.out_ksteps)] = mmi_f32_to_bf16(num / den);
+    constexpr int MAXC = 16;
+    const int bh = (int)blockIdx.x, d = (int)threadIdx.x;
+    if (d >= a.Dh) return;
+    const f32x2* ml = reinterpret_cast<const f32x2*>(a.ml) + (long)bh * a.NS;
+    const float* part = a.opart + (long)bh * a.NS * a.Dh + d;
+    f32x2 s[MAXC];
+    float o[MAXC], M = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {                       // (past the end: the last partial again, not used)
+        const int cc = min(c, a.NS - 1);
+        s[c] = ml[cc];
+        o[c] = part[(long)cc * a.Dh];
     }
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) M = fmaxf(M, s[c][0]);
+    for (int c = MAXC; c < a.NS; ++c) M = fmaxf(M, ml[c][0]);
+    float num = 0.f, den = 0.f;
+    auto add = [&](f32x2 sc, float oc) __attribute__((always_inline)) {
+        const float w = expf(sc[0] - M);
+        const bool none = sc[0] == -INFINITY;
+        num = none ? num : num + w * oc;
+        den = none ? den : den + w * sc[1];
+    };
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c)
+        if (c < a.NS) add(s[c], o[c]);
+    for (int c = MAXC; c < a.NS; ++c) add(ml[c], part[(long)c * a.Dh]);
+    a.out[mmi_xp_index(a.T, bh / a.H, (bh % a.H) * a.Dh + d, a.out_ksteps)] = mmi_f32_to_bf16(num / den);
 }
 
 // ------------------------------------------------------------------------------------------------

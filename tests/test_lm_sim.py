@@ -108,6 +108,14 @@ def test_attention_ring_split_over_several_workgroups(sim_lib, monkeypatch, kern
     lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=61, B=2, S=9)
 
 
+@pytest.mark.parametrize("context", [300, 16 * 256, 16 * 256 + 1, 18 * 256])
+def test_merge_of_few_and_many_partials(sim_lib, monkeypatch, context):
+    """k_lm_attn_combine around the 16 partials that it requests together (2, 16, 17, 18); most are empty here, with a maximum of -inf."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_ATTN_SOLO", "0")
+    lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), context=context), seed=62, B=1, S=4)
+
+
 def test_depformer_attention_inside_out_proj_for_one_session(sim_lib, monkeypatch):
     """One session, bf16 weights: the depth transformer's attention of micro-steps >= 1 runs inside its out_proj
     (k_dep_attn_out_proj; no dep.attn site in the launch list); MMI_NO_DEP_ATTN_FUSION=1 and more sessions keep the launch."""
