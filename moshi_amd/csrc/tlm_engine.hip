@@ -1416,33 +1416,41 @@ MixerOut build_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer
     return MixerOut{&L.out, m->o, L.out.KS};
 }
 
+struct StepShape { int cgp, block, rt; size_t smem; };    // of k_tlm_state_step
+StepShape step_shape(const TlmLinArgs& a) {
+    StepShape z;
+    z.cgp = tlm_step_groups(a.vdim_p);
+    z.block = 64;                                        // rows of S per thread: 4, in larger workgroups 8, at the largest sizes 16
+    while (z.block < 256 && mmi_cdiv(a.dim_p, z.block / z.cgp) > 4) z.block *= 2;
+    while (z.block < 512 && mmi_cdiv(a.dim_p, z.block / z.cgp) > 8) z.block *= 2;
+    while (mmi_cdiv(a.dim_p, z.block / z.cgp) > 16) z.block *= 2;
+    const int parts = z.block / z.cgp, rows = mmi_cdiv(a.dim_p, parts);
+    z.rt = rows <= 4 && z.block <= 256 ? 4 : (rows <= 8 && z.block <= 512 ? 8 : 16);
+    z.smem = (size_t)(3 * parts * z.rt + a.vdim_p + 2 * parts * a.vdim_p) * sizeof(float);
+    return z;
+}
 template <class Tr, bool DELTA>
 int launch_state_step(hipStream_t s, const TlmLinArgs& a, int n) {
-    const int cgp = tlm_step_groups(a.vdim_p);
-    int block = 64;                                      // rows of S per thread: 4, in larger workgroups 8, at the largest sizes 16
-    while (block < 256 && mmi_cdiv(a.dim_p, block / cgp) > 4) block *= 2;
-    while (block < 512 && mmi_cdiv(a.dim_p, block / cgp) > 8) block *= 2;
-    while (mmi_cdiv(a.dim_p, block / cgp) > 16) block *= 2;
-    const int parts = block / cgp, rows = mmi_cdiv(a.dim_p, parts);
-    const int rt = rows <= 4 && block <= 256 ? 4 : (rows <= 8 && block <= 512 ? 8 : 16);
-    const size_t smem = (size_t)(3 * parts * rt + a.vdim_p + 2 * parts * a.vdim_p) * sizeof(float);
-    if (rt == 4) MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 4, 256>), dim3(n, a.heads), block, smem, s, a, cgp);
-    else if (rt == 8) MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 8, 512>), dim3(n, a.heads), block, smem, s, a, cgp);
-    else MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 16, 1024>), dim3(n, a.heads), block, smem, s, a, cgp);
+    const StepShape z = step_shape(a);
+    if (z.rt == 4) MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 4, 256>), dim3(n, a.heads), z.block, z.smem, s, a, z.cgp);
+    else if (z.rt == 8) MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 8, 512>), dim3(n, a.heads), z.block, z.smem, s, a, z.cgp);
+    else MMI_LAUNCH((k_tlm_state_step<Tr, DELTA, 16, 1024>), dim3(n, a.heads), z.block, z.smem, s, a, z.cgp);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
-template <int NP>
-int launch_chunk_delta_t(hipStream_t s, const TlmLinArgs& a, int n_chunk) {
+template <class Tr, int NP>
+int launch_chunk_delta_t(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
     const size_t smem = tlm_chunk_delta_smem();
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta<NP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta<Tr, NP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     MMI_HIP_CHECK(attr);
-    MMI_LAUNCH(k_tlm_chunk_delta<NP>, dim3(n_chunk, a.heads), 512, smem, s, a);
+    MMI_LAUNCH((k_tlm_chunk_delta<Tr, NP>), (n_chunk + n_small) * a.heads, 512, smem, s, a, n_chunk, n_small, tlm_step_groups(a.vdim_p));
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
-int launch_chunk_delta(hipStream_t s, const TlmLinArgs& a, int n_chunk) {
-    return a.dim_p <= 64 ? launch_chunk_delta_t<1>(s, a, n_chunk) : (a.dim_p <= 128 ? launch_chunk_delta_t<2>(s, a, n_chunk) : launch_chunk_delta_t<4>(s, a, n_chunk));
+template <class Tr>
+int launch_chunk_delta(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
+    if (a.dim_p <= 64) return launch_chunk_delta_t<Tr, 1>(s, a, n_chunk, n_small);
+    return a.dim_p <= 128 ? launch_chunk_delta_t<Tr, 2>(s, a, n_chunk, n_small) : launch_chunk_delta_t<Tr, 4>(s, a, n_chunk, n_small);
 }
 template <bool DELTA>
 int launch_chunk_scan(hipStream_t s, const TlmLinArgs& a, int n_unit) {
@@ -1532,7 +1540,10 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         add_jobs(m, P, p, Q, L.a2.bytes() + L.g2.bytes());
     }
     const int n_small = sh.n_small, n_unit = sh.n_unit, n_chunk = sh.n_chunk;
-    if (n_small) {
+    // chunks and single tokens of one step in one launch where both take workgroups of 512
+    const StepShape z = step_shape(a);
+    const bool together = delta && n_small && n_chunk && z.rt == 8 && z.block == 512 && z.smem <= tlm_chunk_delta_smem();
+    if (n_small && !together) {
         P.site(site + "step");
         P.add([=](hipStream_t s) {
             if (f32) return delta ? launch_state_step<TlmF32, true>(s, a, n_small) : launch_state_step<TlmF32, false>(s, a, n_small);
@@ -1552,7 +1563,7 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         P.site(site + "chunk");
         P.add([=](hipStream_t s) {
             if (delta) {
-                const int rc = launch_chunk_delta(s, a, n_chunk);
+                const int beside = together ? n_small : 0, rc = f32 ? launch_chunk_delta<TlmF32>(s, a, n_chunk, beside) : launch_chunk_delta<TlmBf16>(s, a, n_chunk, beside);
                 if (rc != MMI_OK) return rc;
             } else {
                 MMI_LAUNCH(k_tlm_chunk_lightning, dim3(n_chunk, a.heads), 256, 0, s, a);

@@ -104,13 +104,13 @@ inline int tlm_step_groups(int vdim_p) {                  // column groups of 4,
     while (4 * g < vdim_p) g *= 2;
     return g;
 }
-template <class Tr, bool DELTA, int RT, int MAXB>
-__global__ __launch_bounds__(MAXB, MAXB == 512 && !DELTA ? 5 : 4) void k_tlm_state_step(TlmLinArgs a, int cgp) {
-    MMI_DYN_SHARED(float, sh);                             // q, k, g [parts * RT] (zeros from dim_p on), v [vdim_p], red [2][parts][vdim_p]
+// sh: q, k, g [parts * RT] (zeros from dim_p on), v [vdim_p], red [2][parts][vdim_p]
+template <class Tr, bool DELTA, int RT>
+__device__ __forceinline__ void tlm_state_step(const TlmLinArgs& a, float* sh, int cgp, int seq, int h) {
     const int tid = (int)threadIdx.x, nthr = (int)blockDim.x, lane = tid & 63;
     const int parts = nthr / cgp, cg = tid & (cgp - 1), part = tid / cgp, col = 4 * cg;
-    const TlmUnit un = a.small[blockIdx.x];
-    const int h = (int)blockIdx.y, rep = a.heads / a.kv_heads, kh = h / rep, D = a.dim_p, V = a.vdim_p;
+    const TlmUnit un = a.small[seq];
+    const int rep = a.heads / a.kv_heads, kh = h / rep, D = a.dim_p, V = a.vdim_p;
     float *q = sh, *k = q + parts * RT, *g = k + parts * RT, *v = g + parts * RT, *red = v + V;
     for (int i = D + tid; i < parts * RT; i += nthr) q[i] = k[i] = g[i] = 0.f;
     const bool mine = col < V;
@@ -218,6 +218,11 @@ __global__ __launch_bounds__(MAXB, MAXB == 512 && !DELTA ? 5 : 4) void k_tlm_sta
         const int d = part + parts * i;
         if (mine && d < D) mmi_store_nt(reinterpret_cast<f32x4*>(S + (long)d * V + col), s[i]);
     }
+}
+template <class Tr, bool DELTA, int RT, int MAXB>
+__global__ __launch_bounds__(MAXB, MAXB == 512 && !DELTA ? 5 : 4) void k_tlm_state_step(TlmLinArgs a, int cgp) {
+    MMI_DYN_SHARED(float, sh);
+    tlm_state_step<Tr, DELTA, RT>(a, sh, cgp, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -349,17 +354,16 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_chunk_lightning(TlmLinArg
 constexpr int TLM_SUB = 8;               // tokens whose pairs are taken one by one; decays across them are whole products
 inline size_t tlm_chunk_delta_smem() { return (size_t)(3 * TLM_CHUNK * TLM_PST + (3 * (TLM_CHUNK / TLM_SUB) + 1) * 64) * sizeof(float); }
 template <int NP>
-__global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLinArgs a) {
-    MMI_DYN_SHARED(float, sh);
+__device__ __forceinline__ void tlm_chunk_delta(const TlmLinArgs& a, float* sh, int chunk, int h) {
     float *Q = sh, *K = Q + TLM_CHUNK * TLM_PST, *G = K + TLM_CHUNK * TLM_PST;      // [64][TLM_PST] each
     float *tot = G + TLM_CHUNK * TLM_PST, *pre = tot + TLM_CHUNK / TLM_SUB * 64, *suf = pre + TLM_CHUNK / TLM_SUB * 64;      // [8][64] each: decay over 8 tokens, over all 8s before, behind
     float* beta = suf + TLM_CHUNK / TLM_SUB * 64;          // [64]
     float *A = K, *Pl = Q, *part = G, *ti = G;                                      // once the panels are done: [64][TLM_PST] twice; [4][64][4], then [4][16][20]
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), h = (int)blockIdx.y;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6);
     int bl = lane & 15, kq = lane >> 4;
-    const TlmSeg ck = a.chunk[blockIdx.x];
+    const TlmSeg ck = a.chunk[chunk];
     const int D = a.dim_p, V = a.vdim_p, kh = h / (a.heads / a.kv_heads), nd = D / 16, nv = V / 16;
-    const long id = (long)blockIdx.x * a.heads + h;
+    const long id = (long)chunk * a.heads + h;
     const float *qp = a.qkv + (long)ck.row0 * a.conv_c + a.q0 + kh * D, *kp = qp + (a.k0 - a.q0), *vp = a.qkv + (long)ck.row0 * a.conv_c + a.v0 + h * V;
     const float *zp = a.decay + ((long)ck.row0 * a.heads + h) * D, *cp = a.decay_c + h * D;
     float *Wg = a.w + id * TLM_CHUNK * D, *Qg = a.qg + id * TLM_CHUNK * D, *Kt = a.kt + id * TLM_CHUNK * D, *Ug = a.u0 + id * TLM_CHUNK * V;
@@ -672,6 +676,15 @@ __global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLin
             for (int i = 0; i < 4; ++i)
                 tlm_quad(Wg, ((i * nd + st) * 64 + lane) * 4) = *reinterpret_cast<const f32x4*>(T + (16 * i + bl) * 20 + 4 * kq);
     }
+}
+// beside them the single tokens of n_small sequences, where those take workgroups of 512 too: neither fills the chip, and they share nothing.
+// 11 chunks and 14 sequences, 16 heads of 128 x 128: 23.3 + 16.4 us in launches of their own, 27.0 together
+template <class Tr, int NP>
+__global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLinArgs a, int n_chunk, int n_small, int cgp) {
+    MMI_DYN_SHARED(float, sh);
+    const int b = (int)blockIdx.x, own = b - n_chunk * a.heads;
+    if (own < 0) tlm_chunk_delta<NP>(a, sh, b % n_chunk, b / n_chunk);
+    else tlm_state_step<Tr, true, 8>(a, sh, cgp, own % n_small, own / n_small);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -79,6 +79,12 @@ def test_chunk_edges(lib, dim, vdim, n):
     tc.check_chunk_edges(DEV, lib, dim, vdim, n)
 
 
+@pytest.mark.parametrize("dtype", [tc.F32, tc.BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("dim,vdim", tc.BESIDE_CHUNKS)
+def test_tokens_beside_chunks(lib, dim, vdim, dtype):
+    tc.check_tokens_beside_chunks(DEV, lib, dim, vdim, dtype)
+
+
 @pytest.mark.parametrize("window", [70, 64, 0])
 def test_single_keys(lib, window):
     tc.check_single_keys(DEV, lib, window)

@@ -36,6 +36,11 @@ def test_chunk_edges(tlm_lib, dim, vdim, n):
     tc.check_chunk_edges(DEV, tlm_lib, dim, vdim, n)
 
 
+@pytest.mark.parametrize("dim,vdim", tc.BESIDE_CHUNKS)
+def test_tokens_beside_chunks(tlm_lib, dim, vdim):
+    tc.check_tokens_beside_chunks(DEV, tlm_lib, dim, vdim)
+
+
 def test_activation_branches(tlm_lib):
     tc.check_activation_branches(DEV, tlm_lib)
 

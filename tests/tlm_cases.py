@@ -509,6 +509,30 @@ def check_chunk_edges(dev, lib, dim, vdim, n):
         assert rel(run_cut(lm, toks, [n, 6]), orc.logits(toks)) < TOL[F32], mixer
 
 
+# (dim, vdim): single tokens beside chunks in one launch, at 1, 2 and 4 panels of 64 channels; the last one: in a launch of their own
+BESIDE_CHUNKS = [(128, 128), (96, 128), (64, 256), (256, 64), (200, 48), (32, 32)]
+
+
+def check_tokens_beside_chunks(dev, lib, dim, vdim, dtype=F32):
+    """A step of a prompt portion, of 1 and 3 tokens of running sequences and of a new sequence's first token; then a token each on top."""
+    cfg = plain_layer(replace(DELTA, heads=4, kv_heads=2, dim=dim, vdim=vdim))
+    lm, orc = make(cfg, dev, lib, dtype)
+    cuts = {0: (20, 1, 1), 1: (9, 3, 1), 2: (0, 70, 1), 3: (0, 1, 1), 4: (66, 65, 1)}
+    toks = {i: tokens_of(cfg, sum(c), seed=i) for i, c in cuts.items()}
+    slots, got = {i: lm.open() for i in cuts}, {i: [] for i in cuts}
+    at = dict.fromkeys(cuts, 0)
+    for phase in range(3):
+        batch = [(i, c[phase]) for i, c in cuts.items() if c[phase]]
+        out = lm.step([(slots[i], toks[i][at[i]:at[i] + n], list(range(n))) for i, n in batch]).cpu().numpy()
+        row = 0
+        for i, n in batch:
+            got[i].append(out[row:row + n].copy())
+            at[i] += n
+            row += n
+    for i in cuts:
+        assert rel(np.concatenate(got[i]), orc.logits(toks[i])) < TOL[dtype], i
+
+
 def check_glu_limits(dev, lib):
     """Gate above its limit (and far below zero: unlimited), up beyond both of its limits."""
     cfg = MECHANISMS["glu"]
