@@ -1090,20 +1090,25 @@ int launch_attn_t(hipStream_t s, const TlmAttnArgs& a, bool tiled) {
     });
 }
 
-template <class Tr, int D>
-int launch_gqa_d(hipStream_t s, const TlmGqaArgs& a, bool tiled) {
-    if (tiled) {
-        constexpr size_t smem = TlmGqaTile<Tr, D>::smem();
-        static_assert(smem <= 160 * 1024, "LDS of a CU");
-        if (smem > 64 * 1024) {
-            static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gqa_tile<Tr, D>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            MMI_HIP_CHECK(attr);
-        }
-        MMI_LAUNCH((k_tlm_gqa_tile<Tr, D>), dim3(a.n_tiles, a.kv_heads), 256, smem, s, a);
-    } else {
-        MMI_LAUNCH((k_tlm_gqa<Tr, D>), dim3(a.n_tiles, a.kv_heads, a.nsplit), 256, 0, s, a);
-        if (a.nsplit > 1) MMI_LAUNCH((k_tlm_gqa_combine<Tr>), dim3(a.n_tiles, a.kv_heads, mmi_cdiv(a.nd, 4)), 256, 0, s, a);
+// u: column groups for k_tlm_gqa_tile (or none), t: column tiles for k_tlm_gqa, beside them if there are both
+template <class Tr, int D, bool BESIDE>
+int launch_gqa_tile(hipStream_t s, const TlmGqaArgs& u, const TlmGqaArgs& t) {
+    constexpr size_t smem = TlmGqaTile<Tr, D>::smem();
+    static_assert(smem <= 160 * 1024, "LDS of a CU");
+    if (smem > 64 * 1024) {
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_gqa_tile<Tr, D, BESIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        MMI_HIP_CHECK(attr);
     }
+    MMI_LAUNCH((k_tlm_gqa_tile<Tr, D, BESIDE>), u.kv_heads * (u.n_tiles + (BESIDE ? t.n_tiles * t.nsplit : 0)), 256, smem, s, u, t);
+    return MMI_OK;
+}
+template <class Tr, int D>
+int launch_gqa_d(hipStream_t s, const TlmGqaArgs& u, const TlmGqaArgs& t) {
+    int rc = MMI_OK;
+    if (u.n_tiles) rc = t.n_tiles ? launch_gqa_tile<Tr, D, true>(s, u, t) : launch_gqa_tile<Tr, D, false>(s, u, t);
+    else MMI_LAUNCH((k_tlm_gqa<Tr, D>), dim3(t.n_tiles, t.kv_heads, t.nsplit), 256, 0, s, t);
+    if (rc != MMI_OK) return rc;
+    if (t.n_tiles && t.nsplit > 1) MMI_LAUNCH((k_tlm_gqa_combine<Tr>), dim3(t.n_tiles, t.kv_heads, mmi_cdiv(t.nd, 4)), 256, 0, s, t);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
@@ -1112,10 +1117,10 @@ int gqa_bound(const Layer& L, int kstep) {               // the kernels' bound o
     return d <= 64 ? 64 : (d <= 128 ? 128 : 256);
 }
 template <class Tr>
-int launch_gqa_t(hipStream_t s, const TlmGqaArgs& a, int bound, bool tiled) {
-    if (bound == 64) return launch_gqa_d<Tr, 64>(s, a, tiled);
-    if (bound == 128) return launch_gqa_d<Tr, 128>(s, a, tiled);
-    return launch_gqa_d<Tr, 256>(s, a, tiled);
+int launch_gqa_t(hipStream_t s, const TlmGqaArgs& u, const TlmGqaArgs& t, int bound) {
+    if (bound == 64) return launch_gqa_d<Tr, 64>(s, u, t);
+    if (bound == 128) return launch_gqa_d<Tr, 128>(s, u, t);
+    return launch_gqa_d<Tr, 256>(s, u, t);
 }
 
 struct Carry {                    // what the next residual launch has to add
@@ -1400,19 +1405,12 @@ MixerOut build_attention(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer
     t.pages = TlmPages{m->block_table, table_ld(m), m->keep_pages};
     t.po = m->po;
     t.pml = m->pml;
-    auto launch = [&](const TlmGqaArgs& x, bool staged) {
-        P.add([=](hipStream_t s) { return f32 ? launch_gqa_t<TlmF32>(s, x, bound, staged) : launch_gqa_t<TlmBf16>(s, x, bound, staged); });
-    };
     P.site(site + "attn");
-    if (tiled) {
-        TlmGqaArgs u = t;
-        part(u, wide ? 5 : 4, sp[1 + wide], false);
-        launch(u, true);
-        part(t, 3, sp[0], true);
-    } else {
-        part(t, 0, sh.tiles[L.geo], true);
-    }
-    if (t.n_tiles) launch(t, false);
+    TlmGqaArgs u = t;
+    part(u, wide ? 5 : 4, tiled ? sp[1 + wide] : 0, false);
+    if (tiled) part(t, 3, sp[0], true);
+    else part(t, 0, sh.tiles[L.geo], true);
+    P.add([=](hipStream_t s) { return f32 ? launch_gqa_t<TlmF32>(s, u, t, bound) : launch_gqa_t<TlmBf16>(s, u, t, bound); });
     return MixerOut{&L.out, m->o, L.out.KS};
 }
 

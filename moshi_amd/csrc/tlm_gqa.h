@@ -69,14 +69,13 @@ struct TlmGqa {
 // Few column tiles (decoding): the four waves of a workgroup share one column tile, each takes every 4th key block straight from the
 // cache - the block after it is requested fragment by fragment as the registers fall free - and their sums meet in LDS.
 // grid: column tiles (rounded up to 8), kv heads, splits of the keys (k_tlm_gqa_combine)
+constexpr int TLM_GQA_LDS = 4 * 8 * 64 + 32;               // vectors of four floats
 template <class Tr, int D>
-__global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa(TlmGqaArgs a) {
+__device__ __forceinline__ void tlm_gqa(const TlmGqaArgs& a, f32x4* ob, int tile, int g, int split) {      // ob: TLM_GQA_LDS
     typedef TlmGqa<Tr, D> P;
     constexpr int WK = 4, NK = P::NK, ND = P::ND, NB = P::NB, F = P::F, VG = 4 * NB;
-    MMI_SHARED float ml[2][4][16];
-    MMI_SHARED __attribute__((aligned(16))) f32x4 ob[4 * 8 * 64];
+    float (*ml)[4][16] = reinterpret_cast<float (*)[4][16]>(ob + 4 * 8 * 64);      // [2][4][16]
     const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15, kq = lane >> 4;
-    const int tile = (int)blockIdx.x, g = (int)blockIdx.y, split = (int)blockIdx.z;
     const TlmCols c = P::find(a, tile);
     const int col = c.c0 + bl < c.ncol ? c.c0 + bl : c.ncol - 1;
     const int pos0 = a.epos0[c.entry];
@@ -170,6 +169,11 @@ __global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa
         a.pml[part * 32 + 16 + bl] = L;
     }
 }
+template <class Tr, int D>
+__global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa(TlmGqaArgs a) {
+    MMI_SHARED __attribute__((aligned(16))) f32x4 ob[TLM_GQA_LDS];
+    tlm_gqa<Tr, D>(a, ob, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+}
 
 // the splits (at most 16) of one column tile -> output; a wave takes one 16-wide block of values, all its loads in flight together.
 // grid: column tiles, kv heads, blocks / 4
@@ -211,18 +215,16 @@ __global__ __launch_bounds__(256) void k_tlm_gqa_combine(TlmGqaArgs a) {
 template <class Tr, int D>
 struct TlmGqaTile {
     static constexpr int QT = Tr::V == 8 || D <= 128 ? 2 : 1, NF = TlmGqa<Tr, D>::F;
-    static constexpr size_t smem() { return (size_t)2 * NF * 1024; }
+    static constexpr size_t smem() { return std::max((size_t)2 * NF * 1024, (size_t)TLM_GQA_LDS * 16); }
 };
 template <class Tr, int D>
-__global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa_tile(TlmGqaArgs a) {
+__device__ __forceinline__ void tlm_gqa_tile(const TlmGqaArgs& a, u32x4* lds, int tile, int g) {
     typedef TlmGqa<Tr, D> P;
     constexpr int NK = P::NK, ND = P::ND, QT = TlmGqaTile<Tr, D>::QT, NF = P::F, NI = NF / 4;
     typedef TlmAttnStream<Tr, ND, 0, QT, (ND >= 16 ? 4 : 8)> S;
     static_assert(2 * NK % 4 == 0 && NF % 4 == 0 && S::F == NF, "whole fragments per wave, keys and values apart; the stream's order");
-    MMI_DYN_SHARED(u32x4, lds);
     const int lane = (int)threadIdx.x & 63, wave = mmi_uniform((int)threadIdx.x >> 6), bl = lane & 15, kq = lane >> 4;
-    const int g = (int)blockIdx.y;
-    TlmCols c = P::find(a, (int)gridDim.x - 1 - (int)blockIdx.x);  // (tile0 counts groups of 64 QT columns here; the last see most keys: they start first)
+    TlmCols c = P::find(a, a.n_tiles - 1 - tile);  // (tile0 counts groups of 64 QT columns here; the last see most keys: they start first)
     c.c0 *= 4 * QT;
     const int pos0 = a.epos0[c.entry];
     const TlmWalk w(a.mask, pos0 + c.c0 / a.rep, pos0 + min(c.c0 + 64 * QT - 1, c.ncol - 1) / a.rep);
@@ -300,4 +302,14 @@ __global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa
         for (int d = 0; d < ND; ++d)
             if (d < a.nd) P::store(a, o, g, bl, kq, d, sm.acc[t][d] * inv);
     }
+}
+// BESIDE: with the column tiles of sequences with few columns, `t`, in the same launch - neither fills the chip, and they share nothing.  Two portions
+// of 331 tokens and 14 single ones, 16 heads on 4 of 128: 20.5 + 11.8 us in launches of their own, 26.2 together.  (a kernel of its own: the same
+// code without single ones takes 92 us for 1773 tokens, 28 heads on 7, where the plain kernel takes 78)
+template <class Tr, int D, bool BESIDE>
+__global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa_tile(TlmGqaArgs u, TlmGqaArgs t) {
+    MMI_DYN_SHARED(u32x4, lds);
+    const int b = (int)blockIdx.x, own = b - u.n_tiles * u.kv_heads;
+    if (!BESIDE || own < 0) tlm_gqa_tile<Tr, D>(u, lds, b % u.n_tiles, b / u.n_tiles);
+    else tlm_gqa<Tr, D>(t, reinterpret_cast<f32x4*>(lds), own % t.n_tiles, own / t.n_tiles % t.kv_heads, own / t.n_tiles / t.kv_heads);
 }

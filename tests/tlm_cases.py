@@ -323,6 +323,8 @@ def check_long_prompt_beside_decoding(dev, lib, dtype=F32, n=340, name="many_kv_
 
 
 BESIDE = {
+    "heads_of_128": plain_layer(replace(GQA, heads=28, kv_heads=7, dim=128, vdim=96, window=300, keep_first=70, scale=0.1)),
+    "heads_of_256": plain_layer(replace(GQA, heads=26, kv_heads=13, dim=160, vdim=256, window=0, keep_first=0, scale=0.08)),
     "many_kv_heads": plain_layer(replace(GQA, heads=26, kv_heads=13, window=150)),
     "all": plain_layer(None, layers=[TokenLayerConfig(DELTA, GLU), TokenLayerConfig(replace(GQA, heads=26, kv_heads=13, window=100), GLU), TokenLayerConfig(LIGHT, None)],
                        bigram=BigramConfig(buckets=29, mul_prev=7, mul_cur=2), max_positions=2000, loop_start=1, loop_stop=3, loop_times=2),
