@@ -285,34 +285,37 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_conv(TlmLinArgs a, int kg
 }
 
 // ------------------------------------------------------------------------------------------------
-// chunks, lightning: P, the decayed queries, the decayed transposed keys.  grid: chunks, heads
+// chunks, lightning: P, the decayed queries, the decayed transposed keys.  grid: chunks x heads, in eight waves: wave w has
+// token block w % 4 of P and every other column block
 // ------------------------------------------------------------------------------------------------
-inline __global__ __launch_bounds__(256, 4) void k_tlm_chunk_lightning(TlmLinArgs a) {
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), bl = lane & 15, kq = lane >> 4, h = (int)blockIdx.y;
-    const TlmSeg ck = a.chunk[blockIdx.x];
+inline size_t tlm_chunk_lightning_smem() { return (size_t)(2 * TLM_CHUNK * TLM_PST + TLM_CHUNK + 1) * sizeof(float); }
+inline __device__ __forceinline__ void tlm_chunk_lightning(const TlmLinArgs& a, float* sh, int chunk, int h) {
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), bl = lane & 15, kq = lane >> 4;
+    const int tb = wave & 3, j0 = wave >> 2;
+    const TlmSeg ck = a.chunk[chunk];
     const int D = a.dim_p;
-    const long id = (long)blockIdx.x * a.heads + h;
-    MMI_SHARED __attribute__((aligned(16))) float Q[TLM_CHUNK * TLM_PST], K[TLM_CHUNK * TLM_PST], pw[TLM_CHUNK + 1];
-    for (int i = tid; i <= TLM_CHUNK; i += 256) pw[i] = a.decay[h * (TLM_CHUNK + 1) + i];
+    const long id = (long)chunk * a.heads + h;
+    float *Q = sh, *K = Q + TLM_CHUNK * TLM_PST, *pw = K + TLM_CHUNK * TLM_PST;      // [64][TLM_PST] twice, [65]
+    for (int i = tid; i <= TLM_CHUNK; i += 512) pw[i] = a.decay[h * (TLM_CHUNK + 1) + i];
     const float* qp = a.in + (long)ck.row0 * a.in_ld + a.q0 + h * D;
     const float* kp = a.in + (long)ck.row0 * a.in_ld + a.k0 + h * D;
     float *Qg = a.qg + id * TLM_CHUNK * D, *Kt = a.kt + id * TLM_CHUNK * D, *P = a.p + id * (TLM_CHUNK * TLM_CHUNK);
-    f32x4 acc[4];
+    f32x4 acc[2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < D; c0 += 64) {                   // panels of 64 channels (a multiple of 16 in the last one)
         const int cn = min(64, D - c0);
-        f32x4 qv[4], kv[4];
+        f32x4 qv[2], kv[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {                      // (rows and columns past the end: a valid address, as zeros)
-            const int t = (tid >> 4) + 16 * i, c = min(4 * (tid & 15), cn - 4);
+        for (int i = 0; i < 2; ++i) {                      // (rows and columns past the end: a valid address, as zeros)
+            const int t = (tid >> 4) + 32 * i, c = min(4 * (tid & 15), cn - 4);
             qv[i] = *reinterpret_cast<const f32x4*>(qp + (long)min(t, ck.n - 1) * a.in_ld + c0 + c);
             kv[i] = *reinterpret_cast<const f32x4*>(kp + (long)min(t, ck.n - 1) * a.in_ld + c0 + c);
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int t = (tid >> 4) + 16 * i, c = 4 * (tid & 15);
+        for (int i = 0; i < 2; ++i) {
+            const int t = (tid >> 4) + 32 * i, c = 4 * (tid & 15);
             if (t >= ck.n || c >= cn) qv[i] = kv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
             *reinterpret_cast<f32x4*>(Q + t * TLM_PST + c) = qv[i];
             *reinterpret_cast<f32x4*>(K + t * TLM_PST + c) = kv[i];
@@ -320,12 +323,12 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_chunk_lightning(TlmLinArg
         }
         __syncthreads();
         for (int c = 4 * kq; c < cn; c += 16) {
-            const u32x4 q = *reinterpret_cast<const u32x4*>(Q + (16 * wave + bl) * TLM_PST + c);
+            const u32x4 q = *reinterpret_cast<const u32x4*>(Q + (16 * tb + bl) * TLM_PST + c);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (j <= wave) acc[j] = TlmF32::mfma(q, *reinterpret_cast<const u32x4*>(K + (16 * j + bl) * TLM_PST + c), acc[j]);
+            for (int j = 0; j < 2; ++j)
+                if (2 * j + j0 <= tb) acc[j] = TlmF32::mfma(q, *reinterpret_cast<const u32x4*>(K + (16 * (2 * j + j0) + bl) * TLM_PST + c), acc[j]);
         }
-        for (int i = wave; i < cn / 4; i += 4) {           // transposed fragments: 16 channels x 16 tokens
+        for (int i = wave; i < cn / 4; i += 8) {           // transposed fragments: 16 channels x 16 tokens
             const int c = 16 * (i >> 2) + bl, t = 16 * (i & 3) + 4 * kq;
             f32x4 v;
 #pragma unroll
@@ -334,14 +337,23 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_chunk_lightning(TlmLinArg
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (j <= wave)
+    for (int j = 0; j < 2; ++j)
+        if (2 * j + j0 <= tb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int t = 16 * wave + 4 * kq + r, s = 16 * j + bl;
+                const int t = 16 * tb + 4 * kq + r, s = 16 * (2 * j + j0) + bl;
                 P[tlm_tile(t, s, 4)] = s <= t ? acc[j][r] * pw[t - s] : 0.f;
             }
-    for (int d = tid; d < D; d += 256) a.gend[id * D + d] = pw[ck.n];
+    for (int d = tid; d < D; d += 512) a.gend[id * D + d] = pw[ck.n];
+}
+// beside them single tokens, as beside the delta rule's chunks; workgroups of 512 for their sake.  11 chunks and 14 sequences, 16 heads of
+// 128 x 128: 12.2 + 8.8 us in launches of their own, 13.1 together; 896 chunks alone (its bytes: 5 TB/s) 28.5 in four waves, 30.0 in eight
+template <class Tr>
+__global__ __launch_bounds__(512, 4) void k_tlm_chunk_lightning(TlmLinArgs a, int n_chunk, int n_small, int cgp) {
+    MMI_DYN_SHARED(float, sh);
+    const int b = (int)blockIdx.x, own = b - n_chunk * a.heads;
+    if (own < 0) tlm_chunk_lightning(a, sh, b % n_chunk, b / n_chunk);
+    else tlm_state_step<Tr, false, 8>(a, sh, cgp, own % n_small, own / n_small);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -80,9 +80,10 @@ def test_chunk_edges(lib, dim, vdim, n):
 
 
 @pytest.mark.parametrize("dtype", [tc.F32, tc.BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("lightning", [False, True], ids=["delta", "lightning"])
 @pytest.mark.parametrize("dim,vdim", tc.BESIDE_CHUNKS)
-def test_tokens_beside_chunks(lib, dim, vdim, dtype):
-    tc.check_tokens_beside_chunks(DEV, lib, dim, vdim, dtype)
+def test_tokens_beside_chunks(lib, dim, vdim, dtype, lightning):
+    tc.check_tokens_beside_chunks(DEV, lib, dim, vdim, dtype, lightning)
 
 
 @pytest.mark.parametrize("window", [70, 64, 0])

@@ -36,9 +36,10 @@ def test_chunk_edges(tlm_lib, dim, vdim, n):
     tc.check_chunk_edges(DEV, tlm_lib, dim, vdim, n)
 
 
+@pytest.mark.parametrize("lightning", [False, True], ids=["delta", "lightning"])
 @pytest.mark.parametrize("dim,vdim", tc.BESIDE_CHUNKS)
-def test_tokens_beside_chunks(tlm_lib, dim, vdim):
-    tc.check_tokens_beside_chunks(DEV, tlm_lib, dim, vdim)
+def test_tokens_beside_chunks(tlm_lib, dim, vdim, lightning):
+    tc.check_tokens_beside_chunks(DEV, tlm_lib, dim, vdim, lightning=lightning)
 
 
 def test_activation_branches(tlm_lib):

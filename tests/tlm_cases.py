@@ -515,9 +515,9 @@ def check_chunk_edges(dev, lib, dim, vdim, n):
 BESIDE_CHUNKS = [(128, 128), (96, 128), (64, 256), (256, 64), (200, 48), (32, 32)]
 
 
-def check_tokens_beside_chunks(dev, lib, dim, vdim, dtype=F32):
+def check_tokens_beside_chunks(dev, lib, dim, vdim, dtype=F32, lightning=False):
     """A step of a prompt portion, of 1 and 3 tokens of running sequences and of a new sequence's first token; then a token each on top."""
-    cfg = plain_layer(replace(DELTA, heads=4, kv_heads=2, dim=dim, vdim=vdim))
+    cfg = plain_layer(replace(LIGHT, dim=dim, vdim=vdim) if lightning else replace(DELTA, heads=4, kv_heads=2, dim=dim, vdim=vdim))
     lm, orc = make(cfg, dev, lib, dtype)
     cuts = {0: (20, 1, 1), 1: (9, 3, 1), 2: (0, 70, 1), 3: (0, 1, 1), 4: (66, 65, 1)}
     toks = {i: tokens_of(cfg, sum(c), seed=i) for i, c in cuts.items()}
