@@ -1,5 +1,6 @@
 // Version / error plumbing of the C ABI (include/moshi_mi.h).
 #include "mmi_common.h"
+#include <mutex>
 
 static thread_local std::string g_last_error;
 
@@ -12,6 +13,35 @@ int mmi_fail(int code, const std::string& msg) {
 
 extern "C" int mmi_version(void) { return MMI_ABI_VERSION; }
 extern "C" const char* mmi_last_error(void) { return g_last_error.c_str(); }
+
+// ---- device memory (mmi_common.h) --------------------------------------------------------------------------------------
+static std::mutex g_unfreed_mu;
+static std::vector<void*>& unfreed() {                     // (never destroyed: handles may outlive this file's statics)
+    static std::vector<void*>* list = new std::vector<void*>;
+    return *list;
+}
+static void free_unfreed() {
+    std::lock_guard<std::mutex> g(g_unfreed_mu);
+    std::vector<void*>& list = unfreed();
+    while (!list.empty()) {
+        if (hipFree(list.back()) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        list.pop_back();
+    }
+}
+hipError_t mmi_malloc(void** p, size_t bytes) {
+    free_unfreed();
+    return hipMalloc(p, bytes);
+}
+void mmi_free(void* p) {
+    free_unfreed();
+    if (!p || hipFree(p) == hipSuccess) return;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> g(g_unfreed_mu);
+    unfreed().push_back(p);
+}
 
 // ---- launch-list recorder (mmi_graph.h) ------------------------------------------------------------------------------
 static thread_local std::vector<std::string>* g_rec_log = nullptr;

@@ -60,9 +60,13 @@ struct MimiSlab {
         rewind();
         return true;
     }
+    void drop() {                              // with the handle: freed now or later
+        if (!release()) mmi_free(base);
+        base = nullptr;
+    }
     hipError_t reserve(size_t nb) {            // never beside the old one: nothing of it may be in flight
         if (!release()) return hipErrorOutOfMemory;
-        hipError_t e = hipMalloc((void**)&base, nb);
+        hipError_t e = mmi_malloc((void**)&base, nb);
         if (e == hipSuccess) size = nb;
         return e;
     }
@@ -1508,8 +1512,8 @@ extern "C" void mmi_mimi_destroy(mmi_mimi* m) {
     if (!m) return;
     drop_parked(m);
     mmi_mimi_streaming_stop(m);
-    m->enc_grp.slab.release();
-    m->dec_grp.slab.release();
+    m->enc_grp.slab.drop();
+    m->dec_grp.slab.drop();
     m->wts.release();
     if (m->cap_stream) hipStreamDestroy(m->cap_stream);
     delete m;
@@ -1616,7 +1620,9 @@ constexpr size_t MIMI_PARK = (size_t)128 << 20;
 
 extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
-    if (!m || !m->parked || m->batch != batch || m->parked_k != m->n_codebooks || recording((hipStream_t)stream)) return mmi_mimi_streaming_start(m, batch, stream);
+    if (!m || !m->parked || m->batch != batch || m->parked_k != m->n_codebooks) return mmi_mimi_streaming_start(m, batch, stream);
+    // (a stream cannot start there either: it waits for its own state)
+    if (recording((hipStream_t)stream)) return mmi_fail(MMI_ERR_HIP, "a file's stream cannot start while its HIP stream is being captured");
     m->parked = false;
     m->streaming = true;
     m->all_exec = 1;

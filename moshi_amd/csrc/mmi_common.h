@@ -84,6 +84,11 @@ struct MmiWeights {
     }
 };
 
+// hipMalloc and hipFree (api_common.hip).  The runtime does neither while another thread captures in the global mode: what mmi_free could not free
+// stays in a list of the process, and goes with the next call of either.
+hipError_t mmi_malloc(void** p, size_t bytes);
+void mmi_free(void* p);
+
 // device allocation bookkeeping: every engine frees what it allocated
 // chunk > 0: allocations up to an eighth of it are cut out of pieces of that size, zeroed when they are made, instead of each being one of
 // the runtime's (a stream of the codec is some 90 of them: start 0.60 -> 0.20 ms, when its convs still had offset tables, written by the GPU; stop 0.18 -> 0.09)
@@ -94,10 +99,10 @@ struct MmiArena {
     std::vector<char*> chunks;
     std::vector<const void*> own;                  // allocations that name places of this arena: saved like the others, but not loaded
     hipError_t take(void** q, size_t nb) {
-        if (nb > chunk / 8) return hipMalloc(q, nb);
+        if (nb > chunk / 8) return mmi_malloc(q, nb);
         if (chunks.empty() || at + nb > chunk) {
             char* c = nullptr;
-            hipError_t e = hipMalloc((void**)&c, chunk);
+            hipError_t e = mmi_malloc((void**)&c, chunk);
             if (e != hipSuccess) return e;
             chunks.push_back(c);
             at = 0;
@@ -131,7 +136,7 @@ struct MmiArena {
         // (MMI_DEBUG_POISON=0: zero-fill instead - two sessions then start from identical memory, which is what MMI_DEBUG_TRACE's
         // per-op checksums need to be comparable line by line)
         const char* pz = getenv("MMI_DEBUG_POISON");
-        if (pz && (pz[0] == '1' || pz[0] == '0') && (e = hipMemset(q, pz[0] == '1' ? 0xFF : 0x00, nb)) != hipSuccess) { if (!cut(q)) hipFree(q); return e; }
+        if (pz && (pz[0] == '1' || pz[0] == '0') && (e = hipMemset(q, pz[0] == '1' ? 0xFF : 0x00, nb)) != hipSuccess) { if (!cut(q)) mmi_free(q); return e; }
         ptrs.push_back(q);
         sizes.push_back(nb);
         bytes += nb;
@@ -140,8 +145,8 @@ struct MmiArena {
     }
     void release() {
         for (void* p : ptrs)
-            if (!cut(p)) hipFree(p);
-        for (char* c : chunks) hipFree(c);
+            if (!cut(p)) mmi_free(p);
+        for (char* c : chunks) mmi_free(c);
         chunks.clear();
         own.clear();
         at = 0;

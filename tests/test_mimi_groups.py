@@ -282,6 +282,48 @@ def test_what_a_file_leaves_goes_with_the_next_stream(sim_lib):
     assert sim_bytes(sim_lib) == empty
 
 
+@pytest.mark.parametrize("blocking", [False, True])
+def test_files_while_another_thread_captures(sim_lib, blocking):
+    """The runtime does not free while another thread captures: what a file's stream has left is not lost then, whether the next file is of
+    other rows (it fails, as without an earlier one), of the same rows (it fails where the null stream cannot be asked, and the one behind the
+    capture finds everything still there) or the handle goes."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    fs, capture_elsewhere = cfg.frame_size, sim_lib.cdll.hipsim_set_capture_elsewhere
+    x = 0.3 * torch.randn(2, 1, fs, generator=torch.Generator().manual_seed(4))
+    gc.collect()
+    empty = sim_bytes(sim_lib)
+    m = MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+    before = sim_bytes(sim_lib)
+    want = m.encode(x[:1])
+    kept = sim_bytes(sim_lib)
+    assert kept > before
+    try:
+        for _ in range(2):
+            capture_elsewhere(1 + blocking)
+            if blocking:
+                with pytest.raises(RuntimeError):
+                    m.encode(x[:1])
+            else:
+                assert torch.equal(m.encode(x[:1]), want)
+            assert sim_bytes(sim_lib) == kept and not m.is_streaming
+            with pytest.raises(RuntimeError):
+                m.encode(x)
+            capture_elsewhere(0)
+            assert torch.equal(m.encode(x[:1]), want) and sim_bytes(sim_lib) == kept
+        other = MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+        other.encode(torch.cat([x[:1]] * 9, -1))               # (with a group's memory)
+        capture_elsewhere(1 + blocking)
+        del m, other
+        gc.collect()
+        assert sim_bytes(sim_lib) > empty
+    finally:
+        capture_elsewhere(0)
+    MimiModel(sd, cfg, device="cpu", max_batch=2, num_codebooks=4, lib=sim_lib)
+    gc.collect()
+    assert sim_bytes(sim_lib) == empty
+
+
 def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
     """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
     stream it is called on, and leaves the one that the snapshot came from alone."""
