@@ -309,6 +309,9 @@ __device__ __forceinline__ void mmi_here(T& x) { asm volatile("" : "+v"(x)); }
 // a value that is the same in every lane (a wave index, what was loaded through one), told to the compiler: it stays in scalar registers,
 // and loads addressed by it are scalar loads - they do not queue behind the vector loads in flight
 __device__ __forceinline__ int mmi_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// a load from memory that nothing writes while the kernel runs: by a uniform address a scalar load, also where the compiler cannot rule out that
+// one of the kernel's stores meets it
+__device__ __forceinline__ int mmi_load_const(const int* p) { return *(const __attribute__((address_space(4))) int*)p; }
 // true in every lane when any lane's flag is set
 __device__ __forceinline__ bool mmi_any(bool v) { return __any(v) != 0; }
 

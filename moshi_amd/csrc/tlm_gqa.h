@@ -303,9 +303,10 @@ __device__ __forceinline__ void tlm_gqa_tile(const TlmGqaArgs& a, u32x4* lds, in
             if (d < a.nd) P::store(a, o, g, bl, kq, d, sm.acc[t][d] * inv);
     }
 }
-// BESIDE: with the column tiles of sequences with few columns, `t`, in the same launch - neither fills the chip, and they share nothing.  Two portions
-// of 331 tokens and 14 single ones, 16 heads on 4 of 128: 20.5 + 11.8 us in launches of their own, 26.2 together.  (a kernel of its own: the same
-// code without single ones takes 92 us for 1773 tokens, 28 heads on 7, where the plain kernel takes 78)
+// BESIDE: with the column tiles of sequences with few columns, `t`, in the same launch - neither fills the chip, and they share nothing.  16 heads on
+// 4 of 128, in launches of their own and together: two portions of 331 tokens and 14 single ones 31.2 and 22.6 us, one of 1773 and one 79.9 and
+// 66.8; 32 heads on 8: 98.5 and 84.8 for 1773 and 14, 122.5 and 87.4 for 64.  (What a block's page is must be known by a scalar load,
+// mmi_load_const: behind the stores of the other body it became a vector load, and the wait for it one for every key in flight - 85.3 us, not 66.8.)
 template <class Tr, int D, bool BESIDE>
 __global__ __launch_bounds__(256, Tr::V == 8 && D <= 128 ? 2 : 1) void k_tlm_gqa_tile(TlmGqaArgs u, TlmGqaArgs t) {
     MMI_DYN_SHARED(u32x4, lds);

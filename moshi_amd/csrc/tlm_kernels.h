@@ -974,7 +974,7 @@ __global__ __launch_bounds__(256) void k_tlm_latent(TlmLatentArgs a) {
 struct TlmMask { int window, keep; float scale; };
 // pages of a sequence: the block table's first `keep` entries are for the pages that no window releases, the others are a ring
 struct TlmPages { const int* table; int ld, keep; };
-__device__ __forceinline__ int tlm_page(const TlmPages& p, const int* row, int i) { return row[i < p.keep ? i : p.keep + (i - p.keep) % (p.ld - p.keep)]; }
+__device__ __forceinline__ int tlm_page(const TlmPages& p, const int* row, int i) { return mmi_load_const(row + (i < p.keep ? i : p.keep + (i - p.keep) % (p.ld - p.keep))); }
 
 struct TlmAttnArgs {
     const void* q;                       // packed rows token * heads + head

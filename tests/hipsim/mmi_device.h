@@ -389,6 +389,7 @@ inline void mmi_sched_barrier() {}
 template <class T>
 inline void mmi_here(T&) {}
 inline int mmi_uniform(int v) { return v; }
+inline int mmi_load_const(const int* p) { return *p; }
 inline bool mmi_any(bool v) { unsigned x = v ? 1u : 0u; for (int m = 1; m < 64; m <<= 1) { const unsigned o = mmi_shfl_xor(x, m); x = o > x ? o : x; } return x != 0; }
 inline void mmi_load_lds(const void* base, unsigned off, u32x4* lds, int at) { lds[at + (int)(threadIdx.x & 63)] = *(const u32x4*)((const char*)base + off); }
 inline void mmi_load_lds(const u32x4* from, u32x4* lds, int at) { lds[at + (int)(threadIdx.x & 63)] = *from; }
