@@ -1436,23 +1436,30 @@ int launch_state_step(hipStream_t s, const TlmLinArgs& a, int n) {
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
-template <class Tr, int NP>
+template <class Tr, int NP, bool BESIDE>
 int launch_chunk_delta_t(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
     const size_t smem = tlm_chunk_delta_smem();
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta<Tr, NP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tlm_chunk_delta<Tr, NP, BESIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     MMI_HIP_CHECK(attr);
-    MMI_LAUNCH((k_tlm_chunk_delta<Tr, NP>), (n_chunk + n_small) * a.heads, 512, smem, s, a, n_chunk, n_small, tlm_step_groups(a.vdim_p));
+    MMI_LAUNCH((k_tlm_chunk_delta<Tr, NP, BESIDE>), (n_chunk + n_small) * a.heads, 512, smem, s, a, n_chunk, n_small, tlm_step_groups(a.vdim_p));
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
+// (chunks alone: one kernel for both types)
+template <class Tr, int NP>
+int launch_chunk_delta_n(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
+    return n_small ? launch_chunk_delta_t<Tr, NP, true>(s, a, n_chunk, n_small) : launch_chunk_delta_t<TlmF32, NP, false>(s, a, n_chunk, 0);
+}
 template <class Tr>
 int launch_chunk_delta(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
-    if (a.dim_p <= 64) return launch_chunk_delta_t<Tr, 1>(s, a, n_chunk, n_small);
-    return a.dim_p <= 128 ? launch_chunk_delta_t<Tr, 2>(s, a, n_chunk, n_small) : launch_chunk_delta_t<Tr, 4>(s, a, n_chunk, n_small);
+    if (a.dim_p <= 64) return launch_chunk_delta_n<Tr, 1>(s, a, n_chunk, n_small);
+    return a.dim_p <= 128 ? launch_chunk_delta_n<Tr, 2>(s, a, n_chunk, n_small) : launch_chunk_delta_n<Tr, 4>(s, a, n_chunk, n_small);
 }
 template <class Tr>
 int launch_chunk_lightning(hipStream_t s, const TlmLinArgs& a, int n_chunk, int n_small) {
-    MMI_LAUNCH((k_tlm_chunk_lightning<Tr>), (n_chunk + n_small) * a.heads, 512, tlm_chunk_lightning_smem(), s, a, n_chunk, n_small, tlm_step_groups(a.vdim_p));
+    const size_t smem = tlm_chunk_lightning_smem();
+    if (n_small) MMI_LAUNCH((k_tlm_chunk_lightning<Tr, true>), (n_chunk + n_small) * a.heads, 512, smem, s, a, n_chunk, n_small, tlm_step_groups(a.vdim_p));
+    else MMI_LAUNCH((k_tlm_chunk_lightning<TlmF32, false>), n_chunk * a.heads, 512, smem, s, a, n_chunk, 0, 0);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
@@ -1544,7 +1551,7 @@ MixerOut build_linear(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Layer& L
         add_jobs(m, P, p, Q, L.a2.bytes() + L.g2.bytes());
     }
     const int n_small = sh.n_small, n_unit = sh.n_unit, n_chunk = sh.n_chunk;
-    // chunks and single tokens of one step in one launch where both take workgroups of 512 (delta 23.3 + 16.4 -> 27.0 us, lightning 12.2 + 8.8 -> 13.1)
+    // chunks and single tokens of one step in one launch where both take workgroups of 512 (k_tlm_chunk_delta, k_tlm_chunk_lightning: what it gives)
     const StepShape z = step_shape(a);
     const bool together = n_small && n_chunk && z.rt == 8 && z.block == 512 && z.smem <= (delta ? tlm_chunk_delta_smem() : tlm_chunk_lightning_smem());
     if (n_small && !together) {

@@ -346,13 +346,14 @@ inline __device__ __forceinline__ void tlm_chunk_lightning(const TlmLinArgs& a, 
             }
     for (int d = tid; d < D; d += 512) a.gend[id * D + d] = pw[ck.n];
 }
-// beside them single tokens, as beside the delta rule's chunks; workgroups of 512 for their sake.  11 chunks and 14 sequences, 16 heads of
-// 128 x 128: 12.2 + 8.8 us in launches of their own, 13.1 together; 896 chunks alone (its bytes: 5 TB/s) 28.5 in four waves, 30.0 in eight
-template <class Tr>
+// BESIDE: with the single tokens of n_small sequences, as beside the delta rule's chunks.  11 chunks and 14 sequences, 16 heads of 128 x 128: 20.9 us in
+// launches of their own, 13.2 together.  Chunks alone have a kernel without the other body (58 registers, 94 with it; its bytes bound it where
+// chunks are many): 896 of 128 x 128 28.4 us, 31.7 with it, 29.6 in workgroups of four waves; 176 9.5, 9.9 and 12.1.
+template <class Tr, bool BESIDE>
 __global__ __launch_bounds__(512, 4) void k_tlm_chunk_lightning(TlmLinArgs a, int n_chunk, int n_small, int cgp) {
     MMI_DYN_SHARED(float, sh);
     const int b = (int)blockIdx.x, own = b - n_chunk * a.heads;
-    if (own < 0) tlm_chunk_lightning(a, sh, b % n_chunk, b / n_chunk);
+    if (!BESIDE || own < 0) tlm_chunk_lightning(a, sh, b % n_chunk, b / n_chunk);
     else tlm_state_step<Tr, false, 8>(a, sh, cgp, own % n_small, own / n_small);
 }
 
@@ -689,13 +690,15 @@ __device__ __forceinline__ void tlm_chunk_delta(const TlmLinArgs& a, float* sh, 
                 tlm_quad(Wg, ((i * nd + st) * 64 + lane) * 4) = *reinterpret_cast<const f32x4*>(T + (16 * i + bl) * 20 + 4 * kq);
     }
 }
-// beside them the single tokens of n_small sequences, where those take workgroups of 512 too: neither fills the chip, and they share nothing.
-// 11 chunks and 14 sequences, 16 heads of 128 x 128: 23.3 + 16.4 us in launches of their own, 27.0 together
-template <class Tr, int NP>
+// BESIDE: with the single tokens of n_small sequences, where those take workgroups of 512 too: neither fills the chip, and they share nothing.
+// 11 chunks and 14 sequences, 16 heads of 128 x 128: 38.6 us in launches of their own, 26.0 together; 1 - 64 sequences beside 2 - 28 chunks of 16 and
+// 32 heads gain as much or more, but 64 beside 16 chunks of 256 x 64 (one workgroup per CU by its registers) break even.  Chunks alone have a kernel without the
+// other body: with it, scalar registers spill (896 chunks of 128 x 128 71.0 us, 68.0 without).
+template <class Tr, int NP, bool BESIDE>
 __global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLinArgs a, int n_chunk, int n_small, int cgp) {
     MMI_DYN_SHARED(float, sh);
     const int b = (int)blockIdx.x, own = b - n_chunk * a.heads;
-    if (own < 0) tlm_chunk_delta<NP>(a, sh, b % n_chunk, b / n_chunk);
+    if (!BESIDE || own < 0) tlm_chunk_delta<NP>(a, sh, b % n_chunk, b / n_chunk);
     else tlm_state_step<Tr, true, 8>(a, sh, cgp, own % n_small, own / n_small);
 }
 
