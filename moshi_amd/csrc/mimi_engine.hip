@@ -178,6 +178,7 @@ struct mmi_mimi {
     bool use_graph = true;
     bool parked = false;                       // not streaming; the state and the programs of the last file's stream are still here ...
     int parked_k = 0;                          // ... built for so many codebooks
+    bool unfinished = false;                   // the wait behind that stream has failed: work on the device may still use what it has left
 };
 
 namespace {
@@ -1577,13 +1578,23 @@ static int start_stream(mmi_mimi* m, int batch, hipStream_t s) {
     return MMI_OK;
 }
 
+// Work on the device done, for a stream whose own wait has failed
+static int finish_parked(mmi_mimi* m) {
+    if (!m->unfinished) return MMI_OK;
+    MMI_HIP_CHECK(hipDeviceSynchronize());
+    m->unfinished = false;
+    return MMI_OK;
+}
+
 extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
     if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
     if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
+    int rc = finish_parked(m);
+    if (rc) return rc;
     drop_parked(m);
-    int rc = start_stream(m, batch, (hipStream_t)stream);
+    rc = start_stream(m, batch, (hipStream_t)stream);
     if (rc == MMI_ERR_HIP && (m->enc_grp.slab.size || m->dec_grp.slab.size)) {      // without what an earlier stream's groups have left
         m->enc_grp.slab.release();
         m->dec_grp.slab.release();
@@ -1623,6 +1634,8 @@ extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream
     if (!m || !m->parked || m->batch != batch || m->parked_k != m->n_codebooks) return mmi_mimi_streaming_start(m, batch, stream);
     // (a stream cannot start there either: it waits for its own state)
     if (recording((hipStream_t)stream)) return mmi_fail(MMI_ERR_HIP, "a file's stream cannot start while its HIP stream is being captured");
+    int rc = finish_parked(m);
+    if (rc) return rc;
     m->parked = false;
     m->streaming = true;
     m->all_exec = 1;
@@ -1631,7 +1644,7 @@ extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream
         g->refused = false;
         g->earlier = true;
     }
-    const int rc = mmi_mimi_reset(m, nullptr, stream);
+    rc = mmi_mimi_reset(m, nullptr, stream);
     if (rc) mmi_mimi_streaming_stop(m);
     return rc;
 }
@@ -1640,15 +1653,13 @@ extern "C" int mmi_mimi_file_stop(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
     if (!m->streaming) return MMI_OK;
-    const hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess || m->st.held() > MIMI_PARK || getenv("MMI_DEBUG_POISON")) {
-        mmi_mimi_streaming_stop(m);
-        return e == hipSuccess ? (int)MMI_OK : mmi_fail(MMI_ERR_HIP, std::string("hipDeviceSynchronize: ") + hipGetErrorString(e));
-    }
     m->streaming = false;
     m->parked = true;
     m->parked_k = m->n_codebooks;
-    return MMI_OK;
+    m->unfinished = true;
+    int rc = finish_parked(m);                             // (where it fails nothing goes: work on the device may use it)
+    if (!rc && (m->st.held() > MIMI_PARK || getenv("MMI_DEBUG_POISON"))) drop_parked(m);
+    return rc;
 }
 
 extern "C" int mmi_mimi_streaming_batch(const mmi_mimi* m) { return m && m->streaming ? m->batch : 0; }

@@ -171,8 +171,8 @@ class MimiModel:
         try:
             yield
         finally:
+            self._batch = None                             # (also where the stop fails: the engine's stream has ended then, too)
             self._lib.check(self._lib.mmi_mimi_file_stop(self._handle))
-            self._batch = None
 
     @contextmanager
     def streaming(self, batch_size: int):

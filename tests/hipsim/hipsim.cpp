@@ -412,7 +412,8 @@ hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { memset(d, v, 
 hipError_t hipStreamCreate(hipStream_t* s) { *s = new hipsimStream(); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+static std::atomic<bool> g_sync_fails{false};
+hipError_t hipDeviceSynchronize() { return g_sync_fails ? failed(hipErrorUnknown) : hipSuccess; }
 hipError_t hipGetLastError() {
     const hipError_t e = t_last;
     t_last = hipSuccess;
@@ -454,5 +455,7 @@ extern "C" unsigned long long hipsim_peak_bytes(void) {
 }
 // memory of the device from now on (0: unlimited)
 extern "C" void hipsim_set_memory(unsigned long long bytes) { std::lock_guard<std::mutex> g(g_mem_mu); g_mem_total = bytes ? (size_t)bytes : ~(size_t)0; }
+// from now on waits for the device fail
+extern "C" void hipsim_set_sync_fails(int on) { g_sync_fails = on != 0; }
 // from now on another thread captures in the global mode, 1: a stream that does not block the null stream, 2: one that does, 0: it has ended
 extern "C" void hipsim_set_capture_elsewhere(int on) { g_elsewhere = on; }

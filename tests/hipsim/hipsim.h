@@ -47,7 +47,7 @@ int schedule();
 // ---- minimal HIP host API surface used by the engines -------------------------------------
 typedef int hipError_t;
 enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorNotSupported = 801,
-       hipErrorStreamCaptureUnsupported = 900, hipErrorStreamCaptureImplicit = 906 };
+       hipErrorStreamCaptureUnsupported = 900, hipErrorStreamCaptureImplicit = 906, hipErrorUnknown = 999 };
 typedef struct hipsimStream* hipStream_t;
 typedef struct hipsimEvent* hipEvent_t;
 typedef struct hipsimGraph* hipGraph_t;

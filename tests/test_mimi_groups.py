@@ -324,6 +324,35 @@ def test_files_while_another_thread_captures(sim_lib, blocking):
     assert sim_bytes(sim_lib) == empty
 
 
+def test_a_file_whose_wait_fails(sim_lib):
+    """A call on a file that cannot wait for the device raises.  Its stream has ended then, for the model and the engine; what it has left stays
+    until a wait succeeds (work on the device may use it), and the next file is a fresh one."""
+    cfg = tiny_mimi_config()
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    fs, sync_fails = cfg.frame_size, sim_lib.cdll.hipsim_set_sync_fails
+    x = 0.3 * torch.randn(1, 1, 2 * fs, generator=torch.Generator().manual_seed(4))
+    gc.collect()
+    empty = sim_bytes(sim_lib)
+    m = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+    want = m.encode(x)
+    kept = sim_bytes(sim_lib)
+    for begin in (lambda: m.encode(x), lambda: m.decode(want), lambda: m.streaming_forever(1)):
+        try:
+            sync_fails(1)
+            for call in (lambda: m.encode(x), begin):
+                with pytest.raises(RuntimeError, match="hipDeviceSynchronize"):
+                    call()
+                assert not m.is_streaming and sim_bytes(sim_lib) == kept
+        finally:
+            sync_fails(0)
+        assert torch.equal(m.encode(x), want) and sim_bytes(sim_lib) == kept
+    with m.streaming(1):
+        assert torch.equal(m.encode(x), want)
+    del m
+    gc.collect()
+    assert sim_bytes(sim_lib) == empty
+
+
 def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
     """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
     stream it is called on, and leaves the one that the snapshot came from alone."""
