@@ -112,7 +112,10 @@ int mmi_mimi_num_codebooks(const mmi_mimi* m);
 int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream);
 int mmi_mimi_streaming_stop(mmi_mimi* m);
 /* The same around one call on whole files (compression.py:354-359, 412-416): a fresh stream of `batch` rows, which ends with the work on the
- * device done.  What it has allocated and built may stay for the next one (at most 128 MB, until mmi_mimi_streaming_start or destroy). */
+ * device done.  What it has built stays for the next file of as many rows: at most 128 MB of state and, as behind any stream that ran several
+ * frames at once, the buffers of its groups of frames (up to 0.6 GB encoding, 0.8 GB decoding).  The state goes with mmi_mimi_streaming_start, the
+ * buffers with the first single frame behind it; both go when an allocation of this library finds no memory on the device, with
+ * mmi_mimi_streaming_stop of a handle that is not streaming, and with the handle. */
 int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream);
 int mmi_mimi_file_stop(mmi_mimi* m);
 /* Rows of the current stream (StreamingModule._streaming_state.batch_size); 0 when not streaming. */

@@ -31,8 +31,14 @@ static void free_unfreed() {
         list.pop_back();
     }
 }
+static bool (*g_let_go)(int device) = nullptr;
+void mmi_set_let_go(bool (*let_go)(int device)) { g_let_go = let_go; }
 hipError_t mmi_malloc(void** p, size_t bytes) {
     free_unfreed();
+    const hipError_t e = hipMalloc(p, bytes);
+    int device = -1;
+    if (e != hipErrorOutOfMemory || !g_let_go || hipGetDevice(&device) != hipSuccess || !g_let_go(device)) return e;
+    (void)hipGetLastError();
     return hipMalloc(p, bytes);
 }
 void mmi_free(void* p) {

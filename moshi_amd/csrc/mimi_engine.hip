@@ -6,6 +6,7 @@
 
 #include <math.h>
 #include <algorithm>
+#include <mutex>
 
 namespace {
 
@@ -1500,19 +1501,70 @@ extern "C" int mmi_mimi_create(const mmi_mimi_cfg* cfg, const mmi_tensor_desc* w
     return MMI_OK;
 }
 
-// lets go what the last file's stream has left
-static void drop_parked(mmi_mimi* m) {
-    if (!m->parked) return;
-    m->parked = false;
-    m->streaming = true;
-    mmi_mimi_streaming_stop(m);
+// ---- what handles keep while they do not stream ----
+static void stop_stream(mmi_mimi* m) {
+    hipDeviceSynchronize();
+    m->enc_prog.clear();
+    m->dec_prog.clear();
+    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {      // their launches name the state that goes now; the slabs stay (give_back_group)
+        g->prog.clear();
+        g->frames = 0;
+        g->refused = false;
+    }
+    m->st.release();
+    m->partials.clear();
+    m->partial_sizes.clear();
+    m->streaming = m->parked = m->unfinished = false;
+    m->batch = 0;
 }
+static void drop_parked(mmi_mimi* m) {
+    if (m->parked) stop_stream(m);
+}
+
+// A handle that does not stream may keep the stream of its last file (mmi_mimi_file_stop) and the slabs of its groups of frames.  It is in a list
+// of the process then, and an allocation of any thread that finds no memory takes it away (let_go).  A call that starts, stops or ends a
+// stream takes its handle out for as long as it lasts.
+struct IdleHandles {
+    std::mutex mu;
+    std::vector<mmi_mimi*> list;
+};
+static IdleHandles& idle() {                               // (never destroyed: handles may outlive this file's statics)
+    static IdleHandles* h = new IdleHandles;
+    return *h;
+}
+struct OutOfIdle {
+    mmi_mimi* m;
+    explicit OutOfIdle(mmi_mimi* m_) : m(m_) {
+        std::lock_guard<std::mutex> g(idle().mu);
+        std::vector<mmi_mimi*>& list = idle().list;
+        list.erase(std::remove(list.begin(), list.end(), m), list.end());
+    }
+    ~OutOfIdle() {
+        if (!m || m->streaming || m->unfinished || !(m->parked || m->enc_grp.slab.size || m->dec_grp.slab.size)) return;
+        std::lock_guard<std::mutex> g(idle().mu);
+        idle().list.push_back(m);
+    }
+    OutOfIdle(const OutOfIdle&) = delete;
+    OutOfIdle& operator=(const OutOfIdle&) = delete;
+};
+static bool let_go(int device) {
+    std::lock_guard<std::mutex> g(idle().mu);
+    std::vector<mmi_mimi*>& list = idle().list;
+    const size_t n = list.size();
+    list.erase(std::remove_if(list.begin(), list.end(), [&](mmi_mimi* m) {
+        if (m->device != device) return false;
+        drop_parked(m);
+        return m->enc_grp.slab.release() && m->dec_grp.slab.release();
+    }), list.end());
+    return list.size() < n;
+}
+static const bool let_go_set = (mmi_set_let_go(&let_go), true);
 
 extern "C" void mmi_mimi_destroy(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return;
-    drop_parked(m);
-    mmi_mimi_streaming_stop(m);
+    { OutOfIdle out(m); out.m = nullptr; }                 // (for good)
+    if (m->streaming || m->parked) stop_stream(m);
     m->enc_grp.slab.drop();
     m->dec_grp.slab.drop();
     m->wts.release();
@@ -1555,7 +1607,7 @@ static int start_stream(mmi_mimi* m, int batch, hipStream_t s) {
     m->batch = batch;
     int rc = MMI_OK;
     m->st.chunk = (size_t)32 << 20;
-    auto fail = [&](int code) { m->streaming = true; mmi_mimi_streaming_stop(m); return code; };
+    auto fail = [&](int code) { stop_stream(m); return code; };
     if (hipSuccess != m->st.alloc(&m->exec, (size_t)batch) || hipSuccess != m->st.alloc(&m->first, (size_t)batch) ||
         hipSuccess != m->st.alloc(&m->counters, (size_t)2 * batch) || hipSuccess != m->st.alloc(&m->dec_k_dev, (size_t)1))
         return fail(mmi_fail(MMI_ERR_HIP, "out of device memory (state)"));
@@ -1586,9 +1638,8 @@ static int finish_parked(mmi_mimi* m) {
     return MMI_OK;
 }
 
-extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
-    MmiDeviceGuard dev_guard_(m ? m->device : -1);
-    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
+// (the handle is out of the idle ones)
+static int start_any_stream(mmi_mimi* m, int32_t batch, mmi_stream stream) {
     if (m->streaming) return mmi_fail(MMI_ERR_STATE, "already streaming");  // streaming.py:113
     if (batch <= 0 || batch > m->max_batch) return mmi_fail(MMI_ERR_SHAPE, "batch exceeds max_batch");
     int rc = finish_parked(m);
@@ -1603,35 +1654,40 @@ extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream s
     return rc;
 }
 
+extern "C" int mmi_mimi_streaming_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
+    MmiDeviceGuard dev_guard_(m ? m->device : -1);
+    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
+    OutOfIdle out(m);
+    return start_any_stream(m, batch, stream);
+}
+
 extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
-    if (!m->streaming) return MMI_OK;
-    hipDeviceSynchronize();
-    m->enc_prog.clear();
-    m->dec_prog.clear();
-    for (MimiGroup* g : {&m->enc_grp, &m->dec_grp}) {      // their launches name the state that goes now; the slabs stay (give_back_group)
-        g->prog.clear();
-        g->frames = 0;
-        g->refused = false;
+    OutOfIdle out(m);
+    if (m->streaming) {
+        stop_stream(m);
+        return MMI_OK;
     }
-    m->st.release();
-    m->partials.clear();
-    m->partial_sizes.clear();
-    m->streaming = false;
-    m->batch = 0;
+    const int rc = finish_parked(m);
+    if (rc) return rc;
+    drop_parked(m);
+    m->enc_grp.slab.release();
+    m->dec_grp.slab.release();
     return MMI_OK;
 }
 
 // A file is a stream that nobody else sees.  Starting and stopping one took 350 us - 32 MB allocated, zeroed and freed, two launch lists built,
 // captured and dropped - where 8 frames take the GPU some 250; so what it has built stays for the next file of as many streams, which resets the
-// state instead.  At most MIMI_PARK bytes stay (the full-size codec: three streams), until a stream of the caller's own starts, a file of
-// another number of streams or codebooks, or the handle goes.
+// state instead.  At most MIMI_PARK bytes of state stay (the full-size codec: three streams), and the groups' slabs as behind every stream: until a
+// stream of the caller's own starts, a file of another number of streams or codebooks, an allocation finds no memory, or the handle goes.
 constexpr size_t MIMI_PARK = (size_t)128 << 20;
 
 extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
-    if (!m || !m->parked || m->batch != batch || m->parked_k != m->n_codebooks) return mmi_mimi_streaming_start(m, batch, stream);
+    if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
+    OutOfIdle out(m);
+    if (!m->parked || m->batch != batch || m->parked_k != m->n_codebooks) return start_any_stream(m, batch, stream);
     // (a stream cannot start there either: it waits for its own state)
     if (recording((hipStream_t)stream)) return mmi_fail(MMI_ERR_HIP, "a file's stream cannot start while its HIP stream is being captured");
     int rc = finish_parked(m);
@@ -1645,7 +1701,7 @@ extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream
         g->earlier = true;
     }
     rc = mmi_mimi_reset(m, nullptr, stream);
-    if (rc) mmi_mimi_streaming_stop(m);
+    if (rc) stop_stream(m);
     return rc;
 }
 
@@ -1653,6 +1709,7 @@ extern "C" int mmi_mimi_file_stop(mmi_mimi* m) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
     if (!m->streaming) return MMI_OK;
+    OutOfIdle out(m);
     m->streaming = false;
     m->parked = true;
     m->parked_k = m->n_codebooks;

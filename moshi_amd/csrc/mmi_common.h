@@ -85,9 +85,11 @@ struct MmiWeights {
 };
 
 // hipMalloc and hipFree (api_common.hip).  The runtime does neither while another thread captures in the global mode: what mmi_free could not free
-// stays in a list of the process, and goes with the next call of either.
+// stays in a list of the process, and goes with the next call of either.  Where a device has no memory left, mmi_malloc tries again behind
+// `let_go` (mmi_set_let_go): what handles of the process keep there for later is worth less than what is asked for.
 hipError_t mmi_malloc(void** p, size_t bytes);
 void mmi_free(void* p);
+void mmi_set_let_go(bool (*let_go)(int device));           // false: there was nothing
 
 // device allocation bookkeeping: every engine frees what it allocated
 // chunk > 0: allocations up to an eighth of it are cut out of pieces of that size, zeroed when they are made, instead of each being one of

@@ -353,6 +353,65 @@ def test_a_file_whose_wait_fails(sim_lib):
     assert sim_bytes(sim_lib) == empty
 
 
+def test_what_a_file_leaves_goes_where_memory_is_short(sim_lib):
+    """The state and the groups' buffers that a file has left go when an allocation finds no memory - another handle's stream, its groups, a new
+    handle - and when they are asked to (a stop while not streaming).  The handle's next file is what it was, and nothing goes from one that streams."""
+    cfg = replace(tiny_mimi_config(), n_filters=4, ratios=[4, 4, 3, 2], sample_rate=96 * 25)
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    set_memory, fs = sim_lib.cdll.hipsim_set_memory, cfg.frame_size
+    set_memory.argtypes = [ctypes.c_ulonglong]
+    x = 0.3 * torch.randn(1, 1, 9 * fs, generator=torch.Generator().manual_seed(4))
+    gc.collect()
+    empty = sim_bytes(sim_lib)
+    a, b = (MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib) for _ in range(2))
+    handle = (sim_bytes(sim_lib) - empty) // 2
+    before = sim_bytes(sim_lib)
+    codes = b.encode(x)
+    pcm = b.decode(codes)
+    all_of_it = sim_bytes(sim_lib) - before
+    with b.streaming(1):
+        b.encode(x[..., :fs].contiguous()), b.decode(codes[..., :1].contiguous())      # single frames: the groups' buffers go
+        stream = sim_bytes(sim_lib) - before
+    assert sim_bytes(sim_lib) == before and stream < all_of_it
+
+    def leave():
+        assert torch.equal(a.encode(x), codes) and torch.equal(a.decode(codes), pcm)
+        assert sim_bytes(sim_lib) - before == all_of_it
+    try:
+        leave()
+        set_memory(before + all_of_it)
+        with b.streaming(1):                                   # its state: what a has left goes
+            assert sim_bytes(sim_lib) - before == stream
+        set_memory(0)
+        leave()
+        with b.streaming(1):
+            set_memory(before + all_of_it + stream)
+            assert torch.equal(b.encode(x), codes)             # its group: the same
+            assert "k_mimi_group_rope" in {k for _, k in b.launch_list("encode_group")}
+            assert sim_bytes(sim_lib) - before < all_of_it + stream
+            set_memory(sim_bytes(sim_lib))
+            with pytest.raises(RuntimeError):                  # a stream keeps what it has
+                a.encode(x)
+            assert torch.equal(b.decode(codes), pcm)
+        set_memory(0)
+        assert torch.equal(b.encode(x[..., :fs].contiguous()), codes[..., :1])
+        leave_b = sim_bytes(sim_lib) - before
+        set_memory(before + leave_b + handle - 1)
+        c = MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+        assert sim_bytes(sim_lib) == before + handle
+        set_memory(0)
+        assert torch.equal(c.encode(x), codes) and torch.equal(b.encode(x), codes)
+        for m in (b, c):
+            sim_lib.check(sim_lib.mmi_mimi_streaming_stop(m._handle))
+        assert sim_bytes(sim_lib) == before + handle
+    finally:
+        set_memory(0)
+    assert torch.equal(a.encode(x), codes) and torch.equal(c.decode(codes), pcm)
+    del a, b, c, m
+    gc.collect()
+    assert sim_bytes(sim_lib) == empty
+
+
 def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
     """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
     stream it is called on, and leaves the one that the snapshot came from alone."""
