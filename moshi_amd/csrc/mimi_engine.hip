@@ -1683,6 +1683,23 @@ extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
 // stream of the caller's own starts, a file of another number of streams or codebooks, an allocation finds no memory, or the handle goes.
 constexpr size_t MIMI_PARK = (size_t)128 << 20;
 
+// MMI_DEBUG_POISON=1: what the next file may not see - the rings, the buffers with histories, the overlap-adds' partial rows, offsets and flags - is
+// NaNs and -1 in front of its reset, whatever the last file has left there.
+static int poison_parked(mmi_mimi* m, hipStream_t s) {
+    const char* pz = getenv("MMI_DEBUG_POISON");
+    if (!pz || pz[0] != '1') return MMI_OK;
+    std::vector<const void*> places = {m->enc_kv, m->dec_kv, m->counters, m->first, m->exec};
+    places.insert(places.end(), m->partials.begin(), m->partials.end());
+    for (const HistTable* t : {&m->enc_tab, &m->dec_tab})
+        for (int i = 0; i < t->n; ++i) places.push_back(t->d[i].p);
+    for (size_t i = 0; i < m->st.ptrs.size(); ++i) {
+        const char* at = (const char*)m->st.ptrs[i];
+        if (std::any_of(places.begin(), places.end(), [&](const void* p) { return (const char*)p >= at && (const char*)p < at + m->st.sizes[i]; }))
+            MMI_HIP_CHECK(hipMemsetAsync(m->st.ptrs[i], 0xFF, m->st.sizes[i], s));
+    }
+    return MMI_OK;
+}
+
 extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream) {
     MmiDeviceGuard dev_guard_(m ? m->device : -1);
     if (!m) return mmi_fail(MMI_ERR_INVALID, "null handle");
@@ -1700,7 +1717,8 @@ extern "C" int mmi_mimi_file_start(mmi_mimi* m, int32_t batch, mmi_stream stream
         g->refused = false;
         g->earlier = true;
     }
-    rc = mmi_mimi_reset(m, nullptr, stream);
+    rc = poison_parked(m, (hipStream_t)stream);
+    if (!rc) rc = mmi_mimi_reset(m, nullptr, stream);
     if (rc) stop_stream(m);
     return rc;
 }
@@ -1715,7 +1733,7 @@ extern "C" int mmi_mimi_file_stop(mmi_mimi* m) {
     m->parked_k = m->n_codebooks;
     m->unfinished = true;
     int rc = finish_parked(m);                             // (where it fails nothing goes: work on the device may use it)
-    if (!rc && (m->st.held() > MIMI_PARK || getenv("MMI_DEBUG_POISON"))) drop_parked(m);
+    if (!rc && m->st.held() > MIMI_PARK) drop_parked(m);
     return rc;
 }
 

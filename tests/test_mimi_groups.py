@@ -238,8 +238,9 @@ def check_files_in_a_row(make, device, cfg, lengths, K=4):
             assert torch.equal(got, want) or (torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()))
     for n in lengths:
         same(*file(1, n))
-    for bad in (float("nan"), float("inf")):
-        same(*file(1, lengths[0], bad=bad)), same(*file(1, lengths[0]))
+    for bad in (float("nan"), float("inf")):                   # (the longest goes round the ring; behind it a file that is as long, shorter ones, one frame)
+        for n in (max(lengths), lengths[0] - 1, 1, max(lengths)):
+            same(*file(1, max(lengths), bad=bad)), same(*file(1, n))
     same(*file(2, 3)), same(*file(2, 3)), same(*file(1, lengths[0]))
     x, q = file(1, 3)
     with m.streaming(1):
@@ -252,12 +253,25 @@ def check_files_in_a_row(make, device, cfg, lengths, K=4):
     same(x, q[:, :2])
 
 
-def test_files_in_a_row(sim_lib):
-    check_files_in_a_row(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", tiny_mimi_config(), (4, 1, 4, 6))
+# (poison: what a file may not see of the one before it is NaNs in front of its reset, in the decoder too, whose inputs are always finite)
+@pytest.mark.parametrize("poison", [False, True])
+def test_files_in_a_row(sim_lib, monkeypatch, poison):
+    if poison:
+        monkeypatch.setenv("MMI_DEBUG_POISON", "1")
+    cfg = tiny_mimi_config()
+    m = MimiModel(random_mimi_state_dict(cfg, seed=5, device="cpu"), cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib)
+    before = sim_bytes(sim_lib)
+    m.encode(torch.zeros(1, 1, cfg.frame_size))
+    assert sim_bytes(sim_lib) > before                         # (something is kept)
+    assert 2 * 14 > cfg.tr_context
+    check_files_in_a_row(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cpu", max_batch=mb, num_codebooks=K, lib=sim_lib), "cpu", cfg, (4, 1, 4, 14))
 
 
 @pytest.mark.gpu
-def test_full_size_files_in_a_row():
+@pytest.mark.parametrize("poison", [False, True])
+def test_full_size_files_in_a_row(monkeypatch, poison):
+    if poison:
+        monkeypatch.setenv("MMI_DEBUG_POISON", "1")
     check_files_in_a_row(lambda sd, cfg, K, mb: MimiModel(sd, cfg, device="cuda", max_batch=mb, num_codebooks=K), "cuda", MimiConfig(), (40, 1, 40, 170, 9), K=8)
 
 
