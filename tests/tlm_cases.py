@@ -2,6 +2,7 @@
 against the plain oracle (oracle/token_lm_oracle.py) on small random networks of this file's own sizes."""
 from __future__ import annotations
 
+import math
 from dataclasses import replace
 
 import numpy as np
@@ -150,13 +151,16 @@ def check_mechanism(name, dev, lib, dtype=F32, n=90):
     assert lm.free_pages == lm.total_pages and lm.free_slots == 6
 
 
-def check_activation_branches(dev, lib):
+def check_activation_branches(dev, lib, far=False):
     """Both branches of the candidate (u >= 0 and u < 0), gates near 0 and near 1, inputs of squared ReLU on both sides of zero: biases
-    push whole channels to each side."""
+    push whole channels to each side.  far: to where sigmoids underflow, to their clamps and to the infinities."""
     cfg = MECHANISMS["mingru_experts"]
     sd = random_token_lm_state_dict(cfg, seed=9)
     sd["l0.mix.x.b"] = torch.linspace(-6, 6, 16).to(BF16)
     sd["l0.mix.z.b"] = torch.linspace(5, -5, 16).to(BF16)
+    if far:
+        ends = torch.tensor([-math.inf, -3e38, -200., -105., -104., -100., -89., -88.5, -88., -87., -50., -20., 20., 88., 200., math.inf])
+        sd["l0.mix.x.b"], sd["l0.mix.z.b"] = ends.clamp(max=6.).roll(5).to(BF16), ends.to(BF16)
     lm = TokenLM(sd, cfg, device=dev, dtype=F32, lib=lib, max_slots=2, max_tokens=256)
     toks = tokens_of(cfg, 70)
     assert rel(run_cut(lm, toks, [70]), TokenLMOracle(sd, cfg).logits(toks)) < TOL[F32]
