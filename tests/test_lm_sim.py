@@ -110,10 +110,51 @@ def test_attention_ring_split_over_several_workgroups(sim_lib, monkeypatch, kern
 
 @pytest.mark.parametrize("context", [300, 16 * 256, 16 * 256 + 1, 18 * 256])
 def test_merge_of_few_and_many_partials(sim_lib, monkeypatch, context):
-    """k_lm_attn_combine around the 16 partials that it requests together (2, 16, 17, 18); most are empty here, with a maximum of -inf."""
+    """k_lm_attn_combine around the 16 partials that it requests together (2, 16, 17, 18); most are empty here, with a maximum of -inf (full ones:
+    test_merge_of_partials)."""
     from dataclasses import replace
     monkeypatch.setenv("MMI_ATTN_SOLO", "0")
     lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), context=context), seed=62, B=1, S=4)
+
+
+@pytest.fixture(scope="module")
+def combine(tmp_path_factory):
+    import ctypes
+    import subprocess
+    import sys
+    from pathlib import Path
+    here = Path(__file__).resolve().parent / "hipsim"
+    sys.path.insert(0, str(here))
+    import build_sim
+    so = tmp_path_factory.mktemp("combine") / "combine_selftest.so"
+    subprocess.check_call([build_sim._cxx(), "-O1", "-w", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", f"-I{here}", f"-I{build_sim.CSRC}",
+                           str(here / "combine_selftest.cpp"), str(here / "hipsim.cpp"), "-o", str(so)])
+    return ctypes.CDLL(str(so))
+
+
+@pytest.mark.parametrize("top", ["first", "last"])
+@pytest.mark.parametrize("NS", [1, 2, 15, 16, 17, 20, 33])
+@pytest.mark.parametrize("B,H,Dh", [(1, 3, 128), (17, 2, 24)])
+def test_merge_of_partials(combine, NS, B, H, Dh, top):
+    """k_lm_attn_combine requests 16 partials together and walks over the others: all of them full but for a few that are empty (a maximum of -inf,
+    nothing written), the largest maximum in the first or in the last one.  One rounding to bf16, and fp32 sums of NS terms."""
+    import ctypes
+    import torch
+    g = torch.Generator().manual_seed(NS)
+    ml = torch.stack([4 * torch.randn(B, H, NS, generator=g), 0.5 + torch.rand(B, H, NS, generator=g)], -1)
+    part = torch.randn(B, H, NS, Dh, generator=g) * ml[..., 1:]
+    ml[:, :, 0 if top == "first" else NS - 1, 0] = 15.0
+    if NS > 2:
+        for c in (1, NS // 2, NS - 2):
+            ml[0, :, c], part[0, :, c] = torch.tensor([-float("inf"), float("nan")]), float("nan")
+    out = torch.empty(B, H * Dh)
+    combine.combine_selftest_run(*(ctypes.c_void_p(t.data_ptr()) if torch.is_tensor(t) else t for t in (ml, part, B, H, Dh, NS, out)))
+    w = torch.exp(ml[..., 0].double() - ml[..., 0].double().amax(-1, keepdim=True))
+    num = torch.where(w[..., None] > 0, w[..., None] * part.double(), 0.0)
+    den = torch.where(w > 0, w * ml[..., 1].double(), 0.0).sum(-1, keepdim=True)
+    want = num.sum(2) / den
+    size = num.abs().sum(2) / den                              # (what fp32 rounds)
+    assert ((out.view(B, H, Dh).double() - want).abs() <= 2.0 ** -8 * want.abs() + (NS + 8) * 2.0 ** -23 * size).all()
 
 
 def test_depformer_attention_inside_out_proj_for_one_session(sim_lib, monkeypatch):
