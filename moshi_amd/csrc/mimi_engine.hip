@@ -119,7 +119,7 @@ struct DequantScratch {
 // columns, so that a launch is worth its latency.  The streaming state stays where the frame program keeps it: the histories are copied
 // in front of the group's rows before its launches and back behind them, everything else is shared.
 // Measured on one stream, 129 frames encoded and decoded (10.3 s of audio): 140 ms frame by frame (176 dependent launches per frame, most of
-// them at the ~4.7 us a dependent launch costs; 136 launches and 90 ms now), 3.7 ms in one group of 129, both with the stream's start and stop.
+// them at the ~4.7 us a dependent launch costs; 136 launches and 90 ms now), 2.9 ms in one group of 129.
 struct MimiGroup {
     int frames = 0;                            // 0: not built (for this stream)
     bool earlier = false;                      // built for an earlier file, and not used by this one yet
@@ -1677,10 +1677,12 @@ extern "C" int mmi_mimi_streaming_stop(mmi_mimi* m) {
     return MMI_OK;
 }
 
-// A file is a stream that nobody else sees.  Starting and stopping one took 350 us - 32 MB allocated, zeroed and freed, two launch lists built,
-// captured and dropped - where 8 frames take the GPU some 250; so what it has built stays for the next file of as many streams, which resets the
-// state instead.  At most MIMI_PARK bytes of state stay (the full-size codec: three streams), and the groups' slabs as behind every stream: until a
+// A file is a stream that nobody else sees.  Starting and stopping one takes some 400 us - 32 MB allocated, zeroed and freed, two launch lists built,
+// captured and dropped - where 8 frames take the GPU 250; so what it has built stays for the next file of as many streams, which resets the
+// state instead.  At most MIMI_PARK bytes of state stay (the full-size codec: four streams), and the groups' slabs as behind every stream: until a
 // stream of the caller's own starts, a file of another number of streams or codebooks, an allocation finds no memory, or the handle goes.
+// 8 frames of 1, 2, 3, 4 streams encoded and decoded, us: 1755, 1859, 2658, 3318 with a stream's start and stop each, 973, 1085, 1270, 1323 so.
+// (More streams would gain as much, 4312 -> 1581 for five, but for memory, 40 MB a stream, that the process's other allocators cannot ask back.)
 constexpr size_t MIMI_PARK = (size_t)128 << 20;
 
 // MMI_DEBUG_POISON=1: what the next file may not see - the rings, the buffers with histories, the overlap-adds' partial rows, offsets and flags - is

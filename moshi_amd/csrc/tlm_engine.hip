@@ -891,11 +891,12 @@ Form bf16_form(const Plan& p, TlmJobs& J) {
 }
 
 // ---- which launches take k_tlm_gemm_wide, in blocks of which height, with which splits ----
-// What launches take, in us, by their blocks and k-steps: fitted to 120 launches of the two kernels (65 - 2048 rows, widths 2048 and 4096, weights from
-// HBM), which it meets within 5 and 7 % (rms).  The narrower forms: so many blocks to a CU, a k-step of 1 .. that many of them, the rest of a block.
-struct FormTime { int ntw, places; float fixed, step[4]; };
-const FormTime form_times[] = {{16, 2, 12.f, {0.66f, 0.88f}},        {8, 2, 8.f, {0.34f, 0.54f}}, {8, 3, 8.f, {0.50f, 0.66f, 0.82f}},
-                               {8, 3, 6.f, {0.40f, 0.45f, 0.55f}}, {4, 2, 6.f, {0.165f, 0.25f}}, {4, 4, 6.f, {0.25f, 0.28f, 0.37f, 0.50f}}};
+// What launches take, in us, by their blocks and k-steps; fitted to launches of 65 - 2048 rows at widths 2048 and 4096, weights from HBM.  The narrower
+// forms: so many blocks to a CU, a k-step of 1 .. that many of them, the rest of a block.  What the choice gives at those widths and at five
+// others, 17 lengths each: profiles/workloads/wide_products.txt (prompts 21 % faster to as fast; the slowest one + 0.7 %, as two runs differ).
+struct FormTime { int places; float fixed, step[4]; };
+const FormTime form_times[] = {{2, 12.f, {0.66f, 0.88f}},       {2, 8.f, {0.34f, 0.54f}},  {3, 8.f, {0.50f, 0.66f, 0.82f}},         // (in the order of Form)
+                               {3, 6.f, {0.40f, 0.45f, 0.55f}}, {2, 6.f, {0.165f, 0.25f}}, {4, 6.f, {0.25f, 0.28f, 0.37f, 0.50f}}};
 float narrow_time(Form form, const TlmJobs& J) {
     const FormTime& f = form_times[form];
     int longest = 0;

@@ -71,27 +71,26 @@ __device__ __forceinline__ auto& tlm_quad(F* base, int at) {
     return *reinterpret_cast<E*>(reinterpret_cast<C*>(base) + 4u * (unsigned)at);
 }
 
-// channel(s) from c of the convolution at token t of a sequence whose rows start at row0 of the projection; four taps are requested at a
-// time (a tap before the sequence's start reads some valid address and counts as zero).  `now`: where the taps - 1 inputs that the next
-// step's first token needs stay, or null
-template <class T>
-__device__ __forceinline__ T tlm_conv(const TlmLinArgs& a, const float* old, int fresh, int row0, int t, int c, float* now) {
-    T s = T{};
+// channel c of the convolution at token t of a sequence whose rows start at row0 of the projection; four taps are requested at a time (a tap before
+// the sequence's start reads some valid address and counts as zero).  `now`: where the taps - 1 inputs that the next step's first token needs
+// stay, or null
+__device__ __forceinline__ float tlm_conv(const TlmLinArgs& a, const float* old, int fresh, int row0, int t, int c, float* now) {
+    float s = 0.f;
     for (int j0 = 0; j0 < a.taps; j0 += 4) {
-        T x[4], w[4];
+        float x[4], w[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int tap = min(j0 + j, a.taps - 1), at = t - (a.taps - 1) + tap;
-            x[j] = *reinterpret_cast<const T*>(at >= 0 || fresh ? a.in + (long)(row0 + max(at, 0)) * a.in_ld + c : old + (long)(a.taps - 1 + at) * a.conv_c + c);
-            w[j] = *reinterpret_cast<const T*>(a.conv_w + (long)tap * a.conv_c + c);
-            if (j0 + j >= a.taps || (at < 0 && fresh)) x[j] = T{};
+            x[j] = *(at >= 0 || fresh ? a.in + (long)(row0 + max(at, 0)) * a.in_ld + c : old + (long)(a.taps - 1 + at) * a.conv_c + c);
+            w[j] = a.conv_w[(long)tap * a.conv_c + c];
+            if (j0 + j >= a.taps || (at < 0 && fresh)) x[j] = 0.f;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) s += w[j] * x[j];
         if (now)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (j0 + j >= 1 && j0 + j < a.taps) *reinterpret_cast<T*>(now + (long)(j0 + j - 1) * a.conv_c + c) = x[j];
+                if (j0 + j >= 1 && j0 + j < a.taps) now[(long)(j0 + j - 1) * a.conv_c + c] = x[j];
     }
     return s;
 }
@@ -146,7 +145,7 @@ __device__ __forceinline__ void tlm_state_step(const TlmLinArgs& a, float* sh, i
             }
             const int c = i < D ? a.q0 + kh * D + i : (i < 2 * D ? a.k0 + kh * D + i - D : a.v0 + h * V + i - 2 * D);
             float x;
-            if constexpr (DELTA) x = tlm_silu(tlm_conv<float>(a, old, un.fresh, un.row0, t, c, t + 1 == un.n && (i >= 2 * D || h % rep == 0) ? now : nullptr));      // (the heads of a group share query and key channels)
+            if constexpr (DELTA) x = tlm_silu(tlm_conv(a, old, un.fresh, un.row0, t, c, t + 1 == un.n && (i >= 2 * D || h % rep == 0) ? now : nullptr));      // (the heads of a group share query and key channels)
             else x = in[c];
             if (i < D) q[i] = x;
             else if (i < 2 * D) k[i - D] = x;
@@ -228,8 +227,8 @@ __global__ __launch_bounds__(MAXB, MAXB == 512 && !DELTA ? 5 : 4) void k_tlm_sta
 // ------------------------------------------------------------------------------------------------
 // chunks: convolutions and unit norms (delta).  grid: chunks, 2 kv_heads + heads, shares of a chunk; a lane takes 4 channels of 4 tokens in a row, which share
 // seven inputs per four taps; a power of two of lanes stand side by side.  Bound by its bytes with many chunks, by two trips to memory with few,
-// so a workgroup goes round once.  1773 tokens, 32 heads of 128 x 128 (174 MB): 42.7 us with a token per lane, 37.6 now; 662 tokens of 16 heads 16.0
-// and 11.8 (going round twice 13.4); 200 tokens of 8 heads 11.5 and 7.1
+// so a workgroup goes round once.  In a prompt's step, heads of 128 x 128, with a token per lane and now: 1773 tokens of 32 heads (174 MB) 54.0 and 42.6 us,
+// 639 of 16 15.8 and 12.9
 // ------------------------------------------------------------------------------------------------
 inline __global__ __launch_bounds__(256, 4) void k_tlm_conv(TlmLinArgs a, int kgroups, int vgroups) {
     const int y = (int)blockIdx.y;
@@ -359,8 +358,8 @@ __global__ __launch_bounds__(512, 4) void k_tlm_chunk_lightning(TlmLinArgs a, in
 
 // ------------------------------------------------------------------------------------------------
 // chunks, delta: P, W, U0, the decayed queries and transposed keys.  grid: chunks, heads; NP: panels of 64 channels, 1, 2 or 4
-// Its bytes bound it where chunks are many (896 of 128 x 128: 250 MB, 65 us = 3.8 TB/s; 113 before), the chain of one workgroup's phases where
-// they are few (192: 23 us; 47 before).  So: eight waves, two on every SIMD and two workgroups on a CU while the registers (126) allow it; the
+// Its bytes bound it where chunks are many (896 of 128 x 128: 250 MB, 67 us in a step = 3.7 TB/s; 127 before), the chain of one workgroup's phases
+// where they are few (176: 23 us; 47 before).  So: eight waves, two on every SIMD and two workgroups on a CU while the registers (126) allow it; the
 // next panel's operands and U0's are asked for a phase ahead; pairs are taken one by one only inside 8 tokens (half the vector work of 16), all
 // others by the matrix core; no right side goes through memory: W's stay in the registers of the wave that solves for them.
 // ------------------------------------------------------------------------------------------------
@@ -707,8 +706,9 @@ __global__ __launch_bounds__(512, NP <= 2 ? 4 : 2) void k_tlm_chunk_delta(TlmLin
 // and a quarter of the rows of S, in the layout the matrix core leaves them in, which is also the layout it takes them as an operand; S and
 // U go round through LDS.  A chunk is 112 matrix instructions of 32 cycles per SIMD and asks a CU for 116 KB: requests in one burst kept the
 // waves from issuing for 2400 of 7500 cycles, so they stand between the products, a phase or more before their use, and what follows an exchange
-// through LDS does not need it (Q S, P U).  One sequence of 1773 tokens, 32 heads of 128 x 128: 98 us before, 77 now (5200 cycles per chunk; with all
-// of it in the L2 no less: what is left is the distance of dependent instructions in one wave per SIMD); 331 tokens 24.6 and 20.0.
+// through LDS does not need it (Q S, P U).  One sequence of 1773 tokens, 32 heads of 128 x 128: 107 us in a step
+// before, 78 now (5200 cycles per chunk; with all of it in the L2 no less: what is left is the distance of dependent instructions in one wave
+// per SIMD); two of 331 and 294 tokens, 16 heads: 24.2 and 19.8.
 // grid: 8 x ceil(sequences x heads / 8) x vdim_p / 16, the column blocks of one head on one XCD (they read the same W, Qg, Kt, P)
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float tlm_f(unsigned v) { return __builtin_bit_cast(float, v); }
