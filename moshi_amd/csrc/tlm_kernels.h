@@ -52,7 +52,7 @@ MMI_HD long tlm_index(long row, int k, int ks) {
 
 constexpr int TLM_PAGE = 64;         // tokens per cache page
 
-// 1 / (1 + e^-x) in about half the instructions of expf and a division, as good as theirs (largest error 2.6 ulp, rms 0.49): 2^-(x log2 e) with the
+// 1 / (1 + e^-x) in about half the instructions of expf and a division, as good as theirs (largest error of 20 million 2.6 ulp): 2^-(x log2 e) with the
 // product's low part carried along, the reciprocal with one Newton step.  Of e^-x = e 2^n the sum is formed as 2^-n + e where n > 0, so that the
 // reciprocal is a normal number (the instruction would flush another one) and results below 2^-126 are rounded like the others.  0 and 1 at
 // the infinities, NaN where x is
