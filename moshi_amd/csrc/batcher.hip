@@ -119,10 +119,10 @@ void release(mmi_batcher* b) {
     }
     if (b->host.up) hipHostFree(b->host.up);
     if (b->host.down) hipHostFree(b->host.down);
-    if (b->dev.up) hipFree(b->dev.up);
-    if (b->dev.down) hipFree(b->dev.down);
-    if (b->d_codes) hipFree(b->d_codes);
-    if (b->d_dec_codes) hipFree(b->d_dec_codes);
+    mmi_free(b->dev.up);
+    mmi_free(b->dev.down);
+    mmi_free(b->d_codes);
+    mmi_free(b->d_dec_codes);
     if (b->ev_begin) hipEventDestroy(b->ev_begin);
     if (b->ev_end) hipEventDestroy(b->ev_end);
     if (b->stream) hipStreamDestroy(b->stream);
@@ -155,17 +155,17 @@ int create_impl(mmi_batcher* b) {
     b->host.up = hu;
     MMI_HIP_CHECK(hipHostMalloc((void**)&hd, probe.d2h_bytes, 0));
     b->host.down = hd;
-    MMI_HIP_CHECK(hipMalloc((void**)&du, probe.h2d_bytes));
+    MMI_HIP_CHECK(mmi_malloc((void**)&du, probe.h2d_bytes));
     b->dev.up = du;
-    MMI_HIP_CHECK(hipMalloc((void**)&dd, probe.d2h_bytes));
+    MMI_HIP_CHECK(mmi_malloc((void**)&dd, probe.d2h_bytes));
     b->dev.down = dd;
     carve(&b->host, hu, hd, B, b->F, b->NTOK);
     carve(&b->dev, du, dd, B, b->F, b->NTOK);
     MMI_HIP_CHECK(hipMemset(dd, 0, probe.d2h_bytes));   // rows (or, for an ASR model, the whole PCM block) nobody writes read as zero
     memset(hu, 0, probe.h2d_bytes);
     memset(hd, 0, probe.d2h_bytes);
-    MMI_HIP_CHECK(hipMalloc((void**)&b->d_codes, (size_t)B * b->K * sizeof(int64_t)));
-    MMI_HIP_CHECK(hipMalloc((void**)&b->d_dec_codes, (size_t)B * (b->dep_q > 0 ? b->dep_q : 1) * sizeof(int64_t)));
+    MMI_HIP_CHECK(mmi_malloc((void**)&b->d_codes, (size_t)B * b->K * sizeof(int64_t)));
+    MMI_HIP_CHECK(mmi_malloc((void**)&b->d_dec_codes, (size_t)B * (b->dep_q > 0 ? b->dep_q : 1) * sizeof(int64_t)));
     // streaming_forever(batch) on both models (server.py:59-60)
     if ((rc = mmi_mimi_streaming_start(b->mimi, B, b->stream))) return rc;
     b->models_streaming = true;

@@ -139,15 +139,15 @@ void release(mmi_duplex* d) {
     for (int i = 0; i < 2; ++i) {
         if (d->ev_lm[i]) hipEventDestroy(d->ev_lm[i]);
         if (d->ev_phase[i]) hipEventDestroy(d->ev_phase[i]);
-        if (d->codes[i]) hipFree(d->codes[i]);
+        mmi_free(d->codes[i]);
     }
     for (int i = 0; i < 3; ++i) {
         if (d->ev_dec[i]) hipEventDestroy(d->ev_dec[i]);
-        if (d->tokens[i]) hipFree(d->tokens[i]);
+        mmi_free(d->tokens[i]);
     }
-    for (float* p : d->pcm_in) if (p) hipFree(p);
-    if (d->flags) hipFree(d->flags);
-    if (d->stamps) hipFree(d->stamps);
+    for (float* p : d->pcm_in) mmi_free(p);
+    mmi_free(d->flags);
+    mmi_free(d->stamps);
     for (hipEvent_t e : d->tl) if (e) hipEventDestroy(e);
     delete d;
 }
@@ -171,7 +171,7 @@ int create_impl(mmi_duplex* d) {
     if (mc.q_bins != lc.card) return mmi_fail(MMI_ERR_SHAPE, "codec cardinality != LM card");
     // All three streams have the default priority (streams of different priorities in one process have hung on this stack); created
     // back to back, they land on different hardware queues of the pool of GPU_MAX_HW_QUEUES (4).
-    MMI_HIP_CHECK(hipMalloc((void**)&d->flags, (size_t)F_COUNT * 16 * sizeof(long)));
+    MMI_HIP_CHECK(mmi_malloc((void**)&d->flags, (size_t)F_COUNT * 16 * sizeof(long)));
     MMI_HIP_CHECK(hipMemset(d->flags, 0, (size_t)F_COUNT * 16 * sizeof(long)));
     // MMI_DUPLEX_CODEC_CUS=n (experiment): the codec streams confined to n of the CUs (a CU mask of n bits, which the driver
     // deals out over the XCDs), so that the depth transformer's launches - 96..176 workgroups that need a whole CU's wave slots each -
@@ -191,13 +191,13 @@ int create_impl(mmi_duplex* d) {
     for (int i = 0; i < 2; ++i) {
         MMI_HIP_CHECK(hipEventCreateWithFlags(&d->ev_lm[i], hipEventDisableTiming));
         MMI_HIP_CHECK(hipEventCreateWithFlags(&d->ev_phase[i], hipEventDisableTiming));
-        MMI_HIP_CHECK(hipMalloc((void**)&d->codes[i], (size_t)d->B * d->K * sizeof(int64_t)));
+        MMI_HIP_CHECK(mmi_malloc((void**)&d->codes[i], (size_t)d->B * d->K * sizeof(int64_t)));
     }
     for (int i = 0; i < 3; ++i) {
         MMI_HIP_CHECK(hipEventCreateWithFlags(&d->ev_dec[i], hipEventDisableTiming));
-        MMI_HIP_CHECK(hipMalloc((void**)&d->tokens[i], (size_t)d->B * d->NTOK * sizeof(int64_t)));
+        MMI_HIP_CHECK(mmi_malloc((void**)&d->tokens[i], (size_t)d->B * d->NTOK * sizeof(int64_t)));
     }
-    for (int i = 0; i < d->in_slots; ++i) MMI_HIP_CHECK(hipMalloc((void**)&d->pcm_in[i], (size_t)d->B * d->F * sizeof(float)));
+    for (int i = 0; i < d->in_slots; ++i) MMI_HIP_CHECK(mmi_malloc((void**)&d->pcm_in[i], (size_t)d->B * d->F * sizeof(float)));
     return MMI_OK;
 }
 
@@ -356,7 +356,7 @@ extern "C" int mmi_duplex_set_timeline(mmi_duplex* d, int32_t on) {
     if (on && !d->tl[0])
         for (hipEvent_t& e : d->tl) MMI_HIP_CHECK(hipEventCreate(&e));
     if (on && !d->stamps) {
-        MMI_HIP_CHECK(hipMalloc((void**)&d->stamps, (size_t)4 * S_COUNT * sizeof(long)));
+        MMI_HIP_CHECK(mmi_malloc((void**)&d->stamps, (size_t)4 * S_COUNT * sizeof(long)));
         MMI_HIP_CHECK(hipMemset(d->stamps, 0, (size_t)4 * S_COUNT * sizeof(long)));
     }
     d->timeline = on != 0;

@@ -1591,7 +1591,7 @@ extern "C" int mmi_lm_streaming_start_guided(mmi_lm* lm, int32_t batch, const mm
         lm->trace_file = fopen(lm->trace_name.c_str(), "w");
         lm->trace_prev.assign(lm->st.ptrs.size(), 0ull);
         lm->trace_step = 0;
-        if (lm->trace_file && hipMalloc((void**)&lm->trace_dev, lm->st.ptrs.size() * sizeof(unsigned long long)) != hipSuccess) {
+        if (lm->trace_file && mmi_malloc((void**)&lm->trace_dev, lm->st.ptrs.size() * sizeof(unsigned long long)) != hipSuccess) {
             fclose(lm->trace_file);
             lm->trace_file = nullptr;
         }
@@ -1606,7 +1606,8 @@ extern "C" int mmi_lm_streaming_stop(mmi_lm* lm) {
     if (!lm->streaming) return MMI_OK;
     hipDeviceSynchronize();
     if (lm->trace_file) { fclose(lm->trace_file); lm->trace_file = nullptr; }
-    if (lm->trace_dev) { hipFree(lm->trace_dev); lm->trace_dev = nullptr; }
+    mmi_free(lm->trace_dev);
+    lm->trace_dev = nullptr;
     lm->prog.clear();
     lm->st.release();
     lm->streaming = false;

@@ -320,12 +320,12 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
     if (wf->shape[0] != D || wf->shape[1] != dim || of->shape[0] != dim || of->shape[1] != D)
         return mmi_fail(MMI_ERR_SHAPE, "RVQ projection shape mismatch");
     float* tmp = nullptr;
-    MMI_HIP_CHECK(hipMalloc((void**)&tmp, (size_t)2 * D * dim * sizeof(float)));
+    MMI_HIP_CHECK(mmi_malloc((void**)&tmp, (size_t)2 * D * dim * sizeof(float)));
     MMI_HIP_CHECK(hipMemcpy(tmp, wf->data, (size_t)D * dim * sizeof(float), hipMemcpyDeviceToDevice));
     MMI_HIP_CHECK(hipMemcpy(tmp + (size_t)D * dim, wr->data, (size_t)D * dim * sizeof(float), hipMemcpyDeviceToDevice));
     m->q_in.Cin = dim; m->q_in.Cout = 2 * D; m->q_in.K = 1; m->q_in.S = 1;
     rc = pack_matrix(m, tmp, 2 * D, dim, dim, 1, &m->q_in);
-    if (rc) { hipFree(tmp); return rc; }
+    if (rc) { mmi_free(tmp); return rc; }
     MMI_HIP_CHECK(hipDeviceSynchronize());
     // stacked output projection [dim][2D]: columns 0..D-1 = first, D..2D-1 = rest
     int blocks = mmi_cdiv(dim * D, 256);
@@ -335,7 +335,7 @@ int load_rvq(mmi_mimi* m, const MmiWeights& W) {
     m->q_out.Cin = 2 * D; m->q_out.Cout = dim; m->q_out.K = 1; m->q_out.S = 1;
     rc = pack_matrix(m, tmp, dim, 2 * D, 2 * D, 1, &m->q_out);
     MMI_HIP_CHECK(hipDeviceSynchronize());
-    hipFree(tmp);
+    mmi_free(tmp);
     if (rc) return rc;
 
     MMI_HIP_CHECK(m->wts.alloc(&m->E_all, (size_t)nq * bins * D));

@@ -426,6 +426,47 @@ def test_what_a_file_leaves_goes_where_memory_is_short(sim_lib):
     assert sim_bytes(sim_lib) == empty
 
 
+@pytest.mark.parametrize("what", ["duplex", "batcher"])
+def test_what_a_file_leaves_goes_for_a_pipeline(sim_lib, what):
+    """A duplex pipeline and a session batcher ask for memory of their own, beside the models': what other handles' files have left goes for those too."""
+    from moshi_amd.batcher import SessionBatcher
+    from moshi_amd.duplex import DuplexStream
+    from moshi_amd.lm import LMGen
+    from tests.batcher_cases import tiny_pair
+    cfg, set_memory = tiny_mimi_config(), sim_lib.cdll.hipsim_set_memory
+    set_memory.argtypes = [ctypes.c_ulonglong]
+    sd = random_mimi_state_dict(cfg, seed=5, device="cpu")
+    others = [MimiModel(sd, cfg, device="cpu", max_batch=1, num_codebooks=4, lib=sim_lib) for _ in range(4)]
+    mimi, lm, _, _ = tiny_pair("cpu", sim_lib, 2)
+    gen = LMGen(lm, use_sampling=False)
+    gc.collect()
+    before = sim_bytes(sim_lib)
+
+    def leave(spare=0):
+        for m in others:
+            m.encode(torch.zeros(1, 1, cfg.frame_size))
+        set_memory(sim_bytes(sim_lib) + spare)
+    try:
+        if what == "batcher":                                  # its own buffers come before the models' streams
+            with mimi.streaming(2), gen.streaming(2):
+                streams = sim_bytes(sim_lib)
+            with SessionBatcher(mimi, lm, 2, use_sampling=False):
+                own = sim_bytes(sim_lib) - streams             # (half of it pinned host memory, which the simulator counts too, and comes first)
+            leave(own // 2)
+            with SessionBatcher(mimi, lm, 2, use_sampling=False) as b:
+                assert b.step() == 0
+        else:
+            with mimi.streaming(2), gen.streaming(2):
+                leave()
+                d = DuplexStream(mimi, gen)
+                d.join()
+                del d
+    finally:
+        set_memory(0)
+    gc.collect()
+    assert sim_bytes(sim_lib) == before
+
+
 def test_a_snapshot_of_another_stream_is_reset_where_it_was_loaded(sim_lib):
     """The tables of where a stream's histories lie are not part of what a snapshot brings: a reset behind a load clears the histories of the
     stream it is called on, and leaves the one that the snapshot came from alone."""
