@@ -288,7 +288,7 @@ inline __global__ __launch_bounds__(256, 4) void k_tlm_conv(TlmLinArgs a, int kg
 // token block w % 4 of P and every other column block
 // ------------------------------------------------------------------------------------------------
 inline size_t tlm_chunk_lightning_smem() { return (size_t)(2 * TLM_CHUNK * TLM_PST + TLM_CHUNK + 1) * sizeof(float); }
-inline __device__ __forceinline__ void tlm_chunk_lightning(const TlmLinArgs& a, float* sh, int chunk, int h) {
+__device__ __forceinline__ void tlm_chunk_lightning(const TlmLinArgs& a, float* sh, int chunk, int h) {
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), bl = lane & 15, kq = lane >> 4;
     const int tb = wave & 3, j0 = wave >> 2;
     const TlmSeg ck = a.chunk[chunk];
