@@ -247,8 +247,8 @@ int mmi_lm_streaming_batch(const mmi_lm* lm);
  * on that device.  mmi_*_device return the ordinal. */
 int mmi_lm_device(const mmi_lm* lm);
 int mmi_mimi_device(const mmi_mimi* m);
-/* Engine counters for tests / diagnostics.  which = 0: GEMM launches (or captured graph nodes) that took the LDS-resident
- * kernel (k_gemm_xlds); 1: bit v set = step program v (short-ring / deep-ring decode attention) is captured and instantiated -
+/* Engine counters for tests / diagnostics.  which = 0: GEMM launches (or captured graph nodes) that took a kernel
+ * with resident activations (k_gemm_xreg, k_gemm_xlds); 1: bit v set = step program v (short-ring / deep-ring decode attention) is captured and instantiated -
  * both are from the stream's first step on, so that the switch is never a capture inside a live session; 2: the host's bound on
  * the ring depth (steps since streaming_start / seek / the offsets of a restored snapshot); 3: the depth transformer's MFMA tile
  * (16 at <= 32 sessions with bf16 weights, else 32). */

@@ -140,7 +140,7 @@ struct mmi_lm {
     int attn_ns = 1;                                // workgroups per (session, head) of the decode attention (attn_splits)
     long depth_bound = 0;                           // no session's offset exceeds this (steps since streaming_start / the last seek; resets
                                                     // only lower offsets): picks the step program's variant (attn_variant)
-    long xlds_launches = 0;         // launches (or graph nodes captured) that took k_gemm_xlds: mmi_lm_stat(lm, 0)
+    long xlds_launches = 0;         // launches (or graph nodes captured) that took k_gemm_xreg or k_gemm_xlds: mmi_lm_stat(lm, 0)
     bool precapture_failed = false; // capturing the second attention program ahead of time failed once: not tried again for this stream
     const char* dominant_name = ""; // what the profiled (dominant) linear last ran on
     MmiProgram prog;
@@ -377,7 +377,7 @@ int launch_gemm_t(hipStream_t s, const GemmPlan& p, int NT, int mt, const GemmAr
     return mmi_fail(MMI_ERR_UNSUPPORTED, "batch too large for the skinny GEMM");
 }
 
-// k_gemm_xlds (activations resident in LDS, one workgroup per CU): which GEMMs take it, and how.  MMI_GEMM_LDS: "2" = with
+// k_gemm_xlds (activations resident in LDS, one workgroup per CU): which of the GEMMs that plan_xreg leaves take it, and how.  MMI_GEMM_LDS: "2" = with
 // the staggered tail (each tile's epilogue under the last chunk's weight stream; the DEFAULT for bf16 weights at the 32-row
 // tile: same-box A/B of the default benchmark 8.10 / 8.12 ms against 8.17 / 8.20 ms with k_gemm_xp, dominant kernel 38.6
 // against 40.2 us live, profiles/r02_logs/ab_gemm_xlds_stagger_in_step.txt), "1" = plain tails (also what int8 / fp8 weight
@@ -442,6 +442,69 @@ int launch_xlds(hipStream_t s, const XldsPlan& p, const GemmArgs& a) {
     return p.stagger ? launch_xlds_kc<MT, true, 0>(s, p, a) : launch_xlds_kc<MT, false, 0>(s, p, a);
 }
 
+// k_gemm_xreg (activations resident in registers, one workgroup per CU): which GEMMs take it, and how.  nx: entries of a wave's K-slice, as
+// instantiated (0: another kernel).  Every stream it can hold goes there (it was the faster one at all shapes, see the kernel): the 32-row tile,
+// int8 x int8 up to 64 rows and bf16 up to 32, slices of at most 16 / 32 entries (4096 features unsplit; two batch tiles of bf16 do not fit the
+// registers: k_gemm_xlds), 128 tiles or more - with fewer there is no second tile per workgroup to stream under the first one's epilogue.
+// MMI_GEMM_REG: "0" = off, a number = every GEMM whose slices fit, on so many workgroups (tests on tiny shapes).
+struct XregPlan { int nx, ksplit, grid; size_t smem; };
+int xreg_entries(int T, int mt, int wq, int kper) {
+    if (T == 32 && mt == 1 && wq == 0) return kper <= 8 ? 8 : (kper <= 22 ? 22 : (kper <= 32 ? 32 : 0));
+    if (T == 32 && mt <= 2 && wq == 3) return kper <= 4 ? 4 : (kper <= 11 ? 11 : (kper <= 16 ? 16 : 0));
+    return 0;
+}
+XregPlan plan_xreg(const GemmW& g, int epi, int wq, int B, int Dh) {
+    XregPlan p{0, 1, 0, 0};
+    if (epi != MMI_EPI_GATE && epi != MMI_EPI_ROPE_KV && epi != MMI_EPI_STORE && epi != MMI_EPI_PARTIAL) return p;   // no prefetched addend
+    const char* e = getenv("MMI_GEMM_REG");
+    const int forced = e ? atoi(e) : -1;
+    if (forced == 0 || getenv("MMI_GEMM_LDS") || g.T != 32) return p;
+    const int mt = mmi_cdiv(B, g.T);
+    if (forced < 0 && g.NT < 128) return p;
+    if (epi == MMI_EPI_PARTIAL) {
+        p.ksplit = 4;                          // two tiles of N = 4096 per workgroup, on half the activations of two splits
+        if (const char* ek = getenv("MMI_GEMM_KSPLIT")) p.ksplit = atoi(ek);
+        if (p.ksplit < 1 || p.ksplit > 4) return p;
+    }
+    p.grid = (forced > 0 ? forced : 256) / p.ksplit;
+    const int nx = xreg_entries(g.T, mt, wq, mmi_cdiv(mmi_cdiv(g.KSTEPS, p.ksplit), 8));
+    if (p.grid < 1) p.grid = 1;
+    if (p.grid > g.NT) p.grid = g.NT;
+    const int features = (mmi_cdiv(g.NT, p.grid) + 1) * g.T;        // an octet range may reach into one more tile
+    const bool rope = epi == MMI_EPI_ROPE_KV;
+    if (features > 512 || (rope && Dh > 128)) return p;
+    p.smem = mmi_xreg_smem(mt, B, Dh, rope, features);
+    if (p.smem <= 131072) p.nx = nx;
+    return p;
+}
+
+template <int MT, int NX, int RD, int WQ>
+int launch_xreg_v(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        MMI_HIP_CHECK(hipFuncSetAttribute((const void*)k_gemm_xreg<MT, NX, RD, WQ>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+        attr_set = true;
+    }
+    MMI_LAUNCH((k_gemm_xreg<MT, NX, RD, WQ>), dim3(p.grid, p.ksplit), 512, p.smem, s, a);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
+int launch_xreg(hipStream_t s, const XregPlan& p, int mt, const GemmArgs& a) {
+    if (a.wq == 0) {
+        if (p.nx == 8) return launch_xreg_v<1, 8, 8, 0>(s, p, a);
+        if (p.nx == 22) return launch_xreg_v<1, 22, 11, 0>(s, p, a);
+        return launch_xreg_v<1, 32, 8, 0>(s, p, a);
+    }
+    if (mt == 1) {
+        if (p.nx == 4) return launch_xreg_v<1, 4, 4, 3>(s, p, a);
+        if (p.nx == 11) return launch_xreg_v<1, 11, 11, 3>(s, p, a);
+        return launch_xreg_v<1, 16, 8, 3>(s, p, a);
+    }
+    if (p.nx == 4) return launch_xreg_v<2, 4, 4, 3>(s, p, a);
+    if (p.nx == 11) return launch_xreg_v<2, 11, 11, 3>(s, p, a);
+    return launch_xreg_v<2, 16, 8, 3>(s, p, a);
+}
+
 // k_gemm_xp_once (a wave's whole K-slice requested before its first MFMA) for the GEMMs k_gemm_xp would walk in three or more
 // dependent memory round trips although they are a latency chain, not a stream: bf16 weights behind at most 256 workgroups of 8
 // waves whose slice is longer than the two register buffers of k_gemm_xp (2 x 4 k-steps) and short enough for the registers -
@@ -488,7 +551,7 @@ hipError_t dominant_begin(mmi_lm* lm, hipStream_t s, EvPair** ev) {
 }
 
 // its name with the instantiation (launch_xlds, launch_gemm_w) and what it computes; valid for ever, whoever holds it
-const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XldsPlan& xl, int mt, int wq) {
+const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XregPlan& xr, const XldsPlan& xl, int mt, int wq) {
     const std::string on = wq == 3 ? ", int8 weights x int8 activations" : (wq == 1 ? ", int8 weights" : (wq == 2 ? ", fp8 weights on the fp8 MFMA" : ""));
     const auto args = [](std::initializer_list<int> v) {
         std::string t;
@@ -496,7 +559,8 @@ const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XldsPlan& x
         return t;
     };
     const int u = wq == 0 ? (p.waves == 8 && p.u == 2 && mt == 1 ? 2 : 4) : (wq == 3 && q8_four() && p.waves == 8 ? 4 : 2);
-    std::string k = xl.on ? "k_gemm_xlds" + args({mt, xl.kc, 3}) + (xl.stagger ? ", true, " : ", false, ") + std::to_string(wq)
+    std::string k = xr.nx ? "k_gemm_xreg" + args({mt, xr.nx, xr.nx > 16 ? xr.nx / 2 : xr.nx, wq})
+                  : xl.on ? "k_gemm_xlds" + args({mt, xl.kc, 3}) + (xl.stagger ? ", true, " : ", false, ") + std::to_string(wq)
                           : "k_gemm_xp" + args({g.T, mt, 1, p.waves, u}) + (wq ? ", " + std::to_string(wq) : "");
     static std::mutex names_lock;
     static std::set<std::string> names;
@@ -512,13 +576,17 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
     const int mt = mmi_cdiv(a.B, g.T);
     const GemmPlan p = plan_gemm(g, a.epi == MMI_EPI_PARTIAL);
     a.osplit = plan_osplit(g, p, a.epi, g.T);
+    const XregPlan xr = plan_xreg(g, a.epi, a.wq, a.B, a.Dh);
     const XldsPlan xl = plan_xlds(lm, g, a, mt);
     EvPair* ev = nullptr;
-    if (is_dominant && lm->profiling) lm->dominant_name = dominant_kernel(g, p, xl, mt, a.wq);
+    if (is_dominant && lm->profiling) lm->dominant_name = dominant_kernel(g, p, xr, xl, mt, a.wq);
     if (is_dominant) MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
     int rc;
     mmi_record_bytes((long)g.bytes);
-    if (xl.on) {
+    if (xr.nx) {
+        lm->xlds_launches += 1;
+        rc = launch_xreg(s, xr, mt, a);
+    } else if (xl.on) {
         lm->xlds_launches += 1;
         rc = mt == 1 ? launch_xlds<1>(s, xl, a) : launch_xlds<2>(s, xl, a);
     } else if (const int kmax = once_kmax(g, p, mt, a)) {
@@ -606,11 +674,18 @@ void add_dep_attn_out_proj(mmi_lm* lm, const GemmW& g, const DepAttnArgs& da, ui
 // and the norm dequantises (sx = the absmax of the GEMM's input rows, scb = its SCB; k_resid_rmsnorm psx / pscb)
 struct Pending { int P = 0; const float* sx = nullptr; const float* scb = nullptr; };
 
+// over how many workgroups launch_gemm splits the reduction of a GEMM with a residual behind it (1: its epilogue adds the residual itself)
+int resid_ksplit(const GemmW& g, int wq, int B) {
+    const int n = plan_gemm(g, true).ksplit;
+    const XregPlan xr = n > 1 ? plan_xreg(g, MMI_EPI_PARTIAL, wq, B, 0) : XregPlan{0, 1, 0, 0};
+    return xr.nx ? xr.ksplit : n;
+}
+
 // K-split GEMM whose partial sums (lm->partial) the following add_resid_rmsnorm folds into the residual stream.
 // Returns the partials, P = 0 when the GEMM is not split (then it applied the residual itself, in place on x).
 Pending add_gemm_resid(mmi_lm* lm, const GemmW& g, const uint16_t* in, uint16_t* x, int features, const Q8* q8 = nullptr) {
-    const GemmPlan p = plan_gemm(g, true);
-    if (p.ksplit <= 1) {
+    const int ksplit = resid_ksplit(g, q8 ? q8->wq : g.wq, lm->batch);
+    if (ksplit <= 1) {
         add_gemm(lm, g, in, x, features, true, MMI_EPI_RESID, x, nullptr, nullptr, 0, false, nullptr, q8);
         return Pending{};
     }
@@ -621,7 +696,7 @@ Pending add_gemm_resid(mmi_lm* lm, const GemmW& g, const uint16_t* in, uint16_t*
     GemmW gw = g;
     lm->prog.add([lm, gw, a](hipStream_t s) { return launch_gemm(lm, s, gw, a, false); }, (long)g.bytes);
     Pending pd;
-    pd.P = p.ksplit;
+    pd.P = ksplit;
     if (q8 && q8->wq == 3 && g.wq == 1) { pd.sx = q8->sx; pd.scb = g.scb; }
     return pd;
 }
@@ -1986,10 +2061,10 @@ extern "C" int mmi_lm_debug_linear(mmi_lm* lm, const char* weight_name, const ch
         if (a8) { a.xp = reinterpret_cast<const u32x4*>(xq); a.sx = sx; a.wq = 3; }
         Pending pd;
         if (path == MMI_DBG_SPLITK) {
-            const GemmPlan p = plan_gemm(g, true);
-            if (gated || p.ksplit <= 1) return done(mmi_fail(MMI_ERR_UNSUPPORTED, "mmi_lm_debug_linear: the engine does not split this GEMM over K"));
+            const int ksplit = resid_ksplit(g, a.wq ? a.wq : g.wq, rows);
+            if (gated || ksplit <= 1) return done(mmi_fail(MMI_ERR_UNSUPPORTED, "mmi_lm_debug_linear: the engine does not split this GEMM over K"));
             a.epi = MMI_EPI_PARTIAL; a.partial = partial; a.out = nullptr;
-            pd.P = p.ksplit;
+            pd.P = ksplit;
             if (a8) { pd.sx = sx; pd.scb = g.scb; }
         }
         rc = launch_gemm(lm, s, g, a, false);

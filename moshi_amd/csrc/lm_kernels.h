@@ -1263,6 +1263,256 @@ __global__ __launch_bounds__(512) void k_gemm_xlds(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// weight-streaming GEMM with the activations resident in registers
+// ------------------------------------------------------------------------------------------------
+// One workgroup of 8 waves per CU (gridDim.x <= CUs, gridDim.y K splits) walks a contiguous range of 32-row tiles.  The waves split K, so a wave
+// only ever meets its own K-slice of the activations: at 64 int8 or 32 bf16 rows of 4096 features that is 128 registers, read from the L2 once
+// per launch.  What is left of the loop is the weight stream - NX entries of 1 KiB per tile and wave, RD of them on their way in a ring of
+// registers that runs on through the tiles - and the products; no LDS, no barrier.  Each tile ends in the sum over the waves and the epilogue,
+// under the stream of the next one: loads come back in the order they were asked for, so the epilogue's operands (absmax and scales, offsets,
+// angles) are copied to LDS at the start - one that read global memory would wait for all of the ring.
+// Bound by the weight stream (a chain of launches that only read gets 92 MB in 15.2 us, 184 MB in 29), the activations' 1 - 2 us and the last
+// tile's epilogue.  Chains of dependent launches on weights from memory, us, before (int8 k_gemm_xp; bf16 k_gemm_xlds, PARTIAL k_gemm_xp) / here:
+//   64 rows, int8   linear_in 92 MB 25.5 / 19.9, in_proj 50 MB 18.3 / 15.2, linear_out 46 MB 14.5 / 12.4, out_proj 17 MB 7.9 / 7.2
+//   32 rows, bf16   184 MB 35.9 / 33.3, 101 MB 22.9 / 20.8, 92 MB 19.4 / 18.0, 34 MB 10.5 / 9.7
+//   32 rows, int8   92 MB 21.5 / 18.7, 50 MB 15.0 / 13.3, 46 MB 12.0 / 11.1, 17 MB 6.3 / 6.2
+struct XregLocal {
+    const float* sx;                // [B]
+    const float* scb;               // wscb of the workgroup's features; of the value rows of a gated linear: + vals
+    const long* off;                // [B]
+    const float* rope;              // [B][Dh / 2][2]
+    int n0, vals;                   // first feature, features
+};
+
+// Sum over the 8 waves (in their order) and epilogue of one 32-row tile, 4 features per thread and all waves at work: a task that sums 8 features
+// keeps half of the waves or fewer busy for twice as long (three tiles of linear_in at 64 int8 rows: 6.0 us of the launch, here 2.6).
+// Scratch [wave][m][quad][64] of 16-byte sums.  Packed rows (gated): lanes take consecutive rows of one quad.  Otherwise 8 lanes take the 32
+// features of a row - 128 bytes of partial sums, 64 of a row of logits or keys - and the lanes' places are exchanged by quad, so that the eight
+// planes they read from do not meet in the same banks.
+template <int MT, int WQ>
+__device__ __forceinline__ void mmi_xreg_epilogue(const GemmArgs& a, const XregLocal& loc, f32x4* red, const f32x16 (&acc)[MT], int wave, int lane, int nt, int g_lo, int g_hi) {
+    const bool gate = a.epi == MMI_EPI_GATE;
+    auto place = [&](int quad, int l) { return gate ? l : l ^ (4 * quad + 2 * (l >> 5)); };
+    mmi_meet();                                  // the previous tile's sums have been read (the weights in flight stay there)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) red[((wave * MT + m) * 4 + c) * 64 + place(c, lane)] = f32x4{acc[m][4 * c], acc[m][4 * c + 1], acc[m][4 * c + 2], acc[m][4 * c + 3]};
+    mmi_meet();
+    if (wave >= 4 * MT) return;
+    // this lane's quad: accumulator quad c of lane `from` (row from & 31, features 8 c + 4 (from >> 5) ..)
+    const int m = wave >> 2;
+    int c, from;
+    if (gate) {                                  // gate rows in the lower lanes, their value rows in the upper ones
+        c = (wave & 1) + 2 * (lane >> 5);
+        from = 32 * ((wave >> 1) & 1) + (lane & 31);
+    } else {
+        c = (lane & 7) >> 1;
+        from = 32 * (lane & 1) + 8 * (wave & 3) + (lane >> 3);
+    }
+    const int hi = from >> 5, bl = from & 31, b = m * 32 + bl;
+    f32x4 part[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) part[w] = red[((w * MT + m) * 4 + c) * 64 + place(c, from)];
+    float s[4];
+    const int f0 = gate ? nt * 16 + 8 * (c & 1) + 4 * hi : nt * 32 + 8 * c + 4 * hi;       // first of the quad's (hidden) features
+    if constexpr (WQ == 3) {
+        int si[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            const i32x4 v = __builtin_bit_cast(i32x4, part[w]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) si[e] += v[e];
+        }
+        if (a.epi == MMI_EPI_PARTIAL) {          // (the norm launch adds the splits' integers, then dequantises)
+            if (b < a.B && f0 < a.N && c >= g_lo && c < g_hi)
+                *reinterpret_cast<i32x4*>(reinterpret_cast<int*>(a.partial) + ((long)blockIdx.y * a.B + b) * a.N + f0) = i32x4{si[0], si[1], si[2], si[3]};
+            return;
+        }
+        const float sca = loc.sx[b];
+        const f32x4 sc = *reinterpret_cast<const f32x4*>(loc.scb + (gate && (lane >> 5) ? loc.vals : 0) + f0 - loc.n0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = mmi_i8_dequant(si[e], sca, sc[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += part[w][e];
+        if (a.epi == MMI_EPI_PARTIAL) {
+            if (b < a.B && f0 < a.N && c >= g_lo && c < g_hi) *reinterpret_cast<f32x4*>(a.partial + ((long)blockIdx.y * a.B + b) * a.N + f0) = f32x4{s[0], s[1], s[2], s[3]};
+            return;
+        }
+    }
+    if (gate) {
+        // features 0, 1 of the quad to the lower lanes, 2, 3 to the upper ones: (gate, value) pairs on one lane
+        mmi_swap32(s[0], s[2]);
+        mmi_swap32(s[1], s[3]);
+        if (b >= a.B || f0 >= a.N) return;
+        float o[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float g = mmi_round_bf16(s[e]), u = mmi_round_bf16(s[2 + e]);
+            o[e] = mmi_round_bf16(g / (1.0f + expf(-g))) * u;          // F.silu on a bf16 tensor
+        }
+        const int n = f0 + 2 * (lane >> 5);
+        uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(32, b, n, a.out_ksteps) : a.out + (long)b * a.out_ld + n;
+        *reinterpret_cast<uint32_t*>(dst) = mmi_pack_bf16x2(o[0], o[1]);
+        return;
+    }
+    if (b >= a.B || f0 >= a.N || c < g_lo || c >= g_hi) return;
+    if (a.epi == MMI_EPI_ROPE_KV) {
+        const int HD = a.H * a.Dh, sec = f0 / HD, hn = f0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = mmi_round_bf16(s[e]);          // in_proj output is a bf16 tensor
+        if (sec < 2) {
+            const f32x4 cs = *reinterpret_cast<const f32x4*>(loc.rope + b * a.Dh + d0);      // two (cos, sin) pairs
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float re = v[2 * j], im = v[2 * j + 1];
+                mmi_rope_rotate(re, im, cs[2 * j], cs[2 * j + 1], v[2 * j], v[2 * j + 1]);
+            }
+        }
+        const long at = sec == 0 ? 0 : (((long)b * a.H + h) * a.cap + (int)(loc.off[b] % a.cap)) * a.Dh + d0;
+        if (sec != 0 && a.kv8) {
+            *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(sec == 1 ? a.kc : a.vc) + at) =
+                mmi_cvt_fp8x4(mmi_round_bf16(v[0]), mmi_round_bf16(v[1]), mmi_round_bf16(v[2]), mmi_round_bf16(v[3]));
+            return;
+        }
+        uint16_t* dst = sec == 0 ? a.qrot + (long)b * HD + hn : (sec == 1 ? a.kc : a.vc) + at;
+        *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(v[0], v[1]), mmi_pack_bf16x2(v[2], v[3])};
+        return;
+    }
+    uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(32, b, f0, a.out_ksteps) : a.out + (long)b * a.out_ld + f0;
+    *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(s[0], s[1]), mmi_pack_bf16x2(s[2], s[3])};
+}
+
+template <int MT, int NX, int RD, int WQ>
+__global__ __launch_bounds__(512, 2) void k_gemm_xreg(GemmArgs a) {
+    static_assert(WQ == 0 || WQ == 3, "one activation fragment per weight entry");
+    static_assert(RD <= NX && NX % RD == 0, "the ring's places are known at compile time");
+    MMI_DYN_SHARED(float, lds);                 // scratch of the sums, then the epilogue's operands (mmi_xreg_smem)
+    const int tid = (int)threadIdx.x, wave = mmi_uniform(tid >> 6), lane = tid & 63;
+    const int G = (int)gridDim.x, bid = (int)blockIdx.x;
+    // the workgroup's share of the tiles, in row octets where the epilogue's 8-feature groups are weight row octets (k_gemm_xlds)
+    const bool by_octet = a.epi != MMI_EPI_GATE;
+    const long units = by_octet ? 4L * a.NT : (long)a.NT;
+    const long u0 = (long)bid * units / G, u1 = (long)(bid + 1) * units / G;
+    const int t0 = by_octet ? (int)(u0 >> 2) : (int)u0, t1 = by_octet ? (int)((u1 + 3) >> 2) : (int)u1;
+    const int ntiles = u1 > u0 ? t1 - t0 : 0;
+    if (ntiles == 0) return;
+    auto oct_lo = [&](int t) { return by_octet ? (int)max(0L, u0 - 4L * (t0 + t)) : 0; };
+    auto oct_hi = [&](int t) { return by_octet ? (int)min(4L, u1 - 4L * (t0 + t)) : 4; };
+    // K range of this split, then of this wave; entries past its end repeat a valid address and meet zeros
+    const int kb_per = (a.KSTEPS + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int kb0 = min(a.KSTEPS, (int)blockIdx.y * kb_per), kb1 = min(a.KSTEPS, kb0 + kb_per);
+    const int kper = (kb1 - kb0 + 7) / 8;       // <= NX (checked by the launcher)
+    const int ks0 = min(kb1, kb0 + wave * kper), nks = min(kb1, ks0 + kper) - ks0;
+    const int ksl = min(ks0, a.KSTEPS - 1), kl = nks > 0 ? nks - 1 : 0;
+    // the epilogue's operands, to registers
+    XregLocal loc;
+    const int rows_out = by_octet ? 32 : 16;
+    loc.n0 = t0 * rows_out;
+    loc.vals = ntiles * rows_out;
+    float* rope = lds + 8 * MT * 1024;
+    long* off = reinterpret_cast<long*>(rope + (a.epi == MMI_EPI_ROPE_KV ? a.B * a.Dh : 0));
+    float* sx = reinterpret_cast<float*>(off + MT * 32);
+    float* scb = sx + MT * 32;
+    f32x4 rpre[2 * MT];
+    float spre[2] = {0.f, 0.f}, xpre = 0.f;
+    long opre = 0;
+    if (a.epi == MMI_EPI_ROPE_KV) {
+#pragma unroll
+        for (int j = 0; j < 2 * MT; ++j) rpre[j] = *reinterpret_cast<const f32x4*>(a.rope + min(4 * (j * 512 + tid), a.B * a.Dh - 4));
+        opre = a.offsets[min(tid, a.B - 1)];
+    }
+    if constexpr (WQ == 3) {
+        xpre = a.sx[min(tid, a.B - 1)];
+        if (a.epi != MMI_EPI_PARTIAL) {
+            spre[0] = a.wscb[min(loc.n0 + tid, a.N - 1)];
+            if (!by_octet) spre[1] = a.wscb[a.gate_rows + min(loc.n0 + tid, a.N - 1)];
+        }
+    }
+    // entries of tile t at a scalar address, and a lane's place in an entry (lanes of octets it does not own repeat one that it owns)
+    auto wlane = [&](int t) {
+        const int ro = (lane >> 3) & 3, lo = oct_lo(t), hi = oct_hi(t);
+        return (unsigned)((ro >= lo && ro < hi) ? lane : ((lane & ~0x18) | (lo << 3)));
+    };
+    auto wbase = [&](int t) { return a.wp + ((long)(t0 + t) * a.KSTEPS + ksl) * 64; };
+    u32x4 w[RD], x[MT][NX];
+    const u32x4* wp = wbase(0);
+    unsigned wl = wlane(0);
+#pragma unroll
+    for (int e = 0; e < RD; ++e) w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
+    mmi_sched_barrier();
+    if (a.epi == MMI_EPI_ROPE_KV) {
+#pragma unroll
+        for (int j = 0; j < 2 * MT; ++j)
+            if (4 * (j * 512 + tid) < a.B * a.Dh) *reinterpret_cast<f32x4*>(rope + 4 * (j * 512 + tid)) = rpre[j];
+        if (tid < MT * 32) off[tid] = opre;
+    }
+    if constexpr (WQ == 3) {
+        if (tid < MT * 32) sx[tid] = xpre;
+        if (tid < loc.vals) {
+            scb[tid] = spre[0];
+            scb[loc.vals + tid] = spre[1];
+        }
+    }
+    loc.rope = rope; loc.off = off; loc.sx = sx; loc.scb = scb;
+#pragma unroll
+    for (int e = 0; e < NX; ++e)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) x[m][e] = (a.xp + ((long)m * a.KSTEPS + ksl + min(e, kl)) * 64)[(unsigned)lane];
+    mmi_sched_barrier();
+    if (nks < NX) {                             // (full slices: the products of the first entries need not wait for the last ones)
+#pragma unroll
+        for (int e = 0; e < NX; ++e)
+            if (e >= nks) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) x[m][e] = u32x4{0u, 0u, 0u, 0u};
+            }
+    }
+    f32x16 acc[MT];
+    auto tile = [&](const u32x4* next, unsigned nl, auto more_tag) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_tag)::value;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+#pragma unroll
+        for (int e = 0; e < NX; ++e) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if constexpr (WQ == 3) acc[m] = __builtin_bit_cast(f32x16, mmi_mfma_i8_32x32x32(w[e % RD], x[m][e], __builtin_bit_cast(i32x16, acc[m])));
+                else acc[m] = mmi_mfma_bf16_32x32x16(w[e % RD], x[m][e], acc[m]);
+            }
+            if (e + RD < NX) w[e % RD] = mmi_load_nt(wp + min(e + RD, kl) * 64 + wl);
+            else if (MORE) w[e % RD] = mmi_load_nt(next + min(e + RD - NX, kl) * 64 + nl);
+            if (e & 1) mmi_sched_barrier();
+        }
+    };
+#pragma unroll 1
+    for (int t = 0; t < ntiles; ++t) {
+        if (t + 1 < ntiles) {
+            const u32x4* next = wbase(t + 1);
+            const unsigned nl = wlane(t + 1);
+            tile(next, nl, MmiTrue{});
+            wp = next;
+            wl = nl;
+        } else {
+            tile(wp, wl, MmiFalse{});
+        }
+        mmi_xreg_epilogue<MT, WQ>(a, loc, reinterpret_cast<f32x4*>(lds), acc, wave, lane, t0 + t, oct_lo(t), oct_hi(t));
+    }
+}
+// LDS of k_gemm_xreg in bytes: scratch, angles, offsets, rows' absmax, scales of `features` gate and value rows
+static inline size_t mmi_xreg_smem(int MT, int B, int Dh, bool rope, int features) {
+    return (size_t)8 * MT * 4096 + (rope ? (size_t)B * Dh * 4 : 0) + (size_t)MT * 32 * (sizeof(long) + 4) + (size_t)2 * features * 4;
+}
+
+// ------------------------------------------------------------------------------------------------
 // RMSNorm (rms_norm_f32, eps 1e-8): y = (x.float() * (alpha.float() * rsqrt(eps + mean(x^2)))).to(bf16)
 // ------------------------------------------------------------------------------------------------
 // One block per session row b; thread t owns the 16-byte piece (8 features) t, t + blockDim, ... of the packed row

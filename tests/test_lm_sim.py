@@ -241,6 +241,21 @@ def test_gemm_with_activations_resident_in_lds_quantised_weights(sim_lib, monkey
     assert st["xlds_launches"] >= 2 * (2 * 2 + 1)
 
 
+@pytest.mark.parametrize("B,grid,quantize", [(18, 5, False), (32, 8, False), (18, 7, True), (34, 8, True), (64, 64, True)])
+def test_gemm_with_activations_resident_in_registers(sim_lib, monkeypatch, B, grid, quantize):
+    """k_gemm_xreg (one workgroup walking its tiles behind a ring of weights) forced onto every GEMM of the tiny model that it can hold: gated
+    input, in_proj with RoPE and ring write, heads, split sums; one and two batch tiles, bf16 and int8 rows, shares of whole tiles and of row
+    octets, more workgroups than tiles, waves without entries of their own."""
+    monkeypatch.setenv("MMI_GEMM_REG", str(grid))
+    st = {}
+    lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=190 + B, B=B, S=2, quantize=quantize, stats=st)
+    assert st["xlds_launches"] >= 2 * (2 * 2 + 1)
+    monkeypatch.setenv("MMI_GEMM_KSPLIT", "2")
+    lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=191 + B, B=B, S=2, quantize=quantize)
+    if quantize:
+        assert any("[splitk]" in n for n, _ in lm_cases.int8_linears_bit_exact("cpu", sim_lib, tiny_lm_config(), B, seed=192 + B))
+
+
 def test_depformer_in_per_step_launches(sim_lib, monkeypatch):
     """The engine normally runs the dep_q `depformer_in` linears as one grouped GEMM and lets each sampler add its token's
     embedding row; depth widths that are not whole n-tiles fall back to one GEMM per micro-step with the embedding in its
