@@ -449,6 +449,7 @@ int launch_xlds(hipStream_t s, const XldsPlan& p, const GemmArgs& a) {
 // MMI_GEMM_REG: "0" = off, a number = every GEMM whose slices fit, on so many workgroups (tests on tiny shapes).
 struct XregPlan { int nx, ksplit, grid; size_t smem; };
 int xreg_entries(int T, int mt, int wq, int kper) {
+    if (T == 16 && mt == 1 && wq == 0) return kper <= 4 ? 4 : (kper <= 16 ? 16 : 0);
     if (T == 32 && mt == 1 && wq == 0) return kper <= 8 ? 8 : (kper <= 22 ? 22 : (kper <= 32 ? 32 : 0));
     if (T == 32 && mt <= 2 && wq == 3) return kper <= 4 ? 4 : (kper <= 11 ? 11 : (kper <= 16 ? 16 : 0));
     return 0;
@@ -458,8 +459,14 @@ XregPlan plan_xreg(const GemmW& g, int epi, int wq, int B, int Dh) {
     if (epi != MMI_EPI_GATE && epi != MMI_EPI_ROPE_KV && epi != MMI_EPI_STORE && epi != MMI_EPI_PARTIAL) return p;   // no prefetched addend
     const char* e = getenv("MMI_GEMM_REG");
     const int forced = e ? atoi(e) : -1;
-    if (forced == 0 || getenv("MMI_GEMM_LDS") || g.T != 32) return p;
+    if (forced == 0 || getenv("MMI_GEMM_LDS")) return p;
     const int mt = mmi_cdiv(B, g.T);
+    if (g.T == 16) {
+        if (epi == MMI_EPI_PARTIAL || (forced < 0 && g.NT < 512) || (epi == MMI_EPI_ROPE_KV && (B * Dh > MMI_XREG16_MAXROPE || Dh % 4))) return p;
+        p.grid = std::min(forced > 0 ? forced : 256, g.NT);
+        p.nx = xreg_entries(16, mt, wq, mmi_cdiv(g.KSTEPS, 8));
+        return p;
+    }
     if (forced < 0 && g.NT < 128) return p;
     if (epi == MMI_EPI_PARTIAL) {
         p.ksplit = 4;                          // two tiles of N = 4096 per workgroup, on half the activations of two splits
@@ -489,7 +496,15 @@ int launch_xreg_v(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
     MMI_CHECK_LAUNCH();
     return MMI_OK;
 }
-int launch_xreg(hipStream_t s, const XregPlan& p, int mt, const GemmArgs& a) {
+template <bool NORM>
+int launch_xreg16(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
+    if (p.nx == 4) MMI_LAUNCH((k_gemm_xreg16<4, NORM>), p.grid, 512, 0, s, a);
+    else MMI_LAUNCH((k_gemm_xreg16<16, NORM>), p.grid, 512, 0, s, a);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
+int launch_xreg(hipStream_t s, const XregPlan& p, int T, int mt, const GemmArgs& a) {
+    if (T == 16) return launch_xreg16<false>(s, p, a);
     if (a.wq == 0) {
         if (p.nx == 8) return launch_xreg_v<1, 8, 8, 0>(s, p, a);
         if (p.nx == 22) return launch_xreg_v<1, 22, 11, 0>(s, p, a);
@@ -559,7 +574,8 @@ const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XregPlan& x
         return t;
     };
     const int u = wq == 0 ? (p.waves == 8 && p.u == 2 && mt == 1 ? 2 : 4) : (wq == 3 && q8_four() && p.waves == 8 ? 4 : 2);
-    std::string k = xr.nx ? "k_gemm_xreg" + args({mt, xr.nx, xr.nx > 16 ? xr.nx / 2 : xr.nx, wq})
+    std::string k = xr.nx && g.T == 16 ? "k_gemm_xreg16" + args({xr.nx}) + ", false"
+                  : xr.nx ? "k_gemm_xreg" + args({mt, xr.nx, xr.nx > 16 ? xr.nx / 2 : xr.nx, wq})
                   : xl.on ? "k_gemm_xlds" + args({mt, xl.kc, 3}) + (xl.stagger ? ", true, " : ", false, ") + std::to_string(wq)
                           : "k_gemm_xp" + args({g.T, mt, 1, p.waves, u}) + (wq ? ", " + std::to_string(wq) : "");
     static std::mutex names_lock;
@@ -585,7 +601,7 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
     mmi_record_bytes((long)g.bytes);
     if (xr.nx) {
         lm->xlds_launches += 1;
-        rc = launch_xreg(s, xr, mt, a);
+        rc = launch_xreg(s, xr, g.T, mt, a);
     } else if (xl.on) {
         lm->xlds_launches += 1;
         rc = mt == 1 ? launch_xlds<1>(s, xl, a) : launch_xlds<2>(s, xl, a);
@@ -837,7 +853,7 @@ void add_norm_gemm(mmi_lm* lm, const GemmW& g, uint16_t* x, const uint16_t* alph
     }, gbytes);
 }
 
-// Does one launch take norm and linear (k_gemm_norm_one)?  One session, bf16 weights on the 16-row tile, a row of at most 4096 features and whole
+// Does one launch take norm and linear (k_gemm_xreg16, k_gemm_norm_one)?  One session, bf16 weights on the 16-row tile, a row of at most 4096 features and whole
 // pieces of 8, no split sums pending; with more sessions a workgroup's rows would cost as much as its weights.
 bool norm_one(const mmi_lm* lm, const GemmW& g, const Pending& pd, int D) {
     return lm->batch == 1 && lm->T == 16 && g.T == 16 && g.wq == 0 && pd.P == 0 && D % 8 == 0 && D <= 4096 && g.KSTEPS <= 128 && !getenv("MMI_NO_NORM_FUSION");
@@ -845,14 +861,22 @@ bool norm_one(const mmi_lm* lm, const GemmW& g, const Pending& pd, int D) {
 int launch_norm_one(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, const uint16_t* x, const uint16_t* alpha, int D, bool is_dominant) {
     a.xp = reinterpret_cast<const u32x4*>(x); a.alpha = alpha; a.D = D; a.eps = 1e-8f;
     a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT; a.gate_rows = g.gate ? g.N : 0; a.osplit = 1;
+    const XregPlan xr = plan_xreg(g, a.epi, 0, 1, a.Dh);
     mmi_record_bytes((long)g.bytes);
     EvPair* ev = nullptr;
     if (is_dominant) {
-        lm->dominant_name = "k_gemm_norm_one<4> (RMSNorm + temporal FFN linear_in + SiLU gate)";
+        lm->dominant_name = !xr.nx ? "k_gemm_norm_one<4> (RMSNorm + temporal FFN linear_in + SiLU gate)"
+                          : xr.nx == 4 ? "k_gemm_xreg16<4, true> (RMSNorm + temporal FFN linear_in + SiLU gate)" : "k_gemm_xreg16<16, true> (RMSNorm + temporal FFN linear_in + SiLU gate)";
         MMI_HIP_CHECK(dominant_begin(lm, s, &ev));
     }
-    MMI_LAUNCH(k_gemm_norm_one<4>, g.NT, 512, 0, s, a);
-    MMI_CHECK_LAUNCH();
+    if (xr.nx) {
+        lm->xlds_launches += 1;
+        const int rc = launch_xreg16<true>(s, xr, a);
+        if (rc) return rc;
+    } else {
+        MMI_LAUNCH(k_gemm_norm_one<4>, g.NT, 512, 0, s, a);
+        MMI_CHECK_LAUNCH();
+    }
     if (ev) MMI_HIP_CHECK(hipEventRecord(ev->b, s));
     return MMI_OK;
 }

@@ -1513,6 +1513,196 @@ static inline size_t mmi_xreg_smem(int MT, int B, int Dh, bool rope, int feature
 }
 
 // ------------------------------------------------------------------------------------------------
+// the same on the 16-row tile (handles of up to 16 sessions), bf16
+// ------------------------------------------------------------------------------------------------
+// As k_gemm_xreg: one workgroup per CU walks its tiles behind a ring of weights that runs on through them (a whole tile on its way: 128 KiB per
+// CU), a wave's slice of the activations in registers.  A tile is 256 sums: one wave takes them, another one each tile, from one of two
+// scratches, so that a tile costs the others one meeting.  NORM (one session): the workgroup normalises the row first - k_resid_rmsnorm's pieces,
+// sums and roundings, so its bits - behind its first tile of weights, once per CU; every lane then takes 16 bytes of it for all 16 columns.
+template <bool GATE>
+__device__ __forceinline__ void mmi_xreg16_epilogue(const GemmArgs& a, const float* rope, const long* off, const f32x4* red, int lane, int nt, int g_lo, int g_hi) {
+    const int kq = lane >> 4, b = lane & 15;     // (accumulators: row b of the batch, rows 4 kq .. 4 kq + 3 of the tile)
+    f32x4 part[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) part[w] = red[w * 64 + lane];
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 8; ++w)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += part[w][e];
+    if constexpr (GATE) {                        // rows 0 .. 7: gates, on the lower lanes; 8 .. 15 their values, on the upper ones
+        mmi_swap32(s[0], s[2]);
+        mmi_swap32(s[1], s[3]);
+        const int n = nt * 8 + 4 * (kq & 1) + 2 * (lane >> 5);
+        if (b >= a.B || n >= a.N) return;
+        float o[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float g = mmi_round_bf16(s[e]), u = mmi_round_bf16(s[2 + e]);
+            o[e] = mmi_round_bf16(g / (1.0f + expf(-g))) * u;          // F.silu on a bf16 tensor
+        }
+        uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(16, b, n, a.out_ksteps) : a.out + (long)b * a.out_ld + n;
+        *reinterpret_cast<uint32_t*>(dst) = mmi_pack_bf16x2(o[0], o[1]);
+        return;
+    }
+    const int f0 = nt * 16 + 4 * kq;
+    if (b >= a.B || f0 >= a.N || (kq >> 1) < g_lo || (kq >> 1) >= g_hi) return;
+    if (a.epi == MMI_EPI_ROPE_KV) {
+        const int HD = a.H * a.Dh, sec = f0 / HD, hn = f0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = mmi_round_bf16(s[e]);          // in_proj output is a bf16 tensor
+        if (sec < 2) {
+            const f32x4 cs = *reinterpret_cast<const f32x4*>(rope + b * a.Dh + d0);      // two (cos, sin) pairs
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float re = v[2 * j], im = v[2 * j + 1];
+                mmi_rope_rotate(re, im, cs[2 * j], cs[2 * j + 1], v[2 * j], v[2 * j + 1]);
+            }
+        }
+        const long at = sec == 0 ? 0 : (((long)b * a.H + h) * a.cap + (int)(off[b] % a.cap)) * a.Dh + d0;
+        if (sec != 0 && a.kv8) {
+            *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(sec == 1 ? a.kc : a.vc) + at) =
+                mmi_cvt_fp8x4(mmi_round_bf16(v[0]), mmi_round_bf16(v[1]), mmi_round_bf16(v[2]), mmi_round_bf16(v[3]));
+            return;
+        }
+        uint16_t* dst = sec == 0 ? a.qrot + (long)b * HD + hn : (sec == 1 ? a.kc : a.vc) + at;
+        *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(v[0], v[1]), mmi_pack_bf16x2(v[2], v[3])};
+        return;
+    }
+    uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(16, b, f0, a.out_ksteps) : a.out + (long)b * a.out_ld + f0;
+    *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(s[0], s[1]), mmi_pack_bf16x2(s[2], s[3])};
+}
+
+constexpr int MMI_XREG16_MAXROPE = 16 * 128;     // sessions x head features whose angles one piece per thread brings
+// the row of one session, normalised, to LDS (16 bytes per thread; zeros past D): k_resid_rmsnorm's pieces, sums and roundings
+__device__ __forceinline__ void mmi_xreg16_norm(const GemmArgs& a, u32x4* row, float* part, int tid, int wave, int lane, u32x4 v, u32x4 al) {
+    const int i = tid * 8;
+    float f[8], ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        f[2 * q] = mmi_bf16_to_f32((uint16_t)(v[q] & 0xffffu));
+        f[2 * q + 1] = mmi_bf16_to_f32((uint16_t)(v[q] >> 16));
+    }
+    if (i < a.D)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) ss += mmi_shfl_xor(ss, m);
+    if (lane == 0) part[wave] = ss;
+    mmi_meet();
+    float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) tot += part[w];
+    const float rs = mmi_rsqrtf(a.eps + tot / (float)a.D);
+    u32x4 o = {0u, 0u, 0u, 0u};
+    if (i < a.D)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float alo = mmi_bf16_to_f32((uint16_t)(al[q] & 0xffffu)), ahi = mmi_bf16_to_f32((uint16_t)(al[q] >> 16));
+            o[q] = mmi_pack_bf16x2(f[2 * q] * (alo * rs), f[2 * q + 1] * (ahi * rs));
+        }
+    row[tid] = o;
+    mmi_meet();
+}
+
+template <int NX, bool NORM>
+__global__ __launch_bounds__(512, 2) void k_gemm_xreg16(GemmArgs a) {
+    constexpr int RD = NX > 16 ? NX / 2 : NX;
+    MMI_SHARED __attribute__((aligned(16))) f32x4 red[2 * 8 * 64];
+    MMI_SHARED __attribute__((aligned(16))) u32x4 stage[512];            // NORM: the row [k-step][kq]; with RoPE the angles lie behind it
+    MMI_SHARED __attribute__((aligned(16))) float rope[MMI_XREG16_MAXROPE];
+    MMI_SHARED long off[16];
+    MMI_SHARED float part[8];
+    const int tid = (int)threadIdx.x, wave = mmi_uniform(tid >> 6), lane = tid & 63;
+    const int G = (int)gridDim.x, bid = (int)blockIdx.x;
+    const bool gate = a.epi == MMI_EPI_GATE;
+    const long units = gate ? (long)a.NT : 2L * a.NT;       // whole tiles, or row octets where the epilogue's features are weight rows (k_gemm_xlds)
+    const long u0 = (long)bid * units / G, u1 = (long)(bid + 1) * units / G;
+    const int t0 = gate ? (int)u0 : (int)(u0 >> 1), t1 = gate ? (int)u1 : (int)((u1 + 1) >> 1);
+    const int ntiles = u1 > u0 ? t1 - t0 : 0;
+    if (ntiles == 0) return;
+    auto oct_lo = [&](int t) { return gate ? 0 : (int)max(0L, u0 - 2L * (t0 + t)); };
+    auto oct_hi = [&](int t) { return gate ? 2 : (int)min(2L, u1 - 2L * (t0 + t)); };
+    // K range of this wave; entries past its end repeat a valid address and meet zeros
+    const int kper = (a.KSTEPS + 7) / 8;        // <= NX (checked by the launcher)
+    const int ks0 = min(a.KSTEPS, wave * kper), nks = min(a.KSTEPS, ks0 + kper) - ks0;
+    const int ksl = min(ks0, a.KSTEPS - 1), kl = nks > 0 ? nks - 1 : 0;
+    f32x4 rpre = {0.f, 0.f, 0.f, 0.f};
+    long opre = 0;
+    u32x4 xrow = {0u, 0u, 0u, 0u}, al = xrow;
+    if constexpr (NORM) {
+        const int at = min(tid * 8, a.D - 8);
+        xrow = a.xp[(at >> 5) * 64 + ((at >> 3) & 3) * 16];
+        al = *reinterpret_cast<const u32x4*>(a.alpha + at);
+    }
+    if (a.epi == MMI_EPI_ROPE_KV) {
+        rpre = *reinterpret_cast<const f32x4*>(a.rope + min(4 * tid, a.B * a.Dh - 4));
+        opre = a.offsets[min(tid, a.B - 1)];
+    }
+    auto wlane = [&](int t) {
+        const int ro = (lane >> 3) & 1, lo = oct_lo(t), hi = oct_hi(t);
+        return (unsigned)((ro >= lo && ro < hi) ? lane : ((lane & ~8) | (lo << 3)));
+    };
+    auto wbase = [&](int t) { return a.wp + ((long)(t0 + t) * a.KSTEPS + ksl) * 64; };
+    u32x4 w[RD], x[NX];
+    const u32x4* wp = wbase(0);
+    unsigned wl = wlane(0);
+#pragma unroll
+    for (int e = 0; e < RD; ++e) w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
+    mmi_sched_barrier();
+    if (a.epi == MMI_EPI_ROPE_KV) {
+        if (4 * tid < a.B * a.Dh) *reinterpret_cast<f32x4*>(rope + 4 * tid) = rpre;
+        if (tid < 16) off[tid] = opre;
+    }
+    if constexpr (NORM) {
+        mmi_xreg16_norm(a, stage, part, tid, wave, lane, xrow, al);
+#pragma unroll
+        for (int e = 0; e < NX; ++e) x[e] = stage[min((ksl + min(e, kl)) * 4 + (lane >> 4), 511)];
+    } else {
+#pragma unroll
+        for (int e = 0; e < NX; ++e) x[e] = (a.xp + (long)(ksl + min(e, kl)) * 64)[(unsigned)lane];
+    }
+    mmi_sched_barrier();
+    if (nks < NX) {                             // (full slices: the products of the first entries need not wait for the last ones)
+#pragma unroll
+        for (int e = 0; e < NX; ++e)
+            if (e >= nks) x[e] = u32x4{0u, 0u, 0u, 0u};
+    }
+    f32x4 acc;
+    auto tile = [&](const u32x4* next, unsigned nl, auto more_tag) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_tag)::value;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < NX; ++e) {
+            acc = mmi_mfma_bf16_16x16x32(w[e % RD], x[e], acc);
+            if (e + RD < NX) w[e % RD] = mmi_load_nt(wp + min(e + RD, kl) * 64 + wl);
+            else if (MORE) w[e % RD] = mmi_load_nt(next + min(e + RD - NX, kl) * 64 + nl);
+            if (e & 1) mmi_sched_barrier();
+        }
+    };
+#pragma unroll 1
+    for (int t = 0; t < ntiles; ++t) {
+        if (t + 1 < ntiles) {
+            const u32x4* next = wbase(t + 1);
+            const unsigned nl = wlane(t + 1);
+            tile(next, nl, MmiTrue{});
+            wp = next;
+            wl = nl;
+        } else {
+            tile(wp, wl, MmiFalse{});
+        }
+        // (the scratch of two tiles ago: its wave has passed the last tile's meeting since)
+        f32x4* sums = red + (t & 1) * 512;
+        sums[wave * 64 + lane] = acc;
+        mmi_meet();
+        if (wave != (t & 7)) continue;
+        if (gate) mmi_xreg16_epilogue<true>(a, rope, off, sums, lane, t0 + t, 0, 2);
+        else mmi_xreg16_epilogue<false>(a, rope, off, sums, lane, t0 + t, oct_lo(t), oct_hi(t));
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // RMSNorm (rms_norm_f32, eps 1e-8): y = (x.float() * (alpha.float() * rsqrt(eps + mean(x^2)))).to(bf16)
 // ------------------------------------------------------------------------------------------------
 // One block per session row b; thread t owns the 16-byte piece (8 features) t, t + blockDim, ... of the packed row

@@ -256,6 +256,17 @@ def test_gemm_with_activations_resident_in_registers(sim_lib, monkeypatch, B, gr
         assert any("[splitk]" in n for n, _ in lm_cases.int8_linears_bit_exact("cpu", sim_lib, tiny_lm_config(), B, seed=192 + B))
 
 
+@pytest.mark.parametrize("B,grid,kv", [(1, 3, "bf16"), (2, 5, "bf16"), (16, 7, "fp8"), (3, 64, "bf16")])
+def test_gemm_with_activations_resident_in_registers_on_the_16_row_tile(sim_lib, monkeypatch, B, grid, kv):
+    """k_gemm_xreg16 forced onto every linear of the tiny model that it can hold: one session and a full tile, shares of whole tiles and of single
+    row octets, more workgroups than tiles, waves without entries of their own, both rings."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_GEMM_REG", str(grid))
+    st = {}
+    lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), kv_cache_dtype=kv), seed=230 + B, B=B, S=2, stats=st)
+    assert st["xlds_launches"] >= 2 * (2 if B > 1 else 0) + 2
+
+
 def test_depformer_in_per_step_launches(sim_lib, monkeypatch):
     """The engine normally runs the dep_q `depformer_in` linears as one grouped GEMM and lets each sampler add its token's
     embedding row; depth widths that are not whole n-tiles fall back to one GEMM per micro-step with the embedding in its
