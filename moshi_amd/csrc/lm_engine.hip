@@ -520,6 +520,16 @@ int launch_xreg(hipStream_t s, const XregPlan& p, int T, int mt, const GemmArgs&
     return launch_xreg_v<2, 16, 8, 3>(s, p, a);
 }
 
+// k_gemm_xring16 for slices of 16 k-steps and more behind at most one workgroup per CU, bf16 on the 16-row tile: entries of its ring, 0 = another
+// kernel.  MMI_GEMM_RING: "0" = off, "2" = every such GEMM on 8 waves (tests on tiny shapes)
+int ring_entries(const GemmW& g, const GemmPlan& p, int mt, const GemmArgs& a) {
+    const char* e = getenv("MMI_GEMM_RING");
+    if (g.T != 16 || mt != 1 || a.wq != 0 || p.ksplit != 1 || a.osplit > 1 || a.epi == MMI_EPI_PARTIAL || a.epi == MMI_EPI_GATE || (e && e[0] == '0')) return 0;
+    const int kper = mmi_cdiv(g.KSTEPS, 8);
+    if (!(e && e[0] == '2') && (p.waves != 8 || kper < 16 || g.NT > 256)) return 0;
+    return kper <= 16 ? 16 : 22;
+}
+
 // k_gemm_xp_once (a wave's whole K-slice requested before its first MFMA) for the GEMMs k_gemm_xp would walk in three or more
 // dependent memory round trips although they are a latency chain, not a stream: bf16 weights behind at most 256 workgroups of 8
 // waves whose slice is longer than the two register buffers of k_gemm_xp (2 x 4 k-steps) and short enough for the registers -
@@ -605,6 +615,11 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
     } else if (xl.on) {
         lm->xlds_launches += 1;
         rc = mt == 1 ? launch_xlds<1>(s, xl, a) : launch_xlds<2>(s, xl, a);
+    } else if (const int rd = ring_entries(g, p, mt, a)) {
+        if (rd == 16) MMI_LAUNCH(k_gemm_xring16<16>, g.NT, 512, 0, s, a);
+        else MMI_LAUNCH(k_gemm_xring16<22>, g.NT, 512, 0, s, a);
+        MMI_CHECK_LAUNCH();
+        rc = MMI_OK;
     } else if (const int kmax = once_kmax(g, p, mt, a)) {
         rc = launch_once(s, g.T, mt, kmax, dim3(g.NT * (a.osplit > 1 ? a.osplit : 1), p.ksplit), a);
     } else {

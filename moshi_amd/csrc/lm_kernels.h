@@ -707,6 +707,48 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
     mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi);
 }
 
+// k_gemm_xp on the 16-row tile for LONG slices behind at most one workgroup per CU (the temporal out_proj and linear_out of up to 16 sessions): a
+// tile's activations are met once, so they pass through the registers like its weights, RD entries of both on their way in a ring - what one CU
+// streams is what it has under way, and the double buffer of k_gemm_xp stops asking while it multiplies.  Lanes of sessions that are not there
+// repeat the last one's address (one session: a quarter of the lines).  Same K partition, same k order, same reduction and epilogue: k_gemm_xp's bits.
+template <int RD>
+__global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a) {
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63, nt0 = (int)blockIdx.x;
+    const u32x4 pre = mmi_gemm_prefetch_addend<16, 1, 1>(a, nt0);
+    const int kper = (a.KSTEPS + 7) / 8, ks0 = min(a.KSTEPS, wave * kper), nks = min(a.KSTEPS, ks0 + kper) - ks0;
+    const int ksl = min(ks0, a.KSTEPS - 1), kl = nks > 0 ? nks - 1 : 0;
+    const u32x4* wp = a.wp + ((long)nt0 * a.KSTEPS + ksl) * 64;
+    const u32x4* xp = a.xp + (long)ksl * 64;
+    const unsigned wl = (unsigned)lane, xl = (unsigned)((lane & 48) + min(lane & 15, a.B - 1));
+    u32x4 w[RD], x[RD];
+#pragma unroll
+    for (int e = 0; e < RD; ++e) {
+        w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
+        x[e] = (xp + min(e, kl) * 64)[xl];
+    }
+    mmi_sched_barrier();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    int k = 0;
+#pragma unroll 1
+    for (; k + RD < nks; k += RD) {              // (past the slice: its last entry again)
+#pragma unroll
+        for (int e = 0; e < RD; ++e) {
+            acc = mmi_mfma_bf16_16x16x32(w[e], x[e], acc);
+            const int n = min(k + RD + e, kl);
+            w[e] = mmi_load_nt(wp + n * 64 + wl);
+            x[e] = (xp + n * 64)[xl];
+            mmi_sched_barrier();
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < RD; ++e)
+        if (k + e < nks) acc = mmi_mfma_bf16_16x16x32(w[e], x[e], acc);
+    float accv[1][1][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) accv[0][0][r] = acc[r];
+    mmi_gemm_epilogue<16, 1, 1, 8>(a, accv, wave, lane, nt0, pre, nullptr, 0, 2);
+}
+
 // ONE session: RMSNorm + a weight stream on the 16-row tile (the temporal in_proj and linear_in).  A workgroup's 512 threads normalise the row -
 // k_resid_rmsnorm's pieces, sums and roundings, so its bits - into LDS, with the wave's first two groups of weights on their way; the main loop takes its
 // activations from there, 16 bytes for all 16 columns of the tile (column 0 is the session).  The norm was a launch of 4.6 us in front of each, 64 per

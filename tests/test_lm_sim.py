@@ -267,6 +267,17 @@ def test_gemm_with_activations_resident_in_registers_on_the_16_row_tile(sim_lib,
     assert st["xlds_launches"] >= 2 * (2 if B > 1 else 0) + 2
 
 
+@pytest.mark.parametrize("B,hidden_scale", [(1, 4.125), (3, 4.125), (16, 4.125), (1, 135.0), (5, 270.0)])
+def test_gemm_whose_operands_pass_in_a_ring(sim_lib, monkeypatch, B, hidden_scale):
+    """k_gemm_xring16 forced onto every linear of the tiny model that it can hold: slices shorter than its ring, and linear_out of 23 and 45 k-steps per
+    wave (rounds of the ring that end inside it)."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_GEMM_RING", "2")
+    cfg = replace(tiny_lm_config(), hidden_scale=hidden_scale, num_layers=2 if hidden_scale < 100 else 1, dim=128 if hidden_scale < 100 else 64,
+                  num_heads=4 if hidden_scale < 100 else 2)
+    lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=260 + B, B=B, S=2)
+
+
 def test_depformer_in_per_step_launches(sim_lib, monkeypatch):
     """The engine normally runs the dep_q `depformer_in` linears as one grouped GEMM and lets each sampler add its token's
     embedding row; depth widths that are not whole n-tiles fall back to one GEMM per micro-step with the embedding in its
