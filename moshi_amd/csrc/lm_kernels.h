@@ -227,270 +227,211 @@ struct GemmArgs {
                             // that nobody writes), the epilogue writes only the owned 8-feature groups.  Not for gated epilogues.
 };
 
-// The residual (or embedding) vector the thread's FIRST epilogue task will add, requested before the weight stream starts
-// so that its latency is hidden behind the main loop instead of extending the epilogue.
-template <int TN, int MT, int NTW>
-__device__ __forceinline__ u32x4 mmi_gemm_prefetch_addend(const GemmArgs& a, int nt0) {
-    u32x4 pre = {0u, 0u, 0u, 0u};
-    if (a.epi != MMI_EPI_RESID && a.epi != MMI_EPI_EMB) return pre;
-    const int G = TN / 8;
-    const int q = (int)threadIdx.x;
-    if (q >= NTW * MT * G * TN) return pre;
-    const int bl = q % TN;
-    int rest = q / TN;
-    const int gi = rest % G;
-    rest /= G;
-    const int m = rest % MT, t = rest / MT;
-    const int nt = nt0 + t, b = m * TN + bl, n0 = nt * TN + 8 * gi;
-    if (nt >= a.NT || b >= a.B || n0 >= a.N) return pre;
-    if (a.epi == MMI_EPI_RESID) {
-        const uint16_t* rs = a.out_mode == MMI_OUT_PACKED ? a.resid + mmi_xp_index(TN, b, n0, a.out_ksteps) : a.resid + (long)b * a.out_ld + n0;
-        pre = *reinterpret_cast<const u32x4*>(rs);
+// ---- reduction across a workgroup's waves and epilogue, shared by the GEMM kernels ------------------------------------------------
+// One task = one lane = 4 consecutive features of one session, whose sums lie in one accumulator quad (MFMA C layout, top of this file).  32-row tile:
+// a batch tile is 4 waves of tasks (quad c of a lane: rows 8 c + 4 (lane >> 5) .. of the tile), 16-row tile: one wave (rows 4 (lane >> 4) ..).  8 features
+// per task, as it was, left 3 of 4 waves without any, and at a gated tile half the lanes of one to sum for and activate all of it; these launches
+// are dependent chains, so that the epilogue is as long as it takes.  A gated tile holds the gate rows in front of their value rows: value quads
+// go to the upper lanes.  Operands of a wave's first task (addend, scales, row absmax) are requested before the weights.
+// A step of one session (ring 1500 deep) 4312 -> 4095 us, of 32 6144 -> 6092, of 64 at int8 6462 -> 6311.
+struct MmiEpiPre { u32x2 add; f32x4 sc; float sx; };
+enum { MMI_TASK_GATE = 0, MMI_TASK_PACKED = 1, MMI_TASK_ROWS = 2 };
+struct MmiEpiTask { int m, c, from, b, f0; };
+__device__ __forceinline__ int mmi_task_kind(const GemmArgs& a) {
+    if (a.epi == MMI_EPI_GATE) return MMI_TASK_GATE;
+    return a.out_mode == MMI_OUT_PACKED && a.epi != MMI_EPI_PARTIAL && a.epi != MMI_EPI_ROPE_KV ? MMI_TASK_PACKED : MMI_TASK_ROWS;
+}
+// task of a lane in the tw-th wave of tasks: batch tile m, accumulator quad c of lane `from`, row b, first feature f0
+template <int TN>
+__device__ __forceinline__ MmiEpiTask mmi_epi_task(int kind, int tw, int lane, int nt) {
+    MmiEpiTask t;
+    if constexpr (TN == 32) {
+        t.m = tw >> 2;
+        if (kind == MMI_TASK_GATE) {             // lanes take consecutive rows of one quad: gate rows below, their value rows above
+            t.c = (tw & 1) + 2 * (lane >> 5);
+            t.from = 32 * ((tw >> 1) & 1) + (lane & 31);
+        } else if (kind == MMI_TASK_PACKED) {    // a wave of stores is 512 bytes in a row
+            t.c = tw & 3;
+            t.from = lane;
+        } else {                                 // 8 lanes take the 32 features of a row
+            t.c = (lane & 7) >> 1;
+            t.from = 32 * (lane & 1) + 8 * (tw & 3) + (lane >> 3);
+        }
+        t.b = t.m * 32 + (t.from & 31);
+        t.f0 = kind == MMI_TASK_GATE ? nt * 16 + 8 * (t.c & 1) + 4 * (t.from >> 5) : nt * 32 + 8 * t.c + 4 * (t.from >> 5);
     } else {
-        const int tk = a.tok[(long)(b % a.tok_rows) * a.tok_stride];
-        if (tk != -1) pre = *reinterpret_cast<const u32x4*>(a.emb + (long)(tk < 0 ? 0 : tk) * a.N + n0);   // lm_utils.py:102-124
+        t.m = tw;
+        t.c = lane >> 5;                         // (its octet: the only quad is 0)
+        t.from = lane;
+        t.b = t.m * 16 + (lane & 15);
+        t.f0 = kind == MMI_TASK_GATE ? nt * 8 + 4 * ((lane >> 4) & 1) : nt * 16 + 4 * (lane >> 4);
     }
-    return pre;
+    return t;
+}
+__device__ __forceinline__ u32x2 mmi_epi_addend(const GemmArgs& a, int TN, const MmiEpiTask& t) {
+    u32x2 v = {0u, 0u};
+    if (t.b >= a.B || t.f0 >= a.N) return v;
+    if (a.epi == MMI_EPI_RESID) {
+        v = *reinterpret_cast<const u32x2*>(a.out_mode == MMI_OUT_PACKED ? a.resid + mmi_xp_index(TN, t.b, t.f0, a.out_ksteps) : a.resid + (long)t.b * a.out_ld + t.f0);
+    } else if (a.epi == MMI_EPI_EMB) {
+        const int tk = a.tok[(long)(t.b % a.tok_rows) * a.tok_stride];
+        if (tk != -1) v = *reinterpret_cast<const u32x2*>(a.emb + (long)(tk < 0 ? 0 : tk) * a.N + t.f0);   // lm_utils.py:102-124
+    }
+    return v;
+}
+// dequantisation factors of a task's rows (WQ 1, 2: factor per weight row; 3: its raw absmax)
+template <int WQ>
+__device__ __forceinline__ f32x4 mmi_epi_scale(const GemmArgs& a, int kind, int lane, const MmiEpiTask& t) {
+    const float* sc = WQ == 3 ? a.wscb : a.wscale;
+    return *reinterpret_cast<const f32x4*>(sc + (kind == MMI_TASK_GATE && lane >= 32 ? a.gate_rows : 0) + min(t.f0, a.N - 4));
+}
+template <int TN, int MT, int WAVES, int WQ>
+__device__ __forceinline__ MmiEpiPre mmi_epi_prefetch(const GemmArgs& a, int wave, int lane, int nt) {
+    MmiEpiPre p = {{0u, 0u}, {0.f, 0.f, 0.f, 0.f}, 0.f};
+    if (wave >= (TN == 32 ? 4 : 1) * MT) return p;
+    const int kind = mmi_task_kind(a);
+    const MmiEpiTask t = mmi_epi_task<TN>(kind, wave, lane, nt);
+    if constexpr (WQ != 0) {
+        p.sc = mmi_epi_scale<WQ>(a, kind, lane, t);
+        if (WQ == 3 && a.sx) p.sx = a.sx[min(t.b, a.B - 1)];
+    }
+    if (a.epi == MMI_EPI_RESID || a.epi == MMI_EPI_EMB) p.add = mmi_epi_addend(a, TN, t);
+    return p;
 }
 
-// Split-K reduction across the workgroup's waves (fixed order -> deterministic) and the epilogue shared by the GEMM
-// kernels: one task = 8 consecutive output features of one session, written as one 16-byte vector.
-// EXT: the reduction scratch is handed in (`red_ext`, WAVES * NTW * MT * 64 * LS floats) instead of a static LDS array - for
-// kernels that own all of the LDS themselves (k_gemm_xlds).
-// g_lo / g_hi: only the tile's 8-feature groups [g_lo, g_hi) are written (k_gemm_xlds hands a tile's row octets to two
-// workgroups when that balances the chip: 384 in_proj tiles over 256 CUs = 6 octets each); default = the whole tile.
-template <int TN, int MT, int NTW, int WAVES, bool EXT = false>
-__device__ __forceinline__ void mmi_gemm_epilogue(const GemmArgs& a, float (&accv)[NTW][MT][TN == 32 ? 16 : 4], int wave, int lane,
-                                                  int nt0, u32x4 pre, float* red_ext = nullptr, int g_lo = 0, int g_hi = 4,
-                                                  const float* sx_local = nullptr) {
-    constexpr int R = TN == 32 ? 16 : 4;
-    // ---- split-K reduction across the block's waves (fixed order -> deterministic).  LDS layout [wave][tile][lane][LS]:
-    // a lane's accumulators are contiguous, so they go out and come back as 16-byte vectors; LS = 20 floats (80 B)
-    // spreads the 8 lanes of a ds_*_b128 group over all 32 banks.
-    constexpr int LS = R == 4 ? 4 : ((WAVES * NTW * MT * 64 * 20 * 4 <= 65536) ? 20 : 16);
-    constexpr int NE = NTW * MT * 64 * LS;
-    float* red;
+// The sums of one tile over the workgroup's waves (fixed order -> deterministic) and its epilogue.
+// EXT: the reduction scratch is handed in (`red_ext`, WAVES * MT * 64 * TN / 8 * 16 bytes at most) instead of a static LDS array - for kernels
+// that own all of the LDS themselves (k_gemm_xlds). g_lo / g_hi: only the tile's row octets [g_lo, g_hi) are written (tiles shared in
+// octets); default = the whole tile.  pre: of the first task, or null (read here).  sx_local: the rows' absmax in LDS.
+template <int TN, int MT, int WAVES, int WQ, bool EXT = false>
+__device__ __forceinline__ void mmi_gemm_epilogue(const GemmArgs& a, float (&accv)[MT][TN == 32 ? 16 : 4], int wave, int lane, int nt, const MmiEpiPre* pre,
+                                                  float* red_ext = nullptr, int g_lo = 0, int g_hi = 4, const float* sx_local = nullptr) {
+    constexpr int Q = TN == 32 ? 4 : 1;          // accumulator quads per lane
+    f32x4* red;
     if constexpr (EXT) {
-        red = red_ext;
+        red = reinterpret_cast<f32x4*>(red_ext);
     } else {
-        MMI_SHARED __attribute__((aligned(16))) float red_static[WAVES * NE];
+        MMI_SHARED __attribute__((aligned(16))) f32x4 red_static[WAVES * MT * Q * 64];
         red = red_static;
     }
+    const int kind = mmi_task_kind(a);
+    // (the lanes that take a row's features read from 8 planes: their places are exchanged by quad, so that they do not meet in the same banks)
+    auto place = [&](int quad, int l) { return TN == 32 && kind == MMI_TASK_ROWS ? l ^ (4 * quad + 2 * (l >> 5)) : l; };
 #pragma unroll
-    for (int t = 0; t < NTW; ++t)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int c = 0; c < R / 4; ++c) {
-                const f32x4 v4 = {accv[t][m][4 * c], accv[t][m][4 * c + 1], accv[t][m][4 * c + 2], accv[t][m][4 * c + 3]};
-                *reinterpret_cast<f32x4*>(&red[wave * NE + ((t * MT + m) * 64 + lane) * LS + 4 * c]) = v4;
-            }
+        for (int c = 0; c < Q; ++c)
+            red[((wave * MT + m) * Q + c) * 64 + place(c, lane)] = f32x4{accv[m][4 * c], accv[m][4 * c + 1], accv[m][4 * c + 2], accv[m][4 * c + 3]};
     __syncthreads();
-
-    // ---- epilogue: one task = 8 consecutive output features of one session
-    const bool gate = a.epi == MMI_EPI_GATE;
-    const bool iacc = a.sx || sx_local;              // int8 x int8: accv holds int32 bit patterns
-    const int rows_out = gate ? TN / 2 : TN;         // output features per tile
-    const int G = rows_out / 8;                      // feature groups per tile
-    const int ntasks = NTW * MT * G * TN;
-    for (int q = (int)threadIdx.x; q < ntasks; q += WAVES * 64) {
-        const int bl = q % TN;
-        int rest = q / TN;
-        const int gi = rest % G;
-        rest /= G;
-        const int m = rest % MT, t = rest / MT;
-        const int nt = nt0 + t;
-        const int b = m * TN + bl;
-        const int n0 = nt * rows_out + 8 * gi;
-        if (nt >= a.NT || b >= a.B || n0 >= a.N || gi < g_lo || gi >= g_hi) continue;
-        const float* rb = red + (t * MT + m) * 64 * LS;
-        // features 8*gi .. 8*gi+7 of the tile live in two lanes' accumulator quads (MFMA C layout, lm_kernels.h header):
-        //   T = 32: rows i = 8gi+e -> register (e&3) + 4gi of lane bl + 32*(e>>2);  gate partner rows i+16 -> registers + 8
-        //   T = 16: rows i = 8gi+e -> register e&3 of lane bl + 16*(2gi + (e>>2));  gate partner rows i+8 -> lanes + 32
-        int off_lo, off_hi, off2_lo, off2_hi;
-        if constexpr (TN == 32) {
-            off_lo = bl * LS + 4 * gi; off_hi = (bl + 32) * LS + 4 * gi;
-            off2_lo = off_lo + 8; off2_hi = off_hi + 8;
-        } else {
-            off_lo = (bl + 32 * gi) * LS; off_hi = (bl + 32 * gi + 16) * LS;
-            off2_lo = (bl + 32) * LS; off2_hi = (bl + 48) * LS;
-        }
-        float s[8], s2[8];
+#pragma unroll 1
+    for (int tw = wave; tw < Q * MT; tw += WAVES) {
+        const bool first = pre && tw == wave;
+        const MmiEpiTask t = mmi_epi_task<TN>(kind, tw, lane, nt);
+        const int quad = Q == 1 ? 0 : t.c, b = t.b, f0 = t.f0;
+        f32x4 part[WAVES];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { s[e] = 0.f; s2[e] = 0.f; }
-        if (iacc) {
+        for (int w = 0; w < WAVES; ++w) part[w] = red[((w * MT + t.m) * Q + quad) * 64 + place(quad, t.from)];
+        const bool mine = b < a.B && f0 < a.N && (kind == MMI_TASK_GATE || (t.c >= g_lo && t.c < g_hi));
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+        f32x4 sc = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (WQ != 0) sc = first ? pre->sc : mmi_epi_scale<WQ>(a, kind, lane, t);
+        if constexpr (WQ == 3) {
             // int8 x int8: the waves' accumulators are int32 bit patterns; their sum is the EXACT out32 of bitsandbytes'
             // int8_linear_matmul, converted to fp32 once (round to nearest even, like `out32 * float_tensor` in torch)
-            int si[8], si2[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { si[e] = 0; si2[e] = 0; }
+            int si[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int w = 0; w < WAVES; ++w) {
-                const i32x4 lo = *reinterpret_cast<const i32x4*>(rb + w * NE + off_lo);
-                const i32x4 hi = *reinterpret_cast<const i32x4*>(rb + w * NE + off_hi);
+                const i32x4 v = __builtin_bit_cast(i32x4, part[w]);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { si[e] += lo[e]; si[4 + e] += hi[e]; }
-            }
-            if (gate) {
-#pragma unroll
-                for (int w = 0; w < WAVES; ++w) {
-                    const i32x4 lo = *reinterpret_cast<const i32x4*>(rb + w * NE + off2_lo);
-                    const i32x4 hi = *reinterpret_cast<const i32x4*>(rb + w * NE + off2_hi);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { si2[e] += lo[e]; si2[4 + e] += hi[e]; }
-                }
+                for (int e = 0; e < 4; ++e) si[e] += v[e];
             }
             if (a.epi == MMI_EPI_PARTIAL) {      // split-K: the consumer (k_resid_rmsnorm) adds the integer partials, then dequantises
-                int* pd = reinterpret_cast<int*>(a.partial) + ((long)blockIdx.y * a.B + b) * a.N + n0;
-                *reinterpret_cast<i32x4*>(pd) = i32x4{si[0], si[1], si[2], si[3]};
-                *reinterpret_cast<i32x4*>(pd + 4) = i32x4{si[4], si[5], si[6], si[7]};
+                if (mine) *reinterpret_cast<i32x4*>(reinterpret_cast<int*>(a.partial) + ((long)blockIdx.y * a.B + b) * a.N + f0) = i32x4{si[0], si[1], si[2], si[3]};
                 continue;
             }
             // int8_mm_dequant: out32 * (SCA[b] * SCB[n]) * (1 / 127^2), fp32, in that order
-            const float sca = sx_local ? sx_local[m * TN + bl] : a.sx[b];      // sx_local: the kernel's own row absmax (LDS)
-            const f32x4 c0 = *reinterpret_cast<const f32x4*>(a.wscb + n0), c1 = *reinterpret_cast<const f32x4*>(a.wscb + n0 + 4);
+            const float sca = sx_local ? sx_local[b] : (first ? pre->sx : a.sx[min(b, a.B - 1)]);      // sx_local: the kernel's own row absmax (LDS)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                s[e] = mmi_i8_dequant(si[e], sca, c0[e]);
-                s[4 + e] = mmi_i8_dequant(si[4 + e], sca, c1[e]);
-            }
-            if (gate) {
-                const f32x4 g0 = *reinterpret_cast<const f32x4*>(a.wscb + a.gate_rows + n0), g1 = *reinterpret_cast<const f32x4*>(a.wscb + a.gate_rows + n0 + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s2[e] = mmi_i8_dequant(si2[e], sca, g0[e]);
-                    s2[4 + e] = mmi_i8_dequant(si2[4 + e], sca, g1[e]);
-                }
-            }
+            for (int e = 0; e < 4; ++e) s[e] = mmi_i8_dequant(si[e], sca, sc[e]);
         } else {
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(rb + w * NE + off_lo);
-            const f32x4 hi = *reinterpret_cast<const f32x4*>(rb + w * NE + off_hi);
+            for (int w = 0; w < WAVES; ++w)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { s[e] += lo[e]; s[4 + e] += hi[e]; }
-        }
-        if (gate) {
+                for (int e = 0; e < 4; ++e) s[e] += part[w][e];
+            if constexpr (WQ != 0)               // int8 weights, bf16 activations: y = (sum_k q x) * SCB / 127, per original weight row
 #pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const f32x4 lo = *reinterpret_cast<const f32x4*>(rb + w * NE + off2_lo);
-                const f32x4 hi = *reinterpret_cast<const f32x4*>(rb + w * NE + off2_hi);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { s2[e] += lo[e]; s2[4 + e] += hi[e]; }
+                for (int e = 0; e < 4; ++e) s[e] *= sc[e];
+            if (a.epi == MMI_EPI_PARTIAL) {
+                if (mine) *reinterpret_cast<f32x4*>(a.partial + ((long)blockIdx.y * a.B + b) * a.N + f0) = f32x4{s[0], s[1], s[2], s[3]};
+                continue;
             }
         }
-        }
-        if (a.wscale && !iacc) {   // int8 weights, bf16 activations: y = (sum_k q x) * SCB / 127, per original weight row
-            const f32x4 c0 = *reinterpret_cast<const f32x4*>(a.wscale + n0), c1 = *reinterpret_cast<const f32x4*>(a.wscale + n0 + 4);
+        if (kind == MMI_TASK_GATE) {
+            // features 0, 1 of the quad to the lower lanes, 2, 3 to the upper ones: (gate, value) pairs on one lane
+            mmi_swap32(s[0], s[2]);
+            mmi_swap32(s[1], s[3]);
+            if (!mine) continue;
+            float o[2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { s[e] *= c0[e]; s[4 + e] *= c1[e]; }
-            if (gate) {
-                const f32x4 g0 = *reinterpret_cast<const f32x4*>(a.wscale + a.gate_rows + n0), g1 = *reinterpret_cast<const f32x4*>(a.wscale + a.gate_rows + n0 + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { s2[e] *= g0[e]; s2[4 + e] *= g1[e]; }
+            for (int e = 0; e < 2; ++e) {
+                const float g = mmi_round_bf16(s[e]), u = mmi_round_bf16(s[2 + e]);
+                o[e] = mmi_round_bf16(g / (1.0f + expf(-g))) * u;          // F.silu on a bf16 tensor
             }
-        }
-        if (a.epi == MMI_EPI_PARTIAL) {
-            float* pd = a.partial + ((long)blockIdx.y * a.B + b) * a.N + n0;
-            f32x4 lo = {s[0], s[1], s[2], s[3]}, hi = {s[4], s[5], s[6], s[7]};
-            *reinterpret_cast<f32x4*>(pd) = lo;
-            *reinterpret_cast<f32x4*>(pd + 4) = hi;
+            const int n = f0 + 2 * (lane >> 5);
+            uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(TN, b, n, a.out_ksteps) : a.out + (long)b * a.out_ld + n;
+            *reinterpret_cast<uint32_t*>(dst) = mmi_pack_bf16x2(o[0], o[1]);
             continue;
         }
+        if (!mine) continue;
         if (a.epi == MMI_EPI_DEP_QKV0) {
             // in_proj of the depth transformer's FIRST micro-step: its attention sees one position, softmax over one score is
             // exactly 1, so the attention output IS v (1 * v / 1) - the epilogue writes k and v into position 0 of the frame's
             // cache (transformer.py:243-253) and v as out_proj's packed operand; q is not needed; no attention launch
-            const int HD = a.H * a.Dh;
-            const int sec = n0 / HD, hn = n0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
+            const int HD = a.H * a.Dh, sec = f0 / HD, hn = f0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
             if (sec == 0) continue;
-            u32x4 ov;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ov[e] = mmi_pack_bf16x2(s[2 * e], s[2 * e + 1]);      // nn.Linear output in bf16
-            uint16_t* cache = (sec == 1 ? a.kc : a.vc) + (((long)b * a.H + h) * a.cap) * a.Dh + d0;
-            *reinterpret_cast<u32x4*>(cache) = ov;
-            if (sec == 2) *reinterpret_cast<u32x4*>(a.out + mmi_xp_index(TN, b, hn, a.out_ksteps)) = ov;
+            const u32x2 ov = {mmi_pack_bf16x2(s[0], s[1]), mmi_pack_bf16x2(s[2], s[3])};      // nn.Linear output in bf16
+            *reinterpret_cast<u32x2*>((sec == 1 ? a.kc : a.vc) + (((long)b * a.H + h) * a.cap) * a.Dh + d0) = ov;
+            if (sec == 2) *reinterpret_cast<u32x2*>(a.out + mmi_xp_index(TN, b, hn, a.out_ksteps)) = ov;
             continue;
         }
         if (a.epi == MMI_EPI_ROPE_KV) {
-            const int HD = a.H * a.Dh;
-            const int sec = n0 / HD, hn = n0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
+            const int HD = a.H * a.Dh, sec = f0 / HD, hn = f0 - sec * HD, h = hn / a.Dh, d0 = hn - h * a.Dh;
             const long off = a.offsets[b];
-            float v8[8];
+            float v[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v8[e] = mmi_round_bf16(s[e]);          // in_proj output is a bf16 tensor
+            for (int e = 0; e < 4; ++e) v[e] = mmi_round_bf16(s[e]);          // in_proj output is a bf16 tensor
             if (sec < 2) {
-                const float* cs = a.rope + ((long)b * (a.Dh / 2) + d0 / 2) * 2;      // 4 (cos, sin) pairs = 32 contiguous bytes
-                const f32x4 cs0 = *reinterpret_cast<const f32x4*>(cs), cs1 = *reinterpret_cast<const f32x4*>(cs + 4);
-    #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float c = j < 2 ? cs0[2 * j] : cs1[2 * j - 4], sn = j < 2 ? cs0[2 * j + 1] : cs1[2 * j - 3];
-                    // mmi_rope_rotate = four multiplies, a subtract, an add as separate VALU instructions.  Written as
-                    // `re * c - im * sn` the compiler packs the four pairs into v_pk_mul_f32 / v_pk_add_f32 with op_sel swizzles,
-                    // one of them in place, and on gfx950 that sequence inside k_gemm_xp<32, 2, ..> (64 sessions) returned, now and
-                    // then, a stale last element for lanes 48-63 - q / k of 16 sessions wrong in one feature, a different one
-                    // from run to run (profiles/r05_logs/c5_trace_*.txt)
-                    const float re = v8[2 * j], im = v8[2 * j + 1];
-                    mmi_rope_rotate(re, im, c, sn, v8[2 * j], v8[2 * j + 1]);
+                const f32x4 cs = *reinterpret_cast<const f32x4*>(a.rope + ((long)b * (a.Dh / 2) + d0 / 2) * 2);      // two (cos, sin) pairs
+                // mmi_rope_rotate = four multiplies, a subtract, an add as separate VALU instructions.  Written as `re * c - im * sn` the
+                // compiler packed the pairs into v_pk_mul_f32 / v_pk_add_f32 with op_sel swizzles, one of them in place, and on gfx950 that
+                // sequence inside k_gemm_xp<32, 2, ..> (64 sessions) returned, now and then, a stale last element for lanes 48-63 - q / k of
+                // 16 sessions wrong in one feature, a different one from run to run (profiles/r05_logs/c5_trace_*.txt)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float re = v[2 * j], im = v[2 * j + 1];
+                    mmi_rope_rotate(re, im, cs[2 * j], cs[2 * j + 1], v[2 * j], v[2 * j + 1]);
                 }
             }
+            const long at = sec == 0 ? 0 : (((long)b * a.H + h) * a.cap + (int)(off % a.cap)) * a.Dh + d0;
             if (sec != 0 && a.kv8) {   // fp8 ring: the bf16 k / v values (k after RoPE, as the bf16 ring would hold them) -> e4m3
-                uint8_t* d8 = reinterpret_cast<uint8_t*>(sec == 1 ? a.kc : a.vc) + (((long)b * a.H + h) * a.cap + (int)(off % a.cap)) * a.Dh + d0;
-                u32x2 o8;
-                o8[0] = mmi_cvt_fp8x4(mmi_round_bf16(v8[0]), mmi_round_bf16(v8[1]), mmi_round_bf16(v8[2]), mmi_round_bf16(v8[3]));
-                o8[1] = mmi_cvt_fp8x4(mmi_round_bf16(v8[4]), mmi_round_bf16(v8[5]), mmi_round_bf16(v8[6]), mmi_round_bf16(v8[7]));
-                *reinterpret_cast<u32x2*>(d8) = o8;
+                *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(sec == 1 ? a.kc : a.vc) + at) =
+                    mmi_cvt_fp8x4(mmi_round_bf16(v[0]), mmi_round_bf16(v[1]), mmi_round_bf16(v[2]), mmi_round_bf16(v[3]));
                 continue;
             }
-            uint16_t* dst;
-            if (sec == 0) dst = a.qrot + (long)b * HD + hn;
-            else dst = (sec == 1 ? a.kc : a.vc) + (((long)b * a.H + h) * a.cap + (int)(off % a.cap)) * a.Dh + d0;
-            u32x4 ov;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ov[e] = mmi_pack_bf16x2(v8[2 * e], v8[2 * e + 1]);
-            *reinterpret_cast<u32x4*>(dst) = ov;
+            uint16_t* dst = sec == 0 ? a.qrot + (long)b * HD + hn : (sec == 1 ? a.kc : a.vc) + at;
+            *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(v[0], v[1]), mmi_pack_bf16x2(v[2], v[3])};
             continue;
         }
-        uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(TN, b, n0, a.out_ksteps)
-                                                     : a.out + (long)b * a.out_ld + n0;
-        float o[8];
-        if (gate) {
+        if (a.epi == MMI_EPI_RESID || a.epi == MMI_EPI_EMB) {
+            const u32x2 rv = first ? pre->add : mmi_epi_addend(a, TN, t);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float g = mmi_round_bf16(s[e]);
-                const float u = mmi_round_bf16(s2[e]);
-                const float act = mmi_round_bf16(g / (1.0f + expf(-g)));   // F.silu on a bf16 tensor
-                o[e] = act * u;
-            }
-        } else if (a.epi == MMI_EPI_RESID) {
-            const uint16_t* rs = a.out_mode == MMI_OUT_PACKED ? a.resid + mmi_xp_index(TN, b, n0, a.out_ksteps)
-                                                              : a.resid + (long)b * a.out_ld + n0;
-            const u32x4 rv = q == (int)threadIdx.x ? pre : *reinterpret_cast<const u32x4*>(rs);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            for (int e = 0; e < 4; ++e) {
                 const uint16_t h = (uint16_t)((e & 1) ? (rv[e >> 1] >> 16) : (rv[e >> 1] & 0xffffu));
-                o[e] = mmi_round_bf16(s[e]) + mmi_bf16_to_f32(h);           // x_orig + update
+                s[e] = mmi_round_bf16(s[e]) + mmi_bf16_to_f32(h);           // x_orig + update
             }
-        } else if (a.epi == MMI_EPI_EMB) {
-            u32x4 ev = pre;
-            if (q != (int)threadIdx.x) {
-                const int tk = a.tok[(long)(b % a.tok_rows) * a.tok_stride];
-                ev = u32x4{0u, 0u, 0u, 0u};
-                if (tk != -1) ev = *reinterpret_cast<const u32x4*>(a.emb + (long)(tk < 0 ? 0 : tk) * a.N + n0);   // lm_utils.py:102-124
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint16_t h = (uint16_t)((e & 1) ? (ev[e >> 1] >> 16) : (ev[e >> 1] & 0xffffu));
-                o[e] = mmi_round_bf16(s[e]) + mmi_bf16_to_f32(h);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = s[e];                         // nn.Linear output in bf16
         }
-        u32x4 ov;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ov[e] = mmi_pack_bf16x2(o[2 * e], o[2 * e + 1]);
-        *reinterpret_cast<u32x4*>(dst) = ov;
+        uint16_t* dst = a.out_mode == MMI_OUT_PACKED ? a.out + mmi_xp_index(TN, b, f0, a.out_ksteps) : a.out + (long)b * a.out_ld + f0;
+        *reinterpret_cast<u32x2*>(dst) = u32x2{mmi_pack_bf16x2(s[0], s[1]), mmi_pack_bf16x2(s[2], s[3])};
     }
 }
 
@@ -509,7 +450,7 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && MT == 1 && NTW == 1 && WQ 
     constexpr int XS = (WQ == 1 || WQ == 2) ? 2 : 1;   // activation fragments per weight entry
     typedef int iacc_t __attribute__((ext_vector_type(R)));
     typedef float acc_t __attribute__((ext_vector_type(R)));
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     // octet sharing (a.osplit > 1, NTW == 1): workgroup = (n-tile, part); part owns the 8-feature groups [g_lo, g_hi)
     const int os = (NTW == 1 && a.osplit > 1) ? a.osplit : 1;
     const int bx = (int)blockIdx.x / os, part = (int)blockIdx.x - bx * os;
@@ -519,7 +460,9 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && MT == 1 && NTW == 1 && WQ 
     // from the first owned octet instead
     const int ro = (lane >> 3) & (TN / 8 - 1);
     const int wlane = (ro >= g_lo && ro < g_hi) ? lane : ((lane & ~((TN / 8 - 1) << 3)) | (g_lo << 3));
-    const u32x4 pre = mmi_gemm_prefetch_addend<TN, MT, NTW>(a, nt0);
+    MmiEpiPre pre[NTW];
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) pre[t] = mmi_epi_prefetch<TN, MT, WAVES, WQ>(a, wave, lane, nt0 + t);
 
     // K range of this workgroup (gridDim.y > 1: split-K over workgroups), then of this wave
     const int kb_per = (a.KSTEPS + (int)gridDim.y - 1) / (int)gridDim.y;
@@ -639,16 +582,16 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && MT == 1 && NTW == 1 && WQ 
 #undef MMI_G_MMA8
 #undef MMI_G_MFMA
 #undef MMI_G_MFMA8
-    float accv[NTW][MT][R];
 #pragma unroll
-    for (int t = 0; t < NTW; ++t)
+    for (int t = 0; t < NTW; ++t) {
+        float accv[MT][R];                       // WQ == 3: the wave's int32 sums, as their bit patterns (summed as integers by the epilogue)
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                accv[t][m][r] = acc[t][m][r];      // WQ == 3: the wave's int32 sum, as its bit pattern (summed as integers by the epilogue)
-            }
-    mmi_gemm_epilogue<TN, MT, NTW, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi);
+            for (int r = 0; r < R; ++r) accv[m][r] = acc[t][m][r];
+        if (t) __syncthreads();
+        if (nt0 + t < a.NT) mmi_gemm_epilogue<TN, MT, WAVES, WQ>(a, accv, wave, lane, nt0 + t, &pre[t], nullptr, g_lo, g_hi);
+    }
 }
 
 // k_gemm_xp for GEMMs that are a LATENCY chain, not a stream (the depth transformer's linear_out: 5.8 MB behind 128 workgroups,
@@ -661,13 +604,13 @@ template <int TN, int MT, int WAVES, int KMAX>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
     constexpr int R = TN == 32 ? 16 : 4;
     typedef float acc_t __attribute__((ext_vector_type(R)));
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int os = a.osplit > 1 ? a.osplit : 1;
     const int nt0 = (int)blockIdx.x / os, part = (int)blockIdx.x - nt0 * os;
     const int g_lo = part * ((TN / 8) / os), g_hi = os > 1 ? g_lo + (TN / 8) / os : TN / 8;
     const int ro = (lane >> 3) & (TN / 8 - 1);
     const int wlane = (ro >= g_lo && ro < g_hi) ? lane : ((lane & ~((TN / 8 - 1) << 3)) | (g_lo << 3));
-    const u32x4 pre = mmi_gemm_prefetch_addend<TN, MT, 1>(a, nt0);
+    const MmiEpiPre pre = mmi_epi_prefetch<TN, MT, WAVES, 0>(a, wave, lane, nt0);
     const int kb_per = (a.KSTEPS + (int)gridDim.y - 1) / (int)gridDim.y;
     const int kb0 = min(a.KSTEPS, (int)blockIdx.y * kb_per), kb1 = min(a.KSTEPS, kb0 + kb_per);
     const int kper = (kb1 - kb0 + WAVES - 1) / WAVES;            // <= KMAX (checked by the launcher)
@@ -699,12 +642,12 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
             }
         }
     }
-    float accv[1][MT][R];
+    float accv[MT][R];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int r = 0; r < R; ++r) accv[0][m][r] = acc[m][r];
-    mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi);
+        for (int r = 0; r < R; ++r) accv[m][r] = acc[m][r];
+    mmi_gemm_epilogue<TN, MT, WAVES, 0>(a, accv, wave, lane, nt0, &pre, nullptr, g_lo, g_hi);
 }
 
 // k_gemm_xp on the 16-row tile for LONG slices behind at most one workgroup per CU (the temporal out_proj and linear_out of up to 16 sessions): a
@@ -714,7 +657,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
 template <int RD>
 __global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a) {
     const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63, nt0 = (int)blockIdx.x;
-    const u32x4 pre = mmi_gemm_prefetch_addend<16, 1, 1>(a, nt0);
+    const MmiEpiPre pre = mmi_epi_prefetch<16, 1, 8, 0>(a, wave, lane, nt0);
     const int kper = (a.KSTEPS + 7) / 8, ks0 = min(a.KSTEPS, wave * kper), nks = min(a.KSTEPS, ks0 + kper) - ks0;
     const int ksl = min(ks0, a.KSTEPS - 1), kl = nks > 0 ? nks - 1 : 0;
     const u32x4* wp = a.wp + ((long)nt0 * a.KSTEPS + ksl) * 64;
@@ -743,10 +686,10 @@ __global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a) {
 #pragma unroll
     for (int e = 0; e < RD; ++e)
         if (k + e < nks) acc = mmi_mfma_bf16_16x16x32(w[e], x[e], acc);
-    float accv[1][1][4];
+    float accv[1][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) accv[0][0][r] = acc[r];
-    mmi_gemm_epilogue<16, 1, 1, 8>(a, accv, wave, lane, nt0, pre, nullptr, 0, 2);
+    for (int r = 0; r < 4; ++r) accv[0][r] = acc[r];
+    mmi_gemm_epilogue<16, 1, 8, 0>(a, accv, wave, lane, nt0, &pre);
 }
 
 // ONE session: RMSNorm + a weight stream on the 16-row tile (the temporal in_proj and linear_in).  A workgroup's 512 threads normalise the row -
@@ -819,10 +762,10 @@ __global__ __launch_bounds__(512, 4) void k_gemm_norm_one(GemmArgs a) {
         k += 2 * U;
     }
     if (k < nks) mma(wA, k);
-    float accv[1][1][4];
+    float accv[1][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) accv[0][0][r] = acc[r];
-    mmi_gemm_epilogue<16, 1, 1, 8>(a, accv, wave, lane, nt0, u32x4{0u, 0u, 0u, 0u}, nullptr, 0, 2);
+    for (int r = 0; r < 4; ++r) accv[0][r] = acc[r];
+    mmi_gemm_epilogue<16, 1, 8, 0>(a, accv, wave, lane, nt0, nullptr);
 }
 
 // RMSNorm fused into the GEMM that consumes it (the depth transformer: norm1 -> in_proj, norm2 -> linear_in; rows of
@@ -839,7 +782,7 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && KMAX == 4 && WQ == 0) ? 4 
     constexpr int XS = WQ ? 2 : 1;
     constexpr int XMAX = KMAX * XS;                           // activation fragments per wave
     typedef float acc_t __attribute__((ext_vector_type(R)));
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int nt0 = (int)blockIdx.x;                          // one n-tile per workgroup (octet sharing of these GEMMs measured
     const int g_lo = 0, g_hi = TN / 8, wlane = lane;          // neutral, profiles/r02_logs/ab_osplit_norm*: not built in)
     const int kper = (a.KSTEPS + WAVES - 1) / WAVES;          // <= KMAX (checked by the launcher)
@@ -847,6 +790,7 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && KMAX == 4 && WQ == 0) ? 4 
     const int nks = min(a.KSTEPS, ks0 + kper) - ks0;
     const int kq = TN == 32 ? (lane >> 5) : (lane >> 4);
 
+    const MmiEpiPre pre = mmi_epi_prefetch<TN, MT, WAVES, WQ>(a, wave, lane, nt0);
     u32x4 wv[KMAX], xv[MT][XMAX], al[XMAX];
     const u32x4 zero = {0u, 0u, 0u, 0u};
     // every load is unconditional from a clamped (valid) address and masked afterwards: conditional loads would be
@@ -936,14 +880,12 @@ __global__ __launch_bounds__(WAVES * 64, (TN == 16 && KMAX == 4 && WQ == 0) ? 4 
             }
         }
     }
-    float accv[1][MT][R];
+    float accv[MT][R];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            accv[0][m][r] = acc[m][r];
-        }
-    mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0, u32x4{0u, 0u, 0u, 0u}, nullptr, g_lo, g_hi);
+        for (int r = 0; r < R; ++r) accv[m][r] = acc[m][r];
+    mmi_gemm_epilogue<TN, MT, WAVES, WQ>(a, accv, wave, lane, nt0, &pre, nullptr, g_lo, g_hi);
 }
 
 // int8 weights x int8 activations with the row quantisation INSIDE the GEMM (the depth transformer's linears, whose rows are
@@ -983,9 +925,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     constexpr int XMAX = 2 * KMAX;
     // batch tiles handled together: both while a lane's fragments of both fit its registers (short rows), else one after the other
     constexpr int MG = (MT * XMAX <= 16) ? MT : 1;
+    constexpr bool PRE = TN == 32 || KMAX <= 4;               // the epilogue's operands first (long slices on the 16-row tile leave no registers for them)
     typedef int iacc_t __attribute__((ext_vector_type(R)));
     typedef float facc_t __attribute__((ext_vector_type(R)));
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     // octet sharing as in k_gemm_xp (a.osplit > 1): N = 1024 linears have 32 n-tiles for 256 CUs; a workgroup = (tile, part) owns
     // TN / 8 / osplit of the tile's 8-row groups, the lanes of the other groups repeat an owned lane's weight address
     const int os = a.osplit > 1 ? a.osplit : 1;
@@ -997,9 +940,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     const int ks0 = min(a.KSTEPS, wave * kper);
     const int nks = min(a.KSTEPS, ks0 + kper) - ks0;
     const int kq = TN == 32 ? (lane >> 5) : (lane >> 4);
-    u32x4 pre[NTW];
+    MmiEpiPre pre[NTW];
 #pragma unroll
-    for (int t = 0; t < NTW; ++t) pre[t] = mmi_gemm_prefetch_addend<TN, MT, 1>(a, nt0 + t);
+    for (int t = 0; t < NTW; ++t)
+        if constexpr (PRE) pre[t] = mmi_epi_prefetch<TN, MT, WAVES, 3>(a, wave, lane, nt0 + t);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     const int ksl = min(ks0, a.KSTEPS - 1);
     u32x4 wv[NTW][KMAX];
@@ -1120,12 +1064,12 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
         if (t) __syncthreads();                              // the epilogue's scratch
-        float accv[1][MT][R];
+        float accv[MT][R];
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int r = 0; r < R; ++r) accv[0][m][r] = __builtin_bit_cast(facc_t, acc[t][m])[r];     // int32 bit patterns (see the epilogue)
-        mmi_gemm_epilogue<TN, MT, 1, WAVES>(a, accv, wave, lane, nt0 + t, pre[t], nullptr, g_lo, g_hi, sxl);
+            for (int r = 0; r < R; ++r) accv[m][r] = __builtin_bit_cast(facc_t, acc[t][m])[r];     // int32 bit patterns (see the epilogue)
+        if (nt0 + t < a.NT) mmi_gemm_epilogue<TN, MT, WAVES, 3>(a, accv, wave, lane, nt0 + t, PRE ? &pre[t] : nullptr, nullptr, g_lo, g_hi, sxl);
     }
 }
 
@@ -1270,12 +1214,12 @@ __global__ __launch_bounds__(512) void k_gemm_xlds(GemmArgs a) {
                     // the small test chunks are smaller than the scratch, which then sits behind both buffers
                     float* red = reinterpret_cast<float*>(XE * 16 >= 65536 ? xs + (nchunks & 1) * XE : xs + 2 * XE);
                     __syncthreads();            // the previous tile's output tasks are done with the scratch
-                    float accv[1][MT][16];
+                    float accv[MT][16];
 #pragma unroll
                     for (int m = 0; m < MT; ++m)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) accv[0][m][r] = acc[t][m][r];
-                    mmi_gemm_epilogue<32, MT, 1, 8, true>(a, accv, wave, lane, t0 + t, u32x4{0u, 0u, 0u, 0u}, red, oct_lo(t), oct_hi(t));
+                        for (int r = 0; r < 16; ++r) accv[m][r] = acc[t][m][r];
+                    mmi_gemm_epilogue<32, MT, 8, WQ, true>(a, accv, wave, lane, t0 + t, nullptr, red, oct_lo(t), oct_hi(t));
                 }
             }
         }
@@ -1294,12 +1238,12 @@ __global__ __launch_bounds__(512) void k_gemm_xlds(GemmArgs a) {
     for (int t = 0; t < NTMAX; ++t) {
         if (t < ntiles) {
             __syncthreads();                    // the chunk buffers / the previous tile's scratch are no longer read
-            float accv[1][MT][16];
+            float accv[MT][16];
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) accv[0][m][r] = acc[t][m][r];     // WQ == 3: int32 bit patterns (see the epilogue)
-            mmi_gemm_epilogue<32, MT, 1, 8, true>(a, accv, wave, lane, t0 + t, u32x4{0u, 0u, 0u, 0u}, red, oct_lo(t), oct_hi(t));
+                for (int r = 0; r < 16; ++r) accv[m][r] = acc[t][m][r];     // WQ == 3: int32 bit patterns (see the epilogue)
+            mmi_gemm_epilogue<32, MT, 8, WQ, true>(a, accv, wave, lane, t0 + t, nullptr, red, oct_lo(t), oct_hi(t));
         }
     }
 }
@@ -2701,7 +2645,7 @@ __device__ __forceinline__ u32x4 mmi_dep_attn8_wave(const DepAttnArgs& a, int b,
 
 template <int NW>
 __global__ __launch_bounds__(NW * 64) void k_dep_attn8(DepAttnArgs a) {
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int bh = (int)blockIdx.x * NW + wave;
     if (bh >= a.B * a.H) return;
     const int b = bh / a.H, h = bh - b * a.H;
@@ -2721,14 +2665,14 @@ template <int WAVES, int HPW, int BMAX>
 __global__ __launch_bounds__(WAVES * 64) void k_dep_attn_out_proj(GemmArgs a, DepAttnArgs d) {
     constexpr int TN = 16, R = 4, KPWMAX = 4;
     typedef float acc_t __attribute__((ext_vector_type(R)));
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int os = a.osplit > 1 ? a.osplit : 1;                     // octet sharing as in k_gemm_xp
     const int bx = (int)blockIdx.x / os, part = (int)blockIdx.x - bx * os;
     const int nt0 = bx;
     const int g_lo = part * ((TN / 8) / os), g_hi = os > 1 ? g_lo + (TN / 8) / os : TN / 8;
     const int ro = (lane >> 3) & (TN / 8 - 1);
     const int wlane = (ro >= g_lo && ro < g_hi) ? lane : ((lane & ~((TN / 8 - 1) << 3)) | (g_lo << 3));
-    const u32x4 pre = mmi_gemm_prefetch_addend<TN, 1, 1>(a, nt0);
+    const MmiEpiPre pre = mmi_epi_prefetch<TN, 1, WAVES, 0>(a, wave, lane, nt0);
     const int kper = (a.KSTEPS + WAVES - 1) / WAVES;                // <= KPWMAX, kper * 32 a multiple of Dh (launcher)
     const int ks0 = min(a.KSTEPS, wave * kper);
     const int nks = min(a.KSTEPS, ks0 + kper) - ks0;
@@ -2777,10 +2721,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_dep_attn_out_proj(GemmArgs a, De
         const u32x4 xv = (u < nks && (lane & 15) < d.B) ? xs[wave][u][lane] : zero;
         if (u < nks) acc = mmi_mfma_bf16_16x16x32(wv[u], xv, acc);
     }
-    float accv[1][1][R];
+    float accv[1][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) accv[0][0][r] = acc[r];
-    mmi_gemm_epilogue<TN, 1, 1, WAVES>(a, accv, wave, lane, nt0, pre, nullptr, g_lo, g_hi);
+    for (int r = 0; r < R; ++r) accv[0][r] = acc[r];
+    mmi_gemm_epilogue<TN, 1, WAVES, 0>(a, accv, wave, lane, nt0, &pre, nullptr, g_lo, g_hi);
 }
 
 // ------------------------------------------------------------------------------------------------
