@@ -732,6 +732,23 @@ Pending add_gemm_resid(mmi_lm* lm, const GemmW& g, const uint16_t* in, uint16_t*
     return pd;
 }
 
+// a row in `pieces` rounds of 16 bytes per thread, as few threads as that takes
+int norm_threads(int D, int pieces) { return mmi_cdiv(mmi_cdiv(D / 8, pieces), 64) * 64; }
+int launch_resid_rmsnorm(hipStream_t s, int rows, uint16_t* x, const float* partial, int P, const uint16_t* alpha, uint16_t* y, int D, int T, int ksteps, uint8_t* yq, float* sx,
+                         const float* psx, const float* pscb) {
+    if (D <= 8 * 1024) MMI_LAUNCH(k_resid_rmsnorm<1>, rows, norm_threads(D, 1), 0, s, x, partial, P, rows, alpha, y, D, T, ksteps, 1e-8f, yq, sx, psx, pscb);
+    else MMI_LAUNCH(k_resid_rmsnorm<MMI_NORM_MAXP>, rows, 1024, 0, s, x, partial, P, rows, alpha, y, D, T, ksteps, 1e-8f, yq, sx, psx, pscb);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
+int launch_quant_rows(hipStream_t s, int rows, const uint16_t* x, int D, int T, int ksteps, uint8_t* xq, float* sx) {
+    if (D <= 8 * 1024) MMI_LAUNCH(k_quant_rows_i8<1>, rows, norm_threads(D, 1), 0, s, x, rows, D, T, ksteps, xq, sx);
+    else if (D <= 2 * 8 * 1024) MMI_LAUNCH(k_quant_rows_i8<2>, rows, norm_threads(D, 2), 0, s, x, rows, D, T, ksteps, xq, sx);
+    else MMI_LAUNCH(k_quant_rows_i8<MMI_NORM_MAXP>, rows, 1024, 0, s, x, rows, D, T, ksteps, xq, sx);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
+
 // x (+= the P pending split-K partials), y = rms_norm(x) * alpha
 // yq / sx: also store the row quantised row-wise to int8 (+ its absmax) for the int8 linears that read it (lm->act8)
 void add_resid_rmsnorm(mmi_lm* lm, uint16_t* x, Pending pd, const uint16_t* alpha, uint16_t* y, int D, uint8_t* yq = nullptr, float* sx = nullptr,
@@ -741,11 +758,7 @@ void add_resid_rmsnorm(mmi_lm* lm, uint16_t* x, Pending pd, const uint16_t* alph
     const int P = pd.P;
     const float *psx = pd.sx, *pscb = pd.scb;
     lm->prog.add([=](hipStream_t s) {
-        int nth = mmi_cdiv(D / 8, 64) * 64;            // one 16-byte piece per thread where the row allows it
-        if (nth > 1024) nth = 1024;
-        MMI_LAUNCH(k_resid_rmsnorm, B, nth, 0, s, x, partial, P, B, alpha, y, D, T, ksteps, 1e-8f, yq, sx, psx, pscb);
-        MMI_CHECK_LAUNCH();
-        return (int)MMI_OK;
+        return launch_resid_rmsnorm(s, B, x, partial, P, alpha, y, D, T, ksteps, yq, sx, psx, pscb);
     });
 }
 
@@ -900,11 +913,7 @@ int launch_norm_one(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, const
 void add_quant_rows(mmi_lm* lm, const uint16_t* xp, uint8_t* xq, float* sx, int features, int tile = 0) {
     const int B = lm->batch, T = tile ? tile : lm->T, ksteps = packed_ksteps_t(lm, T, features);
     lm->prog.add([=](hipStream_t s) {
-        int nth = mmi_cdiv(features / 8, 64) * 64;
-        if (nth > 1024) nth = 1024;
-        MMI_LAUNCH(k_quant_rows_i8, B, nth, 0, s, xp, B, features, T, ksteps, xq, sx);
-        MMI_CHECK_LAUNCH();
-        return (int)MMI_OK;
+        return launch_quant_rows(s, B, xp, features, T, ksteps, xq, sx);
     });
 }
 
@@ -2054,7 +2063,6 @@ extern "C" int mmi_lm_debug_linear(mmi_lm* lm, const char* weight_name, const ch
     hipStream_t s = (hipStream_t)stream;
     const int T = g.T, mt = mmi_cdiv(rows, T), KS = mmi_kstep(T);
     const int K = g.K, N = g.N, kin = packed_ksteps_t(lm, T, K), kout = packed_ksteps_t(lm, T, N);
-    const int nthK = [&] { int n = mmi_cdiv(K / 8, 64) * 64; return n > 1024 ? 1024 : n; }();
     MmiArena A;
     uint16_t *xp = nullptr, *yp = nullptr, *xres = nullptr, *zeros = nullptr, *outp = (uint16_t*)out_bf16;
     uint8_t* xq = nullptr;
@@ -2086,14 +2094,11 @@ extern "C" int mmi_lm_debug_linear(mmi_lm* lm, const char* weight_name, const ch
     a.out_mode = MMI_OUT_ROWMAJOR; a.out_ld = N; a.out_ksteps = kout;
     int rc = MMI_OK;
     if (path == MMI_DBG_NORM) {                // the norm launch of the step: y (+ its int8 copy) = rms_norm(x) * alpha
-        MMI_LAUNCH(k_resid_rmsnorm, rows, nthK, 0, s, xp, (const float*)nullptr, 0, rows, alpha, yp, K, T, kin, 1e-8f,
-                   a8 ? xq : (uint8_t*)nullptr, a8 ? sx : (float*)nullptr, (const float*)nullptr, (const float*)nullptr);
-        MMI_DBG_LAUNCHED();
+        if ((rc = launch_resid_rmsnorm(s, rows, xp, nullptr, 0, alpha, yp, K, T, kin, a8 ? xq : nullptr, a8 ? sx : nullptr, nullptr, nullptr))) return done(rc);
         operand = yp;
         if (norm_out) MMI_LAUNCH(k_unpack_rows, mmi_cdiv(rows * K, 256), 256, 0, s, (const uint16_t*)yp, rows, K, (uint16_t*)norm_out, T, kin);
     } else if (a8 && (path == MMI_DBG_PLAIN || path == MMI_DBG_SPLITK)) {
-        MMI_LAUNCH(k_quant_rows_i8, rows, nthK, 0, s, (const uint16_t*)xp, rows, K, T, kin, xq, sx);
-        MMI_DBG_LAUNCHED();
+        if ((rc = launch_quant_rows(s, rows, xp, K, T, kin, xq, sx))) return done(rc);
     }
     if (path == MMI_DBG_PLAIN || path == MMI_DBG_NORM || path == MMI_DBG_SPLITK) {
         a.xp = reinterpret_cast<const u32x4*>(operand);
@@ -2109,12 +2114,10 @@ extern "C" int mmi_lm_debug_linear(mmi_lm* lm, const char* weight_name, const ch
         rc = launch_gemm(lm, s, g, a, false);
         if (rc) return done(rc);
         if (path == MMI_DBG_SPLITK) {          // the fold of the next norm launch: x (= 0) + bf16(sum of the partials)
-            const int nthN = [&] { int n = mmi_cdiv(N / 8, 64) * 64; return n > 1024 ? 1024 : n; }();
             if (N > 8 * 1024 * MMI_NORM_MAXP) return done(mmi_fail(MMI_ERR_UNSUPPORTED, "row too long for the norm kernel"));
             uint16_t* ytmp = nullptr;
             if (A.alloc(&ytmp, oelems) != hipSuccess) return done(mmi_fail(MMI_ERR_HIP, "out of device memory"));
-            MMI_LAUNCH(k_resid_rmsnorm, rows, nthN, 0, s, xres, (const float*)partial, pd.P, rows, (const uint16_t*)zeros, ytmp, N, T, kout, 1e-8f,
-                       (uint8_t*)nullptr, (float*)nullptr, pd.sx, pd.scb);
+            if ((rc = launch_resid_rmsnorm(s, rows, xres, partial, pd.P, zeros, ytmp, N, T, kout, nullptr, nullptr, pd.sx, pd.scb))) return done(rc);
             MMI_LAUNCH(k_unpack_rows, mmi_cdiv(rows * N, 256), 256, 0, s, (const uint16_t*)xres, rows, N, outp, T, kout);
             MMI_DBG_LAUNCHED();
         }

@@ -30,7 +30,7 @@
 // A GEMM epilogue writes its result straight into the packed layout of the GEMM that consumes it.
 MMI_HD long mmi_xp_index(int T, int b, int k, int ksteps) {
     const int sh = T == 32 ? 4 : 5;                 // log2(k-step)
-    const int mt = b / T, bl = b - mt * T;
+    const int mt = b >> (T == 32 ? 5 : 4), bl = b & (T - 1);
     const int ks = k >> sh, kq = (k >> 3) & ((1 << (sh - 3)) - 1), e = k & 7;
     return ((((long)mt * ksteps + ks) * 64) + kq * T + bl) * 8 + e;
 }
@@ -1696,27 +1696,69 @@ __global__ __launch_bounds__(512, 2) void k_gemm_xreg16(GemmArgs a) {
 // P > 0: first finish the preceding split-K GEMM (out_proj / linear_out) and its residual connection,
 //        x <- x + bf16(sum_p partial[p][b][:])      (transformer.py:739-741,772-776: x_orig + update, bf16 tensors)
 // then   y <- rms_norm_f32(x) * alpha               (transformer.py:45-58)
+// A dependent launch of a few rows: what it costs is its chain.  So everything it reads is requested at once (the scales, cold, were asked for behind
+// the partial sums), sums over a wave stay in registers (the order of an exchange over 32, 16 .. 1, without six trips through LDS), a
+// row's place takes shifts (it took two 64-bit divisions).  64 rows of 4096, us per launch before / here: with int8 sums and copy 7.5 / 6.9.
 #define MMI_NORM_MAXP 4      // pieces per thread kept in registers (D <= 8 * 1024 * MMI_NORM_MAXP)
+// place of piece i of row b in the int8 operand Xq[mt][kp][lane][16]: the bytes of k-steps 2 kp and 2 kp + 1
+__device__ __forceinline__ long mmi_xq_index(int T, int b, int i, int ksteps) {
+    const int ks = i >> (T == 32 ? 4 : 5), kq = (i >> 3) & (T == 32 ? 1 : 3);
+    return (((long)(b >> (T == 32 ? 5 : 4)) * (ksteps >> 1) + (ks >> 1)) * 64 + kq * T + (b & (T - 1))) * 16 + (ks & 1) * 8;
+}
+// sum / maximum of the waves' values (at most 16 waves; in rising order), every thread gets it
+__device__ __forceinline__ float mmi_block_sum(float x, float* red, int wave, int lane, int waves) {
+    if (lane == 0) red[wave] = x;
+    __syncthreads();
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) t += w < waves ? red[w] : 0.f;
+    return t;
+}
+__device__ __forceinline__ float mmi_block_max(float x, float* red, int wave, int lane, int waves) {       // (not negative)
+    if (lane == 0) red[wave] = x;
+    __syncthreads();
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) t = fmaxf(t, w < waves ? red[w] : 0.f);
+    return t;
+}
 // yq != null (int8 activations): the normalised row is also stored quantised row-wise for the int8 linears that read it -
 // Xq[mt][kp][lane][16] (the bytes of k-steps 2 kp and 2 kp + 1) and sx[b] = its absmax (bitsandbytes' CA / SCA).
+template <int MAXP>
 __global__ __launch_bounds__(1024) void k_resid_rmsnorm(uint16_t* __restrict__ x, const float* __restrict__ partial, int P,
                                                         int B, const uint16_t* __restrict__ alpha, uint16_t* __restrict__ y,
-                                                        int D, int T, int ksteps, float eps, uint8_t* __restrict__ yq = nullptr,
-                                                        float* __restrict__ sx = nullptr, const float* __restrict__ psx = nullptr,
-                                                        const float* __restrict__ pscb = nullptr) {
+                                                        int D, int T, int ksteps, float eps, uint8_t* __restrict__ yq,
+                                                        float* __restrict__ sx, const float* __restrict__ psx,
+                                                        const float* __restrict__ pscb) {
     // psx / pscb != null: the pending GEMM was int8 x int8 - its partials are int32 sums (the exact out32 once added), and the
     // dequantisation out32 * (SCA[b] * SCB[n]) / 127^2 happens here (psx = the absmax of that GEMM's input rows, pscb = its SCB)
-    const int b = blockIdx.x, tid = threadIdx.x, nth = blockDim.x;
-    float f[MMI_NORM_MAXP][8];
-    u32x4 al[MMI_NORM_MAXP];
+    const int b = blockIdx.x, tid = threadIdx.x, nth = blockDim.x, wave = mmi_uniform(tid >> 6), lane = tid & 63, waves = (nth + 63) / 64;
+    MMI_SHARED float red[2][16];
+    float f[MAXP][8];
+    u32x4 al[MAXP];
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < MMI_NORM_MAXP; ++j) {
+    for (int j = 0; j < MAXP; ++j) {
         const int i = (tid + j * nth) * 8;
-        if (i >= D) break;
+        if (i >= D) continue;
         const long at = mmi_xp_index(T, b, i, ksteps);
         u32x4 v = *reinterpret_cast<const u32x4*>(x + at);
         al[j] = *reinterpret_cast<const u32x4*>(alpha + i);
+        f32x4 plo[4], phi[4], c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;      // P <= 4; unconditional (clamped) loads, all in flight
+        float sca = 0.f;
+        if (P > 0) {
+            if (psx) {
+                c0 = *reinterpret_cast<const f32x4*>(pscb + i);
+                c1 = *reinterpret_cast<const f32x4*>(pscb + i + 4);
+                sca = psx[b];
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float* pp = partial + ((long)min(p, P - 1) * B + b) * D + i;
+                plo[p] = *reinterpret_cast<const f32x4*>(pp);
+                phi[p] = *reinterpret_cast<const f32x4*>(pp + 4);
+            }
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             f[j][2 * q] = mmi_bf16_to_f32((uint16_t)(v[q] & 0xffffu));
@@ -1724,38 +1766,27 @@ __global__ __launch_bounds__(1024) void k_resid_rmsnorm(uint16_t* __restrict__ x
         }
         if (P > 0) {
             float u[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) u[e] = 0.f;
-            f32x4 plo[4], phi[4];                                  // P <= 4; unconditional (clamped) loads, all in flight
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const float* pp = partial + ((long)min(p, P - 1) * B + b) * D + i;
-                plo[p] = *reinterpret_cast<const f32x4*>(pp);
-                phi[p] = *reinterpret_cast<const f32x4*>(pp + 4);
-            }
             if (psx) {
                 int si[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) si[e] = 0;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    if (p < P) {
-                        const i32x4 ilo = __builtin_bit_cast(i32x4, plo[p]), ihi = __builtin_bit_cast(i32x4, phi[p]);   // (whole vectors:
+                    const i32x4 ilo = __builtin_bit_cast(i32x4, plo[p]), ihi = __builtin_bit_cast(i32x4, phi[p]);   // (whole vectors:
 #pragma unroll                                                                                                      // an element-wise
-                        for (int e = 0; e < 4; ++e) { si[e] += ilo[e]; si[4 + e] += ihi[e]; }                            // bit_cast is not)
-                    }
+                    for (int e = 0; e < 4; ++e) { si[e] += p < P ? ilo[e] : 0; si[4 + e] += p < P ? ihi[e] : 0; }    // bit_cast is not)
                 }
-                const float sca = psx[b];
-                const f32x4 c0 = *reinterpret_cast<const f32x4*>(pscb + i), c1 = *reinterpret_cast<const f32x4*>(pscb + i + 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) { u[e] = mmi_i8_dequant(si[e], sca, c0[e]); u[4 + e] = mmi_i8_dequant(si[4 + e], sca, c1[e]); }
             } else {
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const float on = p < P ? 1.f : 0.f;                // exact: x*1 = x, finite x*0 = 0
+                for (int e = 0; e < 8; ++e) u[e] = 0.f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { u[e] += plo[p][e] * on; u[4 + e] += phi[p][e] * on; }
-            }
+                for (int p = 0; p < 4; ++p) {
+                    const float on = p < P ? 1.f : 0.f;                // exact: x*1 = x, finite x*0 = 0
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { u[e] += plo[p][e] * on; u[4 + e] += phi[p][e] * on; }
+                }
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[j][e] = mmi_round_bf16(mmi_round_bf16(u[e]) + f[j][e]);
@@ -1766,20 +1797,13 @@ __global__ __launch_bounds__(1024) void k_resid_rmsnorm(uint16_t* __restrict__ x
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += f[j][e] * f[j][e];
     }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) ss += mmi_shfl_xor(ss, m);
-    MMI_SHARED float red[16];
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    float tot = 0.f;
-    for (int w = 0; w < (nth + 63) / 64; ++w) tot += red[w];
-    const float rs = mmi_rsqrtf(eps + tot / (float)D);
-    u32x4 ov[MMI_NORM_MAXP];
+    const float rs = mmi_rsqrtf(eps + mmi_block_sum(mmi_wave_sum_down(ss), red[0], wave, lane, waves) / (float)D);
+    u32x4 ov[MAXP];
     float am = 0.f;
 #pragma unroll
-    for (int j = 0; j < MMI_NORM_MAXP; ++j) {
+    for (int j = 0; j < MAXP; ++j) {
         const int i = (tid + j * nth) * 8;
-        if (i >= D) break;
+        if (i >= D) continue;
         u32x4 o;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -1792,62 +1816,41 @@ __global__ __launch_bounds__(1024) void k_resid_rmsnorm(uint16_t* __restrict__ x
     }
     if (!yq) return;
     // ---- row-wise int8 copy of the normalised row
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) am = fmaxf(am, mmi_shfl_xor(am, m));
-    MMI_SHARED float redm[16];
-    if ((tid & 63) == 0) redm[tid >> 6] = am;
-    __syncthreads();
-    float sca = 0.f;
-    for (int w = 0; w < (nth + 63) / 64; ++w) sca = fmaxf(sca, redm[w]);
+    const float sca = mmi_block_max(mmi_wave_max_f32(am), red[1], wave, lane, waves);
     if (tid == 0) sx[b] = sca;
     const float scale = mmi_i8_scale(sca);
 #pragma unroll
-    for (int j = 0; j < MMI_NORM_MAXP; ++j) {
+    for (int j = 0; j < MAXP; ++j) {
         const int i = (tid + j * nth) * 8;
-        if (i >= D) break;
-        const long at = mmi_xp_index(T, b, i, ksteps);            // bf16 element index of the piece: fragment (mt * ksteps + ks), lane
-        const long frag = at >> 9;
-        const int ln = (int)((at >> 3) & 63);
-        const long mt = frag / ksteps;
-        const int ks = (int)(frag - mt * ksteps);
-        *reinterpret_cast<u32x2*>(yq + ((mt * (ksteps >> 1) + (ks >> 1)) * 64 + ln) * 16 + (ks & 1) * 8) = mmi_quant_i8x8(ov[j], scale);
+        if (i < D) *reinterpret_cast<u32x2*>(yq + mmi_xq_index(T, b, i, ksteps)) = mmi_quant_i8x8(ov[j], scale);
     }
 }
 
 // A packed bf16 tensor [B][D] -> its row-wise int8 copy Xq[mt][kp][lane][16] + the rows' absmax sx[b] (bitsandbytes'
 // int8_vectorwise_quant), for the int8 linears whose input is written by MANY workgroups (the temporal attention output, the
 // gated FFN tensor): one workgroup per row holds the row in registers (as the norm kernel does), reduces the absmax, converts.
+// 64 rows, us per launch before / here: 4096 features 5.4 / 4.9
+template <int MAXP>
 __global__ __launch_bounds__(1024) void k_quant_rows_i8(const uint16_t* __restrict__ x, int B, int D, int T, int ksteps,
                                                         uint8_t* __restrict__ xq, float* __restrict__ sx) {
-    const int b = blockIdx.x, tid = threadIdx.x, nth = blockDim.x;
-    u32x4 v[MMI_NORM_MAXP];
+    const int b = blockIdx.x, tid = threadIdx.x, nth = blockDim.x, wave = mmi_uniform(tid >> 6), lane = tid & 63;
+    MMI_SHARED float red[16];
+    u32x4 v[MAXP];
     float am = 0.f;
 #pragma unroll
-    for (int j = 0; j < MMI_NORM_MAXP; ++j) {
-        const int i = (tid + j * nth) * 8;
-        if (i >= D) break;
+    for (int j = 0; j < MAXP; ++j) {             // (pieces past the row: its last one again)
+        const int i = min((tid + j * nth) * 8, D - 8);
         v[j] = *reinterpret_cast<const u32x4*>(x + mmi_xp_index(T, b, i, ksteps));
-        am = fmaxf(am, mmi_absmax_bf16x8(v[j]));
     }
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) am = fmaxf(am, mmi_shfl_xor(am, m));
-    MMI_SHARED float redm[16];
-    if ((tid & 63) == 0) redm[tid >> 6] = am;
-    __syncthreads();
-    float sca = 0.f;
-    for (int w = 0; w < (nth + 63) / 64; ++w) sca = fmaxf(sca, redm[w]);
+    for (int j = 0; j < MAXP; ++j) am = fmaxf(am, mmi_absmax_bf16x8(v[j]));
+    const float sca = mmi_block_max(mmi_wave_max_f32(am), red, wave, lane, (nth + 63) / 64);
     if (tid == 0) sx[b] = sca;
     const float scale = mmi_i8_scale(sca);
 #pragma unroll
-    for (int j = 0; j < MMI_NORM_MAXP; ++j) {
+    for (int j = 0; j < MAXP; ++j) {
         const int i = (tid + j * nth) * 8;
-        if (i >= D) break;
-        const long at = mmi_xp_index(T, b, i, ksteps);
-        const long frag = at >> 9;
-        const int ln = (int)((at >> 3) & 63);
-        const long mt = frag / ksteps;
-        const int ks = (int)(frag - mt * ksteps);
-        *reinterpret_cast<u32x2*>(xq + ((mt * (ksteps >> 1) + (ks >> 1)) * 64 + ln) * 16 + (ks & 1) * 8) = mmi_quant_i8x8(v[j], scale);
+        if (i < D) *reinterpret_cast<u32x2*>(xq + mmi_xq_index(T, b, i, ksteps)) = mmi_quant_i8x8(v[j], scale);
     }
 }
 

@@ -75,6 +75,16 @@ __device__ __forceinline__ float mmi_row_sum(float x) {
     x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xf, 0xf, true));
     return x;
 }
+// sum over the whole wave in the order of an exchange over distances 32, 16, 8, 4, 2, 1, bit for bit; every lane gets it
+__device__ __forceinline__ float mmi_wave_sum_down(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const unsigned a0 = a[0], a1 = a[1];
+    const unsigned w = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, a0) + __builtin_bit_cast(float, a1));
+    const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    const unsigned b0 = b[0], b1 = b[1];
+    return mmi_row_sum(__builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1));
+}
 // maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48, every one of them gets it: two exchanges of rows between registers
 // (v_permlane16_swap, v_permlane32_swap: a few cycles; the same steps through the LDS crossbar wait some 120 cycles each)
 __device__ __forceinline__ float mmi_rows_max(float x) {

@@ -327,6 +327,10 @@ inline float mmi_row_sum(float x) {
     for (int m = 8; m >= 1; m >>= 1) x += mmi_shfl_xor(x, m);
     return x;
 }
+inline float mmi_wave_sum_down(float x) {
+    for (int m = 32; m >= 1; m >>= 1) x += mmi_shfl_xor(x, m);
+    return x;
+}
 inline float mmi_rows_max(float x) {
     x = fmaxf(x, mmi_shfl_xor(x, 16));
     return fmaxf(x, mmi_shfl_xor(x, 32));
