@@ -179,6 +179,34 @@ __device__ __forceinline__ void mmi_swap32(float& a, float& b) {
     a = __builtin_bit_cast(float, v0);
     b = __builtin_bit_cast(float, v1);
 }
+// the odd rows of 16 lanes of a change places with the even rows of b
+__device__ __forceinline__ void mmi_swap16(float& a, float& b) {
+    const auto v = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned v0 = v[0], v1 = v[1];
+    a = __builtin_bit_cast(float, v0);
+    b = __builtin_bit_cast(float, v1);
+}
+// over the lanes that share lane % LPR: inside a row of 16 (rotations; after a step by 8 a rotation by 4 reaches lane ^ 4's value, and so on), over the wave
+template <int R>
+__device__ __forceinline__ float mmi_row_ror(float x) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + R, 0xf, 0xf, true)); }
+template <int LPR>
+__device__ __forceinline__ float mmi_slots_row_sum(float x) {
+    static_assert(LPR == 2 || LPR == 4 || LPR == 8 || LPR == 16, "a power of two inside a row");
+    if constexpr (LPR <= 8) x += mmi_row_ror<8>(x);
+    if constexpr (LPR <= 4) x += mmi_row_ror<4>(x);
+    if constexpr (LPR <= 2) x += mmi_row_ror<2>(x);
+    return x;
+}
+template <int LPR>
+__device__ __forceinline__ float mmi_slots_sum(float x) { return mmi_rows_sum(mmi_slots_row_sum<LPR>(x)); }
+template <int LPR>
+__device__ __forceinline__ float mmi_slots_max(float x) {
+    static_assert(LPR == 2 || LPR == 4 || LPR == 8 || LPR == 16, "a power of two inside a row");
+    if constexpr (LPR <= 8) x = fmaxf(x, mmi_row_ror<8>(x));
+    if constexpr (LPR <= 4) x = fmaxf(x, mmi_row_ror<4>(x));
+    if constexpr (LPR <= 2) x = fmaxf(x, mmi_row_ror<2>(x));
+    return mmi_rows_max(x);
+}
 // sum / maximum of an unsigned over the whole wave, every lane gets it: four DPP steps inside the rows of 16, two crossbar steps
 // across the rows (a six-step __shfl_xor butterfly is six dependent trips through the LDS crossbar)
 __device__ __forceinline__ unsigned mmi_wave_sum_u32(unsigned x) {
@@ -206,8 +234,6 @@ typedef __bf16 mmi_bf16x2v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float mmi_dot2_bf16(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(mmi_bf16x2v, a), __builtin_bit_cast(mmi_bf16x2v, b), c, false);
 }
-// two fp32 FMAs
-__device__ __forceinline__ f32x2 mmi_pk_fma(f32x2 a, f32x2 b, f32x2 c) { return __builtin_elementwise_fma(a, b, c); }
 
 // D(32x32) += A(32x2) * B(2x32), exact fp32 fma chain.  lane l: a = A[l&31][l>>5], b = B[l>>5][l&31];
 // d[r] = D[(r&3) + 8*(r>>2) + 4*(l>>5)][l&31].
@@ -261,6 +287,11 @@ __device__ __forceinline__ uint32_t mmi_cvt_fp8x4(float a, float b, float c, flo
 __device__ __forceinline__ void mmi_fp8x4_to_f32(uint32_t w, float* o) {
     const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
     o[0] = lo[0]; o[1] = lo[1]; o[2] = hi[0]; o[3] = hi[1];
+}
+// four fp8 bytes -> four bf16 (exact: e4m3 has 3 mantissa bits)
+__device__ __forceinline__ u32x2 mmi_fp8x4_to_bf16(uint32_t w) {
+    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true))};
 }
 // D(32x32) += A(32x16) * B(16x32), fp8 in / fp32 acc.  Same element map as the bf16 32x32x16 form with one byte per
 // element: lane l: a[e] = A[l&31][8*(l>>5)+e], b[e] = B[8*(l>>5)+e][l&31] (8 bytes per operand per lane).

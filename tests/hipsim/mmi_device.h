@@ -211,6 +211,14 @@ inline void mmi_fp8x4_to_f32(uint32_t w, float* o) {
     for (int i = 0; i < 4; ++i) o[i] = hipsim_detail::e4m3_to_f32((uint8_t)(w >> (8 * i)));
 }
 
+inline u32x2 mmi_fp8x4_to_bf16(uint32_t w) {
+    float f[4];
+    mmi_fp8x4_to_f32(w, f);
+    uint32_t b[4];
+    memcpy(b, f, 16);
+    return u32x2{(b[0] >> 16) | (b[1] & 0xffff0000u), (b[2] >> 16) | (b[3] & 0xffff0000u)};
+}
+
 inline f32x16 mmi_mfma_fp8_32x32x16(u32x2 a, u32x2 b, f32x16 c) {
     using namespace hipsim_detail;
     hipsim::Slot* s = hipsim::wave_slots();
@@ -350,6 +358,23 @@ inline void mmi_swap32(float& a, float& b) {
     if (hipsim::lane_id() < 32) b = oa;
     else a = ob;
 }
+inline void mmi_swap16(float& a, float& b) {
+    const float oa = mmi_shfl_xor(a, 16), ob = mmi_shfl_xor(b, 16);
+    if (hipsim::lane_id() & 16) a = ob;
+    else b = oa;
+}
+template <int LPR>
+inline float mmi_slots_row_sum(float x) {
+    for (int m = 8; m >= LPR; m >>= 1) x += mmi_shfl_xor(x, m);
+    return x;
+}
+template <int LPR>
+inline float mmi_slots_sum(float x) { return mmi_rows_sum(mmi_slots_row_sum<LPR>(x)); }
+template <int LPR>
+inline float mmi_slots_max(float x) {
+    for (int m = LPR; m < 64; m <<= 1) x = fmaxf(x, mmi_shfl_xor(x, m));
+    return x;
+}
 inline double mmi_group8_sum_f64(double x) {
     for (int m = 1; m < 8; m <<= 1) x += mmi_shfl_xor(x, m);
     return x;
@@ -379,7 +404,6 @@ inline float mmi_dot2_bf16(uint32_t a, uint32_t b, float c) {
     using hipsim_detail::bf;
     return fmaf(bf((uint16_t)(a >> 16)), bf((uint16_t)(b >> 16)), fmaf(bf((uint16_t)a), bf((uint16_t)b), c));
 }
-inline f32x2 mmi_pk_fma(f32x2 a, f32x2 b, f32x2 c) { return f32x2{fmaf(a[0], b[0], c[0]), fmaf(a[1], b[1], c[1])}; }
 inline float mmi_rint(float x) { return nearbyintf(x); }
 inline uint32_t mmi_pack_low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
     return (a & 0xffu) | ((b & 0xffu) << 8) | ((c & 0xffu) << 16) | ((d & 0xffu) << 24);
