@@ -1129,6 +1129,14 @@ struct Carry {                    // what the next residual launch has to add
     const float* dn = nullptr; int dn_p = 1, top = 1; const float* ls2 = nullptr;
     const float* vec = nullptr; bool replace = false;      // (mix is the whole new residual, plus vec)
 };
+template <class Tr>
+int launch_norm(hipStream_t s, int v, int rows, int block, size_t smem, const TlmResidArgs& a) {
+    if (v == 1) MMI_LAUNCH((k_tlm_resid_norm<Tr, 1>), rows, block, smem, s, a);
+    else if (v == 2) MMI_LAUNCH((k_tlm_resid_norm<Tr, 2>), rows, block, smem, s, a);
+    else MMI_LAUNCH((k_tlm_resid_norm<Tr, 4>), rows, block, smem, s, a);
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
+}
 struct Norms {                    // what it leaves behind: one or two normalised operands, or (raw) the residual itself as an operand
     const float* w = nullptr; void* out = nullptr;
     const float* w2 = nullptr; void* out2 = nullptr;
@@ -1176,14 +1184,14 @@ void add_resid(mmi_tlm* m, MmiProgram& P, const Shape& sh, const Carry& c, int e
     a.out = o.out;
     a.KS = m->h_ks;
     a.rows = rows;
-    const int block = n <= 256 ? std::min(1024, std::max(256, round_up(m->ld / 4, 64))) : 256;     // few rows: one vector per thread
+    a.by_group = tlm_divisor(a.width / a.groups, a.width + 4);
+    // few rows: one vector per thread; many: 256 threads, or as many as leave four vectors each
+    const int vectors = m->ld / 4, block = n <= 256 ? std::min(1024, std::max(256, round_up(vectors, 64))) : std::max(256, round_up(mmi_cdiv(vectors, 4), 64));
+    const int v = vectors <= block ? 1 : (vectors <= 2 * block ? 2 : 4);
     const size_t smem = ((size_t)m->ld + 2 * (size_t)m->cfg.norm_groups + block / 64 + 8) * sizeof(float);
     const bool f32 = m->f32;
     P.add([=](hipStream_t s) {
-        if (f32) MMI_LAUNCH((k_tlm_resid_norm<TlmF32>), n, block, smem, s, a);
-        else MMI_LAUNCH((k_tlm_resid_norm<TlmBf16>), n, block, smem, s, a);
-        MMI_CHECK_LAUNCH();
-        return (int)MMI_OK;
+        return f32 ? launch_norm<TlmF32>(s, v, n, block, smem, a) : launch_norm<TlmBf16>(s, v, n, block, smem, a);
     });
 }
 void add_jobs(mmi_tlm* m, MmiProgram& P, const Plan& p, const TlmJobs& J, long bytes) {

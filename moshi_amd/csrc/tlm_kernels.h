@@ -212,6 +212,14 @@ __device__ __forceinline__ int tlm_row_block(int b, int n) {
     return ((i >> 4) * 8 + (b & 7)) * 16 + (i & 15);
 }
 
+// n / d for what a launch knows: m = 2^32 / d + 1 makes it one multiplication (exact while n d < 2^32, else 0)
+struct TlmDiv { int d; unsigned m; };
+inline TlmDiv tlm_divisor(int d, long n_max) { return TlmDiv{d, d > 1 && n_max * d < (1L << 32) ? (unsigned)((1L << 32) / d + 1) : 0u}; }
+__device__ __forceinline__ int tlm_div(int n, TlmDiv v) {
+    if (v.m) return (int)(((unsigned long)(unsigned)n * v.m) >> 32);
+    return v.d == 1 ? n : n / v.d;
+}
+
 // ------------------------------------------------------------------------------------------------
 // residual update + grouped RMS norm: one workgroup per row
 //   x <- x + ls1 * sum_p mix[p] + ls2 * (1 / top) * sum_choice sum_p dn[p]   (the split-K partials of the two sublayers' last products;
@@ -235,6 +243,7 @@ struct TlmResidArgs {
     const float* vec;
     float* tap;                          // copy of the residual stream before the embedding is added again, or null
     const float* w; int groups; float eps;
+    TlmDiv by_group;                     // by width / groups
     void* out; int KS;                   // packed; null: no norm
     const float* w2; void* out2;
     void* rows_out; int rows_ld;         // what experts gather (by w2 if there is one), row-major, or null
@@ -242,86 +251,240 @@ struct TlmResidArgs {
     void* emb_out; int emb_k0;           // TLM_EMB_SET: packed copy of the embedding from column emb_k0 of rows of raw_ks k-steps, or null
     const int* rows;                     // row list (the residual is then not written back), or null
 };
-template <class Tr>
+// V: vectors of 4 columns per thread, all of them in registers (4 V blockDim >= ld).  A few rows are a chain: what a row reads, the sum over the
+// workgroup, what it writes.  So a thread asks for everything at once (V == 1; up to 8 partial sums of each product, those past the last one again, not
+// added), and where groups are whole waves' vectors (256 columns) the sums need no copy of the row and one meeting.  Before - the partial sums
+// one after the other behind the row, weights cold behind the sums, divisions by the group's width - a row of 2048 took 5.6 us, here 4.4.
+// us per launch before / here: 64 rows of 4096 8.6 / 6.4, 2048 of 2048 26.1 / 19.8, 1773 of 4096 38.8 / 33.1 (their bytes: 3.4 TB/s before).
+template <class Tr, int V>
 __global__ __launch_bounds__(1024) void k_tlm_resid_norm(TlmResidArgs a) {
-    MMI_DYN_SHARED(float, row);          // [ld] the row, then [groups * parts] partial sums, then [groups] 1 / rms
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, nthr = (int)blockDim.x, nw = nthr >> 6;
+    MMI_DYN_SHARED(float, sh);           // one partial sum per wave and vector; other groups: [ld] the row, [groups * parts] partial sums, [groups] 1 / rms
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = mmi_uniform(tid >> 6), nthr = (int)blockDim.x, nw = nthr >> 6;
     const int o = tlm_row_block((int)blockIdx.x, (int)gridDim.x), r = a.rows ? a.rows[o] : o;
     float* x = a.x + (long)r * a.ld;
-    for (int k = 4 * tid; k < a.ld; k += 4 * nthr) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f}, ev = v;
-        if (a.emb_mode != TLM_EMB_NONE) {
-            const TlmEmbArgs& E = a.emb;
-            const uint16_t* e = E.table + (long)E.tok[r] * a.width + k;
-            const uint16_t* eb = E.bigram ? E.bigram + (long)E.brow[r] * a.width + k : nullptr;
-            const uint16_t* ep = E.pos ? E.pos + (long)E.at[r] * a.width + k : nullptr;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, ones = {1.f, 1.f, 1.f, 1.f};
+    int k[V];                            // first column; past the row: its last vector again, not stored
+    bool mine[V];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (k + q < a.width) {
-                    ev[q] = mmi_bf16_to_f32(e[q]) * E.scale;
-                    if (eb) ev[q] += mmi_bf16_to_f32(eb[q]);
-                    if (ep) ev[q] += mmi_bf16_to_f32(ep[q]);
+    for (int i = 0; i < V; ++i) {
+        const int at = 4 * (tid + i * nthr);
+        mine[i] = at < a.ld;
+        k[i] = min(at, a.ld - 4);
+    }
+    f32x4 v[V], d[V], f[V], ev[V], w, w2, l1 = ones, l2 = ones;
+#pragma unroll
+    for (int i = 0; i < V; ++i) v[i] = d[i] = f[i] = ev[i] = zero;
+    const bool update = a.emb_mode != TLM_EMB_SET;
+    if (update && !a.replace)
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = *reinterpret_cast<const f32x4*>(x + k[i]);
+    auto mix = [&](int p, int i) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(a.mix + p * a.mix_ps + (long)r * a.ld + k[i]); };
+    const int dn_n = a.dn ? a.top * a.dn_p : 0, mix_n = a.mix ? a.mix_p : 0;
+    int dc = 0, dp = 0;                  // choice and partial sum that comes next
+    auto dn = [&](int i) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(a.dn + dp * a.dn_ps + ((long)r * a.top + dc) * a.ld + k[i]); };
+    auto next = [&]() __attribute__((always_inline)) {
+        if (++dp == a.dn_p) {
+            dp = 0;
+            ++dc;
+        }
+    };
+    if constexpr (V == 1) {
+        f32x4 m4[8], d4[8];
+#pragma unroll
+        for (int h = 0; h < 8; h += 4) {
+            if (update && mix_n > h)
+#pragma unroll
+                for (int p = h; p < h + 4; ++p) m4[p] = mix(min(p, mix_n - 1), 0);
+            if (update && dn_n > h)
+#pragma unroll
+                for (int p = h; p < h + 4; ++p) {
+                    d4[p] = dn(0);
+                    if (p + 1 < dn_n) next();
                 }
         }
-        if (a.emb_mode == TLM_EMB_SET) {
-            v = ev;
-            if (a.emb_out) Tr::store4((typename Tr::elem*)a.emb_out + tlm_index<Tr>(o, a.emb_k0 + k, a.raw_ks), ev);
-        } else {
-            if (!a.replace) v = *reinterpret_cast<const f32x4*>(x + k);
-            f32x4 d = {0.f, 0.f, 0.f, 0.f};
-            if (a.mix) {
-#pragma unroll 8
-                for (int p = 0; p < a.mix_p; ++p) d += *reinterpret_cast<const f32x4*>(a.mix + p * a.mix_ps + (long)r * a.ld + k);
-                if (a.ls1) d *= *reinterpret_cast<const f32x4*>(a.ls1 + k);
-            }
-            if (a.dn) {
-                f32x4 f = {0.f, 0.f, 0.f, 0.f};
-                for (int c = 0; c < a.top; ++c)
-#pragma unroll 8
-                    for (int p = 0; p < a.dn_p; ++p) f += *reinterpret_cast<const f32x4*>(a.dn + p * a.dn_ps + ((long)r * a.top + c) * a.ld + k);
-                f *= 1.0f / (float)a.top;
-                d += a.ls2 ? f * *reinterpret_cast<const f32x4*>(a.ls2 + k) : f;
-            }
-            v += d;
-            if (a.tap) *reinterpret_cast<f32x4*>(a.tap + (long)r * a.ld + k) = v;
-            if (a.emb_mode == TLM_EMB_ADD) v += ev;
+        if (update && a.ls1) l1 = *reinterpret_cast<const f32x4*>(a.ls1 + k[0]);
+        if (update && a.ls2) l2 = *reinterpret_cast<const f32x4*>(a.ls2 + k[0]);
+        if (a.out) {
+            w = *reinterpret_cast<const f32x4*>(a.w + k[0]);
+            w2 = a.w2 ? *reinterpret_cast<const f32x4*>(a.w2 + k[0]) : w;
         }
-        if (a.vec) v += *reinterpret_cast<const f32x4*>(a.vec + k);
-        if (a.raw) Tr::store4((typename Tr::elem*)a.raw + tlm_index<Tr>(o, k, a.raw_ks), v);
-        if (!a.rows) *reinterpret_cast<f32x4*>(x + k) = v;
-        *reinterpret_cast<f32x4*>(row + k) = v;
+        if (update) {
+#pragma unroll
+            for (int p = 0; p < 8; ++p)
+                if (p < mix_n) d[0] += m4[p];
+#pragma unroll
+            for (int p = 0; p < 8; ++p)
+                if (p < dn_n) f[0] += d4[p];
+#pragma unroll 1
+            for (int p0 = 8; p0 < mix_n; p0 += 4) {
+                f32x4 t[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) t[p] = mix(min(p0 + p, mix_n - 1), 0);
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    if (p0 + p < mix_n) d[0] += t[p];
+            }
+#pragma unroll 1
+            for (int p0 = 8; p0 < dn_n; p0 += 4) {
+                f32x4 t[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    t[p] = dn(0);
+                    if (p0 + p + 1 < dn_n) next();
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    if (p0 + p < dn_n) f[0] += t[p];
+            }
+        }
+    } else if (update) {
+        int p = 0;
+        for (; p + 2 <= mix_n; p += 2) {
+            f32x4 t[2][V];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int i = 0; i < V; ++i) t[q][i] = mix(p + q, i);
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int i = 0; i < V; ++i) d[i] += t[q][i];
+        }
+        if (p < mix_n)
+#pragma unroll
+            for (int i = 0; i < V; ++i) d[i] += mix(p, i);
+        p = 0;
+        for (; p + 2 <= dn_n; p += 2) {
+            f32x4 t[2][V];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) t[q][i] = dn(i);
+                next();
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int i = 0; i < V; ++i) f[i] += t[q][i];
+        }
+        if (p < dn_n)
+#pragma unroll
+            for (int i = 0; i < V; ++i) f[i] += dn(i);
+    }
+    if (a.emb_mode != TLM_EMB_NONE) {
+        const TlmEmbArgs& E = a.emb;
+        const uint16_t* e = E.table + (long)E.tok[r] * a.width;
+        const uint16_t* eb = E.bigram ? E.bigram + (long)E.brow[r] * a.width : nullptr;
+        const uint16_t* ep = E.pos ? E.pos + (long)E.at[r] * a.width : nullptr;
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (k[i] + q < a.width) {
+                    ev[i][q] = mmi_bf16_to_f32(e[k[i] + q]) * E.scale;
+                    if (eb) ev[i][q] += mmi_bf16_to_f32(eb[k[i] + q]);
+                    if (ep) ev[i][q] += mmi_bf16_to_f32(ep[k[i] + q]);
+                }
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        if (!update) {
+            v[i] = ev[i];
+            if (a.emb_out && mine[i]) Tr::store4((typename Tr::elem*)a.emb_out + tlm_index<Tr>(o, a.emb_k0 + k[i], a.raw_ks), ev[i]);
+        } else {
+            if (V > 1 && a.ls1) l1 = *reinterpret_cast<const f32x4*>(a.ls1 + k[i]);
+            if (a.mix && a.ls1) d[i] *= l1;
+            if (a.dn) {
+                f[i] *= 1.0f / (float)a.top;
+                if (V > 1 && a.ls2) l2 = *reinterpret_cast<const f32x4*>(a.ls2 + k[i]);
+                d[i] += a.ls2 ? f[i] * l2 : f[i];
+            }
+            v[i] += d[i];
+            if (a.tap && mine[i]) *reinterpret_cast<f32x4*>(a.tap + (long)r * a.ld + k[i]) = v[i];
+            if (a.emb_mode == TLM_EMB_ADD) v[i] += ev[i];
+        }
+        if (a.vec) v[i] += *reinterpret_cast<const f32x4*>(a.vec + k[i]);
+        if (!mine[i]) continue;
+        if (a.raw) Tr::store4((typename Tr::elem*)a.raw + tlm_index<Tr>(o, k[i], a.raw_ks), v[i]);
+        if (!a.rows) *reinterpret_cast<f32x4*>(x + k[i]) = v[i];
     }
     if (!a.out) return;                                       // uniform over the grid
-    const int gs = a.width / a.groups;
-    const int parts = a.groups < nw ? nw / a.groups : 1;        // waves per group
-    float* part = row + a.ld;
-    float* inv = part + a.groups * parts;
-    __syncthreads();
-    const int per = (gs + parts - 1) / parts;
-    for (int t = wave; t < a.groups * parts; t += nw) {
-        const int g = t / parts, p = t - g * parts;
-        const int lo = p * per, hi = lo + per < gs ? lo + per : gs;
-        float s = 0.f;
-        for (int k = lo + lane; k < hi; k += 64) s = mmi_fma(row[g * gs + k], row[g * gs + k], s);
-        s = tlm_wave_sum(s);
-        if (lane == 0) part[t] = s;
-    }
-    __syncthreads();
-    for (int g = tid; g < a.groups; g += nthr) {
-        float s = 0.f;
-        for (int p = 0; p < parts; ++p) s += part[g * parts + p];
-        inv[g] = 1.0f / sqrtf(s / (float)gs + a.eps);
-    }
-    __syncthreads();
-    typename Tr::elem* out = (typename Tr::elem*)a.out;
-    for (int k = 4 * tid; k < a.ld; k += 4 * nthr) {
-        f32x4 v = *reinterpret_cast<const f32x4*>(row + k);
-        const f32x4 w = *reinterpret_cast<const f32x4*>(a.w + k);
+    const int gs = a.by_group.d;
+    float inv[V][4];
+    if (a.groups == 1 || gs % 256 == 0) {                     // a wave's vector lies in one group
+        float ss[V];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = k + q < a.width ? v[q] * inv[(k + q) / gs] : 0.f;
-        Tr::store4(out + tlm_index<Tr>(o, k, a.KS), v * w);
-        if (a.rows_out) Tr::store4((typename Tr::elem*)a.rows_out + (long)o * a.rows_ld + k, v * (a.w2 ? *reinterpret_cast<const f32x4*>(a.w2 + k) : w));
-        if (a.out2) Tr::store4((typename Tr::elem*)a.out2 + tlm_index<Tr>(o, k, a.KS), v * *reinterpret_cast<const f32x4*>(a.w2 + k));
+        for (int i = 0; i < V; ++i) {
+            ss[i] = 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (mine[i] && k[i] + q < a.width) ss[i] = mmi_fma(v[i][q], v[i][q], ss[i]);
+            if (a.groups > 1) {
+                ss[i] = tlm_wave_sum(ss[i]);
+                if (lane == 0) sh[wave + i * nw] = ss[i];
+            } else if (i) {
+                ss[0] += ss[i];
+            }
+        }
+        if (a.groups == 1) {
+            ss[0] = tlm_wave_sum(ss[0]);
+            if (lane == 0) sh[wave] = ss[0];
+        }
+        __syncthreads();
+        const int n = a.groups == 1 ? nw : gs / 256;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            if (i && a.groups == 1) {
+                inv[i][0] = inv[0][0];
+            } else {
+                const float* part = sh + (a.groups == 1 ? 0 : tlm_div(mmi_uniform(min(256 * (wave + i * nw), a.width - 1)), a.by_group) * n);
+                float t = 0.f;
+                for (int p = 0; p < n; ++p) t += part[p];
+                inv[i][0] = 1.0f / sqrtf(t / (float)gs + a.eps);
+            }
+#pragma unroll
+            for (int q = 1; q < 4; ++q) inv[i][q] = inv[i][0];
+        }
+    } else {
+        const int parts = a.groups < nw ? nw / a.groups : 1;        // waves per group
+        float *row = sh, *part = row + a.ld, *rms = part + a.groups * parts;
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            if (mine[i]) *reinterpret_cast<f32x4*>(row + k[i]) = v[i];
+        __syncthreads();
+        const int per = (gs + parts - 1) / parts;
+        for (int t = wave; t < a.groups * parts; t += nw) {
+            const int g = t / parts, p = t - g * parts;
+            const int lo = p * per, hi = lo + per < gs ? lo + per : gs;
+            float s = 0.f;
+            for (int c = lo + lane; c < hi; c += 64) s = mmi_fma(row[g * gs + c], row[g * gs + c], s);
+            s = tlm_wave_sum(s);
+            if (lane == 0) part[t] = s;
+        }
+        __syncthreads();
+        for (int g = tid; g < a.groups; g += nthr) {
+            float s = 0.f;
+            for (int p = 0; p < parts; ++p) s += part[g * parts + p];
+            rms[g] = 1.0f / sqrtf(s / (float)gs + a.eps);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) inv[i][q] = rms[min(tlm_div(k[i] + q, a.by_group), a.groups - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        if (!mine[i]) continue;
+        if constexpr (V > 1) {
+            w = *reinterpret_cast<const f32x4*>(a.w + k[i]);
+            w2 = a.w2 ? *reinterpret_cast<const f32x4*>(a.w2 + k[i]) : w;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[i][q] = k[i] + q < a.width ? v[i][q] * inv[i][q] : 0.f;
+        Tr::store4((typename Tr::elem*)a.out + tlm_index<Tr>(o, k[i], a.KS), v[i] * w);
+        if (a.rows_out) Tr::store4((typename Tr::elem*)a.rows_out + (long)o * a.rows_ld + k[i], v[i] * w2);
+        if (a.out2) Tr::store4((typename Tr::elem*)a.out2 + tlm_index<Tr>(o, k[i], a.KS), v[i] * w2);
     }
 }
 
