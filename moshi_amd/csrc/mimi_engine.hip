@@ -824,9 +824,9 @@ void launch_lin_norm(hipStream_t s, const MimiLinArgs& a) {
 int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
     if (a.ln_w && (a.J > 64 || a.J * 16 != K)) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi transformer: a width of at most 1024, a multiple of 16");
     // 16 x 16 tiles while the chip holds all workgroups at once (two per CU); with a norm 32 rows share it from 256 tiles on (32 streams 1203 -> 1186
-    // us a frame; with 192 - 256 tiles, 16 streams, 973 -> 1000).  Beyond that 32 x 32 in groups of two fragments (258 columns, K = 2048: 17.5 -> 13.0
-    // us, 16 x 16 13.9), with a norm 128 rows per workgroup where those fill half the chip.  Groups of 4 fragments, not 8: with K = 512 a wave has
-    // 4 (one stream 717 -> 688 us a frame, 16 streams 973 -> 946).  Weights that one tile of columns reads leave no line behind, others' are read
+    // us a frame; with 192 - 256 tiles, 16 streams, 973 -> 1000).  Beyond that 32 x 32 in rings of four fragments (258 columns, K = 2048: 17.5 -> 13.0
+    // us, 16 x 16 13.9), with a norm 128 rows per workgroup where those fill half the chip.  Rings of 4 fragments, of 8 for long reductions: with K = 512 a wave
+    // has 4 (groups of 4 against 8: one stream 717 -> 688 us a frame, 16 streams 973 -> 946).  Weights that one tile of columns reads leave no line behind, others' are read
     // again (32 streams 1211 -> 1201 us).
     const long tiles = (long)mmi_cdiv(a.M, 16) * mmi_cdiv(a.N, 16);
     const bool rows = a.ln_w && a.J <= 60 && (long)mmi_cdiv(a.M, 128) * mmi_cdiv(a.N, 16) >= 128;      // (J KB of LDS and a little more, below 64)
@@ -840,9 +840,11 @@ int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
             if (a.J <= 32) MMI_LAUNCH((k_mimi_lin_rows<4>), grid, 64 * waves, smem, s, a);
             else MMI_LAUNCH((k_mimi_lin_rows<8>), grid, 64 * waves, smem, s, a);
         } else if (!a.ln_w) {
-            if (a.N <= 16) launch_lin<1, 1, 4, true>(s, a);
+            if (a.N <= 16 && a.J > 32) launch_lin<1, 1, 8, true>(s, a);
+            else if (a.N <= 16) launch_lin<1, 1, 4, true>(s, a);
+            else if (tiles <= 512 && a.J > 32) launch_lin<1, 1, 8, false>(s, a);
             else if (tiles <= 512) launch_lin<1, 1, 4, false>(s, a);
-            else launch_lin<2, 2, 2, false>(s, a);
+            else launch_lin<2, 2, 4, false>(s, a);
         } else {
             if (a.N <= 16 && tiles <= 512) launch_lin_norm<1, 1, true>(s, a);
             else if (tiles <= 256) launch_lin_norm<1, 1, false>(s, a);

@@ -986,6 +986,8 @@ struct MimiLinArgs {
 // streams and groups of frames agree.
 // Measured, 1 stream (N = 2): norm + linear 8.2 -> 5.0 us, K = 512 5.9 -> 4.7, K = 2048 9.3 (with a second launch that added its sums) -> 6.6; 32 streams
 // (N = 64): norm + linear 8.4 -> 6.3, K = 2048 9.6 -> 6.9; a file's 258 columns: K = 512 7.9 -> 6.2, K = 2048 19.2 -> 13.0 (norm + linear: k_mimi_lin_rows).
+// Fragments pass in a ring that asks for none past the slice, 8 of them for long reductions (a double buffer of 4 asked for 4 twice): one stream 690.9 -> 680.9
+// us a frame, 32 streams 1178 -> 1169.
 // Bound by latency: one column tile has M / 16 workgroups of 16 KB - 64 KB of weights and a few hundred cycles of matrix work each.  Hence
 // 16-wide tiles (a live stream has two columns: a 32-wide tile keeps the matrix core busy four times as long, 1.7 us at K = 512, on half the
 // CUs), every operand of the epilogue requested ahead of the sums, the norm's whole slice in registers (U fragments per wave), and
@@ -1058,8 +1060,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
         auto column_sum = [&](int which, float (&s)[FN]) __attribute__((always_inline)) {      // over the lanes that hold a column, then over the waves
 #pragma unroll
             for (int n = 0; n < FN; ++n) {
-                s[n] += mmi_shfl_xor(s[n], 16);
-                s[n] += mmi_shfl_xor(s[n], 32);
+                s[n] = mmi_rows_sum(s[n]);
                 if (lane < 16) stat[which][wave][n * 16 + lane] = s[n];
             }
             __syncthreads();
@@ -1107,43 +1108,38 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
                         for (int m = 0; m < FM; ++m) acc[m][n] = mmi_mfma_f32_16x16x4(wv[u][m][e], y, acc[m][n]);
                     }
     } else {
-        f32x4 wA[U][FM], xA[U][FN], wB[U][FM], xB[U][FN];
-        auto load = [&](f32x4 (&w)[U][FM], f32x4 (&x)[U][FN], int at) __attribute__((always_inline)) {
+        // U fragments of weights and operand on their way in a ring: each is asked for again as soon as its products are done, none past the slice
+        f32x4 w[U][FM], x[U][FN];
+        auto load = [&](int u, int at) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int uu = min(at + u, last);
+            for (int m = 0; m < FM; ++m) w[u][m] = weight(wp[m] + (long)at * 64);
 #pragma unroll
-                for (int m = 0; m < FM; ++m) w[u][m] = weight(wp[m] + (long)uu * 64);
-#pragma unroll
-                for (int n = 0; n < FN; ++n) x[u][n] = xp[n][(long)uu * 64];
-            }
+            for (int n = 0; n < FN; ++n) x[u][n] = xp[n][(long)at * 64];
         };
-        auto mma = [&](const f32x4 (&w)[U][FM], const f32x4 (&x)[U][FN], int at) __attribute__((always_inline)) {
+        auto mma = [&](int u, bool on) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool on = at + u < nj;                 // (past the slice: zeros, not a branch - see k_conv_cols)
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
+                for (int n = 0; n < FN; ++n) {
+                    const float v = on ? x[u][n][e] : 0.f;       // (past the slice: zeros, not a branch - see k_conv_cols)
 #pragma unroll
-                    for (int n = 0; n < FN; ++n) {
-                        const float v = on ? x[u][n][e] : 0.f;
-#pragma unroll
-                        for (int m = 0; m < FM; ++m) acc[m][n] = mmi_mfma_f32_16x16x4(w[u][m][e], v, acc[m][n]);
-                    }
-            }
+                    for (int m = 0; m < FM; ++m) acc[m][n] = mmi_mfma_f32_16x16x4(w[u][m][e], v, acc[m][n]);
+                }
         };
-        load(wA, xA, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) load(u, min(u, last));
+        mmi_sched_barrier();
         int at = 0;
-        while (at + U < nj) {
-            load(wB, xB, at + U);
-            mmi_sched_barrier();
-            mma(wA, xA, at);
-            load(wA, xA, at + 2 * U);
-            mmi_sched_barrier();
-            mma(wB, xB, at + U);
-            at += 2 * U;
-        }
-        if (at < nj) mma(wA, xA, at);
+#pragma unroll 1
+        for (; at + U < nj; at += U)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                mma(u, true);
+                load(u, min(at + U + u, last));
+                mmi_sched_barrier();
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u) mma(u, at + u < nj);
     }
 
     MMI_SHARED float red[8 * FM * FN * 256];
