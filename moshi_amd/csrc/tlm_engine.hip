@@ -828,6 +828,24 @@ int split_for(const Plan& p, int KS, int blocks) {
     else while (s < TILE_SPLIT && blocks * s < TILE_BLOCKS && KS / (2 * s) >= 16) s *= 2;
     return s;
 }
+// Up to 16 rows: the products of a launch are split together, the one with the longest blocks first, until the launch has 384 blocks (two of 8 waves
+// on most CUs).  Each until it had 384 of its own left reductions of 2 k-steps per wave and up to 16 partial sums for the norm behind them.  us per
+// step of 1 / 12 sequences, each by itself / together: Bibapel 1024 277 / 260 and 313 / 296, 2048 391 / 377 and 448 / 436, 4096 779 / 761 and 919 / 895; Kesirax 1024
+// 245 / 225 and 339 / 331, 2048 334 / 312 and 620 / 626, 4096 694 / 659 and 1349 / 1324.  Together until 128, 256, 512, 768 blocks: -3 .. +4 % of 384.  More rows
+// keep to themselves: 64 sequences of Kesirax 2048 812 / 867, 4096 1686 / 1757 (Bibapel 1 % the other way).
+int split_blocks(const Plan& p, const TlmJob& j);
+void split_together(const Plan& p, TlmJobs& J, unsigned may_split) {
+    for (;;) {
+        int total = 0, longest = -1;
+        for (int i = 0; i < J.n; ++i) {
+            const TlmJob& j = J.j[i];
+            total += split_blocks(p, j) * j.ksplit;
+            if ((may_split >> i & 1) && j.ksplit < MAX_SPLIT && j.KS / (2 * j.ksplit) >= 8 && (longest < 0 || j.KS / j.ksplit > J.j[longest].KS / J.j[longest].ksplit)) longest = i;
+        }
+        if (total >= 384 || longest < 0) return;
+        J.j[longest].ksplit *= 2;
+    }
+}
 // blocks of the tiled kernel's narrower forms (128 x 128 or 64 x 64, at fp32 64 x 32)
 int tile_blocks(const Plan& p, const TlmJob& j) { return mmi_cdiv(j.NT, p.fm == 4 ? 8 : 4) * (j.list ? j.rblocks : j.groups * mmi_cdiv(j.rows, plan_tile(p))); }
 int split_blocks(const Plan& p, const TlmJob& j) { return p.rows ? j.NT * (j.list ? j.rblocks : 1) : tile_blocks(p, j); }
@@ -956,6 +974,10 @@ void plan_jobs(const mmi_tlm* m, const Plan& p, TlmJobs& J, unsigned may_split) 
     for (int i = 0; i < J.n; ++i) {
         blocks += split_blocks(p, J.j[i]);
         wide = wide && J.j[i].groups == 1 && !J.j[i].list && (J.j[i].KS >= WIDE_KS || m->force_wide);
+    }
+    if (p.rows && p.mt == 1) {
+        split_together(p, J, may_split);
+        return;
     }
     for (int i = 0; i < J.n; ++i)
         if (may_split >> i & 1) J.j[i].ksplit = split_for(p, J.j[i].KS, p.rows ? split_blocks(p, J.j[i]) : blocks);
