@@ -812,16 +812,16 @@ int alloc_tr_stream(mmi_mimi* m, MimiMem& mem, int N, TrStream* x) {
 
 template <int FM, int FN, int U, bool NT>
 void launch_lin(hipStream_t s, const MimiLinArgs& a) {
-    MMI_LAUNCH((k_mimi_lin<FM, FN, U, false, NT>), dim3(mmi_cdiv(a.M, 16 * FM), mmi_cdiv(a.N, 16 * FN)), 512, 0, s, a);
+    MMI_LAUNCH((k_mimi_lin<FM, FN, U, false, NT>), dim3(mmi_cdiv(a.M, 16 * FM) << (FM == 1 ? a.share : 0), mmi_cdiv(a.N, 16 * FN)), 512, 0, s, a);
 }
 template <int FM, int FN, bool NT>
 void launch_lin_norm(hipStream_t s, const MimiLinArgs& a) {
-    const dim3 grid(mmi_cdiv(a.M, 16 * FM), mmi_cdiv(a.N, 16 * FN));
+    const dim3 grid(mmi_cdiv(a.M, 16 * FM) << (FM == 1 ? a.share : 0), mmi_cdiv(a.N, 16 * FN));
     if (a.J <= 32) MMI_LAUNCH((k_mimi_lin<FM, FN, 4, true, NT>), grid, 512, 0, s, a);
     else MMI_LAUNCH((k_mimi_lin<FM, FN, 8, true, NT>), grid, 512, 0, s, a);
 }
 
-int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
+int add_lin(MmiProgram& prog, MimiLinArgs a, int K) {
     if (a.ln_w && (a.J > 64 || a.J * 16 != K)) return mmi_fail(MMI_ERR_UNSUPPORTED, "Mimi transformer: a width of at most 1024, a multiple of 16");
     // 16 x 16 tiles while the chip holds all workgroups at once (two per CU); with a norm 32 rows share it from 256 tiles on (32 streams 1203 -> 1186
     // us a frame; with 192 - 256 tiles, 16 streams, 973 -> 1000).  Beyond that 32 x 32 in rings of four fragments (258 columns, K = 2048: 17.5 -> 13.0
@@ -833,6 +833,9 @@ int add_lin(MmiProgram& prog, const MimiLinArgs& a, int K) {
     int waves = 8;                                           // more of them where that gives every workgroup a CU of its own (2048 x 258: 19.5 -> 15.6 us)
     while (waves < 12 && (long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) ++waves;
     if ((long)mmi_cdiv(a.M, 16 * waves) * mmi_cdiv(a.N, 16) > 256) waves = 8;
+    // two workgroups to a tile of a long reduction while that is one per CU: us a frame of 1, 4, 8, 16, 32 streams 671, 707, 790, 911, 1112 -> 669, 705, 780, 904,
+    // 1104 (four: 672, 709, 784, 905, 1108; short reductions and those with a norm, shared likewise: no faster)
+    a.share = !a.ln_w && a.J > 32 && 2 * tiles <= 256 ? 1 : 0;
     prog.add([=](hipStream_t s) {
         if (rows) {
             const dim3 grid(mmi_cdiv(a.M, 16 * waves), mmi_cdiv(a.N, 16));

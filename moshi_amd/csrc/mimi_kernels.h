@@ -969,6 +969,7 @@ struct MimiLinArgs {
     const float* w;              // [Mt][J] fragments (k_pack_lin)
     const float* x;              // [ceil(N/16)][J] fragments (mmi_lin_index)
     int M, N, J;                 // rows, columns n = b * T + t, 16-deep pieces of the reduction
+    int share;                   // k_mimi_lin, FM = 1: 2^share workgroups share a row tile
     const float *ln_w, *ln_b;    // LayerNorm over the 16 J values of a column in front (k_pack_ln)
     float ln_eps;
     int mode;                    // ROWS: out = W x;  GELU: outp = gelu(W x);  RESID: outp += scale * W x (the residual stream), and out too where it is set
@@ -996,7 +997,9 @@ template <int FM, int FN, int U, bool LN, bool NT>
 __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
     auto weight = [](const f32x4* p) __attribute__((always_inline)) { return NT ? mmi_load_nt(p) : *p; };
     const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int m0 = (int)blockIdx.x * FM, n0 = (int)blockIdx.y * FN;
+    // a row tile shared by 2^share workgroups: 16 >> share rows each; lanes of the others' rows repeat its own (their sums are dropped)
+    const int share = FM == 1 ? a.share : 0, mine = 16 >> share, r0 = ((int)blockIdx.x & ((1 << share) - 1)) * mine;
+    const int m0 = ((int)blockIdx.x >> share) * FM, n0 = (int)blockIdx.y * FN, wl = (lane & 48) + r0 + (lane & (mine - 1));
     const int Mt = (a.M + 15) >> 4, Nt = (a.N + 15) >> 4;
     const int per = (a.J + 7) >> 3;                          // LN: <= U (the planner checks)
     const int j0 = min(a.J, wave * per), nj = min(a.J, j0 + per) - j0;
@@ -1004,7 +1007,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
     const f32x4* wp[FM];
     const f32x4* xp[FN];
 #pragma unroll
-    for (int m = 0; m < FM; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.w) + ((long)min(m0 + m, Mt - 1) * a.J + jl) * 64 + lane;
+    for (int m = 0; m < FM; ++m) wp[m] = reinterpret_cast<const f32x4*>(a.w) + ((long)min(m0 + m, Mt - 1) * a.J + jl) * 64 + wl;
 #pragma unroll
     for (int n = 0; n < FN; ++n)                             // (a column past the last one reads the last one: nobody need have stored it)
         xp[n] = reinterpret_cast<const f32x4*>(a.x) + ((long)min(n0 + n, Nt - 1) * a.J + jl) * 64 + (lane & 48) + min(lane & 15, max(a.N - (n0 + n) * 16, 1) - 1);
@@ -1026,7 +1029,7 @@ __global__ __launch_bounds__(512) void k_mimi_lin(MimiLinArgs a) {
         const int row = a.mode == MIMI_LIN_ROWS ? 4 * ((q >> 4) & 3) + (q >> 6) : 4 * (q & 3) + (q >> 6);
         rm[i] = (m0 + f / FN) * 16 + row;
         rn[i] = (n0 + f % FN) * 16 + (a.mode == MIMI_LIN_ROWS ? q & 15 : (q >> 2) & 15);
-        if (idx >= FM * FN * 256 || rm[i] >= a.M) rn[i] = a.N;          // nothing to store
+        if (idx >= FM * FN * 256 || rm[i] >= a.M || (unsigned)(row - r0) >= (unsigned)mine) rn[i] = a.N;          // nothing to store
         scl[i] = 0.f; res[i] = 0.f;
     }
     if (a.mode == MIMI_LIN_RESID) {
