@@ -616,8 +616,8 @@ int launch_gemm(mmi_lm* lm, hipStream_t s, const GemmW& g, GemmArgs a, bool is_d
         lm->xlds_launches += 1;
         rc = mt == 1 ? launch_xlds<1>(s, xl, a) : launch_xlds<2>(s, xl, a);
     } else if (const int rd = ring_entries(g, p, mt, a)) {
-        if (rd == 16) MMI_LAUNCH(k_gemm_xring16<16>, g.NT, 512, 0, s, a);
-        else MMI_LAUNCH(k_gemm_xring16<22>, g.NT, 512, 0, s, a);
+        if (rd == 16) MMI_LAUNCH((k_gemm_xring16<16, false>), g.NT, 512, 0, s, a, MmiMerge{});
+        else MMI_LAUNCH((k_gemm_xring16<22, false>), g.NT, 512, 0, s, a, MmiMerge{});
         MMI_CHECK_LAUNCH();
         rc = MMI_OK;
     } else if (const int kmax = once_kmax(g, p, mt, a)) {
@@ -879,6 +879,27 @@ void add_norm_gemm(mmi_lm* lm, const GemmW& g, uint16_t* x, const uint16_t* alph
         mmi_record_bytes(gbytes);
         return launch_norm_fused(s, T, mt, wq, NT, a);
     }, gbytes);
+}
+
+// Does out_proj merge the attention's partials itself (k_gemm_xring16<16, true>)?  One session, whose out_proj takes the ring in one round; heads of a
+// power of two features that fill the slices.  MMI_NO_MERGE_FUSION: the launch of its own
+bool merge_fused(const mmi_lm* lm, const GemmW& g, int H, int Dh, int NS) {
+    if (lm->batch != 1 || lm->act8 || NS < 2 || NS > MMI_MERGE_MAX || Dh < 8 || (Dh & (Dh - 1)) || H * Dh != g.KSTEPS * 32 || getenv("MMI_NO_MERGE_FUSION")) return false;
+    GemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.epi = MMI_EPI_RESID; a.wq = g.wq; a.osplit = plan_osplit(g, plan_gemm(g, false), a.epi, g.T);
+    return resid_ksplit(g, g.wq, 1) <= 1 && !plan_xreg(g, a.epi, g.wq, 1, 0).nx && ring_entries(g, plan_gemm(g, false), 1, a) == 16;
+}
+int launch_merge_out_proj(hipStream_t s, const GemmW& g, const LmAttnArgs& d, uint16_t* x, int features, int ksteps) {
+    GemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.out = x; a.epi = MMI_EPI_RESID; a.resid = x; a.B = 1; a.tok_rows = 1;
+    a.out_mode = MMI_OUT_PACKED; a.out_ld = features; a.out_ksteps = ksteps;
+    a.wp = g.wp; a.N = g.N; a.KSTEPS = g.KSTEPS; a.NT = g.NT; a.xp = reinterpret_cast<const u32x4*>(d.out);
+    mmi_record_bytes((long)g.bytes);
+    MMI_LAUNCH((k_gemm_xring16<16, true>), g.NT, 512, 0, s, a, (MmiMerge{d.opart, d.ml, d.NS, __builtin_ctz((unsigned)d.Dh)}));
+    MMI_CHECK_LAUNCH();
+    return MMI_OK;
 }
 
 // Does one launch take norm and linear (k_gemm_xreg16, k_gemm_norm_one)?  One session, bf16 weights on the 16-row tile, a row of at most 4096 features and whole
@@ -1149,13 +1170,15 @@ int build_program(mmi_lm* lm) {
             else P.add([lm, gw, ga](hipStream_t s) { return launch_gemm(lm, s, gw, ga, false); }, (long)gw.bytes);
         }
         P.site("L.attn");
+        const bool fused = !a8 && merge_fused(lm, L.out_proj, H, Dh, NS);
+        const auto partials_left = [=]() { return a.NS > 1 && (!attn_wave_kernel() || lm->prog.variant == 1); };
         P.add([=](hipStream_t s) {
             LmAttnArgs aa = a;
-            const bool merge_launch = a.NS > 1 && (!attn_wave_kernel() || lm->prog.variant == 1);
+            const bool merge_launch = partials_left();
             if (merge_launch) { aa.solo_rows = -1; aa.done = nullptr; }     // every workgroup leaves its partial (m, l, O)
             int rc = launch_attn_split(s, aa, kv8);
             if (rc) return rc;
-            if (merge_launch) MMI_LAUNCH(k_lm_attn_combine, B * H, Dh < 64 ? 64 : Dh, 0, s, aa);
+            if (merge_launch && !fused) MMI_LAUNCH(k_lm_attn_combine, B * H, Dh < 64 ? 64 : Dh, 0, s, aa);
             MMI_CHECK_LAUNCH();
             return (int)MMI_OK;
         });
@@ -1164,6 +1187,16 @@ int build_program(mmi_lm* lm) {
             add_quant_rows(lm, lm->att, lm->attq, lm->sx_att, d);
             Q8 q{3, lm->sx_att};
             pending = add_gemm_resid(lm, L.out_proj, reinterpret_cast<const uint16_t*>(lm->attq), lm->x, d, &q);
+        } else if (fused) {
+            const GemmW gw = L.out_proj;
+            GemmArgs ga;
+            memset(&ga, 0, sizeof(ga));
+            ga.xp = reinterpret_cast<const u32x4*>(lm->att); ga.out = lm->x; ga.epi = MMI_EPI_RESID; ga.resid = lm->x; ga.B = B; ga.tok_rows = lm->gen_batch;
+            ga.out_mode = MMI_OUT_PACKED; ga.out_ld = d; ga.out_ksteps = packed_ksteps(lm, d);
+            uint16_t* x = lm->x;
+            const int ksteps = packed_ksteps(lm, d);
+            P.add([=](hipStream_t s) { return partials_left() ? launch_merge_out_proj(s, gw, a, x, d, ksteps) : launch_gemm(lm, s, gw, ga, false); }, (long)gw.bytes);
+            pending = Pending{};
         } else
         pending = add_gemm_resid(lm, L.out_proj, lm->att, lm->x, d);
         if (c.cross_attention) {   // x = x + cross_attention(norm_cross(x), src, src) (transformer.py:779-786)

@@ -654,8 +654,13 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_xp_once(GemmArgs a) {
 // tile's activations are met once, so they pass through the registers like its weights, RD entries of both on their way in a ring - what one CU
 // streams is what it has under way, and the double buffer of k_gemm_xp stops asking while it multiplies.  Lanes of sessions that are not there
 // repeat the last one's address (one session: a quarter of the lines).  Same K partition, same k order, same reduction and epilogue: k_gemm_xp's bits.
-template <int RD>
-__global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a) {
+// MERGE (one session, a deep ring: the attention left partials): a wave merges the heads of its own slice - k_lm_attn_combine's sums, so its bits - with
+// its weights on their way, 8 features per lane; that launch took 4.6 us in front of out_proj's 7.7, here 10.8 together (12
+// partials of 32 heads of 128).
+struct MmiMerge { const float* opart; const float* ml; int NS, log_dh; };      // LmAttnArgs::opart, ml; head features 2^log_dh
+constexpr int MMI_MERGE_MAX = 12;                // partials per head
+template <int RD, bool MERGE>
+__global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a, MmiMerge g) {
     const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63, nt0 = (int)blockIdx.x;
     const MmiEpiPre pre = mmi_epi_prefetch<16, 1, 8, 0>(a, wave, lane, nt0);
     const int kper = (a.KSTEPS + 7) / 8, ks0 = min(a.KSTEPS, wave * kper), nks = min(a.KSTEPS, ks0 + kper) - ks0;
@@ -664,23 +669,66 @@ __global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a) {
     const u32x4* xp = a.xp + (long)ksl * 64;
     const unsigned wl = (unsigned)lane, xl = (unsigned)((lane & 48) + min(lane & 15, a.B - 1));
     u32x4 w[RD], x[RD];
+    if constexpr (MERGE) {                       // (slices of at most RD k-steps: the launcher checks)
+        // the partials are asked for first: loads come back in order
+        const int f = min(ksl * 32 + 8 * lane, a.KSTEPS * 32 - 8), h = f >> g.log_dh, d = f & ((1 << g.log_dh) - 1);
+        const f32x2* ml = reinterpret_cast<const f32x2*>(g.ml) + (long)h * g.NS;
+        const float* part = g.opart + (((long)h * g.NS) << g.log_dh) + d;
+        f32x2 s[MMI_MERGE_MAX];
+        f32x4 o[MMI_MERGE_MAX][2];
 #pragma unroll
-    for (int e = 0; e < RD; ++e) {
-        w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
-        x[e] = (xp + min(e, kl) * 64)[xl];
+        for (int c = 0; c < MMI_MERGE_MAX; ++c) {          // (past the end: the last partial again, not used)
+            const int cc = min(c, g.NS - 1);
+            s[c] = ml[cc];
+            o[c][0] = *reinterpret_cast<const f32x4*>(part + ((long)cc << g.log_dh));
+            o[c][1] = *reinterpret_cast<const f32x4*>(part + ((long)cc << g.log_dh) + 4);
+        }
+        mmi_sched_barrier();
+#pragma unroll
+        for (int e = 0; e < RD; ++e) w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
+        mmi_sched_barrier();
+        float M = -INFINITY, den = 0.f, num[8];
+#pragma unroll
+        for (int c = 0; c < MMI_MERGE_MAX; ++c) M = fmaxf(M, s[c][0]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) num[e] = 0.f;
+#pragma unroll
+        for (int c = 0; c < MMI_MERGE_MAX; ++c) {
+            const float wc = expf(s[c][0] - M);
+            const bool none = c >= g.NS || s[c][0] == -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) num[e] = none ? num[e] : num[e] + wc * o[c][e >> 2][e & 3];
+            den = none ? den : den + wc * s[c][1];
+        }
+        MMI_SHARED __attribute__((aligned(16))) u32x4 row[8][64];
+        u32x4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = mmi_pack_bf16x2(num[2 * q] / den, num[2 * q + 1] / den);
+        row[wave][lane] = v;
+        mmi_meet();
+#pragma unroll
+        for (int e = 0; e < RD; ++e) x[e] = row[wave][4 * min(e, kl) + (lane >> 4)];
+    } else {
+#pragma unroll
+        for (int e = 0; e < RD; ++e) {
+            w[e] = mmi_load_nt(wp + min(e, kl) * 64 + wl);
+            x[e] = (xp + min(e, kl) * 64)[xl];
+        }
     }
     mmi_sched_barrier();
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     int k = 0;
+    if constexpr (!MERGE) {
 #pragma unroll 1
-    for (; k + RD < nks; k += RD) {              // (past the slice: its last entry again)
+        for (; k + RD < nks; k += RD) {          // (past the slice: its last entry again)
 #pragma unroll
-        for (int e = 0; e < RD; ++e) {
-            acc = mmi_mfma_bf16_16x16x32(w[e], x[e], acc);
-            const int n = min(k + RD + e, kl);
-            w[e] = mmi_load_nt(wp + n * 64 + wl);
-            x[e] = (xp + n * 64)[xl];
-            mmi_sched_barrier();
+            for (int e = 0; e < RD; ++e) {
+                acc = mmi_mfma_bf16_16x16x32(w[e], x[e], acc);
+                const int n = min(k + RD + e, kl);
+                w[e] = mmi_load_nt(wp + n * 64 + wl);
+                x[e] = (xp + n * 64)[xl];
+                mmi_sched_barrier();
+            }
         }
     }
 #pragma unroll
@@ -2260,7 +2308,7 @@ __global__ __launch_bounds__(256) void k_lm_attn_split(LmAttnArgs a) {
 // Half of its time are vector instructions (e4m3 ring: 27 of 53 us at 64 sessions of ~500 rows, 137 instructions per row group of 8 rows): dot products of
 // packed pairs for both rings, an exponential is one v_exp_f32 of the difference to the maximum, rescaling only in rounds in which some maximum rises,
 // and the row slots are merged at once, exchanging halves between the rows of lanes instead of summing every element in all of them.
-// us per launch before / here: 64 sessions x 32 heads, e4m3, 263 MB 53.5 / 48.8; one session, 24.6 MB over 12
+// us per launch before / here: 64 sessions x 32 heads, e4m3, 263 MB 53.5 / 48.8; 32 sessions, bf16, 196 MB 39.0 / 35.9; one session, 24.6 MB over 12
 // workgroups a head 8.5 / 7.6.  The logits' error against 64 bits is the same (0.025, 0.014, 0.012).
 template <int DH, bool KV8 = false>
 __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      // <= 128 VGPRs, 4 workgroups per CU

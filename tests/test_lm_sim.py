@@ -273,9 +273,25 @@ def test_gemm_whose_operands_pass_in_a_ring(sim_lib, monkeypatch, B, hidden_scal
     wave (rounds of the ring that end inside it)."""
     from dataclasses import replace
     monkeypatch.setenv("MMI_GEMM_RING", "2")
+    monkeypatch.setenv("MMI_GEMM_OSPLIT", "0")
     cfg = replace(tiny_lm_config(), hidden_scale=hidden_scale, num_layers=2 if hidden_scale < 100 else 1, dim=128 if hidden_scale < 100 else 64,
                   num_heads=4 if hidden_scale < 100 else 2)
     lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=260 + B, B=B, S=2)
+
+
+@pytest.mark.parametrize("NS,dim,heads", [(2, 128, 4), (3, 256, 4), (12, 512, 4), (12, 1024, 32)])
+def test_partials_merged_inside_out_proj(sim_lib, monkeypatch, NS, dim, heads):
+    """k_gemm_xring16<16, true> at one session: heads of 32 to 128 features, slices of one head, of a part of one, and of several, most and fewest
+    partials, some of them empty."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_GEMM_RING", "2")
+    monkeypatch.setenv("MMI_GEMM_OSPLIT", "0")
+    monkeypatch.setenv("MMI_ATTN_NS", str(NS))
+    monkeypatch.setenv("MMI_ATTN_SOLO", "0")
+    cfg = replace(tiny_lm_config(), dim=dim, num_heads=heads, num_layers=1, context=40)
+    st = {}
+    lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=270 + NS, B=1, S=9, stats=st)
+    assert "k_lm_attn_combine" not in {k for _, k in st["launch_list"]}
 
 
 def test_depformer_in_per_step_launches(sim_lib, monkeypatch):
