@@ -1332,7 +1332,7 @@ int build_program(mmi_lm* lm) {
         TokArgs t = tok_args(lm);
         const int *tt = lm->text_tok, *at = lm->audio_tok; int* out = lm->out_i32; unsigned long long* rng = lm->rng;
         P.add([=](hipStream_t s) {
-            MMI_LAUNCH(k_lm_commit, mmi_cdiv(t.B, 64), 64, 0, s, t, tt, at, out, rng);
+            MMI_LAUNCH(k_lm_commit, t.B, 64, 0, s, t, tt, at, out, rng);
             MMI_CHECK_LAUNCH();
             return (int)MMI_OK;
         });

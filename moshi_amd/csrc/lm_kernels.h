@@ -2101,16 +2101,26 @@ __global__ void k_lm_embed(const int* __restrict__ tokens, int n_codebooks, cons
     const int d = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (d >= D) return;
     const int* tk = tokens + (long)b * n_codebooks;
+    const int t0 = tk[0];
+    const uint16_t text = text_emb[(long)max(t0, 0) * D + d];
     float acc = 0.f;
-    for (int c = 1; c < n_codebooks; ++c) {
-        int t = tk[c];
-        float v = 0.f;
-        if (t != -1) v = mmi_bf16_to_f32(emb[((long)(c - 1) * card1 + (t < 0 ? 0 : t)) * D + d]);
-        acc = c == 1 ? v : mmi_round_bf16(acc + v);
+    // 16 rows asked for at once (absent ones read row 0): one after the other 17 of them took 10.5 - 12.1 us, here 4.4 - 5.9
+    constexpr int N = 16;
+    for (int c0 = 1; c0 < n_codebooks; c0 += N) {
+        int t[N];
+        uint16_t v[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) t[i] = tk[min(c0 + i, n_codebooks - 1)];
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = emb[((long)(min(c0 + i, n_codebooks - 1) - 1) * card1 + max(t[i], 0)) * D + d];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (c0 + i >= n_codebooks) continue;
+            const float f = t[i] != -1 ? mmi_bf16_to_f32(v[i]) : 0.f;
+            acc = c0 + i == 1 ? f : mmi_round_bf16(acc + f);
+        }
     }
-    int t0 = tk[0];
-    float tv = 0.f;
-    if (t0 != -1) tv = mmi_bf16_to_f32(text_emb[(long)(t0 < 0 ? 0 : t0) * D + d]);
+    const float tv = t0 != -1 ? mmi_bf16_to_f32(text) : 0.f;
     acc = n_codebooks > 1 ? mmi_round_bf16(acc + tv) : tv;
     if (cond) acc = acc + mmi_bf16_to_f32(cond[(long)b * D + d]);
     x[mmi_xp_index(T, b, d, ksteps)] = mmi_f32_to_bf16(acc);
@@ -3366,26 +3376,28 @@ __global__ void k_lm_prepare(TokArgs t, const int* __restrict__ user, int n_user
 }
 
 // 4./5. advance offsets, store the sampled tokens, gather the delayed output frame
-__global__ void k_lm_commit(TokArgs t, const int* __restrict__ text_tok, const int* __restrict__ audio_tok,
+// One wave per session, a lane per stream of tokens (a session's 9 streams one after the other, a 64-bit remainder and a trip to memory each, took
+// 6.3 - 9.3 us, here 4.2).
+__global__ __launch_bounds__(64) void k_lm_commit(TokArgs t, const int* __restrict__ text_tok, const int* __restrict__ audio_tok,
                             int* __restrict__ out, unsigned long long* __restrict__ rng) {
-    int b = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (b == 0) rng[1] += 1ull;
-    if (b >= t.B) return;
+    const int b = (int)blockIdx.x, lane = (int)threadIdx.x;
     const bool ex = t.exec[b] != 0;
-    const long off_new = t.offsets[b] + (ex ? 1 : 0);
-    t.offsets[b] = off_new;
-    const int pos = (int)(off_new % t.CT);
+    const long off_new = t.offsets[b] + (ex ? 1 : 0);      // (every lane has it before lane 0 stores)
     int* rows = t.cache + (long)b * t.NC * t.CT;
-    if (ex) {
-        rows[pos] = text_tok[b];
-        for (int k = 0; k < t.dep_q; ++k) rows[(1 + k) * t.CT + pos] = audio_tok[(long)b * t.dep_q + k];
-    }
     const bool hide = off_new <= (long)t.max_delay || !ex;
-    for (int c = 0; c <= t.dep_q; ++c) {
+    for (int c = lane; c <= t.dep_q; c += 64) {
+        const int now = c == 0 ? text_tok[b] : audio_tok[(long)b * t.dep_q + c - 1];
+        const int pos = (int)(off_new % t.CT);
         long i = (off_new - t.max_delay + t.delays[c]) % t.CT;
         if (i < 0) i += t.CT;
-        int v = rows[c * t.CT + (int)i];
-        out[(long)b * (t.dep_q + 1) + c] = hide ? -2 : v;
+        const int old = rows[c * t.CT + (int)i];
+        if (ex) rows[c * t.CT + pos] = now;
+        out[(long)b * (t.dep_q + 1) + c] = hide ? -2 : (ex && (int)i == pos ? now : old);
+    }
+    __syncthreads();
+    if (lane == 0) {
+        t.offsets[b] = off_new;
+        if (b == 0) rng[1] += 1ull;
     }
 }
 
