@@ -789,7 +789,7 @@ int add_dequant_ops(mmi_mimi* m, MimiMem& mem, const DequantScratch& d, MmiProgr
     if (T > 1 && !packed) return mmi_fail(MMI_ERR_UNSUPPORTED, "dequantising several frames needs the packed operand");
     float* qp = packed ? d.qout_bp : nullptr; const int qQ = m->q_out.Q;
     prog.add([=](hipStream_t s) {
-        MMI_LAUNCH(k_rvq_gather, mmi_cdiv(rows * D, 256), 256, 0, s, codes, nq, K, E, bins, D, nsem, q2, rows, kdev, qp, qQ);
+        MMI_LAUNCH(k_rvq_gather, mmi_cdiv(rows * D, 64), 64, 0, s, codes, nq, K, E, bins, D, nsem, q2, rows, kdev, qp, qQ);
         MMI_CHECK_LAUNCH();
         return (int)MMI_OK;
     });

@@ -1399,8 +1399,17 @@ __global__ void k_commit_all(HistTable tab, int total_rows, const uint8_t* __res
     int row = gid - h.row_begin;
     int b = row / h.C;
     if (!exec[b]) return;
+    // eight at a time, all of them read before one is written (source p + T is always ahead of the write; one by one each waited for the last: 6.0 us for
+    // a stream, here 5.3)
     float* r = h.p + (long)row * h.ld;
-    for (int p = 0; p < h.H; ++p) r[p] = r[p + h.T];  // ascending: source p+T is always ahead of the write
+    for (int p0 = 0; p0 < h.H; p0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = r[min(p0 + i, h.H - 1) + h.T];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (p0 + i < h.H) r[p0 + i] = v[i];
+    }
 }
 
 // the histories of one set of buffers -> the same ones of another
@@ -1413,7 +1422,14 @@ __global__ void k_move_history(HistTable from, HistTable to, int total_rows) {
         if (i < from.n && from.d[i].row_begin <= gid) d = i;
     const HistDesc f = from.d[d], t = to.d[d];
     const long row = gid - f.row_begin;
-    for (int p = 0; p < f.H; ++p) t.p[row * t.ld + p] = f.p[row * f.ld + p];
+    for (int p0 = 0; p0 < f.H; p0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = f.p[row * f.ld + min(p0 + i, f.H - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (p0 + i < f.H) t.p[row * t.ld + p0 + i] = v[i];
+    }
 }
 
 // offsets[i][b] += inc where exec; first[b] = 0 where exec
@@ -2047,14 +2063,25 @@ __global__ void k_rvq_gather(const int* __restrict__ codes, int codes_rstride, i
                              const int* __restrict__ n_codes_dev, float* __restrict__ qp, int qpQ) {
     int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (idx >= Bn * D) return;
-    if (n_codes_dev) n_codes = *n_codes_dev;
     int r = idx / D, d = idx % D;
     float first = 0.f, rest = 0.f;
-    for (int k = 0; k < n_codes; ++k) {
-        int c = codes[(long)r * codes_rstride + k];
-        c = c < 0 ? 0 : (c >= bins ? bins - 1 : c);  // the reference crashes on OOB codes (vq.py:144-146); we clamp
-        float e = Eall[((long)k * bins + c) * D + d];
-        if (k < n_sem) first += e; else rest += e;
+    // eight codes, then their eight entries are asked for at once, whatever their number turns out to be (a row holds codes_rstride codes, as many as
+    // there are codebooks): one after the other, 8 of them took 5.5 - 7 us, here 3.7
+    if (n_codes_dev) n_codes = *n_codes_dev;
+    constexpr int N = 8;
+    for (int k0 = 0; k0 < codes_rstride; k0 += N) {
+        int c[N];
+        float e[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) c[i] = codes[(long)r * codes_rstride + min(k0 + i, codes_rstride - 1)];
+#pragma unroll
+        for (int i = 0; i < N; ++i) e[i] = Eall[((long)min(k0 + i, codes_rstride - 1) * bins + max(0, min(c[i], bins - 1))) * D + d];      // the reference crashes on OOB codes (vq.py:144-146); we clamp
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (k0 + i >= n_codes) continue;
+            if (k0 + i < n_sem) first += e[i]; else rest += e[i];
+        }
+        if (k0 + N >= n_codes) break;
     }
     q[(long)r * 2 * D + d] = first;
     q[(long)r * 2 * D + D + d] = rest;
