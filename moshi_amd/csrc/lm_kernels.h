@@ -740,7 +740,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_xring16(GemmArgs a, MmiMerge g)
     mmi_gemm_epilogue<16, 1, 8, 0>(a, accv, wave, lane, nt0, &pre);
 }
 
-// ONE session: RMSNorm + a weight stream on the 16-row tile (the temporal in_proj and linear_in).  A workgroup's 512 threads normalise the row -
+// ONE session: RMSNorm + a weight stream on the 16-row tile (the temporal in_proj and linear_in; from 512 tiles on k_gemm_xreg16).  A workgroup's 512 threads normalise the row -
 // k_resid_rmsnorm's pieces, sums and roundings, so its bits - into LDS, with the wave's first two groups of weights on their way; the main loop takes its
 // activations from there, 16 bytes for all 16 columns of the tile (column 0 is the session).  The norm was a launch of 4.6 us in front of each, 64 per
 // step; here it costs a workgroup a trip for 8 KB under another workgroup's stream: in_proj 21.6 + 4.6 -> 24.1 us, linear_in 36.3 + 4.6 -> 37.4.
