@@ -2315,11 +2315,12 @@ __global__ __launch_bounds__(256) void k_lm_attn_split(LmAttnArgs a) {
 // running (max, sum, accumulator): a round requests NB key groups AND their NB value groups at once (the values do not depend
 // on the scores), the next round's 2 NB loads are issued before this round's arithmetic, and nothing but registers and
 // cross-lane shuffles is touched until the slots and the waves are merged once at the end.
-// Half of its time are vector instructions (e4m3 ring: 27 of 53 us at 64 sessions of ~500 rows, 137 instructions per row group of 8 rows): dot products of
-// packed pairs for both rings, an exponential is one v_exp_f32 of the difference to the maximum, rescaling only in rounds in which some maximum rises,
-// and the row slots are merged at once, exchanging halves between the rows of lanes instead of summing every element in all of them.
-// us per launch before / here: 64 sessions x 32 heads, e4m3, 263 MB 53.5 / 48.8; 32 sessions, bf16, 196 MB 39.0 / 35.9; one session, 24.6 MB over 12
-// workgroups a head 8.5 / 7.6.  The logits' error against 64 bits is the same (0.025, 0.014, 0.012).
+// Half of its time were vector instructions (e4m3 ring: 27 of 53 us at 64 sessions of ~500 rows, 137 instructions per row group of 8 rows): dot products of
+// packed pairs for both rings, rescaling only in rounds in which some maximum rises, and the row slots are merged at once, exchanging halves between
+// the rows of lanes instead of summing every element in all of them.  Exponentials are expf (0.84 units in the last place at most): 2^x of the
+// product with log2 e in one v_exp_f32 is off by up to 64 of them, more the further a score lies below the maximum, and nothing below 2^-126.
+// us per launch in the step, before / here (/ with that exponential): 64 sessions x 32 heads, e4m3, 263 MB 51.3 / 49.7 (/ 49.3); 32 sessions, bf16, 196 MB
+// 39.2 / 37.9 (/ 37.1); one session, 24.6 MB over 12 workgroups a head 8.8 / 8.4 (/ 8.0).  The logits' error against 64 bits is the same (0.025, 0.014, 0.012).
 template <int DH, bool KV8 = false>
 __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      // <= 128 VGPRs, 4 workgroups per CU
     constexpr int EPL = KV8 ? 16 : 8;  // elements per lane (16 bytes)
@@ -2343,7 +2344,6 @@ __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      //
     const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vc) + (long)bh * a.cap * DH * ES;
     const unsigned loff = (unsigned)(seg * EPL * ES);
     const float scale = 1.0f / sqrtf((float)DH);
-    constexpr float LOG2E = 1.44269504088896340736f;
     // One workgroup per (session, head) (gridDim.y == 1: which wave walks which row group does not depend on the ring depth): the
     // FIRST round's keys and values are requested before the session's offset - a cold scalar load of its own, ~1 us into a
     // ~40 us launch - has come back: row groups wave, wave + 4, ... of the ring's first slots, any of which lies inside the
@@ -2412,15 +2412,14 @@ __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      //
                 if (!(pos_ >= 0 && dq_ >= 0 && dq_ < a.context)) s_[i] = -INFINITY;              \
             }                                                                                    \
         _Pragma("unroll") for (int i = 0; i < NB; ++i) mx_ = fmaxf(mx_, s_[i]);                 \
-        /* exp(x) as 2^(x log2 e) of the DIFFERENCE to the maximum: exact up to the last bits of a difference, whatever the scores are */ \
-        const float top_ = mx_ == -INFINITY ? 0.f : mx_;    /* (a slot without valid rows yet: every factor is 2^-inf = 0) */ \
+        const float top_ = mx_ == -INFINITY ? 0.f : mx_;    /* (a slot without valid rows yet: every factor is e^-inf = 0) */ \
         if (mmi_any(mx_ > m_run)) {                                                              \
-            const float resc_ = mmi_fast_exp2f((m_run - top_) * LOG2E);                          \
+            const float resc_ = expf(m_run - top_);                                              \
             l_run *= resc_;                                                                      \
             _Pragma("unroll") for (int e = 0; e < EPL; ++e) acc[e] *= resc_;                    \
         }                                                                                        \
         _Pragma("unroll") for (int i = 0; i < NB; ++i) {                                        \
-            const float p_ = mmi_fast_exp2f((s_[i] - top_) * LOG2E);                             \
+            const float p_ = expf(s_[i] - top_);                                                 \
             l_run += p_;                                                                         \
             float vf_[EPL];                                                                      \
             _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                     \
@@ -2449,7 +2448,7 @@ __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      //
     // ---- merge the RPW row slots of the wave (lanes that share `seg`) at their common maximum.  Sums across the rows of 16 lanes leave every lane
     // with the half it keeps of what both had: EPL / 4 elements in the end, from EPL / 4 ((lane >> 5) 2 + ((lane >> 4) & 1)) on
     const float m_wave = mmi_slots_max<LPR>(m_run);
-    const float to_wave = m_run == -INFINITY ? 0.f : mmi_fast_exp2f((m_run - m_wave) * LOG2E);
+    const float to_wave = m_run == -INFINITY ? 0.f : expf(m_run - m_wave);
     const float l_wave = mmi_slots_sum<LPR>(l_run * to_wave);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc[e] *= to_wave;
@@ -2478,7 +2477,7 @@ __global__ __launch_bounds__(256, 4) void k_lm_attn_wave(LmAttnArgs a) {      //
         float num = 0.f, den = 0.f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            const float sw = wm[w] == -INFINITY ? 0.f : mmi_fast_exp2f((wm[w] - M) * LOG2E);
+            const float sw = wm[w] == -INFINITY ? 0.f : expf(wm[w] - M);
             num += sw * wacc[w * DH + tid];
             den += sw * wl[w];
         }

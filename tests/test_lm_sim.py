@@ -117,8 +117,7 @@ def test_merge_of_few_and_many_partials(sim_lib, monkeypatch, context):
     lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), context=context), seed=62, B=1, S=4)
 
 
-@pytest.fixture(scope="module")
-def combine(tmp_path_factory):
+def kernel_selftest(folder, name):
     import ctypes
     import subprocess
     import sys
@@ -126,10 +125,56 @@ def combine(tmp_path_factory):
     here = Path(__file__).resolve().parent / "hipsim"
     sys.path.insert(0, str(here))
     import build_sim
-    so = tmp_path_factory.mktemp("combine") / "combine_selftest.so"
+    so = folder / f"{name}.so"
     subprocess.check_call([build_sim._cxx(), "-O1", "-w", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", f"-I{here}", f"-I{build_sim.CSRC}",
-                           str(here / "combine_selftest.cpp"), str(here / "hipsim.cpp"), "-o", str(so)])
+                           str(here / f"{name}.cpp"), str(here / "hipsim.cpp"), "-o", str(so)])
     return ctypes.CDLL(str(so))
+
+
+@pytest.fixture(scope="module")
+def combine(tmp_path_factory):
+    return kernel_selftest(tmp_path_factory.mktemp("combine"), "combine_selftest")
+
+
+@pytest.fixture(scope="module")
+def attention(tmp_path_factory):
+    return kernel_selftest(tmp_path_factory.mktemp("attention"), "attn_selftest")
+
+
+@pytest.mark.parametrize("order", ["top first", "rising", "mixed"])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_exponentials_of_the_decode_attention(attention, kv8, order):
+    """k_lm_attn_wave's probabilities keep fp32's precision at every distance to the maximum, down to the subnormal numbers.  Scores are exact (one
+    feature of the query, an eighth of a power of two), value rows single ones, so that a partial sum IS a probability.  With the maximum in the
+    first rows of every slot a probability is one exponential, otherwise it is rescaled in each round in which the maximum rises and at the two
+    merges: an exponential and a product each, together 2 units of 2^-23.  A sum adds some 30 roundings."""
+    import ctypes
+    import torch
+    H, L, Dh = 3, 600, 64
+    g = torch.Generator().manual_seed(5)
+    steps = torch.tensor([0., 1, 2, 3, 5, 7, 9, 10, 13, 15, 18, 20, 22, 26, 30, 36, 40, 44, 52, 56, 64, 72, 80, 88, 96, 104])     # exact in e4m3 too
+    far = steps[torch.randint(0, len(steps), (H, L), generator=g)]
+    if order == "top first":
+        far[:, :128] = 0.0                                     # (128 rows: 8 waves of 16 slots, each one's first row)
+    elif order == "rising":
+        far = far.sort(dim=1, descending=True).values
+    q, k, v = torch.zeros(H, Dh), torch.zeros(H, L, Dh), torch.zeros(H, L, Dh)
+    q[:, 0], k[:, :, 0] = 8.0, -far
+    rows = torch.stack([torch.randperm(L, generator=g)[:Dh] for _ in range(H)])
+    for h in range(H):
+        v[h, rows[h], torch.arange(Dh)] = 1.0
+    kind = torch.float8_e4m3fn if kv8 else torch.bfloat16
+    q, k, v = q.bfloat16(), k.to(kind), v.to(kind)
+    assert torch.equal(k[:, :, 0].float(), -far)
+    ml, part = torch.empty(H, 2, 2), torch.empty(H, 2, Dh)
+    attention.attn_selftest_run(*(ctypes.c_void_p(t.data_ptr()) if torch.is_tensor(t) else t for t in (q, k, v, H, L, int(kv8), ml, part)))
+    top = -far.double().amin(1, keepdim=True)
+    got = (torch.exp(ml[..., 0].double() - top)[..., None] * part.double()).sum(1)
+    want = torch.exp(-torch.gather(far.double(), 1, rows) - top)
+    rounds = 1 if order == "top first" else 3 + 3              # (600 rows: up to 3 rounds of 4 row groups per wave, the row's own, two merges)
+    assert ((got - want).abs() <= rounds * 2.0 ** -22 * want + rounds * 2.0 ** -149).all(), ((got - want).abs() / want).max()
+    total = (torch.exp(ml[..., 0].double() - top) * ml[..., 1].double()).sum(1)
+    assert ((total - torch.exp(-far.double() - top).sum(1)).abs() <= (rounds + 8) * 2.0 ** -22 * total).all()
 
 
 @pytest.mark.parametrize("top", ["first", "last"])
