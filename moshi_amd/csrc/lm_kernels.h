@@ -964,6 +964,8 @@ __device__ __forceinline__ void mmi_gemm_batch_tile_view(GemmArgs& a, int y, int
 // against 8 products, and at 132 registers it has its CU to itself.  Where the tiles go round the chip a second time two of them share that
 // work (1024 -> 2 x 2816 gated, 352 workgroups -> 176: 64 sessions 14.1 -> 11.5 us, 9 sessions 13.8 -> 11.3; two workgroups per CU at 128
 // registers instead: 13.0).
+// Only the operand is masked past a slice's end (an int8 product with zero is zero): masking the weights too took the registers that the
+// epilogue's operands, asked for first, need at 2816 features (8 sessions 7.8 us, here 6.6).
 template <int TN, int MT, int WAVES, int KMAX, bool NORM, int NTW = 1>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     GemmArgs a = a_in;
@@ -973,7 +975,6 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     constexpr int XMAX = 2 * KMAX;
     // batch tiles handled together: both while a lane's fragments of both fit its registers (short rows), else one after the other
     constexpr int MG = (MT * XMAX <= 16) ? MT : 1;
-    constexpr bool PRE = TN == 32 || KMAX <= 4;               // the epilogue's operands first (long slices on the 16-row tile leave no registers for them)
     typedef int iacc_t __attribute__((ext_vector_type(R)));
     typedef float facc_t __attribute__((ext_vector_type(R)));
     const int wave = mmi_uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
@@ -991,10 +992,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
     MmiEpiPre pre[NTW];
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
-        if constexpr (PRE) pre[t] = mmi_epi_prefetch<TN, MT, WAVES, 3>(a, wave, lane, nt0 + t);
+        pre[t] = mmi_epi_prefetch<TN, MT, WAVES, 3>(a, wave, lane, nt0 + t);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     const int ksl = min(ks0, a.KSTEPS - 1);
-    u32x4 wv[NTW][KMAX];
+    u32x4 wv[NTW][KMAX];                                 // (past the slice its last entries again: they meet zeros)
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
@@ -1002,10 +1003,6 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
             const int uu = min(u, nks > 0 ? nks - 1 : 0);
             wv[t][u] = mmi_load_nt(a.wp + ((long)min(nt0 + t, a.NT - 1) * a.KSTEPS + ksl + uu) * 64 + wlane);
         }
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-        for (int u = 0; u < KMAX; ++u) if (u >= nks) wv[t][u] = zero;
     MMI_SHARED float sxl[MT * TN];                       // the rows' absmax, for the epilogue
     MMI_SHARED float redl[2][WAVES][MG][TN];             // [0] sums of squares, [1] absmax, per wave and tile of the group
     iacc_t acc[NTW][MT];
@@ -1117,7 +1114,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_q8(GemmArgs a_in) {
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int r = 0; r < R; ++r) accv[m][r] = __builtin_bit_cast(facc_t, acc[t][m])[r];     // int32 bit patterns (see the epilogue)
-        if (nt0 + t < a.NT) mmi_gemm_epilogue<TN, MT, WAVES, 3>(a, accv, wave, lane, nt0 + t, PRE ? &pre[t] : nullptr, nullptr, g_lo, g_hi, sxl);
+        if (nt0 + t < a.NT) mmi_gemm_epilogue<TN, MT, WAVES, 3>(a, accv, wave, lane, nt0 + t, &pre[t], nullptr, g_lo, g_hi, sxl);
     }
 }
 

@@ -1,8 +1,12 @@
-"""scripts/rocpd_sites.py: the join of the engine's launch list with a rocprofv3 kernel trace, on a synthetic trace."""
+"""The scripts that read traces and the built library: rocpd_sites.py and rocpd_pmc.py on synthetic traces, the code objects' instructions and registers."""
+import csv
+import re
 import sqlite3
 import subprocess
 import sys
 from pathlib import Path
+
+import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -92,8 +96,23 @@ def test_built_library_has_no_in_place_cross_swizzled_packed_fp32_instruction():
     root = Path(__file__).resolve().parent.parent
     lib = root / "moshi_amd" / "libmoshi_mi.so"
     if not lib.exists():
-        import pytest
         pytest.skip("the HIP library is not built")
     r = subprocess.run([sys.executable, str(root / "scripts" / "isa_scan_packed_swizzle.py"), str(lib)], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stderr
     assert r.stdout.strip().splitlines()[-1].startswith("0 kernel(s)"), r.stdout[-2000:]
+
+
+def kernel_resources(lib):
+    """scripts/kernel_resources.py's table of a built library: kernel -> column -> number"""
+    r = subprocess.run([sys.executable, str(ROOT / "scripts" / "kernel_resources.py"), str(lib)], capture_output=True, text=True, timeout=600, check=True)
+    return {row.pop("kernel"): {k: int(v) for k, v in row.items()} for row in csv.DictReader(r.stdout.splitlines())}
+
+
+def test_registers_that_launches_count_on():
+    """k_gemm_q8 of one batch tile keeps weights, operand and the epilogue's operands of a whole slice in registers, none of them in scratch memory."""
+    lib = ROOT / "moshi_amd" / "libmoshi_mi.so"
+    if not lib.exists():
+        pytest.skip("the library is not built")
+    table = kernel_resources(lib)
+    q8 = [n for n in table if re.match(r"k_gemm_q8<\d+, 1,", n)]
+    assert q8 and all(table[n]["scratch_bytes"] == 0 for n in q8)
