@@ -443,8 +443,10 @@ __device__ __forceinline__ void mmi_gemm_epilogue(const GemmArgs& a, float (&acc
 // reduction + epilogue runs under the other's weight stream (136 registers unbounded; 8 spill, outside the loop).  Same-box at
 // 1 / 8 / 16 sessions: -0.12 / -0.14 / -0.12 ms per step (in_proj 20.9 -> 19.4 us, linear_in 38.4 -> 35.5, text head 48.9 ->
 // 44.2; profiles/r04_logs/call_m_summary.txt).
+// So are two batch tiles (33 - 64 sessions; 154 unbounded, 122 bounded, no spill): the text head's 1000 workgroups, 40 sessions 67.7 -> 63.5 us, 64
+// sessions 68.0 -> 63.2.
 template <int TN, int MT, int NTW, int WAVES, int U, int WQ = 0>
-__global__ __launch_bounds__(WAVES * 64, (TN == 16 && MT == 1 && NTW == 1 && WQ == 0 && WAVES == 8) ? 4 : 1) void k_gemm_xp(GemmArgs a) {
+__global__ __launch_bounds__(WAVES * 64, (NTW == 1 && WQ == 0 && WAVES == 8 && ((TN == 16 && MT == 1) || (TN == 32 && MT == 2))) ? 4 : 1) void k_gemm_xp(GemmArgs a) {
     constexpr bool W8 = WQ == 1;
     constexpr int R = TN == 32 ? 16 : 4;          // accumulator registers per MFMA tile
     constexpr int XS = (WQ == 1 || WQ == 2) ? 2 : 1;   // activation fragments per weight entry

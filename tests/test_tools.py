@@ -109,10 +109,13 @@ def kernel_resources(lib):
 
 
 def test_registers_that_launches_count_on():
-    """k_gemm_q8 of one batch tile keeps weights, operand and the epilogue's operands of a whole slice in registers, none of them in scratch memory."""
+    """k_gemm_q8 of one batch tile keeps weights, operand and the epilogue's operands of a whole slice in registers, none of them in scratch memory.
+    k_gemm_xp's 8-wave forms for bf16 weights on full tiles (one of 16 rows, two of 32) have two workgroups on a CU."""
     lib = ROOT / "moshi_amd" / "libmoshi_mi.so"
     if not lib.exists():
         pytest.skip("the library is not built")
     table = kernel_resources(lib)
     q8 = [n for n in table if re.match(r"k_gemm_q8<\d+, 1,", n)]
     assert q8 and all(table[n]["scratch_bytes"] == 0 for n in q8)
+    xp = [n for n in table if re.match(r"k_gemm_xp<(16, 1|32, 2), 1, 8, \d, 0>", n)]
+    assert len(xp) == 3 and all(table[n]["waves_per_simd"] >= 4 and table[n]["scratch_bytes"] == 0 for n in xp), {n: table[n] for n in xp}
