@@ -448,6 +448,7 @@ int launch_xlds(hipStream_t s, const XldsPlan& p, const GemmArgs& a) {
 // registers: k_gemm_xlds), 128 tiles or more - with fewer there is no second tile per workgroup to stream under the first one's epilogue.
 // MMI_GEMM_REG: "0" = off, a number = every GEMM whose slices fit, on so many workgroups (tests on tiny shapes).
 struct XregPlan { int nx, ksplit, grid; size_t smem; };
+constexpr int xreg_ring(int nx) { return nx == 22 ? 11 : (nx >= 16 ? 8 : nx); }      // weights on their way, of the nx entries of a slice (32-row tile)
 int xreg_entries(int T, int mt, int wq, int kper) {
     if (T == 16 && mt == 1 && wq == 0) return kper <= 4 ? 4 : (kper <= 16 ? 16 : 0);
     if (T == 32 && mt == 1 && wq == 0) return kper <= 8 ? 8 : (kper <= 22 ? 22 : (kper <= 32 ? 32 : 0));
@@ -485,8 +486,9 @@ XregPlan plan_xreg(const GemmW& g, int epi, int wq, int B, int Dh) {
     return p;
 }
 
-template <int MT, int NX, int RD, int WQ>
+template <int MT, int NX, int WQ>
 int launch_xreg_v(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
+    constexpr int RD = xreg_ring(NX);
     static bool attr_set = false;
     if (!attr_set) {
         MMI_HIP_CHECK(hipFuncSetAttribute((const void*)k_gemm_xreg<MT, NX, RD, WQ>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
@@ -506,18 +508,18 @@ int launch_xreg16(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
 int launch_xreg(hipStream_t s, const XregPlan& p, int T, int mt, const GemmArgs& a) {
     if (T == 16) return launch_xreg16<false>(s, p, a);
     if (a.wq == 0) {
-        if (p.nx == 8) return launch_xreg_v<1, 8, 8, 0>(s, p, a);
-        if (p.nx == 22) return launch_xreg_v<1, 22, 11, 0>(s, p, a);
-        return launch_xreg_v<1, 32, 8, 0>(s, p, a);
+        if (p.nx == 8) return launch_xreg_v<1, 8, 0>(s, p, a);
+        if (p.nx == 22) return launch_xreg_v<1, 22, 0>(s, p, a);
+        return launch_xreg_v<1, 32, 0>(s, p, a);
     }
     if (mt == 1) {
-        if (p.nx == 4) return launch_xreg_v<1, 4, 4, 3>(s, p, a);
-        if (p.nx == 11) return launch_xreg_v<1, 11, 11, 3>(s, p, a);
-        return launch_xreg_v<1, 16, 8, 3>(s, p, a);
+        if (p.nx == 4) return launch_xreg_v<1, 4, 3>(s, p, a);
+        if (p.nx == 11) return launch_xreg_v<1, 11, 3>(s, p, a);
+        return launch_xreg_v<1, 16, 3>(s, p, a);
     }
-    if (p.nx == 4) return launch_xreg_v<2, 4, 4, 3>(s, p, a);
-    if (p.nx == 11) return launch_xreg_v<2, 11, 11, 3>(s, p, a);
-    return launch_xreg_v<2, 16, 8, 3>(s, p, a);
+    if (p.nx == 4) return launch_xreg_v<2, 4, 3>(s, p, a);
+    if (p.nx == 11) return launch_xreg_v<2, 11, 3>(s, p, a);
+    return launch_xreg_v<2, 16, 3>(s, p, a);
 }
 
 // k_gemm_xring16 for slices of 16 k-steps and more behind at most one workgroup per CU, bf16 on the 16-row tile: entries of its ring, 0 = another
@@ -575,7 +577,7 @@ hipError_t dominant_begin(mmi_lm* lm, hipStream_t s, EvPair** ev) {
     return hipEventRecord((*ev)->a, s);
 }
 
-// its name with the instantiation (launch_xlds, launch_gemm_w) and what it computes; valid for ever, whoever holds it
+// its name with the instantiation (launch_xreg, launch_xlds, launch_gemm_w) and what it computes; valid for ever, whoever holds it
 const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XregPlan& xr, const XldsPlan& xl, int mt, int wq) {
     const std::string on = wq == 3 ? ", int8 weights x int8 activations" : (wq == 1 ? ", int8 weights" : (wq == 2 ? ", fp8 weights on the fp8 MFMA" : ""));
     const auto args = [](std::initializer_list<int> v) {
@@ -585,7 +587,7 @@ const char* dominant_kernel(const GemmW& g, const GemmPlan& p, const XregPlan& x
     };
     const int u = wq == 0 ? (p.waves == 8 && p.u == 2 && mt == 1 ? 2 : 4) : (wq == 3 && q8_four() && p.waves == 8 ? 4 : 2);
     std::string k = xr.nx && g.T == 16 ? "k_gemm_xreg16" + args({xr.nx}) + ", false"
-                  : xr.nx ? "k_gemm_xreg" + args({mt, xr.nx, xr.nx > 16 ? xr.nx / 2 : xr.nx, wq})
+                  : xr.nx ? "k_gemm_xreg" + args({mt, xr.nx, xreg_ring(xr.nx), wq})
                   : xl.on ? "k_gemm_xlds" + args({mt, xl.kc, 3}) + (xl.stagger ? ", true, " : ", false, ") + std::to_string(wq)
                           : "k_gemm_xp" + args({g.T, mt, 1, p.waves, u}) + (wq ? ", " + std::to_string(wq) : "");
     static std::mutex names_lock;

@@ -693,16 +693,23 @@ def test_norm_and_linear_in_one_launch(sim_lib, dim, heads):
     assert st["launch_sites"].get("L.norm1", 0) == 0 and st["launch_sites"].get("L.in_proj", 0) == 2
 
 
-@pytest.mark.parametrize("B,quantize,switch,kernel", [
-    (1, False, None, "k_gemm_norm_one<4>"), (1, False, "MMI_NO_NORM_FUSION", "k_gemm_xp<16, 1, 1, 4, 4>"), (3, False, None, "k_gemm_xp<16, 1, 1, 4, 4>"),
-    (18, False, None, "k_gemm_xp<32, 1, 1, 4, 4>"), (34, False, None, "k_gemm_xp<32, 2, 1, 4, 4>"), (3, True, None, "k_gemm_xp<16, 1, 1, 4, 2, 3>"),
+@pytest.mark.parametrize("B,quantize,switch,dim,kernel", [
+    (1, False, None, 128, "k_gemm_norm_one<4>"), (1, False, "MMI_NO_NORM_FUSION", 128, "k_gemm_xp<16, 1, 1, 4, 4>"), (3, False, None, 128, "k_gemm_xp<16, 1, 1, 4, 4>"),
+    (18, False, None, 128, "k_gemm_xp<32, 1, 1, 4, 4>"), (34, False, None, 128, "k_gemm_xp<32, 2, 1, 4, 4>"), (3, True, None, 128, "k_gemm_xp<16, 1, 1, 4, 2, 3>"),
+    (1, False, "MMI_GEMM_REG", 128, "k_gemm_xreg16<4, true>"), (3, False, "MMI_GEMM_REG", 128, "k_gemm_xreg16<4, false>"),
+    (18, False, "MMI_GEMM_REG", 128, "k_gemm_xreg<1, 8, 8, 0>"), (18, False, "MMI_GEMM_REG", 1152, "k_gemm_xreg<1, 22, 11, 0>"),
+    (18, False, "MMI_GEMM_REG", 2880, "k_gemm_xreg<1, 32, 8, 0>"), (34, True, "MMI_GEMM_REG", 128, "k_gemm_xreg<2, 4, 4, 3>"),
+    (34, True, "MMI_GEMM_REG", 1152, "k_gemm_xreg<2, 11, 11, 3>"), (18, True, "MMI_GEMM_REG", 2880, "k_gemm_xreg<1, 16, 8, 3>"),
+    (34, True, "MMI_GEMM_REG", 2880, "k_gemm_xreg<2, 16, 8, 3>"),
 ])
-def test_profile_names_the_kernel_it_timed(sim_lib, monkeypatch, B, quantize, switch, kernel):
-    """mmi_lm_profile_end's name is that of the launches between its events: the one the launch list has at the same site, at its tile."""
+def test_profile_names_the_kernel_it_timed(sim_lib, monkeypatch, B, quantize, switch, dim, kernel):
+    """mmi_lm_profile_end's name is that of the launches between its events: the one the launch list has at the same site, at its tile; with its
+    instantiation, whose slices and rings depend on the width (2880 features: 23 k-steps of bf16 and 12 of int8 per wave)."""
     import ctypes as C
+    from dataclasses import replace
     if switch:
-        monkeypatch.setenv(switch, "1")
-    cfg = tiny_lm_config()
+        monkeypatch.setenv(switch, "8" if switch == "MMI_GEMM_REG" else "1")
+    cfg = tiny_lm_config() if dim == 128 else replace(tiny_lm_config(), dim=dim, num_heads=dim // 64, num_layers=1, hidden_scale=0.125)
     gen = LMGen(LMModel(random_lm_state_dict(cfg, seed=4), cfg, device="cpu", max_batch=B, lib=sim_lib, quantize=quantize), use_sampling=False)
     h, us, n, nbytes, name = gen.lm_model._handle, C.c_double(), C.c_int64(), C.c_int64(), C.c_char_p()
     with gen.streaming(B):
