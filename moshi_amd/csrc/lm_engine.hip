@@ -7,6 +7,7 @@
 
 #include <math.h>
 #include <stdio.h>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <set>
@@ -414,13 +415,21 @@ XldsPlan plan_xlds(const mmi_lm* lm, const GemmW& g, const GemmArgs& a, int mt) 
     return p;
 }
 
+// up to 128 KiB of dynamic LDS for a kernel: an attribute of the kernel on one device, asked for once on each (`asked`: a bit per device, the kernel's
+// own).  Threads whose first launches meet may both ask
+int allow_lds(const void* kernel, std::atomic<uint64_t>& asked) {
+    int device = 0;
+    MMI_HIP_CHECK(hipGetDevice(&device));
+    const uint64_t bit = 1ull << (device & 63);
+    if (asked.load() & bit) return MMI_OK;
+    MMI_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+    asked |= bit;
+    return MMI_OK;
+}
 template <int MT, int KC, bool STAGGER, int WQ>
 int launch_xlds_v(hipStream_t s, const XldsPlan& p, const GemmArgs& a) {
-    static bool attr_set = false;
-    if (!attr_set) {
-        MMI_HIP_CHECK(hipFuncSetAttribute((const void*)k_gemm_xlds<MT, KC, 3, STAGGER, WQ>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        attr_set = true;
-    }
+    static std::atomic<uint64_t> asked{0};
+    if (const int rc = allow_lds((const void*)k_gemm_xlds<MT, KC, 3, STAGGER, WQ>, asked)) return rc;
     MMI_LAUNCH((k_gemm_xlds<MT, KC, 3, STAGGER, WQ>), p.grid, 512, p.smem, s, a);
     MMI_CHECK_LAUNCH();
     return MMI_OK;
@@ -489,11 +498,8 @@ XregPlan plan_xreg(const GemmW& g, int epi, int wq, int B, int Dh) {
 template <int MT, int NX, int WQ>
 int launch_xreg_v(hipStream_t s, const XregPlan& p, const GemmArgs& a) {
     constexpr int RD = xreg_ring(NX);
-    static bool attr_set = false;
-    if (!attr_set) {
-        MMI_HIP_CHECK(hipFuncSetAttribute((const void*)k_gemm_xreg<MT, NX, RD, WQ>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        attr_set = true;
-    }
+    static std::atomic<uint64_t> asked{0};
+    if (const int rc = allow_lds((const void*)k_gemm_xreg<MT, NX, RD, WQ>, asked)) return rc;
     MMI_LAUNCH((k_gemm_xreg<MT, NX, RD, WQ>), dim3(p.grid, p.ksplit), 512, p.smem, s, a);
     MMI_CHECK_LAUNCH();
     return MMI_OK;

@@ -3,6 +3,7 @@
 
 #include <ucontext.h>
 #include <sys/mman.h>
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -439,8 +440,26 @@ hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return failed(hipErrorNotSupported); }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
-hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+// devices share the host's memory; function attributes are a device's own
+static thread_local int t_device = 0;
+static std::mutex g_attr_mu;
+static std::vector<std::pair<const void*, int>> g_attrs;
+hipError_t hipGetDevice(int* d) { *d = t_device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { t_device = d; return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int) {
+    std::lock_guard<std::mutex> g(g_attr_mu);
+    g_attrs.emplace_back(f, t_device);
+    return hipSuccess;
+}
+extern "C" void hipsim_set_device(int device) { t_device = device; }
+// functions that have an attribute on a device
+extern "C" int hipsim_attributes(int device) {
+    std::lock_guard<std::mutex> g(g_attr_mu);
+    std::vector<const void*> fs;
+    for (auto& a : g_attrs) if (a.second == device) fs.push_back(a.first);
+    std::sort(fs.begin(), fs.end());
+    return (int)(std::unique(fs.begin(), fs.end()) - fs.begin());
+}
 
 // C entry points for the tests (ctypes): 0 forward, 1 reverse, 2 random (seed)
 extern "C" void hipsim_set_schedule(int mode, unsigned long long seed) { hipsim::set_schedule(mode, seed); }

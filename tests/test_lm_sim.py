@@ -301,6 +301,26 @@ def test_gemm_with_activations_resident_in_registers(sim_lib, monkeypatch, B, gr
         assert any("[splitk]" in n for n, _ in lm_cases.int8_linears_bit_exact("cpu", sim_lib, tiny_lm_config(), B, seed=192 + B))
 
 
+@pytest.mark.parametrize("env", [{"MMI_GEMM_REG": "8"}, {"MMI_GEMM_LDS": "2", "MMI_GEMM_LDS_GRID": "8"}])
+def test_large_lds_is_asked_for_on_every_device(sim_lib, monkeypatch, env):
+    """How much LDS a kernel may have is an attribute of the kernel on ONE device: a second handle of the process, on another device, asks for its own
+    kernels again (once, however many steps and handles follow)."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    cfg, dll, asked = tiny_lm_config(), sim_lib.cdll, []
+    sd = random_lm_state_dict(cfg, seed=4)
+    for device in (41, 42, 41):
+        dll.hipsim_set_device(device)
+        try:
+            gen = LMGen(LMModel(sd, cfg, device="cpu", max_batch=18, lib=sim_lib), use_sampling=False)
+            with gen.streaming(18):
+                gen.step(torch.zeros(18, 8, 1, dtype=torch.long))
+        finally:
+            dll.hipsim_set_device(0)
+        asked.append(dll.hipsim_attributes(device))
+    assert asked[0] >= 1 and asked == [asked[0]] * 3
+
+
 @pytest.mark.parametrize("B,grid,kv", [(1, 3, "bf16"), (2, 5, "bf16"), (16, 7, "fp8"), (3, 64, "bf16")])
 def test_gemm_with_activations_resident_in_registers_on_the_16_row_tile(sim_lib, monkeypatch, B, grid, kv):
     """k_gemm_xreg16 forced onto every linear of the tiny model that it can hold: one session and a full tile, shares of whole tiles and of single
