@@ -294,11 +294,31 @@ def test_gemm_with_activations_resident_in_registers(sim_lib, monkeypatch, B, gr
     monkeypatch.setenv("MMI_GEMM_REG", str(grid))
     st = {}
     lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=190 + B, B=B, S=2, quantize=quantize, stats=st)
-    assert st["xlds_launches"] >= 2 * (2 * 2 + 1)
+    assert {("L.in_proj", "k_gemm_xreg"), ("L.ffn_in", "k_gemm_xreg"), ("text_linear", "k_gemm_xreg")} <= set(st["launch_list"])
     monkeypatch.setenv("MMI_GEMM_KSPLIT", "2")
     lm_cases.oracle_vs_engine("cpu", sim_lib, tiny_lm_config(), seed=191 + B, B=B, S=2, quantize=quantize)
     if quantize:
         assert any("[splitk]" in n for n, _ in lm_cases.int8_linears_bit_exact("cpu", sim_lib, tiny_lm_config(), B, seed=192 + B))
+
+
+@pytest.mark.parametrize("B,quantize,dim,hidden,sites", [
+    (18, False, 2880, 240, ("L.in_proj", "L.out_proj", "L.ffn_in")),       # 23 of 32 k-steps per wave, 8 under way; the last wave 19
+    (34, True, 2880, 240, ("L.in_proj", "L.out_proj", "L.ffn_in")),        # 12 of 16 entries, 8 under way; the last wave 6
+    (18, False, 128, 3000, ("L.ffn_out",)),                                # 12 of 22 k-steps, 11 under way
+    (18, False, 128, 6000, ("L.ffn_out",)),                                # 24 of 32
+    (18, True, 128, 6000, ("L.ffn_out",)), (34, True, 128, 6000, ("L.ffn_out",)),      # 12 of 16
+])
+def test_gemm_with_long_slices_resident_in_registers(sim_lib, monkeypatch, B, quantize, dim, hidden, sites):
+    """k_gemm_xreg where the ring goes round inside a tile and on into the next one, several tiles per workgroup, slices shorter than the registers
+    hold and shorter still in the last wave: with every epilogue at 2880 features, with split sums in linear_out."""
+    from dataclasses import replace
+    monkeypatch.setenv("MMI_GEMM_REG", "32" if dim > 128 else "4")
+    monkeypatch.setenv("MMI_GEMM_KSPLIT", "2")
+    st = {}
+    cfg = replace(tiny_lm_config(), dim=dim, num_heads=dim // 64, num_layers=1, hidden_scale=1.5 * hidden / dim)
+    assert cfg.ffn_hidden == hidden
+    lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=200 + B, B=B, S=2, quantize=quantize, stats=st)
+    assert {(s, "k_gemm_xreg") for s in sites} <= set(st["launch_list"])
 
 
 @pytest.mark.parametrize("env", [{"MMI_GEMM_REG": "8"}, {"MMI_GEMM_LDS": "2", "MMI_GEMM_LDS_GRID": "8"}])
@@ -323,25 +343,31 @@ def test_large_lds_is_asked_for_on_every_device(sim_lib, monkeypatch, env):
 
 @pytest.mark.parametrize("B,grid,kv", [(1, 3, "bf16"), (2, 5, "bf16"), (16, 7, "fp8"), (3, 64, "bf16")])
 def test_gemm_with_activations_resident_in_registers_on_the_16_row_tile(sim_lib, monkeypatch, B, grid, kv):
-    """k_gemm_xreg16 forced onto every linear of the tiny model that it can hold: one session and a full tile, shares of whole tiles and of single
-    row octets, more workgroups than tiles, waves without entries of their own, both rings."""
+    """k_gemm_xreg16 forced onto every linear of the tiny model that it can hold: one session (norms inside) and a full tile, shares of whole tiles and
+    of single row octets, more workgroups than tiles, waves without entries of their own, both rings; at 1152 features slices of 5 of 16 k-steps, the
+    last wave's of 1."""
     from dataclasses import replace
     monkeypatch.setenv("MMI_GEMM_REG", str(grid))
-    st = {}
-    lm_cases.oracle_vs_engine("cpu", sim_lib, replace(tiny_lm_config(), kv_cache_dtype=kv), seed=230 + B, B=B, S=2, stats=st)
-    assert st["xlds_launches"] >= 2 * (2 if B > 1 else 0) + 2
+    for cfg in (tiny_lm_config(), replace(tiny_lm_config(), dim=1152, num_heads=18, num_layers=1, hidden_scale=0.125)):
+        st = {}
+        lm_cases.oracle_vs_engine("cpu", sim_lib, replace(cfg, kv_cache_dtype=kv), seed=230 + B, B=B, S=2, stats=st)
+        assert {("L.in_proj", "k_gemm_xreg16"), ("L.ffn_in", "k_gemm_xreg16"), ("text_linear", "k_gemm_xreg16")} <= set(st["launch_list"])
+        assert (st["launch_sites"].get("L.norm1", 0) == 0) == (B == 1)
 
 
 @pytest.mark.parametrize("B,hidden_scale", [(1, 4.125), (3, 4.125), (16, 4.125), (1, 135.0), (5, 270.0)])
 def test_gemm_whose_operands_pass_in_a_ring(sim_lib, monkeypatch, B, hidden_scale):
     """k_gemm_xring16 forced onto every linear of the tiny model that it can hold: slices shorter than its ring, and linear_out of 23 and 45 k-steps per
-    wave (rounds of the ring that end inside it)."""
+    wave (rounds of the ring that end inside it; unsplit, as 11264 features of 256 tiles are)."""
     from dataclasses import replace
     monkeypatch.setenv("MMI_GEMM_RING", "2")
     monkeypatch.setenv("MMI_GEMM_OSPLIT", "0")
+    monkeypatch.setenv("MMI_GEMM_KSPLIT", "1")
     cfg = replace(tiny_lm_config(), hidden_scale=hidden_scale, num_layers=2 if hidden_scale < 100 else 1, dim=128 if hidden_scale < 100 else 64,
                   num_heads=4 if hidden_scale < 100 else 2)
-    lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=260 + B, B=B, S=2)
+    st = {}
+    lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=260 + B, B=B, S=2, stats=st)
+    assert {("L.out_proj", "k_gemm_xring16"), ("L.ffn_out", "k_gemm_xring16")} <= set(st["launch_list"])
 
 
 @pytest.mark.parametrize("NS,dim,heads", [(2, 128, 4), (3, 256, 4), (12, 512, 4), (12, 1024, 32)])
@@ -356,7 +382,7 @@ def test_partials_merged_inside_out_proj(sim_lib, monkeypatch, NS, dim, heads):
     cfg = replace(tiny_lm_config(), dim=dim, num_heads=heads, num_layers=1, context=40)
     st = {}
     lm_cases.oracle_vs_engine("cpu", sim_lib, cfg, seed=270 + NS, B=1, S=9, stats=st)
-    assert "k_lm_attn_combine" not in {k for _, k in st["launch_list"]}
+    assert "k_lm_attn_combine" not in {k for _, k in st["launch_list"]} and ("L.out_proj", "k_gemm_xring16") in st["launch_list"]
 
 
 def test_depformer_in_per_step_launches(sim_lib, monkeypatch):

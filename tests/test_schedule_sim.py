@@ -69,10 +69,16 @@ def test_perturbed_schedules_expose_a_missing_barrier(sim_lib, tmp_path):
 
 @pytest.mark.parametrize("B,quantize,env", [
     (3, False, {}),                                                    # 16-row tiles, the one-session style kernels
-    (18, False, {"MMI_GEMM_LDS": "2", "MMI_GEMM_KSPLIT": "2"}),        # 32-row tile, LDS-resident GEMM with split-K (the benchmark's form)
+    (18, False, {"MMI_GEMM_LDS": "2", "MMI_GEMM_KSPLIT": "2"}),        # 32-row tile, LDS-resident GEMM with split-K
     (34, True, {}),                                                    # two batch tiles, int8 x int8: k_gemm_xp<32, 2> + k_gemm_q8 per tile
     (5, "fp8", {"MMI_ATTN_NS": "3"}),                                  # fp8 MFMA; the ring split over workgroups + merge
     (18, False, {"MMI_GEMM_ONCE": "a", "MMI_GEMM_LDS": "0"}),          # k_gemm_xp_once on every GEMM whose slices fit
+    (18, False, {"MMI_GEMM_REG": "5"}),                                # k_gemm_xreg: register-resident activations, sums of the waves per tile
+    (34, True, {"MMI_GEMM_REG": "8"}),                                 # ... of two batch tiles at int8
+    (1, False, {"MMI_GEMM_REG": "3"}),                                 # k_gemm_xreg16 with the norm inside: two scratches in turn, one meeting per tile
+    (16, False, {"MMI_GEMM_REG": "3"}),                                # ... of a full tile of sessions
+    (5, False, {"MMI_GEMM_RING": "2", "MMI_GEMM_OSPLIT": "0", "MMI_GEMM_KSPLIT": "1"}),                                 # k_gemm_xring16
+    (1, False, {"MMI_GEMM_RING": "2", "MMI_GEMM_OSPLIT": "0", "MMI_ATTN_NS": "3", "MMI_ATTN_SOLO": "0"}),               # ... that merges the attention's partials
     (9, "guided-cross", {}),                                           # guidance twins + cross-attention block + k_cfg_mix
 ])
 def test_lm_step_is_independent_of_the_wave_schedule(sim_lib, monkeypatch, B, quantize, env):
