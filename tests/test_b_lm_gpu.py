@@ -168,30 +168,36 @@ def test_c5_int8_engine_against_the_reference_at_full_depth(gpu_lib):
 
 @pytest.mark.parametrize("B", [40, 64])
 def test_two_batch_tiles_at_full_width_match_oracle(gpu_lib, B):
-    """33..64 sessions at the 7B layer shapes on the DEFAULT GEMM path (k_gemm_xp with two batch tiles per weight fragment:
-    what 64 sessions run on)."""
+    """33..64 sessions at the 7B layer shapes on the default GEMM paths (k_gemm_xlds, k_gemm_xp with two batch tiles per weight fragment), masked."""
     cfg = LMConfig(num_layers=2, context=64)
     lm_cases.oracle_vs_engine(DEV, None, cfg, seed=300 + B, B=B, S=2, use_masks=True)
 
 
-@pytest.mark.parametrize("B", [18, 40])
-def test_lds_resident_gemm_is_the_default_at_full_width(gpu_lib, B):
-    """The default path of the wide temporal GEMMs at 17..64 sessions: k_gemm_xlds with the staggered tail (activations staged in
-    LDS, one workgroup per CU walking 1-3 n-tiles, each tile's epilogue under the last chunk's weight stream), one and two
-    batch tiles, against the oracle - and the engine reports that it took that kernel."""
+@pytest.mark.parametrize("B,quantize,wide,resid", [
+    (1, False, "k_gemm_xreg16", "k_gemm_xring16"), (9, False, "k_gemm_xreg16", "k_gemm_xring16"), (18, False, "k_gemm_xreg", "k_gemm_xreg"),
+    (40, False, "k_gemm_xlds", "k_gemm_xp"), (18, True, "k_gemm_xreg", "k_gemm_xreg"), (40, True, "k_gemm_xreg", "k_gemm_xreg"),
+])
+def test_gemms_with_resident_activations_are_the_default_at_full_width(gpu_lib, B, quantize, wide, resid):
+    """The default paths of the temporal GEMMs at the 7B widths against the oracle, and by name where they run: in_proj and the gated linear_in with
+    their activations in registers (k_gemm_xreg16 up to 16 sessions, at one with the norm inside; k_gemm_xreg beyond, to 64 at int8) or in LDS
+    (k_gemm_xlds with the staggered tail: two batch tiles of bf16); out_proj and linear_out through a ring (k_gemm_xring16), in split sums
+    (k_gemm_xreg), or on k_gemm_xp."""
     st = {}
-    lm_cases.oracle_vs_engine(DEV, None, LMConfig(num_layers=2, context=64), seed=15, B=B, S=2, use_masks=False, stats=st)
-    assert st["xlds_launches"] >= 2 * 2 + 1
+    lm_cases.oracle_vs_engine(DEV, None, LMConfig(num_layers=2, context=64), seed=15, B=B, S=2, use_masks=False, quantize=quantize, stats=st)
+    took = set(st["launch_list"])
+    assert {("L.in_proj", wide), ("L.ffn_in", wide), ("L.out_proj", resid), ("L.ffn_out", resid)} <= took
+    assert (st["launch_sites"].get("L.norm1", 0) == 0) == (B == 1)
+    assert st["xlds_launches"] >= 2 * 2
 
 
 def test_step_hooks_see_and_modify_the_step_like_the_reference(gpu_lib):
     lm_cases.check_step_hooks(DEV, None)
 
 
-@pytest.mark.parametrize("B", [2, 4])
+@pytest.mark.parametrize("B", [1, 2, 4])
 def test_ring_wraps_at_the_real_capacity(gpu_lib, B):
-    """2 sessions: the ring split over 12 workgroups + merge launch; 4: one workgroup per (session, head) over all 3000 rows."""
-    lm_cases.ring_wrap_at_real_capacity(DEV, None, B=B, S=14 if B == 2 else 7, seed=91 if B == 2 else 92)
+    """1 session: the ring split over 12 workgroups, merged inside out_proj; 2: a merge launch; 4: one workgroup per (session, head) over all 3000 rows."""
+    lm_cases.ring_wrap_at_real_capacity(DEV, None, B=B, S=14 if B <= 2 else 7, seed=92 if B == 4 else 91)
 
 
 def _greedy_run(cfg, sd, B, codes, steps, graph=True, monkeypatch=None):
