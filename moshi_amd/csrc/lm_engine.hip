@@ -290,8 +290,9 @@ GemmPlan plan_gemm(const GemmW& g, bool may_split) {
     }
     const int ks = g.KSTEPS / p.ksplit;
     p.waves = ks >= 32 ? 8 : 4;
-    // fragments in flight per register buffer: 2 for the widest GEMM (the temporal FFN linear_in, 704 n-tiles: fewer
-    // registers -> 3 workgroups per CU -> all 704 resident at once; 36.8 vs 39.3 us in the microbenchmark), else 4
+    // fragments in flight per register buffer of k_gemm_xp: 2 for a gated GEMM of very many tiles (linear_in's 704, where neither
+    // k_gemm_xreg nor k_gemm_xlds takes it: fewer registers -> 3 workgroups per CU -> all 704 resident at once; 36.8 vs 39.3 us in the
+    // microbenchmark), else 4
     p.u = (g.gate && g.NT >= 512 && p.waves == 8) ? 2 : 4;
     if (g.scale) p.u = 2;            // int8 entries carry two k-steps each
     // (two n-tiles per workgroup for the 384-tile temporal in_proj look 3.5 us faster in the microbenchmark - 22.5 against
@@ -380,7 +381,7 @@ int launch_gemm_t(hipStream_t s, const GemmPlan& p, int NT, int mt, const GemmAr
 
 // k_gemm_xlds (activations resident in LDS, one workgroup per CU): which of the GEMMs that plan_xreg leaves take it, and how.  MMI_GEMM_LDS: "2" = with
 // the staggered tail (each tile's epilogue under the last chunk's weight stream; the DEFAULT for bf16 weights at the 32-row
-// tile: same-box A/B of the default benchmark 8.10 / 8.12 ms against 8.17 / 8.20 ms with k_gemm_xp, dominant kernel 38.6
+// tile, in place of k_gemm_xp: same-box A/B of 32 sessions 8.10 / 8.12 ms against 8.17 / 8.20 ms with k_gemm_xp, dominant kernel 38.6
 // against 40.2 us live, profiles/r02_logs/ab_gemm_xlds_stagger_in_step.txt), "1" = plain tails (also what int8 / fp8 weight
 // entries take when asked for; they stay on k_gemm_xp by default), "0" = k_gemm_xp everywhere.
 struct XldsPlan { bool on; int kc, grid; size_t smem; bool stagger; };

@@ -402,10 +402,6 @@ __device__ __forceinline__ void mmi_gemm_epilogue(const GemmArgs& a, float (&acc
             for (int e = 0; e < 4; ++e) v[e] = mmi_round_bf16(s[e]);          // in_proj output is a bf16 tensor
             if (sec < 2) {
                 const f32x4 cs = *reinterpret_cast<const f32x4*>(a.rope + ((long)b * (a.Dh / 2) + d0 / 2) * 2);      // two (cos, sin) pairs
-                // mmi_rope_rotate = four multiplies, a subtract, an add as separate VALU instructions.  Written as `re * c - im * sn` the
-                // compiler packed the pairs into v_pk_mul_f32 / v_pk_add_f32 with op_sel swizzles, one of them in place, and on gfx950 that
-                // sequence inside k_gemm_xp<32, 2, ..> (64 sessions) returned, now and then, a stale last element for lanes 48-63 - q / k of
-                // 16 sessions wrong in one feature, a different one from run to run (profiles/r05_logs/c5_trace_*.txt)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const float re = v[2 * j], im = v[2 * j + 1];
@@ -1303,7 +1299,9 @@ __global__ __launch_bounds__(512) void k_gemm_xlds(GemmArgs a) {
 // per launch.  What is left of the loop is the weight stream - NX entries of 1 KiB per tile and wave, RD of them on their way in a ring of
 // registers that runs on through the tiles - and the products; no LDS, no barrier.  Each tile ends in the sum over the waves and the epilogue,
 // under the stream of the next one: loads come back in the order they were asked for, so the epilogue's operands (absmax and scales, offsets,
-// angles) are copied to LDS at the start - one that read global memory would wait for all of the ring.
+// angles) are copied to LDS at the start - one that read global memory would wait for all of the ring.  The two widest forms (4096 features)
+// nevertheless do so where in_proj writes its ring (at int8: a bf16 ring): registers for its addresses are short, 4 and 2 of them lie in scratch memory
+// (32 sessions: in_proj 4.84 TB/s, linear_in, whose epilogue reads none of them, 5.54).
 // Bound by the weight stream (a chain of launches that only read gets 92 MB in 15.2 us, 184 MB in 29), the activations' 1 - 2 us and the last
 // tile's epilogue.  Chains of dependent launches on weights from memory, us, before (int8 k_gemm_xp; bf16 k_gemm_xlds, PARTIAL k_gemm_xp) / here:
 //   64 rows, int8   linear_in 92 MB 25.5 / 19.9, in_proj 50 MB 18.3 / 15.2, linear_out 46 MB 14.5 / 12.4, out_proj 17 MB 7.9 / 7.2

@@ -258,9 +258,11 @@ __device__ __forceinline__ f32x4 mmi_mfma_bf16_16x16x32(u32x4 a, u32x4 b, f32x4 
 }
 
 // One RoPE rotation (re, im) -> (re c - im s, re s + im c) in plain (un-packed) fp32 VALU instructions, each rounded once (no
-// fma), pinned by inline asm so that the compiler cannot re-form them into packed-math (v_pk_mul_f32 / v_pk_add_f32 with op_sel
-// swizzles) - see the note at its call site in lm_kernels.h (mmi_gemm_epilogue, MMI_EPI_ROPE_KV).  Arithmetic unchanged: the same
-// six IEEE operations the C expression means under -ffp-contract=off.
+// fma), pinned by inline asm so that the compiler cannot re-form them into packed math: the same six IEEE operations the C expression
+// means under -ffp-contract=off.  Written as `re * c - im * sn` the compiler packed pairs of rotations into v_pk_mul_f32 / v_pk_add_f32 with
+// op_sel swizzles, one of them in place, and on gfx950 that sequence inside k_gemm_xp<32, 2, ..> (64 sessions) returned, now and then, a
+// stale last element for lanes 48-63 - q / k of 16 sessions wrong in one feature, a different one from run to run
+// (profiles/r05_logs/c5_trace_*.txt).  Every epilogue that rotates takes this.
 __device__ __forceinline__ void mmi_rope_rotate(float re, float im, float c, float sn, float& out_re, float& out_im) {
     float a, b, d, e;
     asm volatile("v_mul_f32 %0, %1, %2" : "=v"(a) : "v"(re), "v"(c));

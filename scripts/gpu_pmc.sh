@@ -10,6 +10,6 @@ for ctr in FETCH_SIZE WRITE_SIZE; do
   cd $GRAFT_REPO_ROOT
   tail -3 $O/rocprof_pmc_$ctr.log | cut -c1-200
   if [ $rc != 0 ] || ! ls /tmp/prof_pmc_$ctr/*.db > /dev/null 2>&1; then break; fi
-  python scripts/rocpd_pmc.py /tmp/prof_pmc_$ctr/pmc_results.db --header "rocprofv3 --pmc $ctr --kernel-trace -- MMI_NO_GRAPH=1 python bench.py --no-cpu-baseline --workload lm --steps 2 --warmup 1 (the LM step of the product library, 32 sessions)" --clusters k_gemm_xlds > $O/pmc_${ctr}_in_step.csv 2>&1
+  python scripts/rocpd_pmc.py /tmp/prof_pmc_$ctr/pmc_results.db --header "rocprofv3 --pmc $ctr --kernel-trace -- MMI_NO_GRAPH=1 python bench.py --no-cpu-baseline --workload lm --steps 2 --warmup 1 (the LM step of the product library, 32 sessions)" --clusters k_gemm_xreg > $O/pmc_${ctr}_in_step.csv 2>&1
 done
 cat $O/pmc_FETCH_SIZE_in_step.csv | cut -c1-200 | tail -8; cat $O/pmc_WRITE_SIZE_in_step.csv | cut -c1-200 | tail -6

@@ -1,6 +1,6 @@
 # Counter passes over the LM step on the product library, eager launches (every dispatch is a packet the counters can be
 # attributed to).
-#  * 32 sessions, bf16, mid-run ring depth: FETCH_SIZE / WRITE_SIZE / TCC for the dominant GEMM (k_gemm_xlds) AND the decode attention
+#  * 32 sessions, bf16, mid-run ring depth: FETCH_SIZE / WRITE_SIZE / TCC for the dominant GEMM (k_gemm_xreg) AND the decode attention
 #    (k_lm_attn_wave), so that roofline.traffic is a figure of THIS round and the attention's clamped re-reads are counted;
 #  * the same FETCH_SIZE pass with every ring 3000 deep (--kv-depth full);
 #  * 64 sessions, int8 x int8 (C5): SQ (busy / wait / MFMA-busy / VALU / LDS) and TCC passes over k_gemm_xp<.., WQ = 3>, and the SQ

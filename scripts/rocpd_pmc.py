@@ -24,7 +24,7 @@ def main():
         name = name if len(name) < 160 else name[:157] + "..."
         corr = avg * 1024 * (2 if ctr == "FETCH_SIZE" else 1)
         print(f'"{name}",{ctr},{n},{avg:.1f},{mn:.1f},{mx:.1f},{corr:.0f},{dur/1e3:.2f}')
-    # One kernel name serves several GEMM shapes (k_gemm_xlds: in_proj, linear_in, the text head): `--clusters <substring>` lists
+    # One kernel name serves several GEMM shapes (k_gemm_xreg: in_proj, linear_in, the text head): `--clusters <substring>` lists
     # that kernel's dispatches grouped by counter value (bins of 4 MiB), i.e. one line per shape it was launched on.
     if "--clusters" in sys.argv:
         sub = sys.argv[sys.argv.index("--clusters") + 1]
